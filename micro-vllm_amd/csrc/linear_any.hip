@@ -3,12 +3,15 @@
 // The wave-tile projections (wgemm.hip, gemm_prefill.hip) want N % 16 == 0, K % 32 / 64 == 0 and a
 // relaid-out weight image; layer stacks whose widths are whatever their configuration says (an
 // input projection of 2*inner + 2*groups*state + heads rows, an inner width of heads * vdim) use
-// this kernel for the shapes those cannot take.  Two forms:
+// this kernel for the shapes those cannot take.
 //   bf16 operands: 64 x 64 output tile per workgroup of 4 waves, k in steps of 32 through LDS,
-//                  v_mfma_f32_16x16x32_bf16, edges zero-filled in LDS;
-//   fp32 operands: the same tile with fused multiply-adds (no reduced-precision matrix mode).
-// Every output is the sum over k in ascending order of 32-wide (bf16) or 16-wide (fp32) steps,
-// whatever M is: a row's result does not depend on which other rows share the launch.
+//                  v_mfma_f32_16x16x32_bf16, edges zero-filled in LDS; the sum over k in ascending order of those
+//                  steps;
+//   fp32 operands: tiles of three sizes on the fp32 matrix instruction (no reduced-precision mode), or, for a few
+//                  rows, the weights streamed past them.  In every form a sum over k is made of four quarters of k
+//                  (in whole steps of 32) that are added up in ascending order, a quarter of the same sequence of
+//                  matrix instructions.
+// So a row's result does not depend on which other rows share the launch.
 #include "common.h"
 #include <type_traits>
 
@@ -190,19 +193,66 @@ __global__ __launch_bounds__(256) void linear_any_bf16_big_kernel(
     }
 }
 
-constexpr int kLfBK = 16;
+// fp32 operands on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: products and sums in 32 bits).  That
+// instruction needs 32 cycles for 2048 FLOP, so a tile is bound by it and not by LDS or loads as long as loads are in
+// flight: PF k-steps of 32 in registers in front of a double buffer in LDS, one barrier a step.  A lane reads four
+// neighbouring k of its row at once and the four instructions behind take one of them each: both operands agree on which
+// k that is, so the sum is over the same sixteen.  LDS rows of 36 floats put the 16 rows of such a read on 16 different
+// groups of four banks.
+// WM x WN accumulator tiles per wave, four waves as 2 x 2: (32 WM) x (32 WN) outputs.  The quarters of k are taken one
+// after the other by the same waves (KG = 1; a second set of accumulators holds the sum so far), or side by side by four
+// groups of four waves (KG = 4): a launch of few tiles is a chain of load latencies (about 0.8 us a step behind HBM),
+// which four groups with four steps ahead each cut by more than four.  The widest tile
+// has 64 accumulators and 32 MFMA times a step to hide a load behind: one step ahead, so that two of its workgroups
+// share a unit (two steps ahead: one workgroup, 97 instead of 128 TFLOP/s).
+// Measured against the 64 x 64 tile of vector fused multiply-adds with k in steps of 16 that was here (outputs x k, us):
+// 567 rows 1024 x 5120 570 -> 105, 9472 x 1024 346 -> 116, 16384 x 4096 2551 -> 642 (119 TFLOP/s); 2048 rows 16384 x
+// 4096 2156 (128 TFLOP/s); 64 rows 1024 x 5120 581 -> 35, 9472 x 1024 126 -> 31.  The error against 64 bits is half of
+// what it was (1024 x 5120: 1.3e-6 -> 6.4e-7): the sums are of quarters.
+constexpr int kLfBK = 32, kLfPad = 36;
 
-__global__ __launch_bounds__(256) void linear_any_f32_kernel(
+// VEC: rows at multiples of 16 bytes and K % 4 == 0.  Columns past the end of k are zeros and nothing is read there; rows
+// past the last one were clamped by the caller (their outputs are not stored).
+template <bool VEC>
+__device__ __forceinline__ f32x4_t lf_load4(const float* p, int col, int k) {
+    f32x4_t v;
+    if (VEC) {
+        v = *reinterpret_cast<const f32x4_t*>(p + (col < k ? col : 0));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = col < k ? v[i] : 0.f;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float e = p[col + i < k ? col + i : 0];
+            v[i] = col + i < k ? e : 0.f;
+        }
+    }
+    return v;
+}
+
+// Tiles of one column of outputs (one piece of W) go to one XCD, whose L2 then holds that piece: workgroups are dealt
+// out over the eight XCDs in turn, so eight columns advance side by side.
+__device__ __forceinline__ bool lf_place(int id, int cols, int rows, int& col, int& row) {
+    col = (id / (8 * rows)) * 8 + (id & 7);
+    row = (id >> 3) % rows;
+    return col < cols;
+}
+
+template <int WM, int WN, int KG, int PF, bool VEC>
+__global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kernel(
     const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
     float* __restrict__ y, int64_t ldy, int M, int N, int K, int64_t zx, int64_t zw, int64_t zy, RowSegments sg) {
+    constexpr int BM = 32 * WM, BN = 32 * WN;
     x += blockIdx.z * zx;
     w += blockIdx.z * zw;
     y += blockIdx.z * zy;
-    __shared__ float xs[kLfBK][kLaBM + 4];
-    __shared__ float ws[kLfBK][kLaBN + 4];
-    const int m0 = blockIdx.y * kLaBM, n0 = blockIdx.x * kLaBN;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int lrow = tid >> 2, lcol = (tid & 3) * 4;
+    extern __shared__ __attribute__((aligned(16))) float lf_lds[];
+    int nb, mb;
+    if (!lf_place(blockIdx.x, (N + BN - 1) / BN, (M + BM - 1) / BM, nb, mb)) return;
+    const int m0 = mb * BM, n0 = nb * BN;
+    const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255;
+    const int wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4, wm = wave >> 1, wn = wave & 1;
+    const int lrow = tid >> 3, lcol = (tid & 7) * 4;
     int64_t y0 = 0;
     if (sg.seg) {
         y0 = sg.seg[blockIdx.z];
@@ -210,45 +260,208 @@ __global__ __launch_bounds__(256) void linear_any_f32_kernel(
         if (m0 >= M) return;
         y += y0 * ldy;
     }
-    {
-        const int mr = m0 + lrow;
-        const int64_t xrow = mr < M ? (sg.src ? sg.src[y0 + mr] / sg.src_div : y0 + mr) : 0;
-        x += xrow * ldx - (int64_t)(m0 + lrow) * ldx;
-    }
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += kLfBK) {
-        __syncthreads();
+    const float* xp[WM];
+    const float* wp[WN];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int kk = k0 + lcol + i;
-            xs[lcol + i][lrow] = (m0 + lrow < M && kk < K) ? x[(int64_t)(m0 + lrow) * ldx + kk] : 0.f;
-            ws[lcol + i][lrow] = (n0 + lrow < N && kk < K) ? w[(int64_t)(n0 + lrow) * ldw + kk] : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < kLfBK; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = xs[kk][ty * 4 + i];
-                b[i] = ws[kk][tx * 4 + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
+    for (int u = 0; u < WM; ++u) {
+        const int mr = m0 + lrow + 32 * u;
+        xp[u] = x + (mr < M ? (sg.src ? sg.src[y0 + mr] / sg.src_div : y0 + mr) : 0) * ldx;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
+    for (int u = 0; u < WN; ++u) wp[u] = w + (int64_t)min(n0 + lrow + 32 * u, N - 1) * ldw;
+    float* buf = lf_lds + grp * 2 * (BM + BN) * kLfPad;
+    f32x4_t acc[WN][WM], sum[WN][WM];
+    const int per = ((K + kLfBK - 1) / kLfBK + 3) / 4;   // k-steps of a quarter
+    auto clear = [&] {
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int b = 0; b < WM; ++b) acc[a][b] = f32x4_t{0, 0, 0, 0};
+    };
+    int fold = per;
+    auto add_quarter = [&] {
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int b = 0; b < WM; ++b)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sum[a][b][j] = fold == per ? acc[a][b][j] : sum[a][b][j] + acc[a][b][j];
+        fold += per;
+    };
+    clear();
+    f32x4_t xr[PF][WM], wr[PF][WN];
+    auto request = [&](int set, int step) {
+        const int col = ((KG > 1 ? grp * per : 0) + step) * kLfBK + lcol;
+#pragma unroll
+        for (int u = 0; u < WM; ++u) xr[set][u] = lf_load4<VEC>(xp[u], col, K);
+#pragma unroll
+        for (int u = 0; u < WN; ++u) wr[set][u] = lf_load4<VEC>(wp[u], col, K);
+    };
+    auto multiply = [&](int set, int half, int step) {
+        float* xs = buf + half * (BM + BN) * kLfPad;
+        float* ws = xs + BM * kLfPad;
+#pragma unroll
+        for (int u = 0; u < WM; ++u) *reinterpret_cast<f32x4_t*>(xs + (lrow + 32 * u) * kLfPad + lcol) = xr[set][u];
+#pragma unroll
+        for (int u = 0; u < WN; ++u) *reinterpret_cast<f32x4_t*>(ws + (lrow + 32 * u) * kLfPad + lcol) = wr[set][u];
+        request(set, step + PF);
+        __syncthreads();   // the other half was read a step ago, before this barrier by every wave
+        if (KG == 1 && step == fold) {
+            add_quarter();
+            clear();
+        }
+#pragma unroll
+        for (int ks = 0; ks < kLfBK; ks += 16) {
+            f32x4_t wf[WN], xf[WM];
+#pragma unroll
+            for (int t = 0; t < WN; ++t)
+                wf[t] = *reinterpret_cast<const f32x4_t*>(ws + (wn * 16 * WN + t * 16 + r) * kLfPad + ks + q * 4);
+#pragma unroll
+            for (int t = 0; t < WM; ++t)
+                xf[t] = *reinterpret_cast<const f32x4_t*>(xs + (wm * 16 * WM + t * 16 + r) * kLfPad + ks + q * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int a = 0; a < WN; ++a)
+#pragma unroll
+                    for (int b = 0; b < WM; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[a][e], xf[b][e], acc[a][b], 0, 0, 0);
+        }
+    };
+    const int steps = KG > 1 ? per : 4 * per;   // of every group alike: the barriers are shared; past the end of k: zeros
+#pragma unroll
+    for (int i = 0; i < PF; ++i) request(i, i);
+    constexpr int TURN = PF > 2 ? PF : 2;   // steps after which register sets and halves are where they were
+    int st = 0;
+    for (; st + TURN <= steps; st += TURN)
+#pragma unroll
+        for (int i = 0; i < TURN; ++i) multiply(i % PF, i & 1, st + i);
+#pragma unroll
+    for (int i = 0; i < TURN - 1; ++i)
+        if (st + i < steps) multiply(i % PF, i & 1, st + i);
+    if (KG == 1) {
+        add_quarter();
+#pragma unroll
+        for (int a = 0; a < WN; ++a)
+#pragma unroll
+            for (int b = 0; b < WM; ++b) acc[a][b] = sum[a][b];
+    }
+    if (KG > 1) {   // group 0 adds up the groups
+        __syncthreads();
+        constexpr int kAcc = WN * WM * 4;
+        float* part = lf_lds + ((grp - 1) * 256 + tid) * (kAcc + 1);
+        if (grp > 0) {
+#pragma unroll
+            for (int a = 0; a < WN; ++a)
+#pragma unroll
+                for (int b = 0; b < WM; ++b)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) part[(a * WM + b) * 4 + j] = acc[a][b][j];
+        }
+        __syncthreads();
+        if (grp > 0) return;
+        for (int g = 0; g < KG - 1; ++g) {
+            const float* o = lf_lds + (g * 256 + tid) * (kAcc + 1);
+#pragma unroll
+            for (int a = 0; a < WN; ++a)
+#pragma unroll
+                for (int b = 0; b < WM; ++b)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[a][b][j] += o[(a * WM + b) * 4 + j];
+        }
+    }
+    // acc[a][b][j] = C[n = n0 + 16 (WN wn + a) + 4 q + j][m = m0 + 16 (WM wm + b) + r]
+#pragma unroll
+    for (int b = 0; b < WM; ++b) {
+        const int m = m0 + (wm * WM + b) * 16 + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n < N) y[(int64_t)m * ldy + n] = acc[i][j];
+        for (int a = 0; a < WN; ++a) {
+            const int n = n0 + (wn * WN + a) * 16 + q * 4;
+            float* dst = y + (int64_t)m * ldy + n;
+            if (n + 3 < N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+                *reinterpret_cast<float4*>(dst) = make_float4(acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (n + j < N) dst[j] = acc[a][b][j];
+            }
         }
     }
+}
+
+// fp32 operands, few rows: the weights are streamed past them, straight from memory into the operand registers of the
+// same matrix instructions.  A workgroup forms sixteen neighbouring outputs of up to sixteen rows, its four waves the
+// four quarters of k; kStreamAhead steps (32 k of sixteen weight rows, 2 KB) of a wave are in flight while the ones before
+// are multiplied.  Rows past the last one repeat it: the matrix instruction takes sixteen either way, and a launch like
+// this waits for memory.
+// Measured (outputs x k, us; before: 64 x 64 tiles of vector FMAs): 1 row 1024 x 5120 477 -> 20, 9472 x 1024 105 -> 15,
+// 32000 x 1024 140 -> 36, 16384 x 4096 416 -> 60 (4.5 TB/s); 8 rows 490 -> 24, 109 -> 18, 144 -> 43, 426 -> 73.  The 32 x
+// 32 tile takes 34, 22, 44, 74 for up to 32 rows: it is ahead from 9 rows on where the output is wide (16 rows, 32000 x
+// 1024: 45 against 53), from 17 on everywhere (32 rows, 1024 x 5120: 35 against 40).
+constexpr int kStreamRows = 8, kStreamRowsNarrow = 16, kStreamNarrow = 8192, kStreamAhead = 4;
+
+__global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __restrict__ x, int64_t ldx,
+                                                                const float* __restrict__ w, int64_t ldw,
+                                                                float* __restrict__ y, int64_t ldy, int M, int N, int K) {
+    __shared__ float part[3][64][5];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4, n0 = blockIdx.x * 16;
+    const int per = ((K + kLfBK - 1) / kLfBK + 3) / 4;
+    const float* wp = w + (int64_t)min(n0 + r, N - 1) * ldw;
+    const float* xp = x + (int64_t)min(r, M - 1) * ldx;
+    f32x4_t acc = {0, 0, 0, 0};
+    constexpr int U = kStreamAhead;
+    f32x4_t wv[2][U][2], xv[2][U][2];
+    auto request = [&](int set, int st) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                // past the quarter nothing is multiplied: its row's start is read instead of another quarter's data
+                const int col = st + u < per ? (wave * per + st + u) * kLfBK + h * 16 + q * 4 : K;
+                const bool in = col < K;
+                wv[set][u][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(wp + (in ? col : 0)));
+                xv[set][u][h] = *reinterpret_cast<const f32x4_t*>(xp + (in ? col : 0));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    wv[set][u][h][e] = in ? wv[set][u][h][e] : 0.f;
+                    xv[set][u][h][e] = in ? xv[set][u][h][e] : 0.f;
+                }
+            }
+    };
+    auto multiply = [&](int set, int st) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (st + u >= per) continue;   // uniform
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[set][u][h][e], xv[set][u][h][e], acc, 0, 0, 0);
+        }
+    };
+    request(0, 0);
+    for (int st = 0; st < per; st += 2 * U) {
+        request(1, st + U);
+        multiply(0, st);
+        request(0, st + 2 * U);
+        multiply(1, st + U);
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[wave - 1][lane][j] = acc[j];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int g = 0; g < 3; ++g)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] += part[g][lane][j];
+    // acc[j] = C[n = n0 + 4 q + j][m = r]
+    if (r >= M) return;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (n0 + q * 4 + j < N) y[(int64_t)r * ldy + n0 + q * 4 + j] = acc[j];
 }
 
 // Few output rows (decoding): a wave forms four neighbouring outputs of ONE row from 16-byte loads of the operand
@@ -323,10 +536,55 @@ __global__ __launch_bounds__(256) void linear_fewrows_kernel(const void* __restr
 
 }  // namespace mv
 
+template <int WM, int WN, int KG, int PF>
+static int launch_linear_f32_tiles(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m,
+                                   int n, int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s,
+                                   mv::RowSegments sg) {
+    using namespace mv;
+    constexpr int BM = 32 * WM, BN = 32 * WN;
+    const int64_t cols = (n + BN - 1) / BN, rows = (m + BM - 1) / BM, groups = (cols + 7) / 8 * 8 * rows;
+    if (groups > 0x7fffffff) return MV_ERR_UNSUPPORTED;
+    size_t lds = (size_t)KG * 2 * (BM + BN) * kLfPad * 4;
+    const size_t meet = (size_t)(KG - 1) * 256 * (WM * WN * 4 + 1) * 4;
+    if (meet > lds) lds = meet;
+    const bool vec = k % 4 == 0 && aligned16(x) && ldx % 4 == 0 && zx % 4 == 0 && aligned16(w) && ldw % 4 == 0 && zw % 4 == 0;
+    static LdsOptIn done[2];
+    const auto kernel = vec ? linear_any_f32_kernel<WM, WN, KG, PF, true> : linear_any_f32_kernel<WM, WN, KG, PF, false>;
+    if (const int rc = ensure_dynamic_lds((const void*)kernel, lds, done[vec])) return rc;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)groups, 1, batch), dim3(256 * KG), lds, s, x, ldx, w, ldw, y, ldy, m, n, k,
+                       zx, zw, zy, sg);
+    return check_launch();
+}
+
+// Which fp32 form.  Few rows of one product stream the weights (see kStreamRows).  Otherwise the tile by the time the
+// launch takes in it: rounds of tiles over the compute units times what a tile costs a unit, in us per 1024 of k as
+// measured - 8 for 32 x 32 (four groups over k), 24 for a 64 x 64 tile by itself and 19 where several share a unit, 73
+// for 128 x 128 - so that a launch of few tiles takes small ones and a large one the tile that reads its operands least
+// often.  With segments `m` bounds a segment, not the launch: the rows are taken to be spread evenly.
+static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
+                             int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s, mv::RowSegments sg,
+                             int total_rows) {
+    using namespace mv;
+    if (m <= (n < kStreamNarrow ? kStreamRowsNarrow : kStreamRows) && !sg.seg && batch == 1 && k % 4 == 0 && ldx % 4 == 0 &&
+        ldw % 4 == 0 && aligned16(x) && aligned16(w)) {
+        hipLaunchKernelGGL(linear_stream_f32_kernel, dim3((n + 15) / 16), dim3(256), 0, s, x, ldx, w, ldw, y, ldy, m, n, k);
+        return check_launch();
+    }
+    const int64_t per = sg.seg ? (total_rows + batch - 1) / batch : m;
+    const int64_t cus = num_cus();
+    auto rounds = [&](int b) { return (((per + b - 1) / b) * ((n + b - 1) / b) * batch + cus - 1) / cus; };
+    const int64_t c32 = 8 * rounds(32), c64 = rounds(64) <= 1 ? 24 : 19 * rounds(64), c128 = 73 * rounds(128);
+    if (c32 <= c64 && c32 <= c128)
+        return launch_linear_f32_tiles<1, 1, 4, 4>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+    if (c64 <= c128)
+        return launch_linear_f32_tiles<2, 2, 1, 2>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+    return launch_linear_f32_tiles<4, 4, 1, 1>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+}
+
 static int launch_linear_any(const void* x, int64_t ldx, const void* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
                              int k, int f32, int batch, int64_t zx, int64_t zw, int64_t zy, mv_stream_t stream,
                              mv::RowSegments sg = mv::RowSegments{nullptr, nullptr, 1}, int few_rows = 0,
-                             bool big_tiles = false) {
+                             bool big_tiles = false, int total_rows = 0) {
     using namespace mv;
     const dim3 grid((n + kLaBN - 1) / kLaBN, (m + kLaBM - 1) / kLaBM, batch);
     if (grid.y > 65535 || batch > 65535) return MV_ERR_UNSUPPORTED;
@@ -343,8 +601,7 @@ static int launch_linear_any(const void* x, int64_t ldx, const void* w, int64_t 
         }
     }
     if (f32) {
-        hipLaunchKernelGGL(linear_any_f32_kernel, grid, dim3(256), 0, s, (const float*)x, ldx, (const float*)w, ldw,
-                           y, ldy, m, n, k, zx, zw, zy, sg);
+        return launch_linear_f32((const float*)x, ldx, (const float*)w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg, total_rows);
     } else {
         const int vx = aligned16(x) && ldx % 8 == 0 && zx % 8 == 0, vw = aligned16(w) && ldw % 8 == 0 && zw % 8 == 0;
         if (big_tiles && n >= kLbBN) {
@@ -390,5 +647,5 @@ extern "C" int mv_linear_segments(const void* x, int64_t ldx, const void* w, int
     if (!x || !w || !y || !seg || ldx < k || ldw < k || ldy < n) return MV_ERR_INVALID_ARG;
     return launch_linear_any(x, ldx, w, ldw, y, ldy, max_rows, n, k, f32, segments, 0, zw, 0, stream,
                              mv::RowSegments{seg, src, src_div}, total_rows <= mv::kFewRows ? total_rows : 0,
-                             total_rows / segments >= 96);
+                             total_rows / segments >= 96, total_rows);
 }

@@ -50,6 +50,27 @@ def test_linear_any(ops, f32, m, n, k):
     assert torch.equal(lin(x[:1].to(DEV)).cpu().double(), got[:1])
 
 
+@pytest.mark.parametrize("m,n,k,pad", [(1, 16, 4, 0), (8, 8200, 36, 4), (9, 8200, 36, 4), (16, 100, 1028, 0), (17, 100, 1028, 0),
+                                       (33, 33, 31, 1), (64, 9000, 132, 0), (200, 9000, 132, 0), (700, 1100, 160, 4),
+                                       (4100, 2100, 64, 0)])
+def test_linear_any_f32_forms(ops, m, n, k, pad):
+    """Streamed weights, the three tiles, vector and scalar loads: each within the bound of a 32-bit sum, and all of them the
+    same sums bit for bit (a row on its own, behind its neighbours, in rows of a wider buffer)."""
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
+    wide = torch.full((m, k + pad), float("nan"), device=DEV)      # nothing beside the operand is read into a sum
+    wide[:, :k] = x.to(DEV)
+    out = torch.full((m, n + 3), 7.0, device=DEV)
+    lin = ops.AnyLinear(w.to(DEV), wave_tiles=False)
+    got = lin(wide[:, :k], out[:, :n])
+    assert bool((out[:, n:] == 7.0).all())
+    err = (got.cpu().double() - x.double() @ w.double().T).abs()
+    # at most k roundings of 2^-24 of partial sums that the absolute products bound
+    assert bool((err <= k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all())
+    for rows in (slice(0, 1), slice(m - 1, m), slice(0, min(m, 20)), slice(m // 2, m)):
+        assert torch.equal(lin(x[rows].to(DEV)), got[rows])
+
+
 def test_wave_tile_and_plain_projection_agree(ops):
     g = torch.Generator().manual_seed(1)
     w = (torch.randn(96, 128, generator=g) / 11).to(torch.bfloat16).to(DEV)
