@@ -39,6 +39,35 @@ def test_sample_matches_oracle(mv, v, top_k):
     assert len(mism) <= 1
 
 
+@pytest.mark.parametrize("v", [8, 64, 512, 8200, 131072, 131080, 151936])
+@pytest.mark.parametrize("kind", ["random", "ties", "zeros", "sorted", "few"])
+def test_selection_through_maxima_equals_radix_selection(mv, v, kind):
+    """A NaN sorts below everything and sends its row through the radix selection; -inf in its place leaves the row on the
+    selection through the threads' maxima (rows of mostly equal logits excepted, which overflow its list)."""
+    from micro_vllm_amd.core.layer.sampler import sample
+
+    g = torch.Generator().manual_seed(v)
+    bs = 6
+    x = torch.randn(bs, v, generator=g) * 3
+    if kind == "ties":
+        x = (x * 2).round() / 2
+    elif kind == "zeros":       # zeros of both signs among the largest
+        x = -x.abs().round()
+    elif kind == "sorted":
+        x = x.sort(dim=-1, descending=True).values
+    elif kind == "few":
+        x[:, 3:] = -float("inf")
+    x = x.to(torch.bfloat16)
+    at = torch.randint(0, v, (bs,), generator=g)
+    a, b = x.clone(), x.clone()
+    a[torch.arange(bs), at], b[torch.arange(bs), at] = -float("inf"), float("nan")
+    temps, top_ps, u = torch.rand(bs, generator=g) + 0.5, torch.rand(bs, generator=g) * 0.5 + 0.5, torch.rand(bs, generator=g)
+    for k in (1, 2, 50, 64, 65, 255, 256):
+        if k > (3 if kind == "few" else v) - 1:
+            continue        # the NaN itself would be among the k
+        assert torch.equal(sample(a.to(DEV), temps, top_ps, k, uniforms=u), sample(b.to(DEV), temps, top_ps, k, uniforms=u)), k
+
+
 def test_sampler_class_uses_device_kernel_and_respects_top_k(mv):
     from micro_vllm_amd.core.layer.sampler import Sampler
 
