@@ -86,7 +86,11 @@ __device__ __forceinline__ void stage_qkv_from_slabs(const AttnArgs& a, uint16_t
 template <int D, int G, int W>
 __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     constexpr int kAW = W;          // waves per workgroup
-    constexpr int kAC = 4;          // row loads per wave per pipeline stage
+    // Row loads per wave per pipeline stage.  With more than four query heads two: four take 305 registers (one
+    // workgroup a unit, and twice the arithmetic of a stage that a short context hardly fills).  32 heads of 64 on 4:
+    // 45 tokens 9.2 -> 8.0 us, one row of 4000 13.3 -> 12.7, 32 rows of 2000 in 4 splits 43 -> 32.  With four heads or
+    // fewer a second workgroup fits either way, and bytes in flight set the pace of long rows.
+    constexpr int kAC = G > 4 ? 2 : 4;
     constexpr int LPR = D / 8;      // lanes per row
     constexpr int RPI = 64 / LPR;   // rows per wave instruction
     constexpr int NS = kAW * RPI;   // softmax states per workgroup
@@ -104,7 +108,6 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     const int split = blockIdx.x % a.nsplit;
     const int bh = blockIdx.x / a.nsplit;
     const int kvh = bh % a.hkv, b = bh / a.hkv;
-    const bool last_split = (split == a.nsplit - 1);
 
     // keys 0..pos-1 are cached, the new key lands at pos; requested first, needed only after the
     // loads that do not depend on it are on their way
@@ -129,6 +132,12 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     int pgA[kAC], pgB[kAC];
     load_pages(pgA, 0);
     load_pages(pgB, 1);
+
+    constexpr int CR = NS * kAC;  // rows per chunk
+    const int seq_chunks = (max(pos, 0) + CR - 1) / CR;
+    const int filled = filled_splits(a.nsplit, seq_chunks);
+    const int nchunk = seq_chunks > split ? (seq_chunks - split + a.nsplit - 1) / a.nsplit : 0;
+    const bool last_split = split == filled - 1;
 
     const bool rotate = (a.rot_cos != nullptr);
     const bool first_half = d0 < D / 2;
@@ -165,6 +174,9 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
 #ifdef MV_ATTN_STAMP
     if (pos >= 0) MV_ASTAMP(11);
 #endif
+    // (behind the requests above: a split with tokens does not wait for the length before it makes them)
+    __builtin_amdgcn_sched_barrier(0);
+    if (split >= filled && (a.nsplit == 1 || a.arrive)) return;   // uniform; nothing of this row is here
     uint4 cosv = make_uint4(0, 0, 0, 0), sinv = cosv;
     if (rotate) {
         const int rp = min(max(pos, 0), a.rot_max_pos - 1);
@@ -172,10 +184,6 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
         cosv = ld16(a.rot_cos + ro);
         sinv = ld16(a.rot_sin + ro);
     }
-    constexpr int CR = NS * kAC;  // rows per chunk
-    const int seq_chunks = (max(pos, 0) + CR - 1) / CR;
-    const int nchunk = seq_chunks > split ? (seq_chunks - split + a.nsplit - 1) / a.nsplit : 0;
-
     auto load_rows = [&](uint4(&kb)[kAC], uint4(&vb)[kAC], bool(&ok)[kAC], const int (&pg)[kAC], int c) {
 #pragma unroll
         for (int i = 0; i < kAC; ++i) {
@@ -361,7 +369,7 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
         *reinterpret_cast<f32x4_t*>(dst) = (f32x4_t){acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
         *reinterpret_cast<f32x4_t*>(dst + 4) = (f32x4_t){acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
     }
-    finish_states<D, G, NS, kAW>(a, lds, b, kvh, bh, split, wid, lane);
+    finish_states<D, G, NS, kAW>(a, lds, b, kvh, bh, split, wid, lane, filled);
 }
 
 // ------------------------------------------------------------ matrix-core form (D = 128, G >= 4)
@@ -398,7 +406,6 @@ __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a)
     const int split = blockIdx.x % a.nsplit;
     const int bh = blockIdx.x / a.nsplit;
     const int kvh = bh % a.hkv, b = bh / a.hkv;
-    const bool last_split = (split == a.nsplit - 1);
 
     const int pos = a.seqlens[b];
     const int32_t* bt = a.block_table + (int64_t)b * a.bt_stride;
@@ -413,6 +420,10 @@ __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a)
         return bt[min(t0 >> a.page_shift, a.bt_stride - 1)];
     };
     int pgA = page_of(0), pgB = page_of(1);   // pages of the current and the next stage
+    const int nblk = (max(pos, 0) + kMRows - 1) / kMRows;
+    const int filled = filled_splits(a.nsplit, (nblk + kAW - 1) / kAW);
+    const int nchunk = nblk > blk_first ? (nblk - blk_first + blk_step - 1) / blk_step : 0;
+    const bool last_split = split == filled - 1;
 
     // ---- query heads (B operand: lane (r, q) = head r, 8 values at 32 kk + 8 q), new k / v ----
     const bool rotate = (a.rot_cos != nullptr);
@@ -469,6 +480,9 @@ __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a)
     uint4 kR[8], vR[8];
     load_k(kR, pgA, 0);
     load_v(vR, pgA, 0);
+    // (behind the requests above: a split with tokens does not wait for the length before it makes them)
+    __builtin_amdgcn_sched_barrier(0);
+    if (split >= filled && (a.nsplit == 1 || a.arrive)) return;   // uniform; nothing of this row is here
     uint4 cosv[2], sinv[2];
     cosv[0] = cosv[1] = sinv[0] = sinv[1] = make_uint4(0, 0, 0, 0);
     if (rotate) {
@@ -479,8 +493,6 @@ __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a)
             sinv[h] = ld16(a.rot_sin + (int64_t)rp * (D / 2) + h * 32 + q * 8);
         }
     }
-    const int nblk = (max(pos, 0) + kMRows - 1) / kMRows;
-    const int nchunk = nblk > blk_first ? (nblk - blk_first + blk_step - 1) / blk_step : 0;
 
     // pieces kk and kk ^ 2 are half a head apart: the rotation needs no other lane
     bf16x8_t qf[4];
@@ -653,7 +665,7 @@ __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a)
             *reinterpret_cast<f32x4_t*>(dst + 4) = (f32x4_t){oacc[p][0][2], oacc[p][1][2], oacc[p][0][3], oacc[p][1][3]};
         }
     }
-    finish_states<D, G, NS, kAW>(a, lds, b, kvh, bh, split, wid, lane);
+    finish_states<D, G, NS, kAW>(a, lds, b, kvh, bh, split, wid, lane, filled);
 }
 
 // Second-launch form of the split merge (used when the arrival counters are unavailable or

@@ -104,7 +104,6 @@ __global__ __launch_bounds__(512) void qkv_attn_kernel(QkvAttnArgs qa) {
     const int J = gridDim.x / a.hkv;            // members per head = bs * nsplit
     const int b = jm / a.nsplit, split = jm - b * a.nsplit;
     const int bh = b * a.hkv + kvh;
-    const bool last_split = (split == a.nsplit - 1);
 
     // the epoch of this launch: one more than the word the last launch left (written through at its
     // end, so a plain - scalar - load across the kernel boundary sees it); nothing waits for it here
@@ -454,6 +453,7 @@ __global__ __launch_bounds__(512) void qkv_attn_kernel(QkvAttnArgs qa) {
 #endif
         const int seq_chunks = (max(pos, 0) + CR - 1) / CR;
         const int nchunk = seq_chunks > split ? (seq_chunks - split + a.nsplit - 1) / a.nsplit : 0;
+        const bool last_split = split == filled_splits(a.nsplit, seq_chunks) - 1;
 
         uint32_t qp[G][4];
 #pragma unroll
@@ -602,7 +602,7 @@ __global__ __launch_bounds__(512) void qkv_attn_kernel(QkvAttnArgs qa) {
         __hip_atomic_store(qa.sync + kQaEpoch, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // (threads past the attention waves take no part in the per-head work of the merge)
-    finish_states<D, G, NS, kAW>(a, lds, b, kvh, bh, split, attn_wave ? wid : 4096, lane);
+    finish_states<D, G, NS, kAW>(a, lds, b, kvh, bh, split, attn_wave ? wid : 4096, lane, a.nsplit);
     MV_QSTAMP(7);   // end (last arrivers: output written)
 }
 

@@ -244,6 +244,26 @@ def test_slots_that_do_not_count_may_hold_anything(mv, D, Hq, Hkv):
         assert torch.equal(vc.cpu().view(torch.int16)[keep], dirty["v_cache"].view(torch.int16)[keep])
 
 
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 1, 64), (4, 1, 64), (4, 1, 128), (7, 1, 128), (8, 1, 128)])
+def test_rows_that_fill_fewer_splits_than_there_are(mv, Hq, Hkv, D):
+    """Splits without a row's tokens leave at once, and the last one with some owns the new token: lengths around the edges
+    of a split's chunk (32 and 64 rows of heads of 128, 64 and 128 of heads of 64), mixed in one launch, against the oracle
+    and against the merge in a second launch, for which every split writes a partial."""
+    from micro_vllm_amd import _native as nv
+
+    case = make_case(12, Hq, Hkv, D, 256, [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 500], seed=D + Hq)
+    for splits in (2, 3, 8, 32):
+        got, _, (kc, vc), (kc_ref, vc_ref) = run_both(case, splits)
+        check_output(got, case, what=f"D={D} G={Hq // Hkv} splits={splits}")
+        assert torch.equal(kc.cpu(), kc_ref) and torch.equal(vc.cpu(), vc_ref)
+        try:
+            assert nv.lib().mv_paged_attn_tune(0, 0) == 0
+            assert torch.equal(run_both(case, splits)[0], got), splits
+        finally:
+            nv.lib().mv_paged_attn_tune(0, 1)
+        assert torch.equal(run_both(case, splits)[0], got), "the arrival counters are back at zero"
+
+
 @pytest.fixture
 def matrix_core_form(mv):
     """Force the matrix-core form of the kernel wherever it applies (D = 128, 4 or 8 query heads per
