@@ -906,17 +906,12 @@ static int launch_mfma(const GemmArgs& a, int grid, hipStream_t s) {
 static int mfma_strip_group(int m, int nt, int kt, bool free_reduce) {
     const int mb = (m + 15) / 16;
     const int most = 4;
-    if (const int forced = g_tune_sg;
-        forced == 1 || forced == 2 || forced == 4 || ((forced == 7 || forced == 3) && mb <= 2))
-        return forced;
+    if (const int forced = g_tune_sg; (forced >= 1 && forced <= 4) || (forced == 7 && mb <= 2)) return forced;
     // Seven strips per workgroup where that deals the strips out to the CUs exactly (Llama-3-8B
     // gate/up: 1792 strips = 7 x 256): in groups of four 448 units fall on 256 CUs as two rounds, the
     // second three quarters full, and every workgroup re-reads x for four strips instead of seven.
     if (mb <= 2 && nt % 7 == 0 && (nt / 7) % num_cus() == 0) return 7;
-    // Three or four row blocks of x: always the widest group - the x traffic out of L2 dominates
-    // otherwise (tools/sweep_mfma_gemv.py).
-    if (mb > 2) return most;
-    // One or two row blocks (5-32 rows).  A small model of the three costs, fitted to the Llama-3-8B
+    // A small model of the three costs, fitted to the Llama-3-8B
     // projections at 8, 16 and 32 rows (tools/bench_mfma_gemv.py, tools/bench_slabs.py): weights
     // stream at 6.45 MB/us over the CUs that have a unit, every unit re-reads its k-slice of x out of
     // L2 at about 12.9 MB/us, and a k-split pays a slab-reduction launch of 3.6 us (QKV at 32 rows:
@@ -926,6 +921,9 @@ static int mfma_strip_group(int m, int nt, int kt, bool free_reduce) {
     // then as many bytes as the weights; the 4096-wide O projection keeps single strips at both,
     // 9.1 against 11.2 us, its split costing more than its x.)
     // With a free slab reduction the same model decides with that term dropped.
+    // At 33-64 rows it picks the widest group wherever that fills the chip, because x is then most of what moves, and
+    // narrower ones for small projections (37 rows, 2560 x 2048 10.4 -> 8.4 us, 2048 x 2048 9.8 -> 8.0, 11264 x 2048 in
+    // threes 14.6 -> 13.5, 6144 x 4096 18.7 -> 16.1; 28672 x 4096 stays with fours, 54).
     const int cus = num_cus();
     int best = 1;
     double best_us = 1e30;
@@ -1067,8 +1065,8 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
             const int mb = (m + 15) / 16;
             if (mb == 1) rc = sg == 7 ? launch_mfma<1, 7>(a, grid, s) : sg == 3 ? launch_mfma<1, 3>(a, grid, s) : sg == 4 ? launch_mfma<1, 4>(a, grid, s) : sg == 2 ? launch_mfma<1, 2>(a, grid, s) : launch_mfma<1, 1>(a, grid, s);
             else if (mb == 2) rc = sg == 7 ? launch_mfma<2, 7>(a, grid, s) : sg == 3 ? launch_mfma<2, 3>(a, grid, s) : sg == 4 ? launch_mfma<2, 4>(a, grid, s) : sg == 2 ? launch_mfma<2, 2>(a, grid, s) : launch_mfma<2, 1>(a, grid, s);
-            else if (mb == 3) rc = sg == 4 ? launch_mfma<3, 4>(a, grid, s) : sg == 2 ? launch_mfma<3, 2>(a, grid, s) : launch_mfma<3, 1>(a, grid, s);
-            else rc = sg == 4 ? launch_mfma<4, 4>(a, grid, s) : sg == 2 ? launch_mfma<4, 2>(a, grid, s) : launch_mfma<4, 1>(a, grid, s);
+            else if (mb == 3) rc = sg == 4 ? launch_mfma<3, 4>(a, grid, s) : sg == 3 ? launch_mfma<3, 3>(a, grid, s) : sg == 2 ? launch_mfma<3, 2>(a, grid, s) : launch_mfma<3, 1>(a, grid, s);
+            else rc = sg == 4 ? launch_mfma<4, 4>(a, grid, s) : sg == 3 ? launch_mfma<4, 3>(a, grid, s) : sg == 2 ? launch_mfma<4, 2>(a, grid, s) : launch_mfma<4, 1>(a, grid, s);
         }
     }
     if (rc != MV_OK || slabs_only) return rc;

@@ -236,3 +236,16 @@ def test_wgemm_postnorm_is_bit_identical_to_separate_kernels(mv, m, n, k):
     y1, n1 = new(), new()
     wgemm_postnorm(x, sw, y1, lw, eps, n1)
     assert torch.equal(y1, y2) and torch.equal(n1, n2), f"norm of projection m={m}"
+
+
+@pytest.mark.parametrize("m", [33, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(2560, 2048), (11264, 2048), (11280, 2048), (6144, 4096)])
+def test_wgemm_widths_at_33_to_64_rows(mv, m, n, k):
+    """Three and four blocks of rows take one to four strips a workgroup by the sizes (11264 x 2048: three, and 11280 leaves
+    a group of three unfilled).  fp32 sums of exact products: k additions of at most 2^-24 of the partial sums each."""
+    from micro_vllm_amd.kernel.linear import StreamedWeight, wgemm
+
+    x, w, _ = _mk(m, n, k, seed=m + n)
+    got = wgemm(x.to(DEV), StreamedWeight.from_linear(w.to(DEV)), torch.empty(m, n, dtype=torch.float32, device=DEV))
+    xd, wd = x.double(), w.double()
+    assert (((got.cpu().double() - xd @ wd.t()).abs()) <= k * 2.0 ** -24 * (xd.abs() @ wd.abs().t())).all()
