@@ -348,6 +348,23 @@ int mv_store_kv(const void* key, const void* value, int64_t kv_stride_t, void* k
                 void* v_cache, const int32_t* slot_mapping, int tokens, int heads, int d,
                 int page, int num_pages, mv_stream_t stream);
 
+/* ------------------------------------------------------------- prefill of a whole stack */
+
+/* All layers of a Llama-shaped prefill on one GPU in one call (core/layer/model_prefill.py:36-59 per layer): `rows`
+ * sequences of `seq` tokens, h [rows * seq, hidden] bf16 in place.  tensors: per layer nine device pointers - ln_1 weight,
+ * QKV tiles, QKV bias or NULL, O tiles, ln_2 weight, gate/up tiles (interleaved, mv_interleave_rows8), down tiles, key
+ * cache, value cache; eps: per layer the two norms' epsilons.  Scratch, 16-byte aligned: normed, resid [T, hidden],
+ * qkv [T, (Hq + 2 Hkv) D], attn [T, Hq D], act [T, inter], all bf16, and proj, T * hidden floats.  workspace: of
+ * mv_llama_prefill_workspace_bytes, as for mv_gemm_prefill_ws (zero-filled when it was allocated).  Results are those of
+ * the layer's ops called one by one, bit for bit. */
+size_t mv_llama_prefill_workspace_bytes(int tokens, int hidden, int inter, int hq, int hkv, int d);
+int mv_llama_prefill_layers(const void* const* tensors, const float* eps, int n_layers, int rows, int seq, int hidden,
+                            int inter, int hq, int hkv, int d, const void* rot_cos, const void* rot_sin,
+                            int rot_max_pos, const int32_t* cache_seqlens, const int32_t* block_table, int bt_stride,
+                            int page, int num_pages, void* h, void* normed, void* qkv, void* attn, void* proj,
+                            void* resid, void* act, float scale, void* workspace, size_t workspace_bytes,
+                            mv_stream_t stream);
+
 /* ------------------------------------------------------------- sampling */
 
 /* ids[r] = argmax_c logits[r, c] over bf16 logits [rows, n] (row stride ld), lowest index on

@@ -23,6 +23,7 @@ SOURCES = [
     "kv_store.hip",
     "attn_prefill.hip",
     "gemm_prefill.hip",
+    "llama_prefill.hip",
     "sampler.hip",
     "allreduce.hip",
     "qkv_attn.hip",

@@ -8,11 +8,13 @@ gate/up projection with SwiGLU in its epilogue -> down projection (+residual) ->
 All projections run on the matrix cores over the same weight image the decode runner streams,
 so both runners share one copy of the weights.
 """
+import ctypes
 import logging
 
 import torch
 
 from .. import parallel_config as pc
+from ... import _native as nv
 from ..prefill_attention import paged_attn_prefill_rows, rope_store_prefill
 from ...kernel.linear import add_, embedding, gemm_prefill, wgemm
 from ...kernel.rmsnorm_add import rmsnorm, rmsnorm_residual_fused
@@ -62,6 +64,48 @@ class ModelPrefillRunner(ModelGraphRunner):
             return self._fast_mlp(normed, block.mlp._gu, block.mlp._d, residual=residual)
         return add_(pc.all_reduce(self._fast_mlp(normed, block.mlp._gu, block.mlp._d)), residual)
 
+    def _prefill_stack(self, h, B, S, cache_manager, cache_lens, block_table):
+        """Every layer on hidden rows h [B*S, hid], in place, from one native call (mv_llama_prefill_layers): what
+        `_prefill_layer` gives layer by layer, bit for bit."""
+        T, dev, L = B * S, h.device, nv.lib()
+        hid, hq, hkv, d = self.hidden_dim, self.num_heads, self.kv_num_heads, self.head_size
+        blocks = self.model.transformer.h
+        tensors, eps = [], []
+        for li in range(self.num_layers):
+            b = blocks[li]
+            k_cache, v_cache = cache_manager.get(li)
+            assert k_cache.shape[2:] == (hkv, d) and k_cache.shape == v_cache.shape, "cache heads/dim mismatch"
+            assert k_cache.is_contiguous() and v_cache.is_contiguous()
+            w = (b.attn._qkv_w, b.attn._o, b.mlp._gu, b.mlp._d)
+            assert (w[0].n, w[0].k, w[1].n, w[1].k) == ((hq + 2 * hkv) * d, hid, hid, hq * d)
+            assert (w[2].n, w[2].k, w[3].n, w[3].k) == (2 * w[3].k, hid, hid, w[2].out_features) and w[2].swiglu
+            for ln in (b.ln_1.weight, b.ln_2.weight):
+                assert ln.dtype == torch.bfloat16 and ln.numel() == hid and ln.is_contiguous()
+            bias = b.attn._qkv_b
+            assert bias is None or (bias.dtype == torch.bfloat16 and bias.numel() == w[0].n and bias.is_contiguous())
+            tensors += [b.ln_1.weight.data_ptr(), w[0].tiles.data_ptr(), nv.ptr(bias), w[1].tiles.data_ptr(),
+                        b.ln_2.weight.data_ptr(), w[2].tiles.data_ptr(), w[3].tiles.data_ptr(), k_cache.data_ptr(),
+                        v_cache.data_ptr()]
+            eps += [float(b.ln_1.eps), float(b.ln_2.eps)]
+        if not tensors:
+            return h
+        NB, page = k_cache.shape[:2]
+        inter = blocks[0].mlp._d.k
+        assert all(blocks[li].mlp._d.k == inter for li in range(self.num_layers))
+        cos, sin = self.attention._cos_pool, self.attention._sin_pool
+        assert block_table.dtype == torch.int32 and block_table.stride(1) == 1 and cache_lens.dtype == torch.int32
+        ws = nv.stream_workspace("gemm_prefill", dev, L.mv_llama_prefill_workspace_bytes(T, hid, inter, hq, hkv, d))
+        rows = lambda n: torch.empty(T, n, dtype=torch.bfloat16, device=dev)   # noqa: E731
+        normed, resid, proj = rows(hid), rows(hid), torch.empty(T, hid, dtype=torch.float32, device=dev)
+        qkv, attn, act = rows((hq + 2 * hkv) * d), rows(hq * d), rows(inter)
+        nv.check("mv_llama_prefill_layers", L.mv_llama_prefill_layers(
+            (ctypes.c_void_p * len(tensors))(*tensors), (ctypes.c_float * len(eps))(*eps), self.num_layers, B, S, hid, inter,
+            hq, hkv, d, cos.data_ptr(), sin.data_ptr(), cos.shape[0], cache_lens.data_ptr(), block_table.data_ptr(),
+            block_table.stride(0), page, NB, h.data_ptr(), normed.data_ptr(), qkv.data_ptr(), attn.data_ptr(),
+            proj.data_ptr(), resid.data_ptr(), act.data_ptr(), float(d) ** -0.5,
+            ws.data_ptr() if ws is not None else None, ws.numel() * 4 if ws is not None else 0, nv.stream_ptr()))
+        return h
+
     def forward(self, input_ids: torch.Tensor, cache_manager, batch_size: int,
                 last_token_only: bool = False, last_token_index=None) -> torch.Tensor:
         """input_ids [B,S] (right-padded to a common S by the caller).  Returns logits [B,S,V], or
@@ -81,7 +125,10 @@ class ModelPrefillRunner(ModelGraphRunner):
         cache_lens = cache_manager._cache_seqlens_buffer[:batch_size].zero_()
         block_table = cache_manager._block_table_buffer[:batch_size]
 
-        for layer_idx in range(self.num_layers):
+        whole = self.world_size == 1 and self.fused     # (several ranks reduce between the launches of a layer)
+        if whole:
+            h = self._prefill_stack(h, B, S, cache_manager, cache_lens, block_table)
+        for layer_idx in range(0 if whole else self.num_layers):
             h = self._prefill_layer(h, layer_idx, B, S, cache_manager, cache_lens, block_table)
 
         if last_token_index is not None:

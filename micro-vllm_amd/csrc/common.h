@@ -117,5 +117,30 @@ int ensure_dynamic_lds(const void* kernel, size_t lds, LdsOptIn& done);
 // wgemm.hip: adds k-slices partial[ks][m][n] (fp32) in order and applies the projection epilogue
 int launch_wgemm_finalize(float* partial, int ksplit, int m, int n, int flags, const uint16_t* bias,
                           const uint16_t* residual, int64_t ld_res, void* y, int64_t ldy, hipStream_t s);
+// What may follow a projection: y = bf16(sum) + bias + residual and out = rmsnorm(y) * ln_w, the variance that of the rounded
+// or the unrounded y.  `done` says that the projection's own reduction did it, in place of the call's own epilogue.
+struct PostNorm {
+    const void* residual;
+    void* y;
+    const void* ln_w;
+    float eps;
+    void* out;
+    int64_t ld;       // of residual, y and out
+    int var_from_rounded;
+    float* slab;      // m * n floats of scratch
+    bool done;
+};
+// wgemm.hip: the same followed by the norm
+int launch_wgemm_finalize_norm(float* partial, int ksplit, int m, int n, const void* bias, PostNorm* norm, hipStream_t s);
+bool wgemm_finalize_norm_takes(int n);
+// wgemm.hip: a projection of up to 64 rows whose sums are those of `ks` slices of k added in order
+bool wgemm_ordered_takes(int m, int kt, int ks);
+int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
+                         int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int ks, int flags, PostNorm* norm,
+                         hipStream_t s);
+// gemm_prefill.hip: mv_gemm_prefill_ws, whose reduction of k-slices (where it has one) also does `norm`
+int gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
+                     int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int flags, void* workspace,
+                     size_t workspace_bytes, PostNorm* norm, mv_stream_t stream);
 
 }  // namespace mv

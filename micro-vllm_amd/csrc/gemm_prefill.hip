@@ -1014,7 +1014,14 @@ extern "C" int mv_gemm_prefill_ws(const void* x, int64_t ldx, const void* w_tile
                                   const void* residual, int64_t ld_res, void* y, int64_t ldy, int m,
                                   int n, int k, int flags, void* workspace, size_t workspace_bytes,
                                   mv_stream_t stream) {
-    using namespace mv;
+    return mv::gemm_prefill_run(x, ldx, w_tiles, bias, residual, ld_res, y, ldy, m, n, k, flags, workspace, workspace_bytes,
+                                nullptr, stream);
+}
+
+int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
+                         int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int flags, void* workspace,
+                         size_t workspace_bytes, PostNorm* norm, mv_stream_t stream) {
+    if (norm) norm->done = false;
     if (m == 0) return MV_OK;
     if (!x || !w_tiles || !y || m < 0 || n <= 0 || k <= 0) return MV_ERR_INVALID_ARG;
     if ((n % 16) != 0 || (k % 64) != 0) return MV_ERR_UNSUPPORTED;
@@ -1065,6 +1072,18 @@ extern "C" int mv_gemm_prefill_ws(const void* x, int64_t ldx, const void* w_tile
             wide = false;
         }
     }
+    // Up to 64 rows a tile of 128 is mostly padding, and its slices are written out and added up by a second launch.  The
+    // single-token projections' kernel walks the same slices one to a wave and adds them in the workgroup, same sums in
+    // the same order (the rule and what it measured: wgemm_ordered_takes).
+    if (!wide && wgemm_ordered_takes(m, a.kt, a.ksplit))
+        return launch_wgemm_ordered(x, ldx, w_tiles, bias, residual, ld_res, y, ldy, m, n, k, a.ksplit, flags, norm,
+                                    (hipStream_t)stream);
+    auto reduce = [&] {
+        if (norm && !sw && !of32 && wgemm_finalize_norm_takes(n))
+            return launch_wgemm_finalize_norm(a.partial, a.ksplit, m, n, bias, norm, (hipStream_t)stream);
+        return launch_wgemm_finalize(a.partial, a.ksplit, m, n, flags, a.bias, a.residual, ld_res, y, ldy,
+                                     (hipStream_t)stream);
+    };
     a.ktps = a.kt / a.ksplit;
     if (wide) {
         static LdsOptIn lds_done[3];
@@ -1102,14 +1121,12 @@ extern "C" int mv_gemm_prefill_ws(const void* x, int64_t ldx, const void* w_tile
             hipLaunchKernelGGL((gemm_prefill_wide_kernel<4, 4>), dim3((unsigned)wgrid), dim3(512), kWLds, (hipStream_t)stream, a);
         rc = check_launch();
         if (rc != MV_OK || a.ksplit == 1) return rc;
-        return launch_wgemm_finalize(a.partial, a.ksplit, m, n, flags, a.bias, a.residual, ld_res, y, ldy,
-                                     (hipStream_t)stream);
+        return reduce();
     }
     const long grid = 8L * a.nb_per_xcd * a.mblocks * a.ksplit;
     if (grid > 0x7fffffffL) return MV_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(gemm_prefill_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
     int rc = check_launch();
     if (rc != MV_OK || a.ksplit == 1) return rc;
-    return launch_wgemm_finalize(a.partial, a.ksplit, m, n, flags, a.bias, a.residual, ld_res, y, ldy,
-                                 (hipStream_t)stream);
+    return reduce();
 }

@@ -439,9 +439,17 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 // A wave loads the x fragments of a k-tile once and uses them against the SG weight tiles of
 // that k-tile: x comes out of L2 for every workgroup, so without the sharing the x requests
 // (MB per weight tile) outnumber the weight requests and the L2 path, not HBM, sets the pace.
-template <int MB, int SG>
+//
+// KS = 0: the waves interleave over the unit's k-tiles.  KS = 4, 8, 16: k in KS whole slices, each added up by one wave
+// and the slices in order - the sums of a prefill projection cut into KS slices (gemm_prefill.hip), bit for bit, without
+// its slabs and their reduction launch.  With four slices two halves of the workgroup take SG strips each; with sixteen a
+// wave takes two slices one after the other.
+template <int MB, int SG, int KS = 0>
 __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
     constexpr int U = (SG + MB <= 6) ? 2 : 1;  // k-tiles per stage (register budget)
+    constexpr int kStep = KS ? 1 : kGW;        // k-tiles between a wave's tiles
+    constexpr int kHalves = KS == 4 ? 2 : 1, kTurns = KS == 16 ? 2 : 1;
+    constexpr int kSlots = KS == 0 || KS == 4 ? kGW : KS;   // accumulator sets that meet in LDS
     // cross-wave reduction buffer [kGW][SG][MB][64 lanes][4]: 8 KiB per (strip, row block) pair,
     // up to 128 KiB (dynamic: past the 64 KiB a static array may have)
     extern __shared__ __attribute__((aligned(16))) float red[];
@@ -456,16 +464,21 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
     for (int b = 0; b < MB; ++b) xrow[b] = a.x + (int64_t)min(b * 16 + r, a.m - 1) * a.ldx + q * 8;
 
     for (int u = blockIdx.x; u < a.nunits; u += gridDim.x) {
-        const int g = u / a.ksplit, ks = u - g * a.ksplit;
-        const int kt0 = ks * a.ktps;
+        const int g = KS ? u : u / a.ksplit, ks = KS ? 0 : u - g * a.ksplit;
+#pragma unroll
+        for (int turn = 0; turn < kTurns; ++turn) {
+        const int slice = KS == 4 ? wid & 3 : wid + turn * kGW;   // (KS > 0)
+        const int slot = KS == 16 ? slice : wid;
+        const int strip0 = (g * kHalves + (KS == 4 ? wid >> 2 : 0)) * SG;
+        const int kt0 = KS ? slice * a.ktps : ks * a.ktps;
         const int kt1 = min(a.kt, kt0 + a.ktps);
-        const int ntile = (kt1 - kt0 - wid + kGW - 1) / kGW;
+        const int ntile = KS ? kt1 - kt0 : (kt1 - kt0 - wid + kGW - 1) / kGW;
         const int last = max(ntile - 1, 0);
-        const int ktw = kt0 + (ntile > 0 ? wid : 0);  // a wave without tiles still loads (clamped)
+        const int ktw = KS ? kt0 : kt0 + (ntile > 0 ? wid : 0);  // a wave without tiles still loads (clamped)
         const uint4* wbase[SG];
 #pragma unroll
         for (int sI = 0; sI < SG; ++sI)
-            wbase[sI] = a.w + ((int64_t)min(g * SG + sI, a.nt - 1) * a.kt + ktw) * 64 + lane;
+            wbase[sI] = a.w + ((int64_t)min(strip0 + sI, a.nt - 1) * a.kt + ktw) * 64 + lane;
 
         f32x4_t acc[SG][MB];
 #pragma unroll
@@ -479,8 +492,8 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
             for (int i = 0; i < U; ++i) {
                 const int t = min(c * U + i, last);
 #pragma unroll
-                for (int sI = 0; sI < SG; ++sI) wb[i][sI] = ld16_nt(wbase[sI] + (int64_t)t * (kGW * 64));
-                const int kcol = (ktw + t * kGW) * 32;
+                for (int sI = 0; sI < SG; ++sI) wb[i][sI] = ld16_nt(wbase[sI] + (int64_t)t * (kStep * 64));
+                const int kcol = (ktw + t * kStep) * 32;
 #pragma unroll
                 // (with these requests removed the four Llama-3-8B projections at M = 32 take 90 us
                 // instead of 104: the x path costs about 13 %)
@@ -539,20 +552,23 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
         for (int sI = 0; sI < SG; ++sI)
 #pragma unroll
             for (int b = 0; b < MB; ++b)
-                *reinterpret_cast<f32x4_t*>(&red[(((wid * SG + sI) * MB + b) * 64 + lane) * 4]) = acc[sI][b];
+                *reinterpret_cast<f32x4_t*>(&red[(((slot * SG + sI) * MB + b) * 64 + lane) * 4]) = acc[sI][b];
+        }
         __syncthreads();
         // one wave per (strip, row block) pair; more pairs than waves take a second turn
-        for (int sb = wid; sb < MB * SG; sb += kGW) {
+        for (int sb = wid; sb < MB * SG * kHalves; sb += kGW) {
             const int l = lane;
-            const int sI = sb / MB, b = sb - sI * MB;
+            const int strip = sb / MB, b = sb - strip * MB;
+            const int half = strip / SG, sI = strip - half * SG;
             const int rr = l & 15, qq = l >> 4;
             const int m = b * 16 + rr;
-            const int nt = g * SG + sI;
+            const int nt = g * kHalves * SG + strip;
             auto sum_at = [&](int ll) {
                 f32x4_t s = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int w8 = 0; w8 < kGW; ++w8)
-                    s += *reinterpret_cast<const f32x4_t*>(&red[(((w8 * SG + sI) * MB + b) * 64 + ll) * 4]);
+                for (int w8 = 0; w8 < kSlots / kHalves; ++w8)
+                    s += *reinterpret_cast<const f32x4_t*>(
+                        &red[((((half * 4 + w8) * SG + sI) * MB + b) * 64 + ll) * 4]);
                 return s;
             };
             if (m < a.m && nt < a.nt) {
@@ -940,6 +956,118 @@ static int mfma_strip_group(int m, int nt, int kt, bool free_reduce) {
         }
     }
     return best;
+}
+
+// Strips per wave of the ordered form: the model above, the workgroup's strips being SG or, with four slices, 2 SG
+static int ordered_strip_group(int m, int nt, int kt, int ks) {
+    const int mb = (m + 15) / 16, halves = ks == 4 ? 2 : 1;
+    const int cus = num_cus();
+    int best = 1;
+    double best_us = 1e30;
+    for (int sg = 4; sg >= 1; sg /= 2) {
+        if (sg * mb > (ks == 16 ? 8 : 16) || (sg == 4 && ks != 8)) continue;   // 128 KiB of LDS; the instances there are
+        const long units = (nt + sg * halves - 1) / (sg * halves);
+        const double fill = (double)units / (double)(((units + cus - 1) / cus) * cus);
+        const double us = (double)nt * kt * 1024e-6 / (6.45 * fill) + (double)units * halves * m * kt * 64e-6 / 12.9;
+        if (us < best_us) {
+            best_us = us;
+            best = sg;
+        }
+    }
+    return best;
+}
+
+template <int MB, int SG, int KS>
+static int launch_ordered(const GemmArgs& a, int grid, hipStream_t s) {
+    constexpr size_t lds = (size_t)(KS == 16 ? 16 : kGW) * SG * MB * 64 * 4 * sizeof(float);
+    static_assert(lds <= 128 * 1024, "reduction buffer fits LDS");
+    static LdsOptIn opted;  // per instantiation
+    if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<MB, SG, KS>, lds, opted)) return rc;
+    hipLaunchKernelGGL((wgemm_mfma_kernel<MB, SG, KS>), dim3(grid), dim3(kGT), lds, s, a);
+    return check_launch();
+}
+template <int MB>
+static int launch_ordered_mb(const GemmArgs& a, int sg, int ks, int grid, hipStream_t s) {
+    switch (ks * 8 + sg) {
+        case 4 * 8 + 1: return launch_ordered<MB, 1, 4>(a, grid, s);
+        case 4 * 8 + 2: return launch_ordered<MB, 2, 4>(a, grid, s);
+        case 8 * 8 + 1: return launch_ordered<MB, 1, 8>(a, grid, s);
+        case 8 * 8 + 2: return launch_ordered<MB, 2, 8>(a, grid, s);
+        case 8 * 8 + 4: return launch_ordered<MB, 4, 8>(a, grid, s);
+        case 16 * 8 + 1: return launch_ordered<MB, 1, 16>(a, grid, s);
+        case 16 * 8 + 2: return launch_ordered<MB, 2, 16>(a, grid, s);
+        default: return MV_ERR_UNSUPPORTED;
+    }
+}
+
+// One block of rows (up to 16), or few k-tiles times blocks: a wave walks its slice alone, and past that its chain of loads
+// is longer than the sliced tiles' two launches.  Measured at 37 rows (n x k, us, sliced tiles -> here): 2560 x 2048
+// 12.5 -> 9.0, 11264 x 2048 19.9 -> 17.8, 6144 x 4096 20.5 -> 18.9, 8192 x 1024 13.3 -> 8.9, but 1280 x 8192 16.5 -> 24.8
+// and 4096 x 14336 33.8 -> 46.5; at 64 rows 2560 x 2048 14.2 -> 12.5 and 4096 x 4096 19.6 -> 23.7; at 5 rows all are
+// faster here, 17.1 -> 9.4 (2048 x 5632) to 31.7 -> 21.9 (4096 x 14336).
+bool wgemm_ordered_takes(int m, int kt, int ks) {
+    const int blocks = (m + 15) / 16;
+    return (ks == 4 || ks == 8 || ks == 16) && blocks <= 4 && (blocks == 1 || blocks * kt <= 384);
+}
+
+// x [m, k] . W^T with the sums of `ks` slices of k added in order, epilogue as mv_gemm_prefill_ws, or the norm's.
+// Arguments as the callers have checked them.
+int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
+                         int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int ks, int flags, PostNorm* norm,
+                         hipStream_t s) {
+    if (norm && ((flags & (MV_GEMM_SWIGLU | MV_GEMM_OUT_F32)) || !wgemm_finalize_norm_takes(n))) norm = nullptr;
+    GemmArgs a = {};
+    a.x = (const uint16_t*)x;
+    a.ldx = ldx;
+    a.w = (const uint4*)w_tiles;
+    a.bias = (const uint16_t*)bias;
+    a.residual = (const uint16_t*)residual;
+    a.ld_res = ld_res;
+    a.y = y;
+    a.ldy = ldy;
+    a.m = m;
+    a.n = n;
+    a.k = k;
+    a.nt = n / 16;
+    a.kt = k / 32;
+    a.flags = flags;
+    a.ksplit = 1;
+    a.ktps = a.kt / ks;
+    a.partial = norm ? norm->slab : nullptr;
+    const int sg = ordered_strip_group(m, a.nt, a.kt, ks), halves = ks == 4 ? 2 : 1;
+    a.nunits = (a.nt + sg * halves - 1) / (sg * halves);
+    const int mb = (m + 15) / 16;
+    // a second workgroup per CU where its reduction buffer fits beside the first
+    const int per_cu = (ks == 16 ? 16 : kGW) * sg * mb <= 64 ? 2 : 1;
+    const int grid = a.nunits < num_cus() * per_cu ? a.nunits : num_cus() * per_cu;
+    const int rc = mb == 1 ? launch_ordered_mb<1>(a, sg, ks, grid, s) : mb == 2 ? launch_ordered_mb<2>(a, sg, ks, grid, s)
+                   : mb == 3 ? launch_ordered_mb<3>(a, sg, ks, grid, s) : launch_ordered_mb<4>(a, sg, ks, grid, s);
+    if (rc != MV_OK || !norm) return rc;
+    return launch_wgemm_finalize_norm(norm->slab, 1, m, n, bias, norm, s);
+}
+
+bool wgemm_finalize_norm_takes(int n) { return n % 8 == 0 && n <= 8 * 256 * kPostChunks; }
+
+// Rows and the norm's weight 16-byte aligned (the callers' checks)
+int launch_wgemm_finalize_norm(float* partial, int ksplit, int m, int n, const void* bias, PostNorm* norm, hipStream_t s) {
+    GemmArgs a = {};
+    a.partial = partial;
+    a.ksplit = ksplit;
+    a.m = m;
+    a.n = n;
+    a.bias = (const uint16_t*)bias;
+    a.residual = (const uint16_t*)norm->residual;
+    a.ld_res = norm->ld;
+    a.y = norm->y;
+    a.ldy = norm->ld;
+    a.post_ln_w = (const uint16_t*)norm->ln_w;
+    a.post_out = (uint16_t*)norm->out;
+    a.ld_post = norm->ld;
+    a.post_eps = norm->eps;
+    a.post_var_from_rounded = norm->var_from_rounded;
+    hipLaunchKernelGGL(wgemm_finalize_norm_kernel, dim3(m), dim3(256), 0, s, a);
+    norm->done = true;
+    return check_launch();
 }
 
 static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_add_r,

@@ -404,3 +404,43 @@ def test_gemm_prefill_k_slices(mv, m, n, k, mode):
         want = want.to(torch.bfloat16)
     assert float((ulp_diff(split, want) == 0).float().mean()) > 0.98
     assert float((ulp_diff(split, whole) == 0).float().mean()) > 0.98
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 37, 48, 49, 64])
+@pytest.mark.parametrize("n,k,mode", [(16, 2048, "plain"), (256, 8192, "f32"), (1280, 8192, "bias"),
+                                      (2048, 5632, "residual"), (4096, 4096, "plain"), (11264, 2048, "swiglu"),
+                                      (6160, 4096, "residual")])
+def test_few_rows_add_the_slices_in_order(mv, m, n, k, mode):
+    """Up to 16 rows, and with a short k up to 64, the k-slices are added within a workgroup.  The result is that of the slices' own products added in
+    order, bit for bit (4, 8 and 16 slices, one to four blocks of rows, n that leaves a part of a workgroup's columns
+    unused)."""
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.linear import StreamedWeight, gemm_prefill
+
+    L = nv.lib()
+    slices = (L.mv_gemm_prefill_workspace_bytes(m, n, k) - 4096) // (4 * m * n)
+    assert slices in (4, 8, 16), "meant to be cut"
+    x, w, g = _mk(m, n, k, seed=m + n + k, scale=0.03)
+    wd = w.to(DEV)
+    sw = StreamedWeight.from_up_gate(wd[:n // 2], wd[n // 2:]) if mode == "swiglu" else StreamedWeight.from_linear(wd)
+    ncols, dt = sw.out_features, torch.float32 if mode == "f32" else torch.bfloat16
+    bias = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if mode == "bias" else None
+    res = torch.randn(m, n, generator=g).to(torch.bfloat16).to(DEV) if mode == "residual" else None
+    xd = x.to(DEV)
+    got = gemm_prefill(xd, sw, torch.full((m, ncols), float("nan"), dtype=dt, device=DEV), bias=bias, residual=res,
+                       swiglu=mode == "swiglu")
+    total = torch.zeros(m, n, device=DEV)
+    kk = k // slices
+    for i in range(slices):
+        xs, part = xd[:, i * kk:(i + 1) * kk].contiguous(), torch.empty(m, n, device=DEV)
+        ws = StreamedWeight.from_linear(wd[:, i * kk:(i + 1) * kk].contiguous())
+        nv.check("mv_gemm_prefill", L.mv_gemm_prefill(xs.data_ptr(), kk, ws.tiles.data_ptr(), None, None, 0, part.data_ptr(),
+                                                      n, m, n, kk, nv.MV_GEMM_OUT_F32, nv.stream_ptr()))
+        total += part
+    want = total if mode == "f32" else total.to(torch.bfloat16)
+    if mode == "swiglu":   # (the activation's own rounding: one unit in the last place)
+        assert_close_bf16(got, swiglu_ref(want.cpu()), atol=1e-6, rtol=2 ** -7, what="swiglu of the slices' sum")
+        return
+    for addend in (bias, res):
+        want = want if addend is None else (want.float() + addend.float()).to(torch.bfloat16)
+    assert torch.equal(got, want)

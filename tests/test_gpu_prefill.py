@@ -350,3 +350,30 @@ def test_tokens_past_the_block_table_width_touch_no_other_sequence(mv):
     want = flash_attn_with_kvcache_ref(q[1:], kc0, vc0, k[1:], k[1:], None, None, starts[1:], bt[1:], causal=True,
                                        p_bf16=True)
     assert_close_bf16(out[1:].cpu(), want, atol=4e-3, rtol=2 ** -6, what="well-formed row")
+
+
+@pytest.mark.parametrize("shape,bias", [("tiny-gqa", True), ("tiny-gqa7", False), ("wide", True)])
+@pytest.mark.parametrize("B,S", [(1, 1), (1, 5), (3, 7), (1, 64), (4, 16), (1, 65), (2, 33), (2, 150)])
+def test_stack_in_one_call_equals_layer_by_layer(mv, shape, bias, B, S, monkeypatch):
+    """mv_llama_prefill_layers against the same layers issued one op at a time: equal bit for bit, where the projections
+    are whole (hidden 256 or less) and where they are cut into slices of k whose reduction norms the rows (wide)."""
+    import dataclasses
+
+    from micro_vllm_amd.models import SHAPES
+
+    if shape == "wide":
+        monkeypatch.setitem(SHAPES, shape, dataclasses.replace(SHAPES["tiny-d128"], hidden_size=1024, ffn_hidden_size=2816))
+    cfg, _, prefill, mgr, _, _ = _build(mv, shape, qkv_bias=bias)
+    for b in range(B):
+        mgr.alloc(b, S)
+    bt, _ = mgr.cache_batch_data(list(range(B)), [S] * B)
+    lens = torch.zeros(B, dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(B * 100 + S)
+    h0 = torch.randn(B * S, cfg.hidden_size, generator=g).to(torch.bfloat16).to(DEV)
+    want = h0
+    for li in range(cfg.num_hidden_layers):
+        want = prefill._prefill_layer(want, li, B, S, mgr, lens, bt)
+    k_want, v_want = mgr._k_store.clone(), mgr._v_store.clone()
+    mgr._k_store.zero_(), mgr._v_store.zero_()
+    got = prefill._prefill_stack(h0.clone(), B, S, mgr, lens, bt)
+    assert torch.equal(got, want) and torch.equal(mgr._k_store, k_want) and torch.equal(mgr._v_store, v_want)
