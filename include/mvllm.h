@@ -588,7 +588,8 @@ int mv_qk_rotary_store(float* qk, int64_t ld, const float* q_bias, const float* 
  * is one more term of the softmax's denominator, unscaled, with no value.  slopes NULL: no distance penalty.
  * part != NULL with splits >= 1 (fp32 [tokens * heads * splits * (dv + 2)]): the tokens the tiled kernel does not take
  * run one workgroup per (token, key/value head, up to eight of its query heads, split of the keys) - every key and value
- * is read once for those heads - and, with splits > 1, a second launch merges the splits' pieces.
+ * is read once for those heads - and, with splits > 1, a second launch merges the splits' pieces.  Head shapes the tiled
+ * kernel is built for take a form of this on the matrix cores, in fp32 too, that may use fewer splits than it is given.
  * short_tokens: how many of the step's tokens lie in rows of up to max_len tokens (-1: not known); 0 lets a step whose
  * rows all went to the tiled kernel skip the launch of the per-token form.  gate != NULL (fp32 [tokens, heads * dv]):
  * out is multiplied by sigmoid(gate) before it is rounded.  chunked != 0: a token sees its own chunk of `window` positions

@@ -500,8 +500,11 @@ class RaggedRunner:
         kc, vc = cache.k_caches[li], cache.v_caches[li]
         ops.qk_unitnorm_store(qkv, kc, vc, step, H, G, d, dv, eps)
         a = self._actbuf(T, H * dv)
-        ops.window_attn(qkv, kc, vc, a, step, w["slopes"], H, G, d, dv, float(L["scale"]), int(L["mask"]["size"]),
-                        tiled=self.tiled_attn)
+        window = int(L["mask"]["size"])
+        splits = ops.window_attn_splits(T, H, G, window) if self.grouped_attn else 0
+        part = self._f32buf(1, T * H * splits * (dv + 2)) if splits else None
+        ops.window_attn(qkv, kc, vc, a, step, w["slopes"], H, G, d, dv, float(L["scale"]), window, tiled=self.tiled_attn,
+                        part=part, splits=splits)
         left = w["left_o"](a, self._f32buf(T, self.width))
 
         Hr, dr, dvr, rot = int(R["heads"]), int(R["dim"]), int(R["vdim"]), int(R["rot"]["dims"])

@@ -1356,28 +1356,351 @@ __global__ __launch_bounds__(256) void window_attn_group_kernel(const float* q, 
     }
 }
 
-// one wave per (token, head): the splits' pieces and the sink become the output row
+// A single token's attention is a chain of trips to memory (token -> page table -> keys and values) and little else, so the
+// head shapes of the tiled kernel below have a form of their own for it.  One workgroup of NW waves per (token, key/value
+// head, group of up to HEADS of its query heads, split of the keys); a wave takes 16-key tiles - those of the kept first
+// positions, then the window's - in steps of NW * splits and requests the whole tile, keys and values, at once.
+//   q.k   bf16 keys: v_mfma_f32_16x16x32_bf16 with q split exactly into three bf16 numbers, a column each: column h + 4 s is
+//         part s of head h, and two rotations within a row of lanes add the parts.  fp32 keys: v_mfma_f32_16x16x4_f32.  Either
+//         way lane l ends with the scores of keys 4 (l / 16) .. + 3 for head l % 4.
+//   P.V   v_mfma_f32_4x4x1_f32: the lanes that hold those four weights read the same four value rows, 16 lanes a row, so
+//         weight j is the first operand where it lies and each element of value row j the second.  (HEADS = 1: plain products,
+//         the instruction's other three rows would be idle.)
+// The waves' partial softmaxes meet in LDS.  A token whose tiles are one to a wave is finished by its first split, and the
+// other splits leave at once; else a split leaves (max, sum, weighted values) in `part` for window_attn_merge_kernel.
+//
+// Measured (us per call, 8 heads on 2 key/value heads, d = dv = 128, window 1024; kernel above with its 64-key tiles, five
+// splits and their merge -> here): one token bf16 at 45 keys 19.0 -> 7.8, 300 21.7 -> 11.4, 1100 23.2 -> 20.3; fp32 19.0 -> 8.0,
+// 22.6 -> 14.1, 26.9 -> 24.0; 64 tokens bf16 21.4 -> 8.1, 26.7 -> 12.4, 51.2 -> 27.9; a prompt of 333 in fp32 at 300 58.8 -> 40.8.
+// 16 heads of 64 with keys of their own, one token 10.4 -> 4.5, 11.5 -> 6.8, 14.5 -> 12.6.
+struct TileRun {
+    int lo, kept, nk, n;      // n tiles: nk of the kept positions [0, kept), then those of [lo, pos]
+};
+__device__ __forceinline__ TileRun tile_run(int pos, int window, int keep_first, int chunked) {
+    TileRun g;
+    g.lo = first_visible(pos, window, chunked);
+    g.kept = keep_first < g.lo ? keep_first : g.lo;
+    g.nk = (g.kept + 15) / 16;
+    g.n = g.nk + (pos - g.lo) / 16 + 1;
+    return g;
+}
+
+__device__ __forceinline__ float swap_add16(float x, float y) {   // rows 0, 2: x summed over a pair of rows; 1, 3: y
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+__device__ __forceinline__ float swap_add32(float x, float y) {   // lower half: x summed over the halves; upper: y
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+__device__ __forceinline__ float rows_max(float x) {              // over the four rows of 16 lanes
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+
+typedef __attribute__((ext_vector_type(8))) __bf16 wa_bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) float wa_f32x4_t;
+
+template <bool F32, int HEADS, int NW, int KS, int VE>
+__global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q, int64_t ldq, const void* kc_, const void* vc_,
+                                                              void* out_, int64_t ldo, float* part, PagedRows pr,
+                                                              const float* slopes, const float* sinks, int H, int G,
+                                                              float scale, int window, int keep_first, const int* row_len,
+                                                              int max_len, int splits, const float* gate, int64_t ldg,
+                                                              int chunked) {
+    typedef typename ActS<F32>::T T_;
+    constexpr int d = 32 * KS, dv = 16 * VE, HB = HEADS == 8 ? 2 : 1, RT = HEADS;
+    constexpr int NK = F32 ? 2 * KS : KS, VW = F32 ? VE : VE / 2;     // 16-byte pieces of a key, words of a value, per lane
+    __shared__ __attribute__((aligned(16))) float red[NW * RT * dv];
+    __shared__ float mm[NW * RT], ll[NW * RT];
+    const T_* kc = (const T_*)kc_;
+    const T_* vc = (const T_*)vc_;
+    const int R = H / G, ngrp = (R + kGrpMax - 1) / kGrpMax;
+    const int unit = blockIdx.x, split = blockIdx.y;
+    const int t = unit / (G * ngrp), g = (unit / ngrp) % G, grp = unit % ngrp;
+    const int h0 = g * R + grp * kGrpMax;
+    const int nh = R - grp * kGrpMax < kGrpMax ? R - grp * kGrpMax : kGrpMax;   // heads of this workgroup, <= RT
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, col = lane & 15, quad = lane >> 4;
+    const int row = pr.tok_row[t], pos = pr.tok_pos[t];
+
+    // q as the second operand: lane `col` holds head col % 4 (of bf16 keys: its part col / 4)
+    wa_bf16x8_t qb[HB][F32 ? 1 : KS];
+    wa_f32x4_t qf[HB][F32 ? NK : 1];
+    float slope[HB];
+#pragma unroll
+    for (int b = 0; b < HB; ++b) {
+        const int h = HEADS == 1 ? 0 : 4 * b + (lane & 3);
+        const bool ok = h < nh;
+        const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (ok ? h : 0)) * d;
+        slope[b] = (slopes && ok) ? slopes[h0 + h] : 0.f;
+        if constexpr (F32) {
+#pragma unroll
+            for (int i = 0; i < NK; ++i) {
+                const wa_f32x4_t x = *reinterpret_cast<const wa_f32x4_t*>(qr + 16 * i + 4 * quad);
+                qf[b][i] = ok ? x : (wa_f32x4_t){0.f, 0.f, 0.f, 0.f};
+            }
+        } else {
+            const int s = col >> 2;
+#pragma unroll
+            for (int i = 0; i < KS; ++i) {
+                const wa_f32x4_t x0 = *reinterpret_cast<const wa_f32x4_t*>(qr + 32 * i + 8 * quad);
+                const wa_f32x4_t x1 = *reinterpret_cast<const wa_f32x4_t*>(qr + 32 * i + 8 * quad + 4);
+                uint16_t p[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    // eight bits of the significand at a time
+                    const float x = e < 4 ? x0[e & 3] : x1[e & 3];
+                    const uint32_t a = __float_as_uint(x) & 0xffff0000u;
+                    const float r1 = x - __uint_as_float(a);
+                    const uint32_t b2 = __float_as_uint(r1) & 0xffff0000u;
+                    const float r2 = r1 - __uint_as_float(b2);
+                    const uint32_t w = s == 0 ? a : s == 1 ? b2 : __float_as_uint(r2);
+                    p[e] = ok && s < 3 ? (uint16_t)(w >> 16) : (uint16_t)0;
+                }
+                qb[b][i] = __builtin_bit_cast(wa_bf16x8_t, *reinterpret_cast<uint4*>(p));
+            }
+        }
+    }
+
+    const TileRun gt = tile_run(pos, window, keep_first, chunked);
+    if (max_len > 0 && row_len[row] > max_len) return;   // the tiled kernel's rows
+    if (split * NW >= gt.n) return;                      // no keys for this split
+    const int* bt = pr.block_table + (int64_t)row * pr.bt_stride;
+    float m[HB], l[HB];
+    wa_f32x4_t acc[HB][VE];
+#pragma unroll
+    for (int b = 0; b < HB; ++b) {
+        m[b] = -INFINITY;
+        l[b] = 0.f;
+#pragma unroll
+        for (int e = 0; e < VE; ++e) acc[b][e] = (wa_f32x4_t){0.f, 0.f, 0.f, 0.f};
+    }
+    // the tile's keys, this lane's key (lane % 16; past the last key: the first) and the place of its row
+    int first, cnt, j;
+    int page_no;
+    auto locate = [&](int u) {
+        if (u >= gt.n) u = gt.n - 1;
+        first = u < gt.nk ? 16 * u : gt.lo + 16 * (u - gt.nk);
+        const int end = u < gt.nk ? gt.kept - 1 : pos;
+        cnt = end - first + 1 < 16 ? end - first + 1 : 16;
+        j = first + (col < cnt ? col : 0);
+        page_no = bt[j / pr.page];
+    };
+    locate(split * NW + wv);
+    for (int u = split * NW + wv; u < gt.n; u += NW * splits) {
+        const unsigned slot = (unsigned)page_no * (unsigned)pr.page + (unsigned)(j % pr.page);
+        const T_* kr = kc + ((uint64_t)slot * G + g) * d;
+        uint4 kq[NK];
+        uint32_t vq[4][VW];
+#pragma unroll
+        for (int i = 0; i < NK; ++i) kq[i] = ld16(kr + (F32 ? 16 * i + 4 * quad : 32 * i + 8 * quad));
+        unsigned vslot[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) vslot[k] = (unsigned)__shfl((int)slot, 4 * quad + k, 64);   // (lanes 0 - 15: keys in order)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t* vr = reinterpret_cast<const uint32_t*>(vc + ((uint64_t)vslot[k] * G + g) * dv) + col * VW;
+            if constexpr (VW % 4 == 0) {
+#pragma unroll
+                for (int w = 0; w < VW; w += 4) {
+                    const uint4 x = ld16(vr + w);
+                    vq[k][w] = x.x; vq[k][w + 1] = x.y; vq[k][w + 2] = x.z; vq[k][w + 3] = x.w;
+                }
+            } else if constexpr (VW % 2 == 0) {
+#pragma unroll
+                for (int w = 0; w < VW; w += 2) {
+                    const uint2 x = *reinterpret_cast<const uint2*>(vr + w);
+                    vq[k][w] = x.x; vq[k][w + 1] = x.y;
+                }
+            } else {
+#pragma unroll
+                for (int w = 0; w < VW; ++w) vq[k][w] = vr[w];
+            }
+        }
+        wa_f32x4_t sc[HB];
+#pragma unroll
+        for (int b = 0; b < HB; ++b) {
+            sc[b] = (wa_f32x4_t){0.f, 0.f, 0.f, 0.f};
+            if constexpr (F32) {
+#pragma unroll
+                for (int i = 0; i < NK; ++i) {
+                    const uint32_t kw[4] = {kq[i].x, kq[i].y, kq[i].z, kq[i].w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        sc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(kw[e]), qf[b][i][e], sc[b], 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < KS; ++i)
+                    sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(wa_bf16x8_t, kq[i]), qb[b][i], sc[b], 0, 0, 0);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    sc[b][k] += dpp<0x128>(sc[b][k]);      // row_ror:8, row_ror:4
+                    sc[b][k] += dpp<0x124>(sc[b][k]);
+                }
+                // an infinite key or query times a part that is zero: the plain sum decides
+                const int h = HEADS == 1 ? 0 : 4 * b + (lane & 3);
+                const bool bad = h < nh && !(sc[b][0] == sc[b][0] && sc[b][1] == sc[b][1] &&
+                                          sc[b][2] == sc[b][2] && sc[b][3] == sc[b][3]);
+                if (__any(bad)) {
+                    const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (h < nh ? h : 0)) * d;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const T_* kp = kc + ((uint64_t)vslot[k] * G + g) * d;
+                        float dot = 0.f;
+#pragma unroll 1
+                        for (int c = 0; c < d; ++c) dot = fmaf(qr[c], ActS<F32>::ld(kp + c), dot);
+                        sc[b][k] = dot;
+                    }
+                }
+            }
+        }
+        if (cnt < 16) {      // rows that repeat the first key: weight zero, and no value that could be infinite
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (4 * quad + k >= cnt)
+#pragma unroll
+                    for (int w = 0; w < VW; ++w) vq[k][w] = 0;
+        }
+#pragma unroll
+        for (int b = 0; b < HB; ++b) {
+            float p[4], mx = -INFINITY;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int key = 4 * quad + k;
+                p[k] = key < cnt ? sc[b][k] * scale - slope[b] * (float)(pos - first - key) : -INFINITY;
+                mx = fmaxf(mx, p[k]);
+            }
+            const float mn = fmaxf(m[b], rows_max(mx));        // finite: a tile holds at least one key
+            const float corr = expf(m[b] - mn);                // m = -inf on the wave's first tile: exp(-inf) = 0
+            float sum = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                p[k] = 4 * quad + k < cnt ? expf(p[k] - mn) : 0.f;
+                sum += p[k];
+            }
+            l[b] = l[b] * corr + sum;                          // this lane's four keys' share
+            m[b] = mn;
+            if (HEADS == 1) {
+#pragma unroll
+                for (int e = 0; e < VE; ++e) acc[b][e][0] *= corr;
+            } else if (__any(corr != 1.f)) {
+                const float c0 = dpp<0x00>(corr), c1 = dpp<0x55>(corr), c2 = dpp<0xAA>(corr), c3 = dpp<0xFF>(corr);
+#pragma unroll
+                for (int e = 0; e < VE; ++e) {
+                    acc[b][e][0] *= c0;
+                    acc[b][e][1] *= c1;
+                    acc[b][e][2] *= c2;
+                    acc[b][e][3] *= c3;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int e = 0; e < VE; ++e) {
+                    const float v = F32 ? __uint_as_float(vq[k][F32 ? e : 0])
+                                    : (e & 1) ? bf16_hi(vq[k][F32 ? 0 : e >> 1]) : bf16_lo(vq[k][F32 ? 0 : e >> 1]);
+                    if (HEADS == 1) acc[b][e][0] = fmaf(p[k], v, acc[b][e][0]);
+                    else acc[b][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(p[k], v, acc[b][e], 0, 0, 0);
+                }
+        }
+        locate(u + NW * splits);
+    }
+    const int nact = gt.n - split * NW < NW ? gt.n - split * NW : NW;   // waves with a tile
+    if (wv < nact) {
+#pragma unroll
+        for (int b = 0; b < HB; ++b) {
+            l[b] = swap_add16(l[b], l[b]);
+            l[b] = swap_add32(l[b], l[b]);
+            if (lane < (HEADS == 1 ? 1 : 4)) {
+                mm[wv * RT + 4 * b + lane] = m[b];
+                ll[wv * RT + 4 * b + lane] = l[b];
+            }
+            // rows of lanes hold different keys: row h keeps the sum of head h
+            float o[VE];
+#pragma unroll
+            for (int e = 0; e < VE; ++e)
+                if (HEADS == 1) o[e] = swap_add16(swap_add32(acc[b][e][0], acc[b][e][0]), swap_add32(acc[b][e][0], acc[b][e][0]));
+                else o[e] = swap_add16(swap_add32(acc[b][e][0], acc[b][e][2]), swap_add32(acc[b][e][1], acc[b][e][3]));
+            float* rw = red + (wv * RT + (HEADS == 1 ? 0 : 4 * b + quad)) * dv + col * VE;
+#pragma unroll
+            for (int e = 0; e < VE; e += 2)
+                if (HEADS > 1 || quad == 0) *reinterpret_cast<float2*>(rw + e) = make_float2(o[e], o[e + 1]);
+        }
+    }
+    __syncthreads();
+    const bool alone = gt.n <= NW || splits == 1;
+    for (int i = tid; i < nh * dv; i += 64 * NW) {
+        const int r = i / dv, c = i - r * dv;
+        float M = -INFINITY;
+        for (int w = 0; w < nact; ++w) M = fmaxf(M, mm[w * RT + r]);
+        float L = 0.f, o = 0.f;
+        for (int w = 0; w < nact; ++w) {
+            const float f = expf(mm[w * RT + r] - M);
+            L = fmaf(ll[w * RT + r], f, L);
+            o = fmaf(red[(w * RT + r) * dv + c], f, o);
+        }
+        const int h = h0 + r;
+        if (alone) {
+            if (sinks) {
+                const float sk = sinks[h], mf = fmaxf(M, sk), f = expf(M - mf);
+                L = L * f + expf(sk - mf);
+                o *= f;
+            }
+            o /= L;
+            if (gate) o *= sigmoid_f(gate[(int64_t)t * ldg + (int64_t)h * dv + c]);
+            ActS<F32>::st((T_*)out_ + (int64_t)t * ldo + (int64_t)h * dv + c, o);
+        } else {
+            float* dst = part + (((int64_t)t * H + h) * splits + split) * (dv + 2);
+            if (c == 0) {
+                dst[0] = M;
+                dst[1] = L;
+            }
+            dst[2 + c] = o;
+        }
+    }
+}
+
+// one wave per (token, head): the splits' pieces and the sink become the output row.  nw > 0: window_attn_few_kernel's splits
+// of nw waves, of which those past the token's tiles left nothing and a single one is the finished row.
 template <bool F32>
 __global__ __launch_bounds__(64) void window_attn_merge_kernel(const float* part, void* out_, int64_t ldo,
-                                                               const int* tok_row, const float* sinks, int H, int dv,
-                                                               int splits, const int* row_len, int max_len,
+                                                               const int* tok_row, const int* tok_pos, const float* sinks,
+                                                               int H, int dv, int splits, int nw, int window, int keep_first,
+                                                               int chunked, const int* row_len, int max_len,
                                                                const float* gate, int64_t ldg) {
     typedef typename ActS<F32>::T T_;
     const int t = blockIdx.x / H, h = blockIdx.x % H, lane = threadIdx.x;
+    int n = splits;                            // pieces there are
+    if (nw > 0) {
+        const int tiles = tile_run(tok_pos[t], window, keep_first, chunked).n;
+        if (tiles <= nw) return;
+        if (tiles < splits * nw) n = (tiles + nw - 1) / nw;
+    }
     if (max_len > 0 && row_len[tok_row[t]] > max_len) return;
     const float* src = part + (int64_t)blockIdx.x * splits * (dv + 2);
-    float M = sinks ? sinks[h] : -INFINITY;
-    for (int s2 = 0; s2 < splits; ++s2) M = fmaxf(M, src[(int64_t)s2 * (dv + 2)]);
-    float L = sinks ? expf(sinks[h] - M) : 0.f;
-    for (int s2 = 0; s2 < splits; ++s2) {
-        const float ms = src[(int64_t)s2 * (dv + 2)];
-        if (ms != -INFINITY) L = fmaf(src[(int64_t)s2 * (dv + 2) + 1], expf(ms - M), L);
+    float M = -INFINITY, L = 0.f;
+    for (int s = lane; s < n; s += 64) M = fmaxf(M, src[(int64_t)s * (dv + 2)]);
+    M = wave_max(M);
+    if (sinks) M = fmaxf(M, sinks[h]);
+    for (int s = lane; s < n; s += 64) {
+        const float ms = src[(int64_t)s * (dv + 2)];
+        if (ms != -INFINITY) L = fmaf(src[(int64_t)s * (dv + 2) + 1], expf(ms - M), L);
     }
+    L = wave_sum(L);
+    if (sinks) L += expf(sinks[h] - M);
     for (int c = lane; c < dv; c += 64) {
         float o = 0.f;
-        for (int s2 = 0; s2 < splits; ++s2) {
-            const float ms = src[(int64_t)s2 * (dv + 2)];
-            if (ms != -INFINITY) o = fmaf(src[(int64_t)s2 * (dv + 2) + 2 + c], expf(ms - M), o);
+#pragma unroll 4
+        for (int s = 0; s < n; ++s) {
+            const float ms = src[(int64_t)s * (dv + 2)], f = ms != -INFINITY ? expf(ms - M) : 0.f;
+            o = fmaf(f != 0.f ? src[(int64_t)s * (dv + 2) + 2 + c] : 0.f, f, o);
         }
         o /= L;
         if (gate) o *= sigmoid_f(gate[(int64_t)t * ldg + (int64_t)h * dv + c]);
@@ -1391,8 +1714,6 @@ __global__ __launch_bounds__(64) void window_attn_merge_kernel(const float* part
 // in fp32 per lane, and P.V with every fp32 weight split exactly into three bf16 numbers, on the same bf16
 // instruction with fp32 accumulators: the score accumulators of a lane, S[key 16 nt + 4 (lane / 16) + j][query
 // lane % 16], serve as its second operand where they lie, so P never leaves the registers.
-typedef __attribute__((ext_vector_type(8))) __bf16 wa_bf16x8_t;
-
 template <int KS, int CT>
 __global__ __launch_bounds__(256) void window_attn_tile_kernel(const float* q, int64_t ldq, const uint16_t* kc,
                                                                const uint16_t* vc, uint16_t* out, int64_t ldo,
@@ -2021,6 +2342,57 @@ int mv_window_attn(const float* q, int64_t ldq, const void* k_cache, const void*
     // head and cuts the keys over several workgroups
     if (part && splits >= 1) {
         const int R = heads / kv_heads, ngrp = (R + kGrpMax - 1) / kGrpMax, top = R < kGrpMax ? R : kGrpMax;
+        auto merge = [&](int pieces, int nw) {
+#define MV_WA_MERGE(F32_)                                                                                              \
+    hipLaunchKernelGGL(window_attn_merge_kernel<F32_>, grid, dim3(64), 0, s, part, out, ldo, tok_row, tok_pos, sinks, heads, \
+                       dv, pieces, nw, window, keep_first, chunked, row_len, skip_len, gate, ldg)
+            if (f32) MV_WA_MERGE(true);
+            else MV_WA_MERGE(false);
+#undef MV_WA_MERGE
+        };
+        if (aligned16(q) && ldq % 4 == 0 && aligned16(k_cache) && aligned16(v_cache)) {
+            // Sixteen waves (eight where the registers of fp32 rows or of eight heads allow no more) while every workgroup has
+            // a compute unit to itself, else four.  A split has 64 keys to a wave of the widest form before another is
+            // opened: one token at 1100 keys took 23.2 us in five splits and takes 20.3 in one, at 45 keys the merge's
+            // launch alone is 2 of 10 us.  fp32 rows, twice as long to read and eight waves, gain from a second split
+            // (1100 keys 30.8 -> 24.0 us, 45 keys 6.6 -> 8.0).
+            const int64_t groups = (int64_t)tokens * kv_heads * ngrp;
+            const int64_t fill = ((int64_t)window + keep_first) / (f32 ? 512 : 1024);
+            const int pieces = fill < 1 ? 1 : fill < splits ? (int)fill : splits;
+            const bool wide = groups * pieces <= num_cus();
+            int nw = 0;      // (0: a head shape without an instance)
+#define MV_WA_FEW(F32_, HB_, NW_, KS_, VE_)                                                                            \
+    hipLaunchKernelGGL((window_attn_few_kernel<F32_, HB_, NW_, KS_, VE_>), dim3((unsigned)groups, pieces), dim3(64 * NW_), 0, s, \
+                       q, ldq, k_cache, v_cache, out, ldo, part, pr, slopes, sinks, heads, kv_heads, scale, window, keep_first, \
+                       row_len, skip_len, pieces, gate, ldg, chunked);                                                 \
+    nw = NW_
+#define MV_WA_FEW_HB(F32_, KS_, VE_)                                                                                   \
+    do {                                                                                                               \
+        if (top > 4) { if (wide) { MV_WA_FEW(F32_, 8, 8, KS_, VE_); } else { MV_WA_FEW(F32_, 8, 4, KS_, VE_); } }      \
+        else if (top > 1) { if (wide) { MV_WA_FEW(F32_, 4, (F32_ ? 8 : 16), KS_, VE_); } else { MV_WA_FEW(F32_, 4, 4, KS_, VE_); } } \
+        else if (wide) { MV_WA_FEW(F32_, 1, 16, KS_, VE_); }                                                           \
+        else { MV_WA_FEW(F32_, 1, 4, KS_, VE_); }                                                                      \
+    } while (0)
+#define MV_WA_FEW_D(F32_)                                                                                              \
+    do {                                                                                                               \
+        if (d == 128 && dv == 128) MV_WA_FEW_HB(F32_, 4, 8);                                                           \
+        else if (d == 64 && dv == 64) MV_WA_FEW_HB(F32_, 2, 4);                                                        \
+        else if (d == 96 && dv == 96) MV_WA_FEW_HB(F32_, 3, 6);                                                        \
+        else if (d == 128 && dv == 64) MV_WA_FEW_HB(F32_, 4, 4);                                                       \
+        else if (d == 64 && dv == 128) MV_WA_FEW_HB(F32_, 2, 8);                                                       \
+        else if (d == 32 && dv == 32) MV_WA_FEW_HB(F32_, 1, 2);                                                        \
+        else if (d == 64 && dv == 32) MV_WA_FEW_HB(F32_, 2, 2);                                                        \
+    } while (0)
+            if (f32) MV_WA_FEW_D(true);
+            else MV_WA_FEW_D(false);
+#undef MV_WA_FEW_D
+#undef MV_WA_FEW_HB
+#undef MV_WA_FEW
+            if (nw) {
+                if (pieces > 1) merge(pieces, nw);
+                return check_launch();
+            }
+        }
         const int rt = top <= 1 ? 1 : top <= 2 ? 2 : top <= 4 ? 4 : 8;
         const int vecw = f32 ? 4 : 8;
         const int vec = dv % vecw == 0 && dv / vecw <= 64 && aligned16(v_cache);
@@ -2039,10 +2411,7 @@ int mv_window_attn(const float* q, int64_t ldq, const void* k_cache, const void*
                 else if (rt == 4) MV_WA_GROUP(false, 4); else MV_WA_GROUP(false, 8);
             }
 #undef MV_WA_GROUP
-            if (splits > 1) {
-                if (f32) hipLaunchKernelGGL(window_attn_merge_kernel<true>, grid, dim3(64), 0, s, part, out, ldo, tok_row, sinks, heads, dv, splits, row_len, skip_len, gate, ldg);
-                else hipLaunchKernelGGL(window_attn_merge_kernel<false>, grid, dim3(64), 0, s, part, out, ldo, tok_row, sinks, heads, dv, splits, row_len, skip_len, gate, ldg);
-            }
+            if (splits > 1) merge(splits, 0);
             return check_launch();
         }
     }

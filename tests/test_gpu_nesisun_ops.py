@@ -467,3 +467,46 @@ def test_routed_experts_with_pass_through(ops, f32, E, n_id, top):
     y = torch.empty(T, W, device=DEV)
     ops.moe_combine(down, place, wts, None, None, y, ids=ids.view(-1), first_pass=E, passed=hd)
     assert (y.cpu().double() - want).abs().max().item() < (3e-5 if f32 else 4e-2)
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("d,dv", [(128, 128), (64, 64), (96, 96), (128, 64), (64, 128), (32, 32), (64, 32)])
+@pytest.mark.parametrize("H,G,rows,page,window,keep,chunked,splits", [
+    (8, 2, 3, 64, 100, 0, False, 1), (3, 3, 5, 48, 300, 20, False, 3), (9, 1, 2, 16, 5000, 0, False, 4), (14, 2, 2, 64, 1024, 70, False, 7),
+    (4, 4, 80, 64, 64, 33, False, 2), (16, 2, 140, 64, 90, 0, True, 1), (2, 1, 300, 64, 40, 0, False, 1)])
+def test_few_token_attention_equals_the_per_head_form(ops, f32, d, dv, H, G, rows, page, window, keep, chunked, splits):
+    """Every instance (one, up to four and up to eight heads a workgroup, few and many workgroups, one split and several)
+    against one workgroup per head: contexts from one key to past the window, an infinite key of weight zero, strides and
+    pages of other sizes, a gate, a sink and a distance penalty.  Both add at most `keys` products in fp32 under weights
+    that differ by the error of scores of up to 6 (d products each): 1e-5 of the values; where that moves a bf16 output across a rounding
+    boundary, the step between two neighbours is at most 2^-7 of the value (8 significant bits)."""
+    from types import SimpleNamespace
+
+    g = torch.Generator().manual_seed(d + dv + H + rows)
+    dt = torch.float32 if f32 else torch.bfloat16
+    ctx = torch.randint(0, 1100, (rows,), generator=g)
+    ctx[0], ctx[-1] = 0, min(1099, window + 17)
+    per = 1100 // page + 1
+    bt = torch.randperm(rows * per, generator=g).int().view(rows, per)
+    kc = torch.randn(rows * per, page, G, d, generator=g).to(dt)
+    vc = torch.randn(rows * per, page, G, dv, generator=g).to(dt)
+    q = torch.randn(rows, H * d + 8, generator=g)
+    q[1, :H * d:d] = -q[1, :H * d:d].abs() - 0.1
+    for i in range(0, int(ctx[1]), 7):           # -infinity for every head: the key's weight is zero
+        kc[bt[1, i // page], i % page, :, 0] = float("inf")
+    step = SimpleNamespace(tok_row=torch.arange(rows).int().to(DEV), tok_pos=ctx.int().to(DEV), block_table=bt.to(DEV),
+                           row_len=torch.ones(rows, dtype=torch.int32, device=DEV), ch_start=None, ch_len=None, n_chunks=0,
+                           page=page, max_page=rows * per - 1, tokens=rows)
+    gate, sink, slopes = torch.randn(rows, H * dv, generator=g).to(DEV), torch.randn(H, generator=g).to(DEV), \
+        (0.01 * torch.rand(H, generator=g)).to(DEV)
+    outs = []
+    for grouped in (False, True):
+        out = torch.empty(rows, H * dv + 8, dtype=dt, device=DEV)[:, :H * dv]
+        part = torch.full((rows * H * splits * (dv + 2),), float("nan"), device=DEV) if grouped else None
+        ops.window_attn(q.to(DEV)[:, :H * d], kc.to(DEV), vc.to(DEV), out, step, slopes, H, G, d, dv, d ** -0.5, window,
+                        keep_first=keep, sinks=sink, part=part, splits=splits, gate=gate, chunked=chunked)
+        outs.append(out.float())
+    top = vc.float().abs().max().item()
+    assert bool(torch.isfinite(outs[0]).all())
+    tol = 1e-5 * top + (0 if f32 else 2 ** -7) * outs[0].abs()
+    assert ((outs[1] - outs[0]).abs() <= tol).all()
