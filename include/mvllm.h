@@ -535,7 +535,8 @@ int mv_scan_outer(const float* q, int64_t ldq, int q_div, const float* k, int64_
 
 /* The same recurrence for long rows, 64 tokens at a time, its products on the fp32 matrix instruction
  * (v_mfma_f32_16x16x4_f32; three launches: sums within each chunk, the states the chunks start from, their
- * contribution to the outputs).  Chunk c covers tokens ch_start[c] ..
+ * contribution to the outputs; or, for sixteen heads and more with n of 64 or 128, the chunks' scores and then every row
+ * from its first chunk to its last with the state in registers).  Chunk c covers tokens ch_start[c] ..
  * + ch_len[c] (<= 64) of one row; row b owns chunks row_ch0[b] .. + row_nch[b] (0: the row is not taken -
  * mv_scan_outer with max_len > 0 leaves exactly the rows longer than max_len to this call).  The decay
  * comes as its logarithm ([tokens, heads], or [heads] with ld_ld == 0).  Scratch: ds [chunks, heads, n, p],

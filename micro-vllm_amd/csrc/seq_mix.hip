@@ -419,6 +419,249 @@ __global__ __launch_bounds__(256) void scan_chunk_inter_kernel(ChunkArgs a) {
     }
 }
 
+// The same in two launches for the usual shapes (n of 64 or 128, p a multiple of 16, 16-byte rows), without the chunks'
+// states in memory.  The columns of a state do not meet, so one workgroup takes a (row, head, 16 CT columns) through all of
+// the row's chunks, its slice of S in registers:
+//   scores  q_t . k_s of every chunk once per group of heads (they were formed once per four heads)
+//   scan    waves 0 - 3 (one per 16 tokens): o_t = exp(L_t) S0^T q_t + sum_s P[t][s] v_s (+ skip v_t); waves 4 - 7: the n rows
+//           of S = exp(L_end) S0 + k^T (w v).  The two kinds run side by side, one of each to a SIMD: S0 goes to the others
+//           through LDS, two buffers, one barrier a chunk; the next chunk's q, k and scores are in flight to registers.
+// The contraction index of a product is dealt out as 16 a + 4 g + e (e: step of the instruction), so a lane's operands of
+// four steps are one 16-byte read.  A chunk takes a SIMD 160 of the fp32 instruction at 32 cycles (2.1 us at 32 columns) and
+// measures 4.5: sums that wait for each other, exponentials, the barrier.  16 columns a workgroup, two workgroups to a unit,
+// read q and k twice as often: 203 against 155 us.  Both launches, against the three above with the chunks' states written,
+// carried and read back (us, n = 128, p = 64): 128 heads in one group, 2048 tokens 727 -> 155; 100 tokens 193 -> 20; 16 heads
+// with q and k of their own, 2048 tokens 157 -> 121, 333 tokens 74 -> 32; 24 heads, n = 64, 65 + 65 + 65 + 900 tokens 124 -> 50.
+__global__ __launch_bounds__(256) void scan_scores_kernel(ChunkArgs a, float* scores) {
+    const int ch = blockIdx.x, grp = blockIdx.y, tt = blockIdx.z;
+    const int st = threadIdx.x >> 6, r = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    if (st > tt) return;
+    const int start = a.ch_start[ch], last = a.ch_len[ch] - 1;
+    const int tq = min(16 * tt + r, last), ts = min(16 * st + r, last);    // (tokens past the end: masked where they are read)
+    const float* qp = a.q + (int64_t)(start + tq) * a.ldq + (int64_t)grp * a.n + 4 * g;
+    const float* kp = a.k + (int64_t)(start + ts) * a.ldk + (int64_t)grp * a.n + 4 * g;
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < a.n; j += 64) {
+        f32x4_t x[4], y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i] = *reinterpret_cast<const f32x4_t*>(qp + j + 16 * i);
+            y[i] = *reinterpret_cast<const f32x4_t*>(kp + j + 16 * i);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) MV_MFMA4(acc, x[i][e], y[i][e]);
+    }
+    float* o = scores + ((int64_t)ch * gridDim.y + grp) * kCh * kCh + (16 * tt + 4 * g) * kCh + 16 * st + r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j * kCh] = acc[j];
+}
+
+template <int NJ, int CT>   // n / 16, column tiles of 16
+__global__ __launch_bounds__(512) void scan_rows_kernel(ChunkArgs a, const float* scores, int groups) {
+    constexpr int n = 16 * NJ, BC = 16 * CT, SV = kCh + 4, SS = n + 4, JW = NJ / 4;
+    __shared__ __attribute__((aligned(16))) float vt[2][BC * SV];       // [column][token]
+    __shared__ __attribute__((aligned(16))) float s0[2][BC * SS];       // [column][state row]
+    __shared__ __attribute__((aligned(16))) float Ls[2][kCh], gs[2][kCh], ws[2][kCh], el[2][kCh];
+    __shared__ float at[2];
+    const int blocks = a.p / BC, h = blockIdx.x / blocks, c0 = (blockIdx.x % blocks) * BC, b = blockIdx.y;
+    const int nch = a.row_nch[b], ch0 = a.row_ch0[b];
+    if (nch == 0) return;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);    // (a scalar: the two kinds of wave branch, they do not mask)
+    const int grp = h / a.q_div, np = n * a.p;
+    float* sp = a.state + ((int64_t)a.r.row_slot[b] * a.H + h) * np + c0;
+    const float* qb = a.q + (int64_t)grp * n;
+    const float* kb = a.k + (int64_t)grp * n;
+    const float* vb = a.v + (int64_t)h * a.p + c0;
+
+    // The workgroup's part of v and the decays of a chunk: requested two chunks ahead, staged one ahead.  (Loads stay plain
+    // requests until they are used: arithmetic on them here would wait for them.)
+    f32x4_t vn;
+    float ldn = 0.f, gn = 1.f;
+    const int vs_ = tid / (BC / 4), vc_ = 4 * (tid % (BC / 4));     // token and first column of this thread's piece of v
+    auto fetch_v = [&](int start, int len) {
+        vn = *reinterpret_cast<const f32x4_t*>(vb + (int64_t)(start + min(vs_, len - 1)) * a.ldv + vc_);
+        if (wv == 0) {
+            const int64_t t = start + min(lane, len - 1);
+            ldn = a.log_decay[t * a.ld_ld + h];
+            if (a.gain) gn = a.gain[t * a.ld_gain + h];
+        }
+    };
+    auto stage = [&](int buf, int len) {
+        if (vs_ < kCh)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) vt[buf][(vc_ + i) * SV + vs_] = vs_ < len ? vn[i] : 0.f;
+        if (wv == 0) {      // inclusive running sum of the log decays
+            float l = lane < len ? fmaxf(ldn, -80.f) : 0.f;
+            const float gain = lane < len ? gn : 0.f;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const float up = __shfl_up(l, o, 64);
+                if (lane >= o) l += up;
+            }
+            const float lend = __shfl(l, len - 1, 64);
+            Ls[buf][lane] = l;
+            gs[buf][lane] = gain;
+            ws[buf][lane] = expf(lend - l) * gain;    // weight of token s in the state the chunk ends with
+            el[buf][lane] = expf(l);
+            if (lane == 0) at[buf] = expf(lend);
+        }
+    };
+    // chunk c of the row (past the end: the last)
+    const int* cs = a.ch_start + ch0;
+    const int* cl = a.ch_len + ch0;
+    auto at_most = [&](int c) { return c < nch ? c : nch - 1; };
+    int st0 = cs[0], ln0 = cl[0], st1 = cs[at_most(1)], ln1 = cl[at_most(1)];
+    fetch_v(st0, ln0);
+    if (wv < 4) {
+        const int tt = wv;
+        const float sk = a.skip ? a.skip[h] : 0.f;
+        f32x4_t fr[NJ], pr[4];
+        auto fetch = [&](int ch, int start, int len) {
+            const float* qp = qb + (int64_t)(start + min(16 * tt + r, len - 1)) * a.ldq + 4 * g;
+#pragma unroll
+            for (int i = 0; i < NJ; ++i) fr[i] = *reinterpret_cast<const f32x4_t*>(qp + 16 * i);
+            const float* pp = scores + ((int64_t)ch * groups + grp) * kCh * kCh + (16 * tt + r) * kCh + 4 * g;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pr[i] = *reinterpret_cast<const f32x4_t*>(pp + 16 * (i <= tt ? i : tt));
+        };
+        fetch(ch0, st0, ln0);
+        stage(0, ln0);
+        fetch_v(st1, ln1);
+        __syncthreads();
+        for (int c = 0; c < nch; ++c) {
+            const int buf = c & 1, start = st0, len = ln0;
+            f32x4_t now[NJ], sc[4];
+#pragma unroll
+            for (int i = 0; i < NJ; ++i) now[i] = fr[i];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sc[i] = pr[i];
+            st0 = st1, ln0 = ln1;
+            st1 = cs[at_most(c + 2)], ln1 = cl[at_most(c + 2)];
+            fetch(ch0 + at_most(c + 1), st0, ln0);
+            f32x4_t o[CT];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) o[ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NJ; ++i) {
+                f32x4_t y[CT];
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) y[ct] = *reinterpret_cast<const f32x4_t*>(&s0[buf][(16 * ct + r) * SS + 16 * i + 4 * g]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) MV_MFMA4(o[ct], now[i][e], y[ct][e]);
+            }
+            const f32x4_t w = *reinterpret_cast<const f32x4_t*>(&el[buf][16 * tt + 4 * g]);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) o[ct] *= w;
+            const float Lt = Ls[buf][16 * tt + r];
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                if (st > tt) break;
+                const f32x4_t L4 = *reinterpret_cast<const f32x4_t*>(&Ls[buf][16 * st + 4 * g]);
+                const f32x4_t g4 = *reinterpret_cast<const f32x4_t*>(&gs[buf][16 * st + 4 * g]);
+                f32x4_t P, y[CT];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool seen = st < tt || 4 * g + e <= r;
+                    P[e] = seen ? sc[st][e] * expf(Lt - L4[e]) * g4[e] : 0.f;
+                }
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) y[ct] = *reinterpret_cast<const f32x4_t*>(&vt[buf][(16 * ct + r) * SV + 16 * st + 4 * g]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) MV_MFMA4(o[ct], P[e], y[ct][e]);
+            }
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const f32x4_t v4 = *reinterpret_cast<const f32x4_t*>(&vt[buf][(16 * ct + r) * SV + 16 * tt + 4 * g]);
+                float* op = a.out + (int64_t)(start + 16 * tt + 4 * g) * a.ldo + (int64_t)h * a.p + c0 + 16 * ct + r;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (16 * tt + 4 * g + j < len) op[j * a.ldo] = a.skip ? fmaf(sk, v4[j], o[ct][j]) : o[ct][j];
+            }
+            stage(buf ^ 1, ln0);
+            fetch_v(st1, ln1);
+            __syncthreads();
+        }
+    } else {
+        const int j0 = 16 * JW * (wv - 4);       // first of this wave's state rows
+        f32x4_t S[JW][CT], fr[NJ];               // S: rows j0 + 16 i + 4 g .. + 3, column 16 ct + r
+        auto fetch = [&](int start, int len) {
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float* kp = kb + (int64_t)(start + min(16 * st + 4 * g + e, len - 1)) * a.ldk + j0 + r;
+#pragma unroll
+                    for (int i = 0; i < JW; ++i) fr[4 * i + st][e] = kp[16 * i];
+                }
+        };
+        auto publish = [&](int buf) {
+#pragma unroll
+            for (int i = 0; i < JW; ++i)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+                    *reinterpret_cast<f32x4_t*>(&s0[buf][(16 * ct + r) * SS + j0 + 16 * i + 4 * g]) = S[i][ct];
+        };
+        fetch(st0, ln0);
+        const bool carried = a.r.row_ctx[b] > 0;
+#pragma unroll
+        for (int i = 0; i < JW; ++i)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    S[i][ct][j] = carried ? sp[(int64_t)(j0 + 16 * i + 4 * g + j) * a.p + 16 * ct + r] : 0.f;
+        publish(0);
+        stage(0, ln0);
+        fetch_v(st1, ln1);
+        __syncthreads();
+        for (int c = 0; c < nch; ++c) {
+            const int buf = c & 1;
+            f32x4_t now[NJ];
+#pragma unroll
+            for (int i = 0; i < NJ; ++i) now[i] = fr[i];
+            st0 = st1, ln0 = ln1;
+            st1 = cs[at_most(c + 2)], ln1 = cl[at_most(c + 2)];
+            fetch(st0, ln0);
+            const float keep = at[buf];
+#pragma unroll
+            for (int i = 0; i < JW; ++i)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) S[i][ct] *= keep;
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                const f32x4_t w4 = *reinterpret_cast<const f32x4_t*>(&ws[buf][16 * st + 4 * g]);
+                f32x4_t y[CT];
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+                    y[ct] = *reinterpret_cast<const f32x4_t*>(&vt[buf][(16 * ct + r) * SV + 16 * st + 4 * g]) * w4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < JW; ++i)
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) MV_MFMA4(S[i][ct], now[4 * i + st][e], y[ct][e]);
+            }
+            publish(buf ^ 1);
+            stage(buf ^ 1, ln0);
+            fetch_v(st1, ln1);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < JW; ++i)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sp[(int64_t)(j0 + 16 * i + 4 * g + j) * a.p + 16 * ct + r] = S[i][ct][j];
+    }
+}
+
 // ---- the gated recurrence in chunks of 64 tokens ----
 // Within a chunk that starts from state S0, with P_t[i] the product of the gates f_s[i] over the chunk's tokens
 // s <= t:  o_t = (local run from a zero state)_t + sum_i q_t[i] P_t[i] S0[i][:],  S_end = diag(P_end) S0 + local.
@@ -2132,6 +2375,26 @@ int mv_scan_chunked(const float* q, int64_t ldq, int q_div, const float* k, int6
     a.ch_start = ch_start; a.ch_len = ch_len; a.row_ch0 = row_ch0; a.row_nch = row_nch;
     a.r = StepRows{nullptr, nullptr, nullptr, nullptr, row_ctx, row_slot};
     a.H = heads; a.n = n; a.p = p;
+    // Whole rows in two launches where the shapes allow it and there are sixteen heads: a row's chunks come one after the
+    // other there (about 3.5 us each), the three launches below take them side by side (about 0.2 us per chunk and head).
+    const int groups = heads / q_div;
+    if ((n == 64 || n == 128) && p % 16 == 0 && q_div == k_div && heads % q_div == 0 && ldq % 4 == 0 && ldk % 4 == 0 &&
+        ldv % 4 == 0 && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(ds) &&
+        (int64_t)groups * kCh * kCh <= (int64_t)heads * n * p && groups <= 65535 && heads >= 16 &&
+        (int64_t)heads * (p / 16) <= 0x7fffffff) {
+        hipStream_t s = (hipStream_t)stream;
+        hipLaunchKernelGGL(scan_scores_kernel, dim3(chunks, groups, 4), dim3(256), 0, s, a, ds);
+        const bool wide = p % 32 == 0 && (int64_t)heads * (p / 32) * rows >= num_cus();
+        const dim3 grid((unsigned)(heads * (p / (wide ? 32 : 16))), rows);
+        if (n == 64) {
+            if (wide) hipLaunchKernelGGL((scan_rows_kernel<4, 2>), grid, dim3(512), 0, s, a, ds, groups);
+            else hipLaunchKernelGGL((scan_rows_kernel<4, 1>), grid, dim3(512), 0, s, a, ds, groups);
+        } else {
+            if (wide) hipLaunchKernelGGL((scan_rows_kernel<8, 2>), grid, dim3(512), 0, s, a, ds, groups);
+            else hipLaunchKernelGGL((scan_rows_kernel<8, 1>), grid, dim3(512), 0, s, a, ds, groups);
+        }
+        return check_launch();
+    }
     // heads that read the same q and k (a group) go four or two to a workgroup
     a.hb = (q_div == k_div && heads % q_div == 0) ? (q_div % 4 == 0 ? 4 : (q_div % 2 == 0 ? 2 : 1)) : 1;
     hipStream_t s = (hipStream_t)stream;

@@ -366,3 +366,9 @@ def test_distance_penalty_is_per_head_and_in_distance(ops):
             js = torch.arange(max(0, i - window + 1), i + 1).double()
             p = torch.softmax(-slopes[h] * (i - js), 0)
             assert abs(out[i, h, 0].item() - (p * js).sum().item()) < 1e-3
+
+
+@pytest.mark.parametrize("H,G,n,p", [(16, 16, 128, 64), (32, 2, 64, 48), (17, 1, 64, 16), (128, 1, 64, 64), (128, 2, 128, 64)])
+def test_scan_of_whole_rows_equals_token_by_token(ops, H, G, n, p):
+    """The two-launch form (n of 64 or 128, sixteen heads and more): both state heights, column slices of 16 and of 32."""
+    test_scan_in_chunks_equals_token_by_token(ops, H, G, n, p)
