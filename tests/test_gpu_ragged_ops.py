@@ -372,3 +372,54 @@ def test_distance_penalty_is_per_head_and_in_distance(ops):
 def test_scan_of_whole_rows_equals_token_by_token(ops, H, G, n, p):
     """The two-launch form (n of 64 or 128, sixteen heads and more): both state heights, column slices of 16 and of 32."""
     test_scan_in_chunks_equals_token_by_token(ops, H, G, n, p)
+
+
+@pytest.mark.parametrize("C,taps", [(4, 4), (1028, 4), (8448, 4), (260, 3), (64, 2), (24, 5), (30, 4)])
+def test_conv_silu_forms(ops, C, taps):
+    """Runs of eight tokens over several rows in one step (row starts inside a run, rows shorter than the taps), then one
+    token a row, then both again: the same sums in the same order, so every output is the plain form's to its last bits
+    (1e-5 covers the exponential against 64 bits)."""
+    g = torch.Generator().manual_seed(C)
+    lens = {"a": 21, "b": 2, "c": 9, "d": 64}
+    x = {k: torch.randn(2 * n + 4, C, generator=g) for k, n in lens.items()}
+    w, b = torch.randn(C, taps, generator=g), torch.randn(C, generator=g)
+    want = {k: ref.causal_conv_silu(v.double(), w.double(), b.double()) for k, v in x.items()}
+    cache = make_cache(state={0: {"conv": (taps - 1, C)}}, slots=6)
+    cache.admit("other")
+    cache.states[0]["conv"].fill_(7.0)
+    pos = {k: 0 for k in lens}
+    for step_lens in (lens, {k: 1 for k in lens}, {k: 1 for k in lens}, {"c": 3, "a": 1}, {"b": 1}, {"a": 19, "b": 2, "c": 4, "d": 63}):
+        st = step_of(cache, [(k, [0] * n) for k, n in step_lens.items()])
+        inp = torch.cat([x[k][pos[k]:pos[k] + n] for k, n in step_lens.items()])
+        o = torch.full(inp.shape, float("nan"), device=DEV)
+        ops.conv_silu(inp.to(DEV), cache.states[0]["conv"], w.to(DEV), b.to(DEV), o, st)
+        at = 0
+        for k, n in step_lens.items():
+            assert (o[at:at + n].cpu().double() - want[k][pos[k]:pos[k] + n]).abs().max().item() < 1e-5, (k, pos[k], n)
+            at, pos[k] = at + n, pos[k] + n
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("rows,n,groups", [(1, 8192, 1), (300, 8192, 1), (3, 1024, 1), (2, 4104, 2), (260, 2052, 2), (1, 33000, 1),
+                                           (300, 9000, 1), (5, 1026, 1)])
+def test_gated_group_norm_of_wide_groups(ops, rows, n, groups, f32):
+    """Values in registers (1024 and 256 threads, one to eight pieces each, the last partly past the end) and the looped form
+    (groups too wide or not in fours), for the three modes, with a weight of a group and of a row."""
+    g = torch.Generator().manual_seed(n + rows)
+    y, z = torch.randn(rows, n, generator=g) * 4, torch.randn(rows, n + 4, generator=g)
+    dt, eps = torch.float32 if f32 else torch.bfloat16, 1e-5
+    for mode, wn in ((0, n), (1, n), (2, n // groups), (0, 0)):
+        w = torch.randn(wn, generator=g) if wn else None
+        out = torch.empty(rows, n, dtype=dt, device=DEV)
+        ops.gated_group_norm(y.to(DEV), z.to(DEV)[:, :n], None if w is None else w.to(DEV), out, groups, mode == 1, eps,
+                             sigmoid=mode == 2)
+        zd = z[:, :n].double()
+        gate = torch.sigmoid(zd) if mode == 2 else zd * torch.sigmoid(zd)
+        u = y.double() * gate if mode == 1 else y.double()
+        want = ref.unit_rms(u.view(rows, groups, -1), eps).reshape(rows, n)
+        if mode != 1:
+            want = want * gate
+        if w is not None:
+            want = want * (w.double() if wn == n else w.double().repeat(groups))
+        tol = (1e-5 if f32 else 2 ** -8) * want.abs() + 1e-6       # fp32 products, a rounding to the output's type
+        assert ((out.cpu().double() - want).abs() <= tol).all(), mode
