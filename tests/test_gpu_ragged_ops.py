@@ -423,3 +423,9 @@ def test_gated_group_norm_of_wide_groups(ops, rows, n, groups, f32):
             want = want * (w.double() if wn == n else w.double().repeat(groups))
         tol = (1e-5 if f32 else 2 ** -8) * want.abs() + 1e-6       # fp32 products, a rounding to the output's type
         assert ((out.cpu().double() - want).abs() <= tol).all(), mode
+
+
+@pytest.mark.parametrize("H,G,n,p", [(4, 2, 64, 64), (3, 1, 128, 128), (3, 3, 256, 64), (2, 1, 64, 192)])
+def test_scan_token_by_token_in_whole_pieces(ops, H, G, n, p):
+    """The form that reads state, q, k and v in 16-byte pieces: its three state heights, one to three column tiles."""
+    test_scan_whole_portions_and_rows(ops, H, G, n, p)
