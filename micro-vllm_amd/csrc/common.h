@@ -134,7 +134,7 @@ struct PostNorm {
 int launch_wgemm_finalize_norm(float* partial, int ksplit, int m, int n, const void* bias, PostNorm* norm, hipStream_t s);
 bool wgemm_finalize_norm_takes(int n);
 // wgemm.hip: a projection of up to 64 rows whose sums are those of `ks` slices of k added in order
-bool wgemm_ordered_takes(int m, int kt, int ks);
+bool wgemm_ordered_takes(int m, int nt, int kt, int ks);
 int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
                          int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int ks, int flags, PostNorm* norm,
                          hipStream_t s);

@@ -22,13 +22,13 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mv {
 
 constexpr int kPM = 128;            // rows of x per workgroup
 constexpr int kPN = 256;            // output columns per workgroup
 constexpr int kPK = 64;             // k per LDS stage
-constexpr int kPStage = kPM * kPK * 2; // bytes of one x stage in LDS
 constexpr int kPMT = kPM / 16;      // m-tiles per wave
 constexpr int kPNT = 4;             // n-tiles per wave
 constexpr int kWSlotBytes = 8 * 32 * 64 * 16;   // a workgroup's accumulators: 8 waves x 32 registers of 16 bytes x 64 lanes
@@ -133,8 +133,8 @@ __device__ __forceinline__ float silu_mul_rounded_quick(float gate_acc, float up
     const float sig = __builtin_amdgcn_rcpf(1.0f + e);
     return (g * sig) * u;
 }
-template <int NT>
-__device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_t (&acc)[NT][kPMT], int nt0,
+template <int NT, int MT>
+__device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_t (&acc)[NT][MT], int nt0,
                                                 int m0, int ks, int r, int q, const unsigned char* lower = nullptr,
                                                 int nlower = 0) {
     const bool sw = (a.flags & MV_GEMM_SWIGLU) != 0, of32 = (a.flags & MV_GEMM_OUT_F32) != 0;
@@ -155,7 +155,7 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
     };
     if (a.partial) {
 #pragma unroll
-        for (int t = 0; t < kPMT; ++t) {
+        for (int t = 0; t < MT; ++t) {
             MV_EPI_FENCE;
             const int m = m0 + t * 16 + r;
             float* const row = a.partial + ((int64_t)ks * a.m + min(m, a.m - 1)) * a.n + nt0 * 16 + q * 4;
@@ -177,7 +177,7 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
         // dword stores covered 16.
         const bool whole = (a.ldy % 8) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
 #pragma unroll
-        for (int t = 0; t < kPMT; ++t) {
+        for (int t = 0; t < MT; ++t) {
             MV_EPI_FENCE;
             const int m = m0 + t * 16 + r;
             uint16_t* const row = reinterpret_cast<uint16_t*>(a.y) + (int64_t)min(m, a.m - 1) * a.ldy + nt0 * 8;
@@ -212,7 +212,7 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
     }
     if (of32) {
 #pragma unroll
-        for (int t = 0; t < kPMT; ++t) {
+        for (int t = 0; t < MT; ++t) {
             MV_EPI_FENCE;
             const int m = m0 + t * 16 + r;
             float* const row = reinterpret_cast<float*>(a.y) + (int64_t)min(m, a.m - 1) * a.ldy + nt0 * 16 + q * 4;
@@ -244,7 +244,7 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
     // store instruction then covers 64 contiguous bytes of each of its 16 rows instead of 32.
     const bool pairs = (a.ldy % 8) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
 #pragma unroll
-    for (int t = 0; t < kPMT; ++t) {
+    for (int t = 0; t < MT; ++t) {
         MV_EPI_FENCE;
         const int m = m0 + t * 16 + r, mc = min(m, a.m - 1);
         uint16_t* const row = reinterpret_cast<uint16_t*>(a.y) + (int64_t)mc * a.ldy + nt0 * 16;
@@ -273,8 +273,16 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
     }
 }
 
-__global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(PGemmArgs a) {
-    __shared__ __attribute__((aligned(16))) unsigned char xs[3][kPStage];
+// MT m-tiles per wave (128 or 64 rows a workgroup), RING k-tiles of weights in registers and BUFS stages of x in LDS.
+// 8, 3, 3: two workgroups to a compute unit hide each other's trips to memory.  RING 8, BUFS 4: for grids of at most one
+// workgroup to a unit, whose waves have the registers to themselves; with two k-tiles ahead a stage of 64 k takes 1.1 us
+// there.  The 64-row tile halves what a wave multiplies per stage and doubles the workgroups.  Sums do not depend on it.
+template <int MT, int RING, int BUFS>
+__global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefill_kernel(PGemmArgs a) {
+    constexpr int kStage = MT * 16 * kPK * 2, XP = MT / 2;   // bytes of a stage of x, pieces of it a wave requests
+    constexpr int kPeriod = RING == 3 ? 3 : RING / 2;     // stages after which slots and buffers repeat
+    static_assert((2 * kPeriod) % RING == 0 && kPeriod % BUFS == 0, "slots and buffers repeat together");
+    __shared__ __attribute__((aligned(16))) unsigned char xs[BUFS][kStage];
 
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -289,7 +297,7 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(PGemmArgs a) {
     const int nb = xcd * a.nb_per_xcd + idx / a.mblocks;
     const int mb = idx % a.mblocks;
     if (nb >= a.nblocks || idx / a.mblocks >= a.nb_per_xcd) return;
-    const int m0 = mb * kPM;
+    const int m0 = mb * (16 * MT);
     const int nt0 = nb * (kPN / 16) + wid * kPNT;
 
     // weight fragment streams of this wave (strips past the end are clamped and never stored)
@@ -298,7 +306,7 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(PGemmArgs a) {
     for (int i = 0; i < kPNT; ++i)
         wp[i] = a.w + ((int64_t)min(nt0 + i, a.nt - 1) * a.kt + kt0) * 64 + lane;
 
-    // ---- x: global -> LDS directly, three stages deep, in fragment order ---------------------
+    // ---- x: global -> LDS directly, BUFS stages deep, in fragment order ---------------------
     // The LDS image of a stage is 16 fragment tiles (8 m-tiles x 2 k-tiles) of 1 KiB in MFMA
     // operand order: lane l of the tile (mt, kk) holds x[16 mt + (l & 15)][32 kk + 8 (l >> 4) ..+7],
     // so a fragment read is linear in the lane (no bank conflicts).  Wave w fills tiles 4w..4w+3
@@ -308,19 +316,19 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(PGemmArgs a) {
     // hidden from it they only make its counted waits wait for more (requests complete in
     // order), never for less.  The wait that makes the data usable is placed by hand.
     const int nstage = a.ktps >> 1;  // a slice is a multiple of 64 k (checked on the host)
-    const uint16_t* xg[4];
+    const uint16_t* xg[XP];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int tile = wid * 4 + j;
+    for (int j = 0; j < XP; ++j) {
+        const int tile = wid * XP + j;
         xg[j] = a.x + (int64_t)min(m0 + (tile >> 1) * 16 + r, a.m - 1) * a.ldx + kt0 * 32 + ((tile & 1) * 4 + q) * 8;
     }
     const unsigned xs_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)&xs[0][0];
     auto x_fetch = [&](int s, int buf) {
         const int sc = min(s, nstage - 1);  // past the end: a harmless re-fetch keeps the counts fixed
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < XP; ++j) {
             const uint16_t* src = xg[j] + sc * kPK;
-            const unsigned dst = xs_base + buf * kPStage + (wid * 4 + j) * 1024;
+            const unsigned dst = xs_base + buf * kStage + (wid * XP + j) * 1024;
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(dst) : "memory");
         }
     };
@@ -332,57 +340,59 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(PGemmArgs a) {
             bf16x8_t, *reinterpret_cast<const uint4*>(&xs[buf][(t * 2 + kk) * 1024 + lane * 16]));
     };
 
-    f32x4_t acc[kPNT][kPMT];
+    f32x4_t acc[kPNT][MT];
 #pragma unroll
     for (int i = 0; i < kPNT; ++i)
 #pragma unroll
-        for (int t = 0; t < kPMT; ++t) acc[i][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < MT; ++t) acc[i][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
-    // weight fragments: a ring of three k-tiles; a slot is refilled (two k-tiles ahead) at the start
-    // of the k-tile after the one that used it
-    uint4 wA[kPNT], wB[kPNT], wC[kPNT];
-    auto w_load = [&](uint4(&w)[kPNT], int kt) {
+    // weight fragments: a ring of k-tiles; a slot is refilled (RING - 1 k-tiles ahead) at the start of the k-tile after the
+    // one that used it
+    uint4 w[RING][kPNT];
+    auto w_load = [&](uint4(&wr)[kPNT], int kt) {
         const int ktc = min(kt, a.ktps - 1);
 #pragma unroll
         for (int i = 0; i < kPNT; ++i) {
 #ifdef MV_EXP_NO_WLOAD
             if (kt > 2) continue;  // timing experiment only: weights never refreshed
 #endif
-            w[i] = ld16(wp[i] + (int64_t)ktc * 64);
+            wr[i] = ld16(wp[i] + (int64_t)ktc * 64);
         }
     };
-    x_fetch(0, 0);
-    x_fetch(1, 1);
-    w_load(wA, 0);
-    w_load(wB, 1);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < BUFS - 1; ++i) x_fetch(i, i);
+#pragma unroll
+    for (int i = 0; i < RING - 1; ++i) w_load(w[i], i);
+    // the first two stages of x (the weights behind them may still be on their way)
+    wait_vmcnt<RING == 3 ? 0 : XP * (BUFS - 3) + kPNT * (RING - 1)>();
+    asm volatile("" ::: "memory");
     __syncthreads();
 
     // x fragments of two k-tiles alternate between X0 and X1; the first half of a k-tile's
     // fragments is read while the previous k-tile is still being multiplied
-    bf16x8_t X0[kPMT], X1[kPMT];
+    bf16x8_t X0[MT], X1[MT];
 #pragma unroll
-    for (int t = 0; t < kPMT / 2; ++t) X0[t] = x_frag(0, t, 0);
+    for (int t = 0; t < MT / 2; ++t) X0[t] = x_frag(0, t, 0);
 
     // one k-tile: (buf, kk) = where it lives; (nbuf, nkk) = the k-tile after it
-    // `w` = this k-tile's weight fragments; `wr` = the ring slot the previous k-tile used, refilled
-    // here, first thing, with the k-tile two ahead (left to itself the scheduler sinks these
+    // `wc` = this k-tile's weight fragments; `wr` = the ring slot the previous k-tile used, refilled
+    // here, first thing, with the k-tile RING - 1 ahead (left to itself the scheduler sinks these
     // requests to the end of the stage, and the next stage then starts by waiting for them).
     // `fetch_stage` >= 0: also request that stage of x, after the first half of the MFMAs.
-    auto ktile = [&](uint4(&w)[kPNT], uint4(&wr)[kPNT], bf16x8_t(&xc)[kPMT], bf16x8_t(&xn)[kPMT], int buf,
+    auto ktile = [&](uint4(&wc)[kPNT], uint4(&wr)[kPNT], bf16x8_t(&xc)[MT], bf16x8_t(&xn)[MT], int buf,
                      int kk, int nbuf, int nkk, int kt_refill, int fetch_stage, int fetch_buf) {
         bf16x8_t wf[kPNT];
 #pragma unroll
-        for (int i = 0; i < kPNT; ++i) wf[i] = __builtin_bit_cast(bf16x8_t, w[i]);
+        for (int i = 0; i < kPNT; ++i) wf[i] = __builtin_bit_cast(bf16x8_t, wc[i]);
         __builtin_amdgcn_sched_barrier(0);
         w_load(wr, kt_refill);
         __builtin_amdgcn_sched_barrier(0);
         // (pinning this order with scheduling fences measured 3 % slower than letting the
         // scheduler interleave reads and MFMAs itself)
 #pragma unroll
-        for (int t = kPMT / 2; t < kPMT; ++t) xc[t] = x_frag(buf, t, kk);
+        for (int t = MT / 2; t < MT; ++t) xc[t] = x_frag(buf, t, kk);
 #pragma unroll
-        for (int t = 0; t < kPMT / 2; ++t)
+        for (int t = 0; t < MT / 2; ++t)
 #pragma unroll
             for (int i = 0; i < kPNT; ++i)
                 MV_MFMA(acc[i][t], wf[i], xc[t]);
@@ -395,41 +405,46 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill_kernel(PGemmArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int t = 0; t < kPMT / 2; ++t) xn[t] = x_frag(nbuf, t, nkk);
+        for (int t = 0; t < MT / 2; ++t) xn[t] = x_frag(nbuf, t, nkk);
 #pragma unroll
-        for (int t = kPMT / 2; t < kPMT; ++t)
+        for (int t = MT / 2; t < MT; ++t)
 #pragma unroll
             for (int i = 0; i < kPNT; ++i)
                 MV_MFMA(acc[i][t], wf[i], xc[t]);
     };
-    // One stage: request stage s+2 of x (its buffer was last read in stage s-1), two k-tiles, wait
-    // for this wave's part of stage s+2 (two weight refills were requested after it), barrier: the
-    // next stage's later reads and the stage after's early reads both see complete data.
-    auto stage = [&](uint4(&w0)[kPNT], uint4(&w1)[kPNT], uint4(&w2)[kPNT], int s, int b0, int b1, int b2) {
+    // One stage, I = s mod kPeriod: request stage s + BUFS - 1 of x (its buffer was last read in stage s - 1), two k-tiles,
+    // wait for this wave's part of stage s + 2, barrier: the next stage's later reads and the stage after's early reads
+    // both see complete data.
+    auto stage = [&](auto index, int s) {
+        constexpr int I = decltype(index)::value, b0 = I % BUFS, b1 = (I + 1) % BUFS;
         MV_STAMP(0);
-        ktile(w0, w2, X0, X1, b0, 0, b0, 1, 2 * s + 2, s + 2, b2);
-        ktile(w1, w0, X1, X0, b0, 1, b1, 0, 2 * s + 3, -1, 0);
+        ktile(w[2 * I % RING], w[(2 * I + RING - 1) % RING], X0, X1, b0, 0, b0, 1, 2 * s + RING - 1, s + BUFS - 1,
+              (I + BUFS - 1) % BUFS);
+        ktile(w[(2 * I + 1) % RING], w[2 * I % RING], X1, X0, b0, 1, b1, 0, 2 * s + RING, -1, 0);
         MV_STAMP(1);
-        wait_vmcnt<kPNT>();   // only the second k-tile's refill was requested after the x stage
+        // requested after that stage of x: the refill behind it and, per stage since, two refills and four pieces of x
+        wait_vmcnt<kPNT + (BUFS - 3) * (2 * kPNT + XP)>();
         MV_STAMP(2);
 #ifndef MV_EXP_NO_BARRIER
         __syncthreads();
 #endif
         MV_STAMP(3);
     };
-    // three stages per pass and no branch inside the pass (a branch between stages makes the
-    // compiler wait for every outstanding request where the paths meet); the one or two stages
-    // left over follow
+    // kPeriod stages per pass and no branch inside the pass (a branch between stages makes the
+    // compiler wait for every outstanding request where the paths meet); the stages left over follow
     int s = 0;
-    for (; s + 2 < nstage; s += 3) {
-        stage(wA, wB, wC, s, 0, 1, 2);
-        stage(wC, wA, wB, s + 1, 1, 2, 0);
-        stage(wB, wC, wA, s + 2, 2, 0, 1);
+    for (; s + kPeriod <= nstage; s += kPeriod) {
+        stage(std::integral_constant<int, 0>{}, s);
+        stage(std::integral_constant<int, 1>{}, s + 1);
+        stage(std::integral_constant<int, 2>{}, s + 2);
+        if constexpr (kPeriod == 4) stage(std::integral_constant<int, 3>{}, s + 3);
     }
-    if (s < nstage) stage(wA, wB, wC, s, 0, 1, 2);
-    if (s + 1 < nstage) stage(wC, wA, wB, s + 1, 1, 2, 0);
+    if (s < nstage) stage(std::integral_constant<int, 0>{}, s);
+    if (s + 1 < nstage) stage(std::integral_constant<int, 1>{}, s + 1);
+    if (kPeriod == 4 && s + 2 < nstage) stage(std::integral_constant<int, 2>{}, s + 2);
+    wait_vmcnt<0>();     // no request into LDS outlives the workgroup
 
-    store_wave_tile(a, acc, nt0, m0, ks, r, q);
+    store_wave_tile<kPNT, MT>(a, acc, nt0, m0, ks, r, q);
 }
 
 
@@ -782,7 +797,7 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
                 nlower = cur.parts - 1;
             }
             if (cur.ntb + wcol < a.nt)
-                store_wave_tile<NT>(a, acc, cur.ntb + wcol, cur.m0 + wm * 128, cur.ks, r, q, lower, nlower);
+                store_wave_tile<NT, kPMT>(a, acc, cur.ntb + wcol, cur.m0 + wm * 128, cur.ks, r, q, lower, nlower);
         }
 #endif
         MV_WSTAMP(g0 + nkt + 1);
@@ -1075,7 +1090,7 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     // Up to 64 rows a tile of 128 is mostly padding, and its slices are written out and added up by a second launch.  The
     // single-token projections' kernel walks the same slices one to a wave and adds them in the workgroup, same sums in
     // the same order (the rule and what it measured: wgemm_ordered_takes).
-    if (!wide && wgemm_ordered_takes(m, a.kt, a.ksplit))
+    if (!wide && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit))
         return launch_wgemm_ordered(x, ldx, w_tiles, bias, residual, ld_res, y, ldy, m, n, k, a.ksplit, flags, norm,
                                     (hipStream_t)stream);
     auto reduce = [&] {
@@ -1125,7 +1140,21 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     }
     const long grid = 8L * a.nb_per_xcd * a.mblocks * a.ksplit;
     if (grid > 0x7fffffffL) return MV_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(gemm_prefill_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
+    // 64-row tiles while each has a compute unit to itself, else 128-row tiles in the deep form (from 16 stages: shorter
+    // slices end before its ring has paid), else two workgroups to a unit.  Measured against the last (us): 512 x 6144 x 2048
+    // 44.8 -> 28.3 and 256 x 16384 x 2048 47.2 -> 31.9 in 64-row tiles, 1408 x 2048 x 2048 39.0 -> 24.0, 1024 x 4096 x 4096 in
+    // two slices 54.4 -> 49.7 in the deep form (64-row tiles in two rounds: 61.3), 192 x 6144 x 2048 in four 24.8 as it was
+    // (deep 25.4, 64 rows 29.1).
+    const int mblocks64 = (m + 63) / 64;
+    const long grid64 = 8L * a.nb_per_xcd * mblocks64 * a.ksplit;
+    if (grid64 <= num_cus()) {
+        a.mblocks = mblocks64;
+        hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4>), dim3((unsigned)grid64), dim3(256), 0, (hipStream_t)stream, a);
+    } else if (grid <= num_cus() && a.ktps >= 32) {
+        hipLaunchKernelGGL((gemm_prefill_kernel<8, 8, 4>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
+    } else {
+        hipLaunchKernelGGL((gemm_prefill_kernel<8, 3, 3>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
+    }
     int rc = check_launch();
     if (rc != MV_OK || a.ksplit == 1) return rc;
     return reduce();

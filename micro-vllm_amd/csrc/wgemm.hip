@@ -1000,14 +1000,15 @@ static int launch_ordered_mb(const GemmArgs& a, int sg, int ks, int grid, hipStr
     }
 }
 
-// One block of rows (up to 16), or few k-tiles times blocks: a wave walks its slice alone, and past that its chain of loads
-// is longer than the sliced tiles' two launches.  Measured at 37 rows (n x k, us, sliced tiles -> here): 2560 x 2048
-// 12.5 -> 9.0, 11264 x 2048 19.9 -> 17.8, 6144 x 4096 20.5 -> 18.9, 8192 x 1024 13.3 -> 8.9, but 1280 x 8192 16.5 -> 24.8
-// and 4096 x 14336 33.8 -> 46.5; at 64 rows 2560 x 2048 14.2 -> 12.5 and 4096 x 4096 19.6 -> 23.7; at 5 rows all are
-// faster here, 17.1 -> 9.4 (2048 x 5632) to 31.7 -> 21.9 (4096 x 14336).
-bool wgemm_ordered_takes(int m, int kt, int ks) {
+// One block of rows (up to 16), or few k-tiles times blocks on enough strips: a wave walks its slice alone, and past that its
+// chain of loads, or on many strips the x each of them reads again, is longer than the sliced tiles and their reduction.
+// Measured (n x k, us, sliced tiles -> here): 5 rows 2048 x 5632 13.6 -> 9.5, 4096 x 14336 31.6 -> 22.4;
+// 37 rows 2560 x 2048 11.7 -> 9.0, 6144 x 4096 19.1 -> 17.9, 8192 x 1024 12.6 -> 8.8, but 1024 x 4096 12.1 -> 14.6,
+// 1280 x 8192 15.2 -> 24.8 and 4096 x 14336 34.0 -> 46.5; 64 rows 2560 x 2048 14.0 -> 12.2, 11264 x 2048 20.3 -> 23.7.
+bool wgemm_ordered_takes(int m, int nt, int kt, int ks) {
     const int blocks = (m + 15) / 16;
-    return (ks == 4 || ks == 8 || ks == 16) && blocks <= 4 && (blocks == 1 || blocks * kt <= 384);
+    if ((ks != 4 && ks != 8 && ks != 16) || blocks > 4) return false;
+    return blocks == 1 || (blocks * kt <= 384 && nt >= 128 && (int64_t)blocks * kt * nt <= 150000);
 }
 
 // x [m, k] . W^T with the sums of `ks` slices of k added in order, epilogue as mv_gemm_prefill_ws, or the norm's.

@@ -444,3 +444,32 @@ def test_few_rows_add_the_slices_in_order(mv, m, n, k, mode):
     for addend in (bias, res):
         want = want if addend is None else (want.float() + addend.float()).to(torch.bfloat16)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m,n,k,mode", [(65, 6144, 2048, "bias"), (129, 16384, 1024, "swiglu"), (512, 4112, 2048, "residual"),
+                                        (700, 2048, 64, "plain"), (700, 2048, 320, "f32"), (1000, 2048, 832, "plain"),
+                                        (1000, 4096, 4096, "residual"), (768, 8192, 2048, "plain")])
+def test_tiles_of_64_and_128_rows_give_the_same_sums(mv, m, n, k, mode):
+    """Grids of less than a workgroup to a compute unit take 64-row tiles or the deep form (remainders of its pass of four
+    stages: k of 64, 320, 832); the same rows inside a product of many take 128-row tiles.  The sums have the same order
+    wherever neither is cut along k."""
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.linear import StreamedWeight
+
+    x, w, g = _mk(m, n, k, seed=m + n + k, scale=0.03)
+    sw = (StreamedWeight.from_up_gate(w[:n // 2].to(DEV), w[n // 2:].to(DEV)) if mode == "swiglu"
+          else StreamedWeight.from_linear(w.to(DEV)))
+    ncols, dt = sw.out_features, torch.float32 if mode == "f32" else torch.bfloat16
+    flags = (nv.MV_GEMM_SWIGLU if mode == "swiglu" else 0) | (nv.MV_GEMM_OUT_F32 if mode == "f32" else 0)
+    bias = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if mode == "bias" else None
+    reps = 4096 // m + 1
+    xd, res = x.to(DEV), torch.randn(m, n, generator=g).to(torch.bfloat16).to(DEV) if mode == "residual" else None
+    outs = []
+    for r in (1, reps):      # without a workspace: k whole in both
+        xr, rr = xd.repeat(r, 1), None if res is None else res.repeat(r, 1)
+        y = torch.full((m * r, ncols), float("nan"), dtype=dt, device=DEV)
+        nv.check("mv_gemm_prefill", nv.lib().mv_gemm_prefill(
+            xr.data_ptr(), k, sw.tiles.data_ptr(), nv.ptr(bias), nv.ptr(rr), n if rr is not None else 0, y.data_ptr(), ncols,
+            m * r, n, k, flags, nv.stream_ptr()))
+        outs.append(y)
+    assert torch.equal(outs[0], outs[1][:m]) and torch.equal(outs[0], outs[1][-m:])
