@@ -416,3 +416,9 @@ def test_arguments_outside_the_kernels_limits_are_refused(ops):
         run_delta(ops, {"a": d}, par, [[("a", 4)]], K, H, n, p, 1e-5)
     with pytest.raises(AssertionError):
         run_delta(ops, {"a": delta_inputs(4, 2, 3, 16, 8)[0]}, delta_inputs(4, 2, 3, 16, 8)[1], [[("a", 4)]], 2, 3, 16, 8, 1e-5)
+
+
+@pytest.mark.parametrize("K,H,n,p", [(2, 4, 128, 128), (1, 2, 64, 128), (3, 3, 128, 64), (2, 2, 64, 64)])
+def test_delta_rule_in_whole_pieces(ops, K, H, n, p):
+    """The token-by-token form that holds state in 16-byte pieces, its four head shapes."""
+    test_delta_rule_over_steps(ops, K, H, n, p)
