@@ -693,23 +693,29 @@ __global__ __launch_bounds__(256) void wgemm_finalize_kernel(GemmArgs a) {
 // Chunk assignment and summation order are those of the stand-alone norm kernels (256 threads,
 // stride 256, block_sum), so the fused and the separate path agree bit for bit.
 constexpr int kPostChunks = 4;  // 16-byte chunks of y a thread keeps: rows up to 8192 wide
-__global__ __launch_bounds__(256) void wgemm_finalize_norm_kernel(GemmArgs a) {
-    __shared__ float red[256 / 64];
+// NT = 256 holds up to four chunks a thread; NT = 512 and 1024, for a few rows, one: a row's slabs then come in through more
+// requests at a time, and the first 256 threads add the squares out of LDS in the order of NT = 256, so the norm is the same
+// bit for bit.  8 rows of 8192 6.5 -> 4.9 us, 32 rows of 4096 5.2 -> 4.8; more rows than compute units keep 256.
+template <int NT>
+__global__ __launch_bounds__(NT) void wgemm_finalize_norm_kernel(GemmArgs a) {
+    constexpr int CH = NT == 256 ? kPostChunks : 1;
+    __shared__ float red[NT / 64];
+    __shared__ __attribute__((aligned(16))) float sq[NT == 256 ? 4 : NT * 8];
     const int m = blockIdx.x;
     const int nvec = a.n >> 3;
-    uint4 keep[kPostChunks];
+    uint4 keep[CH];
     float ss = 0.f;
     // Every operand of every chunk is requested before the first is used - the first kPostAhead slabs
     // included (the usual splits are 2 and 4): the slabs were written by another kernel, so each
     // dependent round of loads is a trip to memory, and this kernel is nothing but such trips.
     // (Chunk rows and slabs that do not exist are skipped: both conditions are uniform.)
     constexpr int kPostAhead = 4;
-    f32x4_t p_lo[kPostChunks][kPostAhead], p_hi[kPostChunks][kPostAhead];
-    uint4 b_in[kPostChunks], r_in[kPostChunks], w_in[kPostChunks];
+    f32x4_t p_lo[CH][kPostAhead], p_hi[CH][kPostAhead];
+    uint4 b_in[CH], r_in[CH], w_in[CH];
 #pragma unroll
-    for (int j = 0; j < kPostChunks; ++j) {
-        if (j * 256 >= nvec) break;
-        const int n0 = min(threadIdx.x + j * 256, nvec - 1) * 8;
+    for (int j = 0; j < CH; ++j) {
+        if (j * NT >= nvec) break;
+        const int n0 = min(threadIdx.x + j * NT, nvec - 1) * 8;
 #pragma unroll
         for (int ks = 0; ks < kPostAhead; ++ks) {
             if (ks >= a.ksplit) break;
@@ -722,8 +728,8 @@ __global__ __launch_bounds__(256) void wgemm_finalize_norm_kernel(GemmArgs a) {
         w_in[j] = ld16(a.post_ln_w + n0);
     }
 #pragma unroll
-    for (int j = 0; j < kPostChunks; ++j) {
-        const int c = threadIdx.x + j * 256;
+    for (int j = 0; j < CH; ++j) {
+        const int c = threadIdx.x + j * NT;
         if (c < nvec) {
             const int n0 = c * 8;
             f32x4_t lo = (f32x4_t){0.f, 0.f, 0.f, 0.f}, hi = lo;
@@ -760,18 +766,37 @@ __global__ __launch_bounds__(256) void wgemm_finalize_norm_kernel(GemmArgs a) {
                     s0 = bf16_lo(o[e]);
                     s1 = bf16_hi(o[e]);
                 }
-                ss += s0 * s0;
-                ss += s1 * s1;
+                if (NT == 256) {
+                    ss += s0 * s0;
+                    ss += s1 * s1;
+                } else {
+                    *reinterpret_cast<float2*>(&sq[c * 8 + 2 * e]) = make_float2(s0 * s0, s1 * s1);
+                }
             }
             keep[j] = make_uint4(o[0], o[1], o[2], o[3]);
             st16(reinterpret_cast<uint16_t*>(a.y) + (int64_t)m * a.ldy + n0, keep[j]);
         }
     }
-    const float total = block_sum(ss, red);
+    if (NT > 256) {
+        __syncthreads();
+        if (threadIdx.x < 256)
+            for (int c = threadIdx.x; c < nvec; c += 256) {
+                const float4 x = *reinterpret_cast<const float4*>(&sq[c * 8]), y = *reinterpret_cast<const float4*>(&sq[c * 8 + 4]);
+                ss += x.x;
+                ss += x.y;
+                ss += x.z;
+                ss += x.w;
+                ss += y.x;
+                ss += y.y;
+                ss += y.z;
+                ss += y.w;
+            }
+    }
+    const float total = block_sum(ss, red);     // (waves past the fourth add zero)
     const float rrms = 1.0f / sqrtf(total / (float)a.n + a.post_eps);
 #pragma unroll
-    for (int j = 0; j < kPostChunks; ++j) {
-        const int c = threadIdx.x + j * 256;
+    for (int j = 0; j < CH; ++j) {
+        const int c = threadIdx.x + j * NT;
         if (c < nvec) {
             const uint4 wv = w_in[j];
             const uint32_t s4[4] = {keep[j].x, keep[j].y, keep[j].z, keep[j].w};
@@ -784,6 +809,14 @@ __global__ __launch_bounds__(256) void wgemm_finalize_norm_kernel(GemmArgs a) {
             st16(a.post_out + (int64_t)m * a.ld_post + c * 8, make_uint4(o[0], o[1], o[2], o[3]));
         }
     }
+}
+
+static int launch_finalize_norm(const GemmArgs& a, hipStream_t s) {
+    const int nvec = a.n / 8;
+    if (nvec > 512 && a.m <= num_cus()) hipLaunchKernelGGL(wgemm_finalize_norm_kernel<1024>, dim3(a.m), dim3(1024), 0, s, a);
+    else if (nvec > 256 && a.m <= num_cus()) hipLaunchKernelGGL(wgemm_finalize_norm_kernel<512>, dim3(a.m), dim3(512), 0, s, a);
+    else hipLaunchKernelGGL(wgemm_finalize_norm_kernel<256>, dim3(a.m), dim3(256), 0, s, a);
+    return check_launch();
 }
 
 // The slab reduction for other kernels of the library that split k (the prefill GEMM): same
@@ -1066,9 +1099,8 @@ int launch_wgemm_finalize_norm(float* partial, int ksplit, int m, int n, const v
     a.ld_post = norm->ld;
     a.post_eps = norm->eps;
     a.post_var_from_rounded = norm->var_from_rounded;
-    hipLaunchKernelGGL(wgemm_finalize_norm_kernel, dim3(m), dim3(256), 0, s, a);
     norm->done = true;
-    return check_launch();
+    return launch_finalize_norm(a, s);
 }
 
 static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_add_r,
@@ -1200,8 +1232,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
     }
     if (rc != MV_OK || slabs_only) return rc;
     if (post_ln_w) {
-        hipLaunchKernelGGL(wgemm_finalize_norm_kernel, dim3(m), dim3(256), 0, s, a);
-        rc = check_launch();
+        rc = launch_finalize_norm(a, s);
     } else if (a.ksplit > 1) {
         const int64_t total = (int64_t)m * ncols;
         int blocks = (int)((total + 255) / 256);
