@@ -249,3 +249,9 @@ def test_wgemm_widths_at_33_to_64_rows(mv, m, n, k):
     got = wgemm(x.to(DEV), StreamedWeight.from_linear(w.to(DEV)), torch.empty(m, n, dtype=torch.float32, device=DEV))
     xd, wd = x.double(), w.double()
     assert (((got.cpu().double() - xd @ wd.t()).abs()) <= k * 2.0 ** -24 * (xd.abs() @ wd.abs().t())).all()
+
+
+@pytest.mark.parametrize("n", [2048, 2064, 5136])
+def test_wgemm_postnorm_with_part_of_a_workgroup_idle(mv, n):
+    """512 and 1024 threads to a row, the last of them past the row's end."""
+    test_wgemm_postnorm_is_bit_identical_to_separate_kernels(mv, 8, n, 1024)
