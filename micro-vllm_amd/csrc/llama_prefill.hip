@@ -40,7 +40,7 @@ extern "C" int mv_llama_prefill_layers(const void* const* tensors, const float* 
                           (const void*)resid, (const void*)act})
         if (!aligned16(p)) return MV_ERR_INVALID_ARG;
     for (int i = 0; i < n_layers * kTensors; ++i)
-        if ((!tensors[i] && i % kTensors != kBqkv) || !aligned16(tensors[i])) return MV_ERR_INVALID_ARG;
+        if (i % kTensors != kBqkv && (!tensors[i] || !aligned16(tensors[i]))) return MV_ERR_INVALID_ARG;
     if (workspace_bytes < mv_llama_prefill_workspace_bytes(rows * seq, hidden, inter, hq, hkv, d) ||
         (workspace_bytes && (!workspace || !aligned16(workspace))))
         return MV_ERR_INVALID_ARG;
