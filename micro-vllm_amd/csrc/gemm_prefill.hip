@@ -414,16 +414,20 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     };
     // One stage, I = s mod kPeriod: request stage s + BUFS - 1 of x (its buffer was last read in stage s - 1), two k-tiles,
     // wait for this wave's part of stage s + 2, barrier: the next stage's later reads and the stage after's early reads
-    // both see complete data.
-    auto stage = [&](auto index, int s) {
+    // both see complete data.  `left`: a stage behind the whole passes, whose refills nobody uses.
+    auto stage = [&](auto index, auto left, int s) {
         constexpr int I = decltype(index)::value, b0 = I % BUFS, b1 = (I + 1) % BUFS;
+        constexpr bool kLeft = decltype(left)::value;
         MV_STAMP(0);
         ktile(w[2 * I % RING], w[(2 * I + RING - 1) % RING], X0, X1, b0, 0, b0, 1, 2 * s + RING - 1, s + BUFS - 1,
               (I + BUFS - 1) % BUFS);
         ktile(w[(2 * I + 1) % RING], w[2 * I % RING], X1, X0, b0, 1, b1, 0, 2 * s + RING, -1, 0);
         MV_STAMP(1);
-        // requested after that stage of x: the refill behind it and, per stage since, two refills and four pieces of x
-        wait_vmcnt<kPNT + (BUFS - 3) * (2 * kPNT + XP)>();
+        // requested after that stage of x: the refill behind it and, per stage since, two refills and XP pieces of x.  In the
+        // stages left over the compiler drops the refills, so only the pieces of x may be counted there: a count that
+        // includes requests that were never made waits for nothing, and the next stage reads what has not arrived.  (Three
+        // buffers: at most two stages are left over, and both have arrived before the first of them.)
+        wait_vmcnt<(kLeft && BUFS > 3) ? (BUFS - 3) * XP : kPNT + (BUFS - 3) * (2 * kPNT + XP)>();
         MV_STAMP(2);
 #ifndef MV_EXP_NO_BARRIER
         __syncthreads();
@@ -433,15 +437,17 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     // kPeriod stages per pass and no branch inside the pass (a branch between stages makes the
     // compiler wait for every outstanding request where the paths meet); the stages left over follow
     int s = 0;
+    constexpr std::false_type whole{};
+    constexpr std::true_type left{};
     for (; s + kPeriod <= nstage; s += kPeriod) {
-        stage(std::integral_constant<int, 0>{}, s);
-        stage(std::integral_constant<int, 1>{}, s + 1);
-        stage(std::integral_constant<int, 2>{}, s + 2);
-        if constexpr (kPeriod == 4) stage(std::integral_constant<int, 3>{}, s + 3);
+        stage(std::integral_constant<int, 0>{}, whole, s);
+        stage(std::integral_constant<int, 1>{}, whole, s + 1);
+        stage(std::integral_constant<int, 2>{}, whole, s + 2);
+        if constexpr (kPeriod == 4) stage(std::integral_constant<int, 3>{}, whole, s + 3);
     }
-    if (s < nstage) stage(std::integral_constant<int, 0>{}, s);
-    if (s + 1 < nstage) stage(std::integral_constant<int, 1>{}, s + 1);
-    if (kPeriod == 4 && s + 2 < nstage) stage(std::integral_constant<int, 2>{}, s + 2);
+    if (s < nstage) stage(std::integral_constant<int, 0>{}, left, s);
+    if (s + 1 < nstage) stage(std::integral_constant<int, 1>{}, left, s + 1);
+    if (kPeriod == 4 && s + 2 < nstage) stage(std::integral_constant<int, 2>{}, left, s + 2);
     wait_vmcnt<0>();     // no request into LDS outlives the workgroup
 
     store_wave_tile<kPNT, MT>(a, acc, nt0, m0, ks, r, q);

@@ -448,11 +448,15 @@ def test_few_rows_add_the_slices_in_order(mv, m, n, k, mode):
 
 @pytest.mark.parametrize("m,n,k,mode", [(65, 6144, 2048, "bias"), (129, 16384, 1024, "swiglu"), (512, 4112, 2048, "residual"),
                                         (700, 2048, 64, "plain"), (700, 2048, 320, "f32"), (1000, 2048, 832, "plain"),
-                                        (1000, 4096, 4096, "residual"), (768, 8192, 2048, "plain")])
+                                        (1000, 4096, 4096, "residual"), (768, 8192, 2048, "plain"),
+                                        (700, 2048, 128, "plain"), (700, 2048, 192, "f32"), (700, 2048, 384, "plain"),
+                                        (700, 2048, 448, "f32"), (1100, 4096, 1600, "f32"), (1100, 4096, 1664, "plain"),
+                                        (1100, 4096, 1728, "f32"), (1100, 4096, 13824, "plain")])
 def test_tiles_of_64_and_128_rows_give_the_same_sums(mv, m, n, k, mode):
-    """Grids of less than a workgroup to a compute unit take 64-row tiles or the deep form (remainders of its pass of four
-    stages: k of 64, 320, 832); the same rows inside a product of many take 128-row tiles.  The sums have the same order
-    wherever neither is cut along k."""
+    """Grids of less than a workgroup to a compute unit take 64-row tiles or the deep form (1100 rows, and 768 of 8192
+    columns); the same rows inside a product of many take 128-row tiles.  The sums have the same order wherever neither is
+    cut along k.  Both forms pass over k in fours of 64: every remainder, with whole passes before it (64-row tiles: k of
+    320, 384, 448; deep form: 1600, 1664, 1728) and without (64, 128, 192)."""
     from micro_vllm_amd import _native as nv
     from micro_vllm_amd.kernel.linear import StreamedWeight
 
