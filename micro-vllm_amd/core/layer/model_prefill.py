@@ -16,6 +16,7 @@ import torch
 from .. import parallel_config as pc
 from ... import _native as nv
 from ..prefill_attention import paged_attn_prefill_rows, rope_store_prefill
+from ...kernel._rows import require_bf16_cuda
 from ...kernel.linear import add_, embedding, gemm_prefill, wgemm
 from ...kernel.rmsnorm_add import rmsnorm, rmsnorm_residual_fused
 from ...kernel.swiglu import swiglu_fused
@@ -66,10 +67,14 @@ class ModelPrefillRunner(ModelGraphRunner):
 
     def _prefill_stack(self, h, B, S, cache_manager, cache_lens, block_table):
         """Every layer on hidden rows h [B*S, hid], in place, from one native call (mv_llama_prefill_layers): what
-        `_prefill_layer` gives layer by layer, bit for bit."""
+        `_prefill_layer` gives layer by layer, bit for bit, and refused where that refuses."""
         T, dev, L = B * S, h.device, nv.lib()
         hid, hq, hkv, d = self.hidden_dim, self.num_heads, self.kv_num_heads, self.head_size
         blocks = self.model.transformer.h
+        assert block_table.dtype == torch.int32 and block_table.stride(1) == 1 and cache_lens.dtype == torch.int32
+        assert block_table.shape[0] >= B and cache_lens.numel() >= B
+        cos, sin = self.attention._cos_pool, self.attention._sin_pool
+        assert cos.dtype == torch.bfloat16 and cos.shape[1] == d // 2 and cos.is_contiguous() and sin.is_contiguous()
         tensors, eps = [], []
         for li in range(self.num_layers):
             b = blocks[li]
@@ -79,8 +84,9 @@ class ModelPrefillRunner(ModelGraphRunner):
             w = (b.attn._qkv_w, b.attn._o, b.mlp._gu, b.mlp._d)
             assert (w[0].n, w[0].k, w[1].n, w[1].k) == ((hq + 2 * hkv) * d, hid, hid, hq * d)
             assert (w[2].n, w[2].k, w[3].n, w[3].k) == (2 * w[3].k, hid, hid, w[2].out_features) and w[2].swiglu
+            require_bf16_cuda(b.ln_1.weight, b.ln_2.weight)
             for ln in (b.ln_1.weight, b.ln_2.weight):
-                assert ln.dtype == torch.bfloat16 and ln.numel() == hid and ln.is_contiguous()
+                assert ln.numel() == hid and ln.is_contiguous()
             bias = b.attn._qkv_b
             assert bias is None or (bias.dtype == torch.bfloat16 and bias.numel() == w[0].n and bias.is_contiguous())
             tensors += [b.ln_1.weight.data_ptr(), w[0].tiles.data_ptr(), nv.ptr(bias), w[1].tiles.data_ptr(),
@@ -92,8 +98,6 @@ class ModelPrefillRunner(ModelGraphRunner):
         NB, page = k_cache.shape[:2]
         inter = blocks[0].mlp._d.k
         assert all(blocks[li].mlp._d.k == inter for li in range(self.num_layers))
-        cos, sin = self.attention._cos_pool, self.attention._sin_pool
-        assert block_table.dtype == torch.int32 and block_table.stride(1) == 1 and cache_lens.dtype == torch.int32
         ws = nv.stream_workspace("gemm_prefill", dev, L.mv_llama_prefill_workspace_bytes(T, hid, inter, hq, hkv, d))
         rows = lambda n: torch.empty(T, n, dtype=torch.bfloat16, device=dev)   # noqa: E731
         normed, resid, proj = rows(hid), rows(hid), torch.empty(T, hid, dtype=torch.float32, device=dev)
