@@ -67,7 +67,9 @@ class ModelPrefillRunner(ModelGraphRunner):
 
     def _prefill_stack(self, h, B, S, cache_manager, cache_lens, block_table):
         """Every layer on hidden rows h [B*S, hid], in place, from one native call (mv_llama_prefill_layers): what
-        `_prefill_layer` gives layer by layer, bit for bit, and refused where that refuses."""
+        `_prefill_layer` gives layer by layer, bit for bit, and refused where that refuses.  None, with nothing done, where
+        the layers are not alike - feed-forwards of several widths, caches of several shapes - or their gate and up
+        projections are not interleaved (weights laid out by a runner with fused=False)."""
         T, dev, L = B * S, h.device, nv.lib()
         hid, hq, hkv, d = self.hidden_dim, self.num_heads, self.kv_num_heads, self.head_size
         blocks = self.model.transformer.h
@@ -75,15 +77,18 @@ class ModelPrefillRunner(ModelGraphRunner):
         assert block_table.shape[0] >= B and cache_lens.numel() >= B
         cos, sin = self.attention._cos_pool, self.attention._sin_pool
         assert cos.dtype == torch.bfloat16 and cos.shape[1] == d // 2 and cos.is_contiguous() and sin.is_contiguous()
-        tensors, eps = [], []
+        tensors, eps, like = [], [], None
         for li in range(self.num_layers):
             b = blocks[li]
             k_cache, v_cache = cache_manager.get(li)
+            w = (b.attn._qkv_w, b.attn._o, b.mlp._gu, b.mlp._d)
+            like = like or (w[3].k, k_cache.shape)
+            if not w[2].swiglu or (w[3].k, k_cache.shape) != like:
+                return None
             assert k_cache.shape[2:] == (hkv, d) and k_cache.shape == v_cache.shape, "cache heads/dim mismatch"
             assert k_cache.is_contiguous() and v_cache.is_contiguous()
-            w = (b.attn._qkv_w, b.attn._o, b.mlp._gu, b.mlp._d)
             assert (w[0].n, w[0].k, w[1].n, w[1].k) == ((hq + 2 * hkv) * d, hid, hid, hq * d)
-            assert (w[2].n, w[2].k, w[3].n, w[3].k) == (2 * w[3].k, hid, hid, w[2].out_features) and w[2].swiglu
+            assert (w[2].n, w[2].k, w[3].n) == (2 * w[3].k, hid, hid)
             require_bf16_cuda(b.ln_1.weight, b.ln_2.weight)
             for ln in (b.ln_1.weight, b.ln_2.weight):
                 assert ln.numel() == hid and ln.is_contiguous()
@@ -93,11 +98,9 @@ class ModelPrefillRunner(ModelGraphRunner):
                         b.ln_2.weight.data_ptr(), w[2].tiles.data_ptr(), w[3].tiles.data_ptr(), k_cache.data_ptr(),
                         v_cache.data_ptr()]
             eps += [float(b.ln_1.eps), float(b.ln_2.eps)]
-        if not tensors:
+        if not tensors or T == 0:
             return h
-        NB, page = k_cache.shape[:2]
-        inter = blocks[0].mlp._d.k
-        assert all(blocks[li].mlp._d.k == inter for li in range(self.num_layers))
+        inter, (NB, page) = like[0], like[1][:2]
         ws = nv.stream_workspace("gemm_prefill", dev, L.mv_llama_prefill_workspace_bytes(T, hid, inter, hq, hkv, d))
         rows = lambda n: torch.empty(T, n, dtype=torch.bfloat16, device=dev)   # noqa: E731
         normed, resid, proj = rows(hid), rows(hid), torch.empty(T, hid, dtype=torch.float32, device=dev)
@@ -130,10 +133,9 @@ class ModelPrefillRunner(ModelGraphRunner):
         block_table = cache_manager._block_table_buffer[:batch_size]
 
         whole = self.world_size == 1 and self.fused     # (several ranks reduce between the launches of a layer)
-        if whole:
-            h = self._prefill_stack(h, B, S, cache_manager, cache_lens, block_table)
-        for layer_idx in range(0 if whole else self.num_layers):
-            h = self._prefill_layer(h, layer_idx, B, S, cache_manager, cache_lens, block_table)
+        if not whole or self._prefill_stack(h, B, S, cache_manager, cache_lens, block_table) is None:
+            for layer_idx in range(self.num_layers):
+                h = self._prefill_layer(h, layer_idx, B, S, cache_manager, cache_lens, block_table)
 
         if last_token_index is not None:
             idx = torch.as_tensor(last_token_index, dtype=torch.long).to(dev)

@@ -377,3 +377,42 @@ def test_stack_in_one_call_equals_layer_by_layer(mv, shape, bias, B, S, monkeypa
     mgr._k_store.zero_(), mgr._v_store.zero_()
     got = prefill._prefill_stack(h0.clone(), B, S, mgr, lens, bt)
     assert torch.equal(got, want) and torch.equal(mgr._k_store, k_want) and torch.equal(mgr._v_store, v_want)
+
+
+@pytest.mark.parametrize("odd", ["feed-forward widths", "weights of an unfused runner", "pages per layer"])
+def test_layers_that_are_not_alike_go_one_by_one(mv, odd):
+    """What mv_llama_prefill_layers has no argument for: forward() takes such a model layer by layer, as it was taken
+    before there was one call for all."""
+    from types import SimpleNamespace
+
+    from micro_vllm_amd.core.cache_manager import KVCacheManager
+    from micro_vllm_amd.core.layer.model_graph import ModelGraphRunner
+    from micro_vllm_amd.core.layer.model_prefill import ModelPrefillRunner
+    from micro_vllm_amd.models import SHAPES, build_synthetic_model
+
+    cfg, B, S = SHAPES["tiny-gqa"], 2, 37
+    model = build_synthetic_model(cfg, "cpu", seed=9).to(DEV)
+    if odd == "feed-forward widths":
+        mlp, keep = model.transformer.h[1].mlp, cfg.ffn_hidden_size - 128
+        mlp.w1.weight, mlp.w2.weight = mlp.w1.weight[:keep], mlp.w2.weight[:keep]
+        mlp.c_proj.weight = mlp.c_proj.weight[:, :keep].contiguous()
+    args = (model, cfg.num_hidden_layers, cfg.num_attention_heads, cfg.head_dim, cfg.num_key_value_heads, cfg.hidden_size,
+            cfg.intermediate_size, DEV)
+    if odd == "weights of an unfused runner":
+        ModelGraphRunner(*args, max_batch_size=B, fused=False)
+    prefill = ModelPrefillRunner(*args, max_batch_size=B)
+    pools = [KVCacheManager(12 + li if odd == "pages per layer" else 12, 256, 1, cfg.num_key_value_heads, cfg.head_dim,
+                            dtype=torch.bfloat16, device=DEV, max_tokens=1024, max_batch_size=B) for li in range(2)]
+    for b in range(B):
+        pools[0].alloc(b, S)
+    bt, _ = pools[0].cache_batch_data(list(range(B)), [S] * B)
+    mgr = SimpleNamespace(get=lambda li: pools[li].get(0), _cache_seqlens_buffer=pools[0]._cache_seqlens_buffer,
+                          _block_table_buffer=pools[0]._block_table_buffer)
+    ids = torch.randint(0, cfg.vocab_size, (B, S), generator=torch.Generator().manual_seed(3)).to(DEV)
+    got = prefill.forward(ids, mgr, B)
+    kv = [x.clone() for p in pools for x in p.get(0)]
+    for p in pools:
+        p._k_store.zero_(), p._v_store.zero_()
+    prefill._prefill_stack = lambda *a: None
+    assert torch.equal(got, prefill.forward(ids, mgr, B))
+    assert all(torch.equal(a, b) for a, b in zip(kv, [x for p in pools for x in p.get(0)]))

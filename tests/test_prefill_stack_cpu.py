@@ -66,3 +66,9 @@ def test_rotary_tables_of_another_head_size(mv, monkeypatch):
     r.attention._cos_pool = torch.ones(16, 8, dtype=torch.bfloat16)
     with pytest.raises(AssertionError):
         _call(r, mgr, h)
+
+
+def test_an_empty_batch_needs_no_launch(mv, monkeypatch):
+    r, mgr, h = _runner(monkeypatch)
+    out = r._prefill_stack(h[:0], 2, 0, mgr, torch.zeros(2, dtype=torch.int32), torch.zeros(2, 4, dtype=torch.int32))
+    assert out is not None and out.shape[0] == 0
