@@ -1368,6 +1368,10 @@ __device__ __forceinline__ int first_visible(int pos, int size, int chunked) {
     return lo > 0 ? lo : 0;
 }
 
+// What weights are taken against: the largest score so far.  Scores can all be -infinity (an infinite key); their weights
+// are zero then, as they are beside a finite score, and not exp(-inf + inf).
+__device__ __forceinline__ float finite_max(float m) { return m == -INFINITY ? 0.f : m; }
+
 // One workgroup per (token, head).  Its NW waves (4, or 16 when a step has too few tokens to fill the
 // chip otherwise: decoding) take the window's 64-key tiles in turn: a lane scores
 // one key (q from LDS, the key row straight from its page), the wave forms max / sum of the tile and
@@ -1427,9 +1431,9 @@ __global__ __launch_bounds__(64 * NW) void window_attn_kernel(const float* q, in
             }
             s = dot * scale - slope * (float)(pos - j);
         }
-        const float mn = fmaxf(m, wave_max(s));
-        const float pj_ = j <= last ? expf(s - mn) : 0.f;
-        const float corr = expf(m - mn);   // m = -inf on the wave's first tile: exp(-inf) = 0
+        const float mn = fmaxf(m, wave_max(s)), at = finite_max(mn);
+        const float pj_ = j <= last ? expf(s - at) : 0.f;
+        const float corr = expf(m - at);   // m = -inf on the wave's first tile: exp(-inf) = 0
         l = l * corr + wave_sum(pj_);
         m = mn;
         __builtin_amdgcn_wave_barrier();
@@ -1479,14 +1483,15 @@ __global__ __launch_bounds__(64 * NW) void window_attn_kernel(const float* q, in
     }
     __syncthreads();
     if (wv == 0) {
-        float M = mm[0];                                   // wave 0 always has a key: finite
+        float M = mm[0];
 #pragma unroll
         for (int w = 1; w < NW; ++w) M = fmaxf(M, mm[w]);
         float L = 0.f;
         if (sinks) {
             M = fmaxf(M, sinks[h]);
-            L = expf(sinks[h] - M);
+            L = expf(sinks[h] - finite_max(M));
         }
+        M = finite_max(M);
         float w4[NW];
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
@@ -1617,9 +1622,9 @@ __global__ __launch_bounds__(256) void window_attn_group_kernel(const float* q, 
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             const float sc = valid ? dot[r] * scale - slope[r] * (float)(pos - j) : -INFINITY;
-            const float mn = fmaxf(m[r], wave_max(sc));        // finite: a tile holds at least one key
-            const float pj = valid ? expf(sc - mn) : 0.f;
-            const float corr = expf(m[r] - mn);                // m = -inf on the wave's first tile: exp(-inf) = 0
+            const float mn = fmaxf(m[r], wave_max(sc)), at = finite_max(mn);
+            const float pj = valid ? expf(sc - at) : 0.f;
+            const float corr = expf(m[r] - at);                // m = -inf on the wave's first tile: exp(-inf) = 0
             l[r] = l[r] * corr + wave_sum(pj);
             m[r] = mn;
             pw[r * 64 + lane] = pj;
@@ -1971,12 +1976,13 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
                 p[k] = key < cnt ? sc[b][k] * scale - slope[b] * (float)(pos - first - key) : -INFINITY;
                 mx = fmaxf(mx, p[k]);
             }
-            const float mn = fmaxf(m[b], rows_max(mx));        // finite: a tile holds at least one key
-            const float corr = expf(m[b] - mn);                // m = -inf on the wave's first tile: exp(-inf) = 0
+            const float mn = fmaxf(m[b], rows_max(mx));
+            const float at = finite_max(mn);
+            const float corr = expf(m[b] - at);                // m = -inf on the wave's first tile: exp(-inf) = 0
             float sum = 0.f;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                p[k] = 4 * quad + k < cnt ? expf(p[k] - mn) : 0.f;
+                p[k] = 4 * quad + k < cnt ? expf(p[k] - at) : 0.f;
                 sum += p[k];
             }
             l[b] = l[b] * corr + sum;                          // this lane's four keys' share
@@ -2035,8 +2041,9 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
         float M = -INFINITY;
         for (int w = 0; w < nact; ++w) M = fmaxf(M, mm[w * RT + r]);
         float L = 0.f, o = 0.f;
+        const float at = finite_max(M);
         for (int w = 0; w < nact; ++w) {
-            const float f = expf(mm[w * RT + r] - M);
+            const float f = expf(mm[w * RT + r] - at);
             L = fmaf(ll[w * RT + r], f, L);
             o = fmaf(red[(w * RT + r) * dv + c], f, o);
         }

@@ -510,3 +510,51 @@ def test_few_token_attention_equals_the_per_head_form(ops, f32, d, dv, H, G, row
     assert bool(torch.isfinite(outs[0]).all())
     tol = 1e-5 * top + (0 if f32 else 2 ** -7) * outs[0].abs()
     assert ((outs[1] - outs[0]).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("form", ["per head", "grouped", "few"])
+@pytest.mark.parametrize("H,G,window,splits,sink", [(4, 2, 5000, 1, False), (8, 1, 5000, 3, False), (2, 2, 700, 2, True), (4, 1, 64, 1, True)])
+def test_infinite_keys_alone_in_their_tile(ops, f32, form, H, G, window, splits, sink):
+    """Keys whose scores are -infinity for every head and that fill a tile of 16 or 64 keys: the newest one where the window's
+    tiles end with it, the first 16 and 64, a whole split's, and (with a sink) every key.  Their weights are zero beside any
+    finite score or sink.  Against softmax in 64 bits; the error of 32-bit scores of up to 8 (d = 64 products) moves a weight by
+    less than 1e-5, and bf16 outputs are rounded (2^-8 of the value)."""
+    from types import SimpleNamespace
+
+    d = dv = page = 64
+    dt = torch.float32 if f32 else torch.bfloat16
+    top = window - 1
+    # (position, infinite keys); rows past the window see [pos - window + 1, pos]
+    cases = [(16, [16]), (64, [64]), (63, range(16)), (130, range(64)), (min(top, 640), range(0, 512))]
+    cases += [(40, range(41))] if sink else []
+    rows, per = len(cases), 700 // page + 1
+    g = torch.Generator().manual_seed(H + window)
+    bt = torch.randperm(rows * per, generator=g).int().view(rows, per)
+    kc, vc = torch.randn(rows * per, page, G, d, generator=g).to(dt), torch.randn(rows * per, page, G, dv, generator=g).to(dt)
+    pad = 1 if form == "grouped" else 0           # (rows that are no multiple of 16 bytes: not the form for few tokens)
+    q = torch.randn(rows, H * d + pad, generator=g)
+    q[:, :H * d:d] = -q[:, :H * d:d].abs() - 0.1
+    ctx = torch.tensor([c for c, _ in cases])
+    for b, (_, inf) in enumerate(cases):
+        for i in inf:
+            kc[bt[b, i // page], i % page, :, 0] = float("inf")
+    sinks = torch.randn(H, generator=g) if sink else None
+    step = SimpleNamespace(tok_row=torch.arange(rows).int().to(DEV), tok_pos=ctx.int().to(DEV), block_table=bt.to(DEV),
+                           row_len=torch.ones(rows, dtype=torch.int32, device=DEV), ch_start=None, ch_len=None, n_chunks=0,
+                           page=page, max_page=rows * per - 1, tokens=rows)
+    out = torch.empty(rows, H * dv, dtype=dt, device=DEV)
+    part = None if form == "per head" else torch.full((rows * H * splits * (dv + 2),), float("nan"), device=DEV)
+    ops.window_attn(q.to(DEV)[:, :H * d], kc.to(DEV), vc.to(DEV), out, step, None, H, G, d, dv, d ** -0.5, window,
+                    sinks=None if sinks is None else sinks.to(DEV), part=part, splits=splits)
+    for b in range(rows):
+        js = torch.arange(max(0, int(ctx[b]) - window + 1), int(ctx[b]) + 1)
+        k, v = (c[bt[b, js // page].long(), js % page].double() for c in (kc, vc))
+        for h in range(H):
+            s = (k[:, h // (H // G)] @ q[b, h * d:(h + 1) * d].double()) * d ** -0.5
+            if sinks is not None:
+                s = torch.cat([s, sinks[h:h + 1].double()])
+            p = torch.softmax(s, 0)[:len(js)]
+            want = p @ v[:, h // (H // G)]
+            got = out[b, h * dv:(h + 1) * dv].cpu().double()
+            assert ((got - want).abs() <= 1e-5 * 4 + (0 if f32 else 2 ** -8) * want.abs()).all(), (b, h)
