@@ -2864,13 +2864,19 @@ int mv_window_attn(const float* q, int64_t ldq, const void* k_cache, const void*
         };
         if (aligned16(q) && ldq % 4 == 0 && aligned16(k_cache) && aligned16(v_cache)) {
             // Sixteen waves (eight where the registers of fp32 rows or of eight heads allow no more) while every workgroup has
-            // a compute unit to itself, else four.  A split has 64 keys to a wave of the widest form before another is
-            // opened: one token at 1100 keys took 23.2 us in five splits and takes 20.3 in one, at 45 keys the merge's
-            // launch alone is 2 of 10 us.  fp32 rows, twice as long to read and eight waves, gain from a second split
-            // (1100 keys 30.8 -> 24.0 us, 45 keys 6.6 -> 8.0).
+            // a compute unit to itself, else four.  One split while the window is up to 1280 keys, five tiles to a wave (640
+            // with fp32 rows, twice as long to read, and with eight waves): a merge is a launch more, 2 of 10 us at 45 keys.
+            // Past that one to 256 keys of the window, but no more workgroups than compute units, where a second round of
+            // them costs more than the splits give.  One token of bf16 at 2000 keys, window 2047, in one split and in eight
+            // (us): 8 heads of 128 on 2 29.6, 16.9; 16 on 2 51.8, 21.0; 8 heads of 64 on 8 18.6, 11.2 (in 64-key tiles 27.3, 34.8, 13.5);
+            // 32 tokens at 4000, 16 heads on 2, in one, four and eight splits 56.5, 28.3, 41.0; one fp32 token at 1100, window 1024, 8 heads on
+            // 2, in one, two and four splits 27.3, 21.8, 17.9.
             const int64_t groups = (int64_t)tokens * kv_heads * ngrp;
-            const int64_t fill = ((int64_t)window + keep_first) / (f32 ? 512 : 1024);
-            const int pieces = fill < 1 ? 1 : fill < splits ? (int)fill : splits;
+            const int64_t keys = (int64_t)window + keep_first, room = num_cus() / groups;
+            int64_t want = keys <= (f32 || top > 4 ? 640 : 1280) ? 1 : (keys + 128) / 256;
+            if (want > room) want = room;
+            if (want > splits) want = splits;
+            const int pieces = want < 1 ? 1 : (int)want;
             const bool wide = groups * pieces <= num_cus();
             int nw = 0;      // (0: a head shape without an instance)
 #define MV_WA_FEW(F32_, HB_, NW_, KS_, VE_)                                                                            \

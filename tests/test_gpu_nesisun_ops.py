@@ -473,7 +473,8 @@ def test_routed_experts_with_pass_through(ops, f32, E, n_id, top):
 @pytest.mark.parametrize("d,dv", [(128, 128), (64, 64), (96, 96), (128, 64), (64, 128), (32, 32), (64, 32)])
 @pytest.mark.parametrize("H,G,rows,page,window,keep,chunked,splits", [
     (8, 2, 3, 64, 100, 0, False, 1), (3, 3, 5, 48, 300, 20, False, 3), (9, 1, 2, 16, 5000, 0, False, 4), (14, 2, 2, 64, 1024, 70, False, 7),
-    (4, 4, 80, 64, 64, 33, False, 2), (16, 2, 140, 64, 90, 0, True, 1), (2, 1, 300, 64, 40, 0, False, 1)])
+    (4, 4, 80, 64, 64, 33, False, 2), (16, 2, 140, 64, 90, 0, True, 1), (2, 1, 300, 64, 40, 0, False, 1),
+    (8, 2, 2, 64, 2047, 0, False, 9), (16, 2, 40, 64, 3000, 0, False, 5)])
 def test_few_token_attention_equals_the_per_head_form(ops, f32, d, dv, H, G, rows, page, window, keep, chunked, splits):
     """Every instance (one, up to four and up to eight heads a workgroup, few and many workgroups, one split and several)
     against one workgroup per head: contexts from one key to past the window, an infinite key of weight zero, strides and
