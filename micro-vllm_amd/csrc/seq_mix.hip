@@ -705,9 +705,9 @@ __global__ __launch_bounds__(512) void scan_rows_kernel(ChunkArgs a, const float
 #pragma unroll
                     for (int ct = 0; ct < CT; ++ct) MV_MFMA4(o[ct], now[i][e], y[ct][e]);
             }
-            const f32x4_t w = *reinterpret_cast<const f32x4_t*>(&el[buf][16 * tt + 4 * g]);
+            f32x4_t in[CT];      // the chunk's own tokens, apart: their sums are rounded at their own size
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) o[ct] *= w;
+            for (int ct = 0; ct < CT; ++ct) in[ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
             const float Lt = Ls[buf][16 * tt + r];
 #pragma unroll
             for (int st = 0; st < 4; ++st) {
@@ -725,10 +725,13 @@ __global__ __launch_bounds__(512) void scan_rows_kernel(ChunkArgs a, const float
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int ct = 0; ct < CT; ++ct) MV_MFMA4(o[ct], P[e], y[ct][e]);
+                    for (int ct = 0; ct < CT; ++ct) MV_MFMA4(in[ct], P[e], y[ct][e]);
             }
+            const f32x4_t w = *reinterpret_cast<const f32x4_t*>(&el[buf][16 * tt + 4 * g]);
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[ct][j] = fmaf(w[j], o[ct][j], in[ct][j]);
                 const f32x4_t v4 = *reinterpret_cast<const f32x4_t*>(&vt[buf][(16 * ct + r) * SV + 16 * tt + 4 * g]);
                 float* op = a.out + (int64_t)(start + 16 * tt + 4 * g) * a.ldo + (int64_t)h * a.p + c0 + 16 * ct + r;
 #pragma unroll
@@ -781,10 +784,11 @@ __global__ __launch_bounds__(512) void scan_rows_kernel(ChunkArgs a, const float
             st1 = cs[at_most(c + 2)], ln1 = cl[at_most(c + 2)];
             fetch(st0, ln0);
             const float keep = at[buf];
+            f32x4_t add[JW][CT];     // what the chunk adds, apart: summed into S one by one its parts would each be rounded at S's size
 #pragma unroll
             for (int i = 0; i < JW; ++i)
 #pragma unroll
-                for (int ct = 0; ct < CT; ++ct) S[i][ct] *= keep;
+                for (int ct = 0; ct < CT; ++ct) add[i][ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int st = 0; st < 4; ++st) {
                 const f32x4_t w4 = *reinterpret_cast<const f32x4_t*>(&ws[buf][16 * st + 4 * g]);
@@ -797,8 +801,14 @@ __global__ __launch_bounds__(512) void scan_rows_kernel(ChunkArgs a, const float
 #pragma unroll
                     for (int i = 0; i < JW; ++i)
 #pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) MV_MFMA4(S[i][ct], now[4 * i + st][e], y[ct][e]);
+                        for (int ct = 0; ct < CT; ++ct) MV_MFMA4(add[i][ct], now[4 * i + st][e], y[ct][e]);
             }
+#pragma unroll
+            for (int i = 0; i < JW; ++i)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) S[i][ct][j] = fmaf(keep, S[i][ct][j], add[i][ct][j]);
             publish(buf ^ 1);
             stage(buf ^ 1, ln0);
             fetch_v(st1, ln1);

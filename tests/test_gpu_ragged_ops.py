@@ -374,6 +374,39 @@ def test_scan_of_whole_rows_equals_token_by_token(ops, H, G, n, p):
     test_scan_in_chunks_equals_token_by_token(ops, H, G, n, p)
 
 
+@pytest.mark.parametrize("H,G,n,p", [(16, 1, 64, 16), (16, 1, 128, 32), (128, 1, 128, 64)])
+def test_scan_of_whole_rows_rounds_the_state_once_a_chunk(ops, H, G, n, p):
+    """States that hardly decay, eight chunks: what a chunk adds is summed apart, so the state is rounded once a chunk, each
+    time by at most 2^-24 of itself and independently: sqrt(8) 2^-24 of it in the 2-norm.  (Added to the state product by
+    product it is rounded sixteen times a chunk.)  The outputs read such states over n products of random sign in n / 4
+    instructions, and a chunk's own 64 terms are rounded like those: as much again as n / 4 roundings of partial sums that grow to the whole."""
+    g = torch.Generator().manual_seed(n + p)
+    T, rep = 8 * 64, H // G
+    q, k, v = torch.randn(T, G * n, generator=g), torch.randn(T, G * n, generator=g), torch.randn(T, H * p, generator=g)
+    logd = -torch.rand(T, H, generator=g) * 4e-4
+    cache = make_cache(state={0: {"s": (H, n, p)}})
+    st = step_of(cache, [("a", [0] * T)])
+    o = torch.empty(T, H * p, device=DEV)
+    ops.scan_outer(q.to(DEV), k.to(DEV), v.to(DEV), torch.exp(logd).to(DEV), None, None, cache.states[0]["s"], o, st, H, n, p,
+                   q_div=rep, k_div=rep, log_decay=logd.to(DEV))
+    # chunk by chunk in 64 bits: S = exp(L_end) S + k^T (w v), o = exp(L) (q S + ...)
+    qd, kd, vd = (x.double().to(DEV).view(T, -1, w).transpose(0, 1) for x, w in ((q, n), (k, n), (v, p)))
+    qd, kd = qd.repeat_interleave(rep, 0), kd.repeat_interleave(rep, 0)
+    L = logd.double().to(DEV).T
+    S, want = torch.zeros(H, n, p, dtype=torch.float64, device=DEV), []
+    for c in range(0, T, 64):
+        s = slice(c, c + 64)
+        l = L[:, s].cumsum(1)
+        P = torch.tril(qd[:, s] @ kd[:, s].transpose(1, 2).contiguous() * torch.exp(l[:, :, None] - l[:, None, :]))
+        want.append(P @ vd[:, s] + torch.exp(l)[:, :, None] * (qd[:, s] @ S))
+        w = torch.exp(l[:, -1:] - l)[:, :, None]
+        S = torch.exp(l[:, -1])[:, None, None] * S + kd[:, s].transpose(1, 2).contiguous() @ (w * vd[:, s])
+    want = torch.cat(want, 1).transpose(0, 1).reshape(T, H * p)
+    state = cache.states[0]["s"][int(st.row_slot[0])].double()
+    assert ((state - S).norm() / S.norm()).item() < 8 ** 0.5 * 2.0 ** -24
+    assert ((o.double() - want).norm() / want.norm()).item() < (8 ** 0.5 + (n / 4) ** 0.5) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("C,taps", [(4, 4), (1028, 4), (8448, 4), (260, 3), (64, 2), (24, 5), (30, 4)])
 def test_conv_silu_forms(ops, C, taps):
     """Runs of eight tokens over several rows in one step (row starts inside a run, rows shorter than the taps), then one
