@@ -776,10 +776,19 @@ __global__ __launch_bounds__(512) void scan_rows_kernel(ChunkArgs a, const float
         fetch_v(st1, ln1);
         __syncthreads();
         for (int c = 0; c < nch; ++c) {
-            const int buf = c & 1;
+            const int buf = c & 1, len = ln0;
             f32x4_t now[NJ];
 #pragma unroll
             for (int i = 0; i < NJ; ++i) now[i] = fr[i];
+            if (len < kCh) {     // (uniform) past the end the last token was read again: its weight is zero, but it may be infinite
+#pragma unroll
+                for (int st = 0; st < 4; ++st)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int i = 0; i < JW; ++i)
+                            if (16 * st + 4 * g + e >= len) now[4 * i + st][e] = 0.f;
+            }
             st0 = st1, ln0 = ln1;
             st1 = cs[at_most(c + 2)], ln1 = cl[at_most(c + 2)];
             fetch(st0, ln0);

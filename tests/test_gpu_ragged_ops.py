@@ -407,6 +407,26 @@ def test_scan_of_whole_rows_rounds_the_state_once_a_chunk(ops, H, G, n, p):
     assert ((o.double() - want).norm() / want.norm()).item() < (8 ** 0.5 + (n / 4) ** 0.5) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("H,n,p", [(16, 64, 16), (16, 128, 64), (4, 64, 32)])
+def test_scan_in_chunks_with_an_infinite_key_at_the_end(ops, H, n, p):
+    """An infinite element of the last token's key: its state row becomes infinite in every column (v has no zero), as in the
+    recurrence itself, and every other state row stays what it is.  Both chunked forms; rows that end inside a chunk."""
+    g = torch.Generator().manual_seed(H + p)
+    T = 70
+    q, k, v = torch.randn(T, n, generator=g), torch.randn(T, n, generator=g), torch.randn(T, H * p, generator=g)
+    v[T - 1] = v[T - 1].abs() + 0.1
+    k[T - 1, 5] = float("inf")
+    logd = -torch.rand(T, H, generator=g)
+    cache = make_cache(state={0: {"s": (H, n, p)}})
+    st = step_of(cache, [("a", [0] * T)])
+    o = torch.empty(T, H * p, device=DEV)
+    ops.scan_outer(q.to(DEV), k.to(DEV), v.to(DEV), torch.exp(logd).to(DEV), None, None, cache.states[0]["s"], o, st, H, n, p,
+                   q_div=H, k_div=H, log_decay=logd.to(DEV))
+    state = cache.states[0]["s"][int(st.row_slot[0])].cpu()
+    assert bool((state[:, 5] == float("inf")).all())
+    assert bool(torch.isfinite(state[:, torch.arange(n) != 5]).all()) and bool(torch.isfinite(o[:T - 1]).all())
+
+
 @pytest.mark.parametrize("C,taps", [(4, 4), (1028, 4), (8448, 4), (260, 3), (64, 2), (24, 5), (30, 4)])
 def test_conv_silu_forms(ops, C, taps):
     """Runs of eight tokens over several rows in one step (row starts inside a run, rows shorter than the taps), then one
