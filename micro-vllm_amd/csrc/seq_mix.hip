@@ -104,7 +104,10 @@ __global__ __launch_bounds__(256) void conv_state_update_kernel(const float* in,
 // The convolution four channels to a thread, for TAPS taps and 16-byte rows: a thread slides over kConvRun consecutive tokens,
 // so an input is read once instead of once per tap, and nothing is divided per element.  Sums in the same order as above.
 // 2048 tokens of 8448 channels (4 taps): 114 -> 36 us; 138 MB that have to move.
+// Below kConvRunLeast outputs a thread's eight tokens are a longer chain than the launch of one thread per output: 64 tokens of
+// 8448 channels 8.5 us that way and 10.2 here, 300 of 2304 9.2 and 10.1, 512 of 2304 11.6 and 10.3.
 constexpr int kConvRun = 8;
+constexpr int64_t kConvRunLeast = 5 << 18;
 
 template <int TAPS>
 __device__ __forceinline__ void load_taps(float (&wt)[4][TAPS], const float* w, int c) {
@@ -2399,10 +2402,11 @@ int mv_conv_silu(const float* in, int64_t ldi, float* state, const float* w, con
     StepRows r{tok_row, nullptr, row_start, row_len, row_ctx, row_slot};
     hipStream_t s = (hipStream_t)stream;
     const int64_t work = (int64_t)tokens * channels;
+    const bool by_row = tokens <= rows;     // one token a row (decoding)
     if (taps >= 2 && taps <= 4 && channels % 4 == 0 && ldi % 4 == 0 && ldo % 4 == 0 && aligned16(in) && aligned16(out) &&
-        aligned16(state) && (!bias || aligned16(bias)) && rows <= 65535 && (tokens + kConvRun - 1) / kConvRun <= 65535) {
+        aligned16(state) && (!bias || aligned16(bias)) && (by_row ? rows : (tokens + kConvRun - 1) / kConvRun) <= 65535 &&
+        (by_row || work >= kConvRunLeast)) {
         const unsigned gx = (unsigned)((channels / 4 + 255) / 256);
-        const bool by_row = tokens <= rows;     // one token a row (decoding)
         const dim3 grid(gx, by_row ? rows : (tokens + kConvRun - 1) / kConvRun);
 #define MV_CONV(T_)                                                                                                    \
     if (by_row) hipLaunchKernelGGL(conv_silu_row_kernel<T_>, grid, dim3(256), 0, s, in, ldi, state, w, bias, out, ldo, r, channels); \

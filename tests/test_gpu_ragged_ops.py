@@ -427,11 +427,12 @@ def test_scan_in_chunks_with_an_infinite_key_at_the_end(ops, H, n, p):
     assert bool(torch.isfinite(state[:, torch.arange(n) != 5]).all()) and bool(torch.isfinite(o[:T - 1]).all())
 
 
-@pytest.mark.parametrize("C,taps", [(4, 4), (1028, 4), (8448, 4), (260, 3), (64, 2), (24, 5), (30, 4)])
+@pytest.mark.parametrize("C,taps", [(4, 4), (1028, 4), (8448, 4), (260, 3), (64, 2), (24, 5), (30, 4), (14336, 4),
+                                    (14336, 3), (14336, 2)])
 def test_conv_silu_forms(ops, C, taps):
-    """Runs of eight tokens over several rows in one step (row starts inside a run, rows shorter than the taps), then one
-    token a row, then both again: the same sums in the same order, so every output is the plain form's to its last bits
-    (1e-5 covers the exponential against 64 bits)."""
+    """Runs of eight tokens over several rows in one step (14336 channels; row starts inside a run, rows shorter than the
+    taps) or a thread per output (fewer), then one token a row, then both again: the same sums in the same order, so every
+    output is the plain form's to its last bits (1e-5 covers the exponential against 64 bits)."""
     g = torch.Generator().manual_seed(C)
     lens = {"a": 21, "b": 2, "c": 9, "d": 64}
     x = {k: torch.randn(2 * n + 4, C, generator=g) for k, n in lens.items()}
