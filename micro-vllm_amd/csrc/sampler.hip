@@ -4,8 +4,8 @@
 //                   Sampler._sample_impl (core/layer/sampler.py:21-43), as one launch instead of
 //                   topk + softmax + sort + cumsum + multinomial + two gathers.  The k largest
 //                   logits are found by a two-pass radix select on the 16 bf16 bits (division by a
-//                   positive temperature does not change the order), or for k up to 512 among the entries
-//                   that reach the k-th largest of the threads' maxima, gathered into LDS (ties at
+//                   positive temperature does not change the order), or for k up to 256 among the entries
+//                   (up to 512) that reach the k-th largest of the threads' maxima, gathered into LDS (ties at
 //                   the threshold by ascending index, so the result is deterministic), sorted there,
 //                   and the draw is the inverse CDF of the caller's uniform number.
 #include "common.h"
@@ -220,28 +220,30 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
     const int tid = threadIdx.x;
     const uint16_t* row = logits + (int64_t)blockIdx.x * ld;
     const int nvec = n >> 3;
-    const int k = min(min(top_k, n), kSmMaxK);
+    int k = min(min(top_k, n), kSmMaxK);
 
-    // The row is read ONCE: the first kSmKeep chunks of every thread (rows up to 131 072 entries
-    // whole) stay in registers for all three passes, requested back to back so that the read costs
+    // A selection reads the row ONCE: the first kSmKeep chunks of every thread (rows up to 131 072 entries
+    // whole) stay in registers for all its passes, requested back to back so that the read costs
     // one memory round trip instead of one per chunk and pass; longer rows stream the rest.
-    uint4 keep[kSmKeep];
+    auto load_row = [&](uint4(&v)[kSmKeep]) {
 #pragma unroll
-    for (int i = 0; i < kSmKeep; ++i) {
-        const int c = tid + i * kSmThreads;
-        keep[i] = ld16(row + (int64_t)min(c, nvec - 1) * 8);
-    }
+        for (int i = 0; i < kSmKeep; ++i) v[i] = ld16(row + (int64_t)min(tid + i * kSmThreads, nvec - 1) * 8);
+    };
     // ---- The k largest through the threads' maxima.  The k-th largest of the 1024 maxima bounds the k-th largest entry
     // from below (k different entries reach it), and few others do: of 128256 random logits 52 reach the bound for k =
     // 50, 295 for 256.  Those are listed and ranked by counting.  Only where more than kSmQuickMost entries reach the
-    // bound (rows of mostly equal logits), for larger k and for rows with a NaN the selection below runs: for k = 512
-    // ranking by counting took longer than it (98 against 90 us).  The maxima take three packed 16-bit instructions an
-    // entry pair; the radix selection makes two LDS atomics an entry.  32 rows of 128256, top 50: 80 -> 19.7 us;
-    // top 200: 85 -> 27.
+    // bound (rows of mostly equal logits), for larger k and for rows with a NaN or of -infinity alone the selection below
+    // runs: for k = 512 ranking by counting took longer than it (98 against 90 us).  The maxima take three packed 16-bit instructions an
+    // entry pair; the radix selection makes two LDS atomics an entry.  32 rows of 128256, top 50: 80 -> 14.8 us;
+    // top 200: 85 -> 22; ten entries left of 128256 and the rest masked 57 -> 13.1.  A row that the selection has to take
+    // after all reads its entries again (kept over both, they do not fit the registers) and is 5 to 11 us later
+    // there: 32 rows of equal logits 57 -> 68.
     auto in_row = [&](int i) { return tid + i * kSmThreads < nvec; };
     auto pair = [](uint32_t v) { return __builtin_bit_cast(s16x2_t, v); };
     bool listed = false;
     if (k <= kSmQuickK) {   // uniform
+        uint4 keep[kSmKeep];
+        load_row(keep);
         s16x2_t hi = {kKeyLow, kKeyLow}, lo = {32767, 32767};
         auto widen = [&](const uint4& keys) {
             const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
@@ -297,33 +299,57 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
             bound |= (unsigned)digit << shift;
             __syncthreads();
         }
-        const int thr = (int)bound - 32768;
-        auto list = [&](const uint4& keys, int c) {
+        // Entries of -infinity (masked out) have no weight beside any other: a row with fewer than k others has only those.
+        const int thr = max((int)bound - 32768, kKeyNegInf + 1);
+        auto reaching = [&](const uint4& keys) {     // how many of eight entries reach the bound
             const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
             const s16x2_t m = __builtin_elementwise_max(__builtin_elementwise_max(pair(w[0]), pair(w[1])),
                                                         __builtin_elementwise_max(pair(w[2]), pair(w[3])));
-            if (m.x < thr && m.y < thr) return;
+            unsigned n = 0;
+            if (m.x >= thr || m.y >= thr) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) n += (unsigned)(pair(w[j]).x >= thr) + (unsigned)(pair(w[j]).y >= thr);
+            }
+            return n;
+        };
+        unsigned slot = 0;
+        auto list = [&](const uint4& keys, int c) {
+            const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const s16x2_t kk = pair(w[j >> 1]);
                 const int key = j & 1 ? kk.y : kk.x;
                 if (key < thr) continue;
-                const unsigned slot = atomicAdd(&sh_u[2], 1u);
-                if (slot < (unsigned)kSmQuickMost) cand[slot] = (uint64_t)(unsigned)(key + 32768) << 32 | (unsigned)~(c * 8 + j);
+                cand[slot++] = (uint64_t)(unsigned)(key + 32768) << 32 | (unsigned)~(c * 8 + j);
                 if (key == -1) sh_u[4] = 1;                  // -0.0
             }
         };
         if (!sh_u[3]) {   // uniform
+            // counted before anything is listed: a full list costs its rows no more than the count
+            unsigned hits = 0, mine_n = 0;
             if (top >= thr) {
 #pragma unroll
                 for (int i = 0; i < kSmKeep; ++i)
-                    if (in_row(i)) list(keep[i], tid + i * kSmThreads);
-                for (int c = kSmKeep * kSmThreads + tid; c < nvec; c += kSmThreads) list(to_keys(ld16(row + (int64_t)c * 8)), c);
+                    if (in_row(i)) {
+                        const unsigned n = reaching(keep[i]);
+                        hits |= n ? 1u << i : 0u;
+                        mine_n += n;
+                    }
+                for (int c = kSmKeep * kSmThreads + tid; c < nvec; c += kSmThreads) mine_n += reaching(to_keys(ld16(row + (int64_t)c * 8)));
+                if (mine_n) slot = atomicAdd(&sh_u[2], mine_n);
             }
             __syncthreads();
             const unsigned found = sh_u[2];
-            if (found <= (unsigned)kSmQuickMost) {   // uniform
+            if (found > 0 && found <= (unsigned)kSmQuickMost) {   // uniform
                 listed = true;
+                k = min(k, (int)found);
+                if (mine_n) {
+#pragma unroll
+                    for (int i = 0; i < kSmKeep; ++i)
+                        if (hits >> i & 1) list(keep[i], tid + i * kSmThreads);
+                    for (int c = kSmKeep * kSmThreads + tid; c < nvec; c += kSmThreads) list(to_keys(ld16(row + (int64_t)c * 8)), c);
+                }
+                __syncthreads();
                 // place among the candidates by counting who comes before: F threads, one for each, for every part of the
                 // list (whole waves read the same entry); the first k stay
                 unsigned F = 64;
@@ -358,13 +384,11 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
                 }
             }
         }
-        if (!listed) {
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < kSmKeep; ++i) keep[i] = to_keys(keep[i]);   // the values again
-        }
+        if (!listed) __syncthreads();
     }
     if (!listed) {
+    uint4 keep[kSmKeep];
+    load_row(keep);
     auto for_each_chunk = [&](auto&& fn) {  // fn(chunk index, 8 values), every thread the same trip count
 #pragma unroll
         for (int i = 0; i < kSmKeep; ++i) fn(tid + i * kSmThreads, keep[i]);

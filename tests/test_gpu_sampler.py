@@ -68,6 +68,28 @@ def test_selection_through_maxima_equals_radix_selection(mv, v, kind):
         assert torch.equal(sample(a.to(DEV), temps, top_ps, k, uniforms=u), sample(b.to(DEV), temps, top_ps, k, uniforms=u)), k
 
 
+@pytest.mark.parametrize("v,left", [(512, 1), (32000, 10), (32000, 64), (128256, 255), (131080, 300)])
+def test_masked_rows_with_fewer_entries_than_k(mv, v, left):
+    """All but `left` entries at -infinity (a constrained vocabulary): they have no weight, so asking for more entries than
+    there are gives the pick among those there are, also where nothing is cut off by top-p."""
+    from micro_vllm_amd.core.layer.sampler import sample
+
+    g = torch.Generator().manual_seed(v + left)
+    bs = 6
+    x = torch.full((bs, v), -float("inf"))
+    for b in range(bs):
+        x[b, torch.randperm(v, generator=g)[:left]] = (torch.randn(left, generator=g) * 3).to(torch.bfloat16).float()
+    x = x.to(torch.bfloat16).to(DEV)
+    temps, u = torch.rand(bs, generator=g) + 0.5, torch.rand(bs, generator=g)
+    temps[0] = 0.0
+    for top_p in (0.7, 1.0, 1.5):
+        want = sample(x, temps, torch.full((bs,), top_p), left, uniforms=u)
+        assert bool(torch.isfinite(x[torch.arange(bs, device=DEV), want].float()).all())
+        for k in (50, 256, 1000):
+            if k > left:
+                assert torch.equal(sample(x, temps, torch.full((bs,), top_p), k, uniforms=u), want), (top_p, k)
+
+
 def test_sampler_class_uses_device_kernel_and_respects_top_k(mv):
     from micro_vllm_amd.core.layer.sampler import Sampler
 
