@@ -63,7 +63,6 @@ __global__ __launch_bounds__(kAmThreads) void argmax_kernel(const uint16_t* __re
 // the workspace over for the first time and are returned to zero by every launch.  The merge is a maximum under a total order (value, then lowest
 // index), so the result does not depend on arrival order.
 constexpr int kAmPartThreads = 256;
-constexpr int kAmAhead = 4;
 constexpr int kAmMaxParts = 64;
 constexpr int kAmMaxRows = 64;
 constexpr size_t kAmTicketBytes = (size_t)kAmMaxRows * 64 * sizeof(unsigned int);  // 256 bytes apart
@@ -76,6 +75,7 @@ struct AmScratch {
     unsigned int* ticket;
 };
 
+template <int AHEAD>
 __global__ __launch_bounds__(kAmPartThreads) void argmax_parts_kernel(const uint16_t* __restrict__ logits,
                                                                       int64_t ld, int n, int parts,
                                                                       int vec_per_part, AmScratch sc,
@@ -89,12 +89,12 @@ __global__ __launch_bounds__(kAmPartThreads) void argmax_parts_kernel(const uint
     int bi = 0x7fffffff;
     const int nvec = n >> 3;
     const int c0 = part * vec_per_part, c1 = min(nvec, c0 + vec_per_part);
-    for (int b = c0 + threadIdx.x; b < c1; b += kAmAhead * kAmPartThreads) {
-        uint4 v[kAmAhead];   // requested together: a part is one trip to memory, not one per 16 bytes of a thread
+    for (int b = c0 + threadIdx.x; b < c1; b += AHEAD * kAmPartThreads) {
+        uint4 v[AHEAD];   // requested together: a part is one trip to memory, not one per 16 bytes of a thread
 #pragma unroll
-        for (int u = 0; u < kAmAhead; ++u) v[u] = ld16(row + (int64_t)min(b + u * kAmPartThreads, c1 - 1) * 8);
+        for (int u = 0; u < AHEAD; ++u) v[u] = ld16(row + (int64_t)min(b + u * kAmPartThreads, c1 - 1) * 8);
 #pragma unroll
-        for (int u = 0; u < kAmAhead; ++u) {
+        for (int u = 0; u < AHEAD; ++u) {
             const int c = min(b + u * kAmPartThreads, c1 - 1);   // (the last one again: it changes nothing)
             const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
@@ -619,10 +619,11 @@ extern "C" int mv_argmax(const void* logits, int64_t ld, int rows, int n, int64_
     if (!mv::aligned16(logits) || (ld % 8) != 0) return MV_ERR_INVALID_ARG;
     // long rows: several workgroups per row, about two for every compute unit in all, meeting in the caller's
     // workspace (without one, or with too small a one, every row gets a single workgroup: same result, slower).
-    // 32 rows of 128256 in four parts each with one load of a thread in flight: 12.0 us; in sixteen parts with four: 6.6.
+    // 32 rows of 128256 in four parts each with one load of a thread in flight: 12.0 us; in sixteen parts with two: 7.3.
+    // (64 rows of 8192 take 5.1 us whole, 5.3 in parts.)
     const int nvec = n >> 3;
     if (workspace && workspace_bytes >= mv::kAmWorkspaceBytes && mv::aligned16(workspace) &&
-        rows <= mv::kAmMaxRows && nvec >= 4 * mv::kAmPartThreads) {
+        rows <= mv::kAmMaxRows && nvec >= (rows * 8 <= mv::num_cus() ? 4 : 8) * mv::kAmPartThreads) {
         const mv::AmScratch sc = mv::am_scratch(workspace);
         int parts = 2 * mv::num_cus() / rows;
         if (parts > mv::kAmMaxParts) parts = mv::kAmMaxParts;
@@ -630,9 +631,11 @@ extern "C" int mv_argmax(const void* logits, int64_t ld, int rows, int n, int64_
         if (parts > most) parts = most;
         if (parts >= 2) {
             const int vec_per_part = (nvec + parts - 1) / parts;
-            hipLaunchKernelGGL(mv::argmax_parts_kernel, dim3(rows * parts), dim3(mv::kAmPartThreads), 0,
-                               (hipStream_t)stream, (const uint16_t*)logits, ld, n, parts, vec_per_part,
-                               sc, ids);
+            // as many loads of a thread in flight as its part has: one row of 8192 in single loads 5.0 us, in fours 6.0
+            const auto kernel = vec_per_part <= mv::kAmPartThreads ? mv::argmax_parts_kernel<1>
+                                : vec_per_part <= 2 * mv::kAmPartThreads ? mv::argmax_parts_kernel<2> : mv::argmax_parts_kernel<4>;
+            hipLaunchKernelGGL(kernel, dim3(rows * parts), dim3(mv::kAmPartThreads), 0, (hipStream_t)stream,
+                               (const uint16_t*)logits, ld, n, parts, vec_per_part, sc, ids);
             return mv::check_launch();
         }
     }
