@@ -328,10 +328,12 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
                         acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[a][e], xf[b][e], acc[a][b], 0, 0, 0);
         }
     };
-    const int steps = KG > 1 ? per : 4 * per;   // of every group alike: the barriers are shared; past the end of k: zeros
 #pragma unroll
     for (int i = 0; i < PF; ++i) request(i, i);
     constexpr int TURN = PF > 2 ? PF : 2;   // steps after which register sets and halves are where they were
+    // Side by side the groups share the barriers, and a step past the end of k multiplies zeros.  One after the other the
+    // quarters end with k, at a whole turn: left-over steps behind the loop cost it a seventh of its pace.
+    const int steps = KG > 1 ? per : ((K + kLfBK - 1) / kLfBK + TURN - 1) / TURN * TURN;
     int st = 0;
     for (; st + TURN <= steps; st += TURN)
 #pragma unroll
@@ -557,10 +559,12 @@ static int launch_linear_f32_tiles(const float* x, int64_t ldx, const float* w, 
 }
 
 // Which fp32 form.  Few rows of one product stream the weights (see kStreamRows).  Otherwise the tile by the time the
-// launch takes in it: rounds of tiles over the compute units times what a tile costs a unit, in us per 1024 of k as
-// measured - 8 for 32 x 32 (four groups over k), 24 for a 64 x 64 tile by itself and 19 where several share a unit, 73
-// for 128 x 128 - so that a launch of few tiles takes small ones and a large one the tile that reads its operands least
-// often.  With segments `m` bounds a segment, not the launch: the rows are taken to be spread evenly.
+// launch takes in it: rounds of tiles over the compute units times what a tile costs a unit, in hundredths of a us as measured,
+// per k-step of 32 and for its start and end - 32 x 32 (four groups, a quarter of the steps each) 200 + 88 a step of a quarter, 64 x
+// 64 200 + 73 by itself and 200 + 59 where several share a unit, 128 x 128 1200 + 228 - so that a launch of few tiles takes
+// small ones and a large one the tile that reads its operands least often, at a short k later than at a long one: 1024 rows 4096 x 128
+// in 64 x 64 17.9 us, in 128 x 128 22.3; 1024 rows of 32 heads 128 x 64 55 and 123.  With segments `m` bounds a
+// segment, not the launch: the rows are taken to be spread evenly.
 static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
                              int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s, mv::RowSegments sg,
                              int total_rows) {
@@ -573,7 +577,9 @@ static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_
     const int64_t per = sg.seg ? (total_rows + batch - 1) / batch : m;
     const int64_t cus = num_cus();
     auto rounds = [&](int b) { return (((per + b - 1) / b) * ((n + b - 1) / b) * batch + cus - 1) / cus; };
-    const int64_t c32 = 8 * rounds(32), c64 = rounds(64) <= 1 ? 24 : 19 * rounds(64), c128 = 73 * rounds(128);
+    const int64_t steps = (k + kLfBK - 1) / kLfBK;
+    const int64_t c32 = rounds(32) * (200 + 88 * ((steps + 3) / 4)), c128 = rounds(128) * (1200 + 228 * steps);
+    const int64_t c64 = rounds(64) <= 1 ? 200 + 73 * steps : rounds(64) * (200 + 59 * steps);
     if (c32 <= c64 && c32 <= c128)
         return launch_linear_f32_tiles<1, 1, 4, 4>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
     if (c64 <= c128)
