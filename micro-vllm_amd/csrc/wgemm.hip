@@ -1033,15 +1033,19 @@ static int launch_ordered_mb(const GemmArgs& a, int sg, int ks, int grid, hipStr
     }
 }
 
-// One block of rows (up to 16), or few k-tiles times blocks on enough strips: a wave walks its slice alone, and past that its
-// chain of loads, or on many strips the x each of them reads again, is longer than the sliced tiles and their reduction.
-// Measured (n x k, us, sliced tiles -> here): 5 rows 2048 x 5632 13.6 -> 9.5, 4096 x 14336 31.6 -> 22.4;
-// 37 rows 2560 x 2048 11.7 -> 9.0, 6144 x 4096 19.1 -> 17.9, 8192 x 1024 12.6 -> 8.8, but 1024 x 4096 12.1 -> 14.6,
-// 1280 x 8192 15.2 -> 24.8 and 4096 x 14336 34.0 -> 46.5; 64 rows 2560 x 2048 14.0 -> 12.2, 11264 x 2048 20.3 -> 23.7.
+// One block of rows (up to 16), or rows times the k-tiles a wave walks up to a limit, on enough strips: a wave walks its slice (of
+// sixteen, two) alone, each k-tile in the time its rows take, and past that its chain, or on many strips the x each of them reads
+// again, is longer than the sliced tiles and their reduction.  The limits lie between what was faster and what was not (n x
+// k, us, 64-row sliced tiles -> here).  Eight and four slices, 512: 64 rows 2560 x 2048 13.1 -> 12.1 and 8192 x 1024 15.0 -> 13.5, 32 rows
+// 16384 x 2048 18.8 -> 16.6 (all 512), but 37 rows (592) 11264 x 2048 16.7 -> 17.7 and 6144 x 4096 17.2 -> 17.7, 64 rows 5120 x 3072
+// (768) 17.0 -> 19.8 and 8192 x 2048 (1024) 16.3 -> 22.7.  Long slices, 448: 17 rows 2048 x 5632 (374) 10.4 -> 12.0 where 128-row tiles took
+// 13.2, 24 rows (528) 10.7 -> 14.2.  Sixteen slices, whose reduction reads most, 592: 37 rows 4096 x 4096 16.5 -> 15.6, 48 rows (768)
+// 17.5 -> 17.6.
 bool wgemm_ordered_takes(int m, int nt, int kt, int ks) {
-    const int blocks = (m + 15) / 16;
+    const int blocks = (m + 15) / 16, walk = ks == 4 ? kt / 4 : kt / 8;
     if ((ks != 4 && ks != 8 && ks != 16) || blocks > 4) return false;
-    return blocks == 1 || (blocks * kt <= 384 && nt >= 128 && (int64_t)blocks * kt * nt <= 150000);
+    const int most = ks == 16 ? 592 : walk > 16 ? 448 : 512;
+    return blocks == 1 || (m * walk <= most && blocks * kt <= 384 && nt >= 128 && (int64_t)blocks * kt * nt <= 150000);
 }
 
 // x [m, k] . W^T with the sums of `ks` slices of k added in order, epilogue as mv_gemm_prefill_ws, or the norm's.

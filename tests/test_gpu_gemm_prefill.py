@@ -409,7 +409,7 @@ def test_gemm_prefill_k_slices(mv, m, n, k, mode):
 @pytest.mark.parametrize("m", [1, 16, 17, 37, 48, 49, 64])
 @pytest.mark.parametrize("n,k,mode", [(16, 2048, "plain"), (256, 8192, "f32"), (1280, 8192, "bias"),
                                       (2048, 5632, "residual"), (4096, 4096, "plain"), (11264, 2048, "swiglu"),
-                                      (6160, 4096, "residual")])
+                                      (6160, 4096, "residual"), (8192, 1024, "plain"), (2560, 2048, "residual")])
 def test_few_rows_add_the_slices_in_order(mv, m, n, k, mode):
     """Up to 16 rows, and with a short k up to 64, the k-slices are added within a workgroup.  The result is that of the slices' own products added in
     order, bit for bit (4, 8 and 16 slices, one to four blocks of rows, n that leaves a part of a workgroup's columns
