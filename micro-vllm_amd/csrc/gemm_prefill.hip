@@ -1146,17 +1146,17 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     }
     const long grid = 8L * a.nb_per_xcd * a.mblocks * a.ksplit;
     if (grid > 0x7fffffffL) return MV_ERR_UNSUPPORTED;
-    // 64-row tiles while each has a compute unit to itself, else 128-row tiles in the deep form (from 16 stages: shorter
+    // 64-row tiles while each has a compute unit to itself, else 128-row tiles in the deep form (from 20 stages: shorter
     // slices end before its ring has paid), else two workgroups to a unit.  Measured against the last (us): 512 x 6144 x 2048
     // 44.8 -> 28.3 and 256 x 16384 x 2048 47.2 -> 31.9 in 64-row tiles, 1408 x 2048 x 2048 39.0 -> 24.0, 1024 x 4096 x 4096 in
-    // two slices 54.4 -> 49.7 in the deep form (64-row tiles in two rounds: 61.3), 192 x 6144 x 2048 in four 24.8 as it was
-    // (deep 25.4, 64 rows 29.1).
+    // two slices 54.4 -> 49.7 in the deep form (64-row tiles in two rounds: 61.3), 700 x 2048 x 5632 in four (22 stages) 36.8 -> 35.6;
+    // but 192 x 6144 x 2048 in four (8 stages) 24.8, deep 25.4, and 96 x 7168 x 8192 in eight (16) 34.1, deep 35.7.
     const int mblocks64 = (m + 63) / 64;
     const long grid64 = 8L * a.nb_per_xcd * mblocks64 * a.ksplit;
     if (grid64 <= num_cus()) {
         a.mblocks = mblocks64;
         hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4>), dim3((unsigned)grid64), dim3(256), 0, (hipStream_t)stream, a);
-    } else if (grid <= num_cus() && a.ktps >= 32) {
+    } else if (grid <= num_cus() && a.ktps >= 40) {
         hipLaunchKernelGGL((gemm_prefill_kernel<8, 8, 4>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
     } else {
         hipLaunchKernelGGL((gemm_prefill_kernel<8, 3, 3>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
