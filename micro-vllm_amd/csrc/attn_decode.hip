@@ -86,11 +86,12 @@ __device__ __forceinline__ void stage_qkv_from_slabs(const AttnArgs& a, uint16_t
 template <int D, int G, int W>
 __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     constexpr int kAW = W;          // waves per workgroup
-    // Row loads per wave per pipeline stage.  With more than four query heads two: four take 305 registers (one
+    // Row loads per wave per pipeline stage.  With more than four query heads of 64 two: four take 305 registers (one
     // workgroup a unit, and twice the arithmetic of a stage that a short context hardly fills).  32 heads of 64 on 4:
     // 45 tokens 9.2 -> 8.0 us, one row of 4000 13.3 -> 12.7, 32 rows of 2000 in 4 splits 43 -> 32.  With four heads or
-    // fewer a second workgroup fits either way, and bytes in flight set the pace of long rows.
-    constexpr int kAC = G > 4 ? 2 : 4;
+    // fewer a second workgroup fits either way, and bytes in flight set the pace of long rows; so they do for heads of 128:
+    // 28 on 4, 64 rows of 8000 in two loads 265 us, in four 252.
+    constexpr int kAC = G > 4 && D == 64 ? 2 : 4;
     constexpr int LPR = D / 8;      // lanes per row
     constexpr int RPI = 64 / LPR;   // rows per wave instruction
     constexpr int NS = kAW * RPI;   // softmax states per workgroup
@@ -174,9 +175,6 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
 #ifdef MV_ATTN_STAMP
     if (pos >= 0) MV_ASTAMP(11);
 #endif
-    // (behind the requests above: a split with tokens does not wait for the length before it makes them)
-    __builtin_amdgcn_sched_barrier(0);
-    if (split >= filled && (a.nsplit == 1 || a.arrive)) return;   // uniform; nothing of this row is here
     uint4 cosv = make_uint4(0, 0, 0, 0), sinv = cosv;
     if (rotate) {
         const int rp = min(max(pos, 0), a.rot_max_pos - 1);
@@ -208,6 +206,9 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     load_pages(pgA, 2);
     load_rows(kB, vB, okB, pgB, 1);
     load_pages(pgB, 3);
+    // behind the requests above: a split with tokens does not wait for the length before it makes them (in front of them
+    // the test cost 0.2 to 0.4 us of 10 wherever most splits have tokens)
+    if (split >= filled && (a.nsplit == 1 || a.arrive)) return;   // uniform; nothing of this row is here
 
     // ---- q (G heads) and the new k/v: rotate, round -------------------------------
     uint32_t qp[G][4];
