@@ -353,7 +353,7 @@ int mv_store_kv(const void* key, const void* value, int64_t kv_stride_t, void* k
 /* All layers of a Llama-shaped prefill on one GPU in one call (core/layer/model_prefill.py:36-59 per layer): `rows`
  * sequences of `seq` tokens, h [rows * seq, hidden] bf16 in place.  tensors: per layer nine device pointers - ln_1 weight,
  * QKV tiles, QKV bias or NULL, O tiles, ln_2 weight, gate/up tiles (interleaved, mv_interleave_rows8), down tiles, key
- * cache, value cache; eps: per layer the two norms' epsilons.  Scratch, 16-byte aligned: normed, resid [T, hidden],
+ * cache, value cache (of num_pages pages in every layer); eps: per layer the two norms' epsilons.  Scratch, 16-byte aligned: normed, resid [T, hidden],
  * qkv [T, (Hq + 2 Hkv) D], attn [T, Hq D], act [T, inter], all bf16, and proj, T * hidden floats.  workspace: of
  * mv_llama_prefill_workspace_bytes, as for mv_gemm_prefill_ws (zero-filled when it was allocated).  Results are those of
  * the layer's ops called one by one, bit for bit. */
@@ -540,7 +540,7 @@ int mv_scan_outer(const float* q, int64_t ldq, int q_div, const float* k, int64_
  * + ch_len[c] (<= 64) of one row; row b owns chunks row_ch0[b] .. + row_nch[b] (0: the row is not taken -
  * mv_scan_outer with max_len > 0 leaves exactly the rows longer than max_len to this call).  The decay
  * comes as its logarithm ([tokens, heads], or [heads] with ld_ld == 0).  Scratch: ds [chunks, heads, n, p],
- * lsum [tokens, heads], atot [chunks, heads], all fp32.  Differs from the token-by-token form by the
+ * lsum [tokens, heads], atot [chunks, heads], all fp32 (rows taken whole use ds alone, for the scores).  Differs from the token-by-token form by the
  * order of the fp32 sums only.  MV_ERR_UNSUPPORTED when n and p need more LDS than a workgroup has
  * (mv_scan_chunked_lds_bytes(n, p) > 150 KiB). */
 size_t mv_scan_chunked_lds_bytes(int n, int p);

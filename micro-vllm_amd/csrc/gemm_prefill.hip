@@ -863,7 +863,9 @@ namespace mv {
 // k-slices for an M x N product over kt k-tiles: none when the output tiles alone fill the chip.
 // Otherwise a small cost model picks the count (measured on MI355X: a workgroup walks k at about
 // 1.1 us per 64-k stage when the chip is mostly idle; the slices cost a second launch, about 4 us,
-// plus writing and re-reading ks x M x N floats at about 3 TB/s).  One 256 x 128 tile per
+// plus writing and re-reading ks x M x N floats at about 3 TB/s; 64-row tiles and the deep form, which small grids take
+// since, walk a stage in 0.7 to 1.0 us, so whole k is priced a little high against slices - the count is kept, since
+// it is also the order of the sums).  One 256 x 128 tile per
 // workgroup walks k serially: at 128 tokens the QKV projection of the 8B shape has 24 tiles and
 // took 70 us with nine tenths of the chip idle, 29 us split; the gate/up projection at 256 tokens
 // (224 tiles) is faster unsplit because its slices would be 117 MB.

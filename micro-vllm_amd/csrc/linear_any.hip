@@ -8,10 +8,12 @@
 //                  v_mfma_f32_16x16x32_bf16, edges zero-filled in LDS; the sum over k in ascending order of those
 //                  steps;
 //   fp32 operands: tiles of three sizes on the fp32 matrix instruction (no reduced-precision mode), or, for a few
-//                  rows, the weights streamed past them.  In every form a sum over k is made of four quarters of k
+//                  rows, the weights streamed past them.  In all of these a sum over k is made of four quarters of k
 //                  (in whole steps of 32) that are added up in ascending order, a quarter of the same sequence of
 //                  matrix instructions.
-// So a row's result does not depend on which other rows share the launch.
+// So in one product (mv_linear_any) a row's result does not depend on which other rows share the launch.  A launch of
+// several products (heads, expert segments) has another form for up to kFewRows rows, linear_fewrows_kernel, whose lanes
+// add every 64th piece of k and then each other: there a row's last bits differ from those of a larger launch.
 #include "common.h"
 #include <type_traits>
 

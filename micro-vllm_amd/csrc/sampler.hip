@@ -619,7 +619,7 @@ extern "C" int mv_argmax(const void* logits, int64_t ld, int rows, int n, int64_
     if (!mv::aligned16(logits) || (ld % 8) != 0) return MV_ERR_INVALID_ARG;
     // long rows: several workgroups per row, about two for every compute unit in all, meeting in the caller's
     // workspace (without one, or with too small a one, every row gets a single workgroup: same result, slower).
-    // 32 rows of 128256 in four parts each with one load of a thread in flight: 12.0 us; in sixteen parts with two: 7.3.
+    // 32 rows of 128256 in four parts each with one load of a thread in flight: 12.0 us; in sixteen parts with four: 7.3.
     // (64 rows of 8192 take 5.1 us whole, 5.3 in parts.)
     const int nvec = n >> 3;
     if (workspace && workspace_bytes >= mv::kAmWorkspaceBytes && mv::aligned16(workspace) &&

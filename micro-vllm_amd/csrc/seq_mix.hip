@@ -581,11 +581,13 @@ __global__ __launch_bounds__(256) void scan_chunk_inter_kernel(ChunkArgs a) {
 //           of S = exp(L_end) S0 + k^T (w v).  The two kinds run side by side, one of each to a SIMD: S0 goes to the others
 //           through LDS, two buffers, one barrier a chunk; the next chunk's q, k and scores are in flight to registers.
 // The contraction index of a product is dealt out as 16 a + 4 g + e (e: step of the instruction), so a lane's operands of
-// four steps are one 16-byte read.  A chunk takes a SIMD 160 of the fp32 instruction at 32 cycles (2.1 us at 32 columns) and
-// measures 4.5: sums that wait for each other, exponentials, the barrier.  16 columns a workgroup, two workgroups to a unit,
-// read q and k twice as often: 203 against 155 us.  Both launches, against the three above with the chunks' states written,
-// carried and read back (us, n = 128, p = 64): 128 heads in one group, 2048 tokens 727 -> 155; 100 tokens 193 -> 20; 16 heads
-// with q and k of their own, 2048 tokens 157 -> 121, 333 tokens 74 -> 32; 24 heads, n = 64, 65 + 65 + 65 + 900 tokens 124 -> 50.
+// four steps are one 16-byte read.  What a chunk adds to the state, and its own part of an output, have accumulators of their own:
+// rounded at the state's size sixteen times a chunk, states were three times as far from 64 bits.  A chunk takes a SIMD 160 of
+// the fp32 instruction at 32 cycles (2.1 us at 32 columns) and measures 4.2: sums that wait for each other, exponentials, the
+// barrier.  16 columns a workgroup, two workgroups to a unit, read q and k twice as often: 203 against 155 us when that was tried.
+// Both launches, against the three above with the chunks' states written, carried and read back (us, n = 128, p = 64): 128 heads
+// in one group, 2048 tokens 693 -> 136; 100 tokens 188 -> 18; 16 heads with q and k of their own, 2048 tokens 153 -> 111, 333
+// tokens 71 -> 31; 24 heads, n = 64, 65 + 65 + 65 + 900 tokens 70 -> 55.
 __global__ __launch_bounds__(256) void scan_scores_kernel(ChunkArgs a, float* scores) {
     const int ch = blockIdx.x, grp = blockIdx.y, tt = blockIdx.z;
     const int st = threadIdx.x >> 6, r = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
@@ -1791,9 +1793,9 @@ __global__ __launch_bounds__(256) void window_attn_group_kernel(const float* q, 
 // other splits leave at once; else a split leaves (max, sum, weighted values) in `part` for window_attn_merge_kernel.
 //
 // Measured (us per call, 8 heads on 2 key/value heads, d = dv = 128, window 1024; kernel above with its 64-key tiles, five
-// splits and their merge -> here): one token bf16 at 45 keys 19.0 -> 7.8, 300 21.7 -> 11.4, 1100 23.2 -> 20.3; fp32 19.0 -> 8.0,
-// 22.6 -> 14.1, 26.9 -> 24.0; 64 tokens bf16 21.4 -> 8.1, 26.7 -> 12.4, 51.2 -> 27.9; a prompt of 333 in fp32 at 300 58.8 -> 40.8.
-// 16 heads of 64 with keys of their own, one token 10.4 -> 4.5, 11.5 -> 6.8, 14.5 -> 12.6.
+// splits and their merge -> here): one token bf16 at 45 keys 19.5 -> 8.0, 300 21.8 -> 11.4, 1100 23.2 -> 19.1; fp32 19.8 -> 8.1,
+// 23.6 -> 13.9, 25.1 -> 17.0; 64 tokens bf16 20.5 -> 8.3, 23.1 -> 12.1, 32.9 -> 21.2; a prompt of 333 in fp32 at 300 53.7 -> 40.
+// 16 heads of 64 with keys of their own, one token 10.6 -> 4.7, 11.7 -> 7.0, 12.2 -> 11.8.
 struct TileRun {
     int lo, kept, nk, n;      // n tiles: nk of the kept positions [0, kept), then those of [lo, pos]
 };
