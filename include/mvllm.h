@@ -213,6 +213,15 @@ size_t mv_gemm_prefill_workspace_bytes(int m, int n, int k);
 int mv_gemm_prefill_ws(const void* x, int64_t ldx, const void* w_tiles, const void* bias,
                        const void* residual, int64_t ld_res, void* y, int64_t ldy, int m, int n,
                        int k, int flags, void* workspace, size_t workspace_bytes, mv_stream_t stream);
+/* x [m, k] bf16 times a weight in wave tiles (mv_shuffle_weight), left in `slabs` as mv_linear_slab_count(m, n, k) k-slices
+ * [slice][m][n] fp32 whose sum, in order, is the product - for a caller whose next kernel adds them
+ * (mv_postnorm_residual_slabs, mv_add_rmsnorm_slabs).  Any m; n % 16 == 0, k % 64 == 0.  workspace: of
+ * mv_linear_slabs_workspace_bytes, zero-filled when it was allocated and used for nothing else (as for
+ * mv_gemm_prefill_ws). */
+int mv_linear_slab_count(int m, int n, int k);
+size_t mv_linear_slabs_workspace_bytes(int m, int n, int k);
+int mv_linear_slabs(const void* x, int64_t ldx, const void* w_tiles, float* slabs, size_t slabs_bytes, int m, int n, int k,
+                    void* workspace, size_t workspace_bytes, mv_stream_t stream);
 /* Which form a call of that shape takes on the current device (for tests and tools; no counterpart
  * in the reference): 0 = 128 x 256 tiles, two workgroups per CU, weights straight into registers;
  * 1 = 256 x 256 tiles, one workgroup per CU, both operands through LDS (taken when its tiles fill
@@ -499,6 +508,12 @@ int mv_postnorm_residual(const float* y1, int64_t ld1, const float* y2, int64_t 
                          const float* bias, const float* w, float eps, float mult, const float* next_w, float* x,
                          int64_t ldx, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream);
 
+/* The same with y1 and y2 as their projections left them in k-slices: y1 = sum over i < ks1 of y1 + i * rows * ld1, in order
+ * (mv_linear_slabs; ks1 = 1: whole). */
+int mv_postnorm_residual_slabs(const float* y1, int64_t ld1, int ks1, const float* y2, int64_t ld2, int ks2, float s1,
+                               float s2, const float* bias, const float* w, float eps, float mult, const float* next_w,
+                               float* x, int64_t ldx, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream);
+
 /* out[r,:] = act( x[idx[r],:] / sqrt(mean(.^2) + eps) * (1 + w) ); idx == NULL: row r itself. */
 int mv_offset_rmsnorm_gather(const float* x, int64_t ldx, const int32_t* idx, const float* w, float eps, void* out,
                              int64_t ldo, int rows, int n, int f32, mv_stream_t stream);
@@ -650,6 +665,9 @@ int mv_embed_pair(const void* table, const void* pairs, const int32_t* ids, cons
 /* x += y1 (+ y2) (y1 == NULL: x as it is); w != NULL: h = act( x / sqrt(mean(x^2) + eps) * w ). */
 int mv_add_rmsnorm(const float* y1, int64_t ld1, const float* y2, int64_t ld2, float* x, int64_t ldx, const float* w,
                    float eps, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream);
+/* The same with y1 in ks1 k-slices, rows * ld1 floats apart, added in order. */
+int mv_add_rmsnorm_slabs(const float* y1, int64_t ld1, int ks1, const float* y2, int64_t ld2, float* x, int64_t ldx,
+                         const float* w, float eps, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream);
 /* out[r,:] = act( x[idx[r],:] / sqrt(mean(.^2) + eps) * (offset + w) ); idx == NULL: row r itself. */
 int mv_rmsnorm_gather(const float* x, int64_t ldx, const int32_t* idx, const float* w, float eps, float offset,
                       void* out, int64_t ldo, int rows, int n, int f32, mv_stream_t stream);

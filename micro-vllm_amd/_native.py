@@ -68,6 +68,9 @@ PROTOTYPES = {
                                           _I, _I, _I, _I, _I, _I, _F, _I, _P]),
     "mv_gemm_prefill": (_I, [_P, _L, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _P]),
     "mv_gemm_prefill_workspace_bytes": (_Z, [_I, _I, _I]),
+    "mv_linear_slab_count": (_I, [_I, _I, _I]),
+    "mv_linear_slabs_workspace_bytes": (_Z, [_I, _I, _I]),
+    "mv_linear_slabs": (_I, [_P, _L, _P, _P, _Z, _I, _I, _I, _P, _Z, _P]),
     "mv_gemm_prefill_form": (_I, [_I, _I, _I]),
     "mv_debug_prefill_options": (None, [_I, _I]),
     "mv_paged_attn_prefill_form": (_I, [_I, _I, _I, _I]),
@@ -97,6 +100,7 @@ PROTOTYPES = {
     "mv_linear_any": (_I, [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _P]),
     "mv_embed_scaled": (_I, [_P, _P, _P, _L, _P, _L, _I, _I, _I, _F, _P, _F, _F, _I, _P]),
     "mv_postnorm_residual": (_I, [_P, _L, _P, _L, _F, _F, _P, _P, _F, _F, _P, _P, _L, _P, _L, _I, _I, _I, _P]),
+    "mv_postnorm_residual_slabs": (_I, [_P, _L, _I, _P, _L, _I, _F, _F, _P, _P, _F, _F, _P, _P, _L, _P, _L, _I, _I, _I, _P]),
     "mv_offset_rmsnorm_gather": (_I, [_P, _L, _P, _P, _F, _P, _L, _I, _I, _I, _P]),
     "mv_relu_squared": (_I, [_P, _L, _P, _L, _I, _I, _I, _P]),
     "mv_softcap": (_I, [_P, _L, _F, _P]),
@@ -118,6 +122,7 @@ PROTOTYPES = {
     "mv_gated_act": (_I, [_P, _L, _P, _L, _I, _I, _I, _F, _F, _I, _P]),
     "mv_embed_pair": (_I, [_P, _P, _P, _P, _P, _L, _I, _I, _I, _L, _L, _L, _F, _P, _F, _P, _L, _I, _P]),
     "mv_add_rmsnorm": (_I, [_P, _L, _P, _L, _P, _L, _P, _F, _P, _L, _I, _I, _I, _P]),
+    "mv_add_rmsnorm_slabs": (_I, [_P, _L, _I, _P, _L, _P, _L, _P, _F, _P, _L, _I, _I, _I, _P]),
     "mv_rmsnorm_gather": (_I, [_P, _L, _P, _P, _F, _F, _P, _L, _I, _I, _I, _P]),
     "mv_moe_route_scored": (_I, [_P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _F, _F, _I, _P]),
     "mv_dyt_shift": (_I, [_P, _L, _P, _P, _P, _P, _P, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _P]),

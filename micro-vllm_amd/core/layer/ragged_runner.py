@@ -490,7 +490,7 @@ class RaggedRunner:
                        q_div=H // G, k_div=H // G, log_decay=log_decay, chunked=self.chunked_scan)
         u = self._actbuf(T, inner)
         ops.gated_group_norm(y, proj[:, :inner], w["norm"], u, groups=s["norm_groups"], gate_first=True, eps=eps)
-        return w["w_o"](u, self._f32buf(T, self.width)), None
+        return w["w_o"].slabs(u, self._f32buf), None
 
     def _parallel(self, li, w, m, h, step: RaggedStep, cache: HybridCacheManager):
         T, eps = step.tokens, self.cfg.eps
@@ -505,7 +505,7 @@ class RaggedRunner:
         part = self._f32buf(1, T * H * splits * (dv + 2)) if splits else None
         ops.window_attn(qkv, kc, vc, a, step, w["slopes"], H, G, d, dv, float(L["scale"]), window, tiled=self.tiled_attn,
                         part=part, splits=splits)
-        left = w["left_o"](a, self._f32buf(T, self.width))
+        left = w["left_o"].slabs(a, self._f32buf)
 
         Hr, dr, dvr, rot = int(R["heads"]), int(R["dim"]), int(R["vdim"]), int(R["rot"]["dims"])
         qkvg = w["right_qkvg"](h, self._f32buf(T, w["right_qkvg"].n))
@@ -518,7 +518,7 @@ class RaggedRunner:
                        step=step, heads=Hr, n=dr, p=dvr, log_decay=w["log_decay"], chunked=self.chunked_scan)
         u = self._actbuf(T, Hr * dvr)
         ops.gated_group_norm(o, g, None, u, groups=Hr, gate_first=False, eps=eps)
-        return left, w["right_o"](u, self._f32buf(T, self.width))
+        return left, w["right_o"].slabs(u, self._f32buf)
 
     @torch.inference_mode()
     def forward(self, step: RaggedStep, cache: HybridCacheManager, want: Optional[torch.Tensor] = None,
@@ -633,7 +633,7 @@ class RaggedRunner:
                     up = w["up"](h, self._f32buf(T, w["up"].n))
                     act = self._actbuf(T, up.shape[1])
                     ops.relu_squared(up, act)
-                    ops.postnorm_residual(w["down"](act, self._f32buf(T, self.width)), w["norm2"], cfg.eps, x, h)
+                    ops.postnorm_residual(w["down"].slabs(act, self._f32buf), w["norm2"], cfg.eps, x, h)
                 if residuals is not None:
                     residuals.append(x.clone())
         rows = T if want is None else want.numel()
@@ -687,7 +687,7 @@ class RaggedRunner:
                         tiled=self.tiled_attn, keep_first=keep, sinks=w["sink"], part=part, splits=splits)
         if dense and not fuse_act:
             ops.gated_act(act[0], act[1], act[2])
-        y1 = w["w_out"](cat, self._f32buf(T, self.width))
+        y1 = w["w_out"].slabs(cat, self._f32buf)
         if not mlp or dense:
             return y1, None
         return y1, self._routed_with_pass(w, mlp, h, T)
@@ -848,7 +848,7 @@ class RaggedRunner:
                 act = self._actbuf(T, ff)
                 ops.gated_act(w["gate_up"](h, self._f32buf(T, 2 * ff)), act, ops.GATE_CLAMPED, float(mlp["limit"]),
                               dugazen.GATE_SLOPE)
-                y, bias = w["down"](act, self._f32buf(T, self.width)), None
+                y, bias = w["down"].slabs(act, self._f32buf), None
                 ops.postnorm_residual(y, w["norm2b"], eps, x, out, mult=mult, next_w=nxt)
             else:
                 ops.postnorm_residual(y, w["norm1b"], eps, x, out, bias=bias, mult=mult, next_w=nxt)
@@ -866,7 +866,7 @@ class RaggedRunner:
         u = self._actbuf(T, H * p)
         ops.delta_rule(qkv, gates[:, :H * n], gates[:, H * n:], beta, w["dt_bias"], w["a_log"], w["norm"], st["delta"], u,
                        step, K, H, n, p, self.cfg.eps, chunked=self.chunked_scan)
-        return w["w_o"](u, self._f32buf(T, self.width))
+        return w["w_o"].slabs(u, self._f32buf)
 
     def _dugazen_attention(self, li, w, m, h, step: RaggedStep, cache: HybridCacheManager, v_first):
         T = step.tokens
@@ -883,7 +883,7 @@ class RaggedRunner:
         part = self._f32buf(1, T * H * splits * (dv + 2)) if splits else None
         ops.window_attn(proj[:, :H * d], kc, vc, a, step, None, H, G, d, dv, float(m["scale"]), window,
                         tiled=self.tiled_attn, part=part, splits=splits, gate=proj[:, C:C + H * dv])
-        return w["w_o"](a, self._f32buf(T, self.width))
+        return w["w_o"].slabs(a, self._f32buf)
 
     # ------------------------------------------------------------------ Sizizen layers
     def _sizizen_stack(self, step: RaggedStep, cache: HybridCacheManager, residuals, x, h, normed):

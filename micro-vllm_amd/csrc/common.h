@@ -141,6 +141,10 @@ int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const 
 // gemm_prefill.hip: mv_gemm_prefill_ws, whose reduction of k-slices (where it has one) also does `norm`
 int gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
                      int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int flags, void* workspace,
-                     size_t workspace_bytes, PostNorm* norm, mv_stream_t stream);
+                     size_t workspace_bytes, PostNorm* norm, mv_stream_t stream, bool keep_slices = false);
+// wgemm.hip: k-slices of a projection of up to 64 rows whose slices the next kernel adds, and the projection
+int wgemm_slices(int m, int n, int k);
+int launch_wgemm_slices(const void* x, int64_t ldx, const void* w_tiles, float* slabs, size_t slabs_bytes, int m, int n, int k,
+                        mv_stream_t stream);
 
 }  // namespace mv

@@ -1041,9 +1041,32 @@ extern "C" int mv_gemm_prefill_ws(const void* x, int64_t ldx, const void* w_tile
                                 nullptr, stream);
 }
 
+extern "C" int mv_linear_slab_count(int m, int n, int k) {
+    using namespace mv;
+    if (m <= 0 || n <= 0 || k <= 0 || (n % 16) != 0 || (k % 64) != 0) return 0;
+    return m <= 64 ? wgemm_slices(m, n, k) : prefill_plan(m, n, k / 32).ks;
+}
+
+extern "C" size_t mv_linear_slabs_workspace_bytes(int m, int n, int k) {
+    // (the slices themselves go to the caller's buffer: left are the cut tiles of a product that is not sliced)
+    return m > 64 && mv_linear_slab_count(m, n, k) == 1 ? mv_gemm_prefill_workspace_bytes(m, n, k) : 0;
+}
+
+extern "C" int mv_linear_slabs(const void* x, int64_t ldx, const void* w_tiles, float* slabs, size_t slabs_bytes, int m, int n,
+                               int k, void* workspace, size_t workspace_bytes, mv_stream_t stream) {
+    if (m == 0 && n > 0 && k > 0) return MV_OK;
+    if (!x || !w_tiles || !slabs || m < 0 || n <= 0 || k <= 0) return MV_ERR_INVALID_ARG;
+    if ((n % 16) != 0 || (k % 64) != 0) return MV_ERR_UNSUPPORTED;
+    if (!mv::aligned16(slabs)) return MV_ERR_INVALID_ARG;
+    if (slabs_bytes < (size_t)mv_linear_slab_count(m, n, k) * m * n * sizeof(float)) return MV_ERR_WORKSPACE;
+    if (m <= 64) return mv::launch_wgemm_slices(x, ldx, w_tiles, slabs, slabs_bytes, m, n, k, stream);
+    return mv::gemm_prefill_run(x, ldx, w_tiles, nullptr, nullptr, 0, slabs, n, m, n, k, MV_GEMM_OUT_F32, workspace,
+                                workspace_bytes, nullptr, stream, true);
+}
+
 int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
                          int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int flags, void* workspace,
-                         size_t workspace_bytes, PostNorm* norm, mv_stream_t stream) {
+                         size_t workspace_bytes, PostNorm* norm, mv_stream_t stream, bool keep_slices) {
     if (norm) norm->done = false;
     if (m == 0) return MV_OK;
     if (!x || !w_tiles || !y || m < 0 || n <= 0 || k <= 0) return MV_ERR_INVALID_ARG;
@@ -1088,7 +1111,9 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     bool wide = plan.wide;
     if (a.ksplit > 1) {
         const size_t need = (size_t)a.ksplit * m * n * sizeof(float);
-        if (data && data_bytes >= need) {
+        if (keep_slices) {
+            a.partial = (float*)y;      // the caller's kernel adds them (room checked by mv_linear_slabs)
+        } else if (data && data_bytes >= need) {
             a.partial = (float*)data;
         } else {
             a.ksplit = 1;  // no room for the slices: whole k per tile (slower, same result class)
@@ -1098,10 +1123,11 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     // Up to 64 rows a tile of 128 is mostly padding, and its slices are written out and added up by a second launch.  The
     // single-token projections' kernel walks the same slices one to a wave and adds them in the workgroup, same sums in
     // the same order (the rule and what it measured: wgemm_ordered_takes).
-    if (!wide && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit))
+    if (!wide && !keep_slices && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit))
         return launch_wgemm_ordered(x, ldx, w_tiles, bias, residual, ld_res, y, ldy, m, n, k, a.ksplit, flags, norm,
                                     (hipStream_t)stream);
     auto reduce = [&] {
+        if (keep_slices) return (int)MV_OK;
         if (norm && !sw && !of32 && wgemm_finalize_norm_takes(n))
             return launch_wgemm_finalize_norm(a.partial, a.ksplit, m, n, bias, norm, (hipStream_t)stream);
         return launch_wgemm_finalize(a.partial, a.ksplit, m, n, flags, a.bias, a.residual, ld_res, y, ldy,

@@ -91,7 +91,29 @@ struct PostnormArgs {
     float* x;
     void* h;
     int n;
+    int ks1, ks2;            // y1 and y2 as k-slices of their projections, added in order (1: whole)
+    int64_t slab1, slab2;    // floats from one slice to the next
 };
+
+// What a projection left in k-slices, at p + [0, ks) * slab: their sum in order.  Four slices are requested at a time: each
+// was written by another launch, so a dependent load is a trip to memory, and the usual cuts are 2 and 4.
+__device__ __forceinline__ float slices(const float* p, int ks, int64_t slab) {
+    float v = *p;
+    for (int i = 1; i < ks; ++i) v += p[i * slab];
+    return v;
+}
+__device__ __forceinline__ f32x4_t slices4(const float* p, int ks, int64_t slab) {
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(p);
+    for (int i = 1; i < ks; i += 3) {      // (uniform)
+        f32x4_t q[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) q[j] = *reinterpret_cast<const f32x4_t*>(p + min(i + j, ks - 1) * slab);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (i + j < ks) v += q[j];
+    }
+    return v;
+}
 
 template <bool F32>
 __global__ __launch_bounds__(256) void postnorm_residual_kernel(PostnormArgs a) {
@@ -102,7 +124,8 @@ __global__ __launch_bounds__(256) void postnorm_residual_kernel(PostnormArgs a) 
     const float* y1 = a.y1 + (int64_t)row * a.ld1;
     const float* y2 = a.y2 ? a.y2 + (int64_t)row * a.ld2 : nullptr;
     auto value = [&](int c) {
-        float v = y2 ? a.s1 * y1[c] + a.s2 * y2[c] : a.s1 * y1[c];
+        float v = a.s1 * slices(y1 + c, a.ks1, a.slab1);
+        if (y2) v += a.s2 * slices(y2 + c, a.ks2, a.slab2);
         return a.bias ? v + a.bias[c] : v;
     };
     float ss = 0.f;
@@ -127,13 +150,19 @@ __global__ __launch_bounds__(256) void postnorm_residual_kernel(PostnormArgs a) 
         Act<F32>::st(h + (int64_t)row * a.ldh + c, (xr[c] * inv2) * (1.0f + a.w2[c]));
 }
 
-// the same with the row in registers: n a multiple of 4 up to 4 * threads * NV, every row 16-byte aligned
-template <bool F32, int NV>
+// The same with the row in registers: n a multiple of 4 up to 4 * threads * NV, every row 16-byte aligned.  Reads memory once
+// and is nothing else; of projections that cut k it takes the slices (SLICES), which saves their reduction's launch and its
+// pass over memory: 2048 rows of 4096 in two slices 24.0 us of reduction and 21.6 here -> 27.3, 8 rows of 2048 in four 3.7 and
+// 4.2 -> 4.8.
+template <bool F32, int NV, bool SLICES>
 __global__ __launch_bounds__(1024) void postnorm_residual_reg_kernel(PostnormArgs a) {
     __shared__ float red[16];
     const int row = blockIdx.x, tid = threadIdx.x, n4 = a.n / 4;
-    const float4* y1 = reinterpret_cast<const float4*>(a.y1 + (int64_t)row * a.ld1);
-    const float4* y2 = a.y2 ? reinterpret_cast<const float4*>(a.y2 + (int64_t)row * a.ld2) : nullptr;
+    const float* y1 = a.y1 + (int64_t)row * a.ld1;
+    const float* y2 = a.y2 ? a.y2 + (int64_t)row * a.ld2 : nullptr;
+    auto at = [](const float* y, int c, int ks, int64_t slab) {
+        return SLICES ? slices4(y + 4 * c, ks, slab) : *reinterpret_cast<const f32x4_t*>(y + 4 * c);
+    };
     const float4* bias = reinterpret_cast<const float4*>(a.bias);
     const float4* w = reinterpret_cast<const float4*>(a.w);
     const float4* w2 = reinterpret_cast<const float4*>(a.w2);
@@ -145,11 +174,11 @@ __global__ __launch_bounds__(1024) void postnorm_residual_reg_kernel(PostnormArg
         const int c = tid + (int)blockDim.x * i;
         v[i] = xv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (c < n4) {
-            const float4 p = y1[c];
-            v[i] = make_float4(a.s1 * p.x, a.s1 * p.y, a.s1 * p.z, a.s1 * p.w);
+            const f32x4_t p = at(y1, c, a.ks1, a.slab1);
+            v[i] = make_float4(a.s1 * p[0], a.s1 * p[1], a.s1 * p[2], a.s1 * p[3]);
             if (y2) {
-                const float4 q = y2[c];
-                v[i].x += a.s2 * q.x; v[i].y += a.s2 * q.y; v[i].z += a.s2 * q.z; v[i].w += a.s2 * q.w;
+                const f32x4_t q = at(y2, c, a.ks2, a.slab2);
+                v[i].x += a.s2 * q[0]; v[i].y += a.s2 * q[1]; v[i].z += a.s2 * q[2]; v[i].w += a.s2 * q[3];
             }
             if (bias) {
                 const float4 q = bias[c];
@@ -427,30 +456,90 @@ __global__ __launch_bounds__(256) void embed_pair_kernel(const void* table_, con
         Act<F32>::st((T*)h_ + (int64_t)row * ldh + c, (x[(int64_t)row * ldx + c] * inv) * norm_w[c]);
 }
 
+struct AddNormArgs {
+    const float *y1, *y2, *w;
+    int64_t ld1, ld2, ldx, ldh;
+    int ks1;           // y1 as k-slices of its projection, added in order (1: whole)
+    int64_t slab1;     // floats from one slice to the next
+    float* x;
+    float eps;
+    void* h;
+    int n;
+};
+
 template <bool F32>
-__global__ __launch_bounds__(256) void add_rmsnorm_kernel(const float* y1, int64_t ld1, const float* y2, int64_t ld2,
-                                                          float* x, int64_t ldx, const float* w, float eps, void* h_,
-                                                          int64_t ldh, int n) {
+__global__ __launch_bounds__(256) void add_rmsnorm_kernel(AddNormArgs a) {
     typedef typename Act<F32>::T T;
     __shared__ float red[4];
-    T* h = (T*)h_;
+    T* h = (T*)a.h;
     const int row = blockIdx.x;
-    float* xr = x + (int64_t)row * ldx;
+    float* xr = a.x + (int64_t)row * a.ldx;
     float ss = 0.f;
 #pragma unroll 4
-    for (int c = threadIdx.x; c < n; c += 256) {
+    for (int c = threadIdx.x; c < a.n; c += 256) {
         float v = xr[c];
-        if (y1) {
-            v += y2 ? y1[(int64_t)row * ld1 + c] + y2[(int64_t)row * ld2 + c] : y1[(int64_t)row * ld1 + c];
+        if (a.y1) {
+            const float y = slices(a.y1 + (int64_t)row * a.ld1 + c, a.ks1, a.slab1);
+            v += a.y2 ? y + a.y2[(int64_t)row * a.ld2 + c] : y;
             xr[c] = v;
         }
         ss += v * v;
     }
+    if (!a.w) return;
+    ss = block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float)a.n + a.eps);
+#pragma unroll 4
+    for (int c = threadIdx.x; c < a.n; c += 256) Act<F32>::st(h + (int64_t)row * a.ldh + c, (xr[c] * inv) * a.w[c]);
+}
+
+// The same with the row in registers and in 16-byte pieces: n a multiple of 4 up to 4 * threads * NV, every row aligned, y1
+// given.  A latency chain: everything it needs is requested at once (a row of 1024 through the plain form, which reads it
+// again behind the sum, 3.5 us; here 2.8, two slices of y1 among what is read).
+template <bool F32, int NV>
+__global__ __launch_bounds__(1024) void add_rmsnorm_reg_kernel(AddNormArgs a) {
+    __shared__ float red[16];
+    const int row = blockIdx.x, tid = threadIdx.x, n4 = a.n / 4;
+    const float* y1 = a.y1 + (int64_t)row * a.ld1;
+    const float* y2 = a.y2 ? a.y2 + (int64_t)row * a.ld2 : nullptr;
+    f32x4_t* xr = reinterpret_cast<f32x4_t*>(a.x + (int64_t)row * a.ldx);
+    const f32x4_t* w = reinterpret_cast<const f32x4_t*>(a.w);
+    f32x4_t v[NV], wv[NV];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = tid + (int)blockDim.x * i;
+        v[i] = wv[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        if (c < n4) {
+            v[i] = xr[c];
+            if (w) wv[i] = w[c];
+            f32x4_t y = slices4(y1 + 4 * c, a.ks1, a.slab1);
+            if (y2) y += *reinterpret_cast<const f32x4_t*>(y2 + 4 * c);
+            v[i] += y;
+        }
+        ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i)      // behind the last load: the compiler orders a load after a store that might be to its place
+        if (tid + (int)blockDim.x * i < n4) xr[tid + (int)blockDim.x * i] = v[i];
     if (!w) return;
     ss = block_sum(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float)n + eps);
-#pragma unroll 4
-    for (int c = threadIdx.x; c < n; c += 256) Act<F32>::st(h + (int64_t)row * ldh + c, (xr[c] * inv) * w[c]);
+    const float inv = 1.0f / sqrtf(ss / (float)a.n + a.eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = tid + (int)blockDim.x * i;
+        if (c >= n4) continue;
+        f32x4_t o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = (v[i][j] * inv) * wv[i][j];
+        if (F32) {
+            reinterpret_cast<f32x4_t*>((float*)a.h + (int64_t)row * a.ldh)[c] = o;
+        } else {
+            uint2 pk;
+            pk.x = pack_bf16x2(o[0], o[1]);
+            pk.y = pack_bf16x2(o[2], o[3]);
+            reinterpret_cast<uint2*>((uint16_t*)a.h + (int64_t)row * a.ldh)[c] = pk;
+        }
+    }
 }
 
 template <bool F32>
@@ -757,25 +846,40 @@ int mv_embed_scaled(const void* table, const int32_t* ids, float* x, int64_t ldx
 int mv_postnorm_residual(const float* y1, int64_t ld1, const float* y2, int64_t ld2, float s1, float s2,
                          const float* bias, const float* w, float eps, float mult, const float* next_w, float* x,
                          int64_t ldx, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream) {
+    return mv_postnorm_residual_slabs(y1, ld1, 1, y2, ld2, 1, s1, s2, bias, w, eps, mult, next_w, x, ldx, h, ldh, rows, n, f32,
+                                      stream);
+}
+
+int mv_postnorm_residual_slabs(const float* y1, int64_t ld1, int ks1, const float* y2, int64_t ld2, int ks2, float s1,
+                               float s2, const float* bias, const float* w, float eps, float mult, const float* next_w,
+                               float* x, int64_t ldx, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream) {
     using namespace mv;
     if (rows < 0 || n <= 0) return MV_ERR_INVALID_ARG;
     if (rows == 0) return MV_OK;
     if (!y1 || !w || !x || !h || ld1 < n || (y2 && ld2 < n) || ldx < n || ldh < n) return MV_ERR_INVALID_ARG;
+    if (ks1 < 1 || (y2 && ks2 < 1)) return MV_ERR_INVALID_ARG;
     hipStream_t s = (hipStream_t)stream;
     PostnormArgs a;
     a.y1 = y1; a.y2 = y2; a.bias = bias; a.w = w; a.w2 = next_w;
     a.ld1 = ld1; a.ld2 = ld2; a.ldx = ldx; a.ldh = ldh;
     a.s1 = s1; a.s2 = s2; a.eps = eps; a.mult = mult;
     a.x = x; a.h = h; a.n = n;
+    a.ks1 = ks1; a.ks2 = y2 ? ks2 : 1;
+    a.slab1 = rows * ld1; a.slab2 = rows * ld2;
     const bool even = n % 4 == 0 && ld1 % 4 == 0 && ldx % 4 == 0 && ldh % 4 == 0 && (!y2 || ld2 % 4 == 0) && aligned16(y1) &&
                       aligned16(x) && aligned16(h) && aligned16(w) && (!y2 || aligned16(y2)) &&
                       (!bias || aligned16(bias)) && (!next_w || aligned16(next_w));
+    const bool cut = a.ks1 > 1 || a.ks2 > 1;
     // a row of a short step has its workgroup to itself on a compute unit: more threads, fewer values each
     const int nt = rows > 512 || n <= 1024 ? 256 : n <= 2048 ? 512 : 1024;
+#define MV_POSTNORM_T(F32_, NV_, CUT_) \
+    hipLaunchKernelGGL((postnorm_residual_reg_kernel<F32_, NV_, CUT_>), dim3(rows), dim3(nt), 0, s, a)
 #define MV_POSTNORM(NV_)                                                                                              \
     do {                                                                                                              \
-        if (f32) hipLaunchKernelGGL((postnorm_residual_reg_kernel<true, NV_>), dim3(rows), dim3(nt), 0, s, a);         \
-        else hipLaunchKernelGGL((postnorm_residual_reg_kernel<false, NV_>), dim3(rows), dim3(nt), 0, s, a);            \
+        if (f32 && cut) MV_POSTNORM_T(true, NV_, true);                                                               \
+        else if (f32) MV_POSTNORM_T(true, NV_, false);                                                                \
+        else if (cut) MV_POSTNORM_T(false, NV_, true);                                                                \
+        else MV_POSTNORM_T(false, NV_, false);                                                                        \
     } while (0)
     if (even && n <= 4 * nt) MV_POSTNORM(1);
     else if (even && n <= 8 * nt) MV_POSTNORM(2);
@@ -784,6 +888,7 @@ int mv_postnorm_residual(const float* y1, int64_t ld1, const float* y2, int64_t 
     else if (f32) hipLaunchKernelGGL(postnorm_residual_kernel<true>, dim3(rows), dim3(256), 0, s, a);
     else hipLaunchKernelGGL(postnorm_residual_kernel<false>, dim3(rows), dim3(256), 0, s, a);
 #undef MV_POSTNORM
+#undef MV_POSTNORM_T
     return check_launch();
 }
 
@@ -820,14 +925,37 @@ int mv_embed_pair(const void* table, const void* pairs, const int32_t* ids, cons
 
 int mv_add_rmsnorm(const float* y1, int64_t ld1, const float* y2, int64_t ld2, float* x, int64_t ldx, const float* w,
                    float eps, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream) {
+    return mv_add_rmsnorm_slabs(y1, ld1, 1, y2, ld2, x, ldx, w, eps, h, ldh, rows, n, f32, stream);
+}
+
+int mv_add_rmsnorm_slabs(const float* y1, int64_t ld1, int ks1, const float* y2, int64_t ld2, float* x, int64_t ldx,
+                         const float* w, float eps, void* h, int64_t ldh, int rows, int n, int f32, mv_stream_t stream) {
     using namespace mv;
     if (rows < 0 || n <= 0) return MV_ERR_INVALID_ARG;
     if (rows == 0) return MV_OK;
-    if (!x || ldx < n || (y1 && ld1 < n) || (y2 && (!y1 || ld2 < n)) || (w && (!h || ldh < n)) || (!w && !y1))
+    if (!x || ldx < n || (y1 && (ld1 < n || ks1 < 1)) || (y2 && (!y1 || ld2 < n)) || (w && (!h || ldh < n)) || (!w && !y1))
         return MV_ERR_INVALID_ARG;
     hipStream_t s = (hipStream_t)stream;
-    if (f32) hipLaunchKernelGGL(add_rmsnorm_kernel<true>, dim3(rows), dim3(256), 0, s, y1, ld1, y2, ld2, x, ldx, w, eps, h, ldh, n);
-    else hipLaunchKernelGGL(add_rmsnorm_kernel<false>, dim3(rows), dim3(256), 0, s, y1, ld1, y2, ld2, x, ldx, w, eps, h, ldh, n);
+    AddNormArgs a;
+    a.y1 = y1; a.y2 = y2; a.w = w;
+    a.ld1 = ld1; a.ld2 = ld2; a.ldx = ldx; a.ldh = ldh;
+    a.ks1 = ks1; a.slab1 = rows * ld1;
+    a.x = x; a.eps = eps; a.h = h; a.n = n;
+    const bool even = y1 && n % 4 == 0 && ld1 % 4 == 0 && ldx % 4 == 0 && (!y2 || ld2 % 4 == 0) && (!w || ldh % 4 == 0) &&
+                      aligned16(y1) && aligned16(x) && (!y2 || aligned16(y2)) && (!w || (aligned16(w) && aligned16(h)));
+    // threads to a row as in mv_postnorm_residual
+    const int nt = rows > 512 || n <= 1024 ? 256 : n <= 2048 ? 512 : 1024;
+#define MV_ADDNORM(NV_)                                                                                              \
+    do {                                                                                                             \
+        if (f32) hipLaunchKernelGGL((add_rmsnorm_reg_kernel<true, NV_>), dim3(rows), dim3(nt), 0, s, a);              \
+        else hipLaunchKernelGGL((add_rmsnorm_reg_kernel<false, NV_>), dim3(rows), dim3(nt), 0, s, a);                 \
+    } while (0)
+    if (even && n <= 4 * nt) MV_ADDNORM(1);
+    else if (even && n <= 8 * nt) MV_ADDNORM(2);
+    else if (even && n <= 16 * nt) MV_ADDNORM(4);
+    else if (f32) hipLaunchKernelGGL(add_rmsnorm_kernel<true>, dim3(rows), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(add_rmsnorm_kernel<false>, dim3(rows), dim3(256), 0, s, a);
+#undef MV_ADDNORM
     return check_launch();
 }
 

@@ -1107,13 +1107,25 @@ int launch_wgemm_finalize_norm(float* partial, int ksplit, int m, int n, const v
     return launch_finalize_norm(a, s);
 }
 
+// k-slices of a projection whose next kernel adds them.  Past four rows as everywhere; up to four (the dot form) two, where the
+// strips are few and long: half the compute units or fewer have one, and they would walk it longer than the chip takes for
+// the whole.  One row, us whole -> two slices: 1024 x 5120 6.2 -> 5.0, 1024 x 4096 5.0 -> 4.1, 512 x 4096 4.8 -> 3.8, 2048 x 8192
+// 9.0 -> 7.6; but 2048 x 4096 5.8 -> 6.3, 2048 x 2048 4.1 -> 4.3, 1024 x 1024 3.5 -> 3.5.  Four slices: 1024 x 5120 5.3, 2048 x
+// 8192 7.0 and of two rows 8.1 where two take 7.7.
+int wgemm_slices(int m, int n, int k) {
+    const int nt = n / 16, kt = k / 32;
+    if (m > 4 || g_tune_ksplit) return pick_ksplit(m, nt, kt, true);
+    return nt <= num_cus() / 2 && kt >= 128 && kt >= 2 * nt ? 2 : 1;
+}
+
 static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_add_r,
                       const void* ln_w, float eps, void* sum_out, int64_t ld_sum_out, int prologue,
                       int var_from_rounded, const void* w_tiles, const void* bias,
                       const void* residual, int64_t ld_res, void* y, int64_t ldy, int m, int n,
                       int k, void* workspace, size_t workspace_bytes, int flags,
                       mv_stream_t stream, const void* post_ln_w = nullptr, float post_eps = 0.f,
-                      void* post_out = nullptr, int64_t ld_post = 0, int post_var_from_rounded = 0) {
+                      void* post_out = nullptr, int64_t ld_post = 0, int post_var_from_rounded = 0,
+                      int slices = 0) {
     const bool slabs_only = (flags & MV_GEMM_SLABS) != 0;
     if (!x || !w_tiles || (!y && !slabs_only) || m <= 0 || n <= 0 || k <= 0) return MV_ERR_INVALID_ARG;
     if (m > 64 || (n % 16) != 0 || (k % 32) != 0) return MV_ERR_UNSUPPORTED;
@@ -1161,7 +1173,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
     a.sum_out = (uint16_t*)sum_out;
     a.ld_sum_out = ld_sum_out;
     const bool free_reduce = slabs_only || post_ln_w != nullptr || (flags & MV_GEMM_PLAN_SLABS) != 0;
-    a.ksplit = pick_ksplit(m, a.nt, a.kt, free_reduce);
+    a.ksplit = slices ? slices : pick_ksplit(m, a.nt, a.kt, free_reduce);
     a.partial = nullptr;
     a.post_ln_w = (const uint16_t*)post_ln_w;
     a.post_out = (uint16_t*)post_out;
@@ -1245,6 +1257,12 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
         rc = check_launch();
     }
     return rc;
+}
+
+int launch_wgemm_slices(const void* x, int64_t ldx, const void* w_tiles, float* slabs, size_t slabs_bytes, int m, int n, int k,
+                        mv_stream_t stream) {
+    return wgemm_impl(x, ldx, nullptr, 0, nullptr, 0.f, nullptr, 0, kProNone, 0, w_tiles, nullptr, nullptr, 0, nullptr, 0, m, n,
+                      k, slabs, slabs_bytes, MV_GEMM_SLABS, stream, nullptr, 0.f, nullptr, 0, 0, wgemm_slices(m, n, k));
 }
 
 }  // namespace mv

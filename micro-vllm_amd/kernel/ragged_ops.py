@@ -75,6 +75,33 @@ class AnyLinear:
         return out
 
 
+    def slabs(self, x: torch.Tensor, take) -> torch.Tensor:
+        """The product as the k-slices its plan cuts, [slices, m, n] fp32 whose sum over the first dimension, in order, is
+        y - for `postnorm_residual` and `add_rmsnorm`, which add them.  `take(rows, cols)` gives the fp32 buffer."""
+        m = x.shape[0]
+        if self.tiles is None or m == 0:
+            return self(x, take(m, self.n)).unsqueeze(0)
+        assert x.is_cuda and x.dim() == 2 and x.shape[1] == self.k and x.stride(1) == 1 and x.dtype == torch.bfloat16
+        L = nv.lib()
+        ks = L.mv_linear_slab_count(m, self.n, self.k)
+        out = take(ks * m, self.n)
+        assert out.dtype == torch.float32 and out.is_contiguous() and out.shape == (ks * m, self.n)
+        # (the buffer of the many-row projections: counters that stay zero between launches)
+        ws = nv.stream_workspace("gemm_prefill", x.device, L.mv_linear_slabs_workspace_bytes(m, self.n, self.k))
+        nv.check("mv_linear_slabs", L.mv_linear_slabs(
+            x.data_ptr(), x.stride(0) if m > 1 else max(self.k, x.stride(0)), self.tiles.tiles.data_ptr(), out.data_ptr(),
+            out.numel() * 4, m, self.n, self.k, nv.ptr(ws), ws.numel() * 4 if ws is not None else 0, nv.stream_ptr()))
+        return out.view(ks, m, self.n)
+
+
+def _slices(y):
+    """(first slice [rows, n], slices): a projection's output, whole or as AnyLinear.slabs left it."""
+    if y.dim() == 2:
+        return y, 1
+    assert y.dim() == 3 and y.is_contiguous() and y.shape[0] >= 1
+    return y[0], y.shape[0]
+
+
 def embed_scaled(table, ids, scale: float, x, h, w=None, eps: float = 0.0, offset: float = 1.0):
     """x = table[ids] * scale; h = act(x), or with `w` act(x / sqrt(mean(x^2) + eps) * (offset + w))."""
     rows, n = x.shape
@@ -90,15 +117,17 @@ def embed_scaled(table, ids, scale: float, x, h, w=None, eps: float = 0.0, offse
 def postnorm_residual(y1, w, eps: float, x, h, y2=None, s1: float = 1.0, s2: float = 0.0, bias=None, mult: float = 1.0,
                       next_w=None):
     """x += mult * unit_rms(s1*y1 + s2*y2 + bias) * (1 + w); h = x in the activation type, or with `next_w` the next
-    sublayer's norm of it, unit_rms(x) * (1 + next_w)."""
+    sublayer's norm of it, unit_rms(x) * (1 + next_w).  y1 and y2 may be k-slices (AnyLinear.slabs)."""
     rows, n = x.shape
+    y1, ks1 = _slices(y1)
+    y2, ks2 = (None, 1) if y2 is None else _slices(y2)
     assert bias is None or (bias.numel() == n and bias.is_contiguous())
     assert next_w is None or (next_w.numel() == n and next_w.is_contiguous())
     assert y1.shape == (rows, n) and h.shape == (rows, n) and w.numel() == n and w.is_contiguous()
     assert y2 is None or y2.shape == (rows, n)
-    nv.check("mv_postnorm_residual", nv.lib().mv_postnorm_residual(
-        _f32(y1).data_ptr(), _ld(y1), None if y2 is None else _f32(y2).data_ptr(), 0 if y2 is None else _ld(y2),
-        float(s1), float(s2), None if bias is None else _f32(bias).data_ptr(), _f32(w).data_ptr(), float(eps), float(mult),
+    nv.check("mv_postnorm_residual", nv.lib().mv_postnorm_residual_slabs(
+        _f32(y1).data_ptr(), _ld(y1) if ks1 == 1 else n, ks1, None if y2 is None else _f32(y2).data_ptr(),
+        0 if y2 is None else _ld(y2) if ks2 == 1 else n, ks2, float(s1), float(s2), None if bias is None else _f32(bias).data_ptr(), _f32(w).data_ptr(), float(eps), float(mult),
         None if next_w is None else _f32(next_w).data_ptr(), _f32(x).data_ptr(), _ld(x), h.data_ptr(), _ld(h),
         rows, n, _is_f32(h), nv.stream_ptr()))
 
@@ -587,13 +616,14 @@ def embed_pair(table, pairs, ids, prev, x, scale: float, buckets: int, mul_prev:
 
 
 def add_rmsnorm(x, y1=None, y2=None, w=None, eps: float = 0.0, h=None):
-    """x += y1 (+ y2); with `w`: h = act(x / sqrt(mean(x^2) + eps) * w)."""
+    """x += y1 (+ y2); with `w`: h = act(x / sqrt(mean(x^2) + eps) * w).  y1 may be k-slices (AnyLinear.slabs)."""
     rows, n = x.shape
+    y1, ks1 = (None, 1) if y1 is None else _slices(y1)
     assert y1 is None or y1.shape == (rows, n)
     assert y2 is None or (y1 is not None and y2.shape == (rows, n))
     assert (w is None) == (h is None) and (w is None or (w.numel() == n and w.is_contiguous() and h.shape == (rows, n)))
-    nv.check("mv_add_rmsnorm", nv.lib().mv_add_rmsnorm(
-        None if y1 is None else _f32(y1).data_ptr(), 0 if y1 is None else _ld(y1),
+    nv.check("mv_add_rmsnorm", nv.lib().mv_add_rmsnorm_slabs(
+        None if y1 is None else _f32(y1).data_ptr(), 0 if y1 is None else _ld(y1) if ks1 == 1 else n, ks1,
         None if y2 is None else _f32(y2).data_ptr(), 0 if y2 is None else _ld(y2), _f32(x).data_ptr(), _ld(x),
         None if w is None else _f32(w).data_ptr(), float(eps), None if h is None else h.data_ptr(),
         0 if h is None else _ld(h), rows, n, 0 if h is None else _is_f32(h), nv.stream_ptr()))

@@ -1,0 +1,68 @@
+"""Projections left in k-slices (mv_linear_slabs) and the residual norms that add them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _take(rows, cols):
+    return torch.full((rows, cols), float("nan"), dtype=torch.float32, device=DEV)
+
+
+# up to four rows strips that leave compute units idle are cut (1, 2, 4 and 8 ways and a k too short for it), 5 to 64 as the
+# batched projections, more as the prompts' (cut, and whole in tiles whose left-overs are cut inside the launch)
+@pytest.mark.parametrize("m,n,k", [(1, 1024, 5120), (1, 1024, 1024), (2, 512, 8192), (3, 2048, 8192), (4, 16, 8192), (4, 4096, 512),
+                                   (5, 2048, 8192), (16, 1040, 2048), (33, 2048, 8192), (64, 1024, 4096), (65, 1024, 4096),
+                                   (300, 2048, 8192), (700, 2048, 8192), (3072, 6144, 4096)])
+def test_slices_add_up_to_the_product(mv, m, n, k):
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV)
+    lin = AnyLinear(w)
+    got = lin.slabs(x, _take)
+    assert got.shape == (nv.lib().mv_linear_slab_count(m, n, k), m, n)
+    want = x.double() @ w.double().t()
+    # fp32 sums of k products of order 1 / sqrt(k): their error stays below sqrt(k) * 2^-24 of the largest partial sum
+    tol = k ** 0.5 * 2 ** -24 * 8
+    assert (got.double().sum(0) - want).abs().max().item() <= tol
+    again = lin.slabs(x, _take)
+    assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize("rows,n", [(1, 64), (1, 1024), (3, 2048), (5, 4096), (2, 8192), (513, 1024), (600, 4096), (7, 100), (3, 33)])
+@pytest.mark.parametrize("ks", [1, 2, 3, 4, 5, 8, 16])
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float32])
+def test_norms_add_the_slices_in_order(mv, rows, n, ks, act):
+    """The residual steps over slices give what they give over the slices' sum taken in order, bit for bit (every width of
+    the register forms and, with n not a multiple of four, the plain one)."""
+    from micro_vllm_amd.kernel import ragged_ops as ops
+
+    g = torch.Generator().manual_seed(rows * n + ks)
+    mk = lambda *s: torch.randn(*s, generator=g).to(DEV)   # noqa: E731
+    y1, y2, x, w, nxt, bias = mk(ks, rows, n), mk(2, rows, n), mk(rows, n), mk(n), mk(n), mk(n)
+    total = y1[0].clone()
+    for i in range(1, ks):
+        total += y1[i]
+    total2 = y2[0] + y2[1]
+    for second in (False, True):
+        res = []
+        for a, b in ((y1, y2), (total, total2)):
+            xs, h = x.clone(), torch.empty(rows, n, dtype=act, device=DEV)
+            ops.postnorm_residual(a, w, 1e-5, xs, h, y2=b if second else None, s1=0.5, s2=2.0, bias=bias, mult=0.7, next_w=nxt)
+            res += [xs, h]
+        assert torch.equal(res[0], res[2]) and torch.equal(res[1], res[3])
+        res = []
+        for a in (y1, total):
+            xs, h = x.clone(), torch.empty(rows, n, dtype=act, device=DEV)
+            ops.add_rmsnorm(xs, a, total2 if second else None, w=w, eps=1e-5, h=h)
+            res += [xs, h]
+        assert torch.equal(res[0], res[2]) and torch.equal(res[1], res[3])
+        want = x.double() + total.double() + (total2.double() if second else 0.0)
+        normed = want / torch.sqrt((want * want).mean(-1, keepdim=True) + 1e-5) * w.double()
+        # the square sum's error grows with the chain of additions, far below one bf16 unit; fp32 results lie within 2^-20
+        tol = 2 ** -8 if act == torch.bfloat16 else 2 ** -18
+        assert ((res[1].double() - normed).abs() <= tol * normed.abs() + 1e-6).all()
