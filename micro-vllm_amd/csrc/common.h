@@ -133,8 +133,9 @@ struct PostNorm {
 // wgemm.hip: the same followed by the norm
 int launch_wgemm_finalize_norm(float* partial, int ksplit, int m, int n, const void* bias, PostNorm* norm, hipStream_t s);
 bool wgemm_finalize_norm_takes(int n);
-// wgemm.hip: a projection of up to 64 rows whose sums are those of `ks` slices of k added in order
-bool wgemm_ordered_takes(int m, int nt, int kt, int ks);
+// wgemm.hip: a projection of up to 64 rows whose sums are those of `ks` slices of k added in order.  `strips`: n-tiles of a
+// wave of the 64-row tiles that would take it otherwise (0: larger ones would)
+bool wgemm_ordered_takes(int m, int nt, int kt, int ks, int strips);
 int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
                          int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int ks, int flags, PostNorm* norm,
                          hipStream_t s);

@@ -276,8 +276,9 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
 // MT m-tiles per wave (128 or 64 rows a workgroup), RING k-tiles of weights in registers and BUFS stages of x in LDS.
 // 8, 3, 3: two workgroups to a compute unit hide each other's trips to memory.  RING 8, BUFS 4: for grids of at most one
 // workgroup to a unit, whose waves have the registers to themselves; with two k-tiles ahead a stage of 64 k takes 1.1 us
-// there.  The 64-row tile halves what a wave multiplies per stage and doubles the workgroups.  Sums do not depend on it.
-template <int MT, int RING, int BUFS>
+// there.  The 64-row tile halves what a wave multiplies per stage and doubles the workgroups, and NT, the n-tiles of a wave,
+// doubles or quadruples them again (tile64_strips).  Sums do not depend on any of it.
+template <int MT, int RING, int BUFS, int NT = kPNT>
 __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefill_kernel(PGemmArgs a) {
     constexpr int kStage = MT * 16 * kPK * 2, XP = MT / 2;   // bytes of a stage of x, pieces of it a wave requests
     constexpr int kPeriod = RING == 3 ? 3 : RING / 2;     // stages after which slots and buffers repeat
@@ -298,12 +299,12 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     const int mb = idx % a.mblocks;
     if (nb >= a.nblocks || idx / a.mblocks >= a.nb_per_xcd) return;
     const int m0 = mb * (16 * MT);
-    const int nt0 = nb * (kPN / 16) + wid * kPNT;
+    const int nt0 = (nb * 4 + wid) * NT;
 
     // weight fragment streams of this wave (strips past the end are clamped and never stored)
-    const uint4* wp[kPNT];
+    const uint4* wp[NT];
 #pragma unroll
-    for (int i = 0; i < kPNT; ++i)
+    for (int i = 0; i < NT; ++i)
         wp[i] = a.w + ((int64_t)min(nt0 + i, a.nt - 1) * a.kt + kt0) * 64 + lane;
 
     // ---- x: global -> LDS directly, BUFS stages deep, in fragment order ---------------------
@@ -340,19 +341,19 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
             bf16x8_t, *reinterpret_cast<const uint4*>(&xs[buf][(t * 2 + kk) * 1024 + lane * 16]));
     };
 
-    f32x4_t acc[kPNT][MT];
+    f32x4_t acc[NT][MT];
 #pragma unroll
-    for (int i = 0; i < kPNT; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[i][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
     // weight fragments: a ring of k-tiles; a slot is refilled (RING - 1 k-tiles ahead) at the start of the k-tile after the
     // one that used it
-    uint4 w[RING][kPNT];
-    auto w_load = [&](uint4(&wr)[kPNT], int kt) {
+    uint4 w[RING][NT];
+    auto w_load = [&](uint4(&wr)[NT], int kt) {
         const int ktc = min(kt, a.ktps - 1);
 #pragma unroll
-        for (int i = 0; i < kPNT; ++i) {
+        for (int i = 0; i < NT; ++i) {
 #ifdef MV_EXP_NO_WLOAD
             if (kt > 2) continue;  // timing experiment only: weights never refreshed
 #endif
@@ -364,7 +365,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
 #pragma unroll
     for (int i = 0; i < RING - 1; ++i) w_load(w[i], i);
     // the first two stages of x (the weights behind them may still be on their way)
-    wait_vmcnt<RING == 3 ? 0 : XP * (BUFS - 3) + kPNT * (RING - 1)>();
+    wait_vmcnt<RING == 3 ? 0 : XP * (BUFS - 3) + NT * (RING - 1)>();
     asm volatile("" ::: "memory");
     __syncthreads();
 
@@ -379,11 +380,11 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     // here, first thing, with the k-tile RING - 1 ahead (left to itself the scheduler sinks these
     // requests to the end of the stage, and the next stage then starts by waiting for them).
     // `fetch_stage` >= 0: also request that stage of x, after the first half of the MFMAs.
-    auto ktile = [&](uint4(&wc)[kPNT], uint4(&wr)[kPNT], bf16x8_t(&xc)[MT], bf16x8_t(&xn)[MT], int buf,
+    auto ktile = [&](uint4(&wc)[NT], uint4(&wr)[NT], bf16x8_t(&xc)[MT], bf16x8_t(&xn)[MT], int buf,
                      int kk, int nbuf, int nkk, int kt_refill, int fetch_stage, int fetch_buf) {
-        bf16x8_t wf[kPNT];
+        bf16x8_t wf[NT];
 #pragma unroll
-        for (int i = 0; i < kPNT; ++i) wf[i] = __builtin_bit_cast(bf16x8_t, wc[i]);
+        for (int i = 0; i < NT; ++i) wf[i] = __builtin_bit_cast(bf16x8_t, wc[i]);
         __builtin_amdgcn_sched_barrier(0);
         w_load(wr, kt_refill);
         __builtin_amdgcn_sched_barrier(0);
@@ -394,7 +395,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
 #pragma unroll
         for (int t = 0; t < MT / 2; ++t)
 #pragma unroll
-            for (int i = 0; i < kPNT; ++i)
+            for (int i = 0; i < NT; ++i)
                 MV_MFMA(acc[i][t], wf[i], xc[t]);
         // The x requests are invisible to the compiler's request counting, so they go out behind
         // the waits for this k-tile's weights: in front of them they would make those waits cover
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
 #pragma unroll
         for (int t = MT / 2; t < MT; ++t)
 #pragma unroll
-            for (int i = 0; i < kPNT; ++i)
+            for (int i = 0; i < NT; ++i)
                 MV_MFMA(acc[i][t], wf[i], xc[t]);
     };
     // One stage, I = s mod kPeriod: request stage s + BUFS - 1 of x (its buffer was last read in stage s - 1), two k-tiles,
@@ -427,7 +428,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
         // stages left over the compiler drops the refills, so only the pieces of x may be counted there: a count that
         // includes requests that were never made waits for nothing, and the next stage reads what has not arrived.  (Three
         // buffers: at most two stages are left over, and both have arrived before the first of them.)
-        wait_vmcnt<(kLeft && BUFS > 3) ? (BUFS - 3) * XP : kPNT + (BUFS - 3) * (2 * kPNT + XP)>();
+        wait_vmcnt<(kLeft && BUFS > 3) ? (BUFS - 3) * XP : NT + (BUFS - 3) * (2 * NT + XP)>();
         MV_STAMP(2);
 #ifndef MV_EXP_NO_BARRIER
         __syncthreads();
@@ -450,7 +451,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     if (kPeriod == 4 && s + 2 < nstage) stage(std::integral_constant<int, 2>{}, left, s + 2);
     wait_vmcnt<0>();     // no request into LDS outlives the workgroup
 
-    store_wave_tile<kPNT, MT>(a, acc, nt0, m0, ks, r, q);
+    store_wave_tile<NT, MT>(a, acc, nt0, m0, ks, r, q);
 }
 
 
@@ -986,6 +987,18 @@ static int wide_tile_strips(int m, int n, int kt) {
     }
     return best;
 }
+// n-tiles of a wave of the 64-row tiles (1, 2 or 4): the fewest whose tiles still have a compute unit each, 0 where not even
+// the widest do.  Few columns or slices leave units idle at four; a narrower tile reads x again for every 64 or 128 columns,
+// which costs less than the idle units until they run out.  Slices of 8 (us, four -> two -> one strip a wave): 37 rows 2048 x 5632
+// (64 tiles of four) 17.4 -> 13.4 -> 12.5, 64 rows 4096 x 4096 (128) 18.0 -> 15.7 -> 17.0; whole k, 128 rows 8192 x 1024 (64) 22.5 -> 14.5
+// -> 11.6, 256 rows (128) 22.4 -> 14.8 -> 18.4; but 128 rows 2560 x 2048 (256) 16.5 -> 17.5 -> 17.7.
+static int tile64_strips(int m, int nt, int ks) {
+    for (int strips = 1; strips <= kPNT; strips *= 2) {
+        const long per_xcd = ((nt + 4 * strips - 1) / (4 * strips) + 7) / 8;
+        if (8L * per_xcd * ((m + 63) / 64) * ks <= num_cus()) return strips;
+    }
+    return 0;
+}
 static PrefillPlan prefill_plan(int m, int n, int kt) {
     static const int forced = [] {
         const char* e = getenv("MVLLM_PREFILL_WIDE");
@@ -1109,6 +1122,11 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
                            ? (void*)((char*)workspace + kWCountBytes) : nullptr;
     const size_t data_bytes = data ? workspace_bytes - kWCountBytes : 0;
     bool wide = plan.wide;
+    // Tiles of 256 rows for 64 or fewer: the 64-row tiles take the same slices where each has a compute unit to itself (28672 x 4096 in two
+    // slices, 8 rows 63.6 -> 48.5 us, 64 rows 67.0 -> 54.5; same sums, so not where the wide form would cut left-over tiles).
+    if (wide && m <= 64 && tile64_strips(m, a.nt, a.ksplit) &&
+        !(a.ksplit == 1 && wide_cuts(1, (a.nt + plan.strips - 1) / plan.strips, a.kt)))
+        wide = false;
     if (a.ksplit > 1) {
         const size_t need = (size_t)a.ksplit * m * n * sizeof(float);
         if (keep_slices) {
@@ -1123,7 +1141,7 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     // Up to 64 rows a tile of 128 is mostly padding, and its slices are written out and added up by a second launch.  The
     // single-token projections' kernel walks the same slices one to a wave and adds them in the workgroup, same sums in
     // the same order (the rule and what it measured: wgemm_ordered_takes).
-    if (!wide && !keep_slices && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit))
+    if (!wide && !keep_slices && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit, tile64_strips(m, a.nt, a.ksplit)))
         return launch_wgemm_ordered(x, ldx, w_tiles, bias, residual, ld_res, y, ldy, m, n, k, a.ksplit, flags, norm,
                                     (hipStream_t)stream);
     auto reduce = [&] {
@@ -1179,11 +1197,15 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     // 44.8 -> 28.3 and 256 x 16384 x 2048 47.2 -> 31.9 in 64-row tiles, 1408 x 2048 x 2048 39.0 -> 24.0, 1024 x 4096 x 4096 in
     // two slices 54.4 -> 49.7 in the deep form (64-row tiles in two rounds: 61.3), 700 x 2048 x 5632 in four (22 stages) 36.8 -> 35.6;
     // but 192 x 6144 x 2048 in four (8 stages) 24.8, deep 25.4, and 96 x 7168 x 8192 in eight (16) 34.1, deep 35.7.
-    const int mblocks64 = (m + 63) / 64;
-    const long grid64 = 8L * a.nb_per_xcd * mblocks64 * a.ksplit;
-    if (grid64 <= num_cus()) {
-        a.mblocks = mblocks64;
-        hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4>), dim3((unsigned)grid64), dim3(256), 0, (hipStream_t)stream, a);
+    const int strips = tile64_strips(m, a.nt, a.ksplit);
+    if (strips) {
+        a.mblocks = (m + 63) / 64;
+        a.nblocks = (a.nt + 4 * strips - 1) / (4 * strips);
+        a.nb_per_xcd = (a.nblocks + 7) / 8;
+        const dim3 grid64((unsigned)(8L * a.nb_per_xcd * a.mblocks * a.ksplit));
+        if (strips == 1) hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 1>), grid64, dim3(256), 0, (hipStream_t)stream, a);
+        else if (strips == 2) hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 2>), grid64, dim3(256), 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 4>), grid64, dim3(256), 0, (hipStream_t)stream, a);
     } else if (grid <= num_cus() && a.ktps >= 40) {
         hipLaunchKernelGGL((gemm_prefill_kernel<8, 8, 4>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
     } else {

@@ -1041,11 +1041,16 @@ static int launch_ordered_mb(const GemmArgs& a, int sg, int ks, int grid, hipStr
 // (768) 17.0 -> 19.8 and 8192 x 2048 (1024) 16.3 -> 22.7.  Long slices, 448: 17 rows 2048 x 5632 (374) 10.4 -> 12.0 where 128-row tiles took
 // 13.2, 24 rows (528) 10.7 -> 14.2.  Sixteen slices, whose reduction reads most, 592: 37 rows 4096 x 4096 16.5 -> 15.6, 48 rows (768)
 // 17.5 -> 17.6.
-bool wgemm_ordered_takes(int m, int nt, int kt, int ks) {
+// Against tiles narrow enough to fill the chip (`strips` of 1 or 2) the limits lie lower, for one block of rows too: 320, 448
+// for two strips and short slices.  16 rows 2048 x 5632 (352) 11.8 -> 10.6 in tiles, 1280 x 8192 (512) 14.0 -> 12.5, 64 rows 2048 x 2048
+// (512) 12.0 -> 10.4, but 37 rows (296) 8.6 against 9.1, 32 rows 3072 x 3072 (384) 10.8 against 11.9.
+bool wgemm_ordered_takes(int m, int nt, int kt, int ks, int strips) {
     const int blocks = (m + 15) / 16, walk = ks == 4 ? kt / 4 : kt / 8;
     if ((ks != 4 && ks != 8 && ks != 16) || blocks > 4) return false;
-    const int most = ks == 16 ? 592 : walk > 16 ? 448 : 512;
-    return blocks == 1 || (m * walk <= most && blocks * kt <= 384 && nt >= 128 && (int64_t)blocks * kt * nt <= 150000);
+    const bool narrow = strips == 1 || strips == 2;
+    const int most = strips == 1 || (narrow && walk > 16) ? 320 : narrow ? 448 : ks == 16 ? 592 : walk > 16 ? 448 : 512;
+    if (blocks == 1) return !narrow || m * walk <= most;
+    return m * walk <= most && blocks * kt <= 384 && nt >= 128 && (int64_t)blocks * kt * nt <= 150000;
 }
 
 // x [m, k] . W^T with the sums of `ks` slices of k added in order, epilogue as mv_gemm_prefill_ws, or the norm's.

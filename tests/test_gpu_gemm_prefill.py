@@ -477,3 +477,37 @@ def test_tiles_of_64_and_128_rows_give_the_same_sums(mv, m, n, k, mode):
             m * r, n, k, flags, nv.stream_ptr()))
         outs.append(y)
     assert torch.equal(outs[0], outs[1][:m]) and torch.equal(outs[0], outs[1][-m:])
+
+
+@pytest.mark.parametrize("mode", ["plain", "bias", "residual", "f32", "swiglu"])
+@pytest.mark.parametrize("m,n,k", [(128, 8192, 1024), (128, 8208, 1024), (256, 4096, 1024), (256, 8192, 1024), (192, 8240, 1024),
+                                   (65, 2064, 512), (300, 8208, 512),
+                                   (37, 28672, 4096), (64, 28672, 4096)])
+def test_narrow_tiles_give_the_sums_of_wide_ones(mv, m, n, k, mode):
+    """64-row tiles of one and two n-tiles a wave (grids of up to a quarter and half of the compute units; n that leaves a part
+    of a workgroup's columns unused) and, of up to 64 rows, in place of the 256-row form in two slices: the same rows as
+    the first of many, whose plan cuts k the same way, bit for bit."""
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.linear import StreamedWeight
+
+    rows, ks = (256, 2) if n == 28672 else (2048, 1)
+    L = nv.lib()
+    for r in (m, rows) if ks == 2 else (m,):
+        assert L.mv_gemm_prefill_workspace_bytes(r, n, k) == (4096 + 8 * r * n if ks == 2 else 0)
+    x, w, g = _mk(rows, n, k, seed=m + n + k, scale=0.03)
+    wd, xd = w.to(DEV), x.to(DEV)
+    sw = StreamedWeight.from_up_gate(wd[:n // 2], wd[n // 2:]) if mode == "swiglu" else StreamedWeight.from_linear(wd)
+    bias = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if mode == "bias" else None
+    res = torch.randn(rows, n, generator=g).to(torch.bfloat16).to(DEV) if mode == "residual" else None
+    flags = {"swiglu": nv.MV_GEMM_SWIGLU, "f32": nv.MV_GEMM_OUT_F32}.get(mode, 0)
+    # (unsliced products without a workspace: left-over tiles of the many rows are not cut along k either)
+    ws = torch.zeros(1024 + 2 * rows * n, device=DEV) if ks == 2 else None
+
+    def run(r):
+        y = torch.full((r, sw.out_features), float("nan"), dtype=torch.float32 if mode == "f32" else torch.bfloat16, device=DEV)
+        nv.check("mv_gemm_prefill_ws", L.mv_gemm_prefill_ws(
+            xd.data_ptr(), k, sw.tiles.data_ptr(), nv.ptr(bias), nv.ptr(res), n, y.data_ptr(), sw.out_features, r, n, k, flags,
+            nv.ptr(ws), 0 if ws is None else ws.numel() * 4, nv.stream_ptr()))
+        return y
+
+    assert torch.equal(run(m), run(rows)[:m])
