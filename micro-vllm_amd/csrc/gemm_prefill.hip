@@ -1203,9 +1203,9 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
         a.nblocks = (a.nt + 4 * strips - 1) / (4 * strips);
         a.nb_per_xcd = (a.nblocks + 7) / 8;
         const dim3 grid64((unsigned)(8L * a.nb_per_xcd * a.mblocks * a.ksplit));
-        if (strips == 1) hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 1>), grid64, dim3(256), 0, (hipStream_t)stream, a);
+        if (strips == 4) hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 4>), grid64, dim3(256), 0, (hipStream_t)stream, a);
         else if (strips == 2) hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 2>), grid64, dim3(256), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 4>), grid64, dim3(256), 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 1>), grid64, dim3(256), 0, (hipStream_t)stream, a);
     } else if (grid <= num_cus() && a.ktps >= 40) {
         hipLaunchKernelGGL((gemm_prefill_kernel<8, 8, 4>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
     } else {

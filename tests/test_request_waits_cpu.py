@@ -76,3 +76,38 @@ def test_a_stage_of_x_has_arrived_at_the_barrier_before_its_first_reader(assembl
     for b in left:                               # behind the prologue or behind whole passes
         for before in (start, again):
             assert run(before, b)[1] == [pieces]
+
+
+@pytest.mark.parametrize("kernel", ["Li4ELi8ELi4ELi1", "Li4ELi8ELi4ELi2", "Li4ELi8ELi4ELi4"])
+def test_tiles_of_fewer_strips_wait_for_no_less(assembly, kernel):
+    """64-row tiles of one, two and four strips a wave: at every barrier, in any run through the loop and the stages behind it,
+    at most the stage's own two requests of x are on their way.  (The compiler may wait for more in front of its own loads.)"""
+    pieces = 2
+    blocks = _blocks(assembly, kernel)
+    prologue, loop = blocks[0], next(b for b in blocks if b.count("barrier") == 4)
+    left = [b for b in blocks if b.count("barrier") == 1 and b is not prologue]
+    assert prologue.count("x") == 3 * pieces and loop.count("x") == 4 * pieces
+    assert len(left) == 3 and all(b.count("x") == pieces for b in left)
+
+    def run(queue, events):
+        queue, most = list(queue), 0
+        for e in events:
+            if isinstance(e, int):
+                queue = queue[max(0, len(queue) - e):]
+            elif e == "barrier":
+                most = max(most, queue.count("x"))
+            else:
+                queue.append(e)
+        return queue, most
+
+    start, most = run([], prologue)
+    assert most == pieces
+    queue = start
+    for _ in range(3):
+        for tail in range(4):      # up to three stages are left
+            q = queue
+            for b in left[:tail]:
+                q, most = run(q, b)
+                assert most <= pieces
+        queue, most = run(queue, loop)
+        assert most <= pieces
