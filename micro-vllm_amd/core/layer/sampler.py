@@ -30,31 +30,45 @@ def greedy(logits: torch.Tensor, out: torch.Tensor = None, workspace: torch.Tens
     return out[:bs]
 
 
+_MANY_K = 256      # past this many candidates long rows go over several workgroups (csrc/sampler.hip)
+
+
+def _row_params(t, bs, dev):
+    """[bs] fp32 on the device, contiguous: as it is where it is that already."""
+    if t.dtype != torch.float32 or t.device != dev or not t.is_contiguous():
+        t = t.to(device=dev, dtype=torch.float32).contiguous()
+    assert t.numel() == bs
+    return t
+
+
 def sample(logits: torch.Tensor, temperatures: torch.Tensor, top_ps: torch.Tensor, top_k: int,
            uniforms: torch.Tensor = None, out: torch.Tensor = None, generator=None,
-           greedy_ids: torch.Tensor = None) -> torch.Tensor:
+           greedy_ids: torch.Tensor = None, workspace: torch.Tensor = None) -> torch.Tensor:
     """logits [bs,V] bf16 -> int64 [bs]; `uniforms` [bs] in [0,1) (drawn here when not given).
     `greedy_ids` [bs] int64: rows with temperature <= 0 take these without reading the logits.
+    `workspace`: zero-initialised float32 buffer of mv_sample_workspace_bytes() where the parts of a long row meet (default: one
+    per device and stream; none under capture, which must not allocate what outlives it: the same ids from one workgroup a row).
     No host synchronisation."""
     assert logits.is_cuda and logits.dtype == torch.bfloat16 and logits.dim() == 2
     assert logits.stride(1) == 1
     bs, v = logits.shape
     dev = logits.device
-    temperatures = temperatures.to(device=dev, dtype=torch.float32).contiguous()
-    top_ps = top_ps.to(device=dev, dtype=torch.float32).contiguous()
+    temperatures, top_ps = _row_params(temperatures, bs, dev), _row_params(top_ps, bs, dev)
     if uniforms is None:
         uniforms = torch.rand(bs, device=dev, dtype=torch.float32, generator=generator)
-    uniforms = uniforms.to(device=dev, dtype=torch.float32).contiguous()
-    assert temperatures.numel() == bs and top_ps.numel() == bs and uniforms.numel() == bs
+    uniforms = _row_params(uniforms, bs, dev)
     if out is None:
         out = torch.empty(bs, dtype=torch.long, device=dev)
     assert out.dtype == torch.long and out.is_contiguous() and out.numel() >= bs
     ld = logits.stride(0) if bs > 1 else max(v, logits.stride(0))
     if greedy_ids is not None:
         assert greedy_ids.dtype == torch.long and greedy_ids.is_contiguous() and greedy_ids.numel() >= bs
-    nv.check("mv_sample_or_greedy", nv.lib().mv_sample_or_greedy(
+    if workspace is None and top_k > _MANY_K and not torch.cuda.is_current_stream_capturing():
+        workspace = nv.stream_workspace("sample", logits.device, nv.lib().mv_sample_workspace_bytes())
+    nv.check("mv_sample_or_greedy", nv.lib().mv_sample_or_greedy_ws(
         logits.data_ptr(), ld, bs, v, temperatures.data_ptr(), top_ps.data_ptr(), int(top_k),
-        uniforms.data_ptr(), nv.ptr(greedy_ids), out.data_ptr(), nv.stream_ptr()))
+        uniforms.data_ptr(), nv.ptr(greedy_ids), out.data_ptr(), nv.ptr(workspace),
+        0 if workspace is None else workspace.numel() * 4, nv.stream_ptr()))
     return out[:bs]
 
 

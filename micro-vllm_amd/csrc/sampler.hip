@@ -1,4 +1,4 @@
-// Token selection on the device, one workgroup per row of bf16 logits.
+// Token selection on the device, one workgroup per row of bf16 logits, or several where that is the faster.
 //   argmax_kernel : greedy pick (lowest index on ties); reads the row once with 16-byte loads.
 //   sample_kernel : temperature -> top-k -> softmax -> top-p -> draw, the recipe of the reference's
 //                   Sampler._sample_impl (core/layer/sampler.py:21-43), as one launch instead of
@@ -192,203 +192,168 @@ __device__ __forceinline__ T block_scan_incl(T v, T* ws, T& total) {
     return v + base;
 }
 
-__global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __restrict__ logits,
-                                                          int64_t ld, int n,
-                                                          const float* __restrict__ temps,
-                                                          const float* __restrict__ top_ps, int top_k,
-                                                          const float* __restrict__ uniforms,
-                                                          const int64_t* __restrict__ greedy_ids,
-                                                          int64_t* __restrict__ ids) {
-    // A row whose greedy pick is already known (temperature <= 0 and the caller has the argmax)
-    // is done at once: the kernel can then sit in a captured decode step at no cost for greedy
-    // batches.
-    if (greedy_ids != nullptr && !(temps[blockIdx.x] > 0.f)) {  // uniform
-        if (threadIdx.x == 0) ids[blockIdx.x] = greedy_ids[blockIdx.x];
-        return;
-    }
+struct SampleShared {
     // Sixteen copies of the 256-bin histogram, one per lane group: logits share a handful of
     // exponents, so with a single copy nearly every lane of a wave adds to the same LDS word and the
     // adds are served one after the other.  A thread also counts runs of equal bins in a register
     // and adds a whole run at once.
-    __shared__ __attribute__((aligned(16))) unsigned hist[16][256];
-    __shared__ unsigned sh_u[8];
-    __shared__ float c_val[kSmMaxK];
-    __shared__ int c_idx[kSmMaxK];
-    __shared__ float ws_f[kSmThreads / 64];
-    __shared__ unsigned ws_u[kSmThreads / 64];
+    __attribute__((aligned(16))) unsigned hist[16][256];
+    unsigned sh_u[8];
+    float c_val[kSmMaxK];
+    int c_idx[kSmMaxK];
+    float ws_f[kSmThreads / 64];
+    unsigned ws_u[kSmThreads / 64];
+};
 
-    const int tid = threadIdx.x;
-    const uint16_t* row = logits + (int64_t)blockIdx.x * ld;
-    const int nvec = n >> 3;
-    int k = min(min(top_k, n), kSmMaxK);
+// A selection reads the row ONCE: the first kSmKeep chunks of every thread (rows up to 131 072 entries
+// whole) stay in registers for all its passes, requested back to back so that the read costs
+// one memory round trip instead of one per chunk and pass; longer rows stream the rest.
+template <int KEEP>
+__device__ __forceinline__ void load_row(uint4 (&v)[KEEP], const uint16_t* row, int nvec) {
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) v[i] = ld16(row + (int64_t)min((int)threadIdx.x + i * kSmThreads, nvec - 1) * 8);
+}
 
-    // A selection reads the row ONCE: the first kSmKeep chunks of every thread (rows up to 131 072 entries
-    // whole) stay in registers for all its passes, requested back to back so that the read costs
-    // one memory round trip instead of one per chunk and pass; longer rows stream the rest.
-    auto load_row = [&](uint4(&v)[kSmKeep]) {
+__device__ __forceinline__ s16x2_t as_pair(uint32_t v) { return __builtin_bit_cast(s16x2_t, v); }
+__device__ __forceinline__ uint4 to_keys(uint4 v) {
+    v.x = __builtin_bit_cast(uint32_t, pair_key(as_pair(v.x)));
+    v.y = __builtin_bit_cast(uint32_t, pair_key(as_pair(v.y)));
+    v.z = __builtin_bit_cast(uint32_t, pair_key(as_pair(v.z)));
+    v.w = __builtin_bit_cast(uint32_t, pair_key(as_pair(v.w)));
+    return v;
+}
+// Largest of the values so far as signed and as unsigned 16-bit numbers, two instructions a pair where keys take five: bf16
+// values of positive sign lie in the order of their keys, and the NaNs of negative sign are the largest unsigned numbers.
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2_t;
+struct Largest {
+    s16x2_t s = {kKeyLow, kKeyLow};
+    u16x2_t u = {0, 0};
+    __device__ __forceinline__ void add(const uint4& v) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int i = 0; i < kSmKeep; ++i) v[i] = ld16(row + (int64_t)min(tid + i * kSmThreads, nvec - 1) * 8);
-    };
-    // ---- The k largest through the threads' maxima.  The k-th largest of the 1024 maxima bounds the k-th largest entry
-    // from below (k different entries reach it), and few others do: of 128256 random logits 52 reach the bound for k =
-    // 50, 295 for 256.  Those are listed and ranked by counting.  Only where more than kSmQuickMost entries reach the
-    // bound (rows of mostly equal logits), for larger k and for rows with a NaN or of -infinity alone the selection below
-    // runs: for k = 512 ranking by counting took longer than it (98 against 90 us).  The maxima take three packed 16-bit instructions an
-    // entry pair; the radix selection makes two LDS atomics an entry.  32 rows of 128256, top 50: 80 -> 14.8 us;
-    // top 200: 85 -> 22; ten entries left of 128256 and the rest masked 57 -> 13.1.  A row that the selection has to take
-    // after all reads its entries again (kept over both, they do not fit the registers) and is 5 to 11 us later
-    // there: 32 rows of equal logits 57 -> 68.
-    auto in_row = [&](int i) { return tid + i * kSmThreads < nvec; };
-    auto pair = [](uint32_t v) { return __builtin_bit_cast(s16x2_t, v); };
-    bool listed = false;
-    if (k <= kSmQuickK) {   // uniform
-        uint4 keep[kSmKeep];
-        load_row(keep);
-        s16x2_t hi = {kKeyLow, kKeyLow}, lo = {32767, 32767};
-        auto widen = [&](const uint4& keys) {
-            const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                hi = __builtin_elementwise_max(hi, pair(w[j]));
-                lo = __builtin_elementwise_min(lo, pair(w[j]));
-            }
-        };
-        auto to_keys = [&](uint4 v) {
-            v.x = __builtin_bit_cast(uint32_t, pair_key(pair(v.x)));
-            v.y = __builtin_bit_cast(uint32_t, pair_key(pair(v.y)));
-            v.z = __builtin_bit_cast(uint32_t, pair_key(pair(v.z)));
-            v.w = __builtin_bit_cast(uint32_t, pair_key(pair(v.w)));
-            return v;
-        };
-#pragma unroll
-        for (int i = 0; i < kSmKeep; ++i) {
-            keep[i] = to_keys(keep[i]);
-            if (in_row(i)) widen(keep[i]);
+        for (int j = 0; j < 4; ++j) {
+            s = __builtin_elementwise_max(s, as_pair(w[j]));
+            u = __builtin_elementwise_max(u, __builtin_bit_cast(u16x2_t, w[j]));
         }
-        for (int c = kSmKeep * kSmThreads + tid; c < nvec; c += kSmThreads) widen(to_keys(ld16(row + (int64_t)c * 8)));
-        const short top = hi.x > hi.y ? hi.x : hi.y, bottom = lo.x < lo.y ? lo.x : lo.y;
-        unsigned short* maxima = reinterpret_cast<unsigned short*>(&hist[0][0]);   // offset by 32768: unsigned order
-        unsigned* reach = &hist[4][0];      // per wave: maxima that reach its candidate
-        uint64_t* cand = reinterpret_cast<uint64_t*>(&hist[5][0]);   // key, then ~index: unsigned order is the row's order
-        unsigned* ranks = &hist[9][0];
-        if (tid == 0) sh_u[2] = sh_u[3] = sh_u[4] = 0;
-        __syncthreads();
-        maxima[tid] = (unsigned short)(top + 32768);
-        if (tid < kSmQuickMost) ranks[tid] = 0;
-        if (top > kKeyInf || bottom < kKeyNegInf) sh_u[3] = 1;     // a NaN
-        __syncthreads();
-        // the k-th largest maximum, four bits a round: wave w counts who reaches digit w
-        const int wave = tid >> 6, lane = tid & 63;
-        const uint4 m0 = *reinterpret_cast<const uint4*>(maxima + lane * 16), m1 = *reinterpret_cast<const uint4*>(maxima + lane * 16 + 8);
-        const uint32_t mw[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-        unsigned bound = 0;
-        for (int shift = 12; shift >= 0; shift -= 4) {
-            const unsigned cand = bound | ((unsigned)wave << shift);
-            unsigned cnt = 0;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                cnt += __popcll(__ballot((mw[j] & 0xffffu) >= cand));
-                cnt += __popcll(__ballot((mw[j] >> 16) >= cand));
-            }
-            if (lane == 0) reach[wave] = cnt;
-            __syncthreads();
-            int digit = 0;
-#pragma unroll
-            for (int w = 1; w < 16; ++w)
-                if (reach[w] >= (unsigned)k) digit = w;    // fewer reach a larger digit
-            bound |= (unsigned)digit << shift;
-            __syncthreads();
-        }
-        // Entries of -infinity (masked out) have no weight beside any other: a row with fewer than k others has only those.
-        const int thr = max((int)bound - 32768, kKeyNegInf + 1);
-        auto reaching = [&](const uint4& keys) {     // how many of eight entries reach the bound
-            const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
-            const s16x2_t m = __builtin_elementwise_max(__builtin_elementwise_max(pair(w[0]), pair(w[1])),
-                                                        __builtin_elementwise_max(pair(w[2]), pair(w[3])));
-            unsigned n = 0;
-            if (m.x >= thr || m.y >= thr) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) n += (unsigned)(pair(w[j]).x >= thr) + (unsigned)(pair(w[j]).y >= thr);
-            }
-            return n;
-        };
-        unsigned slot = 0;
-        auto list = [&](const uint4& keys, int c) {
-            const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const s16x2_t kk = pair(w[j >> 1]);
-                const int key = j & 1 ? kk.y : kk.x;
-                if (key < thr) continue;
-                cand[slot++] = (uint64_t)(unsigned)(key + 32768) << 32 | (unsigned)~(c * 8 + j);
-                if (key == -1) sh_u[4] = 1;                  // -0.0
-            }
-        };
-        if (!sh_u[3]) {   // uniform
-            // counted before anything is listed: a full list costs its rows no more than the count
-            unsigned hits = 0, mine_n = 0;
-            if (top >= thr) {
-#pragma unroll
-                for (int i = 0; i < kSmKeep; ++i)
-                    if (in_row(i)) {
-                        const unsigned n = reaching(keep[i]);
-                        hits |= n ? 1u << i : 0u;
-                        mine_n += n;
-                    }
-                for (int c = kSmKeep * kSmThreads + tid; c < nvec; c += kSmThreads) mine_n += reaching(to_keys(ld16(row + (int64_t)c * 8)));
-                if (mine_n) slot = atomicAdd(&sh_u[2], mine_n);
-            }
-            __syncthreads();
-            const unsigned found = sh_u[2];
-            if (found > 0 && found <= (unsigned)kSmQuickMost) {   // uniform
-                listed = true;
-                k = min(k, (int)found);
-                if (mine_n) {
-#pragma unroll
-                    for (int i = 0; i < kSmKeep; ++i)
-                        if (hits >> i & 1) list(keep[i], tid + i * kSmThreads);
-                    for (int c = kSmKeep * kSmThreads + tid; c < nvec; c += kSmThreads) list(to_keys(ld16(row + (int64_t)c * 8)), c);
-                }
-                __syncthreads();
-                // place among the candidates by counting who comes before: F threads, one for each, for every part of the
-                // list (whole waves read the same entry); the first k stay
-                unsigned F = 64;
-                while (F < found) F <<= 1;
-                const unsigned parts = kSmThreads / F, span = (found + parts - 1) / parts;
-                const unsigned i = tid & (F - 1), j0 = tid / F * span, j1 = min(found, j0 + span);
-                const uint64_t me = i < found ? cand[i] : 0;
-                unsigned before = 0;
-                for (unsigned j = j0; j < j1; ++j) before += cand[j] > me;
-                if (i < found && before) atomicAdd(&ranks[i], before);
-                __syncthreads();
-                const unsigned rank = tid < (int)found ? ranks[tid] : (unsigned)k;
-                const bool mine = rank < (unsigned)k;
-                const int my_idx = (int)~(unsigned)me;      // (threads below F hold entry tid)
-                if (mine) {
-                    const int key = (int)(me >> 32) - 32768;
-                    c_val[rank] = bf16_bits_to_f32((unsigned short)(key ^ ((key >> 15) & 0x7fff)));
-                    c_idx[rank] = my_idx;
-                }
-                __syncthreads();
-                if (sh_u[4]) {   // uniform; zeros of both signs are equal: among those the index decides
-                    const float my_val = mine ? c_val[rank] : 0.f;
-                    unsigned place = 0;
-                    if (mine)
-                        for (int j = 0; j < k; ++j) place += c_val[j] > my_val || (c_val[j] == my_val && c_idx[j] < my_idx);
-                    __syncthreads();
-                    if (mine) {
-                        c_val[place] = my_val;
-                        c_idx[place] = my_idx;
-                    }
-                    __syncthreads();
-                }
-            }
-        }
-        if (!listed) __syncthreads();
     }
-    if (!listed) {
+    __device__ __forceinline__ short top() const { return s.x > s.y ? s.x : s.y; }
+    __device__ __forceinline__ bool nan() const { return top() > kKeyInf || max((int)u.x, (int)u.y) > 0xff80; }
+};
+// largest key of the eight of a chunk or of `top`
+__device__ __forceinline__ short top_key(short top, const uint4& v) {
+    const uint4 k = to_keys(v);
+    const s16x2_t m = __builtin_elementwise_max(__builtin_elementwise_max(as_pair(k.x), as_pair(k.y)),
+                                                __builtin_elementwise_max(as_pair(k.z), as_pair(k.w)));
+    const short t = m.x > m.y ? m.x : m.y;
+    return t > top ? t : top;
+}
+// what stands for the keys beside a bound: the values themselves where the bound is one of positive sign
+__device__ __forceinline__ uint4 keys_beside(int thr, const uint4& v) { return thr >= 0 ? v : to_keys(v); }
+// how many of eight entries reach the bound
+__device__ __forceinline__ unsigned reaching(const uint4& keys, int thr) {
+    const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
+    const s16x2_t m = __builtin_elementwise_max(__builtin_elementwise_max(as_pair(w[0]), as_pair(w[1])),
+                                                __builtin_elementwise_max(as_pair(w[2]), as_pair(w[3])));
+    unsigned n = 0;
+    if (m.x >= thr || m.y >= thr) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) n += (unsigned)(as_pair(w[j]).x >= thr) + (unsigned)(as_pair(w[j]).y >= thr);
+    }
+    return n;
+}
+// those entries of chunk c into cand from `slot` on, as key, then ~index: unsigned order is the row's order
+__device__ __forceinline__ void list_entries(const uint4& keys, int c, int thr, unsigned& slot, uint64_t* cand, unsigned* zero_flag) {
+    const uint32_t w[4] = {keys.x, keys.y, keys.z, keys.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const s16x2_t kk = as_pair(w[j >> 1]);
+        const int key = j & 1 ? kk.y : kk.x;
+        if (key < thr) continue;
+        cand[slot++] = (uint64_t)(unsigned)(key + 32768) << 32 | (unsigned)~(c * 8 + j);
+        if (key == -1) *zero_flag = 1;                  // -0.0
+    }
+}
+// The k-th largest of N 16-bit maxima in LDS (offset by 32768: unsigned order), four bits a round: wave w counts who
+// reaches digit w.  `reach`: two words per wave, in turn, so that a round is one barrier.
+template <int N>
+__device__ __forceinline__ unsigned kth_largest(const unsigned short* maxima, unsigned* reach, int k) {
+    constexpr int PER = N / 64, WORDS = PER / 2;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint32_t mw[WORDS];
+#pragma unroll
+    for (int j = 0; j < WORDS; j += 4) {
+        const uint4 m = *reinterpret_cast<const uint4*>(maxima + (j / 4 * 64 + lane) * 8);
+        mw[j] = m.x; mw[j + 1] = m.y; mw[j + 2] = m.z; mw[j + 3] = m.w;
+    }
+    unsigned bound = 0;
+    for (int shift = 12; shift >= 0; shift -= 4) {
+        const unsigned digit_bound = bound | ((unsigned)wave << shift);
+        unsigned cnt = 0;
+#pragma unroll
+        for (int j = 0; j < WORDS; ++j) {
+            cnt += __popcll(__ballot((mw[j] & 0xffffu) >= digit_bound));
+            cnt += __popcll(__ballot((mw[j] >> 16) >= digit_bound));
+        }
+        unsigned* turn = reach + (shift & 4 ? 16 : 0);
+        if (lane == 0) turn[wave] = cnt;
+        __syncthreads();
+        int digit = 0;
+#pragma unroll
+        for (int w = 1; w < 16; ++w)
+            if (turn[w] >= (unsigned)k) digit = w;    // fewer reach a larger digit
+        bound |= (unsigned)digit << shift;
+    }
+    return bound;
+}
+// Up to kSmQuickMost candidates: the place of each by counting who comes before, F threads, one for each, for every part of
+// the list (whole waves read the same entry); the first k go to c_val / c_idx.  `ranks` is zero.
+__device__ __forceinline__ void place_candidates(SampleShared& sh, const uint64_t* cand, unsigned* ranks, unsigned found, int k) {
+    const int tid = threadIdx.x;
+    unsigned F = 64;
+    while (F < found) F <<= 1;
+    const unsigned parts = kSmThreads / F, span = (found + parts - 1) / parts;
+    const unsigned i = tid & (F - 1), j0 = tid / F * span, j1 = min(found, j0 + span);
+    const uint64_t me = i < found ? cand[i] : 0;
+    unsigned before = 0;
+    for (unsigned j = j0; j < j1; ++j) before += cand[j] > me;
+    if (i < found && before) atomicAdd(&ranks[i], before);
+    __syncthreads();
+    const unsigned rank = tid < (int)found ? ranks[tid] : (unsigned)k;
+    if (rank < (unsigned)k) {      // (threads below F hold entry tid)
+        const int key = (int)(me >> 32) - 32768;
+        sh.c_val[rank] = bf16_bits_to_f32((unsigned short)(key ^ ((key >> 15) & 0x7fff)));
+        sh.c_idx[rank] = (int)~(unsigned)me;
+    }
+    __syncthreads();
+}
+// zeros of both signs are equal: among those the index decides
+__device__ __forceinline__ void order_zeros(SampleShared& sh, int k) {
+    const int tid = threadIdx.x;
+    const bool mine = tid < k;
+    const float my_val = mine ? sh.c_val[tid] : 0.f;
+    const int my_idx = mine ? sh.c_idx[tid] : 0;
+    unsigned place = 0;
+    if (mine)
+        for (int j = 0; j < k; ++j) place += sh.c_val[j] > my_val || (sh.c_val[j] == my_val && sh.c_idx[j] < my_idx);
+    __syncthreads();
+    if (mine) {
+        sh.c_val[place] = my_val;
+        sh.c_idx[place] = my_idx;
+    }
+    __syncthreads();
+}
+
+// The k largest entries of a row in order, by a radix selection over 16-bit keys in two passes: any k, rows with NaNs, equal
+// entries without end.
+__device__ void radix_select(SampleShared& sh, const uint16_t* row, int nvec, int k) {
+    auto& hist = sh.hist;
+    auto& sh_u = sh.sh_u;
+    auto& c_val = sh.c_val;
+    auto& c_idx = sh.c_idx;
+    auto& ws_u = sh.ws_u;
+    const int tid = threadIdx.x;
     uint4 keep[kSmKeep];
-    load_row(keep);
+    load_row(keep, row, nvec);
     auto for_each_chunk = [&](auto&& fn) {  // fn(chunk index, 8 values), every thread the same trip count
 #pragma unroll
         for (int i = 0; i < kSmKeep; ++i) fn(tid + i * kSmThreads, keep[i]);
@@ -543,12 +508,17 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
         }
     }
     __syncthreads();
-    }
+}
 
-    // ---- softmax over the k candidates, top-p prefix, inverse-CDF draw
-    const float temp = temps[blockIdx.x];
+// Softmax over the first k of c_val / c_idx (in order), top-p prefix, inverse-CDF draw
+__device__ __forceinline__ void draw_id(SampleShared& sh, int k, float temp, float top_p, float uniform, int64_t* id) {
+    auto& c_val = sh.c_val;
+    auto& c_idx = sh.c_idx;
+    auto& ws_f = sh.ws_f;
+    auto& ws_u = sh.ws_u;
+    const int tid = threadIdx.x;
     if (!(temp > 0.f)) {  // uniform: greedy limit
-        if (tid == 0) ids[blockIdx.x] = c_idx[0];
+        if (tid == 0) *id = c_idx[0];
         return;
     }
     if (k <= 64) {   // one wave holds the candidates: the same sums without the workgroup's barriers
@@ -561,10 +531,10 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
             if (tid >= o) cum += u;
         }
         const float cump = cum / __shfl(cum, 63, 64);
-        const int m = __popcll(__ballot(tid < k && (cump < top_ps[blockIdx.x] || tid == 0)));
-        const float target = uniforms[blockIdx.x] * __shfl(cump, m - 1, 64);
+        const int m = __popcll(__ballot(tid < k && (cump < top_p || tid == 0)));
+        const float target = uniform * __shfl(cump, m - 1, 64);
         const int nb = __popcll(__ballot(tid < m && cump <= target));
-        if (tid == 0) ids[blockIdx.x] = c_idx[min(nb, m - 1)];
+        if (tid == 0) *id = c_idx[min(nb, m - 1)];
         return;
     }
     const float smax = c_val[0] / temp;
@@ -572,18 +542,297 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
     float total;
     const float cum = block_scan_incl(e, ws_f, total);
     const float cump = cum / total;
-    const float top_p = top_ps[blockIdx.x];
     const unsigned valid = (tid < k) && (cump < top_p || tid == 0);
     unsigned m;
     block_scan_incl(valid, ws_u, m);               // the valid set is a prefix: m = its length
     if (tid == (int)m - 1) ws_f[0] = cump;           // mass kept
     __syncthreads();
-    const float target = uniforms[blockIdx.x] * ws_f[0];
+    const float target = uniform * ws_f[0];
     __syncthreads();
     const unsigned below = (tid < (int)m) && (cump <= target);
     unsigned nb;
     block_scan_incl(below, ws_u, nb);
-    if (tid == 0) ids[blockIdx.x] = c_idx[min(nb, m - 1)];
+    if (tid == 0) *id = c_idx[min(nb, m - 1)];
+}
+
+// KEEP: chunks of the row a thread holds for the quick selection, 4 for rows of up to 32768 entries, whose threads would
+// otherwise request the same chunk again and again (32 rows of 32000, top 50: 13.0 -> 8.7 us with what else changed there).
+template <int KEEP>
+__global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __restrict__ logits,
+                                                          int64_t ld, int n,
+                                                          const float* __restrict__ temps,
+                                                          const float* __restrict__ top_ps, int top_k,
+                                                          const float* __restrict__ uniforms,
+                                                          const int64_t* __restrict__ greedy_ids,
+                                                          int64_t* __restrict__ ids) {
+    // A row whose greedy pick is already known (temperature <= 0 and the caller has the argmax)
+    // is done at once: the kernel can then sit in a captured decode step at no cost for greedy
+    // batches.
+    if (greedy_ids != nullptr && !(temps[blockIdx.x] > 0.f)) {  // uniform
+        if (threadIdx.x == 0) ids[blockIdx.x] = greedy_ids[blockIdx.x];
+        return;
+    }
+    __shared__ SampleShared sh;
+    auto& sh_u = sh.sh_u;
+    const int tid = threadIdx.x;
+    const uint16_t* row = logits + (int64_t)blockIdx.x * ld;
+    const int nvec = n >> 3;
+    int k = min(min(top_k, n), kSmMaxK);
+    // (asked for here: each would be a trip to memory behind the selection)
+    const float temp = temps[blockIdx.x], top_p = top_ps[blockIdx.x], uniform = uniforms[blockIdx.x];
+    // ---- The k largest through the threads' maxima.  The k-th largest of the 1024 maxima bounds the k-th largest entry
+    // from below (k different entries reach it), and few others do: of 128256 random logits 52 reach the bound for k =
+    // 50, 295 for 256.  Those are listed and ranked by counting.  Only where more than kSmQuickMost entries reach the
+    // bound (rows of mostly equal logits), for larger k and for rows with a NaN or of -infinity alone the selection below
+    // runs: for k = 512 ranking by counting took longer than it (98 against 90 us).  The maxima take two packed 16-bit instructions an
+    // entry pair; the radix selection makes two LDS atomics an entry.  32 rows of 128256, top 50: 80 -> 12.3 us;
+    // top 200: 85 -> 18; ten entries left of 128256 and the rest masked 57 -> 11.3.  A row that the selection has to take
+    // after all reads its entries again (kept over both, they do not fit the registers) and is 5 to 11 us later
+    // there: 32 rows of equal logits 57 -> 68.  What a call needs besides the row - temperature, top-p, the uniform number - is
+    // requested in front: three trips to memory behind the selection were 1.5 us of 15.6.
+    auto in_row = [&](int i) { return tid + i * kSmThreads < nvec; };
+    bool listed = false;
+    if (k <= kSmQuickK) {   // uniform
+        uint4 keep[KEEP];
+        load_row(keep, row, nvec);
+        Largest most;
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i)
+            if (in_row(i)) most.add(keep[i]);
+        for (int c = KEEP * kSmThreads + tid; c < nvec; c += kSmThreads) most.add(ld16(row + (int64_t)c * 8));
+        short top = most.top();
+        if (top < 0) {      // nothing of positive sign here: the order of the keys
+            top = kKeyLow;
+#pragma unroll
+            for (int i = 0; i < KEEP; ++i)
+                if (in_row(i)) top = top_key(top, keep[i]);
+            for (int c = KEEP * kSmThreads + tid; c < nvec; c += kSmThreads) top = top_key(top, ld16(row + (int64_t)c * 8));
+        }
+        unsigned short* maxima = reinterpret_cast<unsigned short*>(&sh.hist[0][0]);   // offset by 32768: unsigned order
+        uint64_t* cand = reinterpret_cast<uint64_t*>(&sh.hist[5][0]);
+        unsigned* ranks = &sh.hist[9][0];
+        if (tid == 0) sh_u[2] = sh_u[3] = sh_u[4] = 0;
+        __syncthreads();
+        maxima[tid] = (unsigned short)(top + 32768);
+        if (tid < kSmQuickMost) ranks[tid] = 0;
+        if (most.nan()) sh_u[3] = 1;
+        __syncthreads();
+        const unsigned bound = kth_largest<kSmThreads>(maxima, &sh.hist[4][0], k);
+        // Entries of -infinity (masked out) have no weight beside any other: a row with fewer than k others has only those.
+        const int thr = max((int)bound - 32768, kKeyNegInf + 1);
+        if (!sh_u[3]) {   // uniform
+            // Counted before anything is listed: a full list costs its rows no more than the count.  A chunk with an entry to
+            // list is read again: one body for any chunk, where sixteen over `keep` are twelve KiB of code to fetch (32 rows of
+            // 128256, top 50: 14.7 us with those, 12.3 without).
+            unsigned hits = 0, mine_n = 0, slot = 0;
+            auto count = [&](auto key) {
+#pragma unroll
+                for (int i = 0; i < KEEP; ++i)
+                    if (in_row(i)) {
+                        const unsigned c = reaching(key(keep[i]), thr);
+                        hits |= c ? 1u << i : 0u;
+                        mine_n += c;
+                    }
+            };
+            if (top >= thr) {
+                if (thr >= 0) count([](const uint4& v) { return v; });   // (values of positive sign are their keys)
+                else count([](const uint4& v) { return to_keys(v); });
+                for (int c = KEEP * kSmThreads + tid; c < nvec; c += kSmThreads) mine_n += reaching(to_keys(ld16(row + (int64_t)c * 8)), thr);
+                if (mine_n) slot = atomicAdd(&sh_u[2], mine_n);
+            }
+            __syncthreads();
+            const unsigned found = sh_u[2];
+            if (found > 0 && found <= (unsigned)kSmQuickMost) {   // uniform
+                listed = true;
+                k = min(k, (int)found);
+                auto list = [&](int c) {
+                    const uint4 keys = to_keys(ld16(row + (int64_t)c * 8));
+                    list_entries(keys, c, thr, slot, cand, &sh_u[4]);
+                };
+                if (mine_n) {
+                    for (; hits; hits &= hits - 1) list(tid + (__ffs(hits) - 1) * kSmThreads);
+                    for (int c = KEEP * kSmThreads + tid; c < nvec; c += kSmThreads) list(c);
+                }
+                __syncthreads();
+                place_candidates(sh, cand, ranks, found, k);
+                if (sh_u[4]) order_zeros(sh, k);   // uniform
+            }
+        }
+        if (!listed) __syncthreads();
+    }
+    if (!listed) radix_select(sh, row, nvec, k);
+    draw_id(sh, k, temp, top_p, uniform, ids + blockIdx.x);
+}
+
+// The same with a row cut over kSmParts workgroups, for any k.  One workgroup a row is bound by what a compute unit reads and
+// by the selection's passes over what it read; here each part only takes its threads' maxima (their 4 x 1024 bound the k-th
+// largest entry closer than 1024 do: of 128256 random logits 50 reach it for k = 50, 1160 for 1000), and the workgroup
+// that draws the row's last arrival ticket finds the bound and reads again only what lies behind the maxima that reach it.
+// More than kSmQuickMost candidates are sorted in LDS.  Workspace: tickets | maxima, tickets as in the greedy pick above.
+// For k up to kSmQuickK one workgroup is the faster one: handing the maxima over costs 4 us of its 8 to 18.  Top 1000 of 128256: 1 row
+// 92 -> 37 us, 32 rows 100 -> 39, 64 rows 101 -> 41; of 16384: 39 -> 35; but 128 rows of 32000 52 -> 72, so up to 64 rows.
+constexpr int kSmParts = 4;
+constexpr int kSmMaxRows = 64;
+constexpr int kSmSortMost = 2048;
+constexpr int kSmMinVec = 2 * kSmThreads;   // chunks of a row that is worth cutting
+constexpr size_t kSmTicketBytes = (size_t)kSmMaxRows * 64 * sizeof(unsigned int);
+constexpr size_t kSmWorkspaceBytes = kSmTicketBytes + (size_t)kSmMaxRows * kSmParts * kSmThreads * sizeof(unsigned short);
+
+__global__ __launch_bounds__(kSmThreads) void sample_parts_kernel(const uint16_t* __restrict__ logits, int64_t ld, int n,
+                                                                const float* __restrict__ temps,
+                                                                const float* __restrict__ top_ps, int top_k,
+                                                                const float* __restrict__ uniforms,
+                                                                const int64_t* __restrict__ greedy_ids,
+                                                                int64_t* __restrict__ ids, unsigned int* tickets,
+                                                                unsigned short* row_maxima) {
+    constexpr int kGroups = kSmParts * kSmThreads;
+    const int rowi = blockIdx.x / kSmParts, part = blockIdx.x % kSmParts, tid = threadIdx.x;
+    if (greedy_ids != nullptr && !(temps[rowi] > 0.f)) {  // uniform over the row: nobody takes a ticket
+        if (part == 0 && tid == 0) ids[rowi] = greedy_ids[rowi];
+        return;
+    }
+    __shared__ SampleShared sh;
+    __shared__ __attribute__((aligned(16))) unsigned short maxima[kGroups];
+    __shared__ uint64_t cand[kSmSortMost];
+    auto& sh_u = sh.sh_u;
+    const uint16_t* row = logits + (int64_t)rowi * ld;
+    const int nvec = n >> 3, span = (nvec + kSmParts - 1) / kSmParts;
+    int k = min(min(top_k, n), kSmMaxK);
+    // thread t of part p: chunks p * span + t, + 1024, .. of the part
+    {
+        const int c0 = part * span, c1 = min(nvec, c0 + span);
+        short top = kKeyLow;
+        bool nan = false;
+        for (int b = c0 + tid; b < c1; b += 4 * kSmThreads) {
+            uint4 v[4];
+            Largest most;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = ld16(row + (int64_t)min(b + i * kSmThreads, c1 - 1) * 8);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (b + i * kSmThreads < c1) most.add(v[i]);
+            nan = nan || most.nan();
+            if (most.top() >= 0) {
+                top = most.top() > top ? most.top() : top;
+            } else {      // nothing of positive sign here: the order of the keys
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (b + i * kSmThreads < c1) top = top_key(top, v[i]);
+            }
+        }
+        // a NaN anywhere: the largest maximum there is
+        const unsigned mine = nan ? 0xffffu : (unsigned)(top + 32768), next = __shfl_down(mine, 1, 64);
+        if (!(tid & 1))
+            __hip_atomic_store(reinterpret_cast<unsigned int*>(row_maxima) + ((size_t)rowi * kGroups + part * kSmThreads + tid) / 2,
+                               mine | next << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every storing wave's maxima have left before the ticket
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned old = __hip_atomic_fetch_add(tickets + rowi * 64, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sh_u[5] = old == (unsigned)kSmParts - 1u;
+        if (sh_u[5])  // back to zero for the next launch; nobody else touches it in this one
+            __hip_atomic_store(tickets + rowi * 64, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sh_u[2] = sh_u[3] = sh_u[4] = sh_u[6] = 0;
+    }
+    __syncthreads();
+    if (!sh_u[5]) return;
+    const float temp = temps[rowi], top_p = top_ps[rowi], uniform = uniforms[rowi];
+    // the 4096 maxima of all parts, two words a thread
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const unsigned m = __hip_atomic_load(reinterpret_cast<unsigned int*>(row_maxima) + (size_t)rowi * kGroups / 2 + i * kSmThreads + tid,
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        reinterpret_cast<unsigned int*>(maxima)[i * kSmThreads + tid] = m;
+        nan = nan || (int)(m & 0xffffu) - 32768 > kKeyInf || (int)(m >> 16) - 32768 > kKeyInf;
+    }
+    if (nan) sh_u[3] = 1;
+    __syncthreads();
+    bool listed = false;
+    if (!sh_u[3]) {   // uniform
+        const unsigned bound = kth_largest<kGroups>(maxima, &sh.hist[4][0], k);
+        const int thr = max((int)bound - 32768, kKeyNegInf + 1);     // (-infinity has no weight beside any other, as above)
+        // the threads whose maxima reach the bound
+        unsigned short* groups = reinterpret_cast<unsigned short*>(&sh.hist[0][0]);
+#pragma unroll
+        for (int i = 0; i < kSmParts; ++i) {
+            const int g = i * kSmThreads + tid;
+            if ((int)maxima[g] - 32768 >= thr) {
+                const unsigned at = atomicAdd(&sh_u[6], 1u);
+                if (at < (unsigned)kSmSortMost) groups[at] = (unsigned short)g;
+            }
+        }
+        __syncthreads();
+        const int ngroups = sh_u[6];
+        if (ngroups <= kSmSortMost) {   // uniform (each brings a candidate: more could not be held)
+            for (int it = tid; it < ngroups; it += kSmThreads) {
+                const int g = groups[it], c0 = g / kSmThreads * span, c1 = min(nvec, c0 + span);
+                for (int b = c0 + g % kSmThreads; b < c1; b += 4 * kSmThreads) {
+                    uint4 v[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = ld16(row + (int64_t)min(b + i * kSmThreads, c1 - 1) * 8);
+                    unsigned cnt[4], all = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        v[i] = keys_beside(thr, v[i]);
+                        cnt[i] = b + i * kSmThreads < c1 ? reaching(v[i], thr) : 0;
+                        all += cnt[i];
+                    }
+                    if (!all) continue;
+                    unsigned slot = atomicAdd(&sh_u[2], all);
+                    if (slot + all > (unsigned)kSmSortMost) continue;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (cnt[i]) list_entries(v[i], b + i * kSmThreads, thr, slot, cand, &sh_u[4]);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        const unsigned found = ngroups <= kSmSortMost ? sh_u[2] : 0;
+        if (found > 0 && found <= (unsigned)kSmSortMost) {   // uniform
+            listed = true;
+            k = min(k, (int)found);
+            if (found <= (unsigned)kSmQuickMost) {
+                unsigned* ranks = &sh.hist[8][0];
+                if (tid < kSmQuickMost) ranks[tid] = 0;
+                __syncthreads();
+                place_candidates(sh, cand, ranks, found, k);
+            } else {      // bitonic, descending; a thread orders one pair a step
+                unsigned size2 = kSmQuickMost;
+                while (size2 < found) size2 <<= 1;
+                for (unsigned i = found + tid; i < size2; i += kSmThreads) cand[i] = 0;
+                // (a wave's threads hold 128 neighbouring entries: up to a stride of 64 the steps are its own)
+                for (unsigned size = 2; size <= size2; size <<= 1)
+                    for (unsigned stride = size >> 1; stride > 0; stride >>= 1) {
+                        if (stride >= 64 || size == 2) __syncthreads();
+                        else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        const unsigned i = 2 * stride * (tid / stride) + tid % stride, j = i + stride;
+                        if (j < size2) {
+                            const uint64_t x = cand[i], y = cand[j];
+                            if ((x < y) == ((i & size) == 0)) {
+                                cand[i] = y;
+                                cand[j] = x;
+                            }
+                        }
+                    }
+                __syncthreads();
+                if (tid < k) {
+                    const int key = (int)(cand[tid] >> 32) - 32768;
+                    sh.c_val[tid] = bf16_bits_to_f32((unsigned short)(key ^ ((key >> 15) & 0x7fff)));
+                    sh.c_idx[tid] = (int)~(unsigned)cand[tid];
+                }
+                __syncthreads();
+            }
+            if (sh_u[4]) order_zeros(sh, k);   // uniform
+        }
+    }
+    if (!listed) {
+        __syncthreads();
+        radix_select(sh, row, nvec, k);
+    }
+    draw_id(sh, k, temp, top_p, uniform, ids + rowi);
 }
 
 }  // namespace mv
@@ -599,13 +848,30 @@ extern "C" int mv_sample_or_greedy(const void* logits, int64_t ld, int rows, int
                                    const float* temperatures, const float* top_ps, int top_k,
                                    const float* uniforms, const int64_t* greedy_ids, int64_t* ids,
                                    mv_stream_t stream) {
+    return mv_sample_or_greedy_ws(logits, ld, rows, n, temperatures, top_ps, top_k, uniforms, greedy_ids, ids, nullptr, 0, stream);
+}
+
+extern "C" size_t mv_sample_workspace_bytes(void) { return mv::kSmWorkspaceBytes; }
+
+extern "C" int mv_sample_or_greedy_ws(const void* logits, int64_t ld, int rows, int n,
+                                      const float* temperatures, const float* top_ps, int top_k,
+                                      const float* uniforms, const int64_t* greedy_ids, int64_t* ids,
+                                      void* workspace, size_t workspace_bytes, mv_stream_t stream) {
     if (rows == 0 && n > 0) return MV_OK;
     if (!logits || !ids || !temperatures || !top_ps || !uniforms || rows < 0 || n <= 0 || ld < n ||
         top_k <= 0)
         return MV_ERR_INVALID_ARG;
     if (!mv::aligned16(logits) || (ld % 8) != 0) return MV_ERR_INVALID_ARG;
     if ((n % 8) != 0) return MV_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(mv::sample_kernel, dim3(rows), dim3(mv::kSmThreads), 0, (hipStream_t)stream,
+    if (workspace && workspace_bytes >= mv::kSmWorkspaceBytes && mv::aligned16(workspace) && rows <= mv::kSmMaxRows &&
+        top_k > mv::kSmQuickK && (n >> 3) >= mv::kSmMinVec) {
+        hipLaunchKernelGGL(mv::sample_parts_kernel, dim3(rows * mv::kSmParts), dim3(mv::kSmThreads), 0, (hipStream_t)stream,
+                           (const uint16_t*)logits, ld, n, temperatures, top_ps, top_k, uniforms, greedy_ids, ids,
+                           (unsigned int*)workspace, (unsigned short*)((char*)workspace + mv::kSmTicketBytes));
+        return mv::check_launch();
+    }
+    const auto kernel = (n >> 3) <= 4 * mv::kSmThreads ? mv::sample_kernel<4> : mv::sample_kernel<mv::kSmKeep>;
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(mv::kSmThreads), 0, (hipStream_t)stream,
                        (const uint16_t*)logits, ld, n, temperatures, top_ps, top_k, uniforms, greedy_ids, ids);
     return mv::check_launch();
 }

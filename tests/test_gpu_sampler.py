@@ -158,3 +158,48 @@ def test_greedy_on_two_streams_and_without_workspace(mv):
         nv.check("mv_argmax", nv.lib().mv_argmax(xs[i].data_ptr(), xs[i].stride(0), 2, 128256,
                                                  ids.data_ptr(), None, 0, nv.stream_ptr()))
         assert torch.equal(ids, want[i])
+
+
+@pytest.mark.parametrize("v", [16376, 16384, 16392, 32000, 128256, 131080, 151936])
+@pytest.mark.parametrize("kind", ["random", "ties", "equal", "zeros", "sorted", "few", "nan", "masked"])
+def test_rows_over_several_workgroups_pick_what_one_picks(mv, v, kind):
+    """The same ids with a workspace (rows of 16384 and more over several workgroups) and without: few and many candidates
+    (ranked, sorted, and too many of them: the radix selection), parts that end unevenly, entries of the largest maxima at
+    the row's ends, rows whose greedy pick is given; twice, since the tickets have to be back at zero."""
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.core.layer.sampler import sample
+
+    g = torch.Generator().manual_seed(v)
+    bs = 9
+    x = torch.randn(bs, v, generator=g) * 3
+    if kind == "ties":
+        x = (x * 2).round() / 2
+    elif kind == "equal":
+        x = torch.ones(bs, v)
+    elif kind == "zeros":
+        x = -x.abs().round()
+    elif kind == "sorted":
+        x = x.sort(dim=-1).values
+    elif kind == "few":
+        x[:, 3:-3] = -float("inf")
+    elif kind == "nan":
+        x[:, v // 2] = float("nan")
+    elif kind == "masked":
+        x[:] = -float("inf")
+    x = x.to(torch.bfloat16).to(DEV)
+    temps = (torch.rand(bs, generator=g) * 1.5 + 0.05).to(DEV)
+    temps[2] = 0.0
+    top_ps = (torch.rand(bs, generator=g) * 0.3 + 0.7).to(DEV)
+    top_ps[4] = 2.0
+    u = torch.rand(bs, generator=g).to(DEV)
+    u[5] = 0.99999
+    known = torch.arange(bs, device=DEV)
+    L = nv.lib()
+    for k in (1, 2, 50, 256, 257, 600, 1024, 4096):
+        for greedy_ids in (None, known):
+            want = torch.empty(bs, dtype=torch.long, device=DEV)
+            nv.check("mv_sample_or_greedy", L.mv_sample_or_greedy(
+                x.data_ptr(), v, bs, v, temps.data_ptr(), top_ps.data_ptr(), k, u.data_ptr(), nv.ptr(greedy_ids), want.data_ptr(),
+                nv.stream_ptr()))
+            for _ in range(2):
+                assert torch.equal(sample(x, temps, top_ps, k, uniforms=u, greedy_ids=greedy_ids), want), (k, greedy_ids)
