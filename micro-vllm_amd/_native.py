@@ -245,10 +245,17 @@ def check(fn_name, status):
 
 def stream_ptr(stream=None):
     """hipStream_t of `stream` (default: torch's current stream) as an int."""
+    return stream.cuda_stream if stream is not None else _raw_stream(None)
+
+
+def _raw_stream(index):
+    """hipStream_t of the current stream of device `index` (None: the current one).  Asked of torch's own table: a Stream
+    object made to read its handle from costs 1.5 us, and every launch asks."""
     import torch
 
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(index).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if index is None else index)
 
 
 def ptr(t):
@@ -268,9 +275,9 @@ def stream_workspace(kind, device, nbytes):
 
     if nbytes <= 0:
         return None
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    key = (kind, idx, torch.cuda.current_stream(idx).cuda_stream)
+    key = (kind, idx, _raw_stream(idx))
     ws = _stream_ws.get(key)
     if ws is None or ws.numel() * 4 < nbytes:
         ws = torch.zeros((nbytes + 3) // 4, dtype=torch.float32, device=dev)
