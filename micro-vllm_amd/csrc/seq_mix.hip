@@ -1892,8 +1892,6 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     }
 
     const TileRun gt = tile_run(pos, window, keep_first, chunked);
-    if (max_len > 0 && row_len[row] > max_len) return;   // the tiled kernel's rows
-    if (split * NW >= gt.n) return;                      // no keys for this split
     const int* bt = pr.block_table + (int64_t)row * pr.bt_stride;
     float m[HB], l[HB];
     wa_f32x4_t acc[HB][VE];
@@ -1916,6 +1914,9 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
         page_no = bt[j / pr.page];
     };
     locate(split * NW + wv);
+    // (behind the page's request: the length in front of it would be one more trip to memory)
+    if (max_len > 0 && row_len[row] > max_len) return;   // the tiled kernel's rows
+    if (split * NW >= gt.n) return;                      // no keys for this split
     for (int u = split * NW + wv; u < gt.n; u += NW * splits) {
         const unsigned slot = (unsigned)page_no * (unsigned)pr.page + (unsigned)(j % pr.page);
         const T_* kr = kc + ((uint64_t)slot * G + g) * d;
