@@ -683,6 +683,11 @@ int mv_sigmoid_gate(const float* a, int64_t lda, const float* g, int64_t ldg, vo
 
 /* ---- products per head and per segment (linear_any.hip) --------------------------------------------- */
 
+/* mv_linear_any on fp32 operands, left in `slabs` as mv_linear_any_slab_count(m, n, k) k-slices [slice][m][n] whose sum, in
+ * order, is the product (as mv_linear_slabs).  More than one needs x and w 16-byte aligned and ldx, ldw multiples of 4. */
+int mv_linear_any_slab_count(int m, int n, int k);
+int mv_linear_any_slabs(const float* x, int64_t ldx, const float* w, int64_t ldw, float* slabs, size_t slabs_bytes, int m, int n,
+                        int k, mv_stream_t stream);
 /* `heads` products in one launch: y[:, h*zy .. +n] = x[:, h*zx .. +k] . W_h^T, W_h = w + h*zw ([n,k], row stride ldw). */
 int mv_linear_heads(const void* x, int64_t ldx, int64_t zx, const void* w, int64_t ldw, int64_t zw, float* y,
                     int64_t ldy, int64_t zy, int m, int n, int k, int heads, int f32, mv_stream_t stream);

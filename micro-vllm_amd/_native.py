@@ -68,6 +68,8 @@ PROTOTYPES = {
                                           _I, _I, _I, _I, _I, _I, _F, _I, _P]),
     "mv_gemm_prefill": (_I, [_P, _L, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _P]),
     "mv_gemm_prefill_workspace_bytes": (_Z, [_I, _I, _I]),
+    "mv_linear_any_slab_count": (_I, [_I, _I, _I]),
+    "mv_linear_any_slabs": (_I, [_P, _L, _P, _L, _P, _Z, _I, _I, _I, _P]),
     "mv_linear_slab_count": (_I, [_I, _I, _I]),
     "mv_linear_slabs_workspace_bytes": (_Z, [_I, _I, _I]),
     "mv_linear_slabs": (_I, [_P, _L, _P, _P, _Z, _I, _I, _I, _P, _Z, _P]),

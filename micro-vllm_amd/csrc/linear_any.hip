@@ -204,7 +204,9 @@ __global__ __launch_bounds__(256) void linear_any_bf16_big_kernel(
 // WM x WN accumulator tiles per wave, four waves as 2 x 2: (32 WM) x (32 WN) outputs.  The quarters of k are taken one
 // after the other by the same waves (KG = 1; a second set of accumulators holds the sum so far), or side by side by four
 // groups of four waves (KG = 4): a launch of few tiles is a chain of load latencies (about 0.8 us a step behind HBM),
-// which four groups with four steps ahead each cut by more than four.  The widest tile
+// which four groups with four steps ahead each cut by more than four.  The 64 x 64 tile takes four groups where it has a
+// compute unit to itself: one wave a SIMD leaves its matrix unit idle behind every read (567 rows 1024 x 5120 106.6 -> 94.9 us,
+// 1000 rows 125 -> 96, 1024 x 1024 29.9 -> 25.1; the same sums bit for bit).  The widest tile
 // has 64 accumulators and 32 MFMA times a step to hide a load behind: one step ahead, so that two of its workgroups
 // share a unit (two steps ahead: one workgroup, 97 instead of 128 TFLOP/s).
 // Measured against the 64 x 64 tile of vector fused multiply-adds with k in steps of 16 that was here (outputs x k, us):
@@ -403,14 +405,17 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 // 32000 x 1024 140 -> 36, 16384 x 4096 416 -> 60 (4.5 TB/s); 8 rows 490 -> 24, 109 -> 18, 144 -> 43, 426 -> 73.  The 32 x
 // 32 tile takes 34, 22, 44, 74 for up to 32 rows: it is ahead from 9 rows on where the output is wide (16 rows, 32000 x
 // 1024: 45 against 53), from 17 on everywhere (32 rows, 1024 x 5120: 35 against 40).
-constexpr int kStreamRows = 8, kStreamRowsNarrow = 16, kStreamNarrow = 8192, kStreamAhead = 4;
+constexpr int kStreamRows = 8, kStreamRowsNarrow = 16, kStreamNarrow = 8192, kStreamAhead = 4, kStreamSlice = 8;
 
 __global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __restrict__ x, int64_t ldx,
                                                                 const float* __restrict__ w, int64_t ldw,
                                                                 float* __restrict__ y, int64_t ldy, int M, int N, int K) {
+    // blockIdx.y: a slice of k of its own, [slice][M][N] in y (ldy = N); the wave's share is a quarter of the slice
     __shared__ float part[3][64][5];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4, n0 = blockIdx.x * 16;
-    const int per = ((K + kLfBK - 1) / kLfBK + 3) / 4;
+    const int shares = 4 * gridDim.y, share = 4 * blockIdx.y + wave;
+    const int per = ((K + kLfBK - 1) / kLfBK + shares - 1) / shares;
+    y += (int64_t)blockIdx.y * M * ldy;
     const float* wp = w + (int64_t)min(n0 + r, N - 1) * ldw;
     const float* xp = x + (int64_t)min(r, M - 1) * ldx;
     f32x4_t acc = {0, 0, 0, 0};
@@ -422,7 +427,7 @@ __global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __r
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 // past the quarter nothing is multiplied: its row's start is read instead of another quarter's data
-                const int col = st + u < per ? (wave * per + st + u) * kLfBK + h * 16 + q * 4 : K;
+                const int col = st + u < per ? (share * per + st + u) * kLfBK + h * 16 + q * 4 : K;
                 const bool in = col < K;
                 wv[set][u][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(wp + (in ? col : 0)));
                 xv[set][u][h] = *reinterpret_cast<const f32x4_t*>(xp + (in ? col : 0));
@@ -563,7 +568,8 @@ static int launch_linear_f32_tiles(const float* x, int64_t ldx, const float* w, 
 // Which fp32 form.  Few rows of one product stream the weights (see kStreamRows).  Otherwise the tile by the time the
 // launch takes in it: rounds of tiles over the compute units times what a tile costs a unit, in hundredths of a us as measured,
 // per k-step of 32 and for its start and end - 32 x 32 (four groups, a quarter of the steps each) 200 + 88 a step of a quarter, 64 x
-// 64 200 + 73 by itself and 200 + 59 where several share a unit, 128 x 128 1200 + 228 - so that a launch of few tiles takes
+// 64 where several share a unit 200 + 59, by itself 500 + 56 in four groups and, at a k too short for those, 200 + 73 in one,
+// 128 x 128 1200 + 228 - so that a launch of few tiles takes
 // small ones and a large one the tile that reads its operands least often, at a short k later than at a long one: 1024 rows 4096 x 128
 // in 64 x 64 17.9 us, in 128 x 128 22.3; 1024 rows of 32 heads 128 x 64 55 and 123.  With segments `m` bounds a
 // segment, not the launch: the rows are taken to be spread evenly.
@@ -581,9 +587,12 @@ static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_
     auto rounds = [&](int b) { return (((per + b - 1) / b) * ((n + b - 1) / b) * batch + cus - 1) / cus; };
     const int64_t steps = (k + kLfBK - 1) / kLfBK;
     const int64_t c32 = rounds(32) * (200 + 88 * ((steps + 3) / 4)), c128 = rounds(128) * (1200 + 228 * steps);
-    const int64_t c64 = rounds(64) <= 1 ? 200 + 73 * steps : rounds(64) * (200 + 59 * steps);
+    const bool groups = rounds(64) <= 1 && steps >= 18;
+    const int64_t c64 = groups ? 500 + 56 * steps : rounds(64) <= 1 ? 200 + 73 * steps : rounds(64) * (200 + 59 * steps);
     if (c32 <= c64 && c32 <= c128)
         return launch_linear_f32_tiles<1, 1, 4, 4>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+    if (c64 <= c128 && groups)
+        return launch_linear_f32_tiles<2, 2, 4, 2>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
     if (c64 <= c128)
         return launch_linear_f32_tiles<2, 2, 1, 2>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
     return launch_linear_f32_tiles<4, 4, 1, 1>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
@@ -621,6 +630,34 @@ static int launch_linear_any(const void* x, int64_t ldx, const void* w, int64_t 
         hipLaunchKernelGGL(linear_any_bf16_kernel, grid, dim3(256), 0, s, (const uint16_t*)x, ldx, (const uint16_t*)w,
                            ldw, y, ldy, m, n, k, vx, vw, zx, zw, zy, sg);
     }
+    return check_launch();
+}
+
+// k-slices of a streamed fp32 product whose next kernel adds them: where its strips of sixteen outputs leave compute units
+// idle, as many as there are units for, each wave keeping kStreamSlice steps or more.  3 rows, us whole -> two -> four slices:
+// 1024 x 5120 20.9 -> 14.3 -> 11.5, 1024 x 4096 15.4 -> 10.3 -> 7.6, 2048 x 4096 (128 strips) 16.5 -> 11.6 -> 12.4, 4096 x 16384 (256) 68.5 ->
+// 72.6; 1024 x 1024 (two steps a wave in four) 6.9 -> 6.8 -> 6.6.  The error against 64 bits falls with the slices (6.4e-7 -> 3.2e-7).
+extern "C" int mv_linear_any_slab_count(int m, int n, int k) {
+    using namespace mv;
+    if (m <= 0 || n <= 0 || k <= 0 || m > (n < kStreamNarrow ? kStreamRowsNarrow : kStreamRows) || k % 4) return 1;
+    const int strips = (n + 15) / 16, steps = (k + kLfBK - 1) / kLfBK;
+    int ks = 1;
+    while (2 * ks * strips <= num_cus() && steps >= 2 * ks * 4 * kStreamSlice) ks *= 2;
+    return ks;
+}
+
+extern "C" int mv_linear_any_slabs(const float* x, int64_t ldx, const float* w, int64_t ldw, float* slabs, size_t slabs_bytes,
+                                   int m, int n, int k, mv_stream_t stream) {
+    using namespace mv;
+    if (m < 0 || n <= 0 || k <= 0) return MV_ERR_INVALID_ARG;
+    if (m == 0) return MV_OK;
+    if (!x || !w || !slabs || ldx < k || ldw < k) return MV_ERR_INVALID_ARG;
+    const int ks = mv_linear_any_slab_count(m, n, k);
+    if (slabs_bytes < (size_t)ks * m * n * sizeof(float)) return MV_ERR_WORKSPACE;
+    if (ks == 1) return mv_linear_any(x, ldx, w, ldw, slabs, n, m, n, k, 1, stream);
+    if (ldx % 4 || ldw % 4 || !aligned16(x) || !aligned16(w)) return MV_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(linear_stream_f32_kernel, dim3((n + 15) / 16, ks), dim3(256), 0, (hipStream_t)stream, x, ldx, w, ldw, slabs,
+                       n, m, n, k);
     return check_launch();
 }
 

@@ -80,7 +80,16 @@ class AnyLinear:
         y - for `postnorm_residual` and `add_rmsnorm`, which add them.  `take(rows, cols)` gives the fp32 buffer."""
         m = x.shape[0]
         if self.tiles is None or m == 0:
-            return self(x, take(m, self.n)).unsqueeze(0)
+            ks = nv.lib().mv_linear_any_slab_count(m, self.n, self.k) if self.f32 and m else 1
+            if ks == 1 or x.stride(0) % 4 or x.data_ptr() % 16:
+                return self(x, take(m, self.n)).unsqueeze(0)
+            assert x.is_cuda and x.dim() == 2 and x.shape[1] == self.k and x.stride(1) == 1 and x.dtype == torch.float32
+            out = take(ks * m, self.n)
+            assert out.dtype == torch.float32 and out.is_contiguous() and out.shape == (ks * m, self.n)
+            nv.check("mv_linear_any_slabs", nv.lib().mv_linear_any_slabs(
+                x.data_ptr(), _ld(x), self.w.data_ptr(), self.k, out.data_ptr(), out.numel() * 4, m, self.n, self.k,
+                nv.stream_ptr()))
+            return out.view(ks, m, self.n)
         assert x.is_cuda and x.dim() == 2 and x.shape[1] == self.k and x.stride(1) == 1 and x.dtype == torch.bfloat16
         L = nv.lib()
         ks = L.mv_linear_slab_count(m, self.n, self.k)

@@ -66,3 +66,41 @@ def test_norms_add_the_slices_in_order(mv, rows, n, ks, act):
         # the square sum's error grows with the chain of additions, far below one bf16 unit; fp32 results lie within 2^-20
         tol = 2 ** -8 if act == torch.bfloat16 else 2 ** -18
         assert ((res[1].double() - normed).abs() <= tol * normed.abs() + 1e-6).all()
+
+
+# streamed slices of fp32 weights: whole, two, four, eight; k that is no multiple of a slice's share and one that ends inside a
+# step; rows up to the limit of the streamed form and past it
+@pytest.mark.parametrize("m,n,k", [(1, 1024, 5120), (3, 1024, 1024), (8, 1024, 2048), (16, 512, 4096), (16, 2048, 4100), (2, 40, 8192),
+                                   (1, 16, 12), (3, 1030, 5132), (17, 1024, 5120), (4, 9472, 2048)])
+def test_streamed_fp32_slices_add_up_to_the_product(mv, m, n, k):
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(DEV)
+    lin = AnyLinear((torch.randn(n, k, generator=g) / k ** 0.5).to(DEV))
+    got = lin.slabs(x, _take)
+    ks = nv.lib().mv_linear_any_slab_count(m, n, k)
+    assert got.shape == (ks, m, n) and (ks > 1) == ((m, n, k) in ((1, 1024, 5120), (8, 1024, 2048), (16, 512, 4096), (16, 2048, 4100),
+                                                                 (2, 40, 8192), (3, 1030, 5132)))
+    want = x.double() @ lin.w.double().t()
+    tol = k ** 0.5 * 2 ** -24 * 8      # as above: fp32 sums of products of order 1 / sqrt(k)
+    assert (got.double().sum(0) - want).abs().max().item() <= tol
+    # an operand that is not aligned goes whole, as it did
+    wide = torch.randn(m, k + 1, generator=g).to(DEV)[:, 1:]
+    assert lin.slabs(wide, _take).shape == (1, m, n)
+
+
+# 64 x 64 tiles in four groups: up to one for every compute unit, k from 18 steps of 32 on and one short of it, k that ends
+# inside a step and inside a group of four, rows and columns that end inside a tile
+@pytest.mark.parametrize("m,n,k", [(567, 1024, 5120), (1000, 1024, 576), (1000, 1024, 544), (641, 1601, 1030), (1000, 1000, 1092),
+                                   (70, 9480, 1024), (1024, 1024, 4099)])
+def test_fp32_tiles_by_themselves_on_a_unit(mv, m, n, k):
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(DEV)
+    lin = AnyLinear((torch.randn(n, k, generator=g) / k ** 0.5).to(DEV))
+    got = lin(x, torch.full((m, n), float("nan"), device=DEV))
+    want = x.double() @ lin.w.double().t()
+    assert (got.double() - want).abs().max().item() <= k ** 0.5 * 2 ** -24 * 8
