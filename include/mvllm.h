@@ -222,6 +222,13 @@ int mv_linear_slab_count(int m, int n, int k);
 size_t mv_linear_slabs_workspace_bytes(int m, int n, int k);
 int mv_linear_slabs(const void* x, int64_t ldx, const void* w_tiles, float* slabs, size_t slabs_bytes, int m, int n, int k,
                     void* workspace, size_t workspace_bytes, mv_stream_t stream);
+/* y [m, .] bf16 = an activation of x . W^T, any m, n % 16 == 0, k % 64 == 0, nothing rounded in front of the result:
+ * kind 1: y [m, n] = max(v, 0)^2.  kind 2: W in wave tiles with up and gate interleaved by 8 (mv_interleave_rows8), y [m, n / 2] =
+ * g' sigmoid(slope g') (u' + 1), g' = min(gate, limit), u' = clamp(up, -limit, limit).  workspace: of
+ * mv_linear_act_workspace_bytes; past 64 rows as for mv_gemm_prefill_ws (a buffer of its own, zero-filled when allocated). */
+size_t mv_linear_act_workspace_bytes(int m, int n, int k);
+int mv_linear_act(const void* x, int64_t ldx, const void* w_tiles, void* y, int64_t ldy, int m, int n, int k, int kind,
+                  float limit, float slope, void* workspace, size_t workspace_bytes, mv_stream_t stream);
 /* Which form a call of that shape takes on the current device (for tests and tools; no counterpart
  * in the reference): 0 = 128 x 256 tiles, two workgroups per CU, weights straight into registers;
  * 1 = 256 x 256 tiles, one workgroup per CU, both operands through LDS (taken when its tiles fill

@@ -167,6 +167,11 @@ class RaggedRunner:
         self.weight_bytes += lin.nbytes
         return lin
 
+    def _gated(self, gate, up):
+        lin = ops.GatedLinear(self._act(gate), self._act(up), wave_tiles=self.wave_tiles)
+        self.weight_bytes += lin.nbytes
+        return lin
+
     def _dyt_norm(self, name):
         g = self.model.get
         return (self._small(g(name)), self._small(g(name + ".b")), self._small(g(name + ".alpha")).reshape(1))
@@ -365,7 +370,7 @@ class RaggedRunner:
         mlp = layer.get("mlp")
         if mlp:
             w.update(norm2=self._small(g(p + "norm2")), norm2b=self._small(g(p + "norm2b")),
-                     gate_up=self._linear(g(p + "mlp.gate"), g(p + "mlp.up")), down=self._linear(g(p + "mlp.down")))
+                     gate_up=self._gated(g(p + "mlp.gate"), g(p + "mlp.up")), down=self._linear(g(p + "mlp.down")))
         return w
 
     def _prepare_sizizen(self, i: int, layer: dict) -> dict:
@@ -630,9 +635,7 @@ class RaggedRunner:
                     ops.postnorm_residual(y1, w["norm1"], cfg.eps, x, h, y2=y2, s1=float(m["left_scale"]),
                                           s2=float(m["right_scale"]))
                 if layer.get("mlp"):
-                    up = w["up"](h, self._f32buf(T, w["up"].n))
-                    act = self._actbuf(T, up.shape[1])
-                    ops.relu_squared(up, act)
+                    act = ops.linear_relu_squared(h, w["up"], self._actbuf(T, w["up"].n), self._f32buf)
                     ops.postnorm_residual(w["down"].slabs(act, self._f32buf), w["norm2"], cfg.eps, x, h)
                 if residuals is not None:
                     residuals.append(x.clone())
@@ -846,8 +849,7 @@ class RaggedRunner:
                 ops.postnorm_residual(y, w["norm1b"], eps, x, h, bias=bias, mult=mult, next_w=w["norm2"])
                 ff = int(mlp["ff"])
                 act = self._actbuf(T, ff)
-                ops.gated_act(w["gate_up"](h, self._f32buf(T, 2 * ff)), act, ops.GATE_CLAMPED, float(mlp["limit"]),
-                              dugazen.GATE_SLOPE)
+                w["gate_up"](h, act, self._f32buf, float(mlp["limit"]), dugazen.GATE_SLOPE)
                 y, bias = w["down"].slabs(act, self._f32buf), None
                 ops.postnorm_residual(y, w["norm2b"], eps, x, out, mult=mult, next_w=nxt)
             else:
@@ -961,7 +963,7 @@ class RaggedRunner:
             return down, place, wts, None
         sf = int(mlp["shared"]["ff"])
         s_act = self._actbuf(T, sf)
-        ops.relu_squared(w["s_up"](h, self._f32buf(T, sf)), s_act)
+        ops.linear_relu_squared(h, w["s_up"], s_act, self._f32buf)
         return down, place, wts, w["s_down"](s_act, self._f32buf(T, self.width))
 
     # ------------------------------------------------------------------ Fagunex layers

@@ -114,9 +114,19 @@ int num_cus();  // compute units of the current device (cached)
 // `done` is the caller's per-kernel record of what each device was last configured for.
 struct LdsOptIn { size_t bytes[64] = {}; };
 int ensure_dynamic_lds(const void* kernel, size_t lds, LdsOptIn& done);
+// What a projection of fp32 accumulators may apply in its epilogue, before the only rounding: kind 1 max(v, 0)^2; kind 2 the
+// clamped gate of gated_act_f over rows of W with up and gate interleaved by 8 (MV_GEMM_SWIGLU).  0: nothing
+struct GemmAct {
+    int kind;
+    float limit, slope;
+};
 // wgemm.hip: adds k-slices partial[ks][m][n] (fp32) in order and applies the projection epilogue
 int launch_wgemm_finalize(float* partial, int ksplit, int m, int n, int flags, const uint16_t* bias,
-                          const uint16_t* residual, int64_t ld_res, void* y, int64_t ldy, hipStream_t s);
+                          const uint16_t* residual, int64_t ld_res, void* y, int64_t ldy, hipStream_t s,
+                          GemmAct act);
+// wgemm.hip: a projection of up to 64 rows with `act` in its epilogue
+int launch_wgemm_act(const void* x, int64_t ldx, const void* w_tiles, void* y, int64_t ldy, int m, int n, int k, void* workspace,
+                     size_t workspace_bytes, GemmAct act, mv_stream_t stream);
 // What may follow a projection: y = bf16(sum) + bias + residual and out = rmsnorm(y) * ln_w, the variance that of the rounded
 // or the unrounded y.  `done` says that the projection's own reduction did it, in place of the call's own epilogue.
 struct PostNorm {
@@ -142,7 +152,8 @@ int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const 
 // gemm_prefill.hip: mv_gemm_prefill_ws, whose reduction of k-slices (where it has one) also does `norm`
 int gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
                      int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int flags, void* workspace,
-                     size_t workspace_bytes, PostNorm* norm, mv_stream_t stream, bool keep_slices = false);
+                     size_t workspace_bytes, PostNorm* norm, mv_stream_t stream, bool keep_slices = false,
+                     GemmAct act = {0, 0.f, 0.f});
 // wgemm.hip: k-slices of a projection of up to 64 rows whose slices the next kernel adds, and the projection
 int wgemm_slices(int m, int n, int k);
 int launch_wgemm_slices(const void* x, int64_t ldx, const void* w_tiles, float* slabs, size_t slabs_bytes, int m, int n, int k,

@@ -65,6 +65,7 @@ struct PGemmArgs {
     // counters through which the parts of such a tile count themselves in (zero between launches)
     float* cut_ws;
     unsigned* cut_count;
+    GemmAct act;      // kinds 1 and 2: the kernels' ACT
 };
 
 #ifdef MV_GEMM_STAMP
@@ -133,7 +134,17 @@ __device__ __forceinline__ float silu_mul_rounded_quick(float gate_acc, float up
     const float sig = __builtin_amdgcn_rcpf(1.0f + e);
     return (g * sig) * u;
 }
-template <int NT, int MT>
+// the clamped gate in the same terms (gated_act_f's kind 2, nothing rounded before the result)
+__device__ __forceinline__ float gated_clamped_quick(float gate, float up, const GemmAct& act) {
+    const float g = fminf(gate, act.limit), u = fminf(fmaxf(up, -act.limit), act.limit);
+    const float e = __builtin_amdgcn_exp2f(g * (act.slope * -1.44269504088896341f));
+    return (g * __builtin_amdgcn_rcpf(1.0f + e)) * (u + 1.0f);
+}
+// ACT: an activation of the unrounded sums (GemmAct) in place of the rounded ones' bias and residual - kernels of their own, since
+// the plain forms' registers are full.  Against fp32 sums in memory and a launch that reads them: max(v, 0)^2 of 2048 x 16384
+// 33.9 us and of one row 4.6, the clamped gate of 1400 x 8192 18.7 and of 8 rows 4.6 are gone, and the products in front of them
+// write a half or a quarter of the bytes (1400 x 16384 x 2048 93 -> 86 us).
+template <int NT, int MT, int ACT = 0>
 __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_t (&acc)[NT][MT], int nt0,
                                                 int m0, int ks, int r, int q, const unsigned char* lower = nullptr,
                                                 int nlower = 0) {
@@ -187,8 +198,12 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
                 const f32x4_t c = sum(i, t);
                 const auto s0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(c[0]), __float_as_uint(c[2]), false, false);
                 const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(c[1]), __float_as_uint(c[3]), false, false);
-                o[i] = pack_bf16x2(silu_mul_rounded_quick(__uint_as_float(s0[1]), __uint_as_float(s0[0])),
-                                   silu_mul_rounded_quick(__uint_as_float(s1[1]), __uint_as_float(s1[0])));
+                if constexpr (ACT == 2)
+                    o[i] = pack_bf16x2(gated_clamped_quick(__uint_as_float(s0[1]), __uint_as_float(s0[0]), a.act),
+                                       gated_clamped_quick(__uint_as_float(s1[1]), __uint_as_float(s1[0]), a.act));
+                else
+                    o[i] = pack_bf16x2(silu_mul_rounded_quick(__uint_as_float(s0[1]), __uint_as_float(s0[0])),
+                                       silu_mul_rounded_quick(__uint_as_float(s1[1]), __uint_as_float(s1[0])));
             }
 #ifdef MV_EXP_EPI_NO_WRITE
             asm volatile("" : : "v"(o[0]), "v"(o[1]), "v"(o[2]), "v"(o[3]));   // timing experiment only
@@ -228,6 +243,11 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+            if constexpr (ACT == 1) {
+                v[j] = fmaxf(c[j], 0.f);
+                v[j] *= v[j];
+                continue;
+            }
             float tv = round_bf16(c[j]);
             if (a.bias) tv = round_bf16(tv + bf16_bits_to_f32(bias[j]));
             if (a.residual) tv = round_bf16(tv + bf16_bits_to_f32(res[j]));
@@ -278,7 +298,7 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
 // workgroup to a unit, whose waves have the registers to themselves; with two k-tiles ahead a stage of 64 k takes 1.1 us
 // there.  The 64-row tile halves what a wave multiplies per stage and doubles the workgroups, and NT, the n-tiles of a wave,
 // doubles or quadruples them again (tile64_strips).  Sums do not depend on any of it.
-template <int MT, int RING, int BUFS, int NT = kPNT>
+template <int MT, int RING, int BUFS, int NT = kPNT, int ACT = 0>
 __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefill_kernel(PGemmArgs a) {
     constexpr int kStage = MT * 16 * kPK * 2, XP = MT / 2;   // bytes of a stage of x, pieces of it a wave requests
     constexpr int kPeriod = RING == 3 ? 3 : RING / 2;     // stages after which slots and buffers repeat
@@ -451,7 +471,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     if (kPeriod == 4 && s + 2 < nstage) stage(std::integral_constant<int, 2>{}, left, s + 2);
     wait_vmcnt<0>();     // no request into LDS outlives the workgroup
 
-    store_wave_tile<NT, MT>(a, acc, nt0, m0, ks, r, q);
+    store_wave_tile<NT, MT, ACT>(a, acc, nt0, m0, ks, r, q);
 }
 
 
@@ -514,7 +534,7 @@ __host__ __device__ inline int wide_cut_parts(int rest, int wgs, int nkt) {
 }
 
 // One wave's share of a tile: NT n-tiles from strip `wcol` of a block that is `width` strips wide.
-template <int NT>
+template <int NT, int ACT>
 __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds, int wid, int wm, int wcol,
                                           int width) {
     unsigned char* const xring = lds;
@@ -804,7 +824,7 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
                 nlower = cur.parts - 1;
             }
             if (cur.ntb + wcol < a.nt)
-                store_wave_tile<NT, kPMT>(a, acc, cur.ntb + wcol, cur.m0 + wm * 128, cur.ks, r, q, lower, nlower);
+                store_wave_tile<NT, kPMT, ACT>(a, acc, cur.ntb + wcol, cur.m0 + wm * 128, cur.ks, r, q, lower, nlower);
         }
 #endif
         MV_WSTAMP(g0 + nkt + 1);
@@ -828,22 +848,22 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
 // column, the two rows) always have NTA + NTB n-tiles between them: the matrix pipes stay evenly
 // loaded at the odd width too.  Both kinds of wave run the same copies, waits and barriers per
 // k-tile; only the number of fragments and MFMAs differs.
-template <int NTA, int NTB>
+template <int NTA, int NTB, int ACT = 0>
 __global__ __launch_bounds__(512, 1) void gemm_prefill_wide_kernel(PGemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wid & 3, wm = wid >> 2;
     constexpr int kWidth = 2 * (NTA + NTB);
     if constexpr (NTA == NTB) {
-        wide_tile<NTA>(a, lds, wid, wm, wn * NTA, kWidth);
+        wide_tile<NTA, ACT>(a, lds, wid, wm, wn * NTA, kWidth);
     } else {
         // row 0: A B A B, row 1: B A B A
         const int first = wm ? NTB : NTA;
         const int wcol = (wn >> 1) * (NTA + NTB) + ((wn & 1) ? first : 0);
         if (((wn + wm) & 1) == 0)
-            wide_tile<NTA>(a, lds, wid, wm, wcol, kWidth);
+            wide_tile<NTA, ACT>(a, lds, wid, wm, wcol, kWidth);
         else
-            wide_tile<NTB>(a, lds, wid, wm, wcol, kWidth);
+            wide_tile<NTB, ACT>(a, lds, wid, wm, wcol, kWidth);
     }
 }
 
@@ -1054,6 +1074,30 @@ extern "C" int mv_gemm_prefill_ws(const void* x, int64_t ldx, const void* w_tile
                                 nullptr, stream);
 }
 
+namespace mv {
+template <int ACT>
+static int launch_wide(const PGemmArgs& a, int strips, unsigned grid, hipStream_t s) {
+    static LdsOptIn lds_done[3];
+    const auto kernel = strips == 12   ? gemm_prefill_wide_kernel<3, 3, ACT>
+                        : strips == 14 ? gemm_prefill_wide_kernel<4, 3, ACT>
+                                       : gemm_prefill_wide_kernel<4, 4, ACT>;
+    if (const int rc = ensure_dynamic_lds((const void*)kernel, kWLds, lds_done[(strips - 12) / 2])) return rc;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), kWLds, s, a);
+    return check_launch();
+}
+// `strips`: of a wave of the 64-row tiles, 0 for the 128-row ones, which are deep where a slice is long
+template <int ACT>
+static int launch_tiles(const PGemmArgs& a, int strips, bool deep, unsigned grid, hipStream_t s) {
+    const auto kernel = strips == 1   ? gemm_prefill_kernel<4, 8, 4, 1, ACT>
+                        : strips == 2 ? gemm_prefill_kernel<4, 8, 4, 2, ACT>
+                        : strips == 4 ? gemm_prefill_kernel<4, 8, 4, 4, ACT>
+                        : deep        ? gemm_prefill_kernel<8, 8, 4, 4, ACT>
+                                      : gemm_prefill_kernel<8, 3, 3, 4, ACT>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, a);
+    return check_launch();
+}
+}  // namespace mv
+
 extern "C" int mv_linear_slab_count(int m, int n, int k) {
     using namespace mv;
     if (m <= 0 || n <= 0 || k <= 0 || (n % 16) != 0 || (k % 64) != 0) return 0;
@@ -1063,6 +1107,22 @@ extern "C" int mv_linear_slab_count(int m, int n, int k) {
 extern "C" size_t mv_linear_slabs_workspace_bytes(int m, int n, int k) {
     // (the slices themselves go to the caller's buffer: left are the cut tiles of a product that is not sliced)
     return m > 64 && mv_linear_slab_count(m, n, k) == 1 ? mv_gemm_prefill_workspace_bytes(m, n, k) : 0;
+}
+
+extern "C" size_t mv_linear_act_workspace_bytes(int m, int n, int k) {
+    return m <= 64 ? mv_wgemm_workspace_bytes(m, n, k) : mv_gemm_prefill_workspace_bytes(m, n, k);
+}
+
+extern "C" int mv_linear_act(const void* x, int64_t ldx, const void* w_tiles, void* y, int64_t ldy, int m, int n, int k,
+                             int kind, float limit, float slope, void* workspace, size_t workspace_bytes, mv_stream_t stream) {
+    if (m == 0 && n > 0 && k > 0) return MV_OK;
+    if (kind != 1 && kind != 2) return MV_ERR_INVALID_ARG;
+    if (n <= 0 || k <= 0 || m < 0) return MV_ERR_INVALID_ARG;
+    if ((n % 16) != 0 || (k % 64) != 0) return MV_ERR_UNSUPPORTED;
+    const mv::GemmAct act = {kind, limit, slope};
+    if (m <= 64) return mv::launch_wgemm_act(x, ldx, w_tiles, y, ldy, m, n, k, workspace, workspace_bytes, act, stream);
+    return mv::gemm_prefill_run(x, ldx, w_tiles, nullptr, nullptr, 0, y, ldy, m, n, k, kind == 2 ? MV_GEMM_SWIGLU : 0, workspace,
+                                workspace_bytes, nullptr, stream, false, act);
 }
 
 extern "C" int mv_linear_slabs(const void* x, int64_t ldx, const void* w_tiles, float* slabs, size_t slabs_bytes, int m, int n,
@@ -1079,7 +1139,7 @@ extern "C" int mv_linear_slabs(const void* x, int64_t ldx, const void* w_tiles, 
 
 int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
                          int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int flags, void* workspace,
-                         size_t workspace_bytes, PostNorm* norm, mv_stream_t stream, bool keep_slices) {
+                         size_t workspace_bytes, PostNorm* norm, mv_stream_t stream, bool keep_slices, GemmAct act) {
     if (norm) norm->done = false;
     if (m == 0) return MV_OK;
     if (!x || !w_tiles || !y || m < 0 || n <= 0 || k <= 0) return MV_ERR_INVALID_ARG;
@@ -1117,6 +1177,8 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     a.partial = nullptr;
     a.cut_ws = nullptr;
     a.cut_count = nullptr;
+    a.act = act;
+    // (what is cut is rounded behind the slices: their kernels have no epilogue)
     // the workspace: kWCountBytes of counters, then the data
     void* const data = workspace && workspace_bytes > kWCountBytes && aligned16(workspace)
                            ? (void*)((char*)workspace + kWCountBytes) : nullptr;
@@ -1141,7 +1203,7 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     // Up to 64 rows a tile of 128 is mostly padding, and its slices are written out and added up by a second launch.  The
     // single-token projections' kernel walks the same slices one to a wave and adds them in the workgroup, same sums in
     // the same order (the rule and what it measured: wgemm_ordered_takes).
-    if (!wide && !keep_slices && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit, tile64_strips(m, a.nt, a.ksplit)))
+    if (!wide && !keep_slices && !act.kind && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit, tile64_strips(m, a.nt, a.ksplit)))
         return launch_wgemm_ordered(x, ldx, w_tiles, bias, residual, ld_res, y, ldy, m, n, k, a.ksplit, flags, norm,
                                     (hipStream_t)stream);
     auto reduce = [&] {
@@ -1149,17 +1211,11 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
         if (norm && !sw && !of32 && wgemm_finalize_norm_takes(n))
             return launch_wgemm_finalize_norm(a.partial, a.ksplit, m, n, bias, norm, (hipStream_t)stream);
         return launch_wgemm_finalize(a.partial, a.ksplit, m, n, flags, a.bias, a.residual, ld_res, y, ldy,
-                                     (hipStream_t)stream);
+                                     (hipStream_t)stream, act);
     };
     a.ktps = a.kt / a.ksplit;
     if (wide) {
-        static LdsOptIn lds_done[3];
         const int strips = a.ksplit == 1 ? plan.strips : 16;
-        const void* kernel = strips == 12   ? (const void*)gemm_prefill_wide_kernel<3, 3>
-                             : strips == 14 ? (const void*)gemm_prefill_wide_kernel<4, 3>
-                                            : (const void*)gemm_prefill_wide_kernel<4, 4>;
-        int rc = ensure_dynamic_lds(kernel, kWLds, lds_done[(strips - 12) / 2]);
-        if (rc != MV_OK) return rc;
         a.mblocks = (m + kWM - 1) / kWM;
         a.nblocks = (a.nt + strips - 1) / strips;
         a.nb_per_xcd = (a.nblocks + 7) / 8;
@@ -1180,13 +1236,10 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
             a.cut_ws = (float*)data;
             a.cut_count = (unsigned*)workspace;
         }
-        if (strips == 12)
-            hipLaunchKernelGGL((gemm_prefill_wide_kernel<3, 3>), dim3((unsigned)wgrid), dim3(512), kWLds, (hipStream_t)stream, a);
-        else if (strips == 14)
-            hipLaunchKernelGGL((gemm_prefill_wide_kernel<4, 3>), dim3((unsigned)wgrid), dim3(512), kWLds, (hipStream_t)stream, a);
-        else
-            hipLaunchKernelGGL((gemm_prefill_wide_kernel<4, 4>), dim3((unsigned)wgrid), dim3(512), kWLds, (hipStream_t)stream, a);
-        rc = check_launch();
+        const int kind = a.ksplit == 1 ? act.kind : 0;
+        const int rc = kind == 0   ? launch_wide<0>(a, strips, (unsigned)wgrid, (hipStream_t)stream)
+                       : kind == 1 ? launch_wide<1>(a, strips, (unsigned)wgrid, (hipStream_t)stream)
+                                   : launch_wide<2>(a, strips, (unsigned)wgrid, (hipStream_t)stream);
         if (rc != MV_OK || a.ksplit == 1) return rc;
         return reduce();
     }
@@ -1198,20 +1251,18 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     // two slices 54.4 -> 49.7 in the deep form (64-row tiles in two rounds: 61.3), 700 x 2048 x 5632 in four (22 stages) 36.8 -> 35.6;
     // but 192 x 6144 x 2048 in four (8 stages) 24.8, deep 25.4, and 96 x 7168 x 8192 in eight (16) 34.1, deep 35.7.
     const int strips = tile64_strips(m, a.nt, a.ksplit);
+    long tiles = grid;
     if (strips) {
         a.mblocks = (m + 63) / 64;
         a.nblocks = (a.nt + 4 * strips - 1) / (4 * strips);
         a.nb_per_xcd = (a.nblocks + 7) / 8;
-        const dim3 grid64((unsigned)(8L * a.nb_per_xcd * a.mblocks * a.ksplit));
-        if (strips == 4) hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 4>), grid64, dim3(256), 0, (hipStream_t)stream, a);
-        else if (strips == 2) hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 2>), grid64, dim3(256), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL((gemm_prefill_kernel<4, 8, 4, 1>), grid64, dim3(256), 0, (hipStream_t)stream, a);
-    } else if (grid <= num_cus() && a.ktps >= 40) {
-        hipLaunchKernelGGL((gemm_prefill_kernel<8, 8, 4>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
-    } else {
-        hipLaunchKernelGGL((gemm_prefill_kernel<8, 3, 3>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a);
+        tiles = 8L * a.nb_per_xcd * a.mblocks * a.ksplit;
     }
-    int rc = check_launch();
+    const bool deep = grid <= num_cus() && a.ktps >= 40;
+    const int kind = a.ksplit == 1 ? act.kind : 0;
+    const int rc = kind == 0   ? launch_tiles<0>(a, strips, deep, (unsigned)tiles, (hipStream_t)stream)
+                   : kind == 1 ? launch_tiles<1>(a, strips, deep, (unsigned)tiles, (hipStream_t)stream)
+                               : launch_tiles<2>(a, strips, deep, (unsigned)tiles, (hipStream_t)stream);
     if (rc != MV_OK || a.ksplit == 1) return rc;
     return reduce();
 }

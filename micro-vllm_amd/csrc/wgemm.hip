@@ -73,6 +73,7 @@ struct GemmArgs {
     int64_t ld_post;
     float post_eps;
     int post_var_from_rounded;  // variance from y as stored (bf16) instead of the unrounded t + residual
+    GemmAct act;
 #ifdef MV_WGEMM_STAMP
     int stamp_slot;             // which of the 32 stamp records this launch writes
 #endif
@@ -99,10 +100,19 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 
 // Final value of one output element from its fp32 accumulator.
 __device__ __forceinline__ float epilogue_value(const GemmArgs& a, float acc, int m, int n) {
+    if (a.act.kind == 1) {   // uniform
+        const float v = fmaxf(acc, 0.f);
+        return v * v;
+    }
     float t = round_bf16(acc);
     if (a.bias) t = round_bf16(t + bf16_bits_to_f32(a.bias[n]));
     if (a.residual) t = round_bf16(t + bf16_bits_to_f32(a.residual[(int64_t)m * a.ld_res + n]));
     return t;
+}
+
+// ... and of a pair of rows, up and gate
+__device__ __forceinline__ float epilogue_gated(const GemmArgs& a, float gate, float up) {
+    return a.act.kind == 2 ? gated_act_f(gate, up, 2, a.act.limit, a.act.slope) : silu_mul_rounded(gate, up);
 }
 
 // ------------------------------------------------------------ M <= 4: dot form
@@ -419,7 +429,7 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 #pragma unroll
                     for (int w8 = 0; w8 < GW; ++w8) g += red[(w8 * M + m) * 16 + rr + 8];
                     reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + cur.nt * 8 + rr] =
-                        (uint16_t)f32_to_bf16_bits(silu_mul_rounded(g, s));
+                        (uint16_t)f32_to_bf16_bits(epilogue_gated(a, g, s));
                 }
             } else {
                 reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + n] =
@@ -583,8 +593,8 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
                     if (qq < 2) {  // rows 0..7 = up; their gates sit 8 rows (32 lanes) further
                         const f32x4_t gt = sum_at(l + 32);
                         uint2 o;
-                        o.x = pack_bf16x2(silu_mul_rounded(gt[0], s[0]), silu_mul_rounded(gt[1], s[1]));
-                        o.y = pack_bf16x2(silu_mul_rounded(gt[2], s[2]), silu_mul_rounded(gt[3], s[3]));
+                        o.x = pack_bf16x2(epilogue_gated(a, gt[0], s[0]), epilogue_gated(a, gt[1], s[1]));
+                        o.y = pack_bf16x2(epilogue_gated(a, gt[2], s[2]), epilogue_gated(a, gt[3], s[3]));
                         *reinterpret_cast<uint2*>(&reinterpret_cast<uint16_t*>(
                             a.y)[(int64_t)m * a.ldy + nt * 8 + qq * 4]) = o;
                     }
@@ -675,7 +685,7 @@ __global__ __launch_bounds__(256) void wgemm_finalize_kernel(GemmArgs a) {
             const int nu = (c >> 3) * 16 + (c & 7);
             const float up = slab_sum(nu), gate = slab_sum(nu + 8);
             reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + c] =
-                (uint16_t)f32_to_bf16_bits(silu_mul_rounded(gate, up));
+                (uint16_t)f32_to_bf16_bits(epilogue_gated(a, gate, up));
         } else if (a.flags & MV_GEMM_OUT_F32) {
             reinterpret_cast<float*>(a.y)[(int64_t)m * a.ldy + c] = slab_sum(c);
         } else {
@@ -822,8 +832,9 @@ static int launch_finalize_norm(const GemmArgs& a, hipStream_t s) {
 // The slab reduction for other kernels of the library that split k (the prefill GEMM): same
 // layout partial[ks][m][n], same epilogues.
 int launch_wgemm_finalize(float* partial, int ksplit, int m, int n, int flags, const uint16_t* bias,
-                          const uint16_t* residual, int64_t ld_res, void* y, int64_t ldy, hipStream_t s) {
+                          const uint16_t* residual, int64_t ld_res, void* y, int64_t ldy, hipStream_t s, GemmAct act) {
     GemmArgs a = {};
+    a.act = act;
     a.partial = partial;
     a.ksplit = ksplit;
     a.m = m;
@@ -836,7 +847,7 @@ int launch_wgemm_finalize(float* partial, int ksplit, int m, int n, int flags, c
     a.ldy = ldy;
     const int ncols = (flags & MV_GEMM_SWIGLU) ? n / 2 : n;
     const int most = num_cus() * 8;
-    const bool vec8 = !(flags & (MV_GEMM_SWIGLU | MV_GEMM_OUT_F32)) && ksplit <= kMaxKsplit && (n % 8) == 0 &&
+    const bool vec8 = !act.kind && !(flags & (MV_GEMM_SWIGLU | MV_GEMM_OUT_F32)) && ksplit <= kMaxKsplit && (n % 8) == 0 &&
                       (ldy % 8) == 0 && aligned16(y) && aligned16(partial) && (!bias || aligned16(bias)) &&
                       (!residual || (aligned16(residual) && (ld_res % 8) == 0)) && (int64_t)m * n >= (1 << 16);
     if (vec8) {
@@ -1130,7 +1141,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
                       int k, void* workspace, size_t workspace_bytes, int flags,
                       mv_stream_t stream, const void* post_ln_w = nullptr, float post_eps = 0.f,
                       void* post_out = nullptr, int64_t ld_post = 0, int post_var_from_rounded = 0,
-                      int slices = 0) {
+                      int slices = 0, GemmAct act = {0, 0.f, 0.f}) {
     const bool slabs_only = (flags & MV_GEMM_SLABS) != 0;
     if (!x || !w_tiles || (!y && !slabs_only) || m <= 0 || n <= 0 || k <= 0) return MV_ERR_INVALID_ARG;
     if (m > 64 || (n % 16) != 0 || (k % 32) != 0) return MV_ERR_UNSUPPORTED;
@@ -1169,6 +1180,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
     a.k = k;
     a.nt = n / 16;
     a.kt = k / 32;
+    a.act = act;
     a.prologue = prologue;
     a.var_from_rounded = var_from_rounded;
     a.add_r = (const uint16_t*)add_r;
@@ -1268,6 +1280,12 @@ int launch_wgemm_slices(const void* x, int64_t ldx, const void* w_tiles, float* 
                         mv_stream_t stream) {
     return wgemm_impl(x, ldx, nullptr, 0, nullptr, 0.f, nullptr, 0, kProNone, 0, w_tiles, nullptr, nullptr, 0, nullptr, 0, m, n,
                       k, slabs, slabs_bytes, MV_GEMM_SLABS, stream, nullptr, 0.f, nullptr, 0, 0, wgemm_slices(m, n, k));
+}
+
+int launch_wgemm_act(const void* x, int64_t ldx, const void* w_tiles, void* y, int64_t ldy, int m, int n, int k, void* workspace,
+                     size_t workspace_bytes, GemmAct act, mv_stream_t stream) {
+    return wgemm_impl(x, ldx, nullptr, 0, nullptr, 0.f, nullptr, 0, kProNone, 0, w_tiles, nullptr, nullptr, 0, y, ldy, m, n, k,
+                      workspace, workspace_bytes, act.kind == 2 ? MV_GEMM_SWIGLU : 0, stream, nullptr, 0.f, nullptr, 0, 0, 0, act);
 }
 
 }  // namespace mv

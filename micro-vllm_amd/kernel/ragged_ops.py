@@ -103,6 +103,52 @@ class AnyLinear:
         return out.view(ks, m, self.n)
 
 
+def _linear_act(x, tiles, out, kind, limit=0.0, slope=1.0):
+    m, k = x.shape
+    assert x.is_cuda and x.dtype == torch.bfloat16 and x.stride(1) == 1 and k == tiles.k
+    assert out.shape == (m, tiles.out_features) and out.dtype == torch.bfloat16 and out.stride(1) == 1
+    if m == 0:
+        return out
+    L = nv.lib()
+    ws = nv.stream_workspace("wgemm" if m <= 64 else "gemm_prefill", x.device, L.mv_linear_act_workspace_bytes(m, tiles.n, k))
+    nv.check("mv_linear_act", L.mv_linear_act(
+        x.data_ptr(), _ld(x), tiles.tiles.data_ptr(), out.data_ptr(), _ld(out), m, tiles.n, k, kind, float(limit), float(slope),
+        nv.ptr(ws), ws.numel() * 4 if ws is not None else 0, nv.stream_ptr()))
+    return out
+
+
+def linear_relu_squared(x, lin: AnyLinear, out, take):
+    """out = act(max(x W^T, 0)^2): in the product's epilogue where `lin` is in wave tiles, else behind it."""
+    if lin.tiles is None or out.data_ptr() % 8 or _ld(out) % 4:
+        relu_squared(lin(x, take(x.shape[0], lin.n)), out)
+        return out
+    return _linear_act(x, lin.tiles, out, 1)
+
+
+class GatedLinear:
+    """out = act(g' sigmoid(slope g') (u' + 1)), g' = min(x W_gate^T, limit), u' = clamp(x W_up^T, +-limit): one product whose
+    epilogue is the gate where the weights go into wave tiles (up and gate interleaved), else the product and gated_act."""
+
+    def __init__(self, gate: torch.Tensor, up: torch.Tensor, wave_tiles: bool = True):
+        assert gate.shape == up.shape and gate.dtype == up.dtype
+        self.ff, self.k = gate.shape
+        self.tiles = self.lin = None
+        if wave_tiles and gate.dtype == torch.bfloat16 and self.ff % 8 == 0 and self.k % 64 == 0:
+            self.tiles = StreamedWeight.from_up_gate(up, gate)
+        else:
+            self.lin = AnyLinear(torch.cat([gate, up], dim=0), wave_tiles=wave_tiles)
+
+    @property
+    def nbytes(self):
+        return self.tiles.nbytes if self.lin is None else self.lin.nbytes
+
+    def __call__(self, x, out, take, limit: float, slope: float):
+        if self.lin is None:
+            return _linear_act(x, self.tiles, out, 2, limit, slope)
+        gated_act(self.lin(x, take(x.shape[0], 2 * self.ff)), out, GATE_CLAMPED, limit, slope)
+        return out
+
+
 def _slices(y):
     """(first slice [rows, n], slices): a projection's output, whole or as AnyLinear.slabs left it."""
     if y.dim() == 2:

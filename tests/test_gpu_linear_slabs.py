@@ -104,3 +104,30 @@ def test_fp32_tiles_by_themselves_on_a_unit(mv, m, n, k):
     got = lin(x, torch.full((m, n), float("nan"), device=DEV))
     want = x.double() @ lin.w.double().t()
     assert (got.double() - want).abs().max().item() <= k ** 0.5 * 2 ** -24 * 8
+
+
+# every kernel that has such an epilogue: dot form, matrix form, slices behind a reduction (few rows and many), 64-row tiles of one,
+# two and four strips, 128-row tiles, both wide tiles; columns that end inside a workgroup's
+@pytest.mark.parametrize("m", [1, 4, 5, 40, 64, 65, 300, 700, 2048])
+@pytest.mark.parametrize("n,k", [(1024, 512), (1040, 2048), (8192, 1024), (16384, 2048)])
+@pytest.mark.parametrize("kind", [1, 2])
+def test_activations_in_the_product(mv, m, n, k, kind):
+    from micro_vllm_amd.kernel import ragged_ops as ops
+
+    g = torch.Generator().manual_seed(m + n + k + kind)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = (2.0 * torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV)
+    v = x.double() @ w.double().t()
+    none = lambda *a: pytest.fail("not in the epilogue")   # noqa: E731
+    err = k ** 0.5 * 2 ** -24 * 8      # of the product, as above
+    if kind == 1:
+        got = ops.linear_relu_squared(x, ops.AnyLinear(w), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), none)
+        want, slope = v.clamp(min=0) ** 2, 2 * v.abs()
+    else:
+        gate, up = w[:n // 2].contiguous(), w[n // 2:].contiguous()
+        got = ops.GatedLinear(gate, up)(x, torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV), none, 2.5, 1.702)
+        a, b = v[:, :n // 2].clamp(max=2.5), v[:, n // 2:].clamp(-2.5, 2.5)
+        want, slope = a * torch.sigmoid(1.702 * a) * (b + 1), 1.5 * (b + 1).abs() + a.abs()
+    # half a bf16 unit, the product's error through the function's slope, and 2^-20 for the function itself
+    tol = 2.0 ** -8 * want.abs() + 2 * err * slope + err + 2.0 ** -20 * want.abs()
+    assert ((got.double() - want).abs() <= tol).all()
