@@ -248,6 +248,42 @@ __global__ __launch_bounds__(256) void offset_rmsnorm_gather_kernel(const float*
     for (int c = threadIdx.x; c < n; c += 256) Act<F32>::st(out + (int64_t)row * ldo + c, (a[c] * inv) * (offset + w[c]));
 }
 
+// The same with the row in registers: n a multiple of 4 up to 4 * threads * NV, rows and w 16-byte aligned.  A few rows of a step, so
+// one trip to memory after another is all its time (a row of 4096 8.4 -> 4.5 us, of 1024 4.5 -> 2.3).
+template <bool F32, int NV>
+__global__ __launch_bounds__(1024) void offset_rmsnorm_gather_reg_kernel(const float* x, int64_t ldx, const int* idx,
+                                                                        const float* w, float eps, float offset,
+                                                                        void* out, int64_t ldo, int n) {
+    __shared__ float red[16];
+    const int row = blockIdx.x, tid = threadIdx.x, n4 = n / 4;
+    f32x4_t wv[NV], v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) wv[i] = reinterpret_cast<const f32x4_t*>(w)[min(tid + (int)blockDim.x * i, n4 - 1)];
+    const f32x4_t* a = reinterpret_cast<const f32x4_t*>(x + (int64_t)(idx ? idx[row] : row) * ldx);
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = tid + (int)blockDim.x * i;
+        v[i] = c < n4 ? a[c] : (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+    }
+    ss = block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = tid + (int)blockDim.x * i;
+        if (c >= n4) continue;
+        f32x4_t o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = (v[i][j] * inv) * (offset + wv[i][j]);
+        if (F32) {
+            reinterpret_cast<f32x4_t*>((float*)out + (int64_t)row * ldo)[c] = o;
+        } else {
+            reinterpret_cast<uint2*>((uint16_t*)out + (int64_t)row * ldo)[c] = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+        }
+    }
+}
+
 template <bool F32>
 __global__ __launch_bounds__(256) void relu_squared_kernel(const float* in, int64_t ldi, void* out_, int64_t ldo,
                                                            int n) {
@@ -438,10 +474,16 @@ __global__ __launch_bounds__(256) void embed_pair_kernel(const void* table_, con
     int id = ids[row];
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
     const int pv = prev[row];
-    // every factor reduced first: the products stay below 2^62 for any 31-bit bucket count
-    const int64_t r = pv < 0 ? buckets
-                             : (((int64_t)pv % buckets) * (mul_prev % buckets) % buckets +
-                                ((int64_t)id % buckets) * (mul_cur % buckets) % buckets) % buckets;
+    // Every factor reduced first, the multipliers by the host: the products stay below 2^62 for any 31-bit bucket count, and two
+    // remainders of 64 bits are left of six (each some hundred instructions in front of the row's first load).
+    const uint32_t nb = (uint32_t)buckets;
+    uint32_t at = nb;
+    if (pv >= 0) {
+        const uint32_t r0 = (uint32_t)((uint64_t)((uint32_t)pv % nb) * (uint64_t)mul_prev % nb);
+        const uint32_t r1 = (uint32_t)((uint64_t)((uint32_t)id % nb) * (uint64_t)mul_cur % nb);
+        at = r0 >= nb - r1 ? r0 - (nb - r1) : r0 + r1;
+    }
+    const int64_t r = at;
     float ss = 0.f;
     for (int c = threadIdx.x; c < n; c += 256) {
         const float v = Act<F32>::ld(table + (int64_t)id * n + c) * scale + Act<F32>::ld(pairs + r * n + c);
@@ -904,8 +946,19 @@ int mv_rmsnorm_gather(const float* x, int64_t ldx, const int32_t* idx, const flo
     if (rows == 0) return MV_OK;
     if (!x || !w || !out || ldx < n || ldo < n) return MV_ERR_INVALID_ARG;
     hipStream_t s = (hipStream_t)stream;
-    if (f32) hipLaunchKernelGGL(offset_rmsnorm_gather_kernel<true>, dim3(rows), dim3(256), 0, s, x, ldx, idx, w, eps, offset, out, ldo, n);
+    const bool even = n % 4 == 0 && ldx % 4 == 0 && ldo % 4 == 0 && aligned16(x) && aligned16(w) && aligned16(out);
+    const int nt = rows > 512 || n <= 1024 ? 256 : n <= 2048 ? 512 : 1024;    // as in mv_postnorm_residual
+#define MV_GATHER(NV_)                                                                                                           \
+    do {                                                                                                                         \
+        if (f32) hipLaunchKernelGGL((offset_rmsnorm_gather_reg_kernel<true, NV_>), dim3(rows), dim3(nt), 0, s, x, ldx, idx, w, eps, offset, out, ldo, n); \
+        else hipLaunchKernelGGL((offset_rmsnorm_gather_reg_kernel<false, NV_>), dim3(rows), dim3(nt), 0, s, x, ldx, idx, w, eps, offset, out, ldo, n);    \
+    } while (0)
+    if (even && n <= 4 * nt) MV_GATHER(1);
+    else if (even && n <= 8 * nt) MV_GATHER(2);
+    else if (even && n <= 16 * nt) MV_GATHER(4);
+    else if (f32) hipLaunchKernelGGL(offset_rmsnorm_gather_kernel<true>, dim3(rows), dim3(256), 0, s, x, ldx, idx, w, eps, offset, out, ldo, n);
     else hipLaunchKernelGGL(offset_rmsnorm_gather_kernel<false>, dim3(rows), dim3(256), 0, s, x, ldx, idx, w, eps, offset, out, ldo, n);
+#undef MV_GATHER
     return check_launch();
 }
 
@@ -918,6 +971,8 @@ int mv_embed_pair(const void* table, const void* pairs, const int32_t* ids, cons
     if (rows == 0) return MV_OK;
     if (!table || !pairs || !ids || !prev || !x || ldx < n || (norm_w && (!h || ldh < n))) return MV_ERR_INVALID_ARG;
     hipStream_t s = (hipStream_t)stream;
+    mul_prev %= buckets;
+    mul_cur %= buckets;
     if (f32) hipLaunchKernelGGL(embed_pair_kernel<true>, dim3(rows), dim3(256), 0, s, table, pairs, ids, prev, x, ldx, n, vocab, buckets, mul_prev, mul_cur, scale, norm_w, eps, h, ldh);
     else hipLaunchKernelGGL(embed_pair_kernel<false>, dim3(rows), dim3(256), 0, s, table, pairs, ids, prev, x, ldx, n, vocab, buckets, mul_prev, mul_cur, scale, norm_w, eps, h, ldh);
     return check_launch();

@@ -131,3 +131,21 @@ def test_activations_in_the_product(mv, m, n, k, kind):
     # half a bf16 unit, the product's error through the function's slope, and 2^-20 for the function itself
     tol = 2.0 ** -8 * want.abs() + 2 * err * slope + err + 2.0 ** -20 * want.abs()
     assert ((got.double() - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("rows,n", [(1, 64), (2, 1024), (3, 2048), (5, 4096), (2, 8192), (1, 16384), (513, 1024), (600, 4096), (2, 16388), (3, 33)])
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float32])
+def test_gathered_norms_of_every_width(mv, rows, n, act):
+    from micro_vllm_amd.kernel import ragged_ops as ops
+
+    g = torch.Generator().manual_seed(rows + n)
+    x, w = (torch.randn(rows + 2, n, generator=g) * 3).to(DEV), torch.randn(n, generator=g).to(DEV)
+    idx = torch.randint(0, rows + 2, (rows,), generator=g).to(torch.int32).to(DEV)
+    for offset in (0.0, 1.0):
+        out = torch.empty(rows, n, dtype=act, device=DEV)
+        ops.rmsnorm_gather(x, idx, w, 1e-5, out, offset)
+        v = x.double()[idx.long()]
+        want = v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-5) * (offset + w.double())
+        # one bf16 rounding; in fp32 the square sum's n additions and the four operations behind it
+        tol = 2 ** -8 if act == torch.bfloat16 else 2 ** -18
+        assert ((out.double() - want).abs() <= tol * want.abs() + 1e-6).all()
