@@ -550,6 +550,12 @@ int mv_conv_silu(const float* in, int64_t ldi, float* state, const float* w, con
  * decay[t,h] = exp(log_decay[t,h]). */
 int mv_softplus_decay(const float* raw, int64_t ld, const float* dt_bias, const float* a_log, float* gain,
                       float* decay, float* log_decay, int tokens, int heads, mv_stream_t stream);
+/* mv_conv_silu and mv_softplus_decay, in one launch where every row brings one token. */
+int mv_conv_silu_decay(const float* in, int64_t ldi, float* state, const float* w, const float* bias, float* out, int64_t ldo,
+                       const int32_t* tok_row, const int32_t* row_start, const int32_t* row_len, const int32_t* row_ctx,
+                       const int32_t* row_slot, int tokens, int rows, int channels, int taps, const float* raw, int64_t ld_raw,
+                       const float* dt_bias, const float* a_log, float* gain, float* decay, float* log_decay, int heads,
+                       mv_stream_t stream);
 
 /* Per row and head, token by token: S = decay[t,h] * S + gain[t,h] * k_t v_t^T (S: n x p, fp32, in
  * state[slot][head]); out[t, h*p ..] = S^T q_t (+ skip[h] * v_t).  q and k of head h are read at

@@ -111,6 +111,7 @@ PROTOTYPES = {
     "mv_relu_squared": (_I, [_P, _L, _P, _L, _I, _I, _I, _P]),
     "mv_softcap": (_I, [_P, _L, _F, _P]),
     "mv_conv_silu": (_I, [_P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
+    "mv_conv_silu_decay": (_I, [_P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _L, _P, _P, _P, _P, _P, _I, _P]),
     "mv_softplus_decay": (_I, [_P, _L, _P, _P, _P, _P, _P, _I, _I, _P]),
     "mv_scan_outer": (_I, [_P, _L, _I, _P, _L, _I, _P, _L, _P, _L, _P, _L, _P, _P, _P, _L, _P, _P, _P, _P,
                            _I, _I, _I, _I, _I, _P]),

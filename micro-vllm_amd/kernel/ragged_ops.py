@@ -209,14 +209,27 @@ def softcap_(v, cap: float):
     return v
 
 
-def conv_silu(inp, state, w, bias, out, step):
-    """inp [T,C] (a column slice), state [slots, taps-1, C] fp32, w [C,taps] fp32."""
+def conv_silu(inp, state, w, bias, out, step, decay=None):
+    """inp [T,C] (a column slice), state [slots, taps-1, C] fp32, w [C,taps] fp32.  `decay`: the arguments of softplus_decay, done
+    in the same launch where every row brings one token."""
     tokens, ch = inp.shape
     taps = w.shape[1]
     assert w.shape == (ch, taps) and w.is_contiguous() and out.shape == (tokens, ch)
     assert state.is_contiguous() and state.shape[1:] == (max(taps - 1, 0), ch)
     assert bias is None or (bias.numel() == ch and bias.is_contiguous())
     assert step.tokens == tokens and int(step.max_slot) < state.shape[0]
+    if decay is not None:
+        raw, dt_bias, a_log, gain, dec, log_decay = decay
+        _check_decay(*decay)
+        assert raw.shape[0] == tokens
+        nv.check("mv_conv_silu_decay", nv.lib().mv_conv_silu_decay(
+            _f32(inp).data_ptr(), _ld(inp), _f32(state).data_ptr(), _f32(w).data_ptr(),
+            None if bias is None else _f32(bias).data_ptr(), _f32(out).data_ptr(), _ld(out),
+            step.tok_row.data_ptr(), step.row_start.data_ptr(), step.row_len.data_ptr(), step.row_ctx.data_ptr(),
+            step.row_slot.data_ptr(), tokens, step.rows, ch, taps, _f32(raw).data_ptr(), _ld(raw), _f32(dt_bias).data_ptr(),
+            _f32(a_log).data_ptr(), _f32(gain).data_ptr(), _f32(dec).data_ptr(),
+            None if log_decay is None else _f32(log_decay).data_ptr(), raw.shape[1], nv.stream_ptr()))
+        return
     nv.check("mv_conv_silu", nv.lib().mv_conv_silu(
         _f32(inp).data_ptr(), _ld(inp), _f32(state).data_ptr(), _f32(w).data_ptr(),
         None if bias is None else _f32(bias).data_ptr(), _f32(out).data_ptr(), _ld(out),
@@ -224,11 +237,16 @@ def conv_silu(inp, state, w, bias, out, step):
         step.row_slot.data_ptr(), tokens, step.rows, ch, taps, nv.stream_ptr()))
 
 
-def softplus_decay(raw, dt_bias, a_log, gain, decay, log_decay=None):
+def _check_decay(raw, dt_bias, a_log, gain, decay, log_decay=None):
     tokens, heads = raw.shape
     assert gain.shape == (tokens, heads) and decay.shape == (tokens, heads)
     assert gain.is_contiguous() and decay.is_contiguous() and dt_bias.numel() == heads and a_log.numel() == heads
     assert log_decay is None or (log_decay.shape == (tokens, heads) and log_decay.is_contiguous())
+
+
+def softplus_decay(raw, dt_bias, a_log, gain, decay, log_decay=None):
+    _check_decay(raw, dt_bias, a_log, gain, decay, log_decay)
+    tokens, heads = raw.shape
     nv.check("mv_softplus_decay", nv.lib().mv_softplus_decay(
         _f32(raw).data_ptr(), _ld(raw), _f32(dt_bias).data_ptr(), _f32(a_log).data_ptr(), _f32(gain).data_ptr(),
         _f32(decay).data_ptr(), None if log_decay is None else _f32(log_decay).data_ptr(), tokens, heads,

@@ -483,3 +483,32 @@ def test_gated_group_norm_of_wide_groups(ops, rows, n, groups, f32):
 def test_scan_token_by_token_in_whole_pieces(ops, H, G, n, p):
     """The form that reads state, q, k and v in 16-byte pieces: its three state heights, one to three column tiles."""
     test_scan_whole_portions_and_rows(ops, H, G, n, p)
+
+
+@pytest.mark.parametrize("taps,C,H", [(4, 8448, 128), (3, 260, 300), (2, 64, 1), (4, 70, 5), (1, 64, 8)])
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1], [5, 1, 9]])
+def test_convolution_and_step_decays_in_one_call(ops, taps, C, H, lens):
+    """What conv_silu and softplus_decay give one after the other, bit for bit: one launch where every row brings one token and
+    the channels allow it (heads past one workgroup, one head), two elsewhere."""
+    g = torch.Generator().manual_seed(C + H)
+    T = sum(lens)
+    x = torch.randn(T, C + 4 + H, generator=g).to(DEV)
+    w, b, dt, al = (torch.randn(*s, generator=g).to(DEV) for s in ((C, taps), (C,), (H,), (H,)))
+    start = torch.randn(6, max(taps - 1, 0), C, generator=g).to(DEV)
+    res = []
+    for joint in (True, False):
+        cache = make_cache(state={0: {"conv": (max(taps - 1, 1), C)}}, slots=6)
+        names = [f"r{i}" for i in range(len(lens))]
+        state = start.clone()
+        out = []
+        for _ in range(2):      # the second step carries the first one's inputs
+            st = step_of(cache, [(k, [0] * n) for k, n in zip(names, lens)])
+            o, gain, dec, lg = (torch.full((T, n), float("nan"), device=DEV) for n in (C, H, H, H))
+            d = (x[:, C + 4:], dt, al, gain, dec, lg)
+            ops.conv_silu(x[:, :C], state, w, b, o, st, decay=d if joint else None)
+            if not joint:
+                ops.softplus_decay(*d)
+            out += [o, gain, dec, lg, state.clone()]
+        res.append(out)
+    for a, c in zip(*res):
+        assert torch.equal(a, c)
