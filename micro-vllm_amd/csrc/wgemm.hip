@@ -98,9 +98,11 @@ static int g_stamp_counter = 0;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 
-// Final value of one output element from its fp32 accumulator.
+// Final value of one output element from its fp32 accumulator.  ACT: an activation of the unrounded sum (GemmAct).  Kernels of their
+// own: with the choice made at run time the plain ones carried 1.1 KiB of code more (28672 x 4096 at 32 rows 40.6 -> 41.2 us).
+template <bool ACT = false>
 __device__ __forceinline__ float epilogue_value(const GemmArgs& a, float acc, int m, int n) {
-    if (a.act.kind == 1) {   // uniform
+    if (ACT && a.act.kind == 1) {   // uniform
         const float v = fmaxf(acc, 0.f);
         return v * v;
     }
@@ -111,8 +113,9 @@ __device__ __forceinline__ float epilogue_value(const GemmArgs& a, float acc, in
 }
 
 // ... and of a pair of rows, up and gate
+template <bool ACT = false>
 __device__ __forceinline__ float epilogue_gated(const GemmArgs& a, float gate, float up) {
-    return a.act.kind == 2 ? gated_act_f(gate, up, 2, a.act.limit, a.act.slope) : silu_mul_rounded(gate, up);
+    return ACT ? gated_act_f(gate, up, 2, a.act.limit, a.act.slope) : silu_mul_rounded(gate, up);
 }
 
 // ------------------------------------------------------------ M <= 4: dot form
@@ -123,7 +126,7 @@ struct UnitCtx {
 
 // GW waves per workgroup, each keeping two stages of U weight tiles in flight; PRO = the
 // input transform (kProNone / kProNorm / kProAddNorm).
-template <int M, int GW, int U, int PRO>
+template <int M, int GW, int U, int PRO, bool ACT = false>
 __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
     constexpr int GT = GW * kWave;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -429,11 +432,11 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 #pragma unroll
                     for (int w8 = 0; w8 < GW; ++w8) g += red[(w8 * M + m) * 16 + rr + 8];
                     reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + cur.nt * 8 + rr] =
-                        (uint16_t)f32_to_bf16_bits(epilogue_gated(a, g, s));
+                        (uint16_t)f32_to_bf16_bits(epilogue_gated<ACT>(a, g, s));
                 }
             } else {
                 reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + n] =
-                    (uint16_t)f32_to_bf16_bits(epilogue_value(a, s, m, n));
+                    (uint16_t)f32_to_bf16_bits(epilogue_value<ACT>(a, s, m, n));
             }
         }
         if (!more) break;
@@ -454,7 +457,7 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 // and the slices in order - the sums of a prefill projection cut into KS slices (gemm_prefill.hip), bit for bit, without
 // its slabs and their reduction launch.  With four slices two halves of the workgroup take SG strips each; with sixteen a
 // wave takes two slices one after the other.
-template <int MB, int SG, int KS = 0>
+template <int MB, int SG, int KS = 0, bool ACT = false>
 __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
     constexpr int U = (SG + MB <= 6) ? 2 : 1;  // k-tiles per stage (register budget)
     constexpr int kStep = KS ? 1 : kGW;        // k-tiles between a wave's tiles
@@ -593,15 +596,15 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
                     if (qq < 2) {  // rows 0..7 = up; their gates sit 8 rows (32 lanes) further
                         const f32x4_t gt = sum_at(l + 32);
                         uint2 o;
-                        o.x = pack_bf16x2(epilogue_gated(a, gt[0], s[0]), epilogue_gated(a, gt[1], s[1]));
-                        o.y = pack_bf16x2(epilogue_gated(a, gt[2], s[2]), epilogue_gated(a, gt[3], s[3]));
+                        o.x = pack_bf16x2(epilogue_gated<ACT>(a, gt[0], s[0]), epilogue_gated<ACT>(a, gt[1], s[1]));
+                        o.y = pack_bf16x2(epilogue_gated<ACT>(a, gt[2], s[2]), epilogue_gated<ACT>(a, gt[3], s[3]));
                         *reinterpret_cast<uint2*>(&reinterpret_cast<uint16_t*>(
                             a.y)[(int64_t)m * a.ldy + nt * 8 + qq * 4]) = o;
                     }
                 } else {
                     uint2 o;
-                    o.x = pack_bf16x2(epilogue_value(a, s[0], m, n0), epilogue_value(a, s[1], m, n0 + 1));
-                    o.y = pack_bf16x2(epilogue_value(a, s[2], m, n0 + 2), epilogue_value(a, s[3], m, n0 + 3));
+                    o.x = pack_bf16x2(epilogue_value<ACT>(a, s[0], m, n0), epilogue_value<ACT>(a, s[1], m, n0 + 1));
+                    o.y = pack_bf16x2(epilogue_value<ACT>(a, s[2], m, n0 + 2), epilogue_value<ACT>(a, s[3], m, n0 + 3));
                     *reinterpret_cast<uint2*>(
                         &reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + n0]) = o;
                 }
@@ -659,6 +662,7 @@ __global__ __launch_bounds__(256) void wgemm_finalize_vec8_kernel(GemmArgs a) {
 }
 
 // One thread per output element (per up/gate pair for SWIGLU); slabs added in order.
+template <bool ACT>
 __global__ __launch_bounds__(256) void wgemm_finalize_kernel(GemmArgs a) {
     const bool sw = (a.flags & MV_GEMM_SWIGLU) != 0;
     const int ncols = sw ? a.n / 2 : a.n;
@@ -685,12 +689,12 @@ __global__ __launch_bounds__(256) void wgemm_finalize_kernel(GemmArgs a) {
             const int nu = (c >> 3) * 16 + (c & 7);
             const float up = slab_sum(nu), gate = slab_sum(nu + 8);
             reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + c] =
-                (uint16_t)f32_to_bf16_bits(epilogue_gated(a, gate, up));
+                (uint16_t)f32_to_bf16_bits(epilogue_gated<ACT>(a, gate, up));
         } else if (a.flags & MV_GEMM_OUT_F32) {
             reinterpret_cast<float*>(a.y)[(int64_t)m * a.ldy + c] = slab_sum(c);
         } else {
             reinterpret_cast<uint16_t*>(a.y)[(int64_t)m * a.ldy + c] =
-                (uint16_t)f32_to_bf16_bits(epilogue_value(a, slab_sum(c), m, c));
+                (uint16_t)f32_to_bf16_bits(epilogue_value<ACT>(a, slab_sum(c), m, c));
         }
     }
 }
@@ -859,7 +863,7 @@ int launch_wgemm_finalize(float* partial, int ksplit, int m, int n, int flags, c
     const int64_t total = (int64_t)m * ncols;
     int64_t blocks = (total + 255) / 256;
     if (blocks > most) blocks = most;
-    hipLaunchKernelGGL(wgemm_finalize_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(a.act.kind ? wgemm_finalize_kernel<true> : wgemm_finalize_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, s, a);
     return check_launch();
 }
 
@@ -918,29 +922,29 @@ static int dot_form_waves_for_units(int nunits, int kt) {
 int dot_form_ksplit(int m, int nt, int kt) { return g_tune_contig ? 0 : pick_ksplit(m, nt, kt); }
 int dot_form_waves(int m, int nt, int kt) { return dot_form_waves_for_units(nt * pick_ksplit(m, nt, kt), kt); }
 
-template <int M, int GW, int PRO>
+template <int M, int GW, int PRO, bool ACT = false>
 static int launch_dot(const GemmArgs& a, int grid, hipStream_t s) {
     constexpr int U = (M <= 2) ? 4 : 2;  // tiles per stage (register budget: 128 VGPRs at 16 waves per CU)
     const size_t lds = (size_t)M * a.k * 2 + 16 + (size_t)GW * M * 16 * 4;
     if (lds > 160 * 1024) return MV_ERR_UNSUPPORTED;
     static LdsOptIn opted;  // per instantiation
-    if (int rc = ensure_dynamic_lds((const void*)wgemm_dot_kernel<M, GW, U, PRO>,
+    if (int rc = ensure_dynamic_lds((const void*)wgemm_dot_kernel<M, GW, U, PRO, ACT>,
                                     lds > 64 * 1024 ? 160 * 1024 : lds, opted))
         return rc;
 #ifdef MV_WGEMM_STAMP
     GemmArgs as = a;
     as.stamp_slot = g_stamp_counter++;
-    hipLaunchKernelGGL((wgemm_dot_kernel<M, GW, U, PRO>), dim3(grid), dim3(GW * kWave), lds, s, as);
+    hipLaunchKernelGGL((wgemm_dot_kernel<M, GW, U, PRO, ACT>), dim3(grid), dim3(GW * kWave), lds, s, as);
     return check_launch();
 #endif
-    hipLaunchKernelGGL((wgemm_dot_kernel<M, GW, U, PRO>), dim3(grid), dim3(GW * kWave), lds, s, a);
+    hipLaunchKernelGGL((wgemm_dot_kernel<M, GW, U, PRO, ACT>), dim3(grid), dim3(GW * kWave), lds, s, a);
     return check_launch();
 }
 
 template <int M, int GW>
 static int launch_dot_pro(const GemmArgs& a, int grid, hipStream_t s) {
     switch (a.prologue) {
-        case kProNone: return launch_dot<M, GW, kProNone>(a, grid, s);
+        case kProNone: return a.act.kind ? launch_dot<M, GW, kProNone, true>(a, grid, s) : launch_dot<M, GW, kProNone>(a, grid, s);
         case kProNorm: return launch_dot<M, GW, kProNorm>(a, grid, s);
         default: return launch_dot<M, GW, kProAddNorm>(a, grid, s);
     }
@@ -951,14 +955,19 @@ static int launch_dot_waves(const GemmArgs& a, int waves, int grid, hipStream_t 
     return waves == 16 ? launch_dot_pro<M, 16>(a, grid, s) : launch_dot_pro<M, 8>(a, grid, s);
 }
 
-template <int MB, int SG>
-static int launch_mfma(const GemmArgs& a, int grid, hipStream_t s) {
+template <int MB, int SG, bool ACT>
+static int launch_mfma_act(const GemmArgs& a, int grid, hipStream_t s) {
     constexpr size_t lds = (size_t)kGW * SG * MB * 64 * 4 * sizeof(float);
     static_assert(lds <= 128 * 1024, "reduction buffer fits LDS");
     static LdsOptIn opted;  // per instantiation
-    if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<MB, SG>, lds, opted)) return rc;
-    hipLaunchKernelGGL((wgemm_mfma_kernel<MB, SG>), dim3(grid), dim3(kGT), lds, s, a);
+    if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<MB, SG, 0, ACT>, lds, opted)) return rc;
+    hipLaunchKernelGGL((wgemm_mfma_kernel<MB, SG, 0, ACT>), dim3(grid), dim3(kGT), lds, s, a);
     return check_launch();
+}
+
+template <int MB, int SG>
+static int launch_mfma(const GemmArgs& a, int grid, hipStream_t s) {
+    return a.act.kind ? launch_mfma_act<MB, SG, true>(a, grid, s) : launch_mfma_act<MB, SG, false>(a, grid, s);
 }
 
 // strips per workgroup of the MFMA form: the cross-wave reduction buffer is 8 KiB per
@@ -1270,7 +1279,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
         const int64_t total = (int64_t)m * ncols;
         int blocks = (int)((total + 255) / 256);
         if (blocks > cus * 4) blocks = cus * 4;
-        hipLaunchKernelGGL(wgemm_finalize_kernel, dim3(blocks), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(a.act.kind ? wgemm_finalize_kernel<true> : wgemm_finalize_kernel<false>, dim3(blocks), dim3(256), 0, s, a);
         rc = check_launch();
     }
     return rc;
