@@ -134,16 +134,13 @@ __device__ __forceinline__ float silu_mul_rounded_quick(float gate_acc, float up
     const float sig = __builtin_amdgcn_rcpf(1.0f + e);
     return (g * sig) * u;
 }
-// the clamped gate in the same terms (gated_act_f's kind 2, nothing rounded before the result)
-__device__ __forceinline__ float gated_clamped_quick(float gate, float up, const GemmAct& act) {
-    const float g = fminf(gate, act.limit), u = fminf(fmaxf(up, -act.limit), act.limit);
-    const float e = __builtin_amdgcn_exp2f(g * (act.slope * -1.44269504088896341f));
-    return (g * __builtin_amdgcn_rcpf(1.0f + e)) * (u + 1.0f);
-}
 // ACT: an activation of the unrounded sums (GemmAct) in place of the rounded ones' bias and residual - kernels of their own, since
-// the plain forms' registers are full.  Against fp32 sums in memory and a launch that reads them: max(v, 0)^2 of 2048 x 16384
-// 33.9 us and of one row 4.6, the clamped gate of 1400 x 8192 18.7 and of 8 rows 4.6 are gone, and the products in front of them
-// write a half or a quarter of the bytes (1400 x 16384 x 2048 93 -> 86 us).
+// the plain forms' registers are full.  The clamped gate is gated_act_f itself, as behind slices and in the few-row products: the
+// library's exponential and the exact division, on fp32 sums that nothing has rounded (with the hardware's exp2 and reciprocal the
+// gate's own error grows from 2^-23 to 2^-19 at large negative arguments, and a token's value depends on how many rows its step has).
+// Against the product's fp32 sums in memory and a launch that reads them (us): 704 x 16384 x 2048 64.2 -> 56.4, 1400 rows 114.1 ->
+// 103.4, 2048 rows 140.3 -> 116.1, 4096 x 16384 x 4096 496.8 -> 416.3, 300 x 8192 x 1024 20.8 -> 14.2 (the hardware's functions: 52.9,
+// 100.0, 108.4, 403.9, 13.0); max(v, 0)^2 saves launches of 33.9 (2048 x 16384) and 4.6 (one row).
 template <int NT, int MT, int ACT = 0>
 __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_t (&acc)[NT][MT], int nt0,
                                                 int m0, int ks, int r, int q, const unsigned char* lower = nullptr,
@@ -199,8 +196,8 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
                 const auto s0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(c[0]), __float_as_uint(c[2]), false, false);
                 const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(c[1]), __float_as_uint(c[3]), false, false);
                 if constexpr (ACT == 2)
-                    o[i] = pack_bf16x2(gated_clamped_quick(__uint_as_float(s0[1]), __uint_as_float(s0[0]), a.act),
-                                       gated_clamped_quick(__uint_as_float(s1[1]), __uint_as_float(s1[0]), a.act));
+                    o[i] = pack_bf16x2(gated_act_f(__uint_as_float(s0[1]), __uint_as_float(s0[0]), 2, a.act.limit, a.act.slope),
+                                       gated_act_f(__uint_as_float(s1[1]), __uint_as_float(s1[0]), 2, a.act.limit, a.act.slope));
                 else
                     o[i] = pack_bf16x2(silu_mul_rounded_quick(__uint_as_float(s0[1]), __uint_as_float(s0[0])),
                                        silu_mul_rounded_quick(__uint_as_float(s1[1]), __uint_as_float(s1[0])));

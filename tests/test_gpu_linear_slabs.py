@@ -149,3 +149,32 @@ def test_gathered_norms_of_every_width(mv, rows, n, act):
         # one bf16 rounding; in fp32 the square sum's n additions and the four operations behind it
         tol = 2 ** -8 if act == torch.bfloat16 else 2 ** -18
         assert ((out.double() - want).abs() <= tol * want.abs() + 1e-6).all()
+
+
+# both sides of 64 rows and every form of the product; gates far below zero, where the exponential's argument is large
+@pytest.mark.parametrize("m", [1, 5, 64, 65, 130, 700, 2048])
+@pytest.mark.parametrize("n,k", [(1040, 512), (8192, 1024), (16384, 2048)])
+@pytest.mark.parametrize("kind", [1, 2])
+def test_activations_in_the_product_are_those_behind_it(mv, m, n, k, kind):
+    """The epilogue's functions are the activation kernels' own: bit for bit what they make of the same product's fp32 sums,
+    whatever form the number of rows takes."""
+    from micro_vllm_amd.kernel import ragged_ops as ops
+
+    g = torch.Generator().manual_seed(m + n + k + kind)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = (8.0 * torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV)
+    none = lambda *a: pytest.fail("not in the epilogue")   # noqa: E731
+    sums = ops.AnyLinear(w)(x)
+    if kind == 1:
+        got = ops.linear_relu_squared(x, ops.AnyLinear(w), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), none)
+        want = torch.empty_like(got)
+        ops.relu_squared(sums, want)
+    else:
+        # w as the product holds it: eight rows of up, their eight gates
+        rows = w.view(n // 16, 2, 8, k)
+        up, gate = rows[:, 0].reshape(n // 2, k), rows[:, 1].reshape(n // 2, k)
+        got = ops.GatedLinear(gate, up)(x, torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV), none, 7.0, 1.702)
+        v = sums.view(m, n // 16, 2, 8)
+        want = torch.empty_like(got)
+        ops.gated_act(torch.cat([v[:, :, 1].reshape(m, n // 2), v[:, :, 0].reshape(m, n // 2)], 1), want, ops.GATE_CLAMPED, 7.0, 1.702)
+    assert torch.equal(got, want)
