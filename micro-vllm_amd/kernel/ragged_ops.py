@@ -81,7 +81,8 @@ class AnyLinear:
         m = x.shape[0]
         if self.tiles is None or m == 0:
             ks = nv.lib().mv_linear_any_slab_count(m, self.n, self.k) if self.f32 and m else 1
-            if ks == 1 or x.stride(0) % 4 or x.data_ptr() % 16:
+            # (slices take aligned operands; a weight may be a view at any offset of a checkpoint's buffer)
+            if ks == 1 or x.stride(0) % 4 or x.data_ptr() % 16 or self.w.data_ptr() % 16:
                 return self(x, take(m, self.n)).unsqueeze(0)
             assert x.is_cuda and x.dim() == 2 and x.shape[1] == self.k and x.stride(1) == 1 and x.dtype == torch.float32
             out = take(ks * m, self.n)

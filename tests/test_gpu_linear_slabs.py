@@ -178,3 +178,21 @@ def test_activations_in_the_product_are_those_behind_it(mv, m, n, k, kind):
         want = torch.empty_like(got)
         ops.gated_act(torch.cat([v[:, :, 1].reshape(m, n // 2), v[:, :, 0].reshape(m, n // 2)], 1), want, ops.GATE_CLAMPED, 7.0, 1.702)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1024, 5120), (16, 2048, 4100), (3, 1030, 5132), (1, 16, 12)])
+@pytest.mark.parametrize("x_off,w_off", [(0, 1), (0, 2), (1, 0), (3, 3)])
+def test_unaligned_fp32_operands_go_whole(mv, m, n, k, x_off, w_off):
+    """Weights and rows that are views at any offset of a larger buffer, at shapes that are cut where both are aligned: the whole
+    product, as mv_linear_any gives it."""
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(m + n + k)
+    flat_w = (torch.randn(n * k + w_off, generator=g) / k ** 0.5).to(DEV)
+    flat_x = torch.randn(m * k + x_off, generator=g).to(DEV)
+    x, lin = flat_x[x_off:].view(m, k), AnyLinear(flat_w[w_off:].view(n, k))
+    assert lin.w.data_ptr() % 16 == 4 * w_off
+    got = lin.slabs(x, _take)
+    assert got.shape == (1, m, n) and torch.equal(got[0], lin(x))
+    want = x.double() @ lin.w.double().t()
+    assert (got[0].double() - want).abs().max().item() <= k ** 0.5 * 2 ** -24 * 8      # as above
