@@ -3,8 +3,10 @@
 The library is the only compute path: if it is missing, `lib()` raises - there is
 no PyTorch or CPU fallback behind these ops.
 """
+import contextlib
 import ctypes
 import os
+import threading
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -269,6 +271,21 @@ def ptr(t):
 
 
 _stream_ws = {}
+_recording = threading.local()
+
+
+@contextlib.contextmanager
+def own_workspaces():
+    """Inside, this thread's workspaces come from a table of their own, which is yielded: for launches that are recorded into a
+    graph.  Their addresses are replayed as long as the graph lives, so its owner keeps the table, whatever other calls on the
+    recording's stream (or on one with the same handle: torch deals out 32) make of theirs; and since no other call is given these
+    buffers, a replay on another stream meets nobody in them."""
+    outer = getattr(_recording, "table", None)
+    _recording.table = table = {}
+    try:
+        yield table
+    finally:
+        _recording.table = outer
 
 
 def stream_workspace(kind, device, nbytes):
@@ -283,8 +300,11 @@ def stream_workspace(kind, device, nbytes):
     dev = device if isinstance(device, torch.device) else torch.device(device)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     key = (kind, idx, _raw_stream(idx))
-    ws = _stream_ws.get(key)
+    table = getattr(_recording, "table", None)
+    if table is None:
+        table = _stream_ws
+    ws = table.get(key)
     if ws is None or ws.numel() * 4 < nbytes:
         ws = torch.zeros((nbytes + 3) // 4, dtype=torch.float32, device=dev)
-        _stream_ws[key] = ws
+        table[key] = ws
     return ws

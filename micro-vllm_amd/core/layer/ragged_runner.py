@@ -556,7 +556,7 @@ class RaggedRunner:
 
     def _capture(self, step: RaggedStep, cache: HybridCacheManager):
         """One run of the step on a side stream with fresh allocations (it sizes the arena and lets the
-        projections set up their per-stream workspaces), the recurrent state of the step's slots put back
+        projections set up the recording's workspaces), the recurrent state of the step's slots put back
         as it was, then the same launches recorded over an arena.  Everything a replay reads that
         changes from step to step - tokens, positions, slots, block table - lies in the cache manager's
         one device buffer; keys and values of the step are written again by the replay with the same
@@ -569,7 +569,7 @@ class RaggedRunner:
         saved = [(t, t.index_select(0, idx)) for named in cache.states.values() for t in named.values()]
         side = torch.cuda.Stream(device=self.device)
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
+        with torch.cuda.stream(side), nv.own_workspaces() as workspaces:
             self._arena, self._measured = None, 0
             try:
                 self._run(step, cache, None, None)
@@ -589,7 +589,7 @@ class RaggedRunner:
             nv.check("mv_graph_end_capture", rc)
         torch.cuda.current_stream().wait_stream(side)
         logger.info("captured a decoding step of %d rows (%d KiB of intermediates)", B, arena.numel() >> 10)
-        return HipGraph(handle), arena, logits      # the arena stays alive with the graph
+        return HipGraph(handle), arena, logits, workspaces      # what it writes to stays alive with the graph
 
     def _run(self, step: RaggedStep, cache: HybridCacheManager, want, residuals) -> torch.Tensor:
         cfg, T = self.cfg, step.tokens
