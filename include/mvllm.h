@@ -122,7 +122,8 @@ int mv_wgemm(const void* x, int64_t ldx, const void* w_tiles, const void* bias,
 /* Number of slabs an MV_GEMM_SLABS call leaves for this problem (>= 1). */
 int mv_wgemm_slab_count(int m, int n, int k);
 
-/* mv_wgemm with the input transform of the preceding norm kernel folded in (1 <= M <= 4):
+/* mv_wgemm with the input transform of the preceding norm kernel folded in (1 <= M <= 4, K up to what LDS holds of M rows: 20128
+ * for four, 26944, 40544, 81376 for three, two, one):
  *   add_r == NULL:  x' = rmsnorm(x) * ln_w                       (mv_rmsnorm, then mv_wgemm)
  *   add_r != NULL:  s = x + add_r; sum_out = bf16(s); x' = rmsnorm(s) * ln_w
  *                                                    (mv_rmsnorm_residual, then mv_wgemm)

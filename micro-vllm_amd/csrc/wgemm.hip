@@ -14,7 +14,7 @@
 //    kt0+w+8, ...) so the workgroup reads one contiguous stream.  Partial sums of
 //    the 8 waves meet in LDS in a fixed order: results are run-to-run identical.
 //  * M <= 4: dot-product form (v_dot2c_f32_bf16), x staged once per workgroup in
-//    LDS.  M > 4: v_mfma_f32_16x16x32_bf16 with the x fragment (B operand) loaded
+//    LDS.  M > 4, or x too long for that: v_mfma_f32_16x16x32_bf16 with the x fragment (B operand) loaded
 //    from L2 in the same lane layout.  Both read the same weight tiles.
 //  * ksplit > 1 (picked when strips alone cannot balance the CUs) writes fp32
 //    slabs; a small second kernel adds them in slab order and applies the epilogue.
@@ -868,6 +868,12 @@ int launch_wgemm_finalize(float* partial, int ksplit, int m, int n, int flags, c
 }
 
 // ------------------------------------------------------------ host planning
+// Which form takes m rows: up to four the dot form while their x lies in LDS beside what its waves meet in (four rows up to
+// k = 20128, three up to 26944, two up to 40544), the matrix form otherwise: it streams x.
+static size_t dot_form_lds(int m, int k, int waves) { return (size_t)m * k * 2 + 16 + (size_t)waves * m * 16 * 4; }
+static bool dot_form_fits(int m, int k, int waves) { return dot_form_lds(m, k, waves) + 512 <= 160 * 1024; }
+static bool dot_form_takes(int m, int k) { return m <= 4 && dot_form_fits(m, k, 8); }
+
 // k-slices per strip: balance whole units over the CUs.  Cost in tiles per CU,
 // with a split paying roughly one extra kernel boundary.
 static int mfma_strip_group(int m, int nt, int kt, bool free_reduce);
@@ -890,7 +896,8 @@ static int ksplit_for_units(int units, int kt) {
 // `free_reduce`: the slabs are added by a launch that runs anyway (the caller's next kernel for
 // MV_GEMM_SLABS, the norm kernel of mv_wgemm_postnorm), so a k-split costs no launch of its own.
 static int pick_ksplit(int m, int nt, int kt, bool free_reduce = false) {
-    if (m > 4) {
+    const bool dot = dot_form_takes(m, kt * 32);
+    if (!dot) {
         const int sg = mfma_strip_group(m, nt, kt, free_reduce);
         nt = (nt + sg - 1) / sg;
     }
@@ -906,7 +913,7 @@ static int pick_ksplit(int m, int nt, int kt, bool free_reduce = false) {
     // ... and for the dot form not even then: shards of tensor-parallel runs (tools/sweep_small_gemv.py,
     // M=1) run 5.4 us unsplit against 6.5-8.7 us split at 48 strips (N=768, K=4096), 5.8 against
     // 7.2-10.0 at 96 strips.
-    if (m <= 4 && nt >= 32) return 1;
+    if (dot && nt >= 32) return 1;
     return ksplit_for_units(nt, kt);
 }
 
@@ -925,7 +932,7 @@ int dot_form_waves(int m, int nt, int kt) { return dot_form_waves_for_units(nt *
 template <int M, int GW, int PRO, bool ACT = false>
 static int launch_dot(const GemmArgs& a, int grid, hipStream_t s) {
     constexpr int U = (M <= 2) ? 4 : 2;  // tiles per stage (register budget: 128 VGPRs at 16 waves per CU)
-    const size_t lds = (size_t)M * a.k * 2 + 16 + (size_t)GW * M * 16 * 4;
+    const size_t lds = dot_form_lds(M, a.k, GW);
     if (lds > 160 * 1024) return MV_ERR_UNSUPPORTED;
     static LdsOptIn opted;  // per instantiation
     if (int rc = ensure_dynamic_lds((const void*)wgemm_dot_kernel<M, GW, U, PRO, ACT>,
@@ -1139,7 +1146,7 @@ int launch_wgemm_finalize_norm(float* partial, int ksplit, int m, int n, const v
 // 8192 7.0 and of two rows 8.1 where two take 7.7.
 int wgemm_slices(int m, int n, int k) {
     const int nt = n / 16, kt = k / 32;
-    if (m > 4 || g_tune_ksplit) return pick_ksplit(m, nt, kt, true);
+    if (!dot_form_takes(m, k) || g_tune_ksplit) return pick_ksplit(m, nt, kt, true);
     return nt <= num_cus() / 2 && kt >= 128 && kt >= 2 * nt ? 2 : 1;
 }
 
@@ -1174,6 +1181,8 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
              ld_add_r < k || ld_sum_out < k))
             return MV_ERR_INVALID_ARG;
     }
+    const bool dot = dot_form_takes(m, k);
+    if (prologue != kProNone && !dot) return MV_ERR_UNSUPPORTED;   // the matrix form reads x as it is
 
     GemmArgs a = {};
     a.x = (const uint16_t*)x;
@@ -1233,7 +1242,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
     }
     a.ktps = a.kt / a.ksplit;
     a.contig = g_tune_contig;
-    const int sg = m > 4 ? mfma_strip_group(m, a.nt, a.kt, free_reduce) : 1;
+    const int sg = dot ? 1 : mfma_strip_group(m, a.nt, a.kt, free_reduce);
     a.nunits = ((a.nt + sg - 1) / sg) * a.ksplit;
     a.flags = flags;
 
@@ -1246,12 +1255,11 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
     // short k (K=1792: 4.8 vs 5.8 us) or few strips (48: 5.4 vs 5.8) are faster with eight.
     const int forced_bpc = g_tune_bpc;
     int waves = dot_form_waves_for_units(a.nunits, a.kt);
-    int bpc = forced_bpc ? forced_bpc : (m <= 4 && waves == 8 ? 2 : 1);
-    if (m <= 4) {
+    if (dot && !dot_form_fits(m, k, waves)) waves = 8;
+    int bpc = forced_bpc ? forced_bpc : (dot && waves == 8 ? 2 : 1);
+    if (dot) {
         // LDS limits co-residency; never size the grid past what fits
-        const size_t lds = (size_t)m * k * 2 + 16 + (size_t)waves * m * 64;
-        const int fit = (int)((160 * 1024) / (lds + 512));
-        if (fit < 1) return MV_ERR_UNSUPPORTED;
+        const int fit = (int)((160 * 1024) / (dot_form_lds(m, k, waves) + 512));
         if (bpc > fit) bpc = fit;
     }
     if (bpc > 4) bpc = 4;  // 4 x 512 threads = 32 waves per CU
@@ -1259,7 +1267,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
     hipStream_t s = (hipStream_t)stream;
 
     int rc;
-    switch (m) {
+    switch (dot ? m : 0) {
         case 1: rc = launch_dot_waves<1>(a, waves, grid, s); break;
         case 2: rc = launch_dot_waves<2>(a, waves, grid, s); break;
         case 3: rc = launch_dot_waves<3>(a, waves, grid, s); break;

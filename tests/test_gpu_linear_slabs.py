@@ -196,3 +196,34 @@ def test_unaligned_fp32_operands_go_whole(mv, m, n, k, x_off, w_off):
     assert got.shape == (1, m, n) and torch.equal(got[0], lin(x))
     want = x.double() @ lin.w.double().t()
     assert (got[0].double() - want).abs().max().item() <= k ** 0.5 * 2 ** -24 * 8      # as above
+
+
+# x of two to four rows that just fits the dot form's LDS, that fits with half the waves only (256 strips), and that does not
+@pytest.mark.parametrize("m,k", [(4, 20096), (4, 20160), (4, 20480), (3, 26944), (3, 28672), (2, 40512), (2, 40576)])
+@pytest.mark.parametrize("n", [64, 4096])
+def test_few_rows_of_a_long_k(mv, m, n, k):
+    from micro_vllm_amd.kernel import ragged_ops as ops
+    from micro_vllm_amd.kernel.linear import StreamedWeight, wgemm, wgemm_postnorm
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(DEV)
+    res, ln = torch.randn(m, n, generator=g).to(torch.bfloat16).to(DEV), torch.ones(n, dtype=torch.bfloat16, device=DEV)
+    want = x.double() @ w.double().t()
+    tol = k ** 0.5 * 2 ** -24 * 8      # as above
+    lin = ops.AnyLinear(w)
+    assert (lin(x).double() - want).abs().max().item() <= tol
+    assert (lin.slabs(x, _take).double().sum(0) - want).abs().max().item() <= tol
+    act = ops.linear_relu_squared(x, lin, torch.empty(m, n, dtype=torch.bfloat16, device=DEV), None)
+    sq = want.clamp(min=0) ** 2
+    assert ((act.double() - sq).abs() <= 2 ** -8 * sq + 2 * tol * want.abs() + tol).all()
+    sw = StreamedWeight.from_linear(w)
+    out, out2, normed = (torch.empty(m, n, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    wgemm(x, sw, out, residual=res)
+    # two roundings to bf16, of the product and of the sum
+    assert ((out.double() - want - res.double()).abs() <= 2 ** -8 * (want.abs() + (want + res.double()).abs()) + 2 * tol).all()
+    wgemm_postnorm(x, sw, out2, ln, 1e-5, normed, residual=res, var_from_rounded=True)
+    ref = out2.double() / torch.sqrt((out2.double() ** 2).mean(-1, keepdim=True) + 1e-5)
+    assert ((out2.double() - want - res.double()).abs() <= 2 ** -8 * (want.abs() + (want + res.double()).abs()) + 2 * tol).all()
+    # the norm's factor and the result round to bf16 once each, the weight is one
+    assert ((normed.double() - ref).abs() <= 2 ** -7 * ref.abs() + 1e-6).all()
