@@ -10,6 +10,8 @@
 //                   and the draw is the inverse CDF of the caller's uniform number.
 #include "common.h"
 
+#include <algorithm>
+
 namespace mv {
 
 constexpr int kAmThreads = 1024;
@@ -345,7 +347,7 @@ __device__ __forceinline__ void order_zeros(SampleShared& sh, int k) {
 
 // The k largest entries of a row in order, by a radix selection over 16-bit keys in two passes: any k, rows with NaNs, equal
 // entries without end.
-__device__ void radix_select(SampleShared& sh, const uint16_t* row, int nvec, int k) {
+__device__ __forceinline__ void radix_select(SampleShared& sh, const uint16_t* row, int nvec, int k) {
     auto& hist = sh.hist;
     auto& sh_u = sh.sh_u;
     auto& c_val = sh.c_val;
@@ -510,6 +512,13 @@ __device__ void radix_select(SampleShared& sh, const uint16_t* row, int nvec, in
     __syncthreads();
 }
 
+// ... out of line, for a kernel that takes it by exception: in line its eighteen thousand instructions and what lives across them
+// cost the quick selection 0.1 to 0.3 us (a pick of 32 rows, with the greedy one in front, 19.1 -> 19.4); called it saves 60 registers a
+// lane to memory (32 rows of equal logits 68.8 -> 70.5 us, 128 rows 70.3 -> 79.7).
+__device__ __attribute__((noinline)) void radix_select_called(SampleShared& sh, const uint16_t* row, int nvec, int k) {
+    radix_select(sh, row, nvec, k);
+}
+
 // Softmax over the first k of c_val / c_idx (in order), top-p prefix, inverse-CDF draw
 __device__ __forceinline__ void draw_id(SampleShared& sh, int k, float temp, float top_p, float uniform, int64_t* id) {
     auto& c_val = sh.c_val;
@@ -557,7 +566,8 @@ __device__ __forceinline__ void draw_id(SampleShared& sh, int k, float temp, flo
 
 // KEEP: chunks of the row a thread holds for the quick selection, 4 for rows of up to 32768 entries, whose threads would
 // otherwise request the same chunk again and again (32 rows of 32000, top 50: 13.0 -> 8.7 us with what else changed there).
-template <int KEEP>
+// QUICK: k up to kSmQuickK; beyond it the selection is all there is, in line (128 rows of 128256, top 1000: 106.5 us called, 96.1).
+template <int KEEP, bool QUICK>
 __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __restrict__ logits,
                                                           int64_t ld, int n,
                                                           const float* __restrict__ temps,
@@ -585,14 +595,15 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
     // 50, 295 for 256.  Those are listed and ranked by counting.  Only where more than kSmQuickMost entries reach the
     // bound (rows of mostly equal logits), for larger k and for rows with a NaN or of -infinity alone the selection below
     // runs: for k = 512 ranking by counting took longer than it (98 against 90 us).  The maxima take two packed 16-bit instructions an
-    // entry pair; the radix selection makes two LDS atomics an entry.  32 rows of 128256, top 50: 80 -> 12.3 us;
-    // top 200: 85 -> 18; ten entries left of 128256 and the rest masked 57 -> 11.3.  A row that the selection has to take
-    // after all reads its entries again (kept over both, they do not fit the registers) and is 5 to 11 us later
-    // there: 32 rows of equal logits 57 -> 68.  What a call needs besides the row - temperature, top-p, the uniform number - is
-    // requested in front: three trips to memory behind the selection were 1.5 us of 15.6.
+    // entry pair; the radix selection makes two LDS atomics an entry.  32 rows of 128256, top 50: 80 -> 11.9 us;
+    // top 200: 85 -> 17.7; ten entries left of 128256 and the rest masked 57 -> 11.4.  A row that the selection has to take
+    // after all reads its entries again (kept over both, they do not fit the registers) and saves registers around it: 32 rows of
+    // equal logits, top 50, 70.5 us where the selection alone takes 63.4 (top 257), 128 rows 79.7 and 64.6.  What a call needs besides
+    // the row - temperature, top-p, the uniform number - is requested in front: three trips to memory behind the selection were 1.5 us
+    // of 15.6.
     auto in_row = [&](int i) { return tid + i * kSmThreads < nvec; };
     bool listed = false;
-    if (k <= kSmQuickK) {   // uniform
+    if constexpr (QUICK) {
         uint4 keep[KEEP];
         load_row(keep, row, nvec);
         Largest most;
@@ -623,7 +634,7 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
         if (!sh_u[3]) {   // uniform
             // Counted before anything is listed: a full list costs its rows no more than the count.  A chunk with an entry to
             // list is read again: one body for any chunk, where sixteen over `keep` are twelve KiB of code to fetch (32 rows of
-            // 128256, top 50: 14.7 us with those, 12.3 without).
+            // 128256, top 50: 14.7 us with those, 11.9 without).
             unsigned hits = 0, mine_n = 0, slot = 0;
             auto count = [&](auto key) {
 #pragma unroll
@@ -660,7 +671,8 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
         }
         if (!listed) __syncthreads();
     }
-    if (!listed) radix_select(sh, row, nvec, k);
+    if constexpr (!QUICK) radix_select(sh, row, nvec, k);
+    else if (!listed) radix_select_called(sh, row, nvec, k);
     draw_id(sh, k, temp, top_p, uniform, ids + blockIdx.x);
 }
 
@@ -670,7 +682,9 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
 // that draws the row's last arrival ticket finds the bound and reads again only what lies behind the maxima that reach it.
 // More than kSmQuickMost candidates are sorted in LDS.  Workspace: tickets | maxima, tickets as in the greedy pick above.
 // For k up to kSmQuickK one workgroup is the faster one: handing the maxima over costs 4 us of its 8 to 18.  Top 1000 of 128256: 1 row
-// 92 -> 37 us, 32 rows 100 -> 39, 64 rows 101 -> 41; of 16384: 39 -> 35; but 128 rows of 32000 52 -> 72, so up to 64 rows.
+// 92.7 -> 36.9 us, 32 rows 94.7 -> 38.2, 64 rows 94.7 -> 40.7; 32 rows of 16384 36.0 -> 35.0, of 32000 45.2 -> 35.5; but 128 rows of
+// 32000 52 -> 72, so up to 64 rows.  Rows that are left to the selection after all come later by what the parts took: 32 rows of equal
+// logits 67.8 -> 79.7, with a NaN in each 94.9 -> 98.5.
 constexpr int kSmParts = 4;
 constexpr int kSmMaxRows = 64;
 constexpr int kSmSortMost = 2048;
@@ -870,7 +884,9 @@ extern "C" int mv_sample_or_greedy_ws(const void* logits, int64_t ld, int rows, 
                            (unsigned int*)workspace, (unsigned short*)((char*)workspace + mv::kSmTicketBytes));
         return mv::check_launch();
     }
-    const auto kernel = (n >> 3) <= 4 * mv::kSmThreads ? mv::sample_kernel<4> : mv::sample_kernel<mv::kSmKeep>;
+    const auto kernel = std::min(top_k, n) > mv::kSmQuickK ? mv::sample_kernel<mv::kSmKeep, false>
+                        : (n >> 3) <= 4 * mv::kSmThreads   ? mv::sample_kernel<4, true>
+                                                           : mv::sample_kernel<mv::kSmKeep, true>;
     hipLaunchKernelGGL(kernel, dim3(rows), dim3(mv::kSmThreads), 0, (hipStream_t)stream,
                        (const uint16_t*)logits, ld, n, temperatures, top_ps, top_k, uniforms, greedy_ids, ids);
     return mv::check_launch();
