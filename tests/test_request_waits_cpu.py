@@ -29,8 +29,9 @@ def assembly(tmp_path_factory):
 
 
 def _blocks(text, kernel):
-    """The kernel's basic blocks, each a list of 'x' (request of x into LDS), 'w' (load), wait counts and 'barrier'."""
-    body = re.search(rf"^_ZN2mv19gemm_prefill_kernelI{kernel}E\S*:.*?^\.Lfunc_end", text, re.S | re.M).group(0)
+    """The basic blocks of the kernel of these template arguments (all of them), each a list of 'x' (request of x into LDS), 'w'
+    (load), wait counts and 'barrier'."""
+    body = re.search(rf"^_ZN2mv19gemm_prefill_kernelI{kernel}EEEvNS_9PGemmArgsE:.*?^\.Lfunc_end", text, re.S | re.M).group(0)
     blocks = [[]]
     for line in map(str.strip, body.splitlines()):
         if re.match(r"\.LBB\d+_\d+:", line) or line.startswith(("s_cbranch", "s_branch")):
@@ -46,11 +47,13 @@ def _blocks(text, kernel):
     return [b for b in blocks if "x" in b and "barrier" in b]
 
 
-@pytest.mark.parametrize("kernel,pieces", [("Li8ELi8ELi4", 4), ("Li4ELi8ELi4", 2)])
-def test_a_stage_of_x_has_arrived_at_the_barrier_before_its_first_reader(assembly, kernel, pieces):
+# (every epilogue is a compilation of its own: the plain one, max(v, 0)^2, the clamped gate)
+@pytest.mark.parametrize("act", [0, 1, 2])
+@pytest.mark.parametrize("kernel,pieces", [("Li8ELi8ELi4ELi4", 4), ("Li4ELi8ELi4ELi4", 2)])
+def test_a_stage_of_x_has_arrived_at_the_barrier_before_its_first_reader(assembly, kernel, pieces, act):
     """Four stages of x: behind a stage's barrier the next stage reads what was requested a stage before this one's own
     requests, so at the barrier only the latter may be on their way."""
-    blocks = _blocks(assembly, kernel)
+    blocks = _blocks(assembly, f"{kernel}ELi{act}")
     prologue, loop = blocks[0], next(b for b in blocks if b.count("barrier") == 4)
     left = [b for b in blocks if b.count("barrier") == 1 and b is not prologue]
     assert prologue.count("x") == 3 * pieces and loop.count("x") == 4 * pieces
@@ -78,12 +81,13 @@ def test_a_stage_of_x_has_arrived_at_the_barrier_before_its_first_reader(assembl
             assert run(before, b)[1] == [pieces]
 
 
+@pytest.mark.parametrize("act", [0, 1, 2])
 @pytest.mark.parametrize("kernel", ["Li4ELi8ELi4ELi1", "Li4ELi8ELi4ELi2", "Li4ELi8ELi4ELi4"])
-def test_tiles_of_fewer_strips_wait_for_no_less(assembly, kernel):
+def test_tiles_of_fewer_strips_wait_for_no_less(assembly, kernel, act):
     """64-row tiles of one, two and four strips a wave: at every barrier, in any run through the loop and the stages behind it,
     at most the stage's own two requests of x are on their way.  (The compiler may wait for more in front of its own loads.)"""
     pieces = 2
-    blocks = _blocks(assembly, kernel)
+    blocks = _blocks(assembly, f"{kernel}ELi{act}")
     prologue, loop = blocks[0], next(b for b in blocks if b.count("barrier") == 4)
     left = [b for b in blocks if b.count("barrier") == 1 and b is not prologue]
     assert prologue.count("x") == 3 * pieces and loop.count("x") == 4 * pieces
@@ -111,3 +115,9 @@ def test_tiles_of_fewer_strips_wait_for_no_less(assembly, kernel):
                 assert most <= pieces
         queue, most = run(queue, loop)
         assert most <= pieces
+
+
+def test_every_form_with_counted_waits_is_looked_at(assembly):
+    """The forms above are all there are with four stages of x."""
+    forms = set(re.findall(r"^_ZN2mv19gemm_prefill_kernelI(Li\d+ELi\d+ELi4ELi\d+ELi\d+)EEEvNS_9PGemmArgsE:", assembly, re.M))
+    assert forms == {f"{k}ELi{act}" for k in ("Li8ELi8ELi4ELi4", "Li4ELi8ELi4ELi1", "Li4ELi8ELi4ELi2", "Li4ELi8ELi4ELi4") for act in range(3)}
