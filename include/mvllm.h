@@ -412,9 +412,11 @@ int mv_sample_topk_topp(const void* logits, int64_t ld, int rows, int n, const f
 int mv_sample_or_greedy(const void* logits, int64_t ld, int rows, int n, const float* temperatures,
                         const float* top_ps, int top_k, const float* uniforms,
                         const int64_t* greedy_ids, int64_t* ids, mv_stream_t stream);
-/* The same with a workspace of mv_sample_workspace_bytes() (zero-filled when it was allocated, used by one stream at a time),
- * with which rows of 16384 entries and more go over several workgroups each.  Without one, or with too small a one: as above. */
+/* The same with a workspace of mv_sample_workspace_bytes() (zero-filled when it was allocated, used by one stream at a time), with
+ * which a row goes over several workgroups where mv_sample_parts says so: up to 64 rows of 16384 entries and more, top_k past 256.
+ * Everywhere else, without a workspace or with too small a one: as above.  The ids are the same. */
 size_t mv_sample_workspace_bytes(void);
+int mv_sample_parts(int rows, int n, int top_k);
 int mv_sample_or_greedy_ws(const void* logits, int64_t ld, int rows, int n, const float* temperatures,
                            const float* top_ps, int top_k, const float* uniforms, const int64_t* greedy_ids, int64_t* ids,
                            void* workspace, size_t workspace_bytes, mv_stream_t stream);

@@ -92,6 +92,7 @@ PROTOTYPES = {
     "mv_argmax": (_I, [_P, _L, _I, _I, _P, _P, _Z, _P]),
     "mv_sample_topk_topp": (_I, [_P, _L, _I, _I, _P, _P, _I, _P, _P, _P]),
     "mv_sample_workspace_bytes": (_Z, []),
+    "mv_sample_parts": (_I, [_I, _I, _I]),
     "mv_sample_or_greedy_ws": (_I, [_P, _L, _I, _I, _P, _P, _I, _P, _P, _P, _P, _Z, _P]),
     "mv_sample_or_greedy": (_I, [_P, _L, _I, _I, _P, _P, _I, _P, _P, _P, _P]),
     "mv_allreduce_handle_bytes": (_Z, []),

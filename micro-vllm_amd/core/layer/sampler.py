@@ -30,9 +30,6 @@ def greedy(logits: torch.Tensor, out: torch.Tensor = None, workspace: torch.Tens
     return out[:bs]
 
 
-_MANY_K = 256      # past this many candidates long rows go over several workgroups (csrc/sampler.hip)
-
-
 def _row_params(t, bs, dev):
     """[bs] fp32 on the device, contiguous: as it is where it is that already."""
     if t.dtype != torch.float32 or t.device != dev or not t.is_contiguous():
@@ -63,9 +60,10 @@ def sample(logits: torch.Tensor, temperatures: torch.Tensor, top_ps: torch.Tenso
     ld = logits.stride(0) if bs > 1 else max(v, logits.stride(0))
     if greedy_ids is not None:
         assert greedy_ids.dtype == torch.long and greedy_ids.is_contiguous() and greedy_ids.numel() >= bs
-    if workspace is None and top_k > _MANY_K and not torch.cuda.is_current_stream_capturing():
-        workspace = nv.stream_workspace("sample", logits.device, nv.lib().mv_sample_workspace_bytes())
-    nv.check("mv_sample_or_greedy", nv.lib().mv_sample_or_greedy_ws(
+    L = nv.lib()
+    if workspace is None and L.mv_sample_parts(bs, v, int(top_k)) and not torch.cuda.is_current_stream_capturing():
+        workspace = nv.stream_workspace("sample", logits.device, L.mv_sample_workspace_bytes())
+    nv.check("mv_sample_or_greedy", L.mv_sample_or_greedy_ws(
         logits.data_ptr(), ld, bs, v, temperatures.data_ptr(), top_ps.data_ptr(), int(top_k),
         uniforms.data_ptr(), nv.ptr(greedy_ids), out.data_ptr(), nv.ptr(workspace),
         0 if workspace is None else workspace.numel() * 4, nv.stream_ptr()))

@@ -683,7 +683,7 @@ __global__ __launch_bounds__(kSmThreads) void sample_kernel(const uint16_t* __re
 // More than kSmQuickMost candidates are sorted in LDS.  Workspace: tickets | maxima, tickets as in the greedy pick above.
 // For k up to kSmQuickK one workgroup is the faster one: handing the maxima over costs 4 us of its 8 to 18.  Top 1000 of 128256: 1 row
 // 92.7 -> 36.9 us, 32 rows 94.7 -> 38.2, 64 rows 94.7 -> 40.7; 32 rows of 16384 36.0 -> 35.0, of 32000 45.2 -> 35.5; but 128 rows of
-// 32000 52 -> 72, so up to 64 rows.  Rows that are left to the selection after all come later by what the parts took: 32 rows of equal
+// 32000, whose parts come in several rounds, took 72 (in one workgroup each 45.8), so up to 64 rows.  Rows that are left to the selection after all come later by what the parts took: 32 rows of equal
 // logits 67.8 -> 79.7, with a NaN in each 94.9 -> 98.5.
 constexpr int kSmParts = 4;
 constexpr int kSmMaxRows = 64;
@@ -867,6 +867,11 @@ extern "C" int mv_sample_or_greedy(const void* logits, int64_t ld, int rows, int
 
 extern "C" size_t mv_sample_workspace_bytes(void) { return mv::kSmWorkspaceBytes; }
 
+// the one rule of which picks sample_parts_kernel takes (its comment has both sides)
+extern "C" int mv_sample_parts(int rows, int n, int top_k) {
+    return rows > 0 && rows <= mv::kSmMaxRows && top_k > mv::kSmQuickK && (n >> 3) >= mv::kSmMinVec;
+}
+
 extern "C" int mv_sample_or_greedy_ws(const void* logits, int64_t ld, int rows, int n,
                                       const float* temperatures, const float* top_ps, int top_k,
                                       const float* uniforms, const int64_t* greedy_ids, int64_t* ids,
@@ -877,8 +882,7 @@ extern "C" int mv_sample_or_greedy_ws(const void* logits, int64_t ld, int rows, 
         return MV_ERR_INVALID_ARG;
     if (!mv::aligned16(logits) || (ld % 8) != 0) return MV_ERR_INVALID_ARG;
     if ((n % 8) != 0) return MV_ERR_UNSUPPORTED;
-    if (workspace && workspace_bytes >= mv::kSmWorkspaceBytes && mv::aligned16(workspace) && rows <= mv::kSmMaxRows &&
-        top_k > mv::kSmQuickK && (n >> 3) >= mv::kSmMinVec) {
+    if (workspace && workspace_bytes >= mv::kSmWorkspaceBytes && mv::aligned16(workspace) && mv_sample_parts(rows, n, top_k)) {
         hipLaunchKernelGGL(mv::sample_parts_kernel, dim3(rows * mv::kSmParts), dim3(mv::kSmThreads), 0, (hipStream_t)stream,
                            (const uint16_t*)logits, ld, n, temperatures, top_ps, top_k, uniforms, greedy_ids, ids,
                            (unsigned int*)workspace, (unsigned short*)((char*)workspace + mv::kSmTicketBytes));

@@ -163,9 +163,10 @@ def test_greedy_on_two_streams_and_without_workspace(mv):
 @pytest.mark.parametrize("v", [16376, 16384, 16392, 32000, 128256, 131080, 151936])
 @pytest.mark.parametrize("kind", ["random", "ties", "equal", "zeros", "sorted", "few", "nan", "masked"])
 def test_rows_over_several_workgroups_pick_what_one_picks(mv, v, kind):
-    """The same ids with a workspace (rows of 16384 and more over several workgroups) and without: few and many candidates
-    (ranked, sorted, and too many of them: the radix selection), parts that end unevenly, entries of the largest maxima at
-    the row's ends, rows whose greedy pick is given; twice, since the tickets have to be back at zero."""
+    """The same ids with a workspace (rows of 16384 and more over several workgroups where there are more than 256 candidates; up
+    to those, and of shorter rows, both sides take one) and without: few and many candidates (ranked, sorted, and too many of
+    them: the radix selection), parts that end unevenly, entries of the largest maxima at the row's ends, rows whose greedy
+    pick is given; twice, since the tickets have to be back at zero."""
     from micro_vllm_amd import _native as nv
     from micro_vllm_amd.core.layer.sampler import sample
 
@@ -203,3 +204,32 @@ def test_rows_over_several_workgroups_pick_what_one_picks(mv, v, kind):
                 nv.stream_ptr()))
             for _ in range(2):
                 assert torch.equal(sample(x, temps, top_ps, k, uniforms=u, greedy_ids=greedy_ids), want), (k, greedy_ids)
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 200])
+@pytest.mark.parametrize("kind", ["random", "equal"])
+def test_picks_of_as_many_rows_as_the_workspace_holds(mv, rows, kind):
+    """Up to 64 rows the workspace has a ticket and a place for the maxima of each; more take one workgroup a row."""
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.core.layer.sampler import sample
+
+    v, k, L = 16392, 600, nv.lib()
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, v, generator=g) * 3 if kind == "random" else torch.ones(rows, v)
+    x = x.to(torch.bfloat16).to(DEV)
+    temps, top_ps, u = ((torch.rand(rows, generator=g) * a + b).to(DEV) for a, b in ((1.5, 0.05), (0.3, 0.7), (1.0, 0.0)))
+    want, got = (torch.empty(rows, dtype=torch.long, device=DEV) for _ in range(2))
+    nv.check("mv_sample_or_greedy", L.mv_sample_or_greedy(
+        x.data_ptr(), v, rows, v, temps.data_ptr(), top_ps.data_ptr(), k, u.data_ptr(), None, want.data_ptr(), nv.stream_ptr()))
+    # a buffer of that size and not a byte more is written to (its tickets are back at zero, what lies behind it is as it was)
+    size = L.mv_sample_workspace_bytes()
+    room = torch.full((size + 4096,), 7, dtype=torch.uint8, device=DEV)
+    room[:size] = 0
+    for _ in range(2):
+        nv.check("mv_sample_or_greedy_ws", L.mv_sample_or_greedy_ws(
+            x.data_ptr(), v, rows, v, temps.data_ptr(), top_ps.data_ptr(), k, u.data_ptr(), None, got.data_ptr(),
+            room.data_ptr(), size, nv.stream_ptr()))
+        assert torch.equal(got, want)
+    assert bool((room[size:] == 7).all()) and bool((room[:64 * 64 * 4] == 0).all())
+    assert bool(room[64 * 64 * 4:size].any()) == bool(L.mv_sample_parts(rows, v, k)) == (rows <= 64)
+    assert torch.equal(sample(x, temps, top_ps, k, uniforms=u), want)

@@ -88,3 +88,13 @@ def test_decode_attention_split_choice(mv):
         ws = L.mv_paged_attn_decode_workspace_bytes(bs, 32, 128, s)
         # unsplit calls need none; split ones start with the 1 MiB of arrival tickets
         assert s >= 1 and (ws == 0 if s == 1 else ws >= (1 << 20) + bs * 32 * s * (128 + 1) * 4)
+
+
+def test_which_picks_go_over_several_workgroups(mv):
+    from micro_vllm_amd import _native as nv
+
+    L = nv.lib()
+    takes = lambda *a: bool(L.mv_sample_parts(*a))   # noqa: E731
+    assert takes(1, 16384, 257) and takes(64, 128256, 1000) and takes(32, 128256, 4096)
+    assert not takes(32, 128256, 256) and not takes(65, 128256, 257) and not takes(64, 16376, 257)
+    assert not takes(0, 128256, 257) and not takes(1, 0, 257)
