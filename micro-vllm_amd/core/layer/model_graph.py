@@ -620,8 +620,12 @@ class ModelGraphRunner:
             if use_torch_graph:
                 # a failure here is raised, never swallowed: ranks that captured and ranks that did
                 # not would otherwise issue different sequences of collectives
+                # thread-local mode, as the library's own capture: the process group's watchdog thread
+                # queries the events of the warm-up's collectives whenever it comes round to them, and
+                # under the default (global) mode such a query from any thread is an error while a
+                # capture is open - the watchdog then ends the process
                 g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g, stream=side):
+                with torch.cuda.graph(g, stream=side, capture_error_mode="thread_local"):
                     self.decode(self._input_ids[:bs], bs, cache_manager)
             else:
                 import ctypes
