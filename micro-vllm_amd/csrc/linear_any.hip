@@ -396,66 +396,103 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
     }
 }
 
-// fp32 operands, few rows: the weights are streamed past them, straight from memory into the operand registers of the
-// same matrix instructions.  A workgroup forms sixteen neighbouring outputs of up to sixteen rows, its four waves the
-// four quarters of k; kStreamAhead steps (32 k of sixteen weight rows, 2 KB) of a wave are in flight while the ones before
-// are multiplied.  Rows past the last one repeat it: the matrix instruction takes sixteen either way, and a launch like
-// this waits for memory.
-// Measured (outputs x k, us; before: 64 x 64 tiles of vector FMAs): 1 row 1024 x 5120 477 -> 20, 9472 x 1024 105 -> 15,
-// 32000 x 1024 140 -> 36, 16384 x 4096 416 -> 60 (4.5 TB/s); 8 rows 490 -> 24, 109 -> 18, 144 -> 43, 426 -> 73.  The 32 x
-// 32 tile takes 34, 22, 44, 74 for up to 32 rows: it is ahead from 9 rows on where the output is wide (16 rows, 32000 x
-// 1024: 45 against 53), from 17 on everywhere (32 rows, 1024 x 5120: 35 against 40).
-constexpr int kStreamRows = 8, kStreamRowsNarrow = 16, kStreamNarrow = 8192, kStreamAhead = 4, kStreamSlice = 8;
+// fp32 operands, few rows: the weights are streamed past them.  A workgroup forms sixteen neighbouring outputs of up to
+// sixteen rows, its four waves the four quarters of k, by the same matrix instructions in the same order as the tiles.  Rows
+// past the last one repeat it: the matrix instruction takes sixteen either way, and a launch like this waits for memory.
+// A wave takes 128 k of its sixteen weight rows at a time: half a wave reads 512 neighbouring bytes of a row, so that a
+// request is four whole lines of two rows and not a piece of sixteen, and the rows meet the instruction's operand layout in
+// the wave's own part of LDS (rows 528 bytes apart: the sixteen rows of a read are on different banks; no barrier, a wave's LDS
+// operations are in order).  Two such pieces are in flight, 16 KB a wave.
+// Measured against operands read straight into that layout, 64 bytes of sixteen rows to a request (outputs x k, 3 rows, us):
+// 32000 x 1024 39.8 -> 24.2 (5.4 TB/s), 9472 x 1024 16.1 -> 10.4, 16384 x 4096 61.1 -> 44.1 (6.1 TB/s), 1024 x 5120 20.6 -> 12.3 (in four
+// slices 10.8 -> 7.3), 1024 x 1024 6.7 -> 5.0, 65536 x 64 70 -> 18; 16 rows 1024 x 5120 28.7 -> 16.3, 1280 x 1024 8.4 -> 6.3.
+// From nine rows on the tiles are ahead where the output is wide and k is short (16 rows, 65536 x 64: 10.3 us against 25.6, 32000 x 256 15.4
+// against 15.6; 32000 x 512 28.6 against 18.9, 16384 x 4096 74 against 49), from 17 on everywhere.
+constexpr int kStreamRows = 8, kStreamRowsMore = 16, kStreamNarrow = 8192, kStreamLongK = 512, kStreamSlice = 8;
+constexpr int kStreamK = 128, kStreamPad = kStreamK + 4;   // k of a piece, floats of a row in LDS
 
+// MR: rows of x that are read, 4, 8 or 16
+template <int MR>
 __global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __restrict__ x, int64_t ldx,
                                                                 const float* __restrict__ w, int64_t ldw,
                                                                 float* __restrict__ y, int64_t ldy, int M, int N, int K) {
     // blockIdx.y: a slice of k of its own, [slice][M][N] in y (ldy = N); the wave's share is a quarter of the slice
-    __shared__ float part[3][64][5];
+    extern __shared__ __attribute__((aligned(16))) float ls_lds[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4, n0 = blockIdx.x * 16;
+    const int half = lane >> 5, kl = (lane & 31) * 4;
     const int shares = 4 * gridDim.y, share = 4 * blockIdx.y + wave;
     const int per = ((K + kLfBK - 1) / kLfBK + shares - 1) / shares;
     y += (int64_t)blockIdx.y * M * ldy;
-    const float* wp = w + (int64_t)min(n0 + r, N - 1) * ldw;
-    const float* xp = x + (int64_t)min(r, M - 1) * ldx;
-    f32x4_t acc = {0, 0, 0, 0};
-    constexpr int U = kStreamAhead;
-    f32x4_t wv[2][U][2], xv[2][U][2];
-    auto request = [&](int set, int st) {
+    // k of this wave, in pieces; past the share or the end of k a lane reads its row's start and puts zeros down
+    const int first = share * per * kLfBK, end = min(K, first + per * kLfBK);
+    const int pieces = (per * kLfBK + kStreamK - 1) / kStreamK;
+    const float* wp[8];
+    const float* xp[MR / 2];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+    for (int i = 0; i < 8; ++i) wp[i] = w + (int64_t)min(n0 + 2 * i + half, N - 1) * ldw;
+#pragma unroll
+    for (int i = 0; i < MR / 2; ++i) xp[i] = x + (int64_t)min(2 * i + half, M - 1) * ldx;
+    float* ws = ls_lds + wave * (16 + MR) * kStreamPad;
+    float* xs = ws + 16 * kStreamPad;
+    f32x4_t acc = {0, 0, 0, 0};
+    f32x4_t wv[2][8], xv[2][MR / 2];
+    auto request = [&](int set, int piece) {
+        const int col = first + piece * kStreamK + kl, at = col < end ? col : 0;
+#pragma unroll
+        for (int i = 0; i < MR / 2; ++i) xv[set][i] = *reinterpret_cast<const f32x4_t*>(xp[i] + at);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) wv[set][i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(wp[i] + at));
+    };
+    auto put = [&](int set, int piece) {
+        const bool in = first + piece * kStreamK + kl < end;
+        const f32x4_t zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < MR / 2; ++i)
+            *reinterpret_cast<f32x4_t*>(xs + (2 * i + half) * kStreamPad + kl) = in ? xv[set][i] : zero;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            *reinterpret_cast<f32x4_t*>(ws + (2 * i + half) * kStreamPad + kl) = in ? wv[set][i] : zero;
+    };
+    auto multiply = [&](int piece) {
+#pragma unroll
+        for (int u = 0; u < kStreamK / kLfBK; ++u) {
+            if (piece * (kStreamK / kLfBK) + u >= per) break;   // uniform
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                // past the quarter nothing is multiplied: its row's start is read instead of another quarter's data
-                const int col = st + u < per ? (share * per + st + u) * kLfBK + h * 16 + q * 4 : K;
-                const bool in = col < K;
-                wv[set][u][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(wp + (in ? col : 0)));
-                xv[set][u][h] = *reinterpret_cast<const f32x4_t*>(xp + (in ? col : 0));
+                const int at = u * kLfBK + h * 16 + q * 4;
+                const f32x4_t wf = *reinterpret_cast<const f32x4_t*>(ws + r * kStreamPad + at);
+                const f32x4_t xf = *reinterpret_cast<const f32x4_t*>(xs + min(r, MR - 1) * kStreamPad + at);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    wv[set][u][h][e] = in ? wv[set][u][h][e] : 0.f;
-                    xv[set][u][h][e] = in ? xv[set][u][h][e] : 0.f;
-                }
+                for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[e], xf[e], acc, 0, 0, 0);
             }
-    };
-    auto multiply = [&](int set, int st) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (st + u >= per) continue;   // uniform
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[set][u][h][e], xv[set][u][h][e], acc, 0, 0, 0);
         }
     };
+    auto settle = [] {   // between a wave's own writes and reads of LDS: an order for the compiler, no instruction
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto turn = [&](int set, int piece, bool more) {
+        put(set, piece);
+        if (more) request(set, piece + 2);
+        settle();
+        multiply(piece);
+        settle();
+    };
     request(0, 0);
-    for (int st = 0; st < per; st += 2 * U) {
-        request(1, st + U);
-        multiply(0, st);
-        request(0, st + 2 * U);
-        multiply(1, st + U);
+    if (pieces > 1) {
+        request(1, 1);
+        int p = 0;
+        for (; p + 2 < pieces; p += 2) {
+            turn(0, p, true);
+            turn(1, p + 1, true);
+        }
+        turn(0, p, false);
+        turn(1, p + 1, false);
+    } else {
+        turn(0, 0, false);
     }
+    __syncthreads();
+    float(*part)[64][5] = reinterpret_cast<float(*)[64][5]>(ls_lds);
     if (wave > 0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) part[wave - 1][lane][j] = acc[j];
@@ -565,6 +602,24 @@ static int launch_linear_f32_tiles(const float* x, int64_t ldx, const float* w, 
     return check_launch();
 }
 
+// whether the rows are few enough for the streamed form
+static bool streams_f32(int m, int n, int k) {
+    using namespace mv;
+    return m <= (n < kStreamNarrow || k >= kStreamLongK ? kStreamRowsMore : kStreamRows);
+}
+
+static int launch_linear_stream(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
+                                int k, int slices, hipStream_t s) {
+    using namespace mv;
+    const int form = m <= 4 ? 0 : m <= 8 ? 1 : 2;
+    const size_t lds = (size_t)4 * (16 + (4 << form)) * kStreamPad * 4;
+    static LdsOptIn done[3];
+    const auto kernel = form == 0 ? linear_stream_f32_kernel<4> : form == 1 ? linear_stream_f32_kernel<8> : linear_stream_f32_kernel<16>;
+    if (const int rc = ensure_dynamic_lds((const void*)kernel, lds, done[form])) return rc;
+    hipLaunchKernelGGL(kernel, dim3((n + 15) / 16, slices), dim3(256), lds, s, x, ldx, w, ldw, y, ldy, m, n, k);
+    return check_launch();
+}
+
 // Which fp32 form.  Few rows of one product stream the weights (see kStreamRows).  Otherwise the tile by the time the
 // launch takes in it: rounds of tiles over the compute units times what a tile costs a unit, in hundredths of a us as measured,
 // per k-step of 32 and for its start and end - 32 x 32 (four groups, a quarter of the steps each) 200 + 88 a step of a quarter, 64 x
@@ -577,10 +632,9 @@ static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_
                              int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s, mv::RowSegments sg,
                              int total_rows) {
     using namespace mv;
-    if (m <= (n < kStreamNarrow ? kStreamRowsNarrow : kStreamRows) && !sg.seg && batch == 1 && k % 4 == 0 && ldx % 4 == 0 &&
+    if (streams_f32(m, n, k) && !sg.seg && batch == 1 && k % 4 == 0 && ldx % 4 == 0 &&
         ldw % 4 == 0 && aligned16(x) && aligned16(w)) {
-        hipLaunchKernelGGL(linear_stream_f32_kernel, dim3((n + 15) / 16), dim3(256), 0, s, x, ldx, w, ldw, y, ldy, m, n, k);
-        return check_launch();
+        return launch_linear_stream(x, ldx, w, ldw, y, ldy, m, n, k, 1, s);
     }
     const int64_t per = sg.seg ? (total_rows + batch - 1) / batch : m;
     const int64_t cus = num_cus();
@@ -639,7 +693,7 @@ static int launch_linear_any(const void* x, int64_t ldx, const void* w, int64_t 
 // 72.6; 1024 x 1024 (two steps a wave in four) 6.9 -> 6.8 -> 6.6.  The error against 64 bits falls with the slices (6.4e-7 -> 3.2e-7).
 extern "C" int mv_linear_any_slab_count(int m, int n, int k) {
     using namespace mv;
-    if (m <= 0 || n <= 0 || k <= 0 || m > (n < kStreamNarrow ? kStreamRowsNarrow : kStreamRows) || k % 4) return 1;
+    if (m <= 0 || n <= 0 || k <= 0 || !streams_f32(m, n, k) || k % 4) return 1;
     const int strips = (n + 15) / 16, steps = (k + kLfBK - 1) / kLfBK;
     int ks = 1;
     while (2 * ks * strips <= num_cus() && steps >= 2 * ks * 4 * kStreamSlice) ks *= 2;
@@ -656,9 +710,7 @@ extern "C" int mv_linear_any_slabs(const float* x, int64_t ldx, const float* w, 
     if (slabs_bytes < (size_t)ks * m * n * sizeof(float)) return MV_ERR_WORKSPACE;
     if (ks == 1) return mv_linear_any(x, ldx, w, ldw, slabs, n, m, n, k, 1, stream);
     if (ldx % 4 || ldw % 4 || !aligned16(x) || !aligned16(w)) return MV_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(linear_stream_f32_kernel, dim3((n + 15) / 16, ks), dim3(256), 0, (hipStream_t)stream, x, ldx, w, ldw, slabs,
-                       n, m, n, k);
-    return check_launch();
+    return launch_linear_stream(x, ldx, w, ldw, slabs, n, m, n, k, ks, (hipStream_t)stream);
 }
 
 extern "C" int mv_linear_any(const void* x, int64_t ldx, const void* w, int64_t ldw, float* y, int64_t ldy,

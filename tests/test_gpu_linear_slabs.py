@@ -91,6 +91,23 @@ def test_streamed_fp32_slices_add_up_to_the_product(mv, m, n, k):
     assert lin.slabs(wide, _take).shape == (1, m, n)
 
 
+# streamed fp32 weights: one piece of 128 k a quarter, a piece and a step, three pieces, four and a part; four, eight and sixteen rows of
+# x and one past each; wide outputs from k = 512 on and tiles short of it.  A row by itself has the same bits
+@pytest.mark.parametrize("m,n,k", [(4, 33, 512), (5, 40, 516), (8, 1030, 1100), (9, 17, 2052), (16, 16, 4), (3, 8200, 1668), (9, 8208, 512),
+                                   (16, 8208, 508), (16, 9001, 1024)])
+def test_streamed_fp32_pieces(mv, m, n, k):
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.full((m, k + 4), float("nan"), device=DEV), torch.full((n, k + 4), float("nan"), device=DEV)
+    x[:, :k] = torch.randn(m, k, generator=g).to(DEV)
+    w[:, :k] = (torch.randn(n, k, generator=g) / k ** 0.5).to(DEV)
+    lin = AnyLinear(w[:, :k].contiguous())
+    got = lin(x[:, :k], torch.full((m, n), float("nan"), device=DEV))
+    assert (got.double() - x[:, :k].double() @ lin.w.double().t()).abs().max().item() <= k ** 0.5 * 2 ** -24 * 8
+    assert torch.equal(lin(x[m - 1:, :k].contiguous()), got[m - 1:])
+
+
 # 64 x 64 tiles in four groups: up to one for every compute unit, k from 18 steps of 32 on and one short of it, k that ends
 # inside a step and inside a group of four, rows and columns that end inside a tile
 @pytest.mark.parametrize("m,n,k", [(567, 1024, 5120), (1000, 1024, 576), (1000, 1024, 544), (641, 1601, 1030), (1000, 1000, 1092),
