@@ -929,9 +929,8 @@ static int dot_form_waves_for_units(int nunits, int kt) {
 int dot_form_ksplit(int m, int nt, int kt) { return g_tune_contig ? 0 : pick_ksplit(m, nt, kt); }
 int dot_form_waves(int m, int nt, int kt) { return dot_form_waves_for_units(nt * pick_ksplit(m, nt, kt), kt); }
 
-template <int M, int GW, int PRO, bool ACT = false>
-static int launch_dot(const GemmArgs& a, int grid, hipStream_t s) {
-    constexpr int U = (M <= 2) ? 4 : 2;  // tiles per stage (register budget: 128 VGPRs at 16 waves per CU)
+template <int M, int GW, int U, int PRO, bool ACT>
+static int launch_dot_stage(const GemmArgs& a, int grid, hipStream_t s) {
     const size_t lds = dot_form_lds(M, a.k, GW);
     if (lds > 160 * 1024) return MV_ERR_UNSUPPORTED;
     static LdsOptIn opted;  // per instantiation
@@ -946,6 +945,18 @@ static int launch_dot(const GemmArgs& a, int grid, hipStream_t s) {
 #endif
     hipLaunchKernelGGL((wgemm_dot_kernel<M, GW, U, PRO, ACT>), dim3(grid), dim3(GW * kWave), lds, s, a);
     return check_launch();
+}
+
+// Tiles per stage: four for one and two rows, two for three and four (register budget: 128 VGPRs at 16 waves per CU).  Where a wave
+// has no more than four tiles of a strip (k <= 1024 on eight waves) two as well: a stage of four would hold them all, and the second
+// one ask for its last tile four times over (one row, us, four -> two a stage: 32000 x 1024 15.3 -> 11.6,
+// 9472 x 1024 7.0 -> 5.3, 1024 x 1024 3.5 -> 3.3, 8192 x 512 4.9 -> 4.3).  The sums are the same bits.
+template <int M, int GW, int PRO, bool ACT = false>
+static int launch_dot(const GemmArgs& a, int grid, hipStream_t s) {
+    if constexpr (M <= 2 && GW == 8) {
+        if (std::min(a.kt, a.ktps) <= 4 * GW) return launch_dot_stage<M, GW, 2, PRO, ACT>(a, grid, s);
+    }
+    return launch_dot_stage<M, GW, M <= 2 ? 4 : 2, PRO, ACT>(a, grid, s);
 }
 
 template <int M, int GW>

@@ -244,3 +244,27 @@ def test_few_rows_of_a_long_k(mv, m, n, k):
     assert ((out2.double() - want - res.double()).abs() <= 2 ** -8 * (want.abs() + (want + res.double()).abs()) + 2 * tol).all()
     # the norm's factor and the result round to bf16 once each, the weight is one
     assert ((normed.double() - ref).abs() <= 2 ** -7 * ref.abs() + 1e-6).all()
+
+
+# one and two rows up to the k whose tiles fill one stage, and a tile past it: the sums of the three-row kernel, bit for bit, plain,
+# with a norm in front, with a bias and with a gate; strips that end inside a round of workgroups
+@pytest.mark.parametrize("n,k", [(48, 32), (528, 256), (9472, 992), (1040, 1024), (9472, 1024), (16400, 1024), (1040, 1056)])
+def test_short_k_of_one_and_two_rows(mv, n, k):
+    from micro_vllm_amd.kernel.linear import StreamedWeight, wgemm, wgemm_norm
+
+    g = torch.Generator().manual_seed(n + k)
+    x = torch.randn(3, k, generator=g).bfloat16().to(DEV)
+    wt = (torch.randn(n, k, generator=g) / k ** 0.5).bfloat16().to(DEV)
+    ln, bias = torch.rand(k, generator=g).bfloat16().to(DEV), torch.randn(n, generator=g).bfloat16().to(DEV)
+    w, gu = StreamedWeight.from_linear(wt), StreamedWeight.from_up_gate(wt[:n // 2].contiguous(), wt[n // 2:].contiguous())
+
+    def forms(rows):
+        r, out = x[:rows], lambda c, dt=torch.bfloat16: torch.empty(rows, c, dtype=dt, device=DEV)
+        return (wgemm(r, w, out(n, torch.float32)), wgemm(r, w, out(n), bias=bias), wgemm(r, gu, out(n // 2), swiglu=True),
+                wgemm_norm(r, ln, 1e-5, w, out(n)), wgemm_norm(r, ln, 1e-5, w, out(n), add_r=r, sum_out=out(k)))
+
+    want = forms(3)
+    assert (want[0].double() - x.double() @ wt.double().t()).abs().max().item() <= k ** 0.5 * 2 ** -24 * 64
+    for rows in (1, 2):
+        for a, b in zip(forms(rows), want):
+            assert torch.equal(a, b[:rows])
