@@ -645,6 +645,18 @@ int mv_window_attn(const float* q, int64_t ldq, const void* k_cache, const void*
                    int short_tokens, const float* gate, int64_t ldg, int chunked, mv_stream_t stream);
 /* How many splits of the keys mv_window_attn should be given for a step of `tokens` tokens (1: none). */
 int mv_window_attn_splits(int tokens, int heads, int kv_heads, int window, int keep_first);
+/* mv_qk_rotary_store and mv_window_attn (no slopes, no gate, not chunked) as one launch, for steps in which no two tokens are of one
+ * sequence: a token's own key and value, which it stores, are the only ones of the step that it sees.  Same results, bit for bit, except
+ * that the queries of qk stay as projected.  `part` and `splits` as for mv_window_attn, which must be given.  _ok: whether a step of this
+ * shape has such a launch (otherwise MV_ERR_UNSUPPORTED, as where the caches are not 16-byte aligned). */
+int mv_rotary_window_attn(const float* qk, int64_t ld, const float* q_bias, const float* k_bias, const double* inv_freq, int rot,
+                          int adjacent, void* k_cache, void* v_cache, void* out, int64_t ldo, const int32_t* tok_row,
+                          const int32_t* tok_pos, const int32_t* block_table, int bt_stride, int page, int tokens, int heads,
+                          int kv_heads, int d, int dv, float scale, int window, int keep_first, const float* sinks, float* part,
+                          int splits, const float* act_in, int64_t lda, void* act_out, int64_t ldao, int act_n, int act_kind,
+                          float act_limit, float act_slope, int f32, mv_stream_t stream);
+int mv_rotary_window_attn_ok(int tokens, int heads, int kv_heads, int d, int dv, int rot, int window, int keep_first, int splits,
+                             int f32);
 
 /* ---- further row-wise steps of fp32-stream stacks (stream_ops.hip) ---------------------------------- */
 

@@ -679,15 +679,19 @@ class RaggedRunner:
         # activations' traffic would otherwise push out of the caches
         act = (proj[:, (H + G) * d:], cat[:, H * d:], ops.GATE_GELU_TANH, 0.0, 1.0) if dense else None
         fuse_act = dense and T <= 64
-        ops.qk_rotary_store(qk, w["q_b"], w["k_b"], kc, vc, w["inv_freq"], step, H, G, d, int(m["rot"]["dims"]),
-                            adjacent=True, act=act if fuse_act else None)
         window, keep = int(m["mask"]["size"]), int(m["mask"].get("keep_first", 0))
         # tokens of short rows (decoding): the query heads of a key/value head share its reads, the keys are cut over
         # several workgroups and the pieces meet in `part`
         splits = ops.window_attn_splits(T, H, G, window, keep) if self.grouped_attn else 0
         part = self._f32buf(1, T * H * splits * (d + 2)) if splits else None
-        ops.window_attn(qk, kc, vc, cat[:, :H * d], step, None, H, G, d, d, float(m["scale"]), window,
-                        tiled=self.tiled_attn, keep_first=keep, sinks=w["sink"], part=part, splits=splits)
+        rot, scale = int(m["rot"]["dims"]), float(m["scale"])
+        # one token a row: rotation, gate and attention are one launch
+        if not ops.rotary_window_attn(qk, w["q_b"], w["k_b"], kc, vc, w["inv_freq"], cat[:, :H * d], step, H, G, d, rot, scale, window,
+                                      keep_first=keep, sinks=w["sink"], part=part, splits=splits, act=act if fuse_act else None):
+            ops.qk_rotary_store(qk, w["q_b"], w["k_b"], kc, vc, w["inv_freq"], step, H, G, d, rot, adjacent=True,
+                                act=act if fuse_act else None)
+            ops.window_attn(qk, kc, vc, cat[:, :H * d], step, None, H, G, d, d, scale, window, tiled=self.tiled_attn,
+                            keep_first=keep, sinks=w["sink"], part=part, splits=splits)
         if dense and not fuse_act:
             ops.gated_act(act[0], act[1], act[2])
         y1 = w["w_out"].slabs(cat, self._f32buf)

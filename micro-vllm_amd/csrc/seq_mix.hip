@@ -1857,18 +1857,51 @@ __device__ __forceinline__ float dpp(float x) {
 typedef __attribute__((ext_vector_type(8))) __bf16 wa_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float wa_f32x4_t;
 
-template <bool F32, int HEADS, int NW, int KS, int VE>
+// What a step of single tokens does in front of its attention, in the same launch: qk_rotary_store_kernel's work, same arithmetic.
+// `units` workgroups attend; those behind them form the gate of a feed-forward.
+struct StepRotary {
+    const float *q_bias, *k_new, *k_bias;      // k_new: the step's keys, rows as far apart as q's
+    const double* inv_freq;
+    int rot, adjacent;
+    unsigned units;
+    const float* act_in;
+    void* act_out;
+    int64_t lda, ldao;
+    int act_n, act_kind;
+    float act_limit, act_slope;
+};
+
+// ROT: q and the token's own key come as projected.  A wave each turns a query head or the key (the angles in fp64, as
+// qk_rotary_store_kernel forms them) while the first tiles are on their way; the turned queries lie in LDS, and the tile that holds
+// the token's own position takes key and value from there too: the page is written by the first split and read by later steps.
+// What another split reads of that place meanwhile is not used.
+// One launch in place of two (us, 8 heads of 128 on 2, a gate of 4096 beside them): one token bf16 at 45 keys 9.9 -> 6.6, 300 13.8 -> 11.6,
+// 1100 22.0 -> 20.2; fp32 10.8 -> 8.3, 16.5 -> 15.1, 20.6 -> 20.0; 8 tokens of 16 heads on 4 at 500 keys 17.0 -> 14.7.
+template <bool F32, int HEADS, int NW, int KS, int VE, bool ROT = false>
 __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q, int64_t ldq, const void* kc_, const void* vc_,
                                                               void* out_, int64_t ldo, float* part, PagedRows pr,
                                                               const float* slopes, const float* sinks, int H, int G,
                                                               float scale, int window, int keep_first, const int* row_len,
                                                               int max_len, int splits, const float* gate, int64_t ldg,
-                                                              int chunked) {
+                                                              int chunked, StepRotary ra) {
     typedef typename ActS<F32>::T T_;
     constexpr int d = 32 * KS, dv = 16 * VE, HB = HEADS == 8 ? 2 : 1, RT = HEADS;
     constexpr int NK = F32 ? 2 * KS : KS, VW = F32 ? VE : VE / 2;     // 16-byte pieces of a key, words of a value, per lane
     __shared__ __attribute__((aligned(16))) float red[NW * RT * dv];
     __shared__ float mm[NW * RT], ll[NW * RT];
+    __shared__ __attribute__((aligned(16))) float qs[ROT ? RT * d : 4];          // ROT: turned queries, the token's own key
+    __shared__ __attribute__((aligned(16))) T_ kn[ROT ? d : 8], vn[ROT ? dv : 8];   // and value
+    if constexpr (ROT) {
+        if (blockIdx.x >= ra.units) {
+            const unsigned cb = (ra.act_n + 64 * NW - 1) / (64 * NW), i = blockIdx.x - ra.units;
+            const int64_t r = i / cb;
+            const int c = (i % cb) * 64 * NW + threadIdx.x;
+            if (blockIdx.y == 0 && c < ra.act_n)
+                ActS<F32>::st((T_*)ra.act_out + r * ra.ldao + c, gated_act_f(ra.act_in[r * ra.lda + c], ra.act_in[r * ra.lda + ra.act_n + c],
+                                                                            ra.act_kind, ra.act_limit, ra.act_slope));
+            return;
+        }
+    }
     const T_* kc = (const T_*)kc_;
     const T_* vc = (const T_*)vc_;
     const int R = H / G, ngrp = (R + kGrpMax - 1) / kGrpMax;
@@ -1883,40 +1916,47 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     wa_bf16x8_t qb[HB][F32 ? 1 : KS];
     wa_f32x4_t qf[HB][F32 ? NK : 1];
     float slope[HB];
+    auto take_queries = [&] {
 #pragma unroll
-    for (int b = 0; b < HB; ++b) {
-        const int h = HEADS == 1 ? 0 : 4 * b + (lane & 3);
-        const bool ok = h < nh;
-        const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (ok ? h : 0)) * d;
-        slope[b] = (slopes && ok) ? slopes[h0 + h] : 0.f;
-        if constexpr (F32) {
+        for (int b = 0; b < HB; ++b) {
+            const int h = HEADS == 1 ? 0 : 4 * b + (lane & 3);
+            const bool ok = h < nh;
+            const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (ok ? h : 0)) * d;
+            auto four = [&](int c) {
+                if constexpr (ROT) return *reinterpret_cast<const wa_f32x4_t*>(&qs[(ok ? h : 0) * d + c]);
+                else return *reinterpret_cast<const wa_f32x4_t*>(qr + c);
+            };
+            slope[b] = (slopes && ok) ? slopes[h0 + h] : 0.f;
+            if constexpr (F32) {
 #pragma unroll
-            for (int i = 0; i < NK; ++i) {
-                const wa_f32x4_t x = *reinterpret_cast<const wa_f32x4_t*>(qr + 16 * i + 4 * quad);
-                qf[b][i] = ok ? x : (wa_f32x4_t){0.f, 0.f, 0.f, 0.f};
-            }
-        } else {
-            const int s = col >> 2;
-#pragma unroll
-            for (int i = 0; i < KS; ++i) {
-                const wa_f32x4_t x0 = *reinterpret_cast<const wa_f32x4_t*>(qr + 32 * i + 8 * quad);
-                const wa_f32x4_t x1 = *reinterpret_cast<const wa_f32x4_t*>(qr + 32 * i + 8 * quad + 4);
-                uint16_t p[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    // eight bits of the significand at a time
-                    const float x = e < 4 ? x0[e & 3] : x1[e & 3];
-                    const uint32_t a = __float_as_uint(x) & 0xffff0000u;
-                    const float r1 = x - __uint_as_float(a);
-                    const uint32_t b2 = __float_as_uint(r1) & 0xffff0000u;
-                    const float r2 = r1 - __uint_as_float(b2);
-                    const uint32_t w = s == 0 ? a : s == 1 ? b2 : __float_as_uint(r2);
-                    p[e] = ok && s < 3 ? (uint16_t)(w >> 16) : (uint16_t)0;
+                for (int i = 0; i < NK; ++i) {
+                    const wa_f32x4_t x = four(16 * i + 4 * quad);
+                    qf[b][i] = ok ? x : (wa_f32x4_t){0.f, 0.f, 0.f, 0.f};
                 }
-                qb[b][i] = __builtin_bit_cast(wa_bf16x8_t, *reinterpret_cast<uint4*>(p));
+            } else {
+                const int s = col >> 2;
+#pragma unroll
+                for (int i = 0; i < KS; ++i) {
+                    const wa_f32x4_t x0 = four(32 * i + 8 * quad);
+                    const wa_f32x4_t x1 = four(32 * i + 8 * quad + 4);
+                    uint16_t p[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        // eight bits of the significand at a time
+                        const float x = e < 4 ? x0[e & 3] : x1[e & 3];
+                        const uint32_t a = __float_as_uint(x) & 0xffff0000u;
+                        const float r1 = x - __uint_as_float(a);
+                        const uint32_t b2 = __float_as_uint(r1) & 0xffff0000u;
+                        const float r2 = r1 - __uint_as_float(b2);
+                        const uint32_t w = s == 0 ? a : s == 1 ? b2 : __float_as_uint(r2);
+                        p[e] = ok && s < 3 ? (uint16_t)(w >> 16) : (uint16_t)0;
+                    }
+                    qb[b][i] = __builtin_bit_cast(wa_bf16x8_t, *reinterpret_cast<uint4*>(p));
+                }
             }
         }
-    }
+    };
+    if constexpr (!ROT) take_queries();
 
     const TileRun gt = tile_run(pos, window, keep_first, chunked);
     const int* bt = pr.block_table + (int64_t)row * pr.bt_stride;
@@ -1940,18 +1980,14 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
         j = first + (col < cnt ? col : 0);
         page_no = bt[j / pr.page];
     };
-    locate(split * NW + wv);
-    // (behind the page's request: the length in front of it would be one more trip to memory)
-    if (max_len > 0 && row_len[row] > max_len) return;   // the tiled kernel's rows
-    if (split * NW >= gt.n) return;                      // no keys for this split
-    for (int u = split * NW + wv; u < gt.n; u += NW * splits) {
+    uint4 kq[NK];
+    uint32_t vq[4][VW];
+    unsigned vslot[4];
+    auto fetch = [&] {
         const unsigned slot = (unsigned)page_no * (unsigned)pr.page + (unsigned)(j % pr.page);
         const T_* kr = kc + ((uint64_t)slot * G + g) * d;
-        uint4 kq[NK];
-        uint32_t vq[4][VW];
 #pragma unroll
         for (int i = 0; i < NK; ++i) kq[i] = ld16(kr + (F32 ? 16 * i + 4 * quad : 32 * i + 8 * quad));
-        unsigned vslot[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) vslot[k] = (unsigned)__shfl((int)slot, 4 * quad + k, 64);   // (lanes 0 - 15: keys in order)
 #pragma unroll
@@ -1973,6 +2009,68 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
 #pragma unroll
                 for (int w = 0; w < VW; ++w) vq[k][w] = vr[w];
             }
+        }
+    };
+    locate(split * NW + wv);
+    // (behind the page's request: the length in front of it would be one more trip to memory)
+    if (!ROT && max_len > 0 && row_len[row] > max_len) return;   // the tiled kernel's rows
+    if (split * NW >= gt.n) return;                      // no keys for this split
+    if constexpr (ROT) {
+        if (split * NW + wv < gt.n) fetch();
+        // heads 0 .. nh - 1 of q, then the key
+        for (int hh = wv; hh <= nh; hh += NW) {
+            const bool key = hh == nh;
+            const float* p = key ? ra.k_new + (int64_t)t * ldq + (int64_t)g * d : q + (int64_t)t * ldq + (int64_t)(h0 + hh) * d;
+            const float* bias = key ? (ra.k_bias ? ra.k_bias + (int64_t)g * d : nullptr)
+                                    : (ra.q_bias ? ra.q_bias + (int64_t)(h0 + hh) * d : nullptr);
+            int64_t at = -1;                             // the key's place in the pages, for the one that stores it
+            if (key && split == 0 && grp == 0) {
+                const int pg = bt[pos / pr.page];
+                if (pg >= 0) at = (((int64_t)pg * pr.page + pos % pr.page) * G + g) * d;
+            }
+            auto put = [&](int c, float turned, float plain) {
+                if (!key) {
+                    qs[hh * d + c] = turned;
+                    return;
+                }
+                ActS<F32>::st(kn + c, turned);
+                ActS<F32>::st(vn + c, plain);
+                if (at >= 0) {
+                    ActS<F32>::st((T_*)kc_ + at + c, turned);
+                    ActS<F32>::st((T_*)vc_ + at + c, plain);
+                }
+            };
+            const int half = ra.rot / 2;
+            for (int i = lane; i < half; i += 64) {
+                const int a = ra.adjacent ? 2 * i : i, b = ra.adjacent ? 2 * i + 1 : i + half;
+                const float x0 = bias ? p[a] + bias[a] : p[a], x1 = bias ? p[b] + bias[b] : p[b];
+                const double ang = (double)pos * ra.inv_freq[i];
+                const float cs = (float)cos(ang), sn = (float)sin(ang);
+                put(a, x0 * cs - x1 * sn, x0);
+                put(b, x1 * cs + x0 * sn, x1);
+            }
+            for (int c = ra.rot + lane; c < d; c += 64) {
+                const float x0 = bias ? p[c] + bias[c] : p[c];
+                put(c, x0, x0);
+            }
+        }
+        __syncthreads();
+        take_queries();
+    }
+    for (int u = split * NW + wv; u < gt.n; u += NW * splits) {
+        if constexpr (ROT) {
+            if (j == pos) {
+#pragma unroll
+                for (int i = 0; i < NK; ++i) kq[i] = *reinterpret_cast<const uint4*>(kn + (F32 ? 16 * i + 4 * quad : 32 * i + 8 * quad));
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (first + 4 * quad + k == pos && u >= gt.nk) {
+#pragma unroll
+                    for (int w = 0; w < VW; ++w) vq[k][w] = reinterpret_cast<const uint32_t*>(vn)[col * VW + w];
+                }
+        } else {
+            fetch();
         }
         wa_f32x4_t sc[HB];
 #pragma unroll
@@ -2000,10 +2098,11 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
                 const bool bad = h < nh && !(sc[b][0] == sc[b][0] && sc[b][1] == sc[b][1] &&
                                           sc[b][2] == sc[b][2] && sc[b][3] == sc[b][3]);
                 if (__any(bad)) {
-                    const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (h < nh ? h : 0)) * d;
+                    const float* qr = ROT ? qs + (h < nh ? h : 0) * d : q + (int64_t)t * ldq + (int64_t)(h0 + (h < nh ? h : 0)) * d;
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const T_* kp = kc + ((uint64_t)vslot[k] * G + g) * d;
+                        if (ROT && first + (4 * quad + k < cnt ? 4 * quad + k : 0) == pos) kp = kn;
                         float dot = 0.f;
 #pragma unroll 1
                         for (int c = 0; c < d; ++c) dot = fmaf(qr[c], ActS<F32>::ld(kp + c), dot);
@@ -2063,6 +2162,9 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
                 }
         }
         locate(u + NW * splits);
+        if constexpr (ROT) {
+            if (u + NW * splits < gt.n) fetch();
+        }
     }
     const int nact = gt.n - split * NW < NW ? gt.n - split * NW : NW;   // waves with a tile
     if (wv < nact) {
@@ -2908,6 +3010,30 @@ int mv_qkv_headnorm_rotary_store(float* qkv, int64_t ld, const float* q_bias, co
     return check_launch();
 }
 
+// Sixteen waves (eight where the registers of fp32 rows or of eight heads allow no more) while every workgroup has
+// a compute unit to itself, else four.  One split while the window is up to 1280 keys, five tiles to a wave (640
+// with fp32 rows, twice as long to read, and with eight waves): a merge is a launch more, 2 of 10 us at 45 keys.
+// Past that one to 256 keys of the window, but no more workgroups than compute units, where a second round of
+// them costs more than the splits give.  One token of bf16 at 2000 keys, window 2047, in one split and in eight
+// (us): 8 heads of 128 on 2 29.6, 16.9; 16 on 2 51.8, 21.0; 8 heads of 64 on 8 18.6, 11.2 (in 64-key tiles 27.3, 34.8, 13.5);
+// 32 tokens at 4000, 16 heads on 2, in one, four and eight splits 56.5, 28.3, 41.0; one fp32 token at 1100, window 1024, 8 heads on
+// 2, in one, two and four splits 27.3, 21.8, 17.9.
+struct FewPlan {
+    int64_t groups;      // workgroups of a split
+    int pieces, top;     // splits; query heads of a workgroup
+    bool wide;
+};
+static FewPlan few_plan(int tokens, int heads, int kv_heads, int window, int keep_first, int f32, int splits) {
+    const int R = heads / kv_heads, ngrp = (R + mv::kGrpMax - 1) / mv::kGrpMax, top = R < mv::kGrpMax ? R : mv::kGrpMax;
+    const int64_t groups = (int64_t)tokens * kv_heads * ngrp;
+    const int64_t keys = (int64_t)window + keep_first, room = mv::num_cus() / groups;
+    int64_t want = keys <= (f32 || top > 4 ? 640 : 1280) ? 1 : (keys + 128) / 256;
+    if (want > room) want = room;
+    if (want > splits) want = splits;
+    const int pieces = want < 1 ? 1 : (int)want;
+    return FewPlan{groups, pieces, top, groups * pieces <= mv::num_cus()};
+}
+
 int mv_window_attn_splits(int tokens, int heads, int kv_heads, int window, int keep_first) {
     using namespace mv;
     if (tokens <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || window <= 0 || keep_first < 0) return 1;
@@ -2975,26 +3101,15 @@ int mv_window_attn(const float* q, int64_t ldq, const void* k_cache, const void*
 #undef MV_WA_MERGE
         };
         if (aligned16(q) && ldq % 4 == 0 && aligned16(k_cache) && aligned16(v_cache)) {
-            // Sixteen waves (eight where the registers of fp32 rows or of eight heads allow no more) while every workgroup has
-            // a compute unit to itself, else four.  One split while the window is up to 1280 keys, five tiles to a wave (640
-            // with fp32 rows, twice as long to read, and with eight waves): a merge is a launch more, 2 of 10 us at 45 keys.
-            // Past that one to 256 keys of the window, but no more workgroups than compute units, where a second round of
-            // them costs more than the splits give.  One token of bf16 at 2000 keys, window 2047, in one split and in eight
-            // (us): 8 heads of 128 on 2 29.6, 16.9; 16 on 2 51.8, 21.0; 8 heads of 64 on 8 18.6, 11.2 (in 64-key tiles 27.3, 34.8, 13.5);
-            // 32 tokens at 4000, 16 heads on 2, in one, four and eight splits 56.5, 28.3, 41.0; one fp32 token at 1100, window 1024, 8 heads on
-            // 2, in one, two and four splits 27.3, 21.8, 17.9.
-            const int64_t groups = (int64_t)tokens * kv_heads * ngrp;
-            const int64_t keys = (int64_t)window + keep_first, room = num_cus() / groups;
-            int64_t want = keys <= (f32 || top > 4 ? 640 : 1280) ? 1 : (keys + 128) / 256;
-            if (want > room) want = room;
-            if (want > splits) want = splits;
-            const int pieces = want < 1 ? 1 : (int)want;
-            const bool wide = groups * pieces <= num_cus();
+            const FewPlan fp = few_plan(tokens, heads, kv_heads, window, keep_first, f32, splits);
+            const int64_t groups = fp.groups;
+            const int pieces = fp.pieces;
+            const bool wide = fp.wide;
             int nw = 0;      // (0: a head shape without an instance)
 #define MV_WA_FEW(F32_, HB_, NW_, KS_, VE_)                                                                            \
     hipLaunchKernelGGL((window_attn_few_kernel<F32_, HB_, NW_, KS_, VE_>), dim3((unsigned)groups, pieces), dim3(64 * NW_), 0, s, \
                        q, ldq, k_cache, v_cache, out, ldo, part, pr, slopes, sinks, heads, kv_heads, scale, window, keep_first, \
-                       row_len, skip_len, pieces, gate, ldg, chunked);                                                 \
+                       row_len, skip_len, pieces, gate, ldg, chunked, StepRotary{});                                   \
     nw = NW_
 #define MV_WA_FEW_HB(F32_, KS_, VE_)                                                                                   \
     do {                                                                                                               \
@@ -3056,6 +3171,69 @@ int mv_window_attn(const float* q, int64_t ldq, const void* k_cache, const void*
     } else {
         if (f32) hipLaunchKernelGGL((window_attn_kernel<true, 4>), grid, dim3(256), lds, s, q, ldq, k_cache, v_cache, out, ldo, pr, slopes, tokens, heads, kv_heads, d, dv, scale, window, row_len, skip_len, keep_first, sinks, gate, ldg, chunked);
         else hipLaunchKernelGGL((window_attn_kernel<false, 4>), grid, dim3(256), lds, s, q, ldq, k_cache, v_cache, out, ldo, pr, slopes, tokens, heads, kv_heads, d, dv, scale, window, row_len, skip_len, keep_first, sinks, gate, ldg, chunked);
+    }
+    return check_launch();
+}
+
+// The launches of a step of single tokens that mv_rotary_window_attn has a form for: head shapes with an instance, and few enough
+// tokens that every workgroup has a compute unit to itself (the waves that turn the heads are the sixteen, or eight, of that form).
+int mv_rotary_window_attn_ok(int tokens, int heads, int kv_heads, int d, int dv, int rot, int window, int keep_first, int splits,
+                             int f32) {
+    using namespace mv;
+    if (tokens <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || d != dv || (d != 128 && d != 64) || rot < 0 || rot > d ||
+        rot % 2 || window <= 0 || keep_first < 0 || splits < 1)
+        return 0;
+    const FewPlan fp = few_plan(tokens, heads, kv_heads, window, keep_first, f32, splits);
+    return fp.wide && !(f32 && fp.top == 1 && d == 128);   // sixteen waves of fp32 rows of 128: the registers of the turning spill
+}
+
+int mv_rotary_window_attn(const float* qk, int64_t ld, const float* q_bias, const float* k_bias, const double* inv_freq, int rot,
+                          int adjacent, void* k_cache, void* v_cache, void* out, int64_t ldo, const int32_t* tok_row,
+                          const int32_t* tok_pos, const int32_t* block_table, int bt_stride, int page, int tokens, int heads,
+                          int kv_heads, int d, int dv, float scale, int window, int keep_first, const float* sinks, float* part,
+                          int splits, const float* act_in, int64_t lda, void* act_out, int64_t ldao, int act_n, int act_kind,
+                          float act_limit, float act_slope, int f32, mv_stream_t stream) {
+    using namespace mv;
+    if (tokens < 0 || page <= 0 || ld < (int64_t)(heads + kv_heads) * d) return MV_ERR_INVALID_ARG;
+    if (act_in && (!act_out || act_n <= 0 || lda < 2 * (int64_t)act_n || ldao < act_n || act_kind < 0 || act_kind > 2))
+        return MV_ERR_INVALID_ARG;
+    if (tokens == 0) return MV_OK;
+    if (!mv_rotary_window_attn_ok(tokens, heads, kv_heads, d, dv, rot, window, keep_first, splits, f32)) return MV_ERR_UNSUPPORTED;
+    if (!qk || !k_cache || !v_cache || !out || !part || (rot > 0 && !inv_freq) || !tok_row || !tok_pos || !block_table)
+        return MV_ERR_INVALID_ARG;
+    if (!aligned16(k_cache) || !aligned16(v_cache)) return MV_ERR_UNSUPPORTED;
+    const FewPlan fp = few_plan(tokens, heads, kv_heads, window, keep_first, f32, splits);
+    const int nw = fp.top <= 1 ? 16 : fp.top <= 4 ? (f32 ? 8 : 16) : 8;
+    const int64_t act_blocks = act_in ? (int64_t)tokens * ((act_n + 64 * nw - 1) / (64 * nw)) : 0;
+    if (fp.groups + act_blocks > 0x7fffffff) return MV_ERR_UNSUPPORTED;
+    PagedRows pr{tok_row, tok_pos, block_table, bt_stride, page};
+    const StepRotary ra{q_bias, qk + (int64_t)heads * d, k_bias, inv_freq, rot, adjacent, (unsigned)fp.groups, act_in, act_out, lda, ldao,
+                        act_n, act_kind, act_limit, act_slope};
+    hipStream_t s = (hipStream_t)stream;
+#define MV_RWA(F32_, HB_, NW_, KS_, VE_)                                                                               \
+    hipLaunchKernelGGL((window_attn_few_kernel<F32_, HB_, NW_, KS_, VE_, true>), dim3((unsigned)(fp.groups + act_blocks), fp.pieces), \
+                       dim3(64 * NW_), 0, s, qk, ld, k_cache, v_cache, out, ldo, part, pr, (const float*)nullptr, sinks, heads, kv_heads, \
+                       scale, window, keep_first, (const int*)nullptr, 0, fp.pieces, (const float*)nullptr, (int64_t)0, 0, ra)
+#define MV_RWA_HB(F32_, KS_, VE_)                                                                                      \
+    do {                                                                                                               \
+        if (fp.top > 4) MV_RWA(F32_, 8, 8, KS_, VE_);                                                                  \
+        else if (fp.top > 1) MV_RWA(F32_, 4, (F32_ ? 8 : 16), KS_, VE_);                                               \
+        else MV_RWA(F32_, 1, 16, KS_, VE_);                                                                            \
+    } while (0)
+    if (f32) {
+        if (d == 128 && fp.top > 4) MV_RWA(true, 8, 8, 4, 8);
+        else if (d == 128) MV_RWA(true, 4, 8, 4, 8);
+        else MV_RWA_HB(true, 2, 4);
+    } else {
+        if (d == 128) MV_RWA_HB(false, 4, 8);
+        else MV_RWA_HB(false, 2, 4);
+    }
+#undef MV_RWA_HB
+#undef MV_RWA
+    if (fp.pieces > 1) {
+        const dim3 grid((unsigned)(tokens * heads));
+        if (f32) hipLaunchKernelGGL(window_attn_merge_kernel<true>, grid, dim3(64), 0, s, part, out, ldo, tok_row, tok_pos, sinks, heads, dv, fp.pieces, nw, window, keep_first, 0, (const int*)nullptr, 0, (const float*)nullptr, (int64_t)0);
+        else hipLaunchKernelGGL(window_attn_merge_kernel<false>, grid, dim3(64), 0, s, part, out, ldo, tok_row, tok_pos, sinks, heads, dv, fp.pieces, nw, window, keep_first, 0, (const int*)nullptr, 0, (const float*)nullptr, (int64_t)0);
     }
     return check_launch();
 }

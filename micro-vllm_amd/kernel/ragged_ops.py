@@ -366,6 +366,45 @@ def qk_rotary_store(qk, q_bias, k_bias, k_cache, v_cache, inv_freq, step, heads:
         float(slope), _is_f32(k_cache), nv.stream_ptr()))
 
 
+def rotary_window_attn(qk, q_bias, k_bias, k_cache, v_cache, inv_freq, out, step, heads: int, kv_heads: int, d: int, rot: int,
+                       scale: float, window: int, keep_first: int = 0, sinks=None, part=None, splits: int = 0,
+                       adjacent: bool = True, act=None) -> bool:
+    """`qk_rotary_store` and the `window_attn` behind it in one launch, for a step of one token a row; the same results, but the
+    queries in qk stay as projected.  False, and nothing done, where there is no such launch."""
+    tokens = qk.shape[0]
+    if part is None or step.tokens != step.rows or not nv.lib().mv_rotary_window_attn_ok(
+            tokens, heads, kv_heads, d, d, rot, int(window), int(keep_first), int(splits), _is_f32(k_cache)):
+        return False
+    a_in = a_out = None
+    n_act = kind = 0
+    limit = slope = 0.0
+    if act is not None:
+        a_in, a_out, kind, limit, slope = act
+        n_act = a_out.shape[1]
+        assert a_in.shape == (tokens, 2 * n_act) and a_out.shape[0] == tokens and a_out.dtype == k_cache.dtype
+    assert qk.shape[1] == (heads + kv_heads) * d and step.tokens == tokens
+    assert out.shape == (tokens, heads * d) and out.dtype == k_cache.dtype
+    assert sinks is None or (sinks.numel() == heads and sinks.is_contiguous())
+    assert part.is_contiguous() and part.numel() >= tokens * heads * splits * (d + 2)
+    page = k_cache.shape[1]
+    assert k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.dtype == v_cache.dtype
+    assert k_cache.shape[1:] == (page, kv_heads, d) and v_cache.shape == k_cache.shape
+    assert int(step.max_page) < k_cache.shape[0] and page == step.page
+    assert q_bias is None or (q_bias.numel() == heads * d and q_bias.is_contiguous())
+    assert k_bias is None or (k_bias.numel() == kv_heads * d and k_bias.is_contiguous())
+    assert rot == 0 or (inv_freq.is_cuda and inv_freq.dtype == torch.float64 and inv_freq.numel() == rot // 2)
+    nv.check("mv_rotary_window_attn", nv.lib().mv_rotary_window_attn(
+        _f32(qk).data_ptr(), _ld(qk), None if q_bias is None else _f32(q_bias).data_ptr(),
+        None if k_bias is None else _f32(k_bias).data_ptr(), None if rot == 0 else inv_freq.data_ptr(), rot, int(adjacent),
+        k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), _ld(out), step.tok_row.data_ptr(), step.tok_pos.data_ptr(),
+        step.block_table.data_ptr(), step.block_table.stride(0), page, tokens, heads, kv_heads, d, d, float(scale), int(window),
+        int(keep_first), None if sinks is None else _f32(sinks).data_ptr(), _f32(part).data_ptr(), int(splits),
+        None if a_in is None else _f32(a_in).data_ptr(), 0 if a_in is None else _ld(a_in),
+        None if a_in is None else a_out.data_ptr(), 0 if a_in is None else _ld(a_out), int(n_act), int(kind), float(limit),
+        float(slope), _is_f32(k_cache), nv.stream_ptr()))
+    return True
+
+
 def window_attn(q, k_cache, v_cache, out, step, slopes, heads: int, kv_heads: int, d: int, dv: int,
                 scale: float, window: int, tiled: bool = True, keep_first: int = 0, sinks=None, part=None, splits: int = 0,
                 gate=None, chunked: bool = False):

@@ -559,3 +559,56 @@ def test_infinite_keys_alone_in_their_tile(ops, f32, form, H, G, window, splits,
             want = p @ v[:, h // (H // G)]
             got = out[b, h * dv:(h + 1) * dv].cpu().double()
             assert ((got - want).abs() <= 1e-5 * 4 + (0 if f32 else 2 ** -8) * want.abs()).all(), (b, h)
+
+
+# one token a row: rotation, gate and attention in one launch are the two launches, bit for bit.  Query heads to a key/value head 1, 4, 6 and
+# 12 (two groups), both pair orders, a part of the head turned; the token's own position first of a tile, last of one, first of a page and
+# position 0; kept positions; windows cut over several workgroups; an infinite key of its own
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("H,G,d,rot,adj,window,keep,at", [
+    (8, 2, 128, 128, True, 1024, 64, (44, 0, 15, 16, 63, 64)), (6, 1, 64, 40, False, 37, 5, (200, 36, 37, 5, 1)),
+    (24, 2, 64, 64, True, 100, 0, (127, 128)), (3, 3, 64, 64, True, 1, 0, (0, 70)), (12, 1, 128, 64, False, 2047, 3, (2100, 31)),
+    (4, 4, 128, 0, True, 300, 20, (500, 16)), (8, 2, 128, 128, True, 1500, 64, (1700,))])
+def test_rotation_and_attention_in_one_launch(ops, f32, H, G, d, rot, adj, window, keep, at):
+    from micro_vllm_amd import _native as nv
+    dt = torch.float32 if f32 else torch.bfloat16
+    g = torch.Generator().manual_seed(H * 100 + d + len(at))
+    B, ff = len(at), 1100
+    from micro_vllm_amd.core.state_cache import HybridCacheManager
+    cache = HybridCacheManager(B * 36, 64, B, {0: (G, d, d)}, {}, dtype=dt, device=DEV, max_tokens=2304, max_rows=B, max_step_tokens=2304)
+    for i, n in enumerate(at):
+        if n:
+            step_of(cache, [(i, [0] * n)])
+    for c in (cache.k_caches[0], cache.v_caches[0]):
+        c.copy_(torch.randn(c.shape, generator=g))
+    st = step_of(cache, [(i, [0]) for i in range(B)])
+    inv = (5000.0 ** (-2.0 * torch.arange(max(rot // 2, 1), dtype=torch.float64) / max(rot, 1))).to(DEV)
+    proj = torch.randn(B, (H + G) * d + 2 * ff, generator=g)
+    if B > 1:
+        proj[1, H * d + 3] = math.inf
+    proj, sink = proj.to(DEV), torch.randn(H, generator=g).to(DEV)
+    qb, kb = torch.randn(H * d, generator=g).to(DEV), torch.randn(G * d, generator=g).to(DEV)
+    splits = ops.window_attn_splits(B, H, G, window, keep)
+    found = []
+    for fused in (False, True):
+        x, kc, vc = proj.clone(), cache.k_caches[0].clone(), cache.v_caches[0].clone()
+        qk, out = x[:, :(H + G) * d], torch.full((B, H * d + ff), 9.0, dtype=dt, device=DEV)
+        part = torch.full((B * H * splits * (d + 2),), float("nan"), device=DEV)
+        act = (x[:, (H + G) * d:], out[:, H * d:], ops.GATE_GELU_TANH, 0.0, 1.0)
+        if fused:
+            took = ops.rotary_window_attn(qk, qb, kb, kc, vc, inv, out[:, :H * d], st, H, G, d, rot, d ** -0.5, window, keep_first=keep,
+                                          sinks=sink, part=part, splits=splits, adjacent=adj, act=act)
+            assert took == (not (f32 and H == G and d == 128))
+            if not took:
+                return
+        else:
+            ops.qk_rotary_store(qk, qb, kb, kc, vc, inv, st, H, G, d, rot, adjacent=adj, act=act)
+            ops.window_attn(qk, kc, vc, out[:, :H * d], st, None, H, G, d, d, d ** -0.5, window, keep_first=keep, sinks=sink,
+                            part=part, splits=splits)
+        found.append((out, kc, vc))
+    for a, b in zip(*found):
+        bits = torch.int32 if f32 else torch.int16
+        assert torch.equal(a.view(bits), b.view(bits))
+    assert bool(torch.isfinite(found[0][0][0]).all())
+    # a head shape without such a launch
+    assert not nv.lib().mv_rotary_window_attn_ok(B, H, G, d, d + 1, rot, window, keep, splits, int(f32))
