@@ -1820,8 +1820,8 @@ __global__ __launch_bounds__(256) void window_attn_group_kernel(const float* q, 
 // other splits leave at once; else a split leaves (max, sum, weighted values) in `part` for window_attn_merge_kernel.
 //
 // Measured (us per call, 8 heads on 2 key/value heads, d = dv = 128, window 1024; kernel above with its 64-key tiles, five
-// splits and their merge -> here): one token bf16 at 45 keys 19.5 -> 8.0, 300 21.8 -> 11.4, 1100 23.2 -> 19.1; fp32 19.8 -> 8.1,
-// 23.6 -> 13.9, 25.1 -> 17.0; 64 tokens bf16 20.5 -> 8.3, 23.1 -> 12.1, 32.9 -> 21.2; a prompt of 333 in fp32 at 300 53.7 -> 40.
+// splits and their merge -> here): one token bf16 at 45 keys 19.5 -> 5.4, 300 21.8 -> 9.0, 1100 23.2 -> 17.2; fp32 19.8 -> 7.6,
+// 23.6 -> 13.0, 25.1 -> 17.0; 64 tokens bf16 at 300 23.1 -> 10.0; a prompt of 333 in fp32 at 300 53.7 -> 40.
 // 16 heads of 64 with keys of their own, one token 10.6 -> 4.7, 11.7 -> 7.0, 12.2 -> 11.8.
 struct TileRun {
     int lo, kept, nk, n;      // n tiles: nk of the kept positions [0, kept), then those of [lo, pos]
@@ -1875,8 +1875,8 @@ struct StepRotary {
 // qk_rotary_store_kernel forms them) while the first tiles are on their way; the turned queries lie in LDS, and the tile that holds
 // the token's own position takes key and value from there too: the page is written by the first split and read by later steps.
 // What another split reads of that place meanwhile is not used.
-// One launch in place of two (us, 8 heads of 128 on 2, a gate of 4096 beside them): one token bf16 at 45 keys 9.9 -> 6.6, 300 13.8 -> 11.6,
-// 1100 22.0 -> 20.2; fp32 10.8 -> 8.3, 16.5 -> 15.1, 20.6 -> 20.0; 8 tokens of 16 heads on 4 at 500 keys 17.0 -> 14.7.
+// One launch against two (us, 8 heads of 128 on 2, a gate of 4096 beside them): one token bf16 at 45 keys 8.3 -> 6.2, 300 11.7 -> 11.0,
+// 1100 19.5 -> 19.1; fp32 10.6 -> 8.3, 16.4 -> 15.0, 20.3 -> 19.6; 8 tokens of 16 heads on 4 at 500 keys 14.6 -> 13.3.
 template <bool F32, int HEADS, int NW, int KS, int VE, bool ROT = false>
 __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q, int64_t ldq, const void* kc_, const void* vc_,
                                                               void* out_, int64_t ldo, float* part, PagedRows pr,
@@ -1891,6 +1891,11 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     __shared__ float mm[NW * RT], ll[NW * RT];
     __shared__ __attribute__((aligned(16))) float qs[ROT ? RT * d : 4];          // ROT: turned queries, the token's own key
     __shared__ __attribute__((aligned(16))) T_ kn[ROT ? d : 8], vn[ROT ? dv : 8];   // and value
+    // bf16 keys: the queries' three parts, formed once for the workgroup: a value's split is some eight instructions, and a wave has 32
+    // values a lane to it, while what bounds a tile here is the issue slots of the waves that share a unit (one token of 8 heads on 2,
+    // 45 keys, 7.35 -> 5.45 us, 1100 19.6 -> 17.2).  A single head's are not worth the barrier (4.7 -> 5.0 at 45 keys of a launch of its own)
+    constexpr bool kShareQ = !F32 && (ROT || HEADS > 1);
+    __shared__ __attribute__((aligned(16))) uint16_t qp[kShareQ ? 3 * RT * d : 8];
     if constexpr (ROT) {
         if (blockIdx.x >= ra.units) {
             const unsigned cb = (ra.act_n + 64 * NW - 1) / (64 * NW), i = blockIdx.x - ra.units;
@@ -1916,47 +1921,68 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     wa_bf16x8_t qb[HB][F32 ? 1 : KS];
     wa_f32x4_t qf[HB][F32 ? NK : 1];
     float slope[HB];
+    // three bf16 numbers whose sum is x: eight bits of the significand at a time
+    auto part_query = [&](int at, float x) {
+        const uint32_t a = __float_as_uint(x) & 0xffff0000u;
+        const float r1 = x - __uint_as_float(a);
+        const uint32_t b2 = __float_as_uint(r1) & 0xffff0000u;
+        const float r2 = r1 - __uint_as_float(b2);
+        qp[at] = (uint16_t)(a >> 16);
+        qp[RT * d + at] = (uint16_t)(b2 >> 16);
+        qp[2 * RT * d + at] = (uint16_t)(__float_as_uint(r2) >> 16);
+    };
     auto take_queries = [&] {
 #pragma unroll
         for (int b = 0; b < HB; ++b) {
             const int h = HEADS == 1 ? 0 : 4 * b + (lane & 3);
             const bool ok = h < nh;
-            const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (ok ? h : 0)) * d;
-            auto four = [&](int c) {
-                if constexpr (ROT) return *reinterpret_cast<const wa_f32x4_t*>(&qs[(ok ? h : 0) * d + c]);
-                else return *reinterpret_cast<const wa_f32x4_t*>(qr + c);
-            };
             slope[b] = (slopes && ok) ? slopes[h0 + h] : 0.f;
             if constexpr (F32) {
+                const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (ok ? h : 0)) * d;
 #pragma unroll
                 for (int i = 0; i < NK; ++i) {
-                    const wa_f32x4_t x = four(16 * i + 4 * quad);
+                    wa_f32x4_t x;
+                    if constexpr (ROT) x = *reinterpret_cast<const wa_f32x4_t*>(&qs[(ok ? h : 0) * d + 16 * i + 4 * quad]);
+                    else x = *reinterpret_cast<const wa_f32x4_t*>(qr + 16 * i + 4 * quad);
                     qf[b][i] = ok ? x : (wa_f32x4_t){0.f, 0.f, 0.f, 0.f};
                 }
+            } else if constexpr (kShareQ) {
+                const int s = col >> 2;
+                const bool has = ok && s < 3;
+#pragma unroll
+                for (int i = 0; i < KS; ++i) {
+                    const uint4 x = *reinterpret_cast<const uint4*>(&qp[((has ? s * RT : 0) + (has ? h : 0)) * d + 32 * i + 8 * quad]);
+                    qb[b][i] = __builtin_bit_cast(wa_bf16x8_t, has ? x : make_uint4(0, 0, 0, 0));
+                }
             } else {
+                const float* qr = q + (int64_t)t * ldq + (int64_t)h0 * d;
                 const int s = col >> 2;
 #pragma unroll
                 for (int i = 0; i < KS; ++i) {
-                    const wa_f32x4_t x0 = four(32 * i + 8 * quad);
-                    const wa_f32x4_t x1 = four(32 * i + 8 * quad + 4);
+                    const wa_f32x4_t x0 = *reinterpret_cast<const wa_f32x4_t*>(qr + 32 * i + 8 * quad);
+                    const wa_f32x4_t x1 = *reinterpret_cast<const wa_f32x4_t*>(qr + 32 * i + 8 * quad + 4);
                     uint16_t p[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        // eight bits of the significand at a time
                         const float x = e < 4 ? x0[e & 3] : x1[e & 3];
                         const uint32_t a = __float_as_uint(x) & 0xffff0000u;
                         const float r1 = x - __uint_as_float(a);
                         const uint32_t b2 = __float_as_uint(r1) & 0xffff0000u;
                         const float r2 = r1 - __uint_as_float(b2);
                         const uint32_t w = s == 0 ? a : s == 1 ? b2 : __float_as_uint(r2);
-                        p[e] = ok && s < 3 ? (uint16_t)(w >> 16) : (uint16_t)0;
+                        p[e] = s < 3 ? (uint16_t)(w >> 16) : (uint16_t)0;
                     }
                     qb[b][i] = __builtin_bit_cast(wa_bf16x8_t, *reinterpret_cast<uint4*>(p));
                 }
             }
         }
     };
-    if constexpr (!ROT) take_queries();
+    if constexpr (!ROT && kShareQ) {
+        const float* qr = q + (int64_t)t * ldq + (int64_t)h0 * d;
+        for (int i = tid; i < nh * d; i += 64 * NW) part_query(i, qr[i]);
+    } else if constexpr (!ROT) {
+        take_queries();
+    }
 
     const TileRun gt = tile_run(pos, window, keep_first, chunked);
     const int* bt = pr.block_table + (int64_t)row * pr.bt_stride;
@@ -1972,19 +1998,22 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     // the tile's keys, this lane's key (lane % 16; past the last key: the first) and the place of its row
     int first, cnt, j;
     int page_no;
+    const bool pow2 = (pr.page & (pr.page - 1)) == 0;      // (uniform: a division by a number of the launch is some forty instructions)
+    const int shift = 31 - __builtin_clz(pr.page);
     auto locate = [&](int u) {
         if (u >= gt.n) u = gt.n - 1;
         first = u < gt.nk ? 16 * u : gt.lo + 16 * (u - gt.nk);
         const int end = u < gt.nk ? gt.kept - 1 : pos;
         cnt = end - first + 1 < 16 ? end - first + 1 : 16;
         j = first + (col < cnt ? col : 0);
-        page_no = bt[j / pr.page];
+        page_no = bt[pow2 ? j >> shift : j / pr.page];
     };
     uint4 kq[NK];
     uint32_t vq[4][VW];
     unsigned vslot[4];
     auto fetch = [&] {
-        const unsigned slot = (unsigned)page_no * (unsigned)pr.page + (unsigned)(j % pr.page);
+        const unsigned slot = pow2 ? ((unsigned)page_no << shift) + (unsigned)(j & (pr.page - 1))
+                                   : (unsigned)page_no * (unsigned)pr.page + (unsigned)(j % pr.page);
         const T_* kr = kc + ((uint64_t)slot * G + g) * d;
 #pragma unroll
         for (int i = 0; i < NK; ++i) kq[i] = ld16(kr + (F32 ? 16 * i + 4 * quad : 32 * i + 8 * quad));
@@ -2031,6 +2060,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
             auto put = [&](int c, float turned, float plain) {
                 if (!key) {
                     qs[hh * d + c] = turned;
+                    if constexpr (!F32) part_query(hh * d + c, turned);
                     return;
                 }
                 ActS<F32>::st(kn + c, turned);
@@ -2054,23 +2084,25 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
                 put(c, x0, x0);
             }
         }
+    }
+    if constexpr (ROT || kShareQ) {
         __syncthreads();
-        take_queries();
+        if (split * NW + wv < gt.n) take_queries();
     }
     for (int u = split * NW + wv; u < gt.n; u += NW * splits) {
-        if constexpr (ROT) {
+        if constexpr (!ROT) {
+            fetch();
+        } else if (u == gt.n - 1) {      // (uniform) the tile of the token's own position
             if (j == pos) {
 #pragma unroll
                 for (int i = 0; i < NK; ++i) kq[i] = *reinterpret_cast<const uint4*>(kn + (F32 ? 16 * i + 4 * quad : 32 * i + 8 * quad));
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                if (first + 4 * quad + k == pos && u >= gt.nk) {
+                if (first + 4 * quad + k == pos) {
 #pragma unroll
                     for (int w = 0; w < VW; ++w) vq[k][w] = reinterpret_cast<const uint32_t*>(vn)[col * VW + w];
                 }
-        } else {
-            fetch();
         }
         wa_f32x4_t sc[HB];
 #pragma unroll
