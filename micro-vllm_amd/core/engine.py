@@ -201,10 +201,14 @@ class InferenceEngine:
         for _, toks, wanted in entries:
             want += [start + int(i) for i in wanted]
             start += len(toks)
-        want_t = torch.tensor(want, dtype=torch.int32).to(self.device, non_blocking=True) if want else \
-            torch.zeros(0, dtype=torch.int32, device=self.device)
-        logits = self.runner.forward(step, self.cache_manager, want_t, residuals=residuals,
-                                     want_all=want == list(range(start)))
+        every = want == list(range(start))
+        if every and residuals is None and self.runner.replays(step):
+            want_t = None          # a recorded step leaves every row's logits: no list of them to copy to the device
+        elif want:
+            want_t = torch.tensor(want, dtype=torch.int32).to(self.device, non_blocking=True)
+        else:
+            want_t = torch.zeros(0, dtype=torch.int32, device=self.device)
+        logits = self.runner.forward(step, self.cache_manager, want_t, residuals=residuals, want_all=every)
         self.cache_manager.advance(rows)
         return logits
 

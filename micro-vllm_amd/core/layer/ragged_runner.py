@@ -531,9 +531,13 @@ class RaggedRunner:
         """Run the step; returns fp32 logits [len(want), vocab] for the token indices in `want` (int32 on
         the device; None = every token; `want_all`: the caller knows that `want` lists every token in order).
         `residuals` receives a copy of the stream after every layer run (debugging and tests)."""
-        if (self.use_graphs and residuals is None and step.tokens == step.rows <= self.max_graph_rows):
+        if residuals is None and self.replays(step):
             return self._replay(step, cache, None if want_all else want)
         return self._run(step, cache, want, residuals)
+
+    def replays(self, step: RaggedStep) -> bool:
+        """Whether a step is one of those that are recorded and replayed: one token a row, not too many rows."""
+        return self.use_graphs and step.tokens == step.rows <= self.max_graph_rows
 
     # ------------------------------------------------------------------ captured decoding steps
     def _replay(self, step: RaggedStep, cache: HybridCacheManager, want):
