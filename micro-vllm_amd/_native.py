@@ -84,6 +84,7 @@ PROTOTYPES = {
     "mv_rope_prefill": (_I, [_P, _L, _P, _L, _P, _P, _I, _L, _I, _I, _I, _P]),
     "mv_rope_store_prefill": (_I, [_P, _L, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]),
     "mv_paged_attn_prefill": (_I, [_P, _L, _P, _P, _P, _P, _I, _P, _L, _I, _I, _I, _I, _I, _I, _I, _F, _P]),
+    "mv_rope_attn_prefill": (_I, [_P, _L, _P, _P, _I, _P, _P, _I, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _I, _F, _P]),
     "mv_llama_prefill_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I]),
     "mv_llama_prefill_layers": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P,
                                      _P, _P, _P, _F, _P, _Z, _P]),

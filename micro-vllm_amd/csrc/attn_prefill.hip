@@ -83,6 +83,18 @@ static bool pf_eight_waves(int bs, int seq, int hkv, int g) {
     return seq >= kPfWideFrom;
 }
 
+// Chunks whose attention turns its own queries and keys (paged_attn_prefill_kernel, ROT) against the rotation's own launch in front of it.
+// Heads of 64: up to 128 tokens, up to 256 from four sequences on (us, two launches -> one, 32 heads on 4: 37 tokens 7.7 -> 6.7, 128 9.2 -> 8.2,
+// 256 11.9 -> 11.8; 4 x 256 14.9 -> 12.6, 16 x 64 11.6 -> 7.9).  Heads of 128, whose turning is twice the work of a workgroup that has
+// half its lanes' time: from four sequences and 2 M values of q, k and v on, where the separate launch takes as long (32 heads on 8: 37 tokens
+// 9.9 -> 10.5, 4 x 37 10.6 -> 10.9, 4 x 100 14.2 -> 13.6, 16 x 64 17.7 -> 12.3, 16 x 256 49.7 -> 42.1; 8 on 1: 4 x 256 16.4 -> 19.2, 16 x 128
+// 14.7 -> 13.6).
+static bool pf_rotates(int bs, int seq, int hq, int hkv, int d) {
+    if (pf_eight_waves(bs, seq, hkv, hq / hkv)) return false;
+    if (d == 64) return seq <= 128 || (seq <= 256 && bs >= 4);
+    return seq <= 256 && bs >= 4 && (int64_t)bs * seq * (hq + 2 * hkv) * d >= 2000000;
+}
+
 // ------------------------------------------------------------------ rotate + store
 struct RopeStoreArgs {
     uint16_t* qkv;          // [B*S][row_stride]: q heads | k heads | v heads
@@ -110,6 +122,13 @@ __device__ __forceinline__ void rope_pair(uint32_t x1, uint32_t x2, uint32_t c, 
     o2 = pack_bf16x2(c_lo + d_lo, c_hi + d_hi);
 }
 
+__device__ __forceinline__ void rope_pairs(uint4& x1, uint4& x2, const uint4& c, const uint4& s) {
+    rope_pair(x1.x, x2.x, c.x, s.x, x1.x, x2.x);
+    rope_pair(x1.y, x2.y, c.y, s.y, x1.y, x2.y);
+    rope_pair(x1.z, x2.z, c.z, s.z, x1.z, x2.z);
+    rope_pair(x1.w, x2.w, c.w, s.w, x1.w, x2.w);
+}
+
 // one thread = one 16-byte chunk pair (first half / second half) of one head of one token
 __global__ __launch_bounds__(256) void rope_store_kernel(RopeStoreArgs a) {
     const int cph = a.d >> 4;                       // chunk pairs per head
@@ -128,10 +147,7 @@ __global__ __launch_bounds__(256) void rope_store_kernel(RopeStoreArgs a) {
             const int rp = min(max(pos, 0), a.rot_max_pos - 1);
             const uint4 cv = ld16(a.cos + (int64_t)rp * (a.d >> 1) + c * 8);
             const uint4 sv = ld16(a.sin + (int64_t)rp * (a.d >> 1) + c * 8);
-            rope_pair(v1.x, v2.x, cv.x, sv.x, v1.x, v2.x);
-            rope_pair(v1.y, v2.y, cv.y, sv.y, v1.y, v2.y);
-            rope_pair(v1.z, v2.z, cv.z, sv.z, v1.z, v2.z);
-            rope_pair(v1.w, v2.w, cv.w, sv.w, v1.w, v2.w);
+            rope_pairs(v1, v2, cv, sv);
             st16(base + c * 8, v1);
             st16(base + (a.d >> 1) + c * 8, v2);
         }
@@ -171,10 +187,7 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(const uint16_t* x, int64
         uint4 v1 = ld16(src + c * 8), v2 = ld16(src + (d >> 1) + c * 8);
         const uint4 cv = ld16(cos + (int64_t)pos * (d >> 1) + c * 8);
         const uint4 sv = ld16(sin + (int64_t)pos * (d >> 1) + c * 8);
-        rope_pair(v1.x, v2.x, cv.x, sv.x, v1.x, v2.x);
-        rope_pair(v1.y, v2.y, cv.y, sv.y, v1.y, v2.y);
-        rope_pair(v1.z, v2.z, cv.z, sv.z, v1.z, v2.z);
-        rope_pair(v1.w, v2.w, cv.w, sv.w, v1.w, v2.w);
+        rope_pairs(v1, v2, cv, sv);
         st16(dst + c * 8, v1);
         st16(dst + (d >> 1) + c * 8, v2);
     }
@@ -197,12 +210,21 @@ struct PfArgs {
     int page_shift, num_pages, page;
     float scale_log2;
     float raise;            // pipelined kernel: powers of two a row's maximum may lag (0 = never)
+    // rotating form: q | k | v rows as projected, the tables, and the pages to write (k_cache, v_cache)
+    const uint16_t* cos;    // [max_pos][D/2] or null
+    const uint16_t* sin;
+    int rot_max_pos;
 };
 
 // NW waves per workgroup = 32 NW stacked query rows against every staged K/V tile: 4 (128 rows, two
 // workgroups per CU) or 8 (256 rows, one per CU: each tile fetched and stored to LDS once for twice
 // the matrix work - taken when that still leaves every CU a workgroup and a half).
-template <int D, int NW>
+//
+// ROT: what rope_store_kernel does in front of it, in the same launch and with the same arithmetic, for chunks of few tokens.  Queries
+// turn in the registers that hold them (a lane has both halves of its pairs); the chunk's own keys and values are staged from the
+// projection's rows, the keys turned on the way to LDS, and every workgroup writes those of its own query positions to their pages.
+// Each workgroup turns all the chunk's keys that it sees, so it is for chunks that few workgroups share: pf_rotates.
+template <int D, int NW, bool ROT = false>
 __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_kernel(PfArgs a) {
     constexpr int NT = NW * 64;        // threads
     constexpr int KT = 64;             // keys per LDS tile
@@ -224,10 +246,12 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     const int qb = a.nqb - 1 - (int)(blockIdx.x / per);
     const int rem = blockIdx.x % per;
     const int kvh = rem % a.hkv, b = rem / a.hkv;
-    const int p0 = max(a.start[b], 0);   // a negative start is a contract breach: treated as 0
+    // (ROT: everything is first asked for as if the chunk began at position 0, as whole prompts do, while its true start is on its way)
+    int start = ROT ? 0 : a.start[b];
+    int p0 = max(start, 0);   // a negative start is a contract breach: treated as 0
     const int i0 = qb * a.qt;
-    const int last_key = p0 + min(i0 + a.qt, a.S) - 1;   // last key any row of this block sees
-    const int ntiles = last_key / KT + 1;
+    int last_key = p0 + min(i0 + a.qt, a.S) - 1;   // last key any row of this block sees
+    int ntiles = last_key / KT + 1;
     const int32_t* bt = a.block_table + (int64_t)b * a.bt_stride;
 
     // this lane's query rows (C-layout column r of each of the wave's two tiles)
@@ -248,12 +272,19 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
         for (int ks = 0; ks < KS; ++ks)
             qf[mt][ks] = __builtin_bit_cast(bf16x8_t, ld16(qp + ks * 32));
     }
-
-    // the smallest last-key over the wave's 32 rows (its first query position; rows past S repeat S - 1)
-    int wave_min_limit = min(limit[0], limit[1]);
+    uint4 cq[2][ROT ? KS / 2 : 1], sq[2][ROT ? KS / 2 : 1];
+    auto load_turns = [&] {
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) wave_min_limit = min(wave_min_limit, __shfl_xor(wave_min_limit, o, 64));
-    wave_min_limit = __builtin_amdgcn_readfirstlane(wave_min_limit);
+        for (int mt = 0; mt < 2; ++mt) {
+            const int64_t ro = (int64_t)min(max(start + limit[mt] - p0, 0), a.rot_max_pos - 1) * (D / 2) + q * 8;
+#pragma unroll
+            for (int ks = 0; ks < KS / 2; ++ks) {
+                cq[mt][ks] = ld16(a.cos + ro + ks * 32);
+                sq[mt][ks] = ld16(a.sin + ro + ks * 32);
+            }
+        }
+    };
+    if (ROT && a.cos) load_turns();
 
     // K/V staging: thread moves vectors t + 256 j of the 64 x VPR tile
     auto tile_page = [&](int t) {
@@ -262,7 +293,46 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
         const int pg = bt[min((t * KT) >> a.page_shift, a.bt_stride - 1)];
         return (pg >= 0 && pg < a.num_pages) ? pg : 0;   // unallocated entry: stay inside the cache
     };
+    // ROT: a thread has both halves of its pairs, kr[j] and kr[j + NV / 2], and their turn; values as before
+    const uint16_t* knew = a.q + (int64_t)b * a.S * a.q_stride + (int64_t)(a.hq + kvh) * D;
+    const uint16_t* vnew = knew + (int64_t)a.hkv * D;
+    uint4 cr[ROT ? NV / 2 : 1], sr[ROT ? NV / 2 : 1];
+    int kpg[ROT ? NV / 2 : 1], vpg[ROT ? NV : 1];
+    // the page of a chunk's token that this workgroup writes, else -1 (as in rope_store_kernel)
+    auto own_page = [&](int kp, int i) {
+        const int pos = start + i;
+        if (kp > last_key || i < i0 || i >= i0 + a.qt || pos < 0 || (pos >> a.page_shift) >= a.bt_stride) return -1;
+        const int pg = bt[pos >> a.page_shift];
+        return pg < a.num_pages ? pg : -1;
+    };
     auto g_load = [&](uint4(&kr)[NV], uint4(&vr)[NV], int t, int pg) {
+        if constexpr (ROT) {
+#pragma unroll
+            for (int j = 0; j < NV / 2; ++j) {
+                const int v = threadIdx.x + NT * j, row = v / (VPR / 2), ch = v % (VPR / 2);
+                const int kp = min(t * KT + row, last_key), i = kp - p0;
+                const uint16_t* src = i >= 0 ? knew + (int64_t)i * a.q_stride
+                                             : a.k_cache + (((int64_t)pg * a.page + (kp & (a.page - 1))) * a.hkv + kvh) * D;
+                kr[j] = ld16(src + ch * 8);
+                kr[j + NV / 2] = ld16(src + D / 2 + ch * 8);
+                if (a.cos) {
+                    const int64_t ro = (int64_t)min(max(start + i, 0), a.rot_max_pos - 1) * (D / 2) + ch * 8;
+                    cr[j] = ld16(a.cos + ro);
+                    sr[j] = ld16(a.sin + ro);
+                }
+                kpg[j] = own_page(t * KT + row, t * KT + row - p0);
+            }
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int v = threadIdx.x + NT * j, row = v / VPR, ch = v % VPR;
+                const int kp = min(t * KT + row, last_key), i = kp - p0;
+                const uint16_t* src = i >= 0 ? vnew + (int64_t)i * a.q_stride
+                                             : a.v_cache + (((int64_t)pg * a.page + (kp & (a.page - 1))) * a.hkv + kvh) * D;
+                vr[j] = ld16(src + ch * 8);
+                vpg[j] = own_page(t * KT + row, t * KT + row - p0);
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int v = threadIdx.x + NT * j, row = v / VPR, ch = v % VPR;
@@ -272,7 +342,33 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
             vr[j] = ld16(a.v_cache + off);
         }
     };
-    auto l_store = [&](const uint4(&kr)[NV], const uint4(&vr)[NV], int buf) {
+    auto l_store = [&](uint4(&kr)[NV], const uint4(&vr)[NV], int t) {
+        const int buf = t & 1;
+        if constexpr (ROT) {
+            auto slot = [&](int pg, int row) {
+                const int pos = start + t * KT + row - p0;
+                return (((int64_t)pg * a.page + (pos & (a.page - 1))) * a.hkv + kvh) * D;
+            };
+#pragma unroll
+            for (int j = 0; j < NV / 2; ++j) {
+                const int v = threadIdx.x + NT * j, row = v / (VPR / 2), ch = v % (VPR / 2);
+                if (a.cos && min(t * KT + row, last_key) >= p0) rope_pairs(kr[j], kr[j + NV / 2], cr[j], sr[j]);
+                *reinterpret_cast<uint4*>(&kL[buf][row * KROW + ch * 16]) = kr[j];
+                *reinterpret_cast<uint4*>(&kL[buf][row * KROW + D + ch * 16]) = kr[j + NV / 2];
+                if (kpg[j] >= 0) {
+                    uint16_t* dst = const_cast<uint16_t*>(a.k_cache) + slot(kpg[j], row);
+                    st16(dst + ch * 8, kr[j]);
+                    st16(dst + D / 2 + ch * 8, kr[j + NV / 2]);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int v = threadIdx.x + NT * j, row = v / VPR, ch = v % VPR;
+                *reinterpret_cast<uint4*>(&vL[buf][row * VROW + ch * 16]) = vr[j];
+                if (vpg[j] >= 0) st16(const_cast<uint16_t*>(a.v_cache) + slot(vpg[j], row) + ch * 8, vr[j]);
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int v = threadIdx.x + NT * j, row = v / VPR, ch = v % VPR;
@@ -291,6 +387,37 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     uint4 kr[NV], vr[NV];
     int pg_next = tile_page(0);
     g_load(kr, vr, 0, pg_next);
+    if constexpr (ROT) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int true_start = a.start[b];
+        if (true_start != 0) {   // uniform
+            start = true_start;
+            const int moved = max(start, 0);
+            limit[0] += moved;
+            limit[1] += moved;
+            last_key += moved;
+            p0 = moved;
+            ntiles = last_key / KT + 1;
+            if (a.cos) load_turns();
+            g_load(kr, vr, 0, pg_next);
+        }
+        if (a.cos) {
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int ks = 0; ks < KS / 2; ++ks) {
+                    uint4 x1 = __builtin_bit_cast(uint4, qf[mt][ks]), x2 = __builtin_bit_cast(uint4, qf[mt][ks + KS / 2]);
+                    rope_pairs(x1, x2, cq[mt][ks], sq[mt][ks]);
+                    qf[mt][ks] = __builtin_bit_cast(bf16x8_t, x1);
+                    qf[mt][ks + KS / 2] = __builtin_bit_cast(bf16x8_t, x2);
+                }
+        }
+    }
+    // the smallest last-key over the wave's 32 rows (its first query position; rows past S repeat S - 1)
+    int wave_min_limit = min(limit[0], limit[1]);
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) wave_min_limit = min(wave_min_limit, __shfl_xor(wave_min_limit, o, 64));
+    wave_min_limit = __builtin_amdgcn_readfirstlane(wave_min_limit);
     pg_next = ntiles > 1 ? tile_page(1) : 0;
     l_store(kr, vr, 0);
     __syncthreads();
@@ -418,7 +545,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
                     oacc[mt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[mt][h], oacc[mt][dt], 0, 0, 0);
             }
         }
-        if (more) l_store(kr, vr, buf ^ 1);
+        if (more) l_store(kr, vr, t + 1);
         __syncthreads();
     }
 
@@ -980,10 +1107,11 @@ int mv_paged_attn_prefill_form(int bs, int seq, int hq, int hkv) {
     return mv::pf_eight_waves(bs, seq, hkv, hq / hkv) ? 8 : 4;
 }
 
-int mv_paged_attn_prefill(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
-                          const int32_t* cache_seqlens, const int32_t* block_table, int bt_stride,
-                          void* out, int64_t out_stride, int bs, int seq, int hq, int hkv, int d,
-                          int page, int num_pages, float scale, mv_stream_t stream) {
+static int attn_prefill(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+                        const int32_t* cache_seqlens, const int32_t* block_table, int bt_stride,
+                        void* out, int64_t out_stride, int bs, int seq, int hq, int hkv, int d,
+                        int page, int num_pages, float scale, bool rotates, const void* rot_cos, const void* rot_sin,
+                        int rot_max_pos, mv_stream_t stream) {
     using namespace mv;
     if (bs == 0 || seq == 0) return MV_OK;
     if (!q || !k_cache || !v_cache || !cache_seqlens || !block_table || !out) return MV_ERR_INVALID_ARG;
@@ -1025,12 +1153,19 @@ int mv_paged_attn_prefill(const void* q, int64_t q_stride, const void* k_cache, 
     a.num_pages = num_pages;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.raise = g_pf_raise;
+    a.cos = (const uint16_t*)rot_cos;
+    a.sin = (const uint16_t*)rot_sin;
+    a.rot_max_pos = rot_max_pos;
     const int64_t grid = (int64_t)a.nqb * hkv * bs;
     if (grid > 0x7fffffffLL) return MV_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     // the pipelined form keeps a page's byte size in 32 bits and stores 16 bytes at a time
     const bool pipe = eight && g_pf_pipe && (int64_t)page * hkv * d * 2 < (1LL << 32) && (out_stride % 8) == 0;
-    if (d == 128 && pipe)
+    if (rotates && d == 128)
+        hipLaunchKernelGGL((paged_attn_prefill_kernel<128, 4, true>), dim3((unsigned)grid), dim3(256), 0, st, a);
+    else if (rotates)
+        hipLaunchKernelGGL((paged_attn_prefill_kernel<64, 4, true>), dim3((unsigned)grid), dim3(256), 0, st, a);
+    else if (d == 128 && pipe)
         hipLaunchKernelGGL((paged_attn_prefill_pipe_kernel<128>), dim3((unsigned)grid), dim3(512), 0, st, a);
     else if (pipe)
         hipLaunchKernelGGL((paged_attn_prefill_pipe_kernel<64>), dim3((unsigned)grid), dim3(512), 0, st, a);
@@ -1043,6 +1178,32 @@ int mv_paged_attn_prefill(const void* q, int64_t q_stride, const void* k_cache, 
     else
         hipLaunchKernelGGL((paged_attn_prefill_kernel<64, 4>), dim3((unsigned)grid), dim3(256), 0, st, a);
     return check_launch();
+}
+
+int mv_paged_attn_prefill(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
+                          const int32_t* cache_seqlens, const int32_t* block_table, int bt_stride,
+                          void* out, int64_t out_stride, int bs, int seq, int hq, int hkv, int d,
+                          int page, int num_pages, float scale, mv_stream_t stream) {
+    return attn_prefill(q, q_stride, k_cache, v_cache, cache_seqlens, block_table, bt_stride, out, out_stride, bs, seq, hq, hkv, d,
+                        page, num_pages, scale, false, nullptr, nullptr, 0, stream);
+}
+
+int mv_rope_attn_prefill(void* qkv, int64_t row_stride, const void* rot_cos, const void* rot_sin, int rot_max_pos,
+                         const int32_t* cache_seqlens, const int32_t* block_table, int bt_stride, void* k_cache, void* v_cache,
+                         void* out, int64_t out_stride, int bs, int seq, int hq, int hkv, int d, int page, int num_pages,
+                         float scale, mv_stream_t stream) {
+    using namespace mv;
+    // the one launch where it is the faster form and takes the operands; else, and with operands that are wrong, the two
+    const bool rotates = bs > 0 && seq > 0 && hkv > 0 && hq > 0 && hq % hkv == 0 && hq / hkv <= 8 && (d == 64 || d == 128) &&
+                         pf_rotates(bs, seq, hq, hkv, d) && row_stride >= (int64_t)(hq + 2 * hkv) * d &&
+                         (rot_cos == nullptr) == (rot_sin == nullptr) && (!rot_cos || (rot_max_pos > 0 && aligned16(rot_cos) && aligned16(rot_sin)));
+    if (!rotates) {
+        const int rc = mv_rope_store_prefill(qkv, row_stride, rot_cos, rot_sin, rot_max_pos, cache_seqlens, block_table, bt_stride,
+                                             k_cache, v_cache, bs, seq, hq, hkv, d, page, num_pages, stream);
+        if (rc != MV_OK) return rc;
+    }
+    return attn_prefill(qkv, row_stride, k_cache, v_cache, cache_seqlens, block_table, bt_stride, out, out_stride, bs, seq, hq, hkv, d,
+                        page, num_pages, scale, rotates, rot_cos, rot_sin, rot_max_pos, stream);
 }
 
 }  // extern "C"

@@ -57,11 +57,9 @@ extern "C" int mv_llama_prefill_layers(const void* const* tensors, const float* 
         if (!normed_done) rc = mv_rmsnorm(h, t[kLn1], normed, T, hidden, hidden, hidden, eps[2 * li], stream);
         if (rc == MV_OK) rc = project(normed, hidden, t[kWqkv], t[kBqkv], nullptr, qkv, nqkv, nqkv, 0, nullptr);
         if (rc == MV_OK)
-            rc = mv_rope_store_prefill(qkv, nqkv, rot_cos, rot_sin, rot_max_pos, cache_seqlens, block_table, bt_stride,
-                                       (void*)t[kKcache], (void*)t[kVcache], rows, seq, hq, hkv, d, page, num_pages, stream);
-        if (rc == MV_OK)
-            rc = mv_paged_attn_prefill(qkv, nqkv, t[kKcache], t[kVcache], cache_seqlens, block_table, bt_stride, attn, nq, rows, seq,
-                                       hq, hkv, d, page, num_pages, scale, stream);
+            rc = mv_rope_attn_prefill(qkv, nqkv, rot_cos, rot_sin, rot_max_pos, cache_seqlens, block_table, bt_stride,
+                                      (void*)t[kKcache], (void*)t[kVcache], attn, nq, rows, seq, hq, hkv, d, page, num_pages, scale,
+                                      stream);
         if (rc != MV_OK) break;
         // resid = attention's projection + h with its norm (over the unrounded sum, as mv_rmsnorm_residual takes it)
         PostNorm ln2 = {h, resid, t[kLn2], eps[2 * li + 1], normed, hidden, 0, (float*)proj, false};
