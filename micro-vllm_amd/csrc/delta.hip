@@ -11,6 +11,8 @@
 // All of it in fp32; only what goes to a projection is of the activation type.
 #include "recurrence.h"
 
+#include <type_traits>
+
 namespace mv {
 
 struct DeltaRows {
@@ -421,10 +423,40 @@ constexpr int kDCh = 64;
 // as slabs of 16 columns, bm [64][64], gc [n16]
 constexpr int kIntra = 512;      // threads of the intra kernel: two waves a SIMD, one workgroup a compute unit
 
+// the value of lane T of each row of 16 lanes, in all of them
+template <int T>
+__device__ __forceinline__ float row_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + T, 0xF, 0xF, true));
+}
+// acc + a.w b.w + a.z b.z + a.y b.y + a.x b.x, fused one by one, a that of lane T of the row.  (The compiler folds the exchange into a
+// product, but not into a fused one: a move each.  It cannot see into the block, so the two cycles that an exchange has to keep from a
+// write of its operand stand in it.)
+template <int T>
+__device__ __forceinline__ void add_row_lane(float& acc, const f32x4_t& a, const f32x4_t& b) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %2, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %7 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc)
+        : "v"(a[3]), "v"(a[2]), "v"(a[1]), "v"(a[0]), "v"(b[3]), "v"(b[2]), "v"(b[1]), "v"(b[0]), "n"(T));
+}
+template <int T0, typename F>
+__device__ __forceinline__ void for_tokens(F&& f) {      // f(T0) .. f(T0 + 7), the number a constant
+    f(std::integral_constant<int, T0>{});
+    f(std::integral_constant<int, T0 + 1>{});
+    f(std::integral_constant<int, T0 + 2>{});
+    f(std::integral_constant<int, T0 + 3>{});
+    f(std::integral_constant<int, T0 + 4>{});
+    f(std::integral_constant<int, T0 + 5>{});
+    f(std::integral_constant<int, T0 + 6>{});
+    f(std::integral_constant<int, T0 + 7>{});
+}
+
 __global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int ch = blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
-    const int wv = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, g = lane >> 4;
     const int n = a.n, p = a.p, N = pad16(n), P = pad16(p), SN = N + 4;
     float* Q = lds;                      // raw q, then q * (product of the gates from the block's start)
     float* Kp = Q + kDCh * SN;           // raw k, then the same for k
@@ -436,68 +468,102 @@ __global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) 
     const int start = a.ch_start[ch], len = a.ch_len[ch], kh = h / (a.H / a.K);
     const int64_t unit = (int64_t)ch * a.H + h;
     const float neg_a = -expf(a.a_log[h]);
-    constexpr int kB = 8;            // loads in flight together (addresses clamped, values selected afterwards)
+    // A value's place goes on by kIntra from one of a thread's values to the next: row and column by additions, rows as 32-bit offsets
+    // from the chunk's first.  (A division by N and a 64-bit product a value, with the gates' own functions, were half of what a lone chunk took.)
+    constexpr int kB = 16;           // loads in flight together (addresses clamped, values selected afterwards)
+    const int dt = kIntra / N, dc = kIntra - dt * N;
+    int t_ = tid / N, c_ = tid - t_ * N;
+    const char* qk0 = reinterpret_cast<const char*>(a.qkv + (int64_t)start * a.ldq + (int64_t)kh * n);
+    const char* kk0 = qk0 + (int64_t)a.K * n * 4;
+    const char* ga0 = reinterpret_cast<const char*>(a.a + (int64_t)start * a.lda + (int64_t)h * n);
+    const float* db0 = a.dt_bias + (int64_t)h * n;
     for (int i0 = tid; i0 < kDCh * N; i0 += kIntra * kB) {
         float q_[kB], k_[kB], a_[kB], b_[kB];
+        const int t0 = t_, c0 = c_;
 #pragma unroll
         for (int u = 0; u < kB; ++u) {
-            const int i = i0 + kIntra * u, t = i / N, c = i - t * N;
-            const int64_t tok = start + (t < len ? t : len - 1);
-            const int cc = c < n ? c : n - 1;
-            const float* qp = a.qkv + tok * a.ldq + (int64_t)kh * n + cc;
-            q_[u] = qp[0];
-            k_[u] = qp[(int64_t)a.K * n];
-            a_[u] = a.a[tok * a.lda + (int64_t)h * n + cc];
-            b_[u] = a.dt_bias[(int64_t)h * n + cc];
+            const int t = t_ < len ? t_ : len - 1, cc = c_ < n ? c_ : n - 1;
+            const uint32_t at = ((uint32_t)t * (uint32_t)a.ldq + (uint32_t)cc) * 4u;
+            q_[u] = *reinterpret_cast<const float*>(qk0 + at);
+            k_[u] = *reinterpret_cast<const float*>(kk0 + at);
+            a_[u] = *reinterpret_cast<const float*>(ga0 + ((uint32_t)t * (uint32_t)a.lda + (uint32_t)cc) * 4u);
+            b_[u] = db0[cc];
+            t_ += dt;
+            c_ += dc;
+            if (c_ >= N) {
+                c_ -= N;
+                ++t_;
+            }
         }
+        int t = t0, c = c0;
 #pragma unroll
         for (int u = 0; u < kB; ++u) {
-            const int i = i0 + kIntra * u, t = i / N, c = i - t * N;
-            if (t >= kDCh) continue;
-            const bool ok = t < len && c < n;
-            Q[t * SN + c] = ok ? q_[u] : 0.f;
-            Kp[t * SN + c] = ok ? k_[u] : 0.f;
-            Gn[t * SN + c] = ok ? decay_gate(a_[u], b_[u], neg_a) : 1.f;
+            if (t < kDCh) {
+                const bool ok = t < len && c < n;
+                Q[t * SN + c] = ok ? q_[u] : 0.f;
+                Kp[t * SN + c] = ok ? k_[u] : 0.f;
+                Gn[t * SN + c] = ok ? decay_gate(a_[u], b_[u], neg_a) : 1.f;
+            }
+            t += dt;
+            c += dc;
+            if (c >= N) {
+                c -= N;
+                ++t;
+            }
         }
     }
     if (tid < kDCh) bs[tid] = tid < len ? a.beta[(int64_t)(start + tid) * a.H + h] : 0.f;
     __syncthreads();
-    // diagonal blocks, A by the first four waves and B by the others: lane (r, g) holds column s = r, state rows
-    // 16 m + 4 g .. + 3
+    // diagonal blocks of A and B: lane (r, g) holds column s = r, state rows 16 m + 4 g .. + 3, and walks the tokens t behind its s.  Two waves
+    // share a block: the first takes t up to 7, the second those behind, whose first half it walks for the product alone.  A token's
+    // own values come from the lane of its row (DPP); read from LDS by all sixteen they were 33 reads a wave and step.  A lone chunk of 16 heads of
+    // 128 x 128 33.7 -> 26.5 us, 23 of them 73.6 -> 61, with the places below and the tiles' reads in front of their products.
     {
         const int blk = wv & 3;
-        const bool isb = wv >= 4;
-        float sa[16];
+        const bool late = wv >= 4;
+        float sa[8], sb[8];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) sa[t] = 0.f;
-        const float* l0 = (isb ? Q : Kp) + 16 * blk * SN + 4 * g;
-        const float* k0 = Kp + 16 * blk * SN + 4 * g;
-        const float* g0 = Gn + 16 * blk * SN + 4 * g;
+        for (int t = 0; t < 8; ++t) sa[t] = sb[t] = 0.f;
+        const float* row = Kp + (16 * blk + r) * SN + 4 * g;     // q, k and gates lie the same way
+        const int t0 = late ? 8 : 0;
         for (int m = 0; m < N; m += 16) {
-            const float4 ks = *reinterpret_cast<const float4*>(k0 + r * SN + m);
-            float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+            const f32x4_t kr = *reinterpret_cast<const f32x4_t*>(row + m);
+            const f32x4_t qr = *reinterpret_cast<const f32x4_t*>(row + m - kDCh * SN);
+            const f32x4_t gr = *reinterpret_cast<const f32x4_t*>(row + m + kDCh * SN);
+            f32x4_t w = {0.f, 0.f, 0.f, 0.f};
+            auto walk = [&](auto t) {
+                constexpr int T = decltype(t)::value;
 #pragma unroll
-            for (int t = 0; t < 16; ++t) {
-                const float4 gt = *reinterpret_cast<const float4*>(g0 + t * SN + m);
-                const float4 lt = *reinterpret_cast<const float4*>(l0 + t * SN + m);
-                const bool self = t == r;
-                w.x = self ? ks.x : w.x * gt.x;
-                w.y = self ? ks.y : w.y * gt.y;
-                w.z = self ? ks.z : w.z * gt.z;
-                w.w = self ? ks.w : w.w * gt.w;
-                sa[t] = fmaf(lt.x, w.x, fmaf(lt.y, w.y, fmaf(lt.z, w.z, fmaf(lt.w, w.w, sa[t]))));
+                for (int e = 0; e < 4; ++e) {
+                    const float on = row_lane<T>(gr[e]) * w[e];      // (in every lane: the exchange may stand under no condition)
+                    w[e] = T == r ? kr[e] : on;
+                }
+            };
+            auto add = [&](auto t) {
+                constexpr int T = decltype(t)::value;
+                walk(t);
+                add_row_lane<T>(sa[T & 7], kr, w);
+                add_row_lane<T>(sb[T & 7], qr, w);
+            };
+            if (late) {
+                for_tokens<0>(walk);
+                for_tokens<8>(add);
+            } else {
+                for_tokens<0>(add);
             }
         }
         float* bm = a.bm + unit * (kDCh * kDCh);
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            float x = sa[t];
+        for (int t = 0; t < 8; ++t) {
+            float x = sa[t], y = sb[t];
             x += __shfl_xor(x, 16, 64);
             x += __shfl_xor(x, 32, 64);
-            if ((t >> 2) == g) {
-                const int tt = 16 * blk + t;
-                if (isb) bm[tt * kDCh + 16 * blk + r] = r <= t ? x : 0.f;
-                else Am[tt * 68 + 16 * blk + r] = r < t ? -bs[tt] * x : 0.f;
+            y += __shfl_xor(y, 16, 64);
+            y += __shfl_xor(y, 32, 64);
+            if ((t & 3) == g) {      // (one of the four lanes that hold the sums)
+                const int tb = t0 + t, tt = 16 * blk + tb;
+                bm[tt * kDCh + 16 * blk + r] = r <= tb ? y : 0.f;
+                Am[tt * 68 + 16 * blk + r] = r < tb ? -bs[tt] * x : 0.f;
             }
         }
     }
@@ -529,19 +595,6 @@ __global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) 
         }
         E[blk * N + c] = pre;
     }
-    // inverses of the unit triangular diagonal blocks: lane r owns column r, forward substitution
-    if (wv < 4 && g == 0) {
-        float x[16];
-        const float* m = Am + (16 * wv) * 68 + 16 * wv;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            float s = t == r ? 1.f : 0.f;
-#pragma unroll
-            for (int j = 0; j < t; ++j) s = fmaf(m[t * 68 + j], x[j], s);
-            x[t] = s;
-            Di[(wv * 16 + t) * 20 + r] = s;
-        }
-    }
     __syncthreads();
     // blocks below the diagonal: six block pairs, A and B each
     for (int id = wv; id < 12; id += kIntra / 64) {
@@ -571,6 +624,21 @@ __global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) 
             const int t = 16 * I + 4 * g + j, s = 16 * J + r;
             if (isb) a.bm[unit * (kDCh * kDCh) + t * kDCh + s] = acc[j];
             else Am[t * 68 + s] = -bs[t] * acc[j];
+        }
+    }
+    // inverses of the unit triangular diagonal blocks, by the waves that had one pair above and not two: lane r owns column r, forward
+    // substitution
+    if (wv >= 4 && g == 0) {
+        const int blk = wv - 4;
+        float x[16];
+        const float* m = Am + (16 * blk) * 68 + 16 * blk;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            float s = t == r ? 1.f : 0.f;
+#pragma unroll
+            for (int j = 0; j < t; ++j) s = fmaf(m[t * 68 + j], x[j], s);
+            x[t] = s;
+            Di[(blk * 16 + t) * 20 + r] = s;
         }
     }
     // the wave's first 16 columns of V are under way from here on
@@ -613,27 +681,38 @@ __global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) 
     }
     for (int c = tid; c < N; c += kIntra) a.gc[unit * N + c] = ((E[c] * E[N + c]) * E[2 * N + c]) * E[3 * N + c];
     __syncthreads();
-    // the triangular system, 16 columns at a time: first those of V, then those of G * K
+    // the triangular system, 16 columns at a time: first those of V, then those of G * K.  What a tile starts from is read in one go, in front
+    // of its chain of products
     const int pt = P / 16, ntile = pt + N / 16;
     float* uv = a.uv + unit * (kDCh * P);
-    for (int tile = wv; tile < ntile; tile += kIntra / 64) {
-        const bool isv = tile < pt;
+    f32x4_t be[4];
+#pragma unroll
+    for (int I = 0; I < 4; ++I) be[I] = *reinterpret_cast<const f32x4_t*>(bs + 16 * I + 4 * g);
+    auto solve = [&](auto isv_, int tile) {
+        constexpr bool isv = decltype(isv_)::value;
         const int c = 16 * (isv ? tile : tile - pt) + r;
-        if (isv && tile != wv) load_v(tile);
-        f32x4_t X[4];
-        float e = 1.f;           // product of the blocks before I for column c of G * K
+        f32x4_t X[4], B[4];
+        if constexpr (isv) {
+#pragma unroll
+            for (int I = 0; I < 4; ++I)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int t = 16 * I + 4 * g + j;
+                    B[I][j] = be[I][j] * ((t < len && c < p) ? vv[4 * I + j] : 0.f);
+                }
+        } else {
+            float e[4];              // product of the blocks before I for column c of G * K
+            e[0] = 1.f;
+#pragma unroll
+            for (int I = 1; I < 4; ++I) e[I] = e[I - 1] * E[(I - 1) * N + c];
+#pragma unroll
+            for (int I = 0; I < 4; ++I)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) B[I][j] = be[I][j] * (Kp[(16 * I + 4 * g + j) * SN + c] * e[I]);
+        }
 #pragma unroll
         for (int I = 0; I < 4; ++I) {
-            f32x4_t acc;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int t = 16 * I + 4 * g + j;
-                float v;
-                if (isv) v = (t < len && c < p) ? vv[4 * I + j] : 0.f;
-                else v = Kp[t * SN + c] * e;
-                acc[j] = bs[t] * v;
-            }
-            if (!isv) e *= E[I * N + c];
+            f32x4_t acc = B[I];
 #pragma unroll
             for (int J = 0; J < I; ++J) {
                 const float4 m = *reinterpret_cast<const float4*>(Am + (16 * I + r) * 68 + 16 * J + 4 * g);
@@ -651,9 +730,17 @@ __global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) 
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int t = 16 * I + 4 * g + j;
-                if (isv) uv[(tile * kDCh + t) * 16 + r] = X[I][j];
+                if constexpr (isv) uv[(tile * kDCh + t) * 16 + r] = X[I][j];
                 else Q[t * SN + c] = X[I][j];          // q is not needed any more
             }
+        }
+    };
+    for (int tile = wv; tile < ntile; tile += kIntra / 64) {
+        if (tile < pt) {
+            if (tile != wv) load_v(tile);
+            solve(std::true_type{}, tile);
+        } else {
+            solve(std::false_type{}, tile);
         }
     }
     __syncthreads();
