@@ -140,36 +140,42 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     const int nchunk = seq_chunks > split ? (seq_chunks - split + a.nsplit - 1) / a.nsplit : 0;
     const bool last_split = split == filled - 1;
 
+    // q (G heads) and the new k are turned once for the workgroup, a 16-byte piece a thread, and handed over in LDS behind the states'
+    // arrays.  Each row group turning all of them for itself (G + 1 pieces a lane, some eighty instructions each) was a fifth of what a short
+    // row takes (us; 32 heads of 64 on 4: one row of 45 tokens 7.6 -> 6.1, 4000 12.2 -> 10.9, 32 rows of 2000 30.0 -> 29.2; 32 heads of 128 on
+    // 8: 45 tokens 6.2 -> 5.5, 4096 11.4 -> 10.8).
+    // A single query head is two pieces a lane, and not worth the barrier (8 heads on 8 of 128, 500 tokens: 6.95 -> 7.1 us).
+    constexpr bool kShare = G > 1;
+    constexpr int kPieces = (G + 1) * LPR;
+    static_assert(kPieces <= kAW * 64, "a thread turns one piece");
+    uint16_t* turned = reinterpret_cast<uint16_t*>(lds + 2 * NS * G + NS * G * D);   // [G + 1][D]
     const bool rotate = (a.rot_cos != nullptr);
-    const bool first_half = d0 < D / 2;
-    const int dpart = first_half ? d0 + D / 2 : d0 - D / 2;
-    uint4 qx[G], qo[G], kx, ko, vnew;
-    ko = make_uint4(0, 0, 0, 0);
+    const int piece = min((int)threadIdx.x, kPieces - 1), pseg = kShare ? piece / LPR : 0, pd = kShare ? (piece % LPR) * 8 : d0;
+    const bool first_half = pd < D / 2;
+    const int ppart = first_half ? pd + D / 2 : pd - D / 2;
+    uint4 px, po, kx, ko, vnew;      // this thread's piece and the one half a head away; kx, ko: the key's, where nothing is shared
     if (a.slabs) {
         // (the state arrays this borrows are first written after the main loop)
         uint16_t* stage = reinterpret_cast<uint16_t*>(lds);
         stage_qkv_from_slabs<D, G>(a, stage, b, kvh);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            qx[g] = *reinterpret_cast<const uint4*>(stage + g * D + d0);
-            qo[g] = rotate ? *reinterpret_cast<const uint4*>(stage + g * D + dpart) : qx[g];
+        px = *reinterpret_cast<const uint4*>(stage + pseg * D + pd);
+        po = *reinterpret_cast<const uint4*>(stage + pseg * D + ppart);
+        if (!kShare) {
+            kx = *reinterpret_cast<const uint4*>(stage + D + pd);
+            ko = *reinterpret_cast<const uint4*>(stage + D + ppart);
         }
-        kx = *reinterpret_cast<const uint4*>(stage + G * D + d0);
-        if (rotate) ko = *reinterpret_cast<const uint4*>(stage + G * D + dpart);
         vnew = *reinterpret_cast<const uint4*>(stage + (G + 1) * D + d0);
-        __syncthreads();
+        if (!kShare) __syncthreads();
     } else {
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const uint16_t* qh = a.q + (int64_t)b * a.q_stride_b + (int64_t)(kvh * G + g) * D;
-            qx[g] = ld16(qh + d0);
-            qo[g] = rotate ? ld16(qh + dpart) : qx[g];
-        }
         const uint16_t* kh = a.k_new + (int64_t)b * a.kv_stride_b + (int64_t)kvh * D;
-        const uint16_t* vh = a.v_new + (int64_t)b * a.kv_stride_b + (int64_t)kvh * D;
-        kx = ld16(kh + d0);
-        if (rotate) ko = ld16(kh + dpart);
-        vnew = ld16(vh + d0);
+        const uint16_t* ph = pseg < G ? a.q + (int64_t)b * a.q_stride_b + (int64_t)(kvh * G + pseg) * D : kh;
+        px = ld16(ph + pd);
+        po = ld16(ph + ppart);
+        if (!kShare) {
+            kx = ld16(kh + pd);
+            ko = ld16(kh + ppart);
+        }
+        vnew = ld16(a.v_new + (int64_t)b * a.kv_stride_b + (int64_t)kvh * D + d0);
     }
 
 #ifdef MV_ATTN_STAMP
@@ -187,7 +193,7 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     uint4 cosv = make_uint4(0, 0, 0, 0), sinv = cosv;
     if (rotate) {
         const int rp = min(max(pos, 0), a.rot_max_pos - 1);
-        const int64_t ro = (int64_t)rp * (D / 2) + (first_half ? d0 : d0 - D / 2);
+        const int64_t ro = (int64_t)rp * (D / 2) + (first_half ? pd : ppart);
         cosv = ld16(a.rot_cos + ro);
         sinv = ld16(a.rot_sin + ro);
     }
@@ -217,21 +223,26 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
     load_pages(pgB, 3);
     if (!kLeaveFirst && leave) return;
 
-    // ---- q (G heads) and the new k/v: rotate, round -------------------------------
-    uint32_t qp[G][4];
+    // ---- q (G heads) and the new k: rotate, round -------------------------------
+    auto turn = [&](const uint4& x, const uint4& partner) {
+        if (!rotate) return x;
+        uint32_t o[4];
+        rope8(x, partner, cosv, sinv, first_half, o);
+        return make_uint4(o[0], o[1], o[2], o[3]);
+    };
+    if (kShare) {
+        if (threadIdx.x < kPieces) *reinterpret_cast<uint4*>(turned + pseg * D + pd) = turn(px, po);
+        __syncthreads();
+    }
+    uint32_t qp[G][4], kp[4];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-        if (rotate) {
-            rope8(qx[g], qo[g], cosv, sinv, first_half, qp[g]);
-        } else {
-            qp[g][0] = qx[g].x; qp[g][1] = qx[g].y; qp[g][2] = qx[g].z; qp[g][3] = qx[g].w;
-        }
+        const uint4 t = kShare ? *reinterpret_cast<const uint4*>(turned + g * D + d0) : turn(px, po);
+        qp[g][0] = t.x; qp[g][1] = t.y; qp[g][2] = t.z; qp[g][3] = t.w;
     }
-    uint32_t kp[4];
-    if (rotate) {
-        rope8(kx, ko, cosv, sinv, first_half, kp);
-    } else {
-        kp[0] = kx.x; kp[1] = kx.y; kp[2] = kx.z; kp[3] = kx.w;
+    {
+        const uint4 t = kShare ? *reinterpret_cast<const uint4*>(turned + G * D + d0) : turn(kx, ko);
+        kp[0] = t.x; kp[1] = t.y; kp[2] = t.z; kp[3] = t.w;
     }
     // append: the last split owns the new row; one row group writes it
     if (last_split && wid == 0 && tg == 0) {
@@ -401,6 +412,15 @@ __global__ __launch_bounds__(W * 64) void paged_attn_decode_kernel(AttnArgs a) {
 constexpr int kMRows = 32;        // rows per wave per stage
 constexpr int kMVRow = 272;       // bytes per staged value row (256 + 16: conflict-free both ways)
 
+// LDS of the form below: staged values, or the states they give way to, or what the splits' merge needs
+template <int G>
+constexpr size_t kMfmaLds = [] {
+    constexpr int D = 128, NS = 4, kAT = 256;
+    constexpr size_t stage = (size_t)4 * kMRows * kMVRow, state = (size_t)(2 * NS * G + NS * G * D) * sizeof(float);
+    constexpr size_t merge = (size_t)(G * 128 + kAT * 4) * sizeof(float);
+    return stage > state ? (stage > merge ? stage : merge) : (state > merge ? state : merge);
+}();
+
 template <int G>
 __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a) {
     constexpr int D = 128, kAW = 4, NS = kAW;
@@ -433,31 +453,32 @@ __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a)
     const int nchunk = nblk > blk_first ? (nblk - blk_first + blk_step - 1) / blk_step : 0;
     const bool last_split = split == filled - 1;
 
-    // ---- query heads (B operand: lane (r, q) = head r, 8 values at 32 kk + 8 q), new k / v ----
+    // ---- query heads and the new k: a 16-byte piece a thread turns, in LDS behind what else lies there (as in the form above; every
+    // wave turning all of them was 640 instructions: 8 rows of 8191 17.4 -> 16.1 us, 45 tokens 8.1 -> 6.9, 32 rows of 2000 16.4 -> 15.2) ----
+    constexpr int kPieces = (G + 1) * (D / 8);
+    static_assert(kPieces <= kAW * 64, "a thread turns one piece");
+    uint16_t* turned = reinterpret_cast<uint16_t*>(reinterpret_cast<unsigned char*>(lds) + kMfmaLds<G>);   // [G + 1][D]
     const bool rotate = (a.rot_cos != nullptr);
-    const int gq = r < G ? r : 0;
-    const uint16_t* qh = a.q + (int64_t)b * a.q_stride_b + (int64_t)(kvh * G + gq) * D + q * 8;
-    const uint16_t* kh = a.k_new + (int64_t)b * a.kv_stride_b + (int64_t)kvh * D + q * 8;
+    const int piece = min((int)threadIdx.x, kPieces - 1), pseg = piece / (D / 8), pd = (piece % (D / 8)) * 8;
+    const bool first_half = pd < D / 2;
+    const int ppart = first_half ? pd + D / 2 : pd - D / 2;
     const uint16_t* vh = a.v_new + (int64_t)b * a.kv_stride_b + (int64_t)kvh * D + q * 8;
-    uint4 qx[4], kx[4], vnew[4];
+    uint4 px, po, vnew[4];
     if (a.slabs) {
         // (the value staging this borrows is first written in the main loop, past the barrier below)
         uint16_t* stage = reinterpret_cast<uint16_t*>(lds);
         stage_qkv_from_slabs<128, G>(a, stage, b, kvh);
+        px = *reinterpret_cast<const uint4*>(stage + pseg * D + pd);
+        po = *reinterpret_cast<const uint4*>(stage + pseg * D + ppart);
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            qx[kk] = *reinterpret_cast<const uint4*>(stage + gq * 128 + q * 8 + kk * 32);
-            kx[kk] = *reinterpret_cast<const uint4*>(stage + G * 128 + q * 8 + kk * 32);
-            vnew[kk] = *reinterpret_cast<const uint4*>(stage + (G + 1) * 128 + q * 8 + kk * 32);
-        }
-        __syncthreads();
+        for (int kk = 0; kk < 4; ++kk) vnew[kk] = *reinterpret_cast<const uint4*>(stage + (G + 1) * 128 + q * 8 + kk * 32);
     } else {
+        const uint16_t* ph = pseg < G ? a.q + (int64_t)b * a.q_stride_b + (int64_t)(kvh * G + pseg) * D
+                                      : a.k_new + (int64_t)b * a.kv_stride_b + (int64_t)kvh * D;
+        px = ld16(ph + pd);
+        po = ld16(ph + ppart);
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            qx[kk] = ld16(qh + kk * 32);
-            kx[kk] = ld16(kh + kk * 32);
-            vnew[kk] = ld16(vh + kk * 32);
-        }
+        for (int kk = 0; kk < 4; ++kk) vnew[kk] = ld16(vh + kk * 32);
     }
 
     auto load_k = [&](uint4(&kb)[8], int pg, int c) {
@@ -485,38 +506,38 @@ __global__ __launch_bounds__(256) void paged_attn_decode_mfma_kernel(AttnArgs a)
     // were measured slower even where there is one workgroup per CU anyway (8 sequences x 1 kv
     // head at ctx 8192: 16.4 against 16.2 us; one sequence x 8 kv heads at ctx 4096: 12.7 against
     // 11.3): the second stage's requests are wasted on short splits and lengthen the prologue.
+    // (the turn's table in front of the rows: behind them the heads could not be turned while the rows are on their way)
+    uint4 cosv = make_uint4(0, 0, 0, 0), sinv = cosv;
+    if (rotate) {
+        const int64_t ro = (int64_t)min(max(pos, 0), a.rot_max_pos - 1) * (D / 2) + (first_half ? pd : ppart);
+        cosv = ld16(a.rot_cos + ro);
+        sinv = ld16(a.rot_sin + ro);
+    }
     uint4 kR[8], vR[8];
     load_k(kR, pgA, 0);
     load_v(vR, pgA, 0);
-    // (behind the requests above: a split with tokens does not wait for the length before it makes them)
     __builtin_amdgcn_sched_barrier(0);
     if (split >= filled && (a.nsplit == 1 || a.arrive)) return;   // uniform; nothing of this row is here
-    uint4 cosv[2], sinv[2];
-    cosv[0] = cosv[1] = sinv[0] = sinv[1] = make_uint4(0, 0, 0, 0);
-    if (rotate) {
-        const int rp = min(max(pos, 0), a.rot_max_pos - 1);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            cosv[h] = ld16(a.rot_cos + (int64_t)rp * (D / 2) + h * 32 + q * 8);
-            sinv[h] = ld16(a.rot_sin + (int64_t)rp * (D / 2) + h * 32 + q * 8);
+    if (threadIdx.x < kPieces) {
+        uint4 x = px;
+        if (rotate) {
+            uint32_t o[4];
+            rope8(px, po, cosv, sinv, first_half, o);
+            x = make_uint4(o[0], o[1], o[2], o[3]);
         }
+        *reinterpret_cast<uint4*>(turned + pseg * D + pd) = x;
     }
-
-    // pieces kk and kk ^ 2 are half a head apart: the rotation needs no other lane
+    __syncthreads();
+    // B operand: lane (r, q) = head r, 8 values at 32 kk + 8 q; padding heads score zero
     bf16x8_t qf[4];
     uint32_t kp[4][4];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-        uint32_t o[4];
-        if (rotate) {
-            rope8(qx[kk], qx[kk ^ 2], cosv[kk & 1], sinv[kk & 1], kk < 2, o);
-            rope8(kx[kk], kx[kk ^ 2], cosv[kk & 1], sinv[kk & 1], kk < 2, kp[kk]);
-        } else {
-            o[0] = qx[kk].x; o[1] = qx[kk].y; o[2] = qx[kk].z; o[3] = qx[kk].w;
-            kp[kk][0] = kx[kk].x; kp[kk][1] = kx[kk].y; kp[kk][2] = kx[kk].z; kp[kk][3] = kx[kk].w;
-        }
-        const uint32_t keep = r < G ? 0xFFFFFFFFu : 0u;   // padding heads score zero
-        qf[kk] = __builtin_bit_cast(bf16x8_t, make_uint4(o[0] & keep, o[1] & keep, o[2] & keep, o[3] & keep));
+        const uint32_t keep = r < G ? 0xFFFFFFFFu : 0u;
+        const uint4 o = *reinterpret_cast<const uint4*>(turned + (r < G ? r : 0) * D + kk * 32 + q * 8);
+        qf[kk] = __builtin_bit_cast(bf16x8_t, make_uint4(o.x & keep, o.y & keep, o.z & keep, o.w & keep));
+        const uint4 kn = *reinterpret_cast<const uint4*>(turned + G * D + kk * 32 + q * 8);
+        kp[kk][0] = kn.x; kp[kk][1] = kn.y; kp[kk][2] = kn.z; kp[kk][3] = kn.w;
     }
     // append: the last split owns the new row; the four lanes with r == 0 of wave 0 hold all of it
     if (last_split && wid == 0 && r == 0) {
@@ -731,8 +752,8 @@ template <int D, int G, int W>
 static int launch_decode_w(const AttnArgs& a, hipStream_t s) {
     constexpr int kAT = W * 64;
     constexpr int NS = W * (64 / (D / 8));
-    const size_t lds = (size_t)(2 * NS * G + NS * G * D) * sizeof(float);
-    static_assert((size_t)(2 * NS * G + NS * G * D) * sizeof(float) <= 160 * 1024 - 1024, "state merge fits LDS");
+    const size_t lds = (size_t)(2 * NS * G + NS * G * D) * sizeof(float) + (size_t)(G + 1) * D * 2;   // states, turned q and k
+    static_assert((size_t)(2 * NS * G + NS * G * D) * sizeof(float) <= 160 * 1024 - 4096, "state merge fits LDS");
     static_assert((size_t)(G * 128 + kAT * 4) * sizeof(float) <= (size_t)(2 * NS * G + NS * G * D) * sizeof(float),
                   "split merge reuses the state arrays");
     static LdsOptIn opted;  // per instantiation
@@ -757,11 +778,8 @@ static int launch_decode(const AttnArgs& a, hipStream_t s) {
 
 template <int G>
 static int launch_decode_mfma(const AttnArgs& a, hipStream_t s) {
-    constexpr int D = 128, NS = 4, kAT = 256;
-    constexpr size_t stage = (size_t)4 * kMRows * kMVRow;
-    constexpr size_t state = (size_t)(2 * NS * G + NS * G * D) * sizeof(float);
-    constexpr size_t merge = (size_t)(G * 128 + kAT * 4) * sizeof(float);
-    constexpr size_t lds = stage > state ? (stage > merge ? stage : merge) : (state > merge ? state : merge);
+    constexpr int D = 128, kAT = 256;
+    constexpr size_t lds = kMfmaLds<G> + (G + 1) * D * 2;   // ..., turned q and k
     static_assert(lds <= 64 * 1024, "no opt-in needed");
     hipLaunchKernelGGL((paged_attn_decode_mfma_kernel<G>), dim3(a.bs * a.hkv * a.nsplit), dim3(kAT), lds, s, a);
     int rc = check_launch();
