@@ -77,7 +77,9 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* dkv, int6
         if (j < half) {
             rot_pair(j, rot, interleaved, a, b);
             const double ang = (double)pos * inv_freq[j];
-            const float cs = (float)cos(ang), sn = (float)sin(ang);
+            double sin_, cos_;
+            sincos(ang, &sin_, &cos_);
+            const float cs = (float)cos_, sn = (float)sin_;
             o0 = src[a] * cs - src[b] * sn;
             o1 = src[b] * cs + src[a] * sn;
         } else {

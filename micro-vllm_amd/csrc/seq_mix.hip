@@ -990,7 +990,9 @@ __global__ __launch_bounds__(256) void rotary_pairs_kernel(float* x, int64_t ld,
     float* p = x + (int64_t)t * ld + (int64_t)hh * dim;
     if (j < half) {
         const double ang = (double)tok_pos[t] * inv_freq[j];
-        const float cs = (float)cos(ang), sn = (float)sin(ang);
+        double sin_, cos_;
+        sincos(ang, &sin_, &cos_);
+        const float cs = (float)cos_, sn = (float)sin_;
         const float u = p[j], v = p[j + half];
         p[j] = (u * cs - v * sn) * scale;
         p[j + half] = (v * cs + u * sn) * scale;
@@ -1108,7 +1110,9 @@ __global__ __launch_bounds__(256) void qk_rotary_store_kernel(float* qk, int64_t
     for (int i = lane; i < half; i += 64) {
         const int a = adjacent ? 2 * i : i, b = adjacent ? 2 * i + 1 : i + half;
         const double ang = (double)pos * inv_freq[i];
-        const float cs = (float)cos(ang), sn = (float)sin(ang);     // once for all heads of the wave
+        double sin_, cos_;
+        sincos(ang, &sin_, &cos_);          // once for all heads of the wave
+        const float cs = (float)cos_, sn = (float)sin_;
         for (int u = u0; u < u1; ++u) {
             float* p = row + (int64_t)u * d;
             const float* bias = u < H ? (qb ? qb + (int64_t)u * d : nullptr) : (kb ? kb + (int64_t)(u - H) * d : nullptr);
@@ -2075,7 +2079,9 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
                 const int a = ra.adjacent ? 2 * i : i, b = ra.adjacent ? 2 * i + 1 : i + half;
                 const float x0 = bias ? p[a] + bias[a] : p[a], x1 = bias ? p[b] + bias[b] : p[b];
                 const double ang = (double)pos * ra.inv_freq[i];
-                const float cs = (float)cos(ang), sn = (float)sin(ang);
+                double sin_, cos_;
+                sincos(ang, &sin_, &cos_);
+                const float cs = (float)cos_, sn = (float)sin_;
                 put(a, x0 * cs - x1 * sn, x0);
                 put(b, x1 * cs + x0 * sn, x1);
             }
