@@ -2270,6 +2270,21 @@ __global__ __launch_bounds__(64) void window_attn_merge_kernel(const float* part
                                                                const float* gate, int64_t ldg) {
     typedef typename ActS<F32>::T T_;
     const int t = blockIdx.x / H, h = blockIdx.x % H, lane = threadIdx.x;
+    // The first pieces, their sums and what the row may be multiplied by are asked for before anything says how many there are
+    // (what lies past those is not used): one trip to memory instead of one for every step below.  With the attention in front of it, fp32, 8
+    // heads of 128 on 2 in four splits at 300 keys 13.4 -> 10.6 us, 1100 17.5 -> 13.1; bf16, 32 heads on 8, 2048 keys in eight 16.7 -> 11.3.
+    constexpr int kAhead = 8;
+    const float* src = part + (int64_t)blockIdx.x * splits * (dv + 2);
+    float ahead[kAhead][2];
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+        if (s >= splits) break;   // uniform
+#pragma unroll
+        for (int k = 0; k < 2; ++k) ahead[s][k] = src[(int64_t)s * (dv + 2) + 2 + (lane + 64 * k < dv ? lane + 64 * k : 0)];
+    }
+    const float* mine = src + (int64_t)(lane < splits ? lane : 0) * (dv + 2);
+    const float m0 = mine[0], l0 = mine[1];
+    const float sink = sinks ? sinks[h] : 0.f;
     int n = splits;                            // pieces there are
     if (nw > 0) {
         const int tiles = tile_run(tok_pos[t], window, keep_first, chunked).n;
@@ -2277,17 +2292,37 @@ __global__ __launch_bounds__(64) void window_attn_merge_kernel(const float* part
         if (tiles < splits * nw) n = (tiles + nw - 1) / nw;
     }
     if (max_len > 0 && row_len[tok_row[t]] > max_len) return;
-    const float* src = part + (int64_t)blockIdx.x * splits * (dv + 2);
-    float M = -INFINITY, L = 0.f;
-    for (int s = lane; s < n; s += 64) M = fmaxf(M, src[(int64_t)s * (dv + 2)]);
+    float M = lane < n ? m0 : -INFINITY, L = 0.f;
+    for (int s = lane + 64; s < n; s += 64) M = fmaxf(M, src[(int64_t)s * (dv + 2)]);
     M = wave_max(M);
-    if (sinks) M = fmaxf(M, sinks[h]);
-    for (int s = lane; s < n; s += 64) {
+    if (sinks) M = fmaxf(M, sink);
+    const float f0 = lane < n && m0 != -INFINITY ? expf(m0 - M) : 0.f;      // the weight of piece `lane`
+    if (lane < n && m0 != -INFINITY) L = fmaf(l0, f0, L);
+    for (int s = lane + 64; s < n; s += 64) {
         const float ms = src[(int64_t)s * (dv + 2)];
         if (ms != -INFINITY) L = fmaf(src[(int64_t)s * (dv + 2) + 1], expf(ms - M), L);
     }
     L = wave_sum(L);
-    if (sinks) L += expf(sinks[h] - M);
+    if (sinks) L += expf(sink - M);
+    auto finish = [&](int c, float o) {
+        o /= L;
+        if (gate) o *= sigmoid_f(gate[(int64_t)t * ldg + (int64_t)h * dv + c]);
+        ActS<F32>::st((T_*)out_ + (int64_t)t * ldo + (int64_t)h * dv + c, o);
+    };
+    if (n <= kAhead && dv <= 128) {
+        float o[2] = {0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) {
+            if (s >= n) break;   // uniform
+            const float f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f0), s));
+#pragma unroll
+            for (int k = 0; k < 2; ++k) o[k] = fmaf(f != 0.f ? ahead[s][k] : 0.f, f, o[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (lane + 64 * k < dv) finish(lane + 64 * k, o[k]);
+        return;
+    }
     for (int c = lane; c < dv; c += 64) {
         float o = 0.f;
 #pragma unroll 4
@@ -2295,9 +2330,7 @@ __global__ __launch_bounds__(64) void window_attn_merge_kernel(const float* part
             const float ms = src[(int64_t)s * (dv + 2)], f = ms != -INFINITY ? expf(ms - M) : 0.f;
             o = fmaf(f != 0.f ? src[(int64_t)s * (dv + 2) + 2 + c] : 0.f, f, o);
         }
-        o /= L;
-        if (gate) o *= sigmoid_f(gate[(int64_t)t * ldg + (int64_t)h * dv + c]);
-        ActS<F32>::st((T_*)out_ + (int64_t)t * ldo + (int64_t)h * dv + c, o);
+        finish(c, o);
     }
 }
 

@@ -612,3 +612,33 @@ def test_rotation_and_attention_in_one_launch(ops, f32, H, G, d, rot, adj, windo
     assert bool(torch.isfinite(found[0][0][0]).all())
     # a head shape without such a launch
     assert not nv.lib().mv_rotary_window_attn_ok(B, H, G, d, d + 1, rot, window, keep, splits, int(f32))
+
+
+# the pieces' merge: up to eight of them, whose values are asked for in front, and more; value columns up to 128 in two a lane and past
+# them; a gate and sinks; fewer tiles than pieces
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("H,G,d,at,splits", [(2, 1, 128, 2000, 7), (2, 1, 128, 2000, 8), (2, 1, 128, 2000, 9), (4, 2, 64, 1900, 12),
+                                             (2, 2, 40, 700, 8), (2, 2, 40, 700, 10), (1, 1, 256, 500, 4), (2, 1, 128, 300, 8)])
+def test_pieces_of_long_windows_meet(ops, f32, H, G, d, at, splits):
+    from micro_vllm_amd.core.state_cache import HybridCacheManager
+    dt = torch.float32 if f32 else torch.bfloat16
+    g = torch.Generator().manual_seed(H + d + at)
+    window, scale = 4000, d ** -0.5
+    cache = HybridCacheManager(36, 64, 1, {0: (G, d, d)}, {}, dtype=dt, device=DEV, max_tokens=2304, max_rows=1, max_step_tokens=2304)
+    step_of(cache, [("m", [0] * at)])
+    st = step_of(cache, [("m", [0])])
+    kc, vc = cache.k_caches[0], cache.v_caches[0]
+    for c in (kc, vc):
+        c.copy_(torch.randn(c.shape, generator=g))
+    q, sink = torch.randn(1, H * d, generator=g).to(DEV), torch.randn(H, generator=g).to(DEV)
+    gate = torch.randn(1, H * d, generator=g).to(DEV)
+    out = torch.empty(1, H * d, dtype=dt, device=DEV)
+    part = torch.full((H * splits * (d + 2),), float("nan"), device=DEV)
+    ops.window_attn(q, kc, vc, out, st, None, H, G, d, d, scale, window, sinks=sink, part=part, splits=splits, gate=gate)
+    pages = cache.get_blocks("m")
+    k, v = (torch.cat([c[p] for p in pages])[:at + 1].double() for c in (kc, vc))
+    for h in range(H):
+        s = torch.cat([k[:, h // (H // G)] @ q[0, h * d:(h + 1) * d].double() * scale, sink[h:h + 1].double()])
+        want = torch.softmax(s, 0)[:at + 1] @ v[:, h // (H // G)] * torch.sigmoid(gate[0, h * d:(h + 1) * d].double())
+        got = out[0, h * d:(h + 1) * d].double()
+        assert (got - want).abs().max().item() < (2e-5 if f32 else 2 ** -8) * max(1.0, want.abs().max().item())
