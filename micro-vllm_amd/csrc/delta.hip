@@ -753,8 +753,10 @@ __global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) 
 
 // One workgroup per (head, 16 state columns, row).  Wave w forms U for the tokens 16 w .. + 15 of a chunk and owns the
 // state rows of the 16-row tiles w, w + 4, ...; the state (as operand) and U pass through LDS.  NT: 16-row tiles; FULL: the state has exactly NT of them (no tests between the products).
-template <int NT, bool FULL>
-__global__ __launch_bounds__(256) void delta_chunk_carry_kernel(DeltaArgs a) {
+// SETS: chunks whose operands are in registers, the ones in hand among them.  Three take all the registers of a SIMD's wave; with more
+// workgroups than compute units two, and two workgroups to a unit (8 rows of three chunks, 16 heads of 128 x 128, 27.3 -> 22.67 us).
+template <int NT, bool FULL, int SETS>
+__global__ __launch_bounds__(256, SETS == 2 ? 2 : 1) void delta_chunk_carry_kernel(DeltaArgs a) {
     constexpr int OWN = (NT + 3) / 4;
     __shared__ float Ss[NT * 16][20];
     __shared__ float Us[kDCh][20];
@@ -800,7 +802,7 @@ __global__ __launch_bounds__(256) void delta_chunk_carry_kernel(DeltaArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) x.uv[j] = up[j * 16];
     };
-    // three sets of operands: a chunk's are requested while the two before it are worked on
+    // a chunk's operands are requested while those before it are worked on
     auto body = [&](Operands& cur, int c) {
         const int64_t unit = u0 + (int64_t)c * a.H;
         // two accumulators: neighbouring products do not wait for each other
@@ -852,18 +854,18 @@ __global__ __launch_bounds__(256) void delta_chunk_carry_kernel(DeltaArgs a) {
                 Ss[16 * it + 4 * g + j][r] = S[o][j];
             }
         }
-        if (c + 3 < nch) fetch(unit + 3 * (int64_t)a.H, cur);
+        if (c + SETS < nch) fetch(unit + SETS * (int64_t)a.H, cur);
         __syncthreads();
     };
-    Operands x0, x1, x2;
-    fetch(u0, x0);
-    if (nch > 1) fetch(u0 + a.H, x1);
-    if (nch > 2) fetch(u0 + 2 * (int64_t)a.H, x2);
+    Operands x[SETS];
+#pragma unroll
+    for (int i = 0; i < SETS; ++i)
+        if (nch > i) fetch(u0 + i * (int64_t)a.H, x[i]);
     __syncthreads();
-    for (int c = 0; c < nch; c += 3) {
-        body(x0, c);
-        if (c + 1 < nch) body(x1, c + 1);
-        if (c + 2 < nch) body(x2, c + 2);
+    for (int c = 0; c < nch; c += SETS) {
+#pragma unroll
+        for (int i = 0; i < SETS; ++i)
+            if (c + i < nch) body(x[i], c + i);
     }
 #pragma unroll
     for (int o = 0; o < OWN; ++o)
@@ -1120,12 +1122,19 @@ int mv_delta_rule(const float* qkv, int64_t ldq, const float* gate_in, int64_t l
         if (int rc = ensure_dynamic_lds((const void*)delta_chunk_intra_kernel, lds1, o1)) return rc;
         hipLaunchKernelGGL(delta_chunk_intra_kernel, dim3(heads, chunks), dim3(kIntra), lds1, s, a);
         const dim3 gc(heads, (unsigned)(P / 16), rows);
-        if (N == 128) hipLaunchKernelGGL((delta_chunk_carry_kernel<8, true>), gc, dim3(256), 0, s, a);
-        else if (N == 64) hipLaunchKernelGGL((delta_chunk_carry_kernel<4, true>), gc, dim3(256), 0, s, a);
-        else if (N <= 32) hipLaunchKernelGGL((delta_chunk_carry_kernel<2, false>), gc, dim3(256), 0, s, a);
-        else if (N <= 64) hipLaunchKernelGGL((delta_chunk_carry_kernel<4, false>), gc, dim3(256), 0, s, a);
-        else if (N <= 128) hipLaunchKernelGGL((delta_chunk_carry_kernel<8, false>), gc, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((delta_chunk_carry_kernel<10, false>), gc, dim3(256), 0, s, a);
+        const bool many = (int64_t)heads * (P / 16) * rows > num_cus();
+#define MV_DELTA_CARRY(NT_, FULL_)                                                                                     \
+    do {                                                                                                               \
+        if (many) hipLaunchKernelGGL((delta_chunk_carry_kernel<NT_, FULL_, 2>), gc, dim3(256), 0, s, a);                 \
+        else hipLaunchKernelGGL((delta_chunk_carry_kernel<NT_, FULL_, 3>), gc, dim3(256), 0, s, a);                      \
+    } while (0)
+        if (N == 128) MV_DELTA_CARRY(8, true);
+        else if (N == 64) MV_DELTA_CARRY(4, true);
+        else if (N <= 32) MV_DELTA_CARRY(2, false);
+        else if (N <= 64) MV_DELTA_CARRY(4, false);
+        else if (N <= 128) MV_DELTA_CARRY(8, false);
+        else hipLaunchKernelGGL((delta_chunk_carry_kernel<10, false, 3>), gc, dim3(256), 0, s, a);     // (two would spill at two waves a SIMD)
+#undef MV_DELTA_CARRY
         const dim3 gi(heads, chunks);
 #define MV_DELTA_INTER(F32_, PT_, FULL_, IDX_)                                                                             \
     do {                                                                                                               \
