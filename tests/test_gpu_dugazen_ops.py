@@ -396,6 +396,26 @@ def test_an_early_write_is_read_hundreds_of_tokens_later(ops, chunked):
         assert (got["a"] - want).abs().max().item() < 2e-4 * want.abs().max().item()
 
 
+# rows so far apart that a chunk's last ones lie more than 4 GiB behind its first: in q | k | v, and in the gate inputs
+@pytest.mark.parametrize("far", ["qkv", "gates"])
+@pytest.mark.parametrize("T", [64, 100])
+def test_delta_rule_of_rows_far_apart(ops, far, T):
+    K, H, n, p, eps = 1, 2, 20, 24, 1e-5
+    d, par = delta_inputs(T, K, H, n, p, seed=T)
+    dev = {k: v.to(DEV) for k, v in par.items()}
+    x, beta = {"qkv": d["qkv"].to(DEV), "gates": torch.cat([d["a"], d["z"]], 1).to(DEV)}, d["beta"].to(DEV)
+    wide = torch.empty(T, 2 ** 32 // (63 * 4) + 1000, device=DEV)[:, :x[far].shape[1]].copy_(x[far])
+    found = []
+    for t in (x, {**x, far: wide}):
+        cache = make_cache(kv={0: (1, 8, 8)}, state={0: {"S": (H, n, p)}}, slots=1)
+        st, out = step_of(cache, [("a", [0] * T)]), torch.empty(T, H * p, device=DEV)
+        ops.delta_rule(t["qkv"], t["gates"][:, :H * n], t["gates"][:, H * n:], beta, dev["dt_bias"], dev["a_log"], dev["norm"],
+                       cache.states[0]["S"], out, st, K, H, n, p, eps)
+        found += [out, cache.states[0]["S"].clone()]
+    assert torch.equal(found[0], found[2]) and torch.equal(found[1], found[3])
+    assert (found[0].cpu() - delta_want(d, par, K, H, n, p, eps)[0]).abs().max().item() < 1e-4
+
+
 def test_delta_rule_slots_used_again(ops):
     K, H, n, p, eps = 1, 2, 24, 40, 1e-5
     a, par = delta_inputs(90, K, H, n, p, seed=1)
