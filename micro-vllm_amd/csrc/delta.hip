@@ -453,7 +453,9 @@ __device__ __forceinline__ void for_tokens(F&& f) {      // f(T0) .. f(T0 + 7), 
     f(std::integral_constant<int, T0 + 7>{});
 }
 
-__global__ __launch_bounds__(kIntra) void delta_chunk_intra_kernel(DeltaArgs a) {
+// (128 registers, so that two workgroups share a unit where two heads' LDS does, n <= 64: at 131 they were one, and 64 chunks of 32 heads of
+// 64 x 64 took 226 us with what follows them, 179 at 126; at 128 state rows a unit holds one either way)
+__global__ __launch_bounds__(kIntra, 4) void delta_chunk_intra_kernel(DeltaArgs a) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int ch = blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, g = lane >> 4;
