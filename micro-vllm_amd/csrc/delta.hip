@@ -756,9 +756,12 @@ __global__ __launch_bounds__(kIntra, 4) void delta_chunk_intra_kernel(DeltaArgs 
 
 // One workgroup per (head, 16 state columns, row).  Wave w forms U for the tokens 16 w .. + 15 of a chunk and owns the
 // state rows of the 16-row tiles w, w + 4, ...; the state (as operand) and U pass through LDS.  NT: 16-row tiles; FULL: the state has exactly NT of them (no tests between the products).
-// SETS: chunks whose operands are in registers, the ones in hand among them.  Three take all the registers of a SIMD's wave; with more
-// workgroups than compute units two, and two workgroups to a unit (8 rows of three chunks, 16 heads of 128 x 128, 27.3 -> 22.67 us).
-template <int NT, bool FULL, int SETS>
+// SETS: chunks whose operands are in registers, the ones in hand among them.  Two, in registers that let two workgroups share a unit: three
+// took all of a SIMD's at 128 state rows, and bought nothing where a unit has one workgroup either (whole calls, us, three -> two; 16 heads of
+// 128 x 128: 8 rows of three chunks 126.9 -> 114.2, 16 of one 100.1 -> 82.8, one row of 23 135.7 -> 134.3, of one chunk 46.4 -> 46.7, one of 16
+// beside seven tokens 95.4 -> 94.7; 32 of 64 x 64: 32 rows of two 247.7 -> 235.6, one of 16 74.5 -> 73.3; 32 of 32 x 32: 16 rows of four 143.9
+// -> 138.6, one of 16 55.5 -> 54.9).  With 10 tiles two would spill at two waves a SIMD: three, and one workgroup a unit.
+template <int NT, bool FULL, int SETS = NT <= 8 ? 2 : 3>
 __global__ __launch_bounds__(256, SETS == 2 ? 2 : 1) void delta_chunk_carry_kernel(DeltaArgs a) {
     constexpr int OWN = (NT + 3) / 4;
     __shared__ float Ss[NT * 16][20];
@@ -1125,19 +1128,12 @@ int mv_delta_rule(const float* qkv, int64_t ldq, const float* gate_in, int64_t l
         if (int rc = ensure_dynamic_lds((const void*)delta_chunk_intra_kernel, lds1, o1)) return rc;
         hipLaunchKernelGGL(delta_chunk_intra_kernel, dim3(heads, chunks), dim3(kIntra), lds1, s, a);
         const dim3 gc(heads, (unsigned)(P / 16), rows);
-        const bool many = (int64_t)heads * (P / 16) * rows > num_cus();
-#define MV_DELTA_CARRY(NT_, FULL_)                                                                                     \
-    do {                                                                                                               \
-        if (many) hipLaunchKernelGGL((delta_chunk_carry_kernel<NT_, FULL_, 2>), gc, dim3(256), 0, s, a);                 \
-        else hipLaunchKernelGGL((delta_chunk_carry_kernel<NT_, FULL_, 3>), gc, dim3(256), 0, s, a);                      \
-    } while (0)
-        if (N == 128) MV_DELTA_CARRY(8, true);
-        else if (N == 64) MV_DELTA_CARRY(4, true);
-        else if (N <= 32) MV_DELTA_CARRY(2, false);
-        else if (N <= 64) MV_DELTA_CARRY(4, false);
-        else if (N <= 128) MV_DELTA_CARRY(8, false);
-        else hipLaunchKernelGGL((delta_chunk_carry_kernel<10, false, 3>), gc, dim3(256), 0, s, a);     // (two would spill at two waves a SIMD)
-#undef MV_DELTA_CARRY
+        if (N == 128) hipLaunchKernelGGL((delta_chunk_carry_kernel<8, true>), gc, dim3(256), 0, s, a);
+        else if (N == 64) hipLaunchKernelGGL((delta_chunk_carry_kernel<4, true>), gc, dim3(256), 0, s, a);
+        else if (N <= 32) hipLaunchKernelGGL((delta_chunk_carry_kernel<2, false>), gc, dim3(256), 0, s, a);
+        else if (N <= 64) hipLaunchKernelGGL((delta_chunk_carry_kernel<4, false>), gc, dim3(256), 0, s, a);
+        else if (N <= 128) hipLaunchKernelGGL((delta_chunk_carry_kernel<8, false>), gc, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((delta_chunk_carry_kernel<10, false>), gc, dim3(256), 0, s, a);
         const dim3 gi(heads, chunks);
 #define MV_DELTA_INTER(F32_, PT_, FULL_, IDX_)                                                                             \
     do {                                                                                                               \

@@ -33,3 +33,10 @@ def test_two_workgroups_inside_a_chunk_share_a_unit(kernels):
     """Eight waves a workgroup: two of them are four waves a SIMD, of 128 registers a lane each."""
     intra = [v for n, v in kernels.items() if "delta_chunk_intra_kernel" in n]
     assert len(intra) == 1 and intra[0][0] <= 128 and intra[0][1] == 0, intra
+
+
+def test_two_workgroups_of_the_carry_share_a_unit(kernels):
+    """Two sets of operands in at most half of a SIMD's 512 registers, up to 128 state rows; three in all of them past those."""
+    carry = {n: v for n, v in kernels.items() if "delta_chunk_carry_kernel" in n}
+    assert len(carry) == 6 and all(v[1] == 0 for v in carry.values()), carry
+    assert all(v[0] <= (512 if "ILi10E" in n else 256) for n, v in carry.items()), carry

@@ -416,6 +416,23 @@ def test_delta_rule_of_rows_far_apart(ops, far, T):
     assert (found[0].cpu() - delta_want(d, par, K, H, n, p, eps)[0]).abs().max().item() < 1e-4
 
 
+# the chunks' states, one form for each size of a head's state: rows of one to five chunks, begun and carried on, beside rows without a chunk
+@pytest.mark.parametrize("n,p", [(20, 24), (40, 40), (64, 64), (100, 72), (128, 128), (150, 40)])
+def test_delta_rule_of_one_to_five_chunks(ops, n, p):
+    K, H, eps = 1, 2, 1e-5
+    plan = [[("a", 64), ("b", 130), ("c", 4), ("d", 250)], [("a", 100), ("b", 1), ("c", 70), ("d", 300)]]
+    data = {k: delta_inputs(sum(c for rows in plan for s, c in rows if s == k), K, H, n, p, seed=i) for i, k in enumerate("abcd")}
+    seqs, par = {k: d for k, (d, _) in data.items()}, data["a"][1]
+    cache = make_cache(kv={0: (1, 8, 8)}, state={0: {"S": (H, n, p)}}, slots=4, pages=20)
+    got, states = run_delta(ops, seqs, par, plan, K, H, n, p, eps, cache=cache)
+    for k in seqs:
+        want, S = delta_want(seqs[k], par, K, H, n, p, eps)
+        assert (got[k] - want).abs().max().item() < 1e-4 * max(1.0, want.abs().max().item()), k
+        assert (states[k] - S).abs().max().item() < 2e-5 * max(1.0, S.abs().max().item()), k
+        alone, state = run_delta(ops, {k: seqs[k]}, par, [[r for r in rows if r[0] == k] for rows in plan], K, H, n, p, eps)
+        assert torch.equal(alone[k], got[k]) and torch.equal(state[k], states[k]), k
+
+
 def test_delta_rule_slots_used_again(ops):
     K, H, n, p, eps = 1, 2, 24, 40, 1e-5
     a, par = delta_inputs(90, K, H, n, p, seed=1)
