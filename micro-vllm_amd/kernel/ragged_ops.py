@@ -370,10 +370,12 @@ def rotary_window_attn(qk, q_bias, k_bias, k_cache, v_cache, inv_freq, out, step
                        scale: float, window: int, keep_first: int = 0, sinks=None, part=None, splits: int = 0,
                        adjacent: bool = True, act=None) -> bool:
     """`qk_rotary_store` and the `window_attn` behind it in one launch, for a step of one token a row; the same results, but the
-    queries in qk stay as projected.  False, and nothing done, where there is no such launch."""
+    queries in qk stay as projected.  False, and nothing done, where there is no such launch (stores that are not 16-byte
+    aligned, which the two calls take, among them)."""
     tokens = qk.shape[0]
-    if part is None or step.tokens != step.rows or not nv.lib().mv_rotary_window_attn_ok(
-            tokens, heads, kv_heads, d, d, rot, int(window), int(keep_first), int(splits), _is_f32(k_cache)):
+    if part is None or step.tokens != step.rows or k_cache.data_ptr() % 16 or v_cache.data_ptr() % 16 or \
+            not nv.lib().mv_rotary_window_attn_ok(tokens, heads, kv_heads, d, d, rot, int(window), int(keep_first), int(splits),
+                                                  _is_f32(k_cache)):
         return False
     a_in = a_out = None
     n_act = kind = 0

@@ -614,6 +614,39 @@ def test_rotation_and_attention_in_one_launch(ops, f32, H, G, d, rot, adj, windo
     assert not nv.lib().mv_rotary_window_attn_ok(B, H, G, d, d + 1, rot, window, keep, splits, int(f32))
 
 
+# page stores that begin 8 bytes past a 16-byte place: the one launch says that it has no form and leaves all as it was, the two take them
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("which", [(0,), (1,), (0, 1)])
+def test_rotation_and_attention_of_unaligned_stores(ops, f32, which):
+    from micro_vllm_amd.core.state_cache import HybridCacheManager
+    dt = torch.float32 if f32 else torch.bfloat16
+    g = torch.Generator().manual_seed(len(which))
+    H, G, d, window = 4, 2, 64, 100
+    cache = HybridCacheManager(8, 64, 2, {0: (G, d, d)}, {}, dtype=dt, device=DEV, max_tokens=256, max_rows=2, max_step_tokens=256)
+    step_of(cache, [("a", [0] * 90)])
+    st = step_of(cache, [("a", [0]), ("b", [0])])
+    inv = (5000.0 ** (-2.0 * torch.arange(d // 2, dtype=torch.float64) / d)).to(DEV)
+    proj, n = torch.randn(2, (H + G) * d, generator=g).to(DEV), cache.k_caches[0].numel()
+    pages = [torch.randn(cache.k_caches[0].shape, generator=g).to(DEV, dt) for _ in range(2)]
+    splits = ops.window_attn_splits(2, H, G, window, 0)
+    part = torch.full((2 * H * splits * (d + 2),), float("nan"), device=DEV)
+    found = []
+    for aligned in (True, False):
+        kc, vc = (torch.empty(n + 16, dtype=dt, device=DEV)[0 if aligned or i not in which else 8 // dt.itemsize:][:n].view(p.shape).copy_(p)
+                  for i, p in enumerate(pages))
+        qk, out = proj.clone(), torch.full((2, H * d), 9.0, dtype=dt, device=DEV)
+        took = ops.rotary_window_attn(qk, None, None, kc, vc, inv, out, st, H, G, d, d, d ** -0.5, window, part=part, splits=splits)
+        assert took == aligned and torch.equal(qk, proj)
+        if not took:
+            assert bool((out == 9.0).all()) and torch.equal(kc, pages[0]) and torch.equal(vc, pages[1])
+            ops.qk_rotary_store(qk, None, None, kc, vc, inv, st, H, G, d, d)
+            ops.window_attn(qk, kc, vc, out, st, None, H, G, d, d, d ** -0.5, window, part=part, splits=splits)
+        found.append((out, kc, vc))
+    # another kernel's sums: some 90 terms of weight below one, in fp32, rounded to the stores' type
+    assert (found[0][0].float() - found[1][0].float()).abs().max().item() <= (1e-5 if f32 else 2 ** -7)
+    assert torch.equal(found[0][1], found[1][1]) and torch.equal(found[0][2], found[1][2])
+
+
 # the pieces' merge: up to eight of them, whose values are asked for in front, and more; value columns up to 128 in two a lane and past
 # them; a gate and sinks; fewer tiles than pieces
 @pytest.mark.parametrize("f32", [False, True])
