@@ -438,7 +438,7 @@ __device__ __forceinline__ void add_row_lane(float& acc, const f32x4_t& a, const
         "v_fmac_f32_dpp %0, %2, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f32_dpp %0, %3, %7 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
-        : "+v"(acc)
+        : "+&v"(acc)      // written before the last input is read: never the register of one
         : "v"(a[3]), "v"(a[2]), "v"(a[1]), "v"(a[0]), "v"(b[3]), "v"(b[2]), "v"(b[1]), "v"(b[0]), "n"(T));
 }
 template <int T0, typename F>
