@@ -84,11 +84,14 @@ static bool pf_eight_waves(int bs, int seq, int hkv, int g) {
 }
 
 // Chunks whose attention turns its own queries and keys (paged_attn_prefill_kernel, ROT) against the rotation's own launch in front of it.
-// Heads of 64: up to 128 tokens, up to 256 from four sequences on (us, two launches -> one, 32 heads on 4: 37 tokens 7.7 -> 6.7, 128 9.2 -> 8.2,
-// 256 11.9 -> 11.8; 4 x 256 14.9 -> 12.6, 16 x 64 11.6 -> 7.9).  Heads of 128, whose turning is twice the work of a workgroup that has
+// Heads of 64: up to 128 tokens, up to 256 from four sequences on (us, two launches -> one, 32 heads on 4: 37 tokens 8.0 -> 6.5, 128 9.3 -> 8.0,
+// 256 level; 4 x 256 15.0 -> 12.1, 16 x 64 11.7 -> 7.7).  Heads of 128, whose turning is twice the work of a workgroup that has
 // half its lanes' time: from four sequences and 2 M values of q, k and v on, where the separate launch takes as long (32 heads on 8: 37 tokens
-// 9.9 -> 10.5, 4 x 37 10.6 -> 10.9, 4 x 100 14.2 -> 13.6, 16 x 64 17.7 -> 12.3, 16 x 256 49.7 -> 42.1; 8 on 1: 4 x 256 16.4 -> 19.2, 16 x 128
-// 14.7 -> 13.6).
+// 9.9 -> 10.5, 4 x 37 10.6 -> 10.9, 4 x 100 14.3 -> 13.4, 16 x 64 17.4 -> 12.2, 16 x 256 48.1 -> 41.9; 8 on 1: 4 x 256 16.4 -> 19.2, 16 x 128
+// 14.7 -> 13.3).
+// Behind cached tokens, which the host does not see, heads of 64 stay level or ahead (32 on 4: 37 tokens behind 300 14.4 -> 14.4, behind 2000 46.2
+// -> 44.8; 16 x 256 behind 2000 121 -> 125; 8 on 8, 128 behind 300 15.7 -> 17.3), heads of 128 lose up to a tenth where many tiles of them are
+// few workgroups' (32 on 8: 4 x 256 behind 300 32.5 -> 32.8, behind 2000 78 -> 86; 32 x 64 behind 2000 112 -> 109).
 static bool pf_rotates(int bs, int seq, int hq, int hkv, int d) {
     if (pf_eight_waves(bs, seq, hkv, hq / hkv)) return false;
     if (d == 64) return seq <= 128 || (seq <= 256 && bs >= 4);
@@ -234,6 +237,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     constexpr int VROW = D * 2 + 32;   // ... and conflict-free transposed reads
     constexpr int VPR = D / 8;         // 16-byte vectors per row
     constexpr int NV = KT * VPR / NT;  // vectors per thread per tile
+    using Own = std::integral_constant<bool, ROT>;
     __shared__ __attribute__((aligned(16))) unsigned char kL[2][KT * KROW];
     __shared__ __attribute__((aligned(16))) unsigned char vL[2][KT * VROW];
 
@@ -252,7 +256,10 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     const int i0 = qb * a.qt;
     int last_key = p0 + min(i0 + a.qt, a.S) - 1;   // last key any row of this block sees
     int ntiles = last_key / KT + 1;
-    const int32_t* bt = a.block_table + (int64_t)b * a.bt_stride;
+    // (in the constant address space: nothing here writes the table.  With ROT, which writes pages, it would else be read by vector loads, and
+    // a page number's test wait for all the rows requested in front of it: a tile of 64 cached tokens in 1.37 us instead of 1.29)
+    typedef const int32_t __attribute__((address_space(4))) Entry;
+    Entry* bt = (Entry*)(uintptr_t)(a.block_table + (int64_t)b * a.bt_stride);
 
     // this lane's query rows (C-layout column r of each of the wave's two tiles)
     // (3, 5, 6 or 7 query heads per kv head: the stack has room for the next power of two; the rows
@@ -287,6 +294,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     if (ROT && a.cos) load_turns();
 
     // K/V staging: thread moves vectors t + 256 j of the 64 x VPR tile
+    uint4 kr[NV], vr[NV];
     auto tile_page = [&](int t) {
         // column clamped into the table: keys past its last column have no page (a contract breach:
         // such keys read page-table garbage before; now they read the last column's page)
@@ -305,8 +313,9 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
         const int pg = bt[pos >> a.page_shift];
         return pg < a.num_pages ? pg : -1;
     };
-    auto g_load = [&](uint4(&kr)[NV], uint4(&vr)[NV], int t, int pg) {
-        if constexpr (ROT) {
+    // own: the tile may have keys of the chunk (ROT); tiles of nothing but cached tokens are staged as the plain form stages them
+    auto g_load = [&](auto own, int t, int pg) {
+        if constexpr (decltype(own)::value) {
 #pragma unroll
             for (int j = 0; j < NV / 2; ++j) {
                 const int v = threadIdx.x + NT * j, row = v / (VPR / 2), ch = v % (VPR / 2);
@@ -342,9 +351,9 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
             vr[j] = ld16(a.v_cache + off);
         }
     };
-    auto l_store = [&](uint4(&kr)[NV], const uint4(&vr)[NV], int t) {
+    auto l_store = [&](auto own, int t) {
         const int buf = t & 1;
-        if constexpr (ROT) {
+        if constexpr (decltype(own)::value) {
             auto slot = [&](int pg, int row) {
                 const int pos = start + t * KT + row - p0;
                 return (((int64_t)pg * a.page + (pos & (a.page - 1))) * a.hkv + kvh) * D;
@@ -384,9 +393,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
         for (int dt = 0; dt < DT; ++dt) oacc[mt][dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     float mrun[2] = {kPfNegBig, kPfNegBig}, lrun[2] = {0.f, 0.f};
 
-    uint4 kr[NV], vr[NV];
     int pg_next = tile_page(0);
-    g_load(kr, vr, 0, pg_next);
+    g_load(Own{}, 0, pg_next);
     if constexpr (ROT) {
         __builtin_amdgcn_sched_barrier(0);
         const int true_start = a.start[b];
@@ -399,7 +407,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
             p0 = moved;
             ntiles = last_key / KT + 1;
             if (a.cos) load_turns();
-            g_load(kr, vr, 0, pg_next);
+            if (p0 >= KT) g_load(std::false_type{}, 0, pg_next);
+            else g_load(Own{}, 0, pg_next);
         }
         if (a.cos) {
 #pragma unroll
@@ -419,14 +428,15 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     for (int o = 1; o < 16; o <<= 1) wave_min_limit = min(wave_min_limit, __shfl_xor(wave_min_limit, o, 64));
     wave_min_limit = __builtin_amdgcn_readfirstlane(wave_min_limit);
     pg_next = ntiles > 1 ? tile_page(1) : 0;
-    l_store(kr, vr, 0);
+    if (ROT && p0 >= KT) l_store(std::false_type{}, 0);
+    else l_store(Own{}, 0);
     __syncthreads();
 
     // transposed-read lane address inside a 16-key x 16-column block pair
     const int li = lane & 15;
     const int tr_off = (4 * q + (li >> 2)) * VROW + (li & 3) * 8;
 
-    for (int t = 0; t < ntiles; ++t) {
+    auto pass = [&](auto own, int t) {      // tile t, while the next (own: see g_load) is on its way
         const int buf = t & 1;
 #ifdef MV_EXP_NO_KVLOAD
         const bool more = false;   // timing experiment only (wrong results): every tile re-uses the first two
@@ -434,7 +444,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
         const bool more = t + 1 < ntiles;
 #endif
         if (more) {
-            g_load(kr, vr, t + 1, pg_next);
+            g_load(own, t + 1, pg_next);
             if (t + 2 < ntiles) pg_next = tile_page(t + 2);
         }
         // The 64 keys of the tile in one pass: 32 MFMAs for S^T, one softmax update over 16 scores
@@ -545,9 +555,16 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
                     oacc[mt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[mt][h], oacc[mt][dt], 0, 0, 0);
             }
         }
-        if (more) l_store(kr, vr, t + 1);
+        if (more) l_store(own, t + 1);
         __syncthreads();
+    };
+    int tile = 0;
+    if constexpr (ROT) {
+        // behind cached tokens their tiles have a loop of their own: with the chunk's tests and table in it, 37 tokens of 32 heads of 64 on 4 behind
+        // 2000 took 57 us where the two launches take 46
+        for (const int cached = p0 / KT; tile + 1 < cached; ++tile) pass(std::false_type{}, tile);
     }
+    for (; tile < ntiles; ++tile) pass(Own{}, tile);
 
     // oacc[mt][dt][j] = O^T[d = 16 dt + 4q + j][query row r]
 #pragma unroll
