@@ -1895,10 +1895,12 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     __shared__ float mm[NW * RT], ll[NW * RT];
     __shared__ __attribute__((aligned(16))) float qs[ROT ? RT * d : 4];          // ROT: turned queries, the token's own key
     __shared__ __attribute__((aligned(16))) T_ kn[ROT ? d : 8], vn[ROT ? dv : 8];   // and value
-    // bf16 keys: the queries' three parts, formed once for the workgroup: a value's split is some eight instructions, and a wave has 32
-    // values a lane to it, while what bounds a tile here is the issue slots of the waves that share a unit (one token of 8 heads on 2,
-    // 45 keys, 7.35 -> 5.45 us, 1100 19.6 -> 17.2).  A single head's are not worth the barrier (4.7 -> 5.0 at 45 keys of a launch of its own)
-    constexpr bool kShareQ = !F32 && (ROT || HEADS > 1);
+    // bf16 keys: the queries' three parts, formed once for the workgroup: a value's split is some eight instructions, and a wave has up to 32
+    // values a lane to it, while what bounds a tile here is the issue slots of the waves that share a unit (one token of 8 heads on 2 of 128,
+    // 45 keys, 7.35 -> 5.45 us, 1100 19.6 -> 17.2).  Not worth the barrier with a single head (4.7 -> 5.0 at 45 keys of a launch of its own) and with
+    // 8 values a lane (each wave its own, shared: 16 heads of 32 on 4 at 45 keys 4.0, 4.6, at 1100 11.0 both); 16 are even (45 and 1100 keys: 16
+    // heads of 64 on 4 5.2, 4.9 and 13.1, 12.7, 4 on 2 4.4, 4.7 and 12.4, 12.5).  The turned queries lie in LDS either way
+    constexpr bool kShareQ = !F32 && (ROT || (HEADS > 1 && KS * HB > 1));
     __shared__ __attribute__((aligned(16))) uint16_t qp[kShareQ ? 3 * RT * d : 8];
     if constexpr (ROT) {
         if (blockIdx.x >= ra.units) {
@@ -1959,7 +1961,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
                     qb[b][i] = __builtin_bit_cast(wa_bf16x8_t, has ? x : make_uint4(0, 0, 0, 0));
                 }
             } else {
-                const float* qr = q + (int64_t)t * ldq + (int64_t)h0 * d;
+                const float* qr = q + (int64_t)t * ldq + (int64_t)(h0 + (ok ? h : 0)) * d;
                 const int s = col >> 2;
 #pragma unroll
                 for (int i = 0; i < KS; ++i) {
@@ -1974,7 +1976,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
                         const uint32_t b2 = __float_as_uint(r1) & 0xffff0000u;
                         const float r2 = r1 - __uint_as_float(b2);
                         const uint32_t w = s == 0 ? a : s == 1 ? b2 : __float_as_uint(r2);
-                        p[e] = s < 3 ? (uint16_t)(w >> 16) : (uint16_t)0;
+                        p[e] = ok && s < 3 ? (uint16_t)(w >> 16) : (uint16_t)0;
                     }
                     qb[b][i] = __builtin_bit_cast(wa_bf16x8_t, *reinterpret_cast<uint4*>(p));
                 }

@@ -647,6 +647,36 @@ def test_rotation_and_attention_of_unaligned_stores(ops, f32, which):
     assert torch.equal(found[0][1], found[1][1]) and torch.equal(found[0][2], found[1][2])
 
 
+# short rows' bf16 queries, whose three parts the workgroup forms once or each wave for itself, by the head's size and the heads that share a
+# key: two to four heads, five and eight in pairs of four, nine in two groups; one key, a tile and a key more, several tiles
+@pytest.mark.parametrize("R", [2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("d,dv", [(32, 32), (64, 32), (64, 64), (64, 128), (96, 96), (128, 64)])
+def test_queries_of_heads_that_share_a_key(ops, R, d, dv):
+    from micro_vllm_amd.core.state_cache import HybridCacheManager
+    G, scale, window, lens = 2, d ** -0.5, 300, (0, 16, 100)
+    H, B = R * G, len(lens)
+    g = torch.Generator().manual_seed(R * 1000 + d + dv)
+    cache = HybridCacheManager(8, 64, B, {0: (G, d, dv)}, {}, dtype=torch.bfloat16, device=DEV, max_tokens=256, max_rows=B,
+                               max_step_tokens=256)
+    for i, n in enumerate(lens):
+        if n:
+            step_of(cache, [(i, [0] * n)])
+    st = step_of(cache, [(i, [0]) for i in range(B)])
+    for c in (cache.k_caches[0], cache.v_caches[0]):
+        c.copy_(torch.randn(c.shape, generator=g))
+    q = torch.randn(B, H * d, generator=g).to(DEV)
+    out, splits = torch.empty(B, H * dv, dtype=torch.bfloat16, device=DEV), ops.window_attn_splits(B, H, G, window)
+    part = torch.full((B * H * splits * (dv + 2),), float("nan"), device=DEV)
+    ops.window_attn(q, cache.k_caches[0], cache.v_caches[0], out, st, None, H, G, d, dv, scale, window, part=part, splits=splits)
+    for b, n in enumerate(lens):
+        k, v = (torch.cat([c[p] for p in cache.get_blocks(b)])[:n + 1].double() for c in (cache.k_caches[0], cache.v_caches[0]))
+        for h in range(H):
+            p = torch.softmax(k[:, h // R] @ q[b, h * d:(h + 1) * d].double() * scale, 0)
+            want, got = p @ v[:, h // R], out[b, h * dv:(h + 1) * dv].double()
+            # fp32 sums of up to 128 products and 101 weights (values up to 4), rounded to bf16
+            assert ((got - want).abs() <= 2 ** -8 * want.abs() + 4e-5).all(), (b, h)
+
+
 # the pieces' merge: up to eight of them, whose values are asked for in front, and more; value columns up to 128 in two a lane and past
 # them; a gate and sinks; fewer tiles than pieces
 @pytest.mark.parametrize("f32", [False, True])
