@@ -1862,12 +1862,15 @@ typedef __attribute__((ext_vector_type(8))) __bf16 wa_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float wa_f32x4_t;
 
 // What a step of single tokens does in front of its attention, in the same launch: qk_rotary_store_kernel's work, same arithmetic.
-// `units` workgroups attend; those behind them form the gate of a feed-forward.
+// Workgroups past the splits, in y, form the gate of a feed-forward, `act_blocks` pieces of 64 NW columns.  (Behind each split's in x they were
+// left empty in all splits but one, and an empty workgroup, too, waits for room on a unit that the splits behind it could have: fp32, 24
+// heads of 64 on 2, 4 tokens at 2000 keys in 16 splits, a gate of 4096 22.3 us, here 16.2, in two launches 19.8; bf16, 16 tokens at 1000 17.1,
+// 12.9, 16.9.)
 struct StepRotary {
     const float *q_bias, *k_new, *k_bias;      // k_new: the step's keys, rows as far apart as q's
     const double* inv_freq;
     int rot, adjacent;
-    unsigned units;
+    unsigned act_blocks;
     const float* act_in;
     void* act_out;
     int64_t lda, ldao;
@@ -1903,11 +1906,11 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     constexpr bool kShareQ = !F32 && (ROT || (HEADS > 1 && KS * HB > 1));
     __shared__ __attribute__((aligned(16))) uint16_t qp[kShareQ ? 3 * RT * d : 8];
     if constexpr (ROT) {
-        if (blockIdx.x >= ra.units) {
-            const unsigned cb = (ra.act_n + 64 * NW - 1) / (64 * NW), i = blockIdx.x - ra.units;
+        if ((int)blockIdx.y >= splits) {
+            const unsigned cb = (ra.act_n + 64 * NW - 1) / (64 * NW), i = (blockIdx.y - splits) * gridDim.x + blockIdx.x;
             const int64_t r = i / cb;
             const int c = (i % cb) * 64 * NW + threadIdx.x;
-            if (blockIdx.y == 0 && c < ra.act_n)
+            if (i < ra.act_blocks && c < ra.act_n)
                 ActS<F32>::st((T_*)ra.act_out + r * ra.ldao + c, gated_act_f(ra.act_in[r * ra.lda + c], ra.act_in[r * ra.lda + ra.act_n + c],
                                                                             ra.act_kind, ra.act_limit, ra.act_slope));
             return;
@@ -3277,14 +3280,18 @@ int mv_rotary_window_attn(const float* qk, int64_t ld, const float* q_bias, cons
     if (!aligned16(k_cache) || !aligned16(v_cache)) return MV_ERR_UNSUPPORTED;
     const FewPlan fp = few_plan(tokens, heads, kv_heads, window, keep_first, f32, splits);
     const int nw = fp.top <= 1 ? 16 : fp.top <= 4 ? (f32 ? 8 : 16) : 8;
-    const int64_t act_blocks = act_in ? (int64_t)tokens * ((act_n + 64 * nw - 1) / (64 * nw)) : 0;
-    if (fp.groups + act_blocks > 0x7fffffff) return MV_ERR_UNSUPPORTED;
+    int64_t act_blocks = act_in ? (int64_t)tokens * ((act_n + 64 * nw - 1) / (64 * nw)) : 0;
+    if (act_blocks > (int64_t)(65535 - fp.pieces) * fp.groups) {      // more than the grid's rows hold: a launch of its own
+        if (const int rc = mv_gated_act(act_in, lda, act_out, ldao, tokens, act_n, act_kind, act_limit, act_slope, f32, stream)) return rc;
+        act_blocks = 0;
+    }
+    const int64_t act_rows = (act_blocks + fp.groups - 1) / fp.groups;
     PagedRows pr{tok_row, tok_pos, block_table, bt_stride, page};
-    const StepRotary ra{q_bias, qk + (int64_t)heads * d, k_bias, inv_freq, rot, adjacent, (unsigned)fp.groups, act_in, act_out, lda, ldao,
-                        act_n, act_kind, act_limit, act_slope};
+    const StepRotary ra{q_bias, qk + (int64_t)heads * d, k_bias, inv_freq, rot, adjacent, (unsigned)act_blocks, act_in, act_out, lda,
+                        ldao, act_n, act_kind, act_limit, act_slope};
     hipStream_t s = (hipStream_t)stream;
 #define MV_RWA(F32_, HB_, NW_, KS_, VE_)                                                                               \
-    hipLaunchKernelGGL((window_attn_few_kernel<F32_, HB_, NW_, KS_, VE_, true>), dim3((unsigned)(fp.groups + act_blocks), fp.pieces), \
+    hipLaunchKernelGGL((window_attn_few_kernel<F32_, HB_, NW_, KS_, VE_, true>), dim3((unsigned)fp.groups, (unsigned)(fp.pieces + act_rows)), \
                        dim3(64 * NW_), 0, s, qk, ld, k_cache, v_cache, out, ldo, part, pr, (const float*)nullptr, sinks, heads, kv_heads, \
                        scale, window, keep_first, (const int*)nullptr, 0, fp.pieces, (const float*)nullptr, (int64_t)0, 0, ra)
 #define MV_RWA_HB(F32_, KS_, VE_)                                                                                      \

@@ -568,12 +568,15 @@ def test_infinite_keys_alone_in_their_tile(ops, f32, form, H, G, window, splits,
 @pytest.mark.parametrize("H,G,d,rot,adj,window,keep,at", [
     (8, 2, 128, 128, True, 1024, 64, (44, 0, 15, 16, 63, 64)), (6, 1, 64, 40, False, 37, 5, (200, 36, 37, 5, 1)),
     (24, 2, 64, 64, True, 100, 0, (127, 128)), (3, 3, 64, 64, True, 1, 0, (0, 70)), (12, 1, 128, 64, False, 2047, 3, (2100, 31)),
-    (4, 4, 128, 0, True, 300, 20, (500, 16)), (8, 2, 128, 128, True, 1500, 64, (1700,))])
+    (4, 4, 128, 0, True, 300, 20, (500, 16)), (8, 2, 128, 128, True, 1500, 64, (1700,)),
+    # windows cut over several workgroups, and a workgroup for every compute unit, a wide gate beside them
+    (8, 2, 128, 128, True, 4000, 0, (2000, 0, 100, 1500, 15, 700, 2100, 33)), (9, 1, 64, 32, True, 3900, 7, (2100, 5) * 4),
+    (5, 1, 64, 64, False, 50, 0, (3,) * 256)])
 def test_rotation_and_attention_in_one_launch(ops, f32, H, G, d, rot, adj, window, keep, at):
     from micro_vllm_amd import _native as nv
     dt = torch.float32 if f32 else torch.bfloat16
     g = torch.Generator().manual_seed(H * 100 + d + len(at))
-    B, ff = len(at), 1100
+    B, ff = len(at), 5500 if len(at) > 8 else 1100
     from micro_vllm_amd.core.state_cache import HybridCacheManager
     cache = HybridCacheManager(B * 36, 64, B, {0: (G, d, d)}, {}, dtype=dt, device=DEV, max_tokens=2304, max_rows=B, max_step_tokens=2304)
     for i, n in enumerate(at):
@@ -612,6 +615,21 @@ def test_rotation_and_attention_in_one_launch(ops, f32, H, G, d, rot, adj, windo
     assert bool(torch.isfinite(found[0][0][0]).all())
     # a head shape without such a launch
     assert not nv.lib().mv_rotary_window_attn_ok(B, H, G, d, d + 1, rot, window, keep, splits, int(f32))
+
+
+# a gate of more columns than one row of the grid's pieces of 1024 holds, and one of as many
+@pytest.mark.parametrize("n", [1024 * 65534 + 5, 1024 * 65534])
+def test_a_gate_wider_than_the_grid(ops, n):
+    from micro_vllm_amd.core.state_cache import HybridCacheManager
+    cache = HybridCacheManager(1, 64, 1, {0: (1, 64, 64)}, {}, dtype=torch.bfloat16, device=DEV, max_tokens=64, max_rows=1, max_step_tokens=64)
+    st = step_of(cache, [("a", [0])])
+    qk, a = torch.ones(1, 128, device=DEV), torch.empty(1, 2 * n, device=DEV).uniform_(-2, 2)
+    out, gate, want = (torch.empty(1, c, dtype=torch.bfloat16, device=DEV) for c in (64, n, n))
+    inv, part = torch.ones(32, dtype=torch.float64, device=DEV), torch.empty(66, device=DEV)
+    assert ops.rotary_window_attn(qk, None, None, cache.k_caches[0], cache.v_caches[0], inv, out, st, 1, 1, 64, 64, 1.0, 64, part=part, splits=1,
+                                  act=(a, gate, ops.GATE_GELU_TANH, 0.0, 1.0))
+    ops.gated_act(a, want, ops.GATE_GELU_TANH)
+    assert torch.equal(gate, want) and bool((out == 1.0).all())
 
 
 # page stores that begin 8 bytes past a 16-byte place: the one launch says that it has no form and leaves all as it was, the two take them
