@@ -354,7 +354,9 @@ int mv_paged_attn_prefill(const void* q, int64_t q_stride, const void* k_cache, 
                           void* out, int64_t out_stride, int bs, int seq, int hq, int hkv, int d,
                           int page, int num_pages, float scale, mv_stream_t stream);
 /* mv_rope_store_prefill and mv_paged_attn_prefill on one buffer of q | k | v rows: one launch for chunks of few tokens (qkv then
- * stays as projected), the two otherwise.  The same output and pages, bit for bit. */
+ * stays as projected), the two otherwise.  The same pages, bit for bit, and the same output for every token all of whose visible positions
+ * have a page; a token that sees a position without one (a negative entry or one past the last page, or past the table) gets an
+ * unspecified output from either, and not the same. */
 int mv_rope_attn_prefill(void* qkv, int64_t row_stride, const void* rot_cos, const void* rot_sin, int rot_max_pos,
                          const int32_t* cache_seqlens, const int32_t* block_table, int bt_stride, void* k_cache, void* v_cache,
                          void* out, int64_t out_stride, int bs, int seq, int hq, int hkv, int d, int page, int num_pages,

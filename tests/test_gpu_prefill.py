@@ -419,13 +419,17 @@ def test_layers_that_are_not_alike_go_one_by_one(mv, odd):
 
 
 # rotation, stores and attention of short chunks in one launch are the two launches, bit for bit: heads of 64 up to 128 tokens and, from
-# four sequences on, 256; heads of 128 in batches; tiles that end inside 64 keys, one, three and eight query heads to a key/value head, cached
-# tokens in front of some chunks, no rotation, a page that was never allocated (nothing is stored there)
-@pytest.mark.parametrize("D,Hq,Hkv,S,starts,rot", [
-    (64, 32, 4, 37, (0,), True), (64, 4, 4, 1, (0, 0), True), (64, 6, 2, 64, (0, 300), True), (64, 8, 1, 65, (0, 5, 250), True),
-    (64, 32, 4, 128, (0, 64), False), (64, 16, 2, 256, (0, 0, 100, 0), True), (128, 8, 1, 100, (0,) * 12 + (7, 256, 0, 0), True),
-    (128, 24, 8, 16, (0,) * 26, True), (128, 4, 4, 130, (0,) * 10, False)])
-def test_rotation_and_attention_of_short_chunks_in_one_launch(mv, D, Hq, Hkv, S, starts, rot):
+# four sequences on, 256; heads of 128 in batches; tiles that end inside 64 keys, one, three and eight query heads to a key/value head; cached
+# tokens in front of some chunks, up to a page and a tile, two tiles, and many; no rotation.  hole: a sequence's page, by column, that was
+# never allocated: nothing is stored there, and rows that see a key of it are not compared
+@pytest.mark.parametrize("D,Hq,Hkv,S,starts,rot,hole", [
+    (64, 32, 4, 37, (0,), True, None), (64, 4, 4, 1, (0, 0), True, None), (64, 6, 2, 64, (0, 300), True, None),
+    (64, 8, 1, 65, (0, 5, 250), True, None), (64, 32, 4, 128, (0, 64), False, None), (64, 16, 2, 256, (0, 0, 100, 0), True, None),
+    (128, 8, 1, 100, (0,) * 12 + (7, 256, 0, 0), True, None), (128, 24, 8, 16, (0,) * 26, True, None),
+    (128, 4, 4, 130, (0,) * 10, False, None), (64, 8, 8, 33, (63, 64, 65, 127, 128, 129, 700), True, None),
+    (128, 16, 2, 50, (63, 64, 65, 127, 128, 129, 700, 1000) * 4, True, None), (64, 4, 4, 1, (0, 0), True, (1, 0)),
+    (64, 6, 2, 100, (0, 200), True, (1, 2)), (64, 32, 4, 128, (0, 64), False, (1, 1)), (128, 8, 1, 100, (0,) * 12 + (7, 256, 0, 0), True, (13, 2))])
+def test_rotation_and_attention_of_short_chunks_in_one_launch(mv, D, Hq, Hkv, S, starts, rot, hole):
     from micro_vllm_amd import _native as nv
     from micro_vllm_amd.core.paged_attention import rotary_tables
     L, B, page = nv.lib(), len(starts), 128
@@ -435,10 +439,10 @@ def test_rotation_and_attention_of_short_chunks_in_one_launch(mv, D, Hq, Hkv, S,
     caches = [torch.randn(n_pages, page, Hkv, D, generator=g).bfloat16().to(DEV) for _ in range(2)]
     qkv = torch.randn(B * S, n + 8, generator=g).bfloat16().to(DEV)[:, :n]
     bt = torch.randperm(n_pages, generator=g).to(torch.int32).reshape(B, per)
-    if B == 2:
-        bt[1, -1] = -1
+    if hole:
+        bt[hole] = -1
     bt, sl = bt.to(DEV), torch.tensor(starts, dtype=torch.int32, device=DEV)
-    cos, sin = rotary_tables(D, 300, device=DEV) if rot else (None, None)     # the last positions take the table's last row
+    cos, sin = rotary_tables(D, 300, device=DEV) if rot else (None, None)     # positions past it take the table's last row
     found = []
     for one in (False, True):
         rows, (kc, vc) = torch.empty(B * S, n + 8, dtype=torch.bfloat16, device=DEV)[:, :n].copy_(qkv), [c.clone() for c in caches]
@@ -454,7 +458,9 @@ def test_rotation_and_attention_of_short_chunks_in_one_launch(mv, D, Hq, Hkv, S,
             assert rc == 0
             rc = L.mv_paged_attn_prefill(*head, *kv, *turn[3:], out.data_ptr(), Hq * D, *shape, D ** -0.5, nv.stream_ptr())
         assert rc == 0
-        found.append((out.view(B, S, -1)[:1] if B == 2 else out, kc, vc))
+        if hole:
+            out.view(B, S, -1)[hole[0], max(hole[1] * page - starts[hole[0]], 0):] = 0
+        found.append((out, kc, vc))
     for a, b in zip(*found):
         assert torch.equal(a, b)
     assert not torch.equal(found[0][1], caches[0])
