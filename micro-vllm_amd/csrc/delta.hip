@@ -520,7 +520,7 @@ __global__ __launch_bounds__(kIntra, 4) void delta_chunk_intra_kernel(DeltaArgs 
     // diagonal blocks of A and B: lane (r, g) holds column s = r, state rows 16 m + 4 g .. + 3, and walks the tokens t behind its s.  Two waves
     // share a block: the first takes t up to 7, the second those behind, whose first half it walks for the product alone.  A token's
     // own values come from the lane of its row (DPP); read from LDS by all sixteen they were 33 reads a wave and step.  A lone chunk of 16 heads of
-    // 128 x 128 33.7 -> 26.5 us, 23 of them 73.6 -> 61, with the places below and the tiles' reads in front of their products.
+    // 128 x 128 32.3 -> 27.0 us, 16 of them 40.4 -> 33.4, 23 70 -> 59, with the places below and the tiles' reads in front of their products.
     {
         const int blk = wv & 3;
         const bool late = wv >= 4;

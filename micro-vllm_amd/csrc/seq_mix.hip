@@ -1882,8 +1882,8 @@ struct StepRotary {
 // qk_rotary_store_kernel forms them) while the first tiles are on their way; the turned queries lie in LDS, and the tile that holds
 // the token's own position takes key and value from there too: the page is written by the first split and read by later steps.
 // What another split reads of that place meanwhile is not used.
-// One launch against two (us, 8 heads of 128 on 2, a gate of 4096 beside them): one token bf16 at 45 keys 8.3 -> 6.2, 300 11.7 -> 11.0,
-// 1100 19.5 -> 19.1; fp32 10.6 -> 8.3, 16.4 -> 15.0, 20.3 -> 19.6; 8 tokens of 16 heads on 4 at 500 keys 14.6 -> 13.3.
+// One launch against two (us, 8 heads of 128 on 2, a gate of 4096 beside them): one token bf16 at 45 keys 8.3 -> 6.0, 300 11.8 -> 10.4,
+// 1100 19.0 -> 18.2; fp32 10.8 -> 8.1, 13.3 -> 11.6, 16.6 -> 15.2; 8 tokens of 16 heads on 4 at 500 keys 14.5 -> 13.1.
 template <bool F32, int HEADS, int NW, int KS, int VE, bool ROT = false>
 __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q, int64_t ldq, const void* kc_, const void* vc_,
                                                               void* out_, int64_t ldo, float* part, PagedRows pr,

@@ -949,8 +949,9 @@ static int launch_dot_stage(const GemmArgs& a, int grid, hipStream_t s) {
 
 // Tiles per stage: four for one and two rows, two for three and four (register budget: 128 VGPRs at 16 waves per CU).  Where a wave
 // has no more than four tiles of a strip (k <= 1024 on eight waves) two as well: a stage of four would hold them all, and the second
-// one ask for its last tile four times over (one row, us, four -> two a stage: 32000 x 1024 15.3 -> 11.6,
-// 9472 x 1024 7.0 -> 5.3, 1024 x 1024 3.5 -> 3.3, 8192 x 512 4.9 -> 4.3).  The sums are the same bits.
+// one ask for its last tile four times over (one row, us, four -> two a stage: 32000 x 1024 15.2 -> 11.5, 9472 x 1024 6.9 -> 5.3, 1024 x
+// 1024 3.5 -> 3.3, 8192 x 512 5.0 -> 4.3; two rows 32000 x 1024 15.0 -> 11.5, 1024 x 1024 4.0 -> 3.4, with a norm in front 15.5 -> 12.5, 4.6 -> 4.2;
+// slices of a longer k, 256 x 4096 5.5 -> 5.3; no slower over 22 shapes of plain, gated and normed forms).  The sums are the same bits.
 template <int M, int GW, int PRO, bool ACT = false>
 static int launch_dot(const GemmArgs& a, int grid, hipStream_t s) {
     if constexpr (M <= 2 && GW == 8) {
