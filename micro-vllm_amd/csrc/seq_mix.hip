@@ -1884,7 +1884,8 @@ struct StepRotary {
 // What another split reads of that place meanwhile is not used.
 // One launch against two (us, 8 heads of 128 on 2, a gate of 4096 beside them): one token bf16 at 45 keys 8.3 -> 6.0, 300 11.8 -> 10.4,
 // 1100 19.0 -> 18.2; fp32 10.8 -> 8.1, 13.3 -> 11.6, 16.6 -> 15.2; 8 tokens of 16 heads on 4 at 500 keys 14.5 -> 13.1.
-template <bool F32, int HEADS, int NW, int KS, int VE, bool ROT = false>
+// OWN: bf16 queries are not shared (kShareQ below)
+template <bool F32, int HEADS, int NW, int KS, int VE, bool ROT = false, bool OWN = false>
 __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q, int64_t ldq, const void* kc_, const void* vc_,
                                                               void* out_, int64_t ldo, float* part, PagedRows pr,
                                                               const float* slopes, const float* sinks, int H, int G,
@@ -1901,9 +1902,10 @@ __global__ __launch_bounds__(64 * NW) void window_attn_few_kernel(const float* q
     // bf16 keys: the queries' three parts, formed once for the workgroup: a value's split is some eight instructions, and a wave has up to 32
     // values a lane to it, while what bounds a tile here is the issue slots of the waves that share a unit (one token of 8 heads on 2 of 128,
     // 45 keys, 7.35 -> 5.45 us, 1100 19.6 -> 17.2).  Not worth the barrier with a single head (4.7 -> 5.0 at 45 keys of a launch of its own) and with
-    // 8 values a lane (each wave its own, shared: 16 heads of 32 on 4 at 45 keys 4.0, 4.6, at 1100 11.0 both); 16 are even (45 and 1100 keys: 16
-    // heads of 64 on 4 5.2, 4.9 and 13.1, 12.7, 4 on 2 4.4, 4.7 and 12.4, 12.5).  The turned queries lie in LDS either way
-    constexpr bool kShareQ = !F32 && (ROT || (HEADS > 1 && KS * HB > 1));
+    // 8 values a lane (each wave its own, shared: 16 heads of 32 on 4 at 45 keys 4.0, 4.6, at 1100 11.0 both); 16 are for four heads, which load twice
+    // two heads' rows (16 of 64 on 4 at 45 and 1100 keys 5.2, 4.9 and 13.1, 12.7), and not for two or three (OWN; 4 of 64 on 2 4.4, 4.7 and 12.4, 12.5,
+    // 12 on 4 5.1, 5.3 and 15.2 both).  The turned queries lie in LDS either way
+    constexpr bool kShareQ = !F32 && (ROT || (HEADS > 1 && KS * HB > 1 && !OWN));
     __shared__ __attribute__((aligned(16))) uint16_t qp[kShareQ ? 3 * RT * d : 8];
     if constexpr (ROT) {
         if ((int)blockIdx.y >= splits) {
@@ -3182,17 +3184,19 @@ int mv_window_attn(const float* q, int64_t ldq, const void* k_cache, const void*
             const int pieces = fp.pieces;
             const bool wide = fp.wide;
             int nw = 0;      // (0: a head shape without an instance)
-#define MV_WA_FEW(F32_, HB_, NW_, KS_, VE_)                                                                            \
-    hipLaunchKernelGGL((window_attn_few_kernel<F32_, HB_, NW_, KS_, VE_>), dim3((unsigned)groups, pieces), dim3(64 * NW_), 0, s, \
+#define MV_WA_FEW(F32_, HB_, NW_, KS_, VE_, OWN_)                                                                      \
+    hipLaunchKernelGGL((window_attn_few_kernel<F32_, HB_, NW_, KS_, VE_, false, OWN_>), dim3((unsigned)groups, pieces), dim3(64 * NW_), 0, s, \
                        q, ldq, k_cache, v_cache, out, ldo, part, pr, slopes, sinks, heads, kv_heads, scale, window, keep_first, \
                        row_len, skip_len, pieces, gate, ldg, chunked, StepRotary{});                                   \
     nw = NW_
 #define MV_WA_FEW_HB(F32_, KS_, VE_)                                                                                   \
     do {                                                                                                               \
-        if (top > 4) { if (wide) { MV_WA_FEW(F32_, 8, 8, KS_, VE_); } else { MV_WA_FEW(F32_, 8, 4, KS_, VE_); } }      \
-        else if (top > 1) { if (wide) { MV_WA_FEW(F32_, 4, (F32_ ? 8 : 16), KS_, VE_); } else { MV_WA_FEW(F32_, 4, 4, KS_, VE_); } } \
-        else if (wide) { MV_WA_FEW(F32_, 1, 16, KS_, VE_); }                                                           \
-        else { MV_WA_FEW(F32_, 1, 4, KS_, VE_); }                                                                      \
+        constexpr bool own = !F32_ && KS_ == 2;      /* of two or three heads to a key */                              \
+        if (top > 4) { if (wide) { MV_WA_FEW(F32_, 8, 8, KS_, VE_, false); } else { MV_WA_FEW(F32_, 8, 4, KS_, VE_, false); } } \
+        else if (top == 4) { if (wide) { MV_WA_FEW(F32_, 4, (F32_ ? 8 : 16), KS_, VE_, false); } else { MV_WA_FEW(F32_, 4, 4, KS_, VE_, false); } } \
+        else if (top > 1) { if (wide) { MV_WA_FEW(F32_, 4, (F32_ ? 8 : 16), KS_, VE_, own); } else { MV_WA_FEW(F32_, 4, 4, KS_, VE_, own); } } \
+        else if (wide) { MV_WA_FEW(F32_, 1, 16, KS_, VE_, false); }                                                    \
+        else { MV_WA_FEW(F32_, 1, 4, KS_, VE_, false); }                                                               \
     } while (0)
 #define MV_WA_FEW_D(F32_)                                                                                              \
     do {                                                                                                               \
