@@ -758,7 +758,7 @@ __global__ __launch_bounds__(kIntra, 4) void delta_chunk_intra_kernel(DeltaArgs 
 // state rows of the 16-row tiles w, w + 4, ...; the state (as operand) and U pass through LDS.  NT: 16-row tiles; FULL: the state has exactly NT of them (no tests between the products).
 // SETS: chunks whose operands are in registers, the ones in hand among them.  Two, in registers that let two workgroups share a unit: three
 // took all of a SIMD's at 128 state rows, and bought nothing where a unit has one workgroup either (whole calls, us, three -> two; 16 heads of
-// 128 x 128: 8 rows of three chunks 126.9 -> 114.2, 16 of one 100.1 -> 82.8, one row of 23 135.7 -> 134.3, of one chunk 46.4 -> 46.7, one of 16
+// 128 x 128: 8 rows of three chunks 126.9 -> 114.2, 16 of one 100.1 -> 82.8, one row of 23 135.7 -> 134.3, of one chunk, this launch alone, 6.0 -> 6.1, one of 16
 // beside seven tokens 95.4 -> 94.7; 32 of 64 x 64: 32 rows of two 247.7 -> 235.6, one of 16 74.5 -> 73.3; 32 of 32 x 32: 16 rows of four 143.9
 // -> 138.6, one of 16 55.5 -> 54.9).  With 10 tiles two would spill at two waves a SIMD: three, and one workgroup a unit.
 template <int NT, bool FULL, int SETS = NT <= 8 ? 2 : 3>
@@ -863,14 +863,18 @@ __global__ __launch_bounds__(256, SETS == 2 ? 2 : 1) void delta_chunk_carry_kern
         if (c + SETS < nch) fetch(unit + SETS * (int64_t)a.H, cur);
         __syncthreads();
     };
+    // (the first of each round of sets under no condition: with one, a lone chunk took 0.5 to 1 us more of 4 to 8, 32 rows with ten tiles 119 us
+    // instead of 107)
     Operands x[SETS];
+    fetch(u0, x[0]);
 #pragma unroll
-    for (int i = 0; i < SETS; ++i)
+    for (int i = 1; i < SETS; ++i)
         if (nch > i) fetch(u0 + i * (int64_t)a.H, x[i]);
     __syncthreads();
     for (int c = 0; c < nch; c += SETS) {
+        body(x[0], c);
 #pragma unroll
-        for (int i = 0; i < SETS; ++i)
+        for (int i = 1; i < SETS; ++i)
             if (c + i < nch) body(x[i], c + i);
     }
 #pragma unroll
