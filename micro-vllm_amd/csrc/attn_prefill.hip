@@ -84,18 +84,23 @@ static bool pf_eight_waves(int bs, int seq, int hkv, int g) {
 }
 
 // Chunks whose attention turns its own queries and keys (paged_attn_prefill_kernel, ROT) against the rotation's own launch in front of it.
-// Heads of 64: up to 128 tokens, up to 256 from four sequences on (us, two launches -> one, 32 heads on 4: 37 tokens 8.0 -> 6.5, 128 9.3 -> 8.0,
-// 256 level; 4 x 256 15.0 -> 12.1, 16 x 64 11.7 -> 7.7).  Heads of 128, whose turning is twice the work of a workgroup that has
-// half its lanes' time: from four sequences and 2 M values of q, k and v on, where the separate launch takes as long (32 heads on 8: 37 tokens
-// 9.9 -> 10.5, 4 x 37 10.6 -> 10.9, 4 x 100 14.3 -> 13.4, 16 x 64 17.4 -> 12.2, 16 x 256 48.1 -> 41.9; 8 on 1: 4 x 256 16.4 -> 19.2, 16 x 128
-// 14.7 -> 13.3).
-// Behind cached tokens, which the host does not see, heads of 64 stay level or ahead (32 on 4: 37 tokens behind 300 14.4 -> 14.4, behind 2000 46.2
-// -> 44.8; 16 x 256 behind 2000 121 -> 125; 8 on 8, 128 behind 300 15.7 -> 17.3), heads of 128 lose up to a tenth where many tiles of them are
-// few workgroups' (32 on 8: 4 x 256 behind 300 32.5 -> 32.8, behind 2000 78 -> 86; 32 x 64 behind 2000 112 -> 109).
+// Heads of 64 (us, two launches -> one): up to 64 tokens (32 heads on 4: 37 tokens 8.3 -> 6.8, 16 x 64 11.8 -> 8.0), up to 128 where a key has more
+// than one head (128 tokens 9.6 -> 8.4; 8 on 8 9.7 -> 9.5) or the batch is large (8 x 100 of 16 on 16 12.0 -> 9.9), up to 256 from four sequences on
+// if q, k and v are a million values (4 x 256 of 32 on 4 15.0 -> 12.6, 16 x 256 28.7 -> 22.7).  Heads of 128, whose turning is
+// twice the work of a workgroup that has half its lanes' time: from four sequences and 3.5 M values on, where the separate launch takes as
+// long, with more than one head to a key (32 on 8: 16 x 37 14.9 -> 12.1, 16 x 64 17.5 -> 12.5, 4 x 256 23.2 -> 20.7, 16 x 256 47.0 -> 41.9; left to
+// two launches: 4 x 100 14.5 -> 13.7; 8 on 1, 8 x 256 18.5 -> 19.6; 16 on 16, 4 x 256 22.1 -> 21.9).
+// What is left out gains little from position 0 and loses behind cached tokens, which the host does not see, as the first rows are asked
+// for twice there and one tile more goes through the chunk's tests: behind 300 and 2000 8 on 8 heads of 64, 128 tokens, 16.0 -> 17.7 and 48.5 -> 49.4;
+// of 128, 4 x 128 of 32 on 8 24.5 -> 26.1 and 71.3 -> 75.5, 8 x 128 of 16 on 16 27.4 -> 31.5 and 74.8 -> 80.9.  What is in gains 9 to 29 % from
+// position 0; behind 300 and 2000 heads of 64 lose up to 5 % and nothing (32 on 4: 128 tokens 16.0 -> 16.3 and 48.2 -> 47.7, 16 x 256 41.1 -> 40.2 and
+// 117 -> 115), of 128 up to 6 % and 5 % (32 on 8: 16 x 256 70.7 -> 75.2 and 205 -> 203, 4 x 256 32.3 -> 32.8 and 79 -> 82, 16 x 64 26.0 both and 74.2 ->
+// 74.9, 32 x 64 38.9 -> 36.6 and 117 -> 111).
 static bool pf_rotates(int bs, int seq, int hq, int hkv, int d) {
     if (pf_eight_waves(bs, seq, hkv, hq / hkv)) return false;
-    if (d == 64) return seq <= 128 || (seq <= 256 && bs >= 4);
-    return seq <= 256 && bs >= 4 && (int64_t)bs * seq * (hq + 2 * hkv) * d >= 2000000;
+    const int64_t values = (int64_t)bs * seq * (hq + 2 * hkv) * d;
+    if (d == 64) return seq <= 64 || (seq <= 128 && (hq > hkv || values >= 2000000)) || (seq <= 256 && bs >= 4 && values >= (hq > hkv ? 1000000 : 2000000));
+    return seq <= 256 && bs >= 4 && hq > hkv && values >= 3500000;
 }
 
 // ------------------------------------------------------------------ rotate + store
@@ -227,8 +232,10 @@ struct PfArgs {
 // turn in the registers that hold them (a lane has both halves of its pairs); the chunk's own keys and values are staged from the
 // projection's rows, the keys turned on the way to LDS, and every workgroup writes those of its own query positions to their pages.
 // Each workgroup turns all the chunk's keys that it sees, so it is for chunks that few workgroups share: pf_rotates.
+// (Heads of 64: 168 registers, three workgroups to a unit as without ROT; at 178 they were two, and 16 x 256 of 32 heads on 4 behind 2000 cached tokens
+// took 123.5 us instead of 115.2, the two launches 116.9.)
 template <int D, int NW, bool ROT = false>
-__global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_kernel(PfArgs a) {
+__global__ __launch_bounds__(NW * 64, NW == 4 ? (D == 64 ? 3 : 2) : 1) void paged_attn_prefill_kernel(PfArgs a) {
     constexpr int NT = NW * 64;        // threads
     constexpr int KT = 64;             // keys per LDS tile
     constexpr int KS = D / 32;         // k-steps of K.Q^T
@@ -294,18 +301,19 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     if (ROT && a.cos) load_turns();
 
     // K/V staging: thread moves vectors t + 256 j of the 64 x VPR tile
-    uint4 kr[NV], vr[NV];
     auto tile_page = [&](int t) {
         // column clamped into the table: keys past its last column have no page (a contract breach:
         // such keys read page-table garbage before; now they read the last column's page)
         const int pg = bt[min((t * KT) >> a.page_shift, a.bt_stride - 1)];
         return (pg >= 0 && pg < a.num_pages) ? pg : 0;   // unallocated entry: stay inside the cache
     };
-    // ROT: a thread has both halves of its pairs, kr[j] and kr[j + NV / 2], and their turn; values as before
+    // ROT: a thread has both halves of its pairs, m.k[j] and m.k[j + NV / 2], and their turn; values as before
     const uint16_t* knew = a.q + (int64_t)b * a.S * a.q_stride + (int64_t)(a.hq + kvh) * D;
     const uint16_t* vnew = knew + (int64_t)a.hkv * D;
-    uint4 cr[ROT ? NV / 2 : 1], sr[ROT ? NV / 2 : 1];
-    int kpg[ROT ? NV / 2 : 1], vpg[ROT ? NV : 1];
+    struct Rows {
+        uint4 k[NV], v[NV], cos[ROT ? NV / 2 : 1], sin[ROT ? NV / 2 : 1];
+        int kpg[ROT ? NV / 2 : 1], vpg[ROT ? NV : 1];
+    };
     // the page of a chunk's token that this workgroup writes, else -1 (as in rope_store_kernel)
     auto own_page = [&](int kp, int i) {
         const int pos = start + i;
@@ -314,7 +322,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
         return pg < a.num_pages ? pg : -1;
     };
     // own: the tile may have keys of the chunk (ROT); tiles of nothing but cached tokens are staged as the plain form stages them
-    auto g_load = [&](auto own, int t, int pg) {
+    auto g_load = [&](auto own, Rows& m, int t, int pg) {
         if constexpr (decltype(own)::value) {
 #pragma unroll
             for (int j = 0; j < NV / 2; ++j) {
@@ -322,14 +330,14 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
                 const int kp = min(t * KT + row, last_key), i = kp - p0;
                 const uint16_t* src = i >= 0 ? knew + (int64_t)i * a.q_stride
                                              : a.k_cache + (((int64_t)pg * a.page + (kp & (a.page - 1))) * a.hkv + kvh) * D;
-                kr[j] = ld16(src + ch * 8);
-                kr[j + NV / 2] = ld16(src + D / 2 + ch * 8);
+                m.k[j] = ld16(src + ch * 8);
+                m.k[j + NV / 2] = ld16(src + D / 2 + ch * 8);
                 if (a.cos) {
                     const int64_t ro = (int64_t)min(max(start + i, 0), a.rot_max_pos - 1) * (D / 2) + ch * 8;
-                    cr[j] = ld16(a.cos + ro);
-                    sr[j] = ld16(a.sin + ro);
+                    m.cos[j] = ld16(a.cos + ro);
+                    m.sin[j] = ld16(a.sin + ro);
                 }
-                kpg[j] = own_page(t * KT + row, t * KT + row - p0);
+                m.kpg[j] = own_page(t * KT + row, t * KT + row - p0);
             }
 #pragma unroll
             for (int j = 0; j < NV; ++j) {
@@ -337,8 +345,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
                 const int kp = min(t * KT + row, last_key), i = kp - p0;
                 const uint16_t* src = i >= 0 ? vnew + (int64_t)i * a.q_stride
                                              : a.v_cache + (((int64_t)pg * a.page + (kp & (a.page - 1))) * a.hkv + kvh) * D;
-                vr[j] = ld16(src + ch * 8);
-                vpg[j] = own_page(t * KT + row, t * KT + row - p0);
+                m.v[j] = ld16(src + ch * 8);
+                m.vpg[j] = own_page(t * KT + row, t * KT + row - p0);
             }
             return;
         }
@@ -347,11 +355,11 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
             const int v = threadIdx.x + NT * j, row = v / VPR, ch = v % VPR;
             const int kp = min(t * KT + row, last_key);
             const int64_t off = (((int64_t)pg * a.page + (kp & (a.page - 1))) * a.hkv + kvh) * D + ch * 8;
-            kr[j] = ld16(a.k_cache + off);
-            vr[j] = ld16(a.v_cache + off);
+            m.k[j] = ld16(a.k_cache + off);
+            m.v[j] = ld16(a.v_cache + off);
         }
     };
-    auto l_store = [&](auto own, int t) {
+    auto l_store = [&](auto own, Rows& m, int t) {
         const int buf = t & 1;
         if constexpr (decltype(own)::value) {
             auto slot = [&](int pg, int row) {
@@ -361,28 +369,28 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
 #pragma unroll
             for (int j = 0; j < NV / 2; ++j) {
                 const int v = threadIdx.x + NT * j, row = v / (VPR / 2), ch = v % (VPR / 2);
-                if (a.cos && min(t * KT + row, last_key) >= p0) rope_pairs(kr[j], kr[j + NV / 2], cr[j], sr[j]);
-                *reinterpret_cast<uint4*>(&kL[buf][row * KROW + ch * 16]) = kr[j];
-                *reinterpret_cast<uint4*>(&kL[buf][row * KROW + D + ch * 16]) = kr[j + NV / 2];
-                if (kpg[j] >= 0) {
-                    uint16_t* dst = const_cast<uint16_t*>(a.k_cache) + slot(kpg[j], row);
-                    st16(dst + ch * 8, kr[j]);
-                    st16(dst + D / 2 + ch * 8, kr[j + NV / 2]);
+                if (a.cos && min(t * KT + row, last_key) >= p0) rope_pairs(m.k[j], m.k[j + NV / 2], m.cos[j], m.sin[j]);
+                *reinterpret_cast<uint4*>(&kL[buf][row * KROW + ch * 16]) = m.k[j];
+                *reinterpret_cast<uint4*>(&kL[buf][row * KROW + D + ch * 16]) = m.k[j + NV / 2];
+                if (m.kpg[j] >= 0) {
+                    uint16_t* dst = const_cast<uint16_t*>(a.k_cache) + slot(m.kpg[j], row);
+                    st16(dst + ch * 8, m.k[j]);
+                    st16(dst + D / 2 + ch * 8, m.k[j + NV / 2]);
                 }
             }
 #pragma unroll
             for (int j = 0; j < NV; ++j) {
                 const int v = threadIdx.x + NT * j, row = v / VPR, ch = v % VPR;
-                *reinterpret_cast<uint4*>(&vL[buf][row * VROW + ch * 16]) = vr[j];
-                if (vpg[j] >= 0) st16(const_cast<uint16_t*>(a.v_cache) + slot(vpg[j], row) + ch * 8, vr[j]);
+                *reinterpret_cast<uint4*>(&vL[buf][row * VROW + ch * 16]) = m.v[j];
+                if (m.vpg[j] >= 0) st16(const_cast<uint16_t*>(a.v_cache) + slot(m.vpg[j], row) + ch * 8, m.v[j]);
             }
             return;
         }
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int v = threadIdx.x + NT * j, row = v / VPR, ch = v % VPR;
-            *reinterpret_cast<uint4*>(&kL[buf][row * KROW + ch * 16]) = kr[j];
-            *reinterpret_cast<uint4*>(&vL[buf][row * VROW + ch * 16]) = vr[j];
+            *reinterpret_cast<uint4*>(&kL[buf][row * KROW + ch * 16]) = m.k[j];
+            *reinterpret_cast<uint4*>(&vL[buf][row * VROW + ch * 16]) = m.v[j];
         }
     };
 
@@ -394,7 +402,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     float mrun[2] = {kPfNegBig, kPfNegBig}, lrun[2] = {0.f, 0.f};
 
     int pg_next = tile_page(0);
-    g_load(Own{}, 0, pg_next);
+    Rows m0;
+    g_load(Own{}, m0, 0, pg_next);
     if constexpr (ROT) {
         __builtin_amdgcn_sched_barrier(0);
         const int true_start = a.start[b];
@@ -407,8 +416,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
             p0 = moved;
             ntiles = last_key / KT + 1;
             if (a.cos) load_turns();
-            if (p0 >= KT) g_load(std::false_type{}, 0, pg_next);
-            else g_load(Own{}, 0, pg_next);
+            if (p0 >= KT) g_load(std::false_type{}, m0, 0, pg_next);
+            else g_load(Own{}, m0, 0, pg_next);
         }
         if (a.cos) {
 #pragma unroll
@@ -428,8 +437,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
     for (int o = 1; o < 16; o <<= 1) wave_min_limit = min(wave_min_limit, __shfl_xor(wave_min_limit, o, 64));
     wave_min_limit = __builtin_amdgcn_readfirstlane(wave_min_limit);
     pg_next = ntiles > 1 ? tile_page(1) : 0;
-    if (ROT && p0 >= KT) l_store(std::false_type{}, 0);
-    else l_store(Own{}, 0);
+    if (ROT && p0 >= KT) l_store(std::false_type{}, m0, 0);
+    else l_store(Own{}, m0, 0);
     __syncthreads();
 
     // transposed-read lane address inside a 16-key x 16-column block pair
@@ -438,13 +447,14 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
 
     auto pass = [&](auto own, int t) {      // tile t, while the next (own: see g_load) is on its way
         const int buf = t & 1;
+        Rows m;
 #ifdef MV_EXP_NO_KVLOAD
         const bool more = false;   // timing experiment only (wrong results): every tile re-uses the first two
 #else
         const bool more = t + 1 < ntiles;
 #endif
         if (more) {
-            g_load(own, t + 1, pg_next);
+            g_load(own, m, t + 1, pg_next);
             if (t + 2 < ntiles) pg_next = tile_page(t + 2);
         }
         // The 64 keys of the tile in one pass: 32 MFMAs for S^T, one softmax update over 16 scores
@@ -555,7 +565,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void paged_attn_prefill_k
                     oacc[mt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[mt][h], oacc[mt][dt], 0, 0, 0);
             }
         }
-        if (more) l_store(own, t + 1);
+        if (more) l_store(own, m, t + 1);
         __syncthreads();
     };
     int tile = 0;

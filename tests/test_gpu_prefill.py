@@ -421,14 +421,18 @@ def test_layers_that_are_not_alike_go_one_by_one(mv, odd):
 # rotation, stores and attention of short chunks in one launch are the two launches, bit for bit: heads of 64 up to 128 tokens and, from
 # four sequences on, 256; heads of 128 in batches; tiles that end inside 64 keys, one, three and eight query heads to a key/value head; cached
 # tokens in front of some chunks, up to a page and a tile, two tiles, and many; no rotation.  hole: a sequence's page, by column, that was
-# never allocated: nothing is stored there, and rows that see a key of it are not compared
+# never allocated: nothing is stored there, and rows that see a key of it are not compared.  Heads of 128 with a key each, or in batches of fewer
+# than 3.5 M values, and heads of 64 with a key each past 64 tokens in small batches, take the two launches either way
 @pytest.mark.parametrize("D,Hq,Hkv,S,starts,rot,hole", [
     (64, 32, 4, 37, (0,), True, None), (64, 4, 4, 1, (0, 0), True, None), (64, 6, 2, 64, (0, 300), True, None),
     (64, 8, 1, 65, (0, 5, 250), True, None), (64, 32, 4, 128, (0, 64), False, None), (64, 16, 2, 256, (0, 0, 100, 0), True, None),
     (128, 8, 1, 100, (0,) * 12 + (7, 256, 0, 0), True, None), (128, 24, 8, 16, (0,) * 26, True, None),
     (128, 4, 4, 130, (0,) * 10, False, None), (64, 8, 8, 33, (63, 64, 65, 127, 128, 129, 700), True, None),
+    (128, 8, 1, 100, (0,) * 26 + (7, 256), True, None), (128, 24, 8, 16, (0,) * 42 + (30,), True, None), (128, 8, 4, 130, (0,) * 14, False, None),
+    (64, 8, 8, 100, (0, 40), True, None), (64, 16, 16, 100, (0,) * 7 + (90,), True, None), (64, 8, 2, 200, (0, 0, 64, 100), True, None),
     (128, 16, 2, 50, (63, 64, 65, 127, 128, 129, 700, 1000) * 4, True, None), (64, 4, 4, 1, (0, 0), True, (1, 0)),
-    (64, 6, 2, 100, (0, 200), True, (1, 2)), (64, 32, 4, 128, (0, 64), False, (1, 1)), (128, 8, 1, 100, (0,) * 12 + (7, 256, 0, 0), True, (13, 2))])
+    (64, 6, 2, 100, (0, 200), True, (1, 2)), (64, 32, 4, 128, (0, 64), False, (1, 1)), (128, 8, 1, 100, (0,) * 12 + (7, 256, 0, 0), True, (13, 2)),
+    (128, 8, 1, 100, (0,) * 25 + (7, 256, 0), True, (26, 2))])
 def test_rotation_and_attention_of_short_chunks_in_one_launch(mv, D, Hq, Hkv, S, starts, rot, hole):
     from micro_vllm_amd import _native as nv
     from micro_vllm_amd.core.paged_attention import rotary_tables
@@ -443,6 +447,9 @@ def test_rotation_and_attention_of_short_chunks_in_one_launch(mv, D, Hq, Hkv, S,
         bt[hole] = -1
     bt, sl = bt.to(DEV), torch.tensor(starts, dtype=torch.int32, device=DEV)
     cos, sin = rotary_tables(D, 300, device=DEV) if rot else (None, None)     # positions past it take the table's last row
+    values = B * S * n
+    taken = not rot or (Hq > Hkv and values >= 3500000 if D == 128 else
+                        S <= 64 or values >= (2000000 if Hq == Hkv else 1000000 if S > 128 else 0))
     found = []
     for one in (False, True):
         rows, (kc, vc) = torch.empty(B * S, n + 8, dtype=torch.bfloat16, device=DEV)[:, :n].copy_(qkv), [c.clone() for c in caches]
@@ -452,7 +459,7 @@ def test_rotation_and_attention_of_short_chunks_in_one_launch(mv, D, Hq, Hkv, S,
         kv, shape = (kc.data_ptr(), vc.data_ptr()), (B, S, Hq, Hkv, D, page, n_pages)
         if one:
             rc = L.mv_rope_attn_prefill(*head, *turn, *kv, out.data_ptr(), Hq * D, *shape, D ** -0.5, nv.stream_ptr())
-            assert torch.equal(rows, qkv)         # the one launch was taken: rows stay as projected
+            assert torch.equal(rows, qkv) == taken      # rows of the one launch stay as projected
         else:
             rc = L.mv_rope_store_prefill(*head, *turn, *kv, *shape, nv.stream_ptr())
             assert rc == 0
