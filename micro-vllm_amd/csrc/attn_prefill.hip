@@ -448,11 +448,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? (D == 64 ? 3 : 2) : 1) void page
     auto pass = [&](auto own, int t) {      // tile t, while the next (own: see g_load) is on its way
         const int buf = t & 1;
         Rows m;
-#ifdef MV_EXP_NO_KVLOAD
-        const bool more = false;   // timing experiment only (wrong results): every tile re-uses the first two
-#else
         const bool more = t + 1 < ntiles;
-#endif
         if (more) {
             g_load(own, m, t + 1, pg_next);
             if (t + 2 < ntiles) pg_next = tile_page(t + 2);
@@ -482,21 +478,6 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? (D == 64 ? 3 : 2) : 1) void page
         // tiles wholly at or below every row's last key (all but the one or two on the diagonal)
         // need no mask; keys past the last valid one were clamped on load and are masked here
         const bool all_valid = kb + KT - 1 <= wave_min_limit;   // uniform
-#ifdef MV_EXP_NO_SOFTMAX
-        // timing experiment only (wrong results): the scores go to the second product as they are
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                uint4 pk;
-                pk.x = pack_bf16x2(sacc[mt][2 * h][0], sacc[mt][2 * h][1]);
-                pk.y = pack_bf16x2(sacc[mt][2 * h][2], sacc[mt][2 * h][3]);
-                pk.z = pack_bf16x2(sacc[mt][2 * h + 1][0], sacc[mt][2 * h + 1][1]);
-                pk.w = pack_bf16x2(sacc[mt][2 * h + 1][2], sacc[mt][2 * h + 1][3]);
-                pf[mt][h] = __builtin_bit_cast(bf16x8_t, pk);
-            }
-        if (false)
-#endif
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
             // raw scores; the scale (positive) is applied to the maximum and inside the exponent

@@ -70,8 +70,7 @@ struct PGemmArgs {
 
 #ifdef MV_GEMM_STAMP
 // Phase stamps of one wave (build variant for tools/stamp_gemm_prefill.py): s_memtime ticks at four
-// points of every k stage, for the workgroup selected by kStampBlock.  MV_EXP_NO_WLOAD /
-// MV_EXP_NO_XREAD additionally remove one operand path (wrong results, timing only).
+// points of every k stage, for the workgroup selected by kStampBlock.
 constexpr int kStampBlock = 777;
 static __device__ unsigned long long g_stamp[4 * 512];
 #define MV_STAMP(slot)                                                            \
@@ -106,13 +105,7 @@ static __device__ unsigned long long g_wstamp[4096];
 #else
 #define MV_WSTAMP(i) do {} while (0)
 #endif
-// MV_EXP_NO_MFMA (timing experiment, wrong results): operands are delivered and consumed by an empty
-// asm statement instead of the matrix instruction; MV_EXP_NO_BARRIER drops the per-stage barrier.
-#ifdef MV_EXP_NO_MFMA
-#define MV_MFMA(c, a_, b_) asm volatile("" : "+v"(c) : "v"(a_), "v"(b_))
-#else
 #define MV_MFMA(c, a_, b_) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_, b_, c, 0, 0, 0)
-#endif
 
 // One wave's 64 (n) x 128 (m) block of accumulators to memory, with the projection epilogue:
 // acc[i][t][j] = C[n = 16 (nt0+i) + 4q + j][m = m0 + 16 t + r]
@@ -202,9 +195,6 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
                     o[i] = pack_bf16x2(silu_mul_rounded_quick(__uint_as_float(s0[1]), __uint_as_float(s0[0])),
                                        silu_mul_rounded_quick(__uint_as_float(s1[1]), __uint_as_float(s1[0])));
             }
-#ifdef MV_EXP_EPI_NO_WRITE
-            asm volatile("" : : "v"(o[0]), "v"(o[1]), "v"(o[2]), "v"(o[3]));   // timing experiment only
-#else
             if (whole) {
                 const auto a02 = __builtin_amdgcn_permlane32_swap(o[0], o[2], false, false);
                 const auto a13 = __builtin_amdgcn_permlane32_swap(o[1], o[3], false, false);
@@ -218,7 +208,6 @@ __device__ __forceinline__ void store_wave_tile(const PGemmArgs& a, const f32x4_
                     if (m < a.m && nt0 + i < a.nt)
                         *reinterpret_cast<uint32_t*>(row + i * 8 + (q & 1) * 4 + (q >> 1) * 2) = o[i];
             }
-#endif
         }
         return;
     }
@@ -351,9 +340,6 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
         }
     };
     auto x_frag = [&](int buf, int t, int kk) {
-#ifdef MV_EXP_NO_XREAD
-        return __builtin_bit_cast(bf16x8_t, make_uint4(lane, t, kk, buf));  // timing experiment only
-#endif
         return __builtin_bit_cast(
             bf16x8_t, *reinterpret_cast<const uint4*>(&xs[buf][(t * 2 + kk) * 1024 + lane * 16]));
     };
@@ -371,9 +357,6 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
         const int ktc = min(kt, a.ktps - 1);
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
-#ifdef MV_EXP_NO_WLOAD
-            if (kt > 2) continue;  // timing experiment only: weights never refreshed
-#endif
             wr[i] = ld16(wp[i] + (int64_t)ktc * 64);
         }
     };
@@ -447,9 +430,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
         // buffers: at most two stages are left over, and both have arrived before the first of them.)
         wait_vmcnt<(kLeft && BUFS > 3) ? (BUFS - 3) * XP : NT + (BUFS - 3) * (2 * NT + XP)>();
         MV_STAMP(2);
-#ifndef MV_EXP_NO_BARRIER
         __syncthreads();
-#endif
         MV_STAMP(3);
     };
     // kPeriod stages per pass and no branch inside the pass (a branch between stages makes the
@@ -661,14 +642,6 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
     const int xoff1 = (wm * 8) * 2048 + r * 128 + (((4 + q) ^ ((r >> 1) & 7)) * 16);   // kk = 1
     const int woff = wcol * 1024 + lane * 16;
     auto read_frags = [&](bf16x8_t(&wf)[NT], bf16x8_t(&xf)[kPMT], int kt) {
-#if defined(MV_EXP_MFMA_ONLY) || defined(MV_EXP_NO_FRAG_READ)
-        // timing experiment only: operands made up in registers, nothing read
-#pragma unroll
-        for (int i = 0; i < NT; ++i) wf[i] = __builtin_bit_cast(bf16x8_t, make_uint4(lane * 77 + kt, i * 0x3f803f80u, kt * 0x01010101u, 0x3c003c00u));
-#pragma unroll
-        for (int t = 0; t < kPMT; ++t) xf[t] = __builtin_bit_cast(bf16x8_t, make_uint4(lane * 31 + t, kt * 0x00810081u, 0x3f003f00u + t, 0x3d803d80u));
-        return;
-#endif
         const int st = kt >> 1;
         const unsigned char* wp = wring + (kt & 3) * kWWSlot + woff;
         const unsigned char* xp = xring + (st % 3) * kWXSlot + ((kt & 1) ? xoff1 : xoff0);
@@ -731,11 +704,8 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
 #pragma unroll
         for (int t = 0; t < kPMT; ++t) {
             __builtin_amdgcn_sched_barrier(0);
-#ifndef MV_EXP_NO_COPY
             if (t < 6) copy_piece(g, kt, odd, t);
-#endif
             __builtin_amdgcn_sched_barrier(0);
-#ifndef MV_EXP_NO_FRAG_READ
             if (t < 2) {
                 wnx[2 * t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wp + (2 * t) * 1024));
                 if (2 * t + 1 < NT)
@@ -744,7 +714,6 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
                 xnx[2 * t - 4] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(xp + (2 * t - 4) * 2048));
                 xnx[2 * t - 3] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(xp + (2 * t - 3) * 2048));
             }
-#endif
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < NT; ++i)
@@ -754,9 +723,7 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
         // this wave's pieces of k-tile kt + 2 have landed (8 younger copies may be outstanding), and
         // its fragment reads of kt + 1 are complete before that slot can be written again
         asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-#ifndef MV_EXP_NO_BARRIER
         __syncthreads();
-#endif
     };
     [[maybe_unused]] int tile_no = 0;
     for (int g0 = 0;;) {
@@ -767,13 +734,6 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
             ktile(wB, xB, wA, xA, g0 + kt + 1, kt + 1, true);
         }
         MV_WSTAMP(g0 + nkt);
-#ifdef MV_EXP_NO_STORE
-        // timing experiment only: the accumulators are consumed, nothing is written
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int t = 0; t < kPMT; ++t) asm volatile("" : : "v"(acc[i][t]));
-#else
         if (cur.parts > 1 && cur.part + 1 < cur.parts) {
             // a lower part of a cut tile: the accumulators as they lie in the registers (1 KiB per
             // register and wave), then one count per workgroup once every wave's stores are visible
@@ -823,7 +783,6 @@ __device__ __forceinline__ void wide_tile(const PGemmArgs& a, unsigned char* lds
             if (cur.ntb + wcol < a.nt)
                 store_wave_tile<NT, kPMT, ACT>(a, acc, cur.ntb + wcol, cur.m0 + wm * 128, cur.ks, r, q, lower, nlower);
         }
-#endif
         MV_WSTAMP(g0 + nkt + 1);
         if (!more) break;
 #pragma unroll

@@ -2,11 +2,9 @@
    python tools/stamp_gemm_prefill.py [variant]     (default variant "stamp")
 Build the variants first, e.g.
    python -c "import sys; sys.path.insert(0, 'micro-vllm_amd'); import build; \
-              build.build_variant('stamp', ['MV_GEMM_STAMP'], only=('gemm_prefill.hip',)); \
-              build.build_variant('stamp_now', ['MV_GEMM_STAMP', 'MV_EXP_NO_WLOAD'], only=('gemm_prefill.hip',)); \
-              build.build_variant('stamp_nox', ['MV_GEMM_STAMP', 'MV_EXP_NO_XREAD'], only=('gemm_prefill.hip',))"
+              build.build_variant('stamp', ['MV_GEMM_STAMP'], only=('gemm_prefill.hip',))"
 Phases per stage: 0->1 fragment reads + MFMA issue (incl. waits for weights), 1->2 wait for the x
-tile two stages ahead, 2->3 barrier.  Measured with both operand paths removed a stage takes 1430
+tile two stages ahead, 2->3 barrier.  In copies of the kernel, with both operand paths removed a stage takes 1430
 ticks, with either one present about 2800-2900, with both 3800: the kernel is bound by operand
 delivery, not by the matrix pipe."""
 import ctypes, os, sys
