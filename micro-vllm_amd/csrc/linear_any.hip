@@ -7,10 +7,10 @@
 //   bf16 operands: 64 x 64 output tile per workgroup of 4 waves, k in steps of 32 through LDS,
 //                  v_mfma_f32_16x16x32_bf16, edges zero-filled in LDS; the sum over k in ascending order of those
 //                  steps;
-//   fp32 operands: tiles of three sizes on the fp32 matrix instruction (no reduced-precision mode), or, for a few
-//                  rows, the weights streamed past them.  In all of these a sum over k is made of four quarters of k
-//                  (in whole steps of 32) that are added up in ascending order, a quarter of the same sequence of
-//                  matrix instructions.
+//   fp32 operands: products of 32-bit factors, every factor in three bf16 parts (no reduced-precision mode), on tiles of
+//                  several sizes or, for a few rows, the weights streamed past them.  In all of these a sum over k is
+//                  made of four quarters of k (in whole steps of 32) that are added up in ascending order, a quarter
+//                  of the same sequence of matrix instructions.
 // So in one product (mv_linear_any) a row's result does not depend on which other rows share the launch.  A launch of
 // several products (heads, expert segments) has another form for up to kFewRows rows, linear_fewrows_kernel, whose lanes
 // add every 64th piece of k and then each other: there a row's last bits differ from those of a larger launch.
@@ -195,43 +195,97 @@ __global__ __launch_bounds__(256) void linear_any_bf16_big_kernel(
     }
 }
 
-// fp32 operands on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: products and sums in 32 bits).  That
-// instruction needs 32 cycles for 2048 FLOP, so a tile is bound by it and not by LDS or loads as long as loads are in
-// flight: PF k-steps of 32 in registers in front of a double buffer in LDS, one barrier a step.  A lane reads four
-// neighbouring k of its row at once and the four instructions behind take one of them each: both operands agree on which
-// k that is, so the sum is over the same sixteen.  LDS rows of 36 floats put the 16 rows of such a read on 16 different
-// groups of four banks.
-// WM x WN accumulator tiles per wave, four waves as 2 x 2: (32 WM) x (32 WN) outputs.  The quarters of k are taken one
-// after the other by the same waves (KG = 1; a second set of accumulators holds the sum so far), or side by side by four
-// groups of four waves (KG = 4): a launch of few tiles is a chain of load latencies (about 0.8 us a step behind HBM),
-// which four groups with four steps ahead each cut by more than four.  The 64 x 64 tile takes four groups where it has a
-// compute unit to itself: one wave a SIMD leaves its matrix unit idle behind every read (567 rows 1024 x 5120 106.6 -> 94.9 us,
-// 1000 rows 125 -> 96, 1024 x 1024 29.9 -> 25.1; the same sums bit for bit).  The widest tile
-// has 64 accumulators and 32 MFMA times a step to hide a load behind: one step ahead, so that two of its workgroups
-// share a unit (two steps ahead: one workgroup, 97 instead of 128 TFLOP/s).
-// Measured against the 64 x 64 tile of vector fused multiply-adds with k in steps of 16 that was here (outputs x k, us):
-// 567 rows 1024 x 5120 570 -> 105, 9472 x 1024 346 -> 116, 16384 x 4096 2551 -> 642 (119 TFLOP/s); 2048 rows 16384 x
-// 4096 2156 (128 TFLOP/s); 64 rows 1024 x 5120 581 -> 35, 9472 x 1024 126 -> 31.  The error against 64 bits is half of
-// what it was (1024 x 5120: 1.3e-6 -> 6.4e-7): the sums are of quarters.
-constexpr int kLfBK = 32, kLfPad = 36;
+// fp32 operands on the bf16 matrix instruction, every factor in three bf16 parts: x = hi + mid + lo exactly (8 bits each of the
+// 24), of the nine products of parts the six that reach 2^-24 of x w, each of them exact in the instruction and added up in
+// fp32.  v_mfma_f32_16x16x4_f32 does 256 FLOP a cycle and unit, v_mfma_f32_16x16x32_bf16 4096.  A weight whose low 16 bits are
+// zero is its own hi: sixteen rows of weights that are so over a step of k (those of a bf16 checkpoint in a run of 32 bits)
+// take three products, and the sum is the same bit for bit, for what is left out are zeros.
+// Sums, in every form here: a step is 32 neighbouring k, its products go from the smallest parts to hi hi; steps in ascending
+// order make a quarter of k, the quarters are added in ascending order.
+// What the parts cannot hold is done by the fp32 instruction (lf_by_f32: the same quarters): a sum that is not finite - an
+// infinite or NaN factor, or one that the rounding of hi makes infinite - and a sum below kLfTiny, where parts fall below the
+// smallest bf16 numbers.  Which form an output takes depends on its own row and column alone.
+constexpr int kLfBK = 32;
+constexpr float kLfTiny = 0x1p-60f;
+
+__device__ __forceinline__ bool lf_outside(float v) {   // (an exact zero is what rows of zeros give)
+    const float a = fabsf(v);
+    return !(a >= kLfTiny && a < INFINITY) && v != 0.f;
+}
+
+// four values
+__device__ __forceinline__ void lf_split4(const f32x4_t& v, uint2& hi, uint2& mid, uint2& lo) {
+    hi = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    float a = v[0] - bf16_lo(hi.x), b = v[1] - bf16_hi(hi.x), c = v[2] - bf16_lo(hi.y), d = v[3] - bf16_hi(hi.y);
+    mid = make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
+    a -= bf16_lo(mid.x);
+    b -= bf16_hi(mid.x);
+    c -= bf16_lo(mid.y);
+    d -= bf16_hi(mid.y);
+    lo = make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
+}
+struct LfParts {
+    uint4 hi, mid, lo;   // eight values, two in each word
+};
+__device__ __forceinline__ LfParts lf_split(const f32x4_t& v0, const f32x4_t& v1) {
+    uint2 h[2], m[2], l[2];
+    lf_split4(v0, h[0], m[0], l[0]);
+    lf_split4(v1, h[1], m[1], l[1]);
+    return {make_uint4(h[0].x, h[0].y, h[1].x, h[1].y), make_uint4(m[0].x, m[0].y, m[1].x, m[1].y),
+            make_uint4(l[0].x, l[0].y, l[1].x, l[1].y)};
+}
+// whether any of eight values has bits beside those of bf16, and the values' upper halves
+__device__ __forceinline__ uint32_t lf_low_bits(const f32x4_t& v0, const f32x4_t& v1) {
+    uint32_t any = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) any |= __float_as_uint(v0[i]) | __float_as_uint(v1[i]);
+    return any & 0xffffu;
+}
+__device__ __forceinline__ uint4 lf_upper(const f32x4_t& v0, const f32x4_t& v1) {
+    auto two = [](float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u); };
+    return make_uint4(two(v0[0], v0[1]), two(v0[2], v0[3]), two(v1[0], v1[1]), two(v1[2], v1[3]));
+}
+__device__ __forceinline__ f32x4_t lf_mfma(uint4 w, uint4 x, f32x4_t acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(la_bf16x8_t, w), __builtin_bit_cast(la_bf16x8_t, x), acc, 0, 0, 0);
+}
 
 // VEC: rows at multiples of 16 bytes and K % 4 == 0.  Columns past the end of k are zeros and nothing is read there; rows
 // past the last one were clamped by the caller (their outputs are not stored).
 template <bool VEC>
-__device__ __forceinline__ f32x4_t lf_load4(const float* p, int col, int k) {
+__device__ __forceinline__ f32x4_t lf_load4_any(const float* p, int col, int k) {   // past the end: anything (lf_mask4)
     f32x4_t v;
-    if (VEC) {
-        v = *reinterpret_cast<const f32x4_t*>(p + (col < k ? col : 0));
+    if (VEC) return *reinterpret_cast<const f32x4_t*>(p + (col < k ? col : 0));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = col < k ? v[i] : 0.f;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float e = p[col + i < k ? col + i : 0];
-            v[i] = col + i < k ? e : 0.f;
-        }
-    }
+    for (int i = 0; i < 4; ++i) v[i] = p[col + i < k ? col + i : 0];
     return v;
+}
+__device__ __forceinline__ void lf_mask4(f32x4_t& v, int col, int k) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = col + i < k ? v[i] : 0.f;
+}
+template <bool VEC>
+__device__ __forceinline__ f32x4_t lf_load4(const float* p, int col, int k) {
+    f32x4_t v = lf_load4_any<VEC>(p, col, k);
+    lf_mask4(v, col, k);
+    return v;
+}
+
+// Sixteen outputs by sixteen on the fp32 instruction, straight from memory: lane (r, q)'s row of x and of W, the shares
+// `share` .. `share + count` of `per` steps, added up in ascending order.
+template <bool VEC>
+__device__ __attribute__((noinline)) f32x4_t lf_by_f32(const float* x, const float* w, int q, int K, int per, int share, int count) {
+    f32x4_t sum = {0, 0, 0, 0};
+    for (int s = 0; s < count; ++s) {
+        f32x4_t acc = {0, 0, 0, 0};
+        for (int k0 = (share + s) * per * kLfBK, n = 0; n < 2 * per; ++n, k0 += 16) {
+            const f32x4_t xf = lf_load4<VEC>(x, k0 + q * 4, K), wf = lf_load4<VEC>(w, k0 + q * 4, K);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[e], xf[e], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] = s == 0 ? acc[j] : sum[j] + acc[j];
+    }
+    return sum;
 }
 
 // Tiles of one column of outputs (one piece of W) go to one XCD, whose L2 then holds that piece: workgroups are dealt
@@ -242,21 +296,39 @@ __device__ __forceinline__ bool lf_place(int id, int cols, int rows, int& col, i
     return col < cols;
 }
 
-template <int WM, int WN, int KG, int PF, bool VEC>
+// TM x TN accumulator tiles of 16 x 16 per wave, four waves as 2 x 2: (32 TM) x (32 TN) outputs.  KG groups of four waves take
+// the quarters of k side by side, each its 4 / KG one after the other (a second set of accumulators holds the sum so far).  A
+// step of 32 k: a wave splits sixteen rows at a time on their way into LDS, where a plane of parts of sixteen rows is 1 KB in the
+// instruction's own lane order; the rows of lane group q are exchanged by xor with 2 q, so that neither the writes (four lanes a
+// row, eight lanes a cycle) nor the reads (a lane a row) meet on a bank: counted 0 conflicts, 1.5 cycles of three without.  PF
+// steps are requested ahead.  DB: two buffers and one barrier a step, else one and two.
+// What bounds it: no one unit - at 2048 rows 16384 x 4096 the matrix units are busy 42 % of the time, the vector units 30, LDS 28 - but
+// the chain load, split, LDS, barrier, products of the two or three workgroups of a unit; splitting the next step in front of this
+// one's products, into a second buffer, gained nothing.
+// Against the fp32 matrix instruction (256 FLOP a cycle and unit) that was here, us, weights of bf16 values | of 32 bits:
+// 567 rows 9472 x 1024 122 -> 54 | 84, 1024 x 5120 91 -> 54 | 76, 1024 x 1024 22.5 -> 14.2 | 19.4; 2048 rows 16384 x 4096 2160 -> 869 (316
+// TFLOP/s of fp32 products) | 1402; 64 rows 1024 x 5120 33 -> 27 | 32, 9472 x 1024 24 -> 17 | 21; 1024 rows 4096 x 128 17 -> 14 | 16.5.
+// Error against 64 bits (2-norm): 1024 x 5120 6.4e-7 -> 3.9e-7 | 5.6e-7, 9472 x 1024 2.9e-7 -> 1.7e-7 | 2.3e-7.
+template <int TM, int TN, int KG, int PF, bool DB, bool VEC>
 __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kernel(
     const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
     float* __restrict__ y, int64_t ldy, int M, int N, int K, int64_t zx, int64_t zw, int64_t zy, RowSegments sg) {
-    constexpr int BM = 32 * WM, BN = 32 * WN;
+    constexpr int BM = 32 * TM, BN = 32 * TN, RB = 2 * (TM + TN), U = RB / 4;   // row blocks; of them per wave
+    constexpr int kPlane = RB * 64;                                            // 16-byte pieces of a plane
+    constexpr bool kFold = KG < 4;
+    static_assert(RB % 4 == 0 && (TM % 2 == 0 || (TM == 1 && TN == 1)), "a wave's row block is of x or of W");
     x += blockIdx.z * zx;
     w += blockIdx.z * zw;
     y += blockIdx.z * zy;
     extern __shared__ __attribute__((aligned(16))) float lf_lds[];
+    __shared__ int more_parts[DB ? 2 : 1][KG][2 * TN];   // the step in which these rows of W last had low bits
     int nb, mb;
     if (!lf_place(blockIdx.x, (N + BN - 1) / BN, (M + BM - 1) / BM, nb, mb)) return;
     const int m0 = mb * BM, n0 = nb * BN;
-    const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255;
-    const int wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4, wm = wave >> 1, wn = wave & 1;
-    const int lrow = tid >> 3, lcol = (tid & 7) * 4;
+    const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = threadIdx.x & 255;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int lr = lane >> 2, lq = lane & 3;   // staging: row of the block, piece of the row
     int64_t y0 = 0;
     if (sg.seg) {
         y0 = sg.seg[blockIdx.z];
@@ -264,126 +336,209 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
         if (m0 >= M) return;
         y += y0 * ldy;
     }
-    const float* xp[WM];
-    const float* wp[WN];
+    auto x_row = [&](int i) { return x + (i < M ? (sg.src ? sg.src[y0 + i] / sg.src_div : y0 + i) : 0) * ldx; };
+    auto w_row = [&](int i) { return w + (int64_t)min(i, N - 1) * ldw; };
+    auto of_x = [&](int u) { return TM > 1 ? u < TM / 2 : wave < 2; };
+    const float* p[U];
 #pragma unroll
-    for (int u = 0; u < WM; ++u) {
-        const int mr = m0 + lrow + 32 * u;
-        xp[u] = x + (mr < M ? (sg.src ? sg.src[y0 + mr] / sg.src_div : y0 + mr) : 0) * ldx;
+    for (int u = 0; u < U; ++u) {
+        const int row = (u * 4 + wave) * 16 + lr;
+        p[u] = of_x(u) ? x_row(m0 + row) : w_row(n0 + row - BM);
     }
-#pragma unroll
-    for (int u = 0; u < WN; ++u) wp[u] = w + (int64_t)min(n0 + lrow + 32 * u, N - 1) * ldw;
-    float* buf = lf_lds + grp * 2 * (BM + BN) * kLfPad;
-    f32x4_t acc[WN][WM], sum[WN][WM];
+    uint4* buf = reinterpret_cast<uint4*>(lf_lds) + grp * (DB ? 2 : 1) * 3 * kPlane;
+    if (threadIdx.x < (DB ? 2 : 1) * KG * 2 * TN) (&more_parts[0][0][0])[threadIdx.x] = -1;
+    f32x4_t acc[TN][TM], sum[TN][TM];
     const int per = ((K + kLfBK - 1) / kLfBK + 3) / 4;   // k-steps of a quarter
     auto clear = [&] {
 #pragma unroll
-        for (int a = 0; a < WN; ++a)
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int b = 0; b < WM; ++b) acc[a][b] = f32x4_t{0, 0, 0, 0};
+            for (int b = 0; b < TM; ++b) acc[a][b] = f32x4_t{0, 0, 0, 0};
     };
     int fold = per;
     auto add_quarter = [&] {
 #pragma unroll
-        for (int a = 0; a < WN; ++a)
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int b = 0; b < WM; ++b)
+            for (int b = 0; b < TM; ++b)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) sum[a][b][j] = fold == per ? acc[a][b][j] : sum[a][b][j] + acc[a][b][j];
         fold += per;
     };
     clear();
-    f32x4_t xr[PF][WM], wr[PF][WN];
-    auto request = [&](int set, int step) {
-        const int col = ((KG > 1 ? grp * per : 0) + step) * kLfBK + lcol;
+    f32x4_t v[PF][U][2];
+    const int first = grp * per * (4 / KG);   // this group's first step
 #pragma unroll
-        for (int u = 0; u < WM; ++u) xr[set][u] = lf_load4<VEC>(xp[u], col, K);
+    for (int u = 0; u < U; ++u) p[u] += first * kLfBK + lq * 4;
+    auto request = [&](int set, int step) {   // steps are asked for in ascending order
+        const int k0 = (first + step) * kLfBK;
+        if (VEC && k0 + kLfBK <= K) {   // uniform
 #pragma unroll
-        for (int u = 0; u < WN; ++u) wr[set][u] = lf_load4<VEC>(wp[u], col, K);
+            for (int u = 0; u < U; ++u) {
+                v[set][u][0] = *reinterpret_cast<const f32x4_t*>(p[u]);
+                v[set][u][1] = *reinterpret_cast<const f32x4_t*>(p[u] + 16);
+            }
+        } else {   // the last step of k, or one past it
+            const int col = k0 + lq * 4;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                v[set][u][0] = lf_load4_any<VEC>(p[u] - col, col, K);
+                v[set][u][1] = lf_load4_any<VEC>(p[u] - col, col + 16, K);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) p[u] += kLfBK;
     };
-    auto multiply = [&](int set, int half, int step) {
-        float* xs = buf + half * (BM + BN) * kLfPad;
-        float* ws = xs + BM * kLfPad;
+    const int put = lq * 16 + (lr ^ (lq * 2)), get = q * 16 + (r ^ (q * 2));
+    auto stage = [&](int set, int half, int step) {
+        uint4* at = buf + (DB ? half * 3 * kPlane : 0);
+        if ((first + step + 1) * kLfBK > K) {   // uniform, as above
+            const int col = (first + step) * kLfBK + lq * 4;
 #pragma unroll
-        for (int u = 0; u < WM; ++u) *reinterpret_cast<f32x4_t*>(xs + (lrow + 32 * u) * kLfPad + lcol) = xr[set][u];
+            for (int u = 0; u < U; ++u) {
+                lf_mask4(v[set][u][0], col, K);
+                lf_mask4(v[set][u][1], col + 16, K);
+            }
+        }
 #pragma unroll
-        for (int u = 0; u < WN; ++u) *reinterpret_cast<f32x4_t*>(ws + (lrow + 32 * u) * kLfPad + lcol) = wr[set][u];
+        for (int u = 0; u < U; ++u) {
+            uint4* to = at + (u * 4 + wave) * 64 + put;
+            if (of_x(u) || __any(lf_low_bits(v[set][u][0], v[set][u][1]) != 0)) {   // uniform
+                const LfParts s = lf_split(v[set][u][0], v[set][u][1]);
+                to[0] = s.hi;
+                to[kPlane] = s.mid;
+                to[2 * kPlane] = s.lo;
+                if (!of_x(u) && lane == 0) more_parts[DB ? half : 0][grp][u * 4 + wave - 2 * TM] = step;
+            } else {
+                to[0] = lf_upper(v[set][u][0], v[set][u][1]);
+            }
+        }
         request(set, step + PF);
-        __syncthreads();   // the other half was read a step ago, before this barrier by every wave
-        if (KG == 1 && step == fold) {
+    };
+    uint4 wf[TN], xf[TM][3];
+    int tag[TN];
+    auto fetch = [&](int half) {
+        const uint4* at = buf + (DB ? half * 3 * kPlane : 0);
+#pragma unroll
+        for (int a = 0; a < TN; ++a) {
+            wf[a] = at[(2 * TM + wn * TN + a) * 64 + get];
+            tag[a] = more_parts[DB ? half : 0][grp][wn * TN + a];
+        }
+#pragma unroll
+        for (int b = 0; b < TM; ++b)
+#pragma unroll
+            for (int part = 0; part < 3; ++part) xf[b][part] = at[part * kPlane + (wm * TM + b) * 64 + get];
+    };
+    auto multiply = [&](int half, int step) {
+        if (kFold && step == fold) {
             add_quarter();
             clear();
         }
+        bool more[TN], any = false;
 #pragma unroll
-        for (int ks = 0; ks < kLfBK; ks += 16) {
-            f32x4_t wf[WN], xf[WM];
-#pragma unroll
-            for (int t = 0; t < WN; ++t)
-                wf[t] = *reinterpret_cast<const f32x4_t*>(ws + (wn * 16 * WN + t * 16 + r) * kLfPad + ks + q * 4);
-#pragma unroll
-            for (int t = 0; t < WM; ++t)
-                xf[t] = *reinterpret_cast<const f32x4_t*>(xs + (wm * 16 * WM + t * 16 + r) * kLfPad + ks + q * 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int a = 0; a < WN; ++a)
-#pragma unroll
-                    for (int b = 0; b < WM; ++b)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[a][e], xf[b][e], acc[a][b], 0, 0, 0);
+        for (int a = 0; a < TN; ++a) {
+            more[a] = __builtin_amdgcn_readfirstlane(tag[a]) == step;
+            any = any || more[a];
         }
+        if (any) {   // (rows without low bits beside rows with: their parts here are what an earlier step left)
+            const uint4* ws = buf + (DB ? half * 3 * kPlane : 0) + (2 * TM + wn * TN) * 64 + get;
+#pragma unroll
+            for (int a = 0; a < TN; ++a) {
+                if (!more[a]) continue;
+                const uint4 mid = ws[kPlane + a * 64], lo = ws[2 * kPlane + a * 64];
+#pragma unroll
+                for (int b = 0; b < TM; ++b) acc[a][b] = lf_mfma(lo, xf[b][0], acc[a][b]);
+#pragma unroll
+                for (int b = 0; b < TM; ++b) acc[a][b] = lf_mfma(mid, xf[b][1], acc[a][b]);
+#pragma unroll
+                for (int b = 0; b < TM; ++b) acc[a][b] = lf_mfma(mid, xf[b][0], acc[a][b]);
+            }
+        }
+#pragma unroll
+        for (int part = 2; part >= 0; --part)
+#pragma unroll
+            for (int b = 0; b < TM; ++b)
+#pragma unroll
+                for (int a = 0; a < TN; ++a) acc[a][b] = lf_mfma(wf[a], xf[b][part], acc[a][b]);
+    };
+    auto turn = [&](int set, int half, int step) {
+        stage(set, half, step);
+        __syncthreads();   // (DB: the other buffer was read a step ago, before this barrier by every wave)
+        fetch(half);
+        multiply(half, step);
+        if (!DB) __syncthreads();
     };
 #pragma unroll
     for (int i = 0; i < PF; ++i) request(i, i);
-    constexpr int TURN = PF > 2 ? PF : 2;   // steps after which register sets and halves are where they were
+    __syncthreads();   // (more_parts)
+    constexpr int TURN = PF > (DB ? 2 : 1) ? PF : (DB ? 2 : 1);   // steps after which register sets and buffers are where they were
+    static_assert(!DB || TURN % 2 == 0, "a turn ends on the buffer it began with");
     // Side by side the groups share the barriers, and a step past the end of k multiplies zeros.  One after the other the
-    // quarters end with k, at a whole turn: left-over steps behind the loop cost it a seventh of its pace.
-    const int steps = KG > 1 ? per : ((K + kLfBK - 1) / kLfBK + TURN - 1) / TURN * TURN;
+    // quarters end with k, at a whole turn.
+    const int steps = KG > 1 ? per * (4 / KG) : ((K + kLfBK - 1) / kLfBK + TURN - 1) / TURN * TURN;
     int st = 0;
     for (; st + TURN <= steps; st += TURN)
 #pragma unroll
-        for (int i = 0; i < TURN; ++i) multiply(i % PF, i & 1, st + i);
+        for (int i = 0; i < TURN; ++i) turn(i % PF, i & 1, st + i);
 #pragma unroll
     for (int i = 0; i < TURN - 1; ++i)
-        if (st + i < steps) multiply(i % PF, i & 1, st + i);
-    if (KG == 1) {
+        if (st + i < steps) turn(i % PF, i & 1, st + i);
+    if (kFold) {
         add_quarter();
 #pragma unroll
-        for (int a = 0; a < WN; ++a)
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int b = 0; b < WM; ++b) acc[a][b] = sum[a][b];
+            for (int b = 0; b < TM; ++b) acc[a][b] = sum[a][b];
     }
     if (KG > 1) {   // group 0 adds up the groups
         __syncthreads();
-        constexpr int kAcc = WN * WM * 4;
+        constexpr int kAcc = TN * TM * 4;
         float* part = lf_lds + ((grp - 1) * 256 + tid) * (kAcc + 1);
         if (grp > 0) {
 #pragma unroll
-            for (int a = 0; a < WN; ++a)
+            for (int a = 0; a < TN; ++a)
 #pragma unroll
-                for (int b = 0; b < WM; ++b)
+                for (int b = 0; b < TM; ++b)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) part[(a * WM + b) * 4 + j] = acc[a][b][j];
+                    for (int j = 0; j < 4; ++j) part[(a * TM + b) * 4 + j] = acc[a][b][j];
         }
         __syncthreads();
         if (grp > 0) return;
         for (int g = 0; g < KG - 1; ++g) {
             const float* o = lf_lds + (g * 256 + tid) * (kAcc + 1);
 #pragma unroll
-            for (int a = 0; a < WN; ++a)
+            for (int a = 0; a < TN; ++a)
 #pragma unroll
-                for (int b = 0; b < WM; ++b)
+                for (int b = 0; b < TM; ++b)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[a][b][j] += o[(a * WM + b) * 4 + j];
+                    for (int j = 0; j < 4; ++j) acc[a][b][j] += o[(a * TM + b) * 4 + j];
         }
     }
-    // acc[a][b][j] = C[n = n0 + 16 (WN wn + a) + 4 q + j][m = m0 + 16 (WM wm + b) + r]
+    // acc[a][b][j] = C[n = n0 + 16 (TN wn + a) + 4 q + j][m = m0 + 16 (TM wm + b) + r]
+    bool outside = false;
 #pragma unroll
-    for (int b = 0; b < WM; ++b) {
-        const int m = m0 + (wm * WM + b) * 16 + r;
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) outside = outside || lf_outside(acc[a][b][j]);
+    if (__any(outside)) {
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int b = 0; b < TM; ++b) {
+                const f32x4_t o = lf_by_f32<VEC>(x_row(m0 + (wm * TM + b) * 16 + r), w_row(n0 + (wn * TN + a) * 16 + r), q, K, per, 0, 4);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[a][b][j] = lf_outside(acc[a][b][j]) ? o[j] : acc[a][b][j];
+            }
+    }
+#pragma unroll
+    for (int b = 0; b < TM; ++b) {
+        const int m = m0 + (wm * TM + b) * 16 + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int a = 0; a < WN; ++a) {
-            const int n = n0 + (wn * WN + a) * 16 + q * 4;
+        for (int a = 0; a < TN; ++a) {
+            const int n = n0 + (wn * TN + a) * 16 + q * 4;
             float* dst = y + (int64_t)m * ldy + n;
             if (n + 3 < N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
                 *reinterpret_cast<float4*>(dst) = make_float4(acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]);
@@ -404,16 +559,21 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 // the wave's own part of LDS (rows 528 bytes apart: the sixteen rows of a read are on different banks; no barrier, a wave's LDS
 // operations are in order).  Two such pieces are in flight, 16 KB a wave.
 // Measured against operands read straight into that layout, 64 bytes of sixteen rows to a request (outputs x k, 3 rows, us):
-// 32000 x 1024 39.8 -> 24.2 (5.4 TB/s), 9472 x 1024 16.1 -> 10.4, 16384 x 4096 61.1 -> 44.1 (6.1 TB/s), 1024 x 5120 20.6 -> 12.3 (in four
-// slices 10.8 -> 7.3), 1024 x 1024 6.7 -> 5.0, 65536 x 64 70 -> 18; 16 rows 1024 x 5120 28.7 -> 16.3, 1280 x 1024 8.4 -> 6.3.
+// 32000 x 1024 39.8 -> 22 (5.9 TB/s), 9472 x 1024 16.1 -> 10, 16384 x 4096 61.1 -> 43.5 (6.2 TB/s), 1024 x 5120 20.6 -> 12.3 (in four
+// slices 10.8 -> 7.3), 65536 x 64 70 -> 18; 16 rows 1024 x 5120 28.7 -> 16.3, 1280 x 1024 8.4 -> 6.6.  The parts take the fp32
+// instruction's time where weights are bf16 values; where they are not, the second split costs 3 to 10 % (16384 x 4096 46).
 // From nine rows on the tiles are ahead where the output is wide and k is short (16 rows, 65536 x 64: 10.3 us against 25.6, 32000 x 256 15.4
 // against 15.6; 32000 x 512 28.6 against 18.9, 16384 x 4096 74 against 49), from 17 on everywhere.
 constexpr int kStreamRows = 8, kStreamRowsMore = 16, kStreamNarrow = 8192, kStreamLongK = 512, kStreamSlice = 8;
 constexpr int kStreamK = 128, kStreamPad = kStreamK + 4;   // k of a piece, floats of a row in LDS
+constexpr int kStreamParts = kStreamK * 2 + 16;            // bytes of a row's parts in LDS
+// A wave's rows of x lie in LDS split (a lane of the instruction whose column is a row past MR reads a row again, so split behind
+// LDS the work would be done 16 / MR times), up to eight of them; sixteen as they are.
+constexpr int stream_x_bytes(int mr) { return mr == 16 ? mr * kStreamPad * 4 : 3 * mr * kStreamParts; }
 
 // MR: rows of x that are read, 4, 8 or 16
 template <int MR>
-__global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __restrict__ x, int64_t ldx,
+__global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel(const float* __restrict__ x, int64_t ldx,
                                                                 const float* __restrict__ w, int64_t ldw,
                                                                 float* __restrict__ y, int64_t ldy, int M, int N, int K) {
     // blockIdx.y: a slice of k of its own, [slice][M][N] in y (ldy = N); the wave's share is a quarter of the slice
@@ -432,8 +592,10 @@ __global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __r
     for (int i = 0; i < 8; ++i) wp[i] = w + (int64_t)min(n0 + 2 * i + half, N - 1) * ldw;
 #pragma unroll
     for (int i = 0; i < MR / 2; ++i) xp[i] = x + (int64_t)min(2 * i + half, M - 1) * ldx;
-    float* ws = ls_lds + wave * (16 + MR) * kStreamPad;
+    constexpr bool kSplitFirst = MR < 16;
+    float* ws = ls_lds + wave * (16 * kStreamPad + stream_x_bytes(MR) / 4);
     float* xs = ws + 16 * kStreamPad;
+    unsigned char* xb = reinterpret_cast<unsigned char*>(xs);
     f32x4_t acc = {0, 0, 0, 0};
     f32x4_t wv[2][8], xv[2][MR / 2];
     auto request = [&](int set, int piece) {
@@ -447,25 +609,77 @@ __global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __r
         const bool in = first + piece * kStreamK + kl < end;
         const f32x4_t zero = {0, 0, 0, 0};
 #pragma unroll
-        for (int i = 0; i < MR / 2; ++i)
-            *reinterpret_cast<f32x4_t*>(xs + (2 * i + half) * kStreamPad + kl) = in ? xv[set][i] : zero;
+        for (int i = 0; i < MR / 2; ++i) {
+            const f32x4_t v = in ? xv[set][i] : zero;
+            if (kSplitFirst) {   // four values: a half of what lane (row, k / 4 % 4) of the instruction takes of their step
+                uint2 hi, mid, lo;
+                lf_split4(v, hi, mid, lo);
+                unsigned char* to = xb + (2 * i + half) * kStreamParts + (kl >> 5) * 64 + ((kl >> 2) & 3) * 16 + ((kl >> 4) & 1) * 8;
+                *reinterpret_cast<uint2*>(to) = hi;
+                *reinterpret_cast<uint2*>(to + MR * kStreamParts) = mid;
+                *reinterpret_cast<uint2*>(to + 2 * MR * kStreamParts) = lo;
+            } else {
+                *reinterpret_cast<f32x4_t*>(xs + (2 * i + half) * kStreamPad + kl) = v;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             *reinterpret_cast<f32x4_t*>(ws + (2 * i + half) * kStreamPad + kl) = in ? wv[set][i] : zero;
     };
-    auto multiply = [&](int piece) {
+    // `count` steps without a branch between them, so that one's split runs beside another's products (zeros past the share's end)
+    auto multiply_steps = [&](auto count, int at) {
+        constexpr int C = decltype(count)::value;
+        f32x4_t wv0[C], wv1[C];
+        uint32_t low = 0;
 #pragma unroll
-        for (int u = 0; u < kStreamK / kLfBK; ++u) {
-            if (piece * (kStreamK / kLfBK) + u >= per) break;   // uniform
+        for (int u = 0; u < C; ++u) {
+            const float* wr = ws + r * kStreamPad + (at + u) * kLfBK + q * 4;
+            wv0[u] = *reinterpret_cast<const f32x4_t*>(wr);
+            wv1[u] = *reinterpret_cast<const f32x4_t*>(wr + 16);
+            low |= lf_low_bits(wv0[u], wv1[u]);
+        }
+        auto parts_of_x = [&](int u) {
+            LfParts p;
+            if (kSplitFirst) {
+                const unsigned char* xr = xb + min(r, MR - 1) * kStreamParts + (at + u) * 64 + q * 16;
+                p.hi = *reinterpret_cast<const uint4*>(xr);
+                p.mid = *reinterpret_cast<const uint4*>(xr + MR * kStreamParts);
+                p.lo = *reinterpret_cast<const uint4*>(xr + 2 * MR * kStreamParts);
+            } else {
+                const float* xr = xs + r * kStreamPad + (at + u) * kLfBK + q * 4;
+                p = lf_split(*reinterpret_cast<const f32x4_t*>(xr), *reinterpret_cast<const f32x4_t*>(xr + 16));
+            }
+            return p;
+        };
+        LfParts first;
+        if (C == 1) first = parts_of_x(0);   // (its way out of LDS beside W's; of four steps they do not all fit)
+        if (__any(low != 0)) {   // uniform
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int at = u * kLfBK + h * 16 + q * 4;
-                const f32x4_t wf = *reinterpret_cast<const f32x4_t*>(ws + r * kStreamPad + at);
-                const f32x4_t xf = *reinterpret_cast<const f32x4_t*>(xs + min(r, MR - 1) * kStreamPad + at);
+            for (int u = 0; u < C; ++u) {
+                const LfParts xp = C == 1 ? first : parts_of_x(u), wp = lf_split(wv0[u], wv1[u]);
+                acc = lf_mfma(wp.lo, xp.hi, acc);
+                acc = lf_mfma(wp.mid, xp.mid, acc);
+                acc = lf_mfma(wp.mid, xp.hi, acc);
+                acc = lf_mfma(wp.hi, xp.lo, acc);
+                acc = lf_mfma(wp.hi, xp.mid, acc);
+                acc = lf_mfma(wp.hi, xp.hi, acc);
+            }
+        } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[e], xf[e], acc, 0, 0, 0);
+            for (int u = 0; u < C; ++u) {
+                const LfParts xp = C == 1 ? first : parts_of_x(u);
+                const uint4 hi = lf_upper(wv0[u], wv1[u]);
+                acc = lf_mfma(hi, xp.lo, acc);
+                acc = lf_mfma(hi, xp.mid, acc);
+                acc = lf_mfma(hi, xp.hi, acc);
             }
         }
+    };
+    constexpr int kSteps = MR == 4 ? 1 : 4;   // (more at a time take more registers than three of its workgroups on a unit have)
+    auto multiply = [&](int piece) {
+#pragma unroll
+        for (int at = 0; at < kStreamK / kLfBK; at += kSteps)
+            if (per - piece * (kStreamK / kLfBK) > at) multiply_steps(std::integral_constant<int, kSteps>(), at);   // uniform
     };
     auto settle = [] {   // between a wave's own writes and reads of LDS: an order for the compiler, no instruction
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -504,6 +718,12 @@ __global__ __launch_bounds__(256) void linear_stream_f32_kernel(const float* __r
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[j] += part[g][lane][j];
     // acc[j] = C[n = n0 + 4 q + j][m = r]
+    if (__any(lf_outside(acc[0]) || lf_outside(acc[1]) || lf_outside(acc[2]) || lf_outside(acc[3]))) {
+        const f32x4_t o = lf_by_f32<true>(x + (int64_t)min(r, M - 1) * ldx, w + (int64_t)min(n0 + r, N - 1) * ldw, q, K, per,
+                                          4 * blockIdx.y, 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = lf_outside(acc[j]) ? o[j] : acc[j];
+    }
     if (r >= M) return;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -582,20 +802,20 @@ __global__ __launch_bounds__(256) void linear_fewrows_kernel(const void* __restr
 
 }  // namespace mv
 
-template <int WM, int WN, int KG, int PF>
+template <int TM, int TN, int KG, int PF, bool DB>
 static int launch_linear_f32_tiles(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m,
                                    int n, int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s,
                                    mv::RowSegments sg) {
     using namespace mv;
-    constexpr int BM = 32 * WM, BN = 32 * WN;
+    constexpr int BM = 32 * TM, BN = 32 * TN;
     const int64_t cols = (n + BN - 1) / BN, rows = (m + BM - 1) / BM, groups = (cols + 7) / 8 * 8 * rows;
     if (groups > 0x7fffffff) return MV_ERR_UNSUPPORTED;
-    size_t lds = (size_t)KG * 2 * (BM + BN) * kLfPad * 4;
-    const size_t meet = (size_t)(KG - 1) * 256 * (WM * WN * 4 + 1) * 4;
+    size_t lds = (size_t)KG * (DB ? 2 : 1) * 3 * (BM + BN) * kLfBK * 2;
+    const size_t meet = (size_t)(KG - 1) * 256 * (TM * TN * 4 + 1) * 4;
     if (meet > lds) lds = meet;
     const bool vec = k % 4 == 0 && aligned16(x) && ldx % 4 == 0 && zx % 4 == 0 && aligned16(w) && ldw % 4 == 0 && zw % 4 == 0;
     static LdsOptIn done[2];
-    const auto kernel = vec ? linear_any_f32_kernel<WM, WN, KG, PF, true> : linear_any_f32_kernel<WM, WN, KG, PF, false>;
+    const auto kernel = vec ? linear_any_f32_kernel<TM, TN, KG, PF, DB, true> : linear_any_f32_kernel<TM, TN, KG, PF, DB, false>;
     if (const int rc = ensure_dynamic_lds((const void*)kernel, lds, done[vec])) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)groups, 1, batch), dim3(256 * KG), lds, s, x, ldx, w, ldw, y, ldy, m, n, k,
                        zx, zw, zy, sg);
@@ -612,7 +832,7 @@ static int launch_linear_stream(const float* x, int64_t ldx, const float* w, int
                                 int k, int slices, hipStream_t s) {
     using namespace mv;
     const int form = m <= 4 ? 0 : m <= 8 ? 1 : 2;
-    const size_t lds = (size_t)4 * (16 + (4 << form)) * kStreamPad * 4;
+    const size_t lds = (size_t)4 * (16 * kStreamPad * 4 + stream_x_bytes(4 << form));
     static LdsOptIn done[3];
     const auto kernel = form == 0 ? linear_stream_f32_kernel<4> : form == 1 ? linear_stream_f32_kernel<8> : linear_stream_f32_kernel<16>;
     if (const int rc = ensure_dynamic_lds((const void*)kernel, lds, done[form])) return rc;
@@ -620,14 +840,15 @@ static int launch_linear_stream(const float* x, int64_t ldx, const float* w, int
     return check_launch();
 }
 
-// Which fp32 form.  Few rows of one product stream the weights (see kStreamRows).  Otherwise the tile by the time the
-// launch takes in it: rounds of tiles over the compute units times what a tile costs a unit, in hundredths of a us as measured,
-// per k-step of 32 and for its start and end - 32 x 32 (four groups, a quarter of the steps each) 200 + 88 a step of a quarter, 64 x
-// 64 where several share a unit 200 + 59, by itself 500 + 56 in four groups and, at a k too short for those, 200 + 73 in one,
-// 128 x 128 1200 + 228 - so that a launch of few tiles takes
-// small ones and a large one the tile that reads its operands least often, at a short k later than at a long one: 1024 rows 4096 x 128
-// in 64 x 64 17.9 us, in 128 x 128 22.3; 1024 rows of 32 heads 128 x 64 55 and 123.  With segments `m` bounds a
-// segment, not the launch: the rows are taken to be spread evenly.
+// Which fp32 form.  Few rows of one product stream the weights (see kStreamRows).  Otherwise the tile by the time the launch
+// takes in it, in hundredths of a us as measured: with n = tiles over compute units, rounded up, a tile of a whole quarter a group
+// takes n times its own time (one workgroup fills a unit), and the others a step in which n workgroups of a unit take turns at
+// its matrix unit, vector unit and LDS.  A launch of few tiles takes small ones and many groups, a large one the tile that reads
+// and splits its operands least often.  us in (outputs of the tile, groups), weights of bf16 values:
+//   567 rows 9472 x 1024: 149 (32 x 32, 4), 82 (64 x 64, 4), 64 (64 x 64, 2), 61 (64 x 64), 49 (64 x 128), 62 (128 x 128)
+//   567 rows 1024 x 5120:  78, 54, 61, 89, 129, 203        33 rows 1024 x 5120: 26, 49, 58, 88, 127, 200
+//   2048 rows 16384 x 4096: 2724, 1632, 1273, 1208, 944, 873
+// With segments `m` bounds a segment, not the launch: the rows are taken to be spread evenly.
 static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
                              int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s, mv::RowSegments sg,
                              int total_rows) {
@@ -638,18 +859,23 @@ static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_
     }
     const int64_t per = sg.seg ? (total_rows + batch - 1) / batch : m;
     const int64_t cus = num_cus();
-    auto rounds = [&](int b) { return (((per + b - 1) / b) * ((n + b - 1) / b) * batch + cus - 1) / cus; };
-    const int64_t steps = (k + kLfBK - 1) / kLfBK;
-    const int64_t c32 = rounds(32) * (200 + 88 * ((steps + 3) / 4)), c128 = rounds(128) * (1200 + 228 * steps);
-    const bool groups = rounds(64) <= 1 && steps >= 18;
-    const int64_t c64 = groups ? 500 + 56 * steps : rounds(64) <= 1 ? 200 + 73 * steps : rounds(64) * (200 + 59 * steps);
-    if (c32 <= c64 && c32 <= c128)
-        return launch_linear_f32_tiles<1, 1, 4, 4>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
-    if (c64 <= c128 && groups)
-        return launch_linear_f32_tiles<2, 2, 4, 2>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
-    if (c64 <= c128)
-        return launch_linear_f32_tiles<2, 2, 1, 2>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
-    return launch_linear_f32_tiles<4, 4, 1, 1>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+    auto turns = [&](int bm, int bn) { return (((per + bm - 1) / bm) * ((n + bn - 1) / bn) * batch + cus - 1) / cus; };
+    const int64_t steps = (k + kLfBK - 1) / kLfBK, quarter = (steps + 3) / 4;
+    const int64_t n32 = turns(32, 32), n64 = turns(64, 64), n128 = turns(64, 128), n256 = turns(128, 128);
+    const int64_t cost[6] = {100 + n32 * (250 + 57 * quarter),       n64 * (400 + 128 * quarter),
+                             400 + 2 * quarter * (15 + 58 * n64),    300 + 100 * n64 + steps * (30 + 25 * n64),
+                             300 + 200 * n128 + steps * (30 + 43 * n128), 600 + 400 * n256 + steps * (40 + 82 * n256)};
+    int best = 0;
+    for (int i = 1; i < 6; ++i)
+        if (cost[i] < cost[best]) best = i;
+    switch (best) {
+        case 0: return launch_linear_f32_tiles<1, 1, 4, 2, true>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+        case 1: return launch_linear_f32_tiles<2, 2, 4, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+        case 2: return launch_linear_f32_tiles<2, 2, 2, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+        case 3: return launch_linear_f32_tiles<2, 2, 1, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+        case 4: return launch_linear_f32_tiles<2, 4, 1, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+        default: return launch_linear_f32_tiles<4, 4, 1, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
+    }
 }
 
 static int launch_linear_any(const void* x, int64_t ldx, const void* w, int64_t ldw, float* y, int64_t ldy, int m, int n,

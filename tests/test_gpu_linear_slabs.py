@@ -268,3 +268,43 @@ def test_short_k_of_one_and_two_rows(mv, n, k):
     for rows in (1, 2):
         for a, b in zip(forms(rows), want):
             assert torch.equal(a, b[:rows])
+
+
+# fp32 factors in three bf16 parts: what those cannot hold (infinities, NaN, values that round to an infinite bf16, sums in the
+# range of the smallest numbers) has the value of fp32 arithmetic, and only it: neighbours keep their bits.  One shape for each
+# form: streamed, six tiles, a k that ends inside a step
+@pytest.mark.parametrize("m,n,k", [(3, 1024, 1024), (16, 50, 516), (20, 1000, 1022), (33, 9472, 256), (200, 4000, 128),
+                                   (567, 1024, 640), (333, 9472, 68), (2048, 4096, 64)])
+def test_fp32_values_beyond_the_parts(mv, m, n, k):
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(DEV)
+    w = (torch.randn(n, k, generator=g) / k ** 0.5).bfloat16().float().to(DEV)
+    w[n // 2:] += 2.0 ** -12 * torch.randn(n - n // 2, k, generator=g).to(DEV)     # rows of bf16 values, and rows of more
+    plain = AnyLinear(w)(x)
+    err = (plain.double() - x.double() @ w.double().t()).abs()
+    assert bool((err <= k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())).all())
+    big, odd = torch.finfo(torch.float32).max, x.clone()
+    odd[0, 1], odd[1, 2], odd[2, :] = float("inf"), float("nan"), x[2] * 2.0 ** -116
+    wo = w.clone()
+    wo[3, 0], wo[5, :] = -float("inf"), 0.0
+    wo[7, :] = 0.0
+    wo[7, 4] = 1.0
+    if m > 3:
+        odd[3, :] = 0.0
+        odd[3, 4] = big          # its bf16 is infinite
+    got = AnyLinear(wo)(odd)
+    want = odd.double() @ wo.double().t()
+    assert torch.equal(got.isnan(), want.isnan())
+    inf = want.isinf()
+    assert torch.equal(got[inf].double(), want[inf])
+    fine = [i for i in range(m) if i > 3]
+    cols = [j for j in range(n) if j not in (3, 5, 7)]
+    if fine:
+        assert torch.equal(got[fine][:, cols], plain[fine][:, cols])
+    tiny = (got[2].double() - want[2]).abs() <= k * 2.0 ** -24 * (odd[2].double().abs() @ wo.double().abs().t()) + k * 2.0 ** -149
+    assert bool(tiny[torch.tensor([j for j in range(n) if j != 3])].all())
+    assert bool((got[:, 5][torch.isfinite(odd).all(1)] == 0).all())
+    if m > 3:
+        assert got[3, 7].item() == big
