@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include <atomic>
+#include <type_traits>
 
 namespace mv {
 
@@ -448,19 +449,35 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 }
 
 // ------------------------------------------------------------ M > 4: MFMA form
-// MB = number of 16-row blocks of x (M <= 16*MB); SG = strips a workgroup multiplies together.
+// HB = number of 8-row blocks of x (M <= 8*HB), MB of 16-row blocks; SG = strips a workgroup multiplies together.
 // A wave loads the x fragments of a k-tile once and uses them against the SG weight tiles of
 // that k-tile: x comes out of L2 for every workgroup, so without the sharing the x requests
 // (MB per weight tile) outnumber the weight requests and the L2 path, not HBM, sets the pace.
 //
-// KS = 0: the waves interleave over the unit's k-tiles.  KS = 4, 8, 16: k in KS whole slices, each added up by one wave
+// What a request of x costs is the compute unit's address path: neighbouring lanes in different lines are taken one after the
+// other.  Sixteen rows of 64 bytes with a row to each lane - the operand's own layout - are 37 bytes a ns and unit, two lanes to
+// a line 68, a weight tile's 1 KiB in one piece 130.  So a request is eight rows of two k-tiles, lane (r, q) taking 16 bytes q of
+// row r / 2 and k-tile r % 2 (the odd 8-row block: k-tile 1 - r % 2), and the operands are made of two of them: the first k-tile's
+// is the first block's even lanes and the second's odd ones, the second k-tile's the other lanes, exchanged with their neighbours
+// (three vector instructions a register pair).  Column r of the product is then row r / 2 + 8 (r % 2) of its 16.  us, before ->
+// after:
+//   decoding (KS = 0)  64 rows 28672 x 4096 58.2 -> 50.8, 14336 wide down 28.0 -> 24.8, 2560 x 2048 8.2 -> 6.7; 24 rows 7168 x 8192 26.7 ->
+//                      23.1; 16384 x 2048 at 8 rows 16.5 -> 13.5, at 32 17.6 -> 14.8
+//   k in slices        37 rows 2560 x 2048 8.6 -> 6.9, 2048 x 2048 8.3 -> 6.8, 4096 x 4096 15.4 -> 11.6; 16 rows 4096 x 14336 28.7 -> 22.8
+//
+// KS = 0: the waves interleave over the unit's pairs of k-tiles.  KS = 4, 8, 16: k in KS whole slices, each added up by one wave
 // and the slices in order - the sums of a prefill projection cut into KS slices (gemm_prefill.hip), bit for bit, without
 // its slabs and their reduction launch.  With four slices two halves of the workgroup take SG strips each; with sixteen a
 // wave takes two slices one after the other.
-template <int MB, int SG, int KS = 0, bool ACT = false>
+__device__ __forceinline__ int mfma_row(int b, int r) { return b * 16 + (r >> 1) + 8 * (r & 1); }
+
+template <int HB, int SG, int KS = 0, bool ACT = false, bool PAIR = true>
 __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
-    constexpr int U = (SG + MB <= 6) ? 2 : 1;  // k-tiles per stage (register budget)
-    constexpr int kStep = KS ? 1 : kGW;        // k-tiles between a wave's tiles
+    constexpr int MB = (HB + 1) / 2;
+    constexpr int U = PAIR || SG + MB <= 6 ? 2 : 1;          // k-tiles per stage
+    constexpr int kNext = PAIR ? 1 : kGW;                    // k-tiles between two of a stage
+    constexpr int kStep = KS ? U : U * kGW;                  // ... and between a wave's stages
+    static_assert(PAIR || KS == 0, "slices go by pairs");
     constexpr int kHalves = KS == 4 ? 2 : 1, kTurns = KS == 16 ? 2 : 1;
     constexpr int kSlots = KS == 0 || KS == 4 ? kGW : KS;   // accumulator sets that meet in LDS
     // cross-wave reduction buffer [kGW][SG][MB][64 lanes][4]: 8 KiB per (strip, row block) pair,
@@ -470,11 +487,13 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
+    const bool odd = r & 1;
 
-    // this lane's x rows (B operand column), clamped into [0, M)
-    const uint16_t* xrow[MB];
+    // this lane's x rows, clamped into [0, M), at its 16 bytes of the first of two k-tiles; and which of the two it takes
+    const uint16_t* xrow[HB];
 #pragma unroll
-    for (int b = 0; b < MB; ++b) xrow[b] = a.x + (int64_t)min(b * 16 + r, a.m - 1) * a.ldx + q * 8;
+    for (int h = 0; h < HB; ++h) xrow[h] = a.x + (int64_t)min(PAIR ? h * 8 + (r >> 1) : h * 8 + r, a.m - 1) * a.ldx + q * 8;
+    const int second = odd ? 32 : 0;
 
     for (int u = blockIdx.x; u < a.nunits; u += gridDim.x) {
         const int g = KS ? u : u / a.ksplit, ks = KS ? 0 : u - g * a.ksplit;
@@ -485,13 +504,16 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
         const int strip0 = (g * kHalves + (KS == 4 ? wid >> 2 : 0)) * SG;
         const int kt0 = KS ? slice * a.ktps : ks * a.ktps;
         const int kt1 = min(a.kt, kt0 + a.ktps);
-        const int ntile = KS ? kt1 - kt0 : (kt1 - kt0 - wid + kGW - 1) / kGW;
-        const int last = max(ntile - 1, 0);
-        const int ktw = KS ? kt0 : kt0 + (ntile > 0 ? wid : 0);  // a wave without tiles still loads (clamped)
+        // this wave's stages, and the first k-tile; a wave without tiles still loads (clamped)
+        const int ntile = PAIR ? (kt1 - kt0 + 1) >> 1 : kt1 - kt0;   // (PAIR: of two)
+        const int mine = KS ? ntile : (ntile - wid + kGW - 1) / kGW;
+        const int nchunk = PAIR ? mine : (mine + U - 1) / U;
+        const int last = max(nchunk - 1, 0);
+        const int ktw = KS ? kt0 : kt0 + (mine > 0 ? (PAIR ? 2 : 1) * wid : 0);
         const uint4* wbase[SG];
 #pragma unroll
         for (int sI = 0; sI < SG; ++sI)
-            wbase[sI] = a.w + ((int64_t)min(strip0 + sI, a.nt - 1) * a.kt + ktw) * 64 + lane;
+            wbase[sI] = a.w + ((int64_t)min(strip0 + sI, a.nt - 1) * a.kt) * 64 + lane;
 
         f32x4_t acc[SG][MB];
 #pragma unroll
@@ -499,37 +521,67 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
 #pragma unroll
             for (int b = 0; b < MB; ++b) acc[sI][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
-        uint4 wA[U][SG], wB[U][SG], xA[U][MB], xB[U][MB];
-        auto load = [&](uint4(&wb)[U][SG], uint4(&xb)[U][MB], int c) {
+        constexpr int XR = PAIR ? HB : U * MB;   // requests of x in a stage
+        uint4 wA[U][SG], wB[U][SG], xA[XR], xB[XR];
+        auto load = [&](uint4(&wb)[U][SG], uint4(&xb)[XR], int c) {
+            const int t = ktw + min(c, last) * kStep;
+            const bool whole = t + kNext < kt1;   // uniform: half a stage at the end is asked for twice
+            if constexpr (PAIR) {
+                const int even_block = t * 32 + (whole ? second : 0), odd_block = t * 32 + (whole ? 32 - second : 0);
+#pragma unroll
+                for (int h = 0; h < HB; ++h) xb[h] = ld16(xrow[h] + (h & 1 ? odd_block : even_block));
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int i = 0; i < U; ++i) {
-                const int t = min(c * U + i, last);
+                const int ti = whole ? t + i * kNext : t;
 #pragma unroll
-                for (int sI = 0; sI < SG; ++sI) wb[i][sI] = ld16_nt(wbase[sI] + (int64_t)t * (kStep * 64));
-                const int kcol = (ktw + t * kStep) * 32;
+                for (int sI = 0; sI < SG; ++sI) wb[i][sI] = ld16_nt(wbase[sI] + (int64_t)ti * 64);
+                if constexpr (!PAIR) {
 #pragma unroll
-                // (with these requests removed the four Llama-3-8B projections at M = 32 take 90 us
-                // instead of 104: the x path costs about 13 %)
-                for (int b = 0; b < MB; ++b) xb[i][b] = ld16(xrow[b] + kcol);
+                    for (int b = 0; b < MB; ++b) xb[i * MB + b] = ld16(xrow[2 * b] + ti * 32);
+                }
             }
         };
-        auto compute = [&](const uint4(&wb)[U][SG], const uint4(&xb)[U][MB], int c, bool all) {
+        auto compute = [&](const uint4(&wb)[U][SG], const uint4(&xb)[XR], int c, bool all) {
+            if (!all && c >= nchunk) return;   // wave-uniform
+            auto swap = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true); };   // lanes 1 0 3 2
+            auto one = [&](uint32_t e, uint32_t o) { return odd ? o : e; };
+            auto operand = [&](int i, int b) {
+                if constexpr (!PAIR) return __builtin_bit_cast(bf16x8_t, xb[i * MB + b]);
+                const uint4 e = xb[2 * b], o = xb[2 * b + 1 < HB ? 2 * b + 1 : 2 * b];
+                const uint4 v = i == 0 ? make_uint4(one(e.x, o.x), one(e.y, o.y), one(e.z, o.z), one(e.w, o.w))
+                                       : make_uint4(swap(one(o.x, e.x)), swap(one(o.y, e.y)), swap(one(o.z, e.z)), swap(one(o.w, e.w)));
+                return __builtin_bit_cast(bf16x8_t, v);
+            };
+            auto multiply = [&](int i, int b, bf16x8_t xf) {
 #pragma unroll
-            for (int i = 0; i < U; ++i) {
-                if (all || c * U + i < ntile) {  // wave-uniform
+                for (int sI = 0; sI < SG; ++sI)
+                    acc[sI][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wb[i][sI]), xf, acc[sI][b], 0, 0, 0);
+            };
+            const bool whole = U == 2 && (all || ktw + c * kStep + kNext < kt1);   // wave-uniform (only the last stage may be half of one)
+            if constexpr (SG * MB >= 8) {   // (a row block at a time: the operands of all of them do not fit)
 #pragma unroll
-                    for (int sI = 0; sI < SG; ++sI) {
-                        const bf16x8_t wf = __builtin_bit_cast(bf16x8_t, wb[i][sI]);
+                for (int b = 0; b < MB; ++b) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    multiply(0, b, operand(0, b));
+                    if (whole) multiply(U - 1, b, operand(U - 1, b));
+                }
+            } else {
+                bf16x8_t f[U][MB];
 #pragma unroll
-                        for (int b = 0; b < MB; ++b)
-                            acc[sI][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                wf, __builtin_bit_cast(bf16x8_t, xb[i][b]), acc[sI][b], 0, 0, 0);
-                    }
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int i = 0; i < U; ++i) f[i][b] = operand(i, b);
+#pragma unroll
+                for (int b = 0; b < MB; ++b) multiply(0, b, f[0][b]);
+                if (whole) {
+#pragma unroll
+                    for (int b = 0; b < MB; ++b) multiply(U - 1, b, f[U - 1][b]);
                 }
             }
         };
 
-        const int nchunk = (ntile + U - 1) / U;
         // Both first stages go out unconditionally (indices past the end are clamped) and the steady
         // state has no branch around a request, so the compiler's wait counts are exact: with a
         // request under an `if` anywhere before or inside the loop every wait covers both stages
@@ -560,7 +612,7 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
             if (c + 2 < nchunk) compute(wA, xA, c + 2, false);
         }
 
-        // acc[s][b][j] = C[n = 16 (g SG + s) + 4q + j][m = 16b + r]
+        // acc[s][b][j] = C[n = 16 (g SG + s) + 4q + j][m = 16 b + r, PAIR: mfma_row(b, r)]
 #pragma unroll
         for (int sI = 0; sI < SG; ++sI)
 #pragma unroll
@@ -574,7 +626,7 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
             const int strip = sb / MB, b = sb - strip * MB;
             const int half = strip / SG, sI = strip - half * SG;
             const int rr = l & 15, qq = l >> 4;
-            const int m = b * 16 + rr;
+            const int m = PAIR ? mfma_row(b, rr) : b * 16 + rr;
             const int nt = g * kHalves * SG + strip;
             auto sum_at = [&](int ll) {
                 f32x4_t s = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -974,19 +1026,53 @@ static int launch_dot_waves(const GemmArgs& a, int waves, int grid, hipStream_t 
     return waves == 16 ? launch_dot_pro<M, 16>(a, grid, s) : launch_dot_pro<M, 8>(a, grid, s);
 }
 
-template <int MB, int SG, bool ACT>
+template <int HB, int SG, bool ACT, bool PAIR>
 static int launch_mfma_act(const GemmArgs& a, int grid, hipStream_t s) {
-    constexpr size_t lds = (size_t)kGW * SG * MB * 64 * 4 * sizeof(float);
+    constexpr size_t lds = (size_t)kGW * SG * ((HB + 1) / 2) * 64 * 4 * sizeof(float);
     static_assert(lds <= 128 * 1024, "reduction buffer fits LDS");
     static LdsOptIn opted;  // per instantiation
-    if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<MB, SG, 0, ACT>, lds, opted)) return rc;
-    hipLaunchKernelGGL((wgemm_mfma_kernel<MB, SG, 0, ACT>), dim3(grid), dim3(kGT), lds, s, a);
+    if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<HB, SG, 0, ACT, PAIR>, lds, opted)) return rc;
+    hipLaunchKernelGGL((wgemm_mfma_kernel<HB, SG, 0, ACT, PAIR>), dim3(grid), dim3(kGT), lds, s, a);
     return check_launch();
 }
 
-template <int MB, int SG>
-static int launch_mfma(const GemmArgs& a, int grid, hipStream_t s) {
-    return a.act.kind ? launch_mfma_act<MB, SG, true>(a, grid, s) : launch_mfma_act<MB, SG, false>(a, grid, s);
+// Pairs of k-tiles, or a k-tile a request (PAIR = false).  By pairs the waves read their weights two tiles at a time, which a long
+// stream takes 3 to 7 % slower (128256 x 8192 at 8 rows 317 -> 339 us, 128256 x 4096 169 -> 175: the eight waves' 1 KiB pieces no longer
+// lie side by side), so it is for where x is what costs: not up to 16 rows of k past 2048 in groups of strips, nor in groups of
+// seven (28672 x 4096 at 32 rows 38.4, 39.6 by pairs), nor one 8-row block, whose operand repeats its rows, in groups narrower
+// than four.
+template <int HB>
+static int launch_mfma(const GemmArgs& a, int sg, int grid, hipStream_t s) {
+    auto strips = [&](auto count) {
+        constexpr int SG = decltype(count)::value;
+        if constexpr ((HB <= 2 && SG > 1) || HB == 1 || SG == 7) {
+            constexpr int rows = HB <= 2 ? 2 : 4;
+            if (a.k > 2048 || (HB == 1 && SG < 4))
+                return a.act.kind ? launch_mfma_act<rows, SG, true, false>(a, grid, s) : launch_mfma_act<rows, SG, false, false>(a, grid, s);
+        }
+        return a.act.kind ? launch_mfma_act<HB, SG, true, true>(a, grid, s) : launch_mfma_act<HB, SG, false, true>(a, grid, s);
+    };
+    if constexpr (HB <= 4) {
+        if (sg == 7) return strips(std::integral_constant<int, 7>());
+    }
+    return sg == 4   ? strips(std::integral_constant<int, 4>())
+           : sg == 3 ? strips(std::integral_constant<int, 3>())
+           : sg == 2 ? strips(std::integral_constant<int, 2>())
+                     : strips(std::integral_constant<int, 1>());
+}
+// `launch` with the 8-row blocks of `m` rows
+template <class F>
+static int with_row_blocks(int m, F launch) {
+    switch ((m + 7) / 8) {
+        case 1: return launch(std::integral_constant<int, 1>());
+        case 2: return launch(std::integral_constant<int, 2>());
+        case 3: return launch(std::integral_constant<int, 3>());
+        case 4: return launch(std::integral_constant<int, 4>());
+        case 5: return launch(std::integral_constant<int, 5>());
+        case 6: return launch(std::integral_constant<int, 6>());
+        case 7: return launch(std::integral_constant<int, 7>());
+        default: return launch(std::integral_constant<int, 8>());
+    }
 }
 
 // strips per workgroup of the MFMA form: the cross-wave reduction buffer is 8 KiB per
@@ -1049,25 +1135,25 @@ static int ordered_strip_group(int m, int nt, int kt, int ks) {
     return best;
 }
 
-template <int MB, int SG, int KS>
+template <int HB, int SG, int KS>
 static int launch_ordered(const GemmArgs& a, int grid, hipStream_t s) {
-    constexpr size_t lds = (size_t)(KS == 16 ? 16 : kGW) * SG * MB * 64 * 4 * sizeof(float);
+    constexpr size_t lds = (size_t)(KS == 16 ? 16 : kGW) * SG * ((HB + 1) / 2) * 64 * 4 * sizeof(float);
     static_assert(lds <= 128 * 1024, "reduction buffer fits LDS");
     static LdsOptIn opted;  // per instantiation
-    if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<MB, SG, KS>, lds, opted)) return rc;
-    hipLaunchKernelGGL((wgemm_mfma_kernel<MB, SG, KS>), dim3(grid), dim3(kGT), lds, s, a);
+    if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<HB, SG, KS>, lds, opted)) return rc;
+    hipLaunchKernelGGL((wgemm_mfma_kernel<HB, SG, KS>), dim3(grid), dim3(kGT), lds, s, a);
     return check_launch();
 }
-template <int MB>
-static int launch_ordered_mb(const GemmArgs& a, int sg, int ks, int grid, hipStream_t s) {
+template <int HB>
+static int launch_ordered_rows(const GemmArgs& a, int sg, int ks, int grid, hipStream_t s) {
     switch (ks * 8 + sg) {
-        case 4 * 8 + 1: return launch_ordered<MB, 1, 4>(a, grid, s);
-        case 4 * 8 + 2: return launch_ordered<MB, 2, 4>(a, grid, s);
-        case 8 * 8 + 1: return launch_ordered<MB, 1, 8>(a, grid, s);
-        case 8 * 8 + 2: return launch_ordered<MB, 2, 8>(a, grid, s);
-        case 8 * 8 + 4: return launch_ordered<MB, 4, 8>(a, grid, s);
-        case 16 * 8 + 1: return launch_ordered<MB, 1, 16>(a, grid, s);
-        case 16 * 8 + 2: return launch_ordered<MB, 2, 16>(a, grid, s);
+        case 4 * 8 + 1: return launch_ordered<HB, 1, 4>(a, grid, s);
+        case 4 * 8 + 2: return launch_ordered<HB, 2, 4>(a, grid, s);
+        case 8 * 8 + 1: return launch_ordered<HB, 1, 8>(a, grid, s);
+        case 8 * 8 + 2: return launch_ordered<HB, 2, 8>(a, grid, s);
+        case 8 * 8 + 4: return launch_ordered<HB, 4, 8>(a, grid, s);
+        case 16 * 8 + 1: return launch_ordered<HB, 1, 16>(a, grid, s);
+        case 16 * 8 + 2: return launch_ordered<HB, 2, 16>(a, grid, s);
         default: return MV_ERR_UNSUPPORTED;
     }
 }
@@ -1122,8 +1208,7 @@ int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const 
     // a second workgroup per CU where its reduction buffer fits beside the first
     const int per_cu = (ks == 16 ? 16 : kGW) * sg * mb <= 64 ? 2 : 1;
     const int grid = a.nunits < num_cus() * per_cu ? a.nunits : num_cus() * per_cu;
-    const int rc = mb == 1 ? launch_ordered_mb<1>(a, sg, ks, grid, s) : mb == 2 ? launch_ordered_mb<2>(a, sg, ks, grid, s)
-                   : mb == 3 ? launch_ordered_mb<3>(a, sg, ks, grid, s) : launch_ordered_mb<4>(a, sg, ks, grid, s);
+    const int rc = with_row_blocks(m, [&](auto hb) { return launch_ordered_rows<decltype(hb)::value>(a, sg, ks, grid, s); });
     if (rc != MV_OK || !norm) return rc;
     return launch_wgemm_finalize_norm(norm->slab, 1, m, n, bias, norm, s);
 }
@@ -1285,11 +1370,7 @@ static int wgemm_impl(const void* x, int64_t ldx, const void* add_r, int64_t ld_
         case 3: rc = launch_dot_waves<3>(a, waves, grid, s); break;
         case 4: rc = launch_dot_waves<4>(a, waves, grid, s); break;
         default: {
-            const int mb = (m + 15) / 16;
-            if (mb == 1) rc = sg == 7 ? launch_mfma<1, 7>(a, grid, s) : sg == 3 ? launch_mfma<1, 3>(a, grid, s) : sg == 4 ? launch_mfma<1, 4>(a, grid, s) : sg == 2 ? launch_mfma<1, 2>(a, grid, s) : launch_mfma<1, 1>(a, grid, s);
-            else if (mb == 2) rc = sg == 7 ? launch_mfma<2, 7>(a, grid, s) : sg == 3 ? launch_mfma<2, 3>(a, grid, s) : sg == 4 ? launch_mfma<2, 4>(a, grid, s) : sg == 2 ? launch_mfma<2, 2>(a, grid, s) : launch_mfma<2, 1>(a, grid, s);
-            else if (mb == 3) rc = sg == 4 ? launch_mfma<3, 4>(a, grid, s) : sg == 3 ? launch_mfma<3, 3>(a, grid, s) : sg == 2 ? launch_mfma<3, 2>(a, grid, s) : launch_mfma<3, 1>(a, grid, s);
-            else rc = sg == 4 ? launch_mfma<4, 4>(a, grid, s) : sg == 3 ? launch_mfma<4, 3>(a, grid, s) : sg == 2 ? launch_mfma<4, 2>(a, grid, s) : launch_mfma<4, 1>(a, grid, s);
+            rc = with_row_blocks(m, [&](auto hb) { return launch_mfma<decltype(hb)::value>(a, sg, grid, s); });
         }
     }
     if (rc != MV_OK || slabs_only) return rc;

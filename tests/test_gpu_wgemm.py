@@ -255,3 +255,29 @@ def test_wgemm_widths_at_33_to_64_rows(mv, m, n, k):
 def test_wgemm_postnorm_with_part_of_a_workgroup_idle(mv, n):
     """512 and 1024 threads to a row, the last of them past the row's end."""
     test_wgemm_postnorm_is_bit_identical_to_separate_kernels(mv, 8, n, 1024)
+
+
+# requests of x by two k-tiles: every count of 8-row blocks and its edges, k that ends in half a pair (for the whole unit, for one wave, for a
+# unit shorter than the waves), groups of one to seven strips, and the k past which up to 16 rows go a k-tile a request
+@pytest.mark.parametrize("m", [5, 8, 9, 15, 16, 17, 24, 25, 33, 40, 41, 56, 57, 64])
+@pytest.mark.parametrize("n,k,sg", [(48, 32, 0), (64, 96, 0), (1040, 2016, 0), (336, 2080, 1), (336, 1056, 2), (336, 544, 4), (336, 2080, 4),
+                                    (336, 288, 7), (336, 2208, 7)])
+def test_wgemm_by_pairs_of_k_tiles(mv, m, n, k, sg):
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.linear import StreamedWeight, wgemm
+
+    if sg == 7 and m > 32:
+        pytest.skip("seven strips go with up to 32 rows")
+    x, w, _ = _mk(m, n, k, seed=m + n + k, scale=k ** -0.5)
+    wide = torch.full((m, k + 24), float("nan"), dtype=torch.bfloat16, device=DEV)    # nothing beside the rows reaches a sum
+    wide[:, :k] = x.to(DEV)
+    sw = StreamedWeight.from_linear(w.to(DEV))
+    nv.lib().mv_wgemm_tune(3, sg)
+    try:
+        acc = wgemm(wide[:, :k], sw, torch.full((m, n), float("nan"), dtype=torch.float32, device=DEV))
+    finally:
+        nv.lib().mv_wgemm_tune(3, 0)
+    want = x.double() @ w.double().t()
+    # fp32 sums of exact products: at most k roundings of 2^-24 of partial sums that the absolute products bound
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((acc.cpu().double() - want).abs() <= bound).all())
