@@ -314,10 +314,14 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
         wp[i] = a.w + ((int64_t)min(nt0 + i, a.nt - 1) * a.kt + kt0) * 64 + lane;
 
     // ---- x: global -> LDS directly, BUFS stages deep, in fragment order ---------------------
-    // The LDS image of a stage is 16 fragment tiles (8 m-tiles x 2 k-tiles) of 1 KiB in MFMA
-    // operand order: lane l of the tile (mt, kk) holds x[16 mt + (l & 15)][32 kk + 8 (l >> 4) ..+7],
-    // so a fragment read is linear in the lane (no bank conflicts).  Wave w fills tiles 4w..4w+3
-    // with global_load_lds (no staging registers, no LDS store instructions).  These loads are
+    // The LDS image of a stage is an m-tile after the other, 16 rows of 128 bytes (64 k) each; the 16-byte chunk c of row r sits
+    // at position c ^ ((r >> 1) & 7) of its row, which keeps the fragment reads (lane (r, q) reads chunk 4 kk + q of row r) free
+    // of bank conflicts, and a request of global_load_lds is eight whole rows of it (no staging registers, no LDS store
+    // instructions).  Requests in the operand's own order, sixteen rows of 64 bytes with a row to each lane, come in at half that
+    // pace: the address path takes the lines that neighbouring lanes do not share one after the other, and x was more of a
+    // stage's time than its weights.  us: 64 rows 2048 x 2048
+    // 10.4 -> 9.6, 500 rows 11264 x 2048 37.5 -> 32.2, 704 rows 6144 x 4096 68.2 -> 60.4, 1024 rows 4096 x 14336 133 -> 121, 1408 rows 2048 x 5632
+    // 64.9 -> 59.0.  These loads are
     // issued through inline assembly: when the compiler sees them it stops trusting request
     // order and waits for ALL outstanding loads before every weight use and every LDS read;
     // hidden from it they only make its counted waits wait for more (requests complete in
@@ -326,8 +330,8 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     const uint16_t* xg[XP];
 #pragma unroll
     for (int j = 0; j < XP; ++j) {
-        const int tile = wid * XP + j;
-        xg[j] = a.x + (int64_t)min(m0 + (tile >> 1) * 16 + r, a.m - 1) * a.ldx + kt0 * 32 + ((tile & 1) * 4 + q) * 8;
+        const int piece = wid * XP + j, row = piece * 8 + (lane >> 3);
+        xg[j] = a.x + (int64_t)min(m0 + row, a.m - 1) * a.ldx + kt0 * 32 + ((lane & 7) ^ ((row >> 1) & 7)) * 8;
     }
     const unsigned xs_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)&xs[0][0];
     auto x_fetch = [&](int s, int buf) {
@@ -339,9 +343,10 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(dst) : "memory");
         }
     };
+    const int frag = r * 128 + ((q ^ ((r >> 1) & 7)) * 16);
     auto x_frag = [&](int buf, int t, int kk) {
         return __builtin_bit_cast(
-            bf16x8_t, *reinterpret_cast<const uint4*>(&xs[buf][(t * 2 + kk) * 1024 + lane * 16]));
+            bf16x8_t, *reinterpret_cast<const uint4*>(&xs[buf][t * 2048 + (frag ^ (kk * 64))]));
     };
 
     f32x4_t acc[NT][MT];

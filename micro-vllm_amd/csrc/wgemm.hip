@@ -1116,9 +1116,10 @@ static int mfma_strip_group(int m, int nt, int kt, bool free_reduce) {
     return best;
 }
 
-// Strips per wave of the ordered form: the model above, the workgroup's strips being SG or, with four slices, 2 SG
+// Strips per wave of the ordered form: the model above, the workgroup's strips being SG or, with four slices, 2 SG, and x out of
+// L2 at 17 MB/us, in 8-row blocks (requests of two k-tiles; the groups that measured fastest at 31 of 33 shapes, 29 at 12.9)
 static int ordered_strip_group(int m, int nt, int kt, int ks) {
-    const int mb = (m + 15) / 16, halves = ks == 4 ? 2 : 1;
+    const int mb = (m + 15) / 16, rows = (m + 7) / 8 * 8, halves = ks == 4 ? 2 : 1;
     const int cus = num_cus();
     int best = 1;
     double best_us = 1e30;
@@ -1126,7 +1127,7 @@ static int ordered_strip_group(int m, int nt, int kt, int ks) {
         if (sg * mb > (ks == 16 ? 8 : 16) || (sg == 4 && ks != 8)) continue;   // 128 KiB of LDS; the instances there are
         const long units = (nt + sg * halves - 1) / (sg * halves);
         const double fill = (double)units / (double)(((units + cus - 1) / cus) * cus);
-        const double us = (double)nt * kt * 1024e-6 / (6.45 * fill) + (double)units * halves * m * kt * 64e-6 / 12.9;
+        const double us = (double)nt * kt * 1024e-6 / (6.45 * fill) + (double)units * halves * rows * kt * 64e-6 / 17.0;
         if (us < best_us) {
             best_us = us;
             best = sg;
@@ -1158,24 +1159,18 @@ static int launch_ordered_rows(const GemmArgs& a, int sg, int ks, int grid, hipS
     }
 }
 
-// One block of rows (up to 16), or rows times the k-tiles a wave walks up to a limit, on enough strips: a wave walks its slice (of
-// sixteen, two) alone, each k-tile in the time its rows take, and past that its chain, or on many strips the x each of them reads
-// again, is longer than the sliced tiles and their reduction.  The limits lie between what was faster and what was not (n x
-// k, us, 64-row sliced tiles -> here).  Eight and four slices, 512: 64 rows 2560 x 2048 13.1 -> 12.1 and 8192 x 1024 15.0 -> 13.5, 32 rows
-// 16384 x 2048 18.8 -> 16.6 (all 512), but 37 rows (592) 11264 x 2048 16.7 -> 17.7 and 6144 x 4096 17.2 -> 17.7, 64 rows 5120 x 3072
-// (768) 17.0 -> 19.8 and 8192 x 2048 (1024) 16.3 -> 22.7.  Long slices, 448: 17 rows 2048 x 5632 (374) 10.4 -> 12.0 where 128-row tiles took
-// 13.2, 24 rows (528) 10.7 -> 14.2.  Sixteen slices, whose reduction reads most, 592: 37 rows 4096 x 4096 16.5 -> 15.6, 48 rows (768)
-// 17.5 -> 17.6.
-// Against tiles narrow enough to fill the chip (`strips` of 1 or 2) the limits lie lower, for one block of rows too: 320, 448
-// for two strips and short slices.  16 rows 2048 x 5632 (352) 11.8 -> 10.6 in tiles, 1280 x 8192 (512) 14.0 -> 12.5, 64 rows 2048 x 2048
-// (512) 12.0 -> 10.4, but 37 rows (296) 8.6 against 9.1, 32 rows 3072 x 3072 (384) 10.8 against 11.9.
+// Up to a limit on rows x k-tiles: a workgroup reads all of x for the strips it has, whatever their number, where the sliced tiles
+// read a piece and pay for slabs and their reduction.  Sixty a strip and no fewer than 4096 (n x k, us, sliced
+// tiles and their reduction -> here): 37 rows 2048 x 2048 8.8 -> 6.9, 11264 x 2048 17.3 -> 13.9, 6144 x 4096 18.3 -> 14.4, 7168 x 8192 35.2 ->
+// 26.3, 8192 x 3584 19.8 -> 13.7, 4096 x 3584 12.8 -> 10.4; 64 rows 2048 x 2048 9.7 -> 8.3, 8192 x 1024 13.6 -> 9.1, 1536 x 4096 13.4 -> 13.6
+// (8192 for 96 strips: out); 256 strips of 448 k-tiles 32 rows 31.2 -> 29.4, 40 rows (17920) 32.0 -> 32.9; 80 strips of 256 16 rows 13.1 ->
+// 12.4, 20 rows (6144) 12.9 -> 13.5.  Tiles narrow enough to give every unit a slice (`strips` of 1) of a long k are ahead from nine rows on:
+// 2048 x 5632 8 rows 9.1, 9.1, 16 rows 9.2, 9.8, 37 rows 10.9, 13.4.
 bool wgemm_ordered_takes(int m, int nt, int kt, int ks, int strips) {
-    const int blocks = (m + 15) / 16, walk = ks == 4 ? kt / 4 : kt / 8;
-    if ((ks != 4 && ks != 8 && ks != 16) || blocks > 4) return false;
-    const bool narrow = strips == 1 || strips == 2;
-    const int most = strips == 1 || (narrow && walk > 16) ? 320 : narrow ? 448 : ks == 16 ? 592 : walk > 16 ? 448 : 512;
-    if (blocks == 1) return !narrow || m * walk <= most;
-    return m * walk <= most && blocks * kt <= 384 && nt >= 128 && (int64_t)blocks * kt * nt <= 150000;
+    if ((ks != 4 && ks != 8 && ks != 16) || m > 64) return false;
+    const int rows = (m + 7) / 8 * 8;
+    if (strips == 1 && kt > 128) return rows <= 8;
+    return (int64_t)rows * kt <= std::max(60 * nt, 4096);
 }
 
 // x [m, k] . W^T with the sums of `ks` slices of k added in order, epilogue as mv_gemm_prefill_ws, or the norm's.
