@@ -467,19 +467,23 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 //
 // KS = 0: the waves interleave over the unit's pairs of k-tiles.  KS = 4, 8, 16: k in KS whole slices, each added up by one wave
 // and the slices in order - the sums of a prefill projection cut into KS slices (gemm_prefill.hip), bit for bit, without
-// its slabs and their reduction launch.  With four slices two halves of the workgroup take SG strips each; with sixteen a
-// wave takes two slices one after the other.
+// its slabs and their reduction launch.  With four slices a workgroup has four waves, each with four stages in flight (a wave a
+// SIMD has the registers; two halves of eight waves on strips of their own read x twice: 37 rows 11264 x 2048 14.0 us, 12.2 so, 8192 x
+// 1024 7.7 -> 7.0, 4096 x 1024 6.9 -> 5.3); with sixteen a wave takes two slices one after the other.  Three or four stages elsewhere cost
+// 0 to 35 %: a wave has few stages, and those past the end are asked for as well.
 __device__ __forceinline__ int mfma_row(int b, int r) { return b * 16 + (r >> 1) + 8 * (r & 1); }
 
 template <int HB, int SG, int KS = 0, bool ACT = false, bool PAIR = true>
-__global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
+__global__ __launch_bounds__(KS == 4 ? 4 * kWave : kGT) void wgemm_mfma_kernel(GemmArgs a) {
+    constexpr int kWaves = KS == 4 ? 4 : kGW;
+    constexpr int ST = KS == 4 ? 4 : 2;                      // stages in flight
     constexpr int MB = (HB + 1) / 2;
     constexpr int U = PAIR || SG + MB <= 6 ? 2 : 1;          // k-tiles per stage
     constexpr int kNext = PAIR ? 1 : kGW;                    // k-tiles between two of a stage
     constexpr int kStep = KS ? U : U * kGW;                  // ... and between a wave's stages
     static_assert(PAIR || KS == 0, "slices go by pairs");
-    constexpr int kHalves = KS == 4 ? 2 : 1, kTurns = KS == 16 ? 2 : 1;
-    constexpr int kSlots = KS == 0 || KS == 4 ? kGW : KS;   // accumulator sets that meet in LDS
+    constexpr int kTurns = KS == 16 ? 2 : 1;
+    constexpr int kSlots = KS == 0 ? kGW : KS;   // accumulator sets that meet in LDS
     // cross-wave reduction buffer [kGW][SG][MB][64 lanes][4]: 8 KiB per (strip, row block) pair,
     // up to 128 KiB (dynamic: past the 64 KiB a static array may have)
     extern __shared__ __attribute__((aligned(16))) float red[];
@@ -499,9 +503,9 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
         const int g = KS ? u : u / a.ksplit, ks = KS ? 0 : u - g * a.ksplit;
 #pragma unroll
         for (int turn = 0; turn < kTurns; ++turn) {
-        const int slice = KS == 4 ? wid & 3 : wid + turn * kGW;   // (KS > 0)
+        const int slice = wid + turn * kGW;   // (KS > 0)
         const int slot = KS == 16 ? slice : wid;
-        const int strip0 = (g * kHalves + (KS == 4 ? wid >> 2 : 0)) * SG;
+        const int strip0 = g * SG;
         const int kt0 = KS ? slice * a.ktps : ks * a.ktps;
         const int kt1 = min(a.kt, kt0 + a.ktps);
         // this wave's stages, and the first k-tile; a wave without tiles still loads (clamped)
@@ -522,7 +526,7 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
             for (int b = 0; b < MB; ++b) acc[sI][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
         constexpr int XR = PAIR ? HB : U * MB;   // requests of x in a stage
-        uint4 wA[U][SG], wB[U][SG], xA[XR], xB[XR];
+        uint4 wr[ST][U][SG], xr[ST][XR];
         auto load = [&](uint4(&wb)[U][SG], uint4(&xb)[XR], int c) {
             const int t = ktw + min(c, last) * kStep;
             const bool whole = t + kNext < kt1;   // uniform: half a stage at the end is asked for twice
@@ -582,35 +586,36 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
             }
         };
 
-        // Both first stages go out unconditionally (indices past the end are clamped) and the steady
+        // The first stages go out unconditionally (indices past the end are clamped) and the steady
         // state has no branch around a request, so the compiler's wait counts are exact: with a
-        // request under an `if` anywhere before or inside the loop every wait covers both stages
-        // and only one is ever in flight.  The last three chunks at most are handled after it.
-        // (The fences keep the two first stages in the order the loop issues them: interleaved by
+        // request under an `if` anywhere before or inside the loop every wait covers all stages
+        // and only one is ever in flight.  The last 2 ST - 1 chunks at most are handled after it.
+        // (The fences keep the first stages in the order the loop issues them: interleaved by
         // the scheduler they would make the loop's first wait, and through the back edge all of
-        // them, cover both stages.)
+        // them, cover them all.)
         __builtin_amdgcn_sched_barrier(0);
-        load(wA, xA, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        load(wB, xB, 1);
-        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < ST; ++i) {
+            load(wr[i], xr[i], i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         int c = 0;
-        for (; c + 3 < nchunk; c += 2) {
-            compute(wA, xA, c, true);
-            __builtin_amdgcn_sched_barrier(0);
-            load(wA, xA, c + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(wB, xB, c + 1, true);
-            __builtin_amdgcn_sched_barrier(0);
-            load(wB, xB, c + 3);
-            __builtin_amdgcn_sched_barrier(0);
+        for (; c + 2 * ST <= nchunk; c += ST) {
+#pragma unroll
+            for (int i = 0; i < ST; ++i) {
+                compute(wr[i], xr[i], c + i, true);
+                __builtin_amdgcn_sched_barrier(0);
+                load(wr[i], xr[i], c + i + ST);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        if (c < nchunk) {
-            compute(wA, xA, c, false);
-            if (c + 2 < nchunk) load(wA, xA, c + 2);
-            if (c + 1 < nchunk) compute(wB, xB, c + 1, false);
-            if (c + 2 < nchunk) compute(wA, xA, c + 2, false);
+#pragma unroll
+        for (int i = 0; i < ST; ++i) {
+            compute(wr[i], xr[i], c + i, false);
+            if (i < ST - 1 && c + i + ST < nchunk) load(wr[i], xr[i], c + i + ST);
         }
+#pragma unroll
+        for (int i = 0; i < ST - 1; ++i) compute(wr[i], xr[i], c + i + ST, false);
 
         // acc[s][b][j] = C[n = 16 (g SG + s) + 4q + j][m = 16 b + r, PAIR: mfma_row(b, r)]
 #pragma unroll
@@ -621,19 +626,18 @@ __global__ __launch_bounds__(kGT) void wgemm_mfma_kernel(GemmArgs a) {
         }
         __syncthreads();
         // one wave per (strip, row block) pair; more pairs than waves take a second turn
-        for (int sb = wid; sb < MB * SG * kHalves; sb += kGW) {
+        for (int sb = wid; sb < MB * SG; sb += kWaves) {
             const int l = lane;
-            const int strip = sb / MB, b = sb - strip * MB;
-            const int half = strip / SG, sI = strip - half * SG;
+            const int sI = sb / MB, b = sb - sI * MB;
             const int rr = l & 15, qq = l >> 4;
             const int m = PAIR ? mfma_row(b, rr) : b * 16 + rr;
-            const int nt = g * kHalves * SG + strip;
+            const int nt = g * SG + sI;
             auto sum_at = [&](int ll) {
                 f32x4_t s = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int w8 = 0; w8 < kSlots / kHalves; ++w8)
+                for (int w8 = 0; w8 < kSlots; ++w8)
                     s += *reinterpret_cast<const f32x4_t*>(
-                        &red[((((half * 4 + w8) * SG + sI) * MB + b) * 64 + ll) * 4]);
+                        &red[(((w8 * SG + sI) * MB + b) * 64 + ll) * 4]);
                 return s;
             };
             if (m < a.m && nt < a.nt) {
@@ -1116,18 +1120,17 @@ static int mfma_strip_group(int m, int nt, int kt, bool free_reduce) {
     return best;
 }
 
-// Strips per wave of the ordered form: the model above, the workgroup's strips being SG or, with four slices, 2 SG, and x out of
-// L2 at 17 MB/us, in 8-row blocks (requests of two k-tiles; the groups that measured fastest at 31 of 33 shapes, 29 at 12.9)
+// Strips per wave of the ordered form: the model above, x out of L2 at 17 MB/us, in 8-row blocks (requests of two k-tiles; the groups that measured fastest at 31 of 33 shapes, 29 at 12.9)
 static int ordered_strip_group(int m, int nt, int kt, int ks) {
-    const int mb = (m + 15) / 16, rows = (m + 7) / 8 * 8, halves = ks == 4 ? 2 : 1;
+    const int mb = (m + 15) / 16, rows = (m + 7) / 8 * 8;
     const int cus = num_cus();
     int best = 1;
     double best_us = 1e30;
-    for (int sg = 4; sg >= 1; sg /= 2) {
-        if (sg * mb > (ks == 16 ? 8 : 16) || (sg == 4 && ks != 8)) continue;   // 128 KiB of LDS; the instances there are
-        const long units = (nt + sg * halves - 1) / (sg * halves);
+    for (int sg = 4; sg >= 1; --sg) {
+        if (ks != 4 && (sg * mb > (ks == 16 ? 8 : 16) || sg == 3 || (sg == 4 && ks == 16))) continue;   // 128 KiB of LDS; the instances there are
+        const long units = (nt + sg - 1) / sg;
         const double fill = (double)units / (double)(((units + cus - 1) / cus) * cus);
-        const double us = (double)nt * kt * 1024e-6 / (6.45 * fill) + (double)units * halves * rows * kt * 64e-6 / 17.0;
+        const double us = (double)nt * kt * 1024e-6 / (6.45 * fill) + (double)units * rows * kt * 64e-6 / 17.0;
         if (us < best_us) {
             best_us = us;
             best = sg;
@@ -1138,11 +1141,11 @@ static int ordered_strip_group(int m, int nt, int kt, int ks) {
 
 template <int HB, int SG, int KS>
 static int launch_ordered(const GemmArgs& a, int grid, hipStream_t s) {
-    constexpr size_t lds = (size_t)(KS == 16 ? 16 : kGW) * SG * ((HB + 1) / 2) * 64 * 4 * sizeof(float);
+    constexpr size_t lds = (size_t)KS * SG * ((HB + 1) / 2) * 64 * 4 * sizeof(float);
     static_assert(lds <= 128 * 1024, "reduction buffer fits LDS");
     static LdsOptIn opted;  // per instantiation
     if (int rc = ensure_dynamic_lds((const void*)wgemm_mfma_kernel<HB, SG, KS>, lds, opted)) return rc;
-    hipLaunchKernelGGL((wgemm_mfma_kernel<HB, SG, KS>), dim3(grid), dim3(kGT), lds, s, a);
+    hipLaunchKernelGGL((wgemm_mfma_kernel<HB, SG, KS>), dim3(grid), dim3(KS == 4 ? 4 * kWave : kGT), lds, s, a);
     return check_launch();
 }
 template <int HB>
@@ -1150,6 +1153,8 @@ static int launch_ordered_rows(const GemmArgs& a, int sg, int ks, int grid, hipS
     switch (ks * 8 + sg) {
         case 4 * 8 + 1: return launch_ordered<HB, 1, 4>(a, grid, s);
         case 4 * 8 + 2: return launch_ordered<HB, 2, 4>(a, grid, s);
+        case 4 * 8 + 3: return launch_ordered<HB, 3, 4>(a, grid, s);
+        case 4 * 8 + 4: return launch_ordered<HB, 4, 4>(a, grid, s);
         case 8 * 8 + 1: return launch_ordered<HB, 1, 8>(a, grid, s);
         case 8 * 8 + 2: return launch_ordered<HB, 2, 8>(a, grid, s);
         case 8 * 8 + 4: return launch_ordered<HB, 4, 8>(a, grid, s);
@@ -1161,8 +1166,8 @@ static int launch_ordered_rows(const GemmArgs& a, int sg, int ks, int grid, hipS
 
 // Up to a limit on rows x k-tiles: a workgroup reads all of x for the strips it has, whatever their number, where the sliced tiles
 // read a piece and pay for slabs and their reduction.  Sixty a strip and no fewer than 4096 (n x k, us, sliced
-// tiles and their reduction -> here): 37 rows 2048 x 2048 8.8 -> 6.9, 11264 x 2048 17.3 -> 13.9, 6144 x 4096 18.3 -> 14.4, 7168 x 8192 35.2 ->
-// 26.3, 8192 x 3584 19.8 -> 13.7, 4096 x 3584 12.8 -> 10.4; 64 rows 2048 x 2048 9.7 -> 8.3, 8192 x 1024 13.6 -> 9.1, 1536 x 4096 13.4 -> 13.6
+// tiles and their reduction -> here): 37 rows 2048 x 2048 8.8 -> 6.9, 11264 x 2048 17.3 -> 12.2, 6144 x 4096 18.3 -> 14.4, 7168 x 8192 35.2 ->
+// 26.3, 8192 x 3584 19.8 -> 13.7, 4096 x 3584 12.8 -> 10.4; 64 rows 2048 x 2048 9.7 -> 8.3, 8192 x 1024 13.6 -> 8.2, 1536 x 4096 13.4 -> 13.6
 // (8192 for 96 strips: out); 256 strips of 448 k-tiles 32 rows 31.2 -> 29.4, 40 rows (17920) 32.0 -> 32.9; 80 strips of 256 16 rows 13.1 ->
 // 12.4, 20 rows (6144) 12.9 -> 13.5.  Tiles narrow enough to give every unit a slice (`strips` of 1) of a long k are ahead from nine rows on:
 // 2048 x 5632 8 rows 9.1, 9.1, 16 rows 9.2, 9.8, 37 rows 10.9, 13.4.
@@ -1197,11 +1202,11 @@ int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const 
     a.ksplit = 1;
     a.ktps = a.kt / ks;
     a.partial = norm ? norm->slab : nullptr;
-    const int sg = ordered_strip_group(m, a.nt, a.kt, ks), halves = ks == 4 ? 2 : 1;
-    a.nunits = (a.nt + sg * halves - 1) / (sg * halves);
+    const int sg = ordered_strip_group(m, a.nt, a.kt, ks);
+    a.nunits = (a.nt + sg - 1) / sg;
     const int mb = (m + 15) / 16;
     // a second workgroup per CU where its reduction buffer fits beside the first
-    const int per_cu = (ks == 16 ? 16 : kGW) * sg * mb <= 64 ? 2 : 1;
+    const int per_cu = ks == 4 ? 4 : ks * sg * mb <= 64 ? 2 : 1;
     const int grid = a.nunits < num_cus() * per_cu ? a.nunits : num_cus() * per_cu;
     const int rc = with_row_blocks(m, [&](auto hb) { return launch_ordered_rows<decltype(hb)::value>(a, sg, ks, grid, s); });
     if (rc != MV_OK || !norm) return rc;

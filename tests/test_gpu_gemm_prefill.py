@@ -511,3 +511,28 @@ def test_narrow_tiles_give_the_sums_of_wide_ones(mv, m, n, k, mode):
         return y
 
     assert torch.equal(run(m), run(rows)[:m])
+
+
+# slices added in the workgroup: four, eight and sixteen slices, every count of 8-row blocks, k-tiles of a slice that are fewer than the
+# stages in flight, as many, and a few more, groups of one to four strips with strips left over: the sums of the sliced 64-row tiles bit for bit
+@pytest.mark.parametrize("m", [5, 8, 9, 17, 25, 33, 40, 41, 49, 57, 64])
+@pytest.mark.parametrize("n,k", [(4112, 1024), (8224, 1024), (11280, 2048), (16400, 1024), (2064, 2048), (1536, 4096), (6160, 4096)])
+def test_short_prompts_add_their_slices_in_the_workgroup(mv, m, n, k):
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.linear import StreamedWeight, gemm_prefill
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    sw = StreamedWeight.from_linear(w)
+    got = gemm_prefill(x, sw, torch.full((m, n), float("nan"), dtype=torch.float32, device=DEV))
+    want = x.double() @ w.double().t()
+    # fp32 sums of exact products: at most k roundings of 2^-24 of partial sums that the absolute products bound
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((got.double() - want).abs() <= bound).all())
+    # a row among 65 goes through tiles, bit for bit the same where the plan cuts both into as many slices
+    L, ks = nv.lib(), nv.lib().mv_linear_slab_count(65, n, k)
+    counters = L.mv_gemm_prefill_workspace_bytes(65, n, k) - ks * 65 * n * 4
+    if L.mv_gemm_prefill_workspace_bytes(m, n, k) - counters == ks * m * n * 4:
+        more = torch.cat([x, torch.zeros(65 - m, k, dtype=torch.bfloat16, device=DEV)])
+        assert torch.equal(gemm_prefill(more, sw, torch.empty(65, n, dtype=torch.float32, device=DEV))[:m], got)
