@@ -317,9 +317,9 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     // The LDS image of a stage is an m-tile after the other, 16 rows of 128 bytes (64 k) each; the 16-byte chunk c of row r sits
     // at position c ^ ((r >> 1) & 7) of its row, which keeps the fragment reads (lane (r, q) reads chunk 4 kk + q of row r) free
     // of bank conflicts, and a request of global_load_lds is eight whole rows of it (no staging registers, no LDS store
-    // instructions).  Requests in the operand's own order, sixteen rows of 64 bytes with a row to each lane, come in at half that
-    // pace: the address path takes the lines that neighbouring lanes do not share one after the other, and x was more of a
-    // stage's time than its weights.  us: 64 rows 2048 x 2048
+    // instructions).  Requests in the operand's own order, sixteen rows of 64 bytes with a row to each lane, come in at 37 bytes
+    // a ns and unit, these at 100: the address path takes the lines that neighbouring lanes do not share one after the other, and x
+    // was more of a stage's time than its weights.  us: 64 rows 2048 x 2048
     // 10.4 -> 9.6, 500 rows 11264 x 2048 37.5 -> 32.2, 704 rows 6144 x 4096 68.2 -> 60.4, 1024 rows 4096 x 14336 133 -> 121, 1408 rows 2048 x 5632
     // 64.9 -> 59.0.  These loads are
     // issued through inline assembly: when the compiler sees them it stops trusting request

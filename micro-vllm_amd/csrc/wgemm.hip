@@ -456,7 +456,7 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 //
 // What a request of x costs is the compute unit's address path: neighbouring lanes in different lines are taken one after the
 // other.  Sixteen rows of 64 bytes with a row to each lane - the operand's own layout - are 37 bytes a ns and unit, two lanes to
-// a line 68, a weight tile's 1 KiB in one piece 130.  So a request is eight rows of two k-tiles, lane (r, q) taking 16 bytes q of
+// a line 73, a weight tile's 1 KiB in one piece 120.  So a request is eight rows of two k-tiles, lane (r, q) taking 16 bytes q of
 // row r / 2 and k-tile r % 2 (the odd 8-row block: k-tile 1 - r % 2), and the operands are made of two of them: the first k-tile's
 // is the first block's even lanes and the second's odd ones, the second k-tile's the other lanes, exchanged with their neighbours
 // (three vector instructions a register pair).  Column r of the product is then row r / 2 + 8 (r % 2) of its 16.  us, before ->
