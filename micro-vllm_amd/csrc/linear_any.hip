@@ -300,11 +300,11 @@ __device__ __forceinline__ bool lf_place(int id, int cols, int rows, int& col, i
 // the quarters of k side by side, each its 4 / KG one after the other (a second set of accumulators holds the sum so far).  A
 // step of 32 k: a wave splits sixteen rows at a time on their way into LDS, where a plane of parts of sixteen rows is 1 KB in the
 // instruction's own lane order; the rows of lane group q are exchanged by xor with 2 q, so that neither the writes (four lanes a
-// row, eight lanes a cycle) nor the reads (a lane a row) meet on a bank: counted 0 conflicts, 1.5 cycles of three without.  PF
+// row, eight lanes a cycle) nor the reads (a lane a row) meet on a bank: no conflicts counted, without it in three of five cycles that LDS is busy.  PF
 // steps are requested ahead.  DB: two buffers and one barrier a step, else one and two.
 // What bounds it: no one unit - at 2048 rows 16384 x 4096 the matrix units are busy 42 % of the time, the vector units 30, LDS 28 - but
 // the chain load, split, LDS, barrier, products of the two or three workgroups of a unit; splitting the next step in front of this
-// one's products, into a second buffer, gained nothing.
+// one's products, into a second buffer, gained nothing, nor did requests of eight rows of 128 bytes.
 // Against the fp32 matrix instruction (256 FLOP a cycle and unit) that was here, us, weights of bf16 values | of 32 bits:
 // 567 rows 9472 x 1024 122 -> 54 | 84, 1024 x 5120 91 -> 54 | 76, 1024 x 1024 22.5 -> 14.2 | 19.4; 2048 rows 16384 x 4096 2160 -> 869 (316
 // TFLOP/s of fp32 products) | 1402; 64 rows 1024 x 5120 33 -> 27 | 32, 9472 x 1024 24 -> 17 | 21; 1024 rows 4096 x 128 17 -> 14 | 16.5.
