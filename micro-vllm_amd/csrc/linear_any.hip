@@ -202,15 +202,31 @@ __global__ __launch_bounds__(256) void linear_any_bf16_big_kernel(
 // take three products, and the sum is the same bit for bit, for what is left out are zeros.
 // Sums, in every form here: a step is 32 neighbouring k, its products go from the smallest parts to hi hi; steps in ascending
 // order make a quarter of k, the quarters are added in ascending order.
-// What the parts cannot hold is done by the fp32 instruction (lf_by_f32: the same quarters): a sum that is not finite - an
-// infinite or NaN factor, or one that the rounding of hi makes infinite - and a sum below kLfTiny, where parts fall below the
-// smallest bf16 numbers.  Which form an output takes depends on its own row and column alone.
+// The parts are exact while their lowest bits are bf16 numbers: of a factor below about 2^-103 bits are lost, up to 2^-125 of it at
+// the worst.  Times another factor of at most kLfHuge that is 2^-95, under 2^-35 of a sum that is not below kLfTiny.  Every other
+// output is done by the fp32 instruction (lf_by_f32: the same quarters): where the largest magnitude of its row of x or of its row
+// of W is past kLfHuge (an infinite factor among them, or one that the rounding of hi makes infinite), where the sum is not finite,
+// below kLfTiny, or zero without a row of zeros.  NaN in a row is NaN in its sums either way.  Which form an output takes depends
+// on its own row and column alone; the largest magnitudes cost half an instruction a value on its way into LDS.
 constexpr int kLfBK = 32;
-constexpr float kLfTiny = 0x1p-60f;
+constexpr float kLfTiny = 0x1p-60f, kLfHuge = 0x1p30f;
 
-__device__ __forceinline__ bool lf_outside(float v) {   // (an exact zero is what rows of zeros give)
+__device__ __forceinline__ float lf_largest(float a, float b) { return __builtin_elementwise_maximum(a, b); }   // NaN stays
+__device__ __forceinline__ float lf_largest(const f32x4_t& v, float so_far) {   // magnitudes
+    // (assembly keeps it where it stands; moved about by the scheduler it holds the values longer: 16 to 30 registers, a workgroup a unit)
+    asm volatile("v_maximum3_f32 %0, |%1|, |%2|, %0\n\tv_maximum3_f32 %0, |%3|, |%4|, %0" : "+v"(so_far) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]));
+    return so_far;
+}
+__device__ __forceinline__ float lf_least(const f32x4_t& v, float so_far) {   // of magnitudes, NaN stays
+    auto least = [](float a, float b) { return __builtin_elementwise_minimum(a, b); };
+    return least(least(fabsf(v[2]), fabsf(v[3])), least(least(fabsf(v[0]), fabsf(v[1])), so_far));
+}
+// of a sum and the largest magnitudes of its two rows
+__device__ __forceinline__ bool lf_outside(float v, float xmax, float wmax) {
     const float a = fabsf(v);
-    return !(a >= kLfTiny && a < INFINITY) && v != 0.f;
+    const bool inside = a >= kLfTiny && a < INFINITY && xmax <= kLfHuge && wmax <= kLfHuge;
+    const bool zeros = v == 0.f && (xmax == 0.f || wmax == 0.f);
+    return !inside && !zeros && !(xmax != xmax || wmax != wmax);
 }
 
 // four values
@@ -322,6 +338,8 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
     y += blockIdx.z * zy;
     extern __shared__ __attribute__((aligned(16))) float lf_lds[];
     __shared__ int more_parts[DB ? 2 : 1][KG][2 * TN];   // the step in which these rows of W last had low bits
+    __shared__ float row_max[KG][RB * 16][4];   // largest magnitudes of the rows, x in front of W: of each staging lane
+    __shared__ int far_rows;                 // whether any of them is NaN or past kLfHuge
     int nb, mb;
     if (!lf_place(blockIdx.x, (N + BN - 1) / BN, (M + BM - 1) / BM, nb, mb)) return;
     const int m0 = mb * BM, n0 = nb * BN;
@@ -347,6 +365,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
     }
     uint4* buf = reinterpret_cast<uint4*>(lf_lds) + grp * (DB ? 2 : 1) * 3 * kPlane;
     if (threadIdx.x < (DB ? 2 : 1) * KG * 2 * TN) (&more_parts[0][0][0])[threadIdx.x] = -1;
+    if (threadIdx.x == 0) far_rows = 0;
     f32x4_t acc[TN][TM], sum[TN][TM];
     const int per = ((K + kLfBK - 1) / kLfBK + 3) / 4;   // k-steps of a quarter
     auto clear = [&] {
@@ -367,6 +386,9 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
     };
     clear();
     f32x4_t v[PF][U][2];
+    float largest[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) largest[u] = 0.f;
     const int first = grp * per * (4 / KG);   // this group's first step
 #pragma unroll
     for (int u = 0; u < U; ++u) p[u] += first * kLfBK + lq * 4;
@@ -403,6 +425,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             uint4* to = at + (u * 4 + wave) * 64 + put;
+            largest[u] = lf_largest(v[set][u][1], lf_largest(v[set][u][0], largest[u]));
             if (of_x(u) || __any(lf_low_bits(v[set][u][0], v[set][u][1]) != 0)) {   // uniform
                 const LfParts s = lf_split(v[set][u][0], v[set][u][1]);
                 to[0] = s.hi;
@@ -461,21 +484,21 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 #pragma unroll
                 for (int a = 0; a < TN; ++a) acc[a][b] = lf_mfma(wf[a], xf[b][part], acc[a][b]);
     };
+    constexpr int TURN = PF > (DB ? 2 : 1) ? PF : (DB ? 2 : 1);   // steps after which register sets and buffers are where they were
+    // Side by side the groups share the barriers, and a step past the end of k multiplies zeros.  One after the other the
+    // quarters end with k, at a whole turn.
+    const int steps = KG > 1 ? per * (4 / KG) : ((K + kLfBK - 1) / kLfBK + TURN - 1) / TURN * TURN;
     auto turn = [&](int set, int half, int step) {
         stage(set, half, step);
         __syncthreads();   // (DB: the other buffer was read a step ago, before this barrier by every wave)
         fetch(half);
         multiply(half, step);
-        if (!DB) __syncthreads();
+        if (!DB && (KG > 1 || step + 1 < steps)) __syncthreads();
     };
 #pragma unroll
     for (int i = 0; i < PF; ++i) request(i, i);
     __syncthreads();   // (more_parts)
-    constexpr int TURN = PF > (DB ? 2 : 1) ? PF : (DB ? 2 : 1);   // steps after which register sets and buffers are where they were
     static_assert(!DB || TURN % 2 == 0, "a turn ends on the buffer it began with");
-    // Side by side the groups share the barriers, and a step past the end of k multiplies zeros.  One after the other the
-    // quarters end with k, at a whole turn.
-    const int steps = KG > 1 ? per * (4 / KG) : ((K + kLfBK - 1) / kLfBK + TURN - 1) / TURN * TURN;
     int st = 0;
     for (; st + TURN <= steps; st += TURN)
 #pragma unroll
@@ -490,8 +513,15 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 #pragma unroll
             for (int b = 0; b < TM; ++b) acc[a][b] = sum[a][b];
     }
+    bool far = false;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        row_max[grp][(u * 4 + wave) * 16 + lr][lq] = largest[u];
+        far = far || !(largest[u] <= kLfHuge);
+    }
+    if (__any(far) && lane == 0) far_rows = 1;
+    __syncthreads();
     if (KG > 1) {   // group 0 adds up the groups
-        __syncthreads();
         constexpr int kAcc = TN * TM * 4;
         float* part = lf_lds + ((grp - 1) * 256 + tid) * (kAcc + 1);
         if (grp > 0) {
@@ -515,23 +545,6 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
         }
     }
     // acc[a][b][j] = C[n = n0 + 16 (TN wn + a) + 4 q + j][m = m0 + 16 (TM wm + b) + r]
-    bool outside = false;
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) outside = outside || lf_outside(acc[a][b][j]);
-    if (__any(outside)) {
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-            for (int b = 0; b < TM; ++b) {
-                const f32x4_t o = lf_by_f32<VEC>(x_row(m0 + (wm * TM + b) * 16 + r), w_row(n0 + (wn * TN + a) * 16 + r), q, K, per, 0, 4);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[a][b][j] = lf_outside(acc[a][b][j]) ? o[j] : acc[a][b][j];
-            }
-    }
 #pragma unroll
     for (int b = 0; b < TM; ++b) {
         const int m = m0 + (wm * TM + b) * 16 + r;
@@ -548,6 +561,46 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
                     if (n + j < N) dst[j] = acc[a][b][j];
             }
         }
+    }
+    // which of them are not the parts' (over what was stored)
+    float most = 0.f, least = INFINITY;
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b) {
+            most = lf_largest(acc[a][b], most);
+            least = lf_least(acc[a][b], least);
+        }
+    if (!far_rows && !__any(!(most < INFINITY && least >= kLfTiny))) return;
+    auto largest_at = [&](int row) {
+        float m = 0.f;
+#pragma unroll
+        for (int g = 0; g < KG; ++g)
+#pragma unroll
+            for (int l = 0; l < 4; ++l) m = lf_largest(m, row_max[g][row][l]);
+        return m;
+    };
+    uint64_t out = 0;   // a bit for j of a block
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int n = (wn * TN + a) * 16 + q * 4 + j;
+            const float w_max = largest_at(BM + n);
+#pragma unroll
+            for (int b = 0; b < TM; ++b) {
+                const int m = (wm * TM + b) * 16 + r;
+                if (m0 + m < M && n0 + n < N && lf_outside(acc[a][b][j], largest_at(m), w_max)) out |= 1ull << ((a * TM + b) * 4 + j);
+            }
+        }
+    for (int i = 0; i < TN * TM; ++i) {
+        const unsigned mine = (unsigned)(out >> (i * 4)) & 15u;
+        if (!__any(mine != 0)) continue;
+        const int m = m0 + (wm * TM + i % TM) * 16, n = n0 + (wn * TN + i / TM) * 16;
+        const f32x4_t o = lf_by_f32<VEC>(x_row(m + r), w_row(n + r), q, K, per, 0, 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (mine >> j & 1) y[(int64_t)(m + r) * ldy + n + q * 4 + j] = o[j];
     }
 }
 
@@ -598,6 +651,10 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
     unsigned char* xb = reinterpret_cast<unsigned char*>(xs);
     f32x4_t acc = {0, 0, 0, 0};
     f32x4_t wv[2][8], xv[2][MR / 2];
+    constexpr int kXMax = kSplitFirst ? MR / 2 : 1;
+    float w_max = 0.f, x_max[kXMax];   // largest magnitudes: of row r of W, of rows 2 i + half of x (sixteen rows: of row r)
+#pragma unroll
+    for (int i = 0; i < kXMax; ++i) x_max[i] = 0.f;
     auto request = [&](int set, int piece) {
         const int col = first + piece * kStreamK + kl, at = col < end ? col : 0;
 #pragma unroll
@@ -612,6 +669,7 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
         for (int i = 0; i < MR / 2; ++i) {
             const f32x4_t v = in ? xv[set][i] : zero;
             if (kSplitFirst) {   // four values: a half of what lane (row, k / 4 % 4) of the instruction takes of their step
+                x_max[i] = lf_largest(v, x_max[i]);
                 uint2 hi, mid, lo;
                 lf_split4(v, hi, mid, lo);
                 unsigned char* to = xb + (2 * i + half) * kStreamParts + (kl >> 5) * 64 + ((kl >> 2) & 3) * 16 + ((kl >> 4) & 1) * 8;
@@ -637,6 +695,7 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
             wv0[u] = *reinterpret_cast<const f32x4_t*>(wr);
             wv1[u] = *reinterpret_cast<const f32x4_t*>(wr + 16);
             low |= lf_low_bits(wv0[u], wv1[u]);
+            w_max = lf_largest(wv1[u], lf_largest(wv0[u], w_max));
         }
         auto parts_of_x = [&](int u) {
             LfParts p;
@@ -647,7 +706,9 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
                 p.lo = *reinterpret_cast<const uint4*>(xr + 2 * MR * kStreamParts);
             } else {
                 const float* xr = xs + r * kStreamPad + (at + u) * kLfBK + q * 4;
-                p = lf_split(*reinterpret_cast<const f32x4_t*>(xr), *reinterpret_cast<const f32x4_t*>(xr + 16));
+                const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(xr), x1 = *reinterpret_cast<const f32x4_t*>(xr + 16);
+                x_max[0] = lf_largest(x1, lf_largest(x0, x_max[0]));
+                p = lf_split(x0, x1);
             }
             return p;
         };
@@ -705,8 +766,20 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
     } else {
         turn(0, 0, false);
     }
+    __shared__ int far_rows[4];
+    {
+        float most = w_max;
+#pragma unroll
+        for (int i = 0; i < kXMax; ++i) most = lf_largest(most, x_max[i]);
+        const bool far = __any(!(most <= kLfHuge));
+        if (lane == 0) far_rows[wave] = far;
+    }
     __syncthreads();
     float(*part)[64][5] = reinterpret_cast<float(*)[64][5]>(ls_lds);
+    float(*row_max)[64][1 + kXMax] = reinterpret_cast<float(*)[64][1 + kXMax]>(ls_lds + 3 * 64 * 5);   // of each wave's lanes
+    row_max[wave][lane][0] = w_max;
+#pragma unroll
+    for (int i = 0; i < kXMax; ++i) row_max[wave][lane][1 + i] = x_max[i];
     if (wave > 0) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) part[wave - 1][lane][j] = acc[j];
@@ -718,16 +791,38 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[j] += part[g][lane][j];
     // acc[j] = C[n = n0 + 4 q + j][m = r]
-    if (__any(lf_outside(acc[0]) || lf_outside(acc[1]) || lf_outside(acc[2]) || lf_outside(acc[3]))) {
-        const f32x4_t o = lf_by_f32<true>(x + (int64_t)min(r, M - 1) * ldx, w + (int64_t)min(n0 + r, N - 1) * ldw, q, K, per,
-                                          4 * blockIdx.y, 4);
+    if (r < M) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = lf_outside(acc[j]) ? o[j] : acc[j];
+        for (int j = 0; j < 4; ++j)
+            if (n0 + q * 4 + j < N) y[(int64_t)r * ldy + n0 + q * 4 + j] = acc[j];
     }
-    if (r >= M) return;
+    // which of them are not the parts' (over what was stored)
+    if (!(far_rows[0] | far_rows[1] | far_rows[2] | far_rows[3]) &&
+        !__any(!(lf_largest(acc, 0.f) < INFINITY && lf_least(acc, INFINITY) >= kLfTiny))) return;
+    auto largest_of = [&](int first_lane, int step, int lanes, int i) {
+        float m = 0.f;
+        for (int g = 0; g < 4; ++g)
+            for (int l = 0; l < lanes; ++l) m = lf_largest(m, row_max[g][first_lane + l * step][i]);
+        return m;
+    };
+    const int row = min(r, MR - 1);
+    float xm = 0.f;
+    if (kSplitFirst) {
+#pragma unroll
+        for (int i = 0; i < kXMax; ++i)
+            if (i == row >> 1) xm = largest_of((row & 1) * 32, 1, 32, 1 + i);
+    } else {
+        xm = largest_of(row, 16, 4, 1);
+    }
+    unsigned out = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-        if (n0 + q * 4 + j < N) y[(int64_t)r * ldy + n0 + q * 4 + j] = acc[j];
+        if (r < M && n0 + q * 4 + j < N && lf_outside(acc[j], xm, largest_of(q * 4 + j, 16, 4, 0))) out |= 1u << j;
+    if (!__any(out != 0)) return;
+    const f32x4_t o = lf_by_f32<true>(x + (int64_t)min(r, M - 1) * ldx, w + (int64_t)min(n0 + r, N - 1) * ldw, q, K, per, 4 * blockIdx.y, 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (out >> j & 1) y[(int64_t)r * ldy + n0 + q * 4 + j] = o[j];
 }
 
 // Few output rows (decoding): a wave forms four neighbouring outputs of ONE row from 16-byte loads of the operand

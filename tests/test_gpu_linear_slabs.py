@@ -308,3 +308,37 @@ def test_fp32_values_beyond_the_parts(mv, m, n, k):
     assert bool((got[:, 5][torch.isfinite(odd).all(1)] == 0).all())
     if m > 3:
         assert got[3, 7].item() == big
+
+
+# fp32 factors far apart in size, whose sum is an ordinary number: of a small factor the parts lose bits, and a sum of zeros may be
+# parts that are all lost.  The shapes go to each form: streamed with 4, 8, 16 rows, whole and in slices, the six tiles (the last
+# four by scalar loads)
+@pytest.mark.parametrize("m,n,k", [(3, 1024, 1024), (3, 1024, 5120), (8, 528, 516), (16, 50, 516), (33, 9472, 256), (333, 9472, 68), (1000, 5000, 516),
+                                   (567, 9472, 1024), (2050, 9472, 1028), (20, 1000, 1022), (200, 16390, 514), (700, 5001, 514),
+                                   (2050, 9001, 1022)])
+def test_fp32_factors_of_any_size(mv, m, n, k):
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k, generator=g).to(DEV), (torch.randn(n, k, generator=g) / k ** 0.5).to(DEV)
+    plain = AnyLinear(w)(x)
+    odd, wo = x.clone(), w.clone()
+    odd[0] *= 2.0 ** -120                    # against row 1: 2^-50
+    wo[1] *= 2.0 ** 70
+    odd[1] *= 2.0 ** 66                      # against row 2: 2^-54
+    wo[2] = (wo[2] * 2.0 ** -120).bfloat16().float()
+    odd[2] = 0.0
+    odd[2, 5] = 2.0 ** -140                  # no part of it is a bf16 number
+    wo[3, 5], wo[4, 5] = 2.0 ** 100, 1.0     # 2^-40, 2^-140
+    wo[5, 0::2], wo[5, 1::2] = 2.0 ** 100, 0.0
+    odd[min(3, m - 1), 0::2] *= 2.0 ** -118   # beside ordinary factors
+    got = AnyLinear(wo)(odd)
+    want, size = odd.double() @ wo.double().t(), odd.double().abs() @ wo.double().abs().t()
+    held = size < 2.0 ** 127
+    # a fp32 rounding of each product and each sum, and the smallest fp32 number for each
+    off = lambda y: (y - want).abs() > k * 2.0 ** -24 * size + k * 2.0 ** -149   # noqa: E731
+    assert not bool((off(got.double()) & held).any())
+    assert not bool((off(AnyLinear(wo).slabs(odd, _take).double().sum(0)) & held).any())
+    assert got[2, 3].item() == 2.0 ** -40 and got[2, 4].item() == 2.0 ** -140
+    assert torch.equal(AnyLinear(wo)(odd[:3].contiguous())[held[:3]], got[:3][held[:3]])
+    assert torch.equal(got[4:, 6:], plain[4:, 6:])
