@@ -287,19 +287,41 @@ __device__ __forceinline__ f32x4_t lf_load4(const float* p, int col, int k) {
 }
 
 // Sixteen outputs by sixteen on the fp32 instruction, straight from memory: lane (r, q)'s row of x and of W, the shares
-// `share` .. `share + count` of `per` steps, added up in ascending order.
+// `share` .. `share + count` of `per` steps, added up in ascending order.  It is for few outputs: four steps are asked for together,
+// for one by one it is a chain of latencies, but every block reads its operands for itself.  us with one row of activations below
+// 2^-100 (a step at a time -> four; all on the fp32 instruction): 567 rows 9472 x 1024 138 -> 101 (114), 1024 x 5120 267 -> 185
+// (95), 2048 rows 16384 x 4096 1500 -> 1250 (2155).
 template <bool VEC>
-__device__ __attribute__((noinline)) f32x4_t lf_by_f32(const float* x, const float* w, int q, int K, int per, int share, int count) {
-    f32x4_t sum = {0, 0, 0, 0};
-    for (int s = 0; s < count; ++s) {
-        f32x4_t acc = {0, 0, 0, 0};
-        for (int k0 = (share + s) * per * kLfBK, n = 0; n < 2 * per; ++n, k0 += 16) {
-            const f32x4_t xf = lf_load4<VEC>(x, k0 + q * 4, K), wf = lf_load4<VEC>(w, k0 + q * 4, K);
+__device__ __forceinline__ f32x4_t lf_by_f32(const float* x, const float* w, int q, int K, int per, int share, int count) {
+    constexpr int kAhead = 4;   // steps asked for together
+    f32x4_t sum = {0, 0, 0, 0}, acc = {0, 0, 0, 0};
+    const int first = share * per, end = min(K, (share + count) * per * kLfBK);   // (zeros past it)
+    int left = per;   // steps of the share that acc holds a part of
+    for (int i = 0; i < count * per; i += kAhead) {
+        f32x4_t xf[kAhead][2], wf[kAhead][2];
+        const int k0 = (first + i) * kLfBK + q * 4;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[e], xf[e], acc, 0, 0, 0);
+        for (int n = 0; n < kAhead; ++n)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                xf[n][h] = lf_load4<VEC>(x, k0 + n * kLfBK + h * 16, end);
+                wf[n][h] = lf_load4<VEC>(w, k0 + n * kLfBK + h * 16, end);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < kAhead; ++n) {   // (no branch: it would take the loads with it)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[n][h][e], xf[n][h][e], acc, 0, 0, 0);
+            const bool whole = --left == 0;   // uniform
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                sum[j] = whole ? sum[j] + acc[j] : sum[j];
+                acc[j] = whole ? 0.f : acc[j];
+            }
+            left = whole ? per : left;
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sum[j] = s == 0 ? acc[j] : sum[j] + acc[j];
     }
     return sum;
 }
