@@ -354,6 +354,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
     constexpr int BM = 32 * TM, BN = 32 * TN, RB = 2 * (TM + TN), U = RB / 4;   // row blocks; of them per wave
     constexpr int kPlane = RB * 64;                                            // 16-byte pieces of a plane
     constexpr bool kFold = KG < 4;
+    static_assert(KG == 1 || KG == 2 || KG == 4, "a group has one quarter, two or all of them");
     static_assert(RB % 4 == 0 && (TM % 2 == 0 || (TM == 1 && TN == 1)), "a wave's row block is of x or of W");
     x += blockIdx.z * zx;
     w += blockIdx.z * zw;
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 #pragma unroll
     for (int i = 0; i < TURN - 1; ++i)
         if (st + i < steps) turn(i % PF, i & 1, st + i);
-    if (kFold) {
+    if (kFold && (KG == 1 || grp == 0)) {
         add_quarter();
 #pragma unroll
         for (int a = 0; a < TN; ++a)
@@ -543,27 +544,33 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
     }
     if (__any(far) && lane == 0) far_rows = 1;
     __syncthreads();
-    if (KG > 1) {   // group 0 adds up the groups
-        constexpr int kAcc = TN * TM * 4;
-        float* part = lf_lds + ((grp - 1) * 256 + tid) * (kAcc + 1);
+    if (KG > 1) {   // group 0 adds up the others' quarters, one by one
+        constexpr int kAcc = TN * TM * 4, kQuarters = 4 / KG;
+        float* part = lf_lds + ((grp - 1) * 256 + tid) * (kQuarters * kAcc + 1);
         if (grp > 0) {
 #pragma unroll
             for (int a = 0; a < TN; ++a)
 #pragma unroll
                 for (int b = 0; b < TM; ++b)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) part[(a * TM + b) * 4 + j] = acc[a][b][j];
+                    for (int j = 0; j < 4; ++j) {
+                        const int at = (a * TM + b) * 4 + j;
+                        if (kFold) part[at] = sum[a][b][j];
+                        part[(kQuarters - 1) * kAcc + at] = acc[a][b][j];
+                    }
         }
         __syncthreads();
         if (grp > 0) return;
         for (int g = 0; g < KG - 1; ++g) {
-            const float* o = lf_lds + (g * 256 + tid) * (kAcc + 1);
+            const float* o = lf_lds + (g * 256 + tid) * (kQuarters * kAcc + 1);
 #pragma unroll
-            for (int a = 0; a < TN; ++a)
+            for (int p = 0; p < kQuarters; ++p)
 #pragma unroll
-                for (int b = 0; b < TM; ++b)
+                for (int a = 0; a < TN; ++a)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[a][b][j] += o[(a * TM + b) * 4 + j];
+                    for (int b = 0; b < TM; ++b)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[a][b][j] += o[p * kAcc + (a * TM + b) * 4 + j];
         }
     }
     // acc[a][b][j] = C[n = n0 + 16 (TN wn + a) + 4 q + j][m = m0 + 16 (TM wm + b) + r]
@@ -928,7 +935,7 @@ static int launch_linear_f32_tiles(const float* x, int64_t ldx, const float* w, 
     const int64_t cols = (n + BN - 1) / BN, rows = (m + BM - 1) / BM, groups = (cols + 7) / 8 * 8 * rows;
     if (groups > 0x7fffffff) return MV_ERR_UNSUPPORTED;
     size_t lds = (size_t)KG * (DB ? 2 : 1) * 3 * (BM + BN) * kLfBK * 2;
-    const size_t meet = (size_t)(KG - 1) * 256 * (TM * TN * 4 + 1) * 4;
+    const size_t meet = (size_t)(KG - 1) * 256 * (4 / KG * TM * TN * 4 + 1) * 4;
     if (meet > lds) lds = meet;
     const bool vec = k % 4 == 0 && aligned16(x) && ldx % 4 == 0 && zx % 4 == 0 && aligned16(w) && ldw % 4 == 0 && zw % 4 == 0;
     static LdsOptIn done[2];

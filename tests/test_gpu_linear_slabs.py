@@ -342,3 +342,16 @@ def test_fp32_factors_of_any_size(mv, m, n, k):
     assert got[2, 3].item() == 2.0 ** -40 and got[2, 4].item() == 2.0 ** -140
     assert torch.equal(AnyLinear(wo)(odd[:3].contiguous())[held[:3]], got[:3][held[:3]])
     assert torch.equal(got[4:, 6:], plain[4:, 6:])
+
+
+# the sums of a row are those of four quarters of k in ascending order in every form: streamed, and the six tiles
+@pytest.mark.parametrize("many,n,k", [(20, 1000, 1022), (33, 9472, 256), (567, 1024, 640), (333, 9472, 68), (700, 3000, 250),
+                                      (1100, 4112, 1000), (1000, 5000, 516), (567, 9472, 1024), (2050, 9472, 1028)])
+def test_fp32_rows_do_not_depend_on_the_others(mv, many, n, k):
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(many + n + k)
+    x, lin = torch.randn(many, k, generator=g).to(DEV), AnyLinear((torch.randn(n, k, generator=g) / k ** 0.5).to(DEV))
+    want = lin(x)
+    for rows in (1, 5, 9, 17, 40, 130):
+        assert torch.equal(lin(x[:rows]), want[:rows])
