@@ -229,24 +229,34 @@ __device__ __forceinline__ bool lf_outside(float v, float xmax, float wmax) {
     return !inside && !zeros && !(xmax != xmax || wmax != wmax);
 }
 
-// four values
+// Four values.  A part is subtracted by v_dot2_f32_bf16, (-1, 0) or (0, -1) times the packed pair, where that is faster than to
+// unpack it (streamed 16 rows 16384 x 4096 52.5 -> 50 us, 32 x 32 tiles 33 rows 1024 x 5120 28.8 -> 26.5; the wider tiles 0 to 3 % slower): every
+// result is exact either way.
+template <bool DOT>
 __device__ __forceinline__ void lf_split4(const f32x4_t& v, uint2& hi, uint2& mid, uint2& lo) {
-    hi = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-    float a = v[0] - bf16_lo(hi.x), b = v[1] - bf16_hi(hi.x), c = v[2] - bf16_lo(hi.y), d = v[3] - bf16_hi(hi.y);
-    mid = make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
-    a -= bf16_lo(mid.x);
-    b -= bf16_hi(mid.x);
-    c -= bf16_lo(mid.y);
-    d -= bf16_hi(mid.y);
-    lo = make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
+    uint32_t minus_lo = 0x0000bf80u, minus_hi = 0xbf800000u;
+    asm("" : "+s"(minus_lo), "+s"(minus_hi));   // (in registers: as an inline constant the second is another pair)
+    auto less = [&](const f32x4_t& x, const uint2& p) {
+        if constexpr (DOT)
+            return f32x4_t{dot2_bf16(p.x, minus_lo, x[0]), dot2_bf16(p.x, minus_hi, x[1]), dot2_bf16(p.y, minus_lo, x[2]),
+                           dot2_bf16(p.y, minus_hi, x[3])};
+        else
+            return f32x4_t{x[0] - bf16_lo(p.x), x[1] - bf16_hi(p.x), x[2] - bf16_lo(p.y), x[3] - bf16_hi(p.y)};
+    };
+    auto pack = [](const f32x4_t& x) { return make_uint2(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])); };
+    hi = pack(v);
+    const f32x4_t rest = less(v, hi);
+    mid = pack(rest);
+    lo = pack(less(rest, mid));
 }
 struct LfParts {
     uint4 hi, mid, lo;   // eight values, two in each word
 };
+template <bool DOT>
 __device__ __forceinline__ LfParts lf_split(const f32x4_t& v0, const f32x4_t& v1) {
     uint2 h[2], m[2], l[2];
-    lf_split4(v0, h[0], m[0], l[0]);
-    lf_split4(v1, h[1], m[1], l[1]);
+    lf_split4<DOT>(v0, h[0], m[0], l[0]);
+    lf_split4<DOT>(v1, h[1], m[1], l[1]);
     return {make_uint4(h[0].x, h[0].y, h[1].x, h[1].y), make_uint4(m[0].x, m[0].y, m[1].x, m[1].y),
             make_uint4(l[0].x, l[0].y, l[1].x, l[1].y)};
 }
@@ -343,9 +353,10 @@ __device__ __forceinline__ bool lf_place(int id, int cols, int rows, int& col, i
 // What bounds it: no one unit - at 2048 rows 16384 x 4096 the matrix units are busy 42 % of the time, the vector units 30, LDS 28 - but
 // the chain load, split, LDS, barrier, products of the two or three workgroups of a unit; splitting the next step in front of this
 // one's products, into a second buffer, gained nothing, nor did requests of eight rows of 128 bytes.
-// Against the fp32 matrix instruction (256 FLOP a cycle and unit) that was here, us, weights of bf16 values | of 32 bits:
-// 567 rows 9472 x 1024 122 -> 54 | 84, 1024 x 5120 91 -> 54 | 76, 1024 x 1024 22.5 -> 14.2 | 19.4; 2048 rows 16384 x 4096 2160 -> 869 (316
-// TFLOP/s of fp32 products) | 1402; 64 rows 1024 x 5120 33 -> 27 | 32, 9472 x 1024 24 -> 17 | 21; 1024 rows 4096 x 128 17 -> 14 | 16.5.
+// Against the fp32 matrix instruction (256 FLOP a cycle and unit) that was here, us, weights of bf16 values | of 32 bits, out of memory:
+// 567 rows 9472 x 1024 114 -> 55 | 85, 1024 x 5120 95 -> 61 | 81, 1024 x 1024 22.5 -> 14.2 | 19.4; 2048 rows 16384 x 4096 2155 -> 905 (304
+// TFLOP/s of fp32 products) | 1460; 33 rows 1024 x 5120 37 -> 26.5 | 33.6; 64 rows 9472 x 1024 25.4 -> 18.4 | 22.2; 1024 rows 4096 x 128 17.3 ->
+// 15.1 | 17.6.  9 to 16 rows of 65536 x 64 take 12.9 | 14.0, 10.1 on it.
 // Error against 64 bits (2-norm): 1024 x 5120 6.4e-7 -> 3.9e-7 | 5.6e-7, 9472 x 1024 2.9e-7 -> 1.7e-7 | 2.3e-7.
 template <int TM, int TN, int KG, int PF, bool DB, bool VEC>
 __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kernel(
@@ -450,7 +461,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
             uint4* to = at + (u * 4 + wave) * 64 + put;
             largest[u] = lf_largest(v[set][u][1], lf_largest(v[set][u][0], largest[u]));
             if (of_x(u) || __any(lf_low_bits(v[set][u][0], v[set][u][1]) != 0)) {   // uniform
-                const LfParts s = lf_split(v[set][u][0], v[set][u][1]);
+                const LfParts s = lf_split<TM == 1>(v[set][u][0], v[set][u][1]);
                 to[0] = s.hi;
                 to[kPlane] = s.mid;
                 to[2 * kPlane] = s.lo;
@@ -641,21 +652,31 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 // the wave's own part of LDS (rows 528 bytes apart: the sixteen rows of a read are on different banks; no barrier, a wave's LDS
 // operations are in order).  Two such pieces are in flight, 16 KB a wave.
 // Measured against operands read straight into that layout, 64 bytes of sixteen rows to a request (outputs x k, 3 rows, us):
-// 32000 x 1024 39.8 -> 22 (5.9 TB/s), 9472 x 1024 16.1 -> 10, 16384 x 4096 61.1 -> 43.5 (6.2 TB/s), 1024 x 5120 20.6 -> 12.3 (in four
-// slices 10.8 -> 7.3), 65536 x 64 70 -> 18; 16 rows 1024 x 5120 28.7 -> 16.3, 1280 x 1024 8.4 -> 6.6.  The parts take the fp32
-// instruction's time where weights are bf16 values; where they are not, the second split costs 3 to 10 % (16384 x 4096 46).
-// From nine rows on the tiles are ahead where the output is wide and k is short (16 rows, 65536 x 64: 10.3 us against 25.6, 32000 x 256 15.4
-// against 15.6; 32000 x 512 28.6 against 18.9, 16384 x 4096 74 against 49), from 17 on everywhere.
-constexpr int kStreamRows = 8, kStreamRowsMore = 16, kStreamNarrow = 8192, kStreamLongK = 512, kStreamSlice = 8;
+// 32000 x 1024 39.8 -> 22.8 (5.7 TB/s), 9472 x 1024 16.1 -> 10.1, 16384 x 4096 61.1 -> 43.3 (6.2 TB/s), 1024 x 5120 20.6 -> 12.3 (in four
+// slices 10.8 -> 7.3), 65536 x 64 70 -> 16; 16 rows 1024 x 5120 28.7 -> 17.7, 1280 x 1024 8.4 -> 6.6.
+// Against the fp32 instruction in this same form, us, it -> weights of bf16 values | of 32 bits.  Up to 8 rows: 32000 x 1024 22.9 ->
+// 22.8 | 23.8, 16384 x 4096 44.2 -> 43.3 | 46.6 (8 rows 45 -> 44.4 | 48), 4096 x 2048 9.0 -> 8.5 | 9.8; few workgroups, each a chain of its own split:
+// 1024 x 5120 12.6 -> 12.3 | 15.3 (8 rows 13.7 -> 13.4 | 16.1), 512 x 8192 17.4 -> 17.3 | 21.9.  16 rows split x behind LDS as well:
+// 16384 x 4096 49.6 -> 50.1 | 56, 1024 x 5120 16.4 -> 17.7 | 20.7.  Rows of bf16 values are what a checkpoint in that type gives.
+// Four steps' operands are read out of LDS before the first is used (1024 x 5120 13.8 -> 12.3 | 16.8 -> 15.3); one at a time leaves registers for a third
+// workgroup on a unit, which is ahead where a wave has two pieces or fewer (3 rows 32000 x 1024 22.8 against 23.5, 65536 x 256
+// 18.6 against 23.2; 32000 x 2048 42.0 against 40.8).
+// From nine rows on the tiles are ahead where the output is wide and k is short (16 rows, 65536 x 256: 18.9 us against 25, 32000 x 448
+// 16.3 against 22.5; 32000 x 512 28.6 against 18.9, 16384 x 4096 74 against 49), from 17 on everywhere; at k of up to 256 and
+// 16384 outputs from five (8 rows 65536 x 256 19 against 25, 32000 x 256 10.4 against 13.7, 16384 x 256 7.8 against 8.3, 9472 x 256 7.2 against
+// 6.8; 32000 x 448 15.8 each).
+constexpr int kStreamRowsLess = 4, kStreamRows = 8, kStreamRowsMore = 16, kStreamNarrow = 8192, kStreamWide = 16384;
+constexpr int kStreamShortK = 256, kStreamLongK = 512;
+constexpr int kStreamSlice = 8, kStreamOneStep = 1024;   // (a slice's k up to which steps go one by one)
 constexpr int kStreamK = 128, kStreamPad = kStreamK + 4;   // k of a piece, floats of a row in LDS
 constexpr int kStreamParts = kStreamK * 2 + 16;            // bytes of a row's parts in LDS
 // A wave's rows of x lie in LDS split (a lane of the instruction whose column is a row past MR reads a row again, so split behind
 // LDS the work would be done 16 / MR times), up to eight of them; sixteen as they are.
 constexpr int stream_x_bytes(int mr) { return mr == 16 ? mr * kStreamPad * 4 : 3 * mr * kStreamParts; }
 
-// MR: rows of x that are read, 4, 8 or 16
-template <int MR>
-__global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel(const float* __restrict__ x, int64_t ldx,
+// MR: rows of x that are read, 4, 8 or 16; STEPS of 32 k whose operands are read out of LDS together, for 4 rows also one
+template <int MR, int STEPS>
+__global__ __launch_bounds__(256, STEPS == 1 ? 3 : 2) void linear_stream_f32_kernel(const float* __restrict__ x, int64_t ldx,
                                                                 const float* __restrict__ w, int64_t ldw,
                                                                 float* __restrict__ y, int64_t ldy, int M, int N, int K) {
     // blockIdx.y: a slice of k of its own, [slice][M][N] in y (ldy = N); the wave's share is a quarter of the slice
@@ -700,7 +721,7 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
             if (kSplitFirst) {   // four values: a half of what lane (row, k / 4 % 4) of the instruction takes of their step
                 x_max[i] = lf_largest(v, x_max[i]);
                 uint2 hi, mid, lo;
-                lf_split4(v, hi, mid, lo);
+                lf_split4<true>(v, hi, mid, lo);
                 unsigned char* to = xb + (2 * i + half) * kStreamParts + (kl >> 5) * 64 + ((kl >> 2) & 3) * 16 + ((kl >> 4) & 1) * 8;
                 *reinterpret_cast<uint2*>(to) = hi;
                 *reinterpret_cast<uint2*>(to + MR * kStreamParts) = mid;
@@ -723,8 +744,6 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
             const float* wr = ws + r * kStreamPad + (at + u) * kLfBK + q * 4;
             wv0[u] = *reinterpret_cast<const f32x4_t*>(wr);
             wv1[u] = *reinterpret_cast<const f32x4_t*>(wr + 16);
-            low |= lf_low_bits(wv0[u], wv1[u]);
-            w_max = lf_largest(wv1[u], lf_largest(wv0[u], w_max));
         }
         auto parts_of_x = [&](int u) {
             LfParts p;
@@ -737,16 +756,25 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
                 const float* xr = xs + r * kStreamPad + (at + u) * kLfBK + q * 4;
                 const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(xr), x1 = *reinterpret_cast<const f32x4_t*>(xr + 16);
                 x_max[0] = lf_largest(x1, lf_largest(x0, x_max[0]));
-                p = lf_split(x0, x1);
+                p = lf_split<true>(x0, x1);
             }
             return p;
         };
-        LfParts first;
-        if (C == 1) first = parts_of_x(0);   // (its way out of LDS beside W's; of four steps they do not all fit)
+        LfParts xs_of[C];
+        if (kSplitFirst) {
+#pragma unroll
+            for (int u = 0; u < C; ++u) xs_of[u] = parts_of_x(u);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // (all asked for before the first is used)
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            low |= lf_low_bits(wv0[u], wv1[u]);
+            w_max = lf_largest(wv1[u], lf_largest(wv0[u], w_max));
+        }
         if (__any(low != 0)) {   // uniform
 #pragma unroll
             for (int u = 0; u < C; ++u) {
-                const LfParts xp = C == 1 ? first : parts_of_x(u), wp = lf_split(wv0[u], wv1[u]);
+                const LfParts xp = kSplitFirst ? xs_of[u] : parts_of_x(u), wp = lf_split<true>(wv0[u], wv1[u]);
                 acc = lf_mfma(wp.lo, xp.hi, acc);
                 acc = lf_mfma(wp.mid, xp.mid, acc);
                 acc = lf_mfma(wp.mid, xp.hi, acc);
@@ -757,7 +785,7 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
         } else {
 #pragma unroll
             for (int u = 0; u < C; ++u) {
-                const LfParts xp = C == 1 ? first : parts_of_x(u);
+                const LfParts xp = kSplitFirst ? xs_of[u] : parts_of_x(u);
                 const uint4 hi = lf_upper(wv0[u], wv1[u]);
                 acc = lf_mfma(hi, xp.lo, acc);
                 acc = lf_mfma(hi, xp.mid, acc);
@@ -765,11 +793,10 @@ __global__ __launch_bounds__(256, MR == 4 ? 3 : 2) void linear_stream_f32_kernel
             }
         }
     };
-    constexpr int kSteps = MR == 4 ? 1 : 4;   // (more at a time take more registers than three of its workgroups on a unit have)
     auto multiply = [&](int piece) {
 #pragma unroll
-        for (int at = 0; at < kStreamK / kLfBK; at += kSteps)
-            if (per - piece * (kStreamK / kLfBK) > at) multiply_steps(std::integral_constant<int, kSteps>(), at);   // uniform
+        for (int at = 0; at < kStreamK / kLfBK; at += STEPS)
+            if (per - piece * (kStreamK / kLfBK) > at) multiply_steps(std::integral_constant<int, STEPS>(), at);   // uniform
     };
     auto settle = [] {   // between a wave's own writes and reads of LDS: an order for the compiler, no instruction
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -949,16 +976,20 @@ static int launch_linear_f32_tiles(const float* x, int64_t ldx, const float* w, 
 // whether the rows are few enough for the streamed form
 static bool streams_f32(int m, int n, int k) {
     using namespace mv;
-    return m <= (n < kStreamNarrow || k >= kStreamLongK ? kStreamRowsMore : kStreamRows);
+    if (n < kStreamNarrow || k >= kStreamLongK) return m <= kStreamRowsMore;
+    return m <= (n < kStreamWide || k > kStreamShortK ? kStreamRows : kStreamRowsLess);
 }
 
 static int launch_linear_stream(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
                                 int k, int slices, hipStream_t s) {
     using namespace mv;
-    const int form = m <= 4 ? 0 : m <= 8 ? 1 : 2;
-    const size_t lds = (size_t)4 * (16 * kStreamPad * 4 + stream_x_bytes(4 << form));
-    static LdsOptIn done[3];
-    const auto kernel = form == 0 ? linear_stream_f32_kernel<4> : form == 1 ? linear_stream_f32_kernel<8> : linear_stream_f32_kernel<16>;
+    const int form = m > 8 ? 3 : m > 4 ? 2 : k / slices > kStreamOneStep ? 1 : 0;
+    const size_t lds = (size_t)4 * (16 * kStreamPad * 4 + stream_x_bytes(form == 3 ? 16 : form == 2 ? 8 : 4));
+    static LdsOptIn done[4];
+    const auto kernel = form == 0   ? linear_stream_f32_kernel<4, 1>
+                        : form == 1 ? linear_stream_f32_kernel<4, 4>
+                        : form == 2 ? linear_stream_f32_kernel<8, 4>
+                                    : linear_stream_f32_kernel<16, 4>;
     if (const int rc = ensure_dynamic_lds((const void*)kernel, lds, done[form])) return rc;
     hipLaunchKernelGGL(kernel, dim3((n + 15) / 16, slices), dim3(256), lds, s, x, ldx, w, ldw, y, ldy, m, n, k);
     return check_launch();

@@ -355,3 +355,30 @@ def test_fp32_rows_do_not_depend_on_the_others(mv, many, n, k):
     want = lin(x)
     for rows in (1, 5, 9, 17, 40, 130):
         assert torch.equal(lin(x[:rows]), want[:rows])
+
+
+# fp32 weights that are bf16 values but in single steps of 32 k: which rows take six products and which three changes from step to
+# step, from one block of sixteen rows to the next, and with how many steps a form looks at together.  A row alone (streamed, a step
+# or four at a time, both sides of k = 1024), 5, 8, 9 and 16 rows (streamed, and tiles where k is short and n wide) and many (tiles of every
+# size that goes with k) are the same bits
+@pytest.mark.parametrize("n,k,many", [(48, 1024, 40), (1040, 1028, 300), (1040, 1030, 300), (8208, 256, 70), (8208, 260, 600), (16400, 256, 70), (9472, 544, 600),
+                                      (4112, 1000, 1100)])
+def test_low_bits_in_some_steps_only(mv, n, k, many):
+    from micro_vllm_amd.kernel.ragged_ops import AnyLinear
+
+    g = torch.Generator().manual_seed(n + k)
+    x = torch.randn(many, k, generator=g).to(DEV)
+    full = (torch.randn(n, k, generator=g) / k ** 0.5).to(DEV)
+    w, step, block = full.bfloat16().float(), torch.arange(k, device=DEV) // 32, torch.arange(n, device=DEV) // 16
+    last = (k - 1) // 32
+    odd = ((block[:, None] % 5 == 1) & (step % 2 == 1)) | ((block[:, None] % 5 == 2) & (step == 0)) | \
+          ((block[:, None] % 5 == 3) & (step == last)) | ((block[:, None] % 5 == 4) & (step % 7 == 3))
+    odd &= torch.arange(n, device=DEV)[:, None] % 16 == 11       # one row of a block
+    w = torch.where(odd, full, w)
+    lin = AnyLinear(w)
+    want = lin(x)
+    err = (want.double() - x.double() @ w.double().t()).abs()
+    # a rounding of each product and each sum
+    assert bool((err <= k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())).all())
+    for rows in (1, 4, 5, 8, 9, 16, 33):
+        assert torch.equal(lin(x[:rows]), want[:rows])
