@@ -237,6 +237,8 @@ int mv_linear_act(const void* x, int64_t ldx, const void* w_tiles, void* y, int6
  * with tiles of 192 and of 224 columns, where those fill the CUs in fewer or fuller rounds
  * (MVLLM_PREFILL_WIDE_STRIPS=12/14/16 forces the width, in 16-column strips). */
 int mv_gemm_prefill_form(int m, int n, int k);
+/* 16-column strips of a workgroup where a call of up to 64 rows adds its k-slices within the workgroup, else 0 (for tests). */
+int mv_gemm_prefill_group(int m, int n, int k);
 /* Overrides for tests and A/B runs inside one process (no counterpart in the reference): cut = 0 / 1
  * switches the cutting of left-over tiles off / on, strips = 12 / 14 / 16 forces the tile width, for
  * every call that follows; -1 returns a choice to the environment (MVLLM_PREFILL_CUT,

@@ -146,6 +146,7 @@ bool wgemm_finalize_norm_takes(int n);
 // wgemm.hip: a projection of up to 64 rows whose sums are those of `ks` slices of k added in order.  `strips`: n-tiles of a
 // wave of the 64-row tiles that would take it otherwise (0: larger ones would)
 bool wgemm_ordered_takes(int m, int nt, int kt, int ks, int strips);
+int wgemm_ordered_group(int m, int nt, int kt, int ks);   // strips of a workgroup
 int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const void* bias, const void* residual,
                          int64_t ld_res, void* y, int64_t ldy, int m, int n, int k, int ks, int flags, PostNorm* norm,
                          hipStream_t s);

@@ -993,6 +993,11 @@ static PrefillPlan prefill_plan(int m, int n, int kt) {
     if (narrow_ks == 1 && (forced == 1 || 2 * tiles >= cus)) return {true, 1, wide_tile_strips(m, n, kt)};
     return {false, narrow_ks, 16};
 }
+// Tiles of 256 rows for 64 or fewer: the 64-row tiles take the same slices where each has a compute unit to itself (28672 x 4096 in two
+// slices, 8 rows 63.6 -> 48.5 us, 64 rows 67.0 -> 54.5; same sums, so not where the wide form would cut left-over tiles).
+static bool few_rows_leave_wide(const PrefillPlan& plan, int m, int nt, int kt) {
+    return m <= 64 && tile64_strips(m, nt, plan.ks) && !(plan.ks == 1 && wide_cuts(1, (nt + plan.strips - 1) / plan.strips, kt));
+}
 }  // namespace mv
 
 // Experiments only (tools/ab_gemm_prefill.py): whether left-over tiles are cut (0 / 1) and the tile width
@@ -1018,6 +1023,17 @@ extern "C" int mv_gemm_prefill_form(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0 || (n % 16) != 0 || (k % 64) != 0) return 0;
     const PrefillPlan plan = prefill_plan(m, n, k / 32);
     return !plan.wide ? 0 : plan.ks > 1 || plan.strips == 16 ? 1 : plan.strips == 12 ? 2 : 3;
+}
+
+// strips of a workgroup where the slices are added within it, 0 in any other form (given a workspace and rows less than 2^28 apart)
+extern "C" int mv_gemm_prefill_group(int m, int n, int k) {
+    using namespace mv;
+    if (m <= 0 || n <= 0 || k <= 0 || (n % 16) != 0 || (k % 64) != 0) return 0;
+    const int nt = n / 16, kt = k / 32;
+    const PrefillPlan plan = prefill_plan(m, n, kt);
+    if ((plan.wide && !few_rows_leave_wide(plan, m, nt, kt)) || !wgemm_ordered_takes(m, nt, kt, plan.ks, tile64_strips(m, nt, plan.ks)))
+        return 0;
+    return wgemm_ordered_group(m, nt, kt, plan.ks);
 }
 
 extern "C" int mv_gemm_prefill(const void* x, int64_t ldx, const void* w_tiles, const void* bias,
@@ -1145,11 +1161,7 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
                            ? (void*)((char*)workspace + kWCountBytes) : nullptr;
     const size_t data_bytes = data ? workspace_bytes - kWCountBytes : 0;
     bool wide = plan.wide;
-    // Tiles of 256 rows for 64 or fewer: the 64-row tiles take the same slices where each has a compute unit to itself (28672 x 4096 in two
-    // slices, 8 rows 63.6 -> 48.5 us, 64 rows 67.0 -> 54.5; same sums, so not where the wide form would cut left-over tiles).
-    if (wide && m <= 64 && tile64_strips(m, a.nt, a.ksplit) &&
-        !(a.ksplit == 1 && wide_cuts(1, (a.nt + plan.strips - 1) / plan.strips, a.kt)))
-        wide = false;
+    if (wide && few_rows_leave_wide(plan, m, a.nt, a.kt)) wide = false;
     if (a.ksplit > 1) {
         const size_t need = (size_t)a.ksplit * m * n * sizeof(float);
         if (keep_slices) {
@@ -1164,7 +1176,7 @@ int mv::gemm_prefill_run(const void* x, int64_t ldx, const void* w_tiles, const 
     // Up to 64 rows a tile of 128 is mostly padding, and its slices are written out and added up by a second launch.  The
     // single-token projections' kernel walks the same slices one to a wave and adds them in the workgroup, same sums in
     // the same order (the rule and what it measured: wgemm_ordered_takes).
-    if (!wide && !keep_slices && !act.kind && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit, tile64_strips(m, a.nt, a.ksplit)))
+    if (!wide && !keep_slices && !act.kind && ldx < (1 << 28) && wgemm_ordered_takes(m, a.nt, a.kt, a.ksplit, tile64_strips(m, a.nt, a.ksplit)))
         return launch_wgemm_ordered(x, ldx, w_tiles, bias, residual, ld_res, y, ldy, m, n, k, a.ksplit, flags, norm,
                                     (hipStream_t)stream);
     auto reduce = [&] {

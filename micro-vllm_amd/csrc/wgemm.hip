@@ -11,11 +11,15 @@
 //    The tiles of one 16-row strip are contiguous along K.
 //  * A unit of work is (strip nt, k-slice ks).  A 512-thread workgroup takes whole
 //    units; its 8 waves interleave over the unit's tiles (wave w takes tile kt0+w,
-//    kt0+w+8, ...) so the workgroup reads one contiguous stream.  Partial sums of
-//    the 8 waves meet in LDS in a fixed order: results are run-to-run identical.
+//    kt0+w+8, ..., or pairs of tiles kt0+2w, kt0+2w+1, kt0+2w+16, ...) so the workgroup
+//    reads one contiguous stream.  Partial sums of the 8 waves meet in LDS in a fixed
+//    order: results are run-to-run identical.  Which tiles a wave adds up goes with the
+//    form, so a row's last bits may change with the number of rows.  (Whole slices of k a
+//    wave, for prompts: wgemm_mfma_kernel with KS > 0, four waves where there are four.)
 //  * M <= 4: dot-product form (v_dot2c_f32_bf16), x staged once per workgroup in
 //    LDS.  M > 4, or x too long for that: v_mfma_f32_16x16x32_bf16 with the x fragment (B operand) loaded
-//    from L2 in the same lane layout.  Both read the same weight tiles.
+//    from L2, in the same lane layout or by lines of two k-tiles that are exchanged between lanes behind
+//    the load.  Both read the same weight tiles.
 //  * ksplit > 1 (picked when strips alone cannot balance the CUs) writes fp32
 //    slabs; a small second kernel adds them in slab order and applies the epilogue.
 //
@@ -467,7 +471,9 @@ __global__ __launch_bounds__(GW * kWave) void wgemm_dot_kernel(GemmArgs a) {
 //
 // KS = 0: the waves interleave over the unit's pairs of k-tiles.  KS = 4, 8, 16: k in KS whole slices, each added up by one wave
 // and the slices in order - the sums of a prefill projection cut into KS slices (gemm_prefill.hip), bit for bit, without
-// its slabs and their reduction launch.  With four slices a workgroup has four waves, each with four stages in flight (a wave a
+// its slabs and their reduction launch.  Here every request is a scalar address and a 32-bit offset, three offsets for x and one for the
+// weights: with a pair of registers for each the groups of four strips spilled from 49 rows on (<8, 4, 8> 20 registers, <7, 4, 8> 6,
+// <8, 2, 16> 2; none so), 64 rows 16384 x 14336 102 -> 86 us, 12304 x 4096 30.9 -> 26.8, 56 rows 14336 x 14336 83 -> 77.  With four slices a workgroup has four waves, each with four stages in flight (a wave a
 // SIMD has the registers; two halves of eight waves on strips of their own read x twice: 37 rows 11264 x 2048 14.0 us, 12.2 so, 8192 x
 // 1024 7.7 -> 7.0, 4096 x 1024 6.9 -> 5.3); with sixteen a wave takes two slices one after the other.  Three or four stages elsewhere cost
 // 0 to 35 %: a wave has few stages, and those past the end are asked for as well.
@@ -484,20 +490,23 @@ __global__ __launch_bounds__(KS == 4 ? 4 * kWave : kGT) void wgemm_mfma_kernel(G
     static_assert(PAIR || KS == 0, "slices go by pairs");
     constexpr int kTurns = KS == 16 ? 2 : 1;
     constexpr int kSlots = KS == 0 ? kGW : KS;   // accumulator sets that meet in LDS
-    // cross-wave reduction buffer [kGW][SG][MB][64 lanes][4]: 8 KiB per (strip, row block) pair,
-    // up to 128 KiB (dynamic: past the 64 KiB a static array may have)
+    // cross-wave reduction buffer [kSlots][SG][MB][64 lanes][4]: 4 KiB per (strip, row block) pair with four slices, 8, or 16 with
+    // sixteen, up to 128 KiB (dynamic: past the 64 KiB a static array may have)
     extern __shared__ __attribute__((aligned(16))) float red[];
 
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
     const bool odd = r & 1;
-
     // this lane's x rows, clamped into [0, M), at its 16 bytes of the first of two k-tiles; and which of the two it takes
     const uint16_t* xrow[HB];
+    const int second = odd ? 32 : 0;
 #pragma unroll
     for (int h = 0; h < HB; ++h) xrow[h] = a.x + (int64_t)min(PAIR ? h * 8 + (r >> 1) : h * 8 + r, a.m - 1) * a.ldx + q * 8;
-    const int second = odd ? 32 : 0;
+    // KS > 0: bytes behind the scalar address of a block's first row - of the blocks that are whole, even and odd, and of the last
+    const uint32_t row_bytes = 2 * (uint32_t)a.ldx, mine = 2 * (q * 8 + second), other = 2 * (q * 8 + 32 - second);
+    const uint32_t x_even = (r >> 1) * row_bytes + mine, x_odd = (r >> 1) * row_bytes + other;
+    const uint32_t x_last = min(r >> 1, a.m - 1 - (HB - 1) * 8) * row_bytes + (HB & 1 ? mine : other);
 
     for (int u = blockIdx.x; u < a.nunits; u += gridDim.x) {
         const int g = KS ? u : u / a.ksplit, ks = KS ? 0 : u - g * a.ksplit;
@@ -517,7 +526,7 @@ __global__ __launch_bounds__(KS == 4 ? 4 * kWave : kGT) void wgemm_mfma_kernel(G
         const uint4* wbase[SG];
 #pragma unroll
         for (int sI = 0; sI < SG; ++sI)
-            wbase[sI] = a.w + ((int64_t)min(strip0 + sI, a.nt - 1) * a.kt) * 64 + lane;
+            wbase[sI] = a.w + ((int64_t)min(strip0 + sI, a.nt - 1) * a.kt) * 64;   // uniform, in scalar registers
 
         f32x4_t acc[SG][MB];
 #pragma unroll
@@ -531,16 +540,26 @@ __global__ __launch_bounds__(KS == 4 ? 4 * kWave : kGT) void wgemm_mfma_kernel(G
             const int t = ktw + min(c, last) * kStep;
             const bool whole = t + kNext < kt1;   // uniform: half a stage at the end is asked for twice
             if constexpr (PAIR) {
-                const int even_block = t * 32 + (whole ? second : 0), odd_block = t * 32 + (whole ? 32 - second : 0);
+                if constexpr (KS > 0) {
+                    const uint32_t even_back = whole ? 0 : 2 * second, odd_back = whole ? 0 : 2 * (32 - second);
+                    const uint32_t e = x_even - even_back, o = x_odd - odd_back, l = x_last - (HB & 1 ? even_back : odd_back);
 #pragma unroll
-                for (int h = 0; h < HB; ++h) xb[h] = ld16(xrow[h] + (h & 1 ? odd_block : even_block));
+                    for (int h = 0; h < HB; ++h)
+                        xb[h] = ld16(reinterpret_cast<const char*>(a.x + h * 8 * a.ldx + t * 32) + (h == HB - 1 ? l : h & 1 ? o : e));
+                } else {
+                    const int even_block = t * 32 + (whole ? second : 0), odd_block = t * 32 + (whole ? 32 - second : 0);
+#pragma unroll
+                    for (int h = 0; h < HB; ++h) xb[h] = ld16(xrow[h] + (h & 1 ? odd_block : even_block));
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int i = 0; i < U; ++i) {
                 const int ti = whole ? t + i * kNext : t;
+                uint32_t lane_bytes = lane * 16u;
+                asm("" : "+v"(lane_bytes));   // (the address stays a scalar one and an offset: summed outside the loop it is SG pairs of registers)
 #pragma unroll
-                for (int sI = 0; sI < SG; ++sI) wb[i][sI] = ld16_nt(wbase[sI] + (int64_t)ti * 64);
+                for (int sI = 0; sI < SG; ++sI) wb[i][sI] = ld16_nt(reinterpret_cast<const char*>(wbase[sI] + (int64_t)ti * 64) + lane_bytes);
                 if constexpr (!PAIR) {
 #pragma unroll
                     for (int b = 0; b < MB; ++b) xb[i * MB + b] = ld16(xrow[2 * b] + ti * 32);
@@ -1120,14 +1139,16 @@ static int mfma_strip_group(int m, int nt, int kt, bool free_reduce) {
     return best;
 }
 
-// Strips per wave of the ordered form: the model above, x out of L2 at 17 MB/us, in 8-row blocks (requests of two k-tiles; the groups that measured fastest at 31 of 33 shapes, 29 at 12.9)
-static int ordered_strip_group(int m, int nt, int kt, int ks) {
+// Strips of a workgroup of the ordered form: the model above, x out of L2 at 17 MB/us, in 8-row blocks (requests of two k-tiles; the
+// groups that measured fastest at 31 of 33 shapes, 29 at 12.9).  Groups of three where those deal the strips out (two -> four -> three):
+// 64 rows 8208 x 4096 29.2 -> 25.7 -> 20.2 us, 37 rows 11264 x 4096 27.0 -> 23.1 -> 19.8, but 12304 x 4096 27.4 -> 24.2 -> 29.4.
+int wgemm_ordered_group(int m, int nt, int kt, int ks) {
     const int mb = (m + 15) / 16, rows = (m + 7) / 8 * 8;
     const int cus = num_cus();
     int best = 1;
     double best_us = 1e30;
     for (int sg = 4; sg >= 1; --sg) {
-        if (ks != 4 && (sg * mb > (ks == 16 ? 8 : 16) || sg == 3 || (sg == 4 && ks == 16))) continue;   // 128 KiB of LDS; the instances there are
+        if (ks == 16 && sg > 2) continue;   // 128 KiB of LDS
         const long units = (nt + sg - 1) / sg;
         const double fill = (double)units / (double)(((units + cus - 1) / cus) * cus);
         const double us = (double)nt * kt * 1024e-6 / (6.45 * fill) + (double)units * rows * kt * 64e-6 / 17.0;
@@ -1157,6 +1178,7 @@ static int launch_ordered_rows(const GemmArgs& a, int sg, int ks, int grid, hipS
         case 4 * 8 + 4: return launch_ordered<HB, 4, 4>(a, grid, s);
         case 8 * 8 + 1: return launch_ordered<HB, 1, 8>(a, grid, s);
         case 8 * 8 + 2: return launch_ordered<HB, 2, 8>(a, grid, s);
+        case 8 * 8 + 3: return launch_ordered<HB, 3, 8>(a, grid, s);
         case 8 * 8 + 4: return launch_ordered<HB, 4, 8>(a, grid, s);
         case 16 * 8 + 1: return launch_ordered<HB, 1, 16>(a, grid, s);
         case 16 * 8 + 2: return launch_ordered<HB, 2, 16>(a, grid, s);
@@ -1167,14 +1189,18 @@ static int launch_ordered_rows(const GemmArgs& a, int sg, int ks, int grid, hipS
 // Up to a limit on rows x k-tiles: a workgroup reads all of x for the strips it has, whatever their number, where the sliced tiles
 // read a piece and pay for slabs and their reduction.  Sixty a strip and no fewer than 4096 (n x k, us, sliced
 // tiles and their reduction -> here): 37 rows 2048 x 2048 8.8 -> 6.9, 11264 x 2048 17.3 -> 12.2, 6144 x 4096 18.3 -> 14.4, 7168 x 8192 35.2 ->
-// 26.3, 8192 x 3584 19.8 -> 13.7, 4096 x 3584 12.8 -> 10.4; 64 rows 2048 x 2048 9.7 -> 8.3, 8192 x 1024 13.6 -> 8.2, 1536 x 4096 13.4 -> 13.6
-// (8192 for 96 strips: out); 256 strips of 448 k-tiles 32 rows 31.2 -> 29.4, 40 rows (17920) 32.0 -> 32.9; 80 strips of 256 16 rows 13.1 ->
-// 12.4, 20 rows (6144) 12.9 -> 13.5.  Tiles narrow enough to give every unit a slice (`strips` of 1) of a long k are ahead from nine rows on:
-// 2048 x 5632 8 rows 9.1, 9.1, 16 rows 9.2, 9.8, 37 rows 10.9, 13.4.
+// 26.3, 8192 x 3584 19.8 -> 13.7, 4096 x 3584 12.8 -> 10.4; 64 rows 2048 x 2048 9.7 -> 8.3, 8192 x 1024 13.6 -> 8.2, 8208 x 4096 30 -> 20,
+// 14336 x 14336 91 -> 83, 6144 x 11264 (22528) 42.1 -> 43.3, 5120 x 14336 (28672, out) 46 -> 52; 256 strips of 448 k-tiles 32 rows 31.2 ->
+// 29.4, 40 rows (17920) 32.0 -> 32.9.
+// Tiles narrow enough to give every unit a slice are ahead sooner.  One strip a wave and a long k: eight rows, and of those 512 x 14336
+// (3584) 12.3 -> 12.8, 768 x 11264 (2816) 11.7 -> 11.8.  Two: 65536 over the slices - in sixteen 1536 x 5120 at 24 rows (3840) 12.3 ->
+// 11.3, 2048 x 8192 at 16 (4096) 13.9 -> 13.0, but 2048 x 5120 at 24 10.9 -> 11.5, at 40 (6400) 11.1 -> 14.5, 2048 x 6144 at 24 (4608) 11.2 ->
+// 12.2, 1536 x 11264 at 16 (5632) 15.2 -> 16.6; in eight 4096 x 4096 at 64 (8192) 14.4 -> 13.9, 4096 x 5120 at 64 (10240) 16.0 -> 18.2.
 bool wgemm_ordered_takes(int m, int nt, int kt, int ks, int strips) {
     if ((ks != 4 && ks != 8 && ks != 16) || m > 64) return false;
     const int rows = (m + 7) / 8 * 8;
-    if (strips == 1 && kt > 128) return rows <= 8;
+    if (strips == 1 && kt > 128) return rows * kt <= 3072 && rows <= 8;
+    if (strips == 2) return rows * kt <= 65536 / ks;
     return (int64_t)rows * kt <= std::max(60 * nt, 4096);
 }
 
@@ -1202,10 +1228,10 @@ int launch_wgemm_ordered(const void* x, int64_t ldx, const void* w_tiles, const 
     a.ksplit = 1;
     a.ktps = a.kt / ks;
     a.partial = norm ? norm->slab : nullptr;
-    const int sg = ordered_strip_group(m, a.nt, a.kt, ks);
+    const int sg = wgemm_ordered_group(m, a.nt, a.kt, ks);
     a.nunits = (a.nt + sg - 1) / sg;
     const int mb = (m + 15) / 16;
-    // a second workgroup per CU where its reduction buffer fits beside the first
+    // more workgroups a CU where their registers allow it (four waves of four slices) or their reduction buffers do
     const int per_cu = ks == 4 ? 4 : ks * sg * mb <= 64 ? 2 : 1;
     const int grid = a.nunits < num_cus() * per_cu ? a.nunits : num_cus() * per_cu;
     const int rc = with_row_blocks(m, [&](auto hb) { return launch_ordered_rows<decltype(hb)::value>(a, sg, ks, grid, s); });

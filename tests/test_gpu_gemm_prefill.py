@@ -514,7 +514,7 @@ def test_narrow_tiles_give_the_sums_of_wide_ones(mv, m, n, k, mode):
 
 
 # slices added in the workgroup: four, eight and sixteen slices, every count of 8-row blocks, k-tiles of a slice that are fewer than the
-# stages in flight, as many, and a few more, groups of one to four strips with strips left over: the sums of the sliced 64-row tiles bit for bit
+# stages in flight, as many, and a few more, strips left over: the sums of the sliced 64-row tiles, bit for bit where both are cut alike
 @pytest.mark.parametrize("m", [5, 8, 9, 17, 25, 33, 40, 41, 49, 57, 64])
 @pytest.mark.parametrize("n,k", [(4112, 1024), (8224, 1024), (11280, 2048), (16400, 1024), (2064, 2048), (1536, 4096), (6160, 4096)])
 def test_short_prompts_add_their_slices_in_the_workgroup(mv, m, n, k):
@@ -536,3 +536,34 @@ def test_short_prompts_add_their_slices_in_the_workgroup(mv, m, n, k):
     if L.mv_gemm_prefill_workspace_bytes(m, n, k) - counters == ks * m * n * 4:
         more = torch.cat([x, torch.zeros(65 - m, k, dtype=torch.bfloat16, device=DEV)])
         assert torch.equal(gemm_prefill(more, sw, torch.empty(65, n, dtype=torch.float32, device=DEV))[:m], got)
+
+
+# slices added in the workgroup: every instance of the kernel, that is four slices in groups of one to four strips, eight in one to four,
+# sixteen in one and two, by every count of 8-row blocks; more k-tiles in a slice than stages in flight and fewer, strips left over.  The
+# slices' own products added in order, bit for bit
+@pytest.mark.parametrize("m", [5, 8, 9, 17, 25, 33, 40, 41, 49, 57, 64])
+@pytest.mark.parametrize("n,k,slices,group", [(528, 1024, 4, 1), (4112, 1024, 4, 2), (8224, 1024, 4, 3), (12560, 1024, 4, 4),
+                                              (528, 2048, 8, 1), (4112, 2048, 8, 2), (8208, 3072, 8, 3), (12304, 4096, 8, 4),
+                                              (2560, 4096, 16, 1), (5120, 8192, 16, 2)])
+def test_every_instance_adds_its_slices_in_order(mv, m, n, k, slices, group):
+    from micro_vllm_amd import _native as nv
+    from micro_vllm_amd.kernel.linear import StreamedWeight, gemm_prefill
+
+    L = nv.lib()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (L.mv_gemm_prefill_workspace_bytes(m, n, k) - 4096) // (4 * m * n) == slices
+        assert L.mv_gemm_prefill_group(m, n, k) == group
+    g = torch.Generator().manual_seed(m + n + k)
+    wide = torch.full((m, k + 24), float("nan"), dtype=torch.bfloat16, device=DEV)    # nothing beside the rows reaches a sum
+    wide[:, :k] = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    x = wide[:, :k]
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    got = gemm_prefill(x, StreamedWeight.from_linear(w), torch.full((m, n), float("nan"), dtype=torch.float32, device=DEV))
+    total, kk = torch.zeros(m, n, device=DEV), k // slices
+    for i in range(slices):
+        xs, part = x[:, i * kk:(i + 1) * kk].contiguous(), torch.empty(m, n, device=DEV)
+        ws = StreamedWeight.from_linear(w[:, i * kk:(i + 1) * kk].contiguous())
+        nv.check("mv_gemm_prefill", L.mv_gemm_prefill(xs.data_ptr(), kk, ws.tiles.data_ptr(), None, None, 0, part.data_ptr(),
+                                                      n, m, n, kk, nv.MV_GEMM_OUT_F32, nv.stream_ptr()))
+        total += part
+    assert torch.equal(got, total)
