@@ -1061,19 +1061,25 @@ static int launch_mfma_act(const GemmArgs& a, int grid, hipStream_t s) {
 
 // Pairs of k-tiles, or a k-tile a request (PAIR = false).  By pairs the waves read their weights two tiles at a time, which a long
 // stream takes 3 to 7 % slower (128256 x 8192 at 8 rows 317 -> 339 us, 128256 x 4096 169 -> 175: the eight waves' 1 KiB pieces no longer
-// lie side by side), so it is for where x is what costs: not up to 16 rows of k past 2048 in groups of strips, nor in groups of
-// seven (28672 x 4096 at 32 rows 38.4, 39.6 by pairs), nor one 8-row block, whose operand repeats its rows, in groups narrower
-// than four.
+// lie side by side), so it is for where x is what costs.  A k-tile a request instead:
+//   groups of seven strips (32 rows, 28672 x 1024 13.3 us, 13.9 by pairs, 28672 x 2048 21.9, 22.7, 28672 x 4096 47.5, 49.5);
+//   one 8-row block, whose operand repeats its rows, in groups narrower than four;
+//   up to 16 rows of k past 2048 in groups;
+//   groups of four strips of 128 KB up to 48 rows: their requests by pairs meet on memory channels (24 rows 16384 x 4096 25.0, 28.8 by pairs,
+//   128256 x 4096 175, 190; 48 rows 32000 x 4096 52.9, 55.7; of 96 or 160 KB pairs are ahead: 32000 x 5120 55, 51).
 template <int HB>
 static int launch_mfma(const GemmArgs& a, int sg, int grid, hipStream_t s) {
     auto strips = [&](auto count) {
         constexpr int SG = decltype(count)::value;
-        if constexpr ((HB <= 2 && SG > 1) || HB == 1 || SG == 7) {
-            constexpr int rows = HB <= 2 ? 2 : 4;
-            if (a.k > 2048 || (HB == 1 && SG < 4))
+        constexpr bool kNever = SG == 7 || (HB == 1 && SG < 4);
+        constexpr bool kLong = HB <= 2 && SG > 1, kMeet = SG == 4 && HB > 2 && HB <= 6;
+        if constexpr (kNever || kLong || kMeet) {
+            constexpr int rows = (HB + 1) / 2 * 2;
+            if (kNever || (kLong && a.k > 2048) || (kMeet && a.kt == 128))
                 return a.act.kind ? launch_mfma_act<rows, SG, true, false>(a, grid, s) : launch_mfma_act<rows, SG, false, false>(a, grid, s);
         }
-        return a.act.kind ? launch_mfma_act<HB, SG, true, true>(a, grid, s) : launch_mfma_act<HB, SG, false, true>(a, grid, s);
+        if constexpr (!kNever)
+            return a.act.kind ? launch_mfma_act<HB, SG, true, true>(a, grid, s) : launch_mfma_act<HB, SG, false, true>(a, grid, s);
     };
     if constexpr (HB <= 4) {
         if (sg == 7) return strips(std::integral_constant<int, 7>());

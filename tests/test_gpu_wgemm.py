@@ -281,3 +281,9 @@ def test_wgemm_by_pairs_of_k_tiles(mv, m, n, k, sg):
     # fp32 sums of exact products: at most k roundings of 2^-24 of partial sums that the absolute products bound
     bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
     assert bool(((acc.cpu().double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m", [16, 17, 24, 25, 40, 41, 48, 49])
+def test_wgemm_groups_of_strips_of_128_KB(mv, m):
+    """k = 4096 in groups of four strips: a k-tile a request up to 48 rows, pairs past them."""
+    test_wgemm_by_pairs_of_k_tiles(mv, m, 336, 4096, 4)
