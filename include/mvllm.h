@@ -518,7 +518,11 @@ int mv_graph_destroy(void* graph_exec);
  * 1 = fp32 (the whole model in 32 bits).  Everything else is fp32 in both.
  * ------------------------------------------------------------------------------------------------ */
 
-/* y[M,N] (fp32) = x[M,K] . W[N,K]^T, row-major operands of the activation type, any M, N, K. */
+/* Which form a product of aligned fp32 rows takes (for tests): 0 to 3 = the weights streamed past up to 4 rows (a step of 32 k at a
+ * time, four), 8 and 16; 4 to 9 = tiles of 32 x 32 (four groups of waves), 64 x 64 (four, two, one), 64 x 128, 128 x 128. */
+int mv_linear_any_form(int m, int n, int k);
+/* y[M,N] (fp32) = x[M,K] . W[N,K]^T, row-major operands of the activation type, any M, N, K.  fp32: products and sums of 32 bits
+ * over the whole range of the type. */
 int mv_linear_any(const void* x, int64_t ldx, const void* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
                   int k, int f32, mv_stream_t stream);
 

@@ -71,6 +71,7 @@ PROTOTYPES = {
     "mv_gemm_prefill": (_I, [_P, _L, _P, _P, _P, _L, _P, _L, _I, _I, _I, _I, _P]),
     "mv_gemm_prefill_workspace_bytes": (_Z, [_I, _I, _I]),
     "mv_linear_any_slab_count": (_I, [_I, _I, _I]),
+    "mv_linear_any_form": (_I, [_I, _I, _I]),
     "mv_linear_any_slabs": (_I, [_P, _L, _P, _L, _P, _Z, _I, _I, _I, _P]),
     "mv_linear_act_workspace_bytes": (_Z, [_I, _I, _I]),
     "mv_linear_act": (_I, [_P, _L, _P, _P, _L, _I, _I, _I, _I, _F, _F, _P, _Z, _P]),

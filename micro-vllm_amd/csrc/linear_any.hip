@@ -980,10 +980,12 @@ static bool streams_f32(int m, int n, int k) {
     return m <= (n < kStreamWide || k > kStreamShortK ? kStreamRows : kStreamRowsLess);
 }
 
+static int stream_form(int m, int k, int slices) { return m > 8 ? 3 : m > 4 ? 2 : k / slices > mv::kStreamOneStep ? 1 : 0; }
+
 static int launch_linear_stream(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
                                 int k, int slices, hipStream_t s) {
     using namespace mv;
-    const int form = m > 8 ? 3 : m > 4 ? 2 : k / slices > kStreamOneStep ? 1 : 0;
+    const int form = stream_form(m, k, slices);
     const size_t lds = (size_t)4 * (16 * kStreamPad * 4 + stream_x_bytes(form == 3 ? 16 : form == 2 ? 8 : 4));
     static LdsOptIn done[4];
     const auto kernel = form == 0   ? linear_stream_f32_kernel<4, 1>
@@ -1004,17 +1006,10 @@ static int launch_linear_stream(const float* x, int64_t ldx, const float* w, int
 //   567 rows 1024 x 5120:  78, 54, 61, 89, 129, 203        33 rows 1024 x 5120: 26, 49, 58, 88, 127, 200
 //   2048 rows 16384 x 4096: 2724, 1632, 1273, 1208, 944, 873
 // With segments `m` bounds a segment, not the launch: the rows are taken to be spread evenly.
-static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
-                             int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s, mv::RowSegments sg,
-                             int total_rows) {
+static int f32_tiles(int64_t rows, int n, int k, int batch) {
     using namespace mv;
-    if (streams_f32(m, n, k) && !sg.seg && batch == 1 && k % 4 == 0 && ldx % 4 == 0 &&
-        ldw % 4 == 0 && aligned16(x) && aligned16(w)) {
-        return launch_linear_stream(x, ldx, w, ldw, y, ldy, m, n, k, 1, s);
-    }
-    const int64_t per = sg.seg ? (total_rows + batch - 1) / batch : m;
     const int64_t cus = num_cus();
-    auto turns = [&](int bm, int bn) { return (((per + bm - 1) / bm) * ((n + bn - 1) / bn) * batch + cus - 1) / cus; };
+    auto turns = [&](int bm, int bn) { return (((rows + bm - 1) / bm) * ((n + bn - 1) / bn) * batch + cus - 1) / cus; };
     const int64_t steps = (k + kLfBK - 1) / kLfBK, quarter = (steps + 3) / 4;
     const int64_t n32 = turns(32, 32), n64 = turns(64, 64), n128 = turns(64, 128), n256 = turns(128, 128);
     const int64_t cost[6] = {100 + n32 * (250 + 57 * quarter),       n64 * (400 + 128 * quarter),
@@ -1023,7 +1018,18 @@ static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_
     int best = 0;
     for (int i = 1; i < 6; ++i)
         if (cost[i] < cost[best]) best = i;
-    switch (best) {
+    return best;
+}
+
+static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_t ldw, float* y, int64_t ldy, int m, int n,
+                             int k, int batch, int64_t zx, int64_t zw, int64_t zy, hipStream_t s, mv::RowSegments sg,
+                             int total_rows) {
+    using namespace mv;
+    if (streams_f32(m, n, k) && !sg.seg && batch == 1 && k % 4 == 0 && ldx % 4 == 0 &&
+        ldw % 4 == 0 && aligned16(x) && aligned16(w)) {
+        return launch_linear_stream(x, ldx, w, ldw, y, ldy, m, n, k, 1, s);
+    }
+    switch (f32_tiles(sg.seg ? (total_rows + batch - 1) / batch : m, n, k, batch)) {
         case 0: return launch_linear_f32_tiles<1, 1, 4, 2, true>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
         case 1: return launch_linear_f32_tiles<2, 2, 4, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
         case 2: return launch_linear_f32_tiles<2, 2, 2, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
@@ -1031,6 +1037,11 @@ static int launch_linear_f32(const float* x, int64_t ldx, const float* w, int64_
         case 4: return launch_linear_f32_tiles<2, 4, 1, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
         default: return launch_linear_f32_tiles<4, 4, 1, 1, false>(x, ldx, w, ldw, y, ldy, m, n, k, batch, zx, zw, zy, s, sg);
     }
+}
+
+extern "C" int mv_linear_any_form(int m, int n, int k) {
+    if (m <= 0 || n <= 0 || k <= 0) return -1;
+    return streams_f32(m, n, k) && k % 4 == 0 ? stream_form(m, k, 1) : 4 + f32_tiles(m, n, k, 1);
 }
 
 static int launch_linear_any(const void* x, int64_t ldx, const void* w, int64_t ldw, float* y, int64_t ldy, int m, int n,

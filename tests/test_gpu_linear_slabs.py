@@ -271,10 +271,13 @@ def test_short_k_of_one_and_two_rows(mv, n, k):
 
 
 # fp32 factors in three bf16 parts: what those cannot hold (infinities, NaN, values that round to an infinite bf16, sums in the
-# range of the smallest numbers) has the value of fp32 arithmetic, and only it: neighbours keep their bits.  One shape for each
-# form: streamed, six tiles, a k that ends inside a step
-@pytest.mark.parametrize("m,n,k", [(3, 1024, 1024), (16, 50, 516), (20, 1000, 1022), (33, 9472, 256), (200, 4000, 128),
-                                   (567, 1024, 640), (333, 9472, 68), (2048, 4096, 64)])
+# range of the smallest numbers) has the value of fp32 arithmetic, and only it: neighbours keep their bits.  Every form has a shape
+# (test_fp32_forms_of_the_shapes_here): streamed, six tiles, a k that ends inside a step
+_BEYOND = [(3, 1024, 1024), (16, 50, 516), (20, 1000, 1022), (33, 9472, 256), (200, 4000, 128), (567, 1024, 640), (333, 9472, 68),
+           (2048, 4096, 64), (4, 1024, 2048), (8, 528, 516), (1000, 5000, 516), (700, 5001, 514), (567, 9472, 1024), (2050, 9472, 1028)]
+
+
+@pytest.mark.parametrize("m,n,k", _BEYOND)
 def test_fp32_values_beyond_the_parts(mv, m, n, k):
     from micro_vllm_amd.kernel.ragged_ops import AnyLinear
 
@@ -313,9 +316,11 @@ def test_fp32_values_beyond_the_parts(mv, m, n, k):
 # fp32 factors far apart in size, whose sum is an ordinary number: of a small factor the parts lose bits, and a sum of zeros may be
 # parts that are all lost.  The shapes go to each form: streamed with 4, 8, 16 rows, whole and in slices, the six tiles (the last
 # four by scalar loads)
-@pytest.mark.parametrize("m,n,k", [(3, 1024, 1024), (3, 1024, 5120), (8, 528, 516), (16, 50, 516), (33, 9472, 256), (333, 9472, 68), (1000, 5000, 516),
-                                   (567, 9472, 1024), (2050, 9472, 1028), (20, 1000, 1022), (200, 16390, 514), (700, 5001, 514),
-                                   (2050, 9001, 1022)])
+_FAR_APART = [(3, 1024, 1024), (3, 1024, 5120), (8, 528, 516), (16, 50, 516), (33, 9472, 256), (333, 9472, 68), (1000, 5000, 516),
+              (567, 9472, 1024), (2050, 9472, 1028), (20, 1000, 1022), (200, 16390, 514), (700, 5001, 514), (2050, 9001, 1022)]
+
+
+@pytest.mark.parametrize("m,n,k", _FAR_APART)
 def test_fp32_factors_of_any_size(mv, m, n, k):
     from micro_vllm_amd.kernel.ragged_ops import AnyLinear
 
@@ -345,8 +350,11 @@ def test_fp32_factors_of_any_size(mv, m, n, k):
 
 
 # the sums of a row are those of four quarters of k in ascending order in every form: streamed, and the six tiles
-@pytest.mark.parametrize("many,n,k", [(20, 1000, 1022), (33, 9472, 256), (567, 1024, 640), (333, 9472, 68), (700, 3000, 250),
-                                      (1100, 4112, 1000), (1000, 5000, 516), (567, 9472, 1024), (2050, 9472, 1028)])
+_AMONG_MANY = [(20, 1000, 1022), (33, 9472, 256), (567, 1024, 640), (333, 9472, 68), (700, 3000, 250), (1100, 4112, 1000),
+               (1000, 5000, 516), (567, 9472, 1024), (2050, 9472, 1028)]
+
+
+@pytest.mark.parametrize("many,n,k", _AMONG_MANY)
 def test_fp32_rows_do_not_depend_on_the_others(mv, many, n, k):
     from micro_vllm_amd.kernel.ragged_ops import AnyLinear
 
@@ -382,3 +390,15 @@ def test_low_bits_in_some_steps_only(mv, n, k, many):
     assert bool((err <= k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())).all())
     for rows in (1, 4, 5, 8, 9, 16, 33):
         assert torch.equal(lin(x[:rows]), want[:rows])
+
+
+def test_fp32_forms_of_the_shapes_here(mv):
+    """The lists above reach what they say they do: all streamed forms and all six tiles."""
+    from micro_vllm_amd import _native as nv
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("laid out for 256 compute units")
+    forms = lambda shapes: {nv.lib().mv_linear_any_form(*s) for s in shapes}   # noqa: E731
+    assert forms(_BEYOND) == forms(_FAR_APART) == set(range(10))
+    assert forms(_AMONG_MANY) == set(range(4, 10))
+    assert [nv.lib().mv_linear_any_form(rows, 1024, 2048) for rows in (1, 5, 9, 17)] == [1, 2, 3, 4]

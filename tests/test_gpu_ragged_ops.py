@@ -54,7 +54,7 @@ def test_linear_any(ops, f32, m, n, k):
                                        (33, 33, 31, 1), (64, 9000, 132, 0), (200, 9000, 132, 0), (700, 1100, 160, 4),
                                        (4100, 2100, 64, 0)])
 def test_linear_any_f32_forms(ops, m, n, k, pad):
-    """Streamed weights, the three tiles, vector and scalar loads: each within the bound of a 32-bit sum, and all of them the
+    """Streamed weights, tiles, vector and scalar loads: each within the bound of a 32-bit sum, and all of them the
     same sums bit for bit (a row on its own, behind its neighbours, in rows of a wider buffer)."""
     g = torch.Generator().manual_seed(m + n + k)
     x, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
