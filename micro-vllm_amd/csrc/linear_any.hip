@@ -998,13 +998,16 @@ static int launch_linear_stream(const float* x, int64_t ldx, const float* w, int
 }
 
 // Which fp32 form.  Few rows of one product stream the weights (see kStreamRows).  Otherwise the tile by the time the launch
-// takes in it, in hundredths of a us as measured: with n = tiles over compute units, rounded up, a tile of a whole quarter a group
-// takes n times its own time (one workgroup fills a unit), and the others a step in which n workgroups of a unit take turns at
-// its matrix unit, vector unit and LDS.  A launch of few tiles takes small ones and many groups, a large one the tile that reads
-// and splits its operands least often.  us in (outputs of the tile, groups), weights of bf16 values:
+// takes in it, in hundredths of a us: with n = tiles over compute units, rounded up, a start, an end of every tile (its sums' way
+// out), and a step in which the workgroups of a unit take turns at its matrix unit, vector unit and LDS (in four groups a quarter of the
+// steps, one workgroup to a unit).  A launch of few tiles takes small ones and many groups, a large one the tile that reads
+// and splits its operands least often; a short k is told by the tiles' ends.  Fitted to 1000 shapes of 17 to 2048 rows, 64 to 65536
+// outputs and k of 64 to 8192: the tile it names takes 0.9 % more than the best of the six in the mean, 33 % at most (few rows of wide
+// outputs, which wait for memory: 17 rows 48000 x 2048 108 us, 81 in 32 x 32; 65536 x 1024 69, 53 in 64 x 64 by two groups).  us in (outputs of the tile, groups), weights of bf16 values:
 //   567 rows 9472 x 1024: 149 (32 x 32, 4), 82 (64 x 64, 4), 64 (64 x 64, 2), 61 (64 x 64), 49 (64 x 128), 62 (128 x 128)
 //   567 rows 1024 x 5120:  78, 54, 61, 89, 129, 203        33 rows 1024 x 5120: 26, 49, 58, 88, 127, 200
 //   2048 rows 16384 x 4096: 2724, 1632, 1273, 1208, 944, 873
+//   1024 rows 32000 x 64: 350, 163, 103, 62.5, 61, 60.5 (70 on the fp32 instruction)    567 rows 9472 x 256: -, 37, 26.8, 23.7, 22, 27.5
 // With segments `m` bounds a segment, not the launch: the rows are taken to be spread evenly.
 static int f32_tiles(int64_t rows, int n, int k, int batch) {
     using namespace mv;
@@ -1012,9 +1015,12 @@ static int f32_tiles(int64_t rows, int n, int k, int batch) {
     auto turns = [&](int bm, int bn) { return (((rows + bm - 1) / bm) * ((n + bn - 1) / bn) * batch + cus - 1) / cus; };
     const int64_t steps = (k + kLfBK - 1) / kLfBK, quarter = (steps + 3) / 4;
     const int64_t n32 = turns(32, 32), n64 = turns(64, 64), n128 = turns(64, 128), n256 = turns(128, 128);
-    const int64_t cost[6] = {100 + n32 * (250 + 57 * quarter),       n64 * (400 + 128 * quarter),
-                             400 + 2 * quarter * (15 + 58 * n64),    300 + 100 * n64 + steps * (30 + 25 * n64),
-                             300 + 200 * n128 + steps * (30 + 43 * n128), 600 + 400 * n256 + steps * (40 + 82 * n256)};
+    const int64_t cost[6] = {284 + n32 * (333 + 47 * quarter),
+                             175 + n64 * (265 + 141 * quarter),
+                             226 + 206 * n64 + 2 * quarter * (24 + 48 * n64),
+                             294 + 133 * n64 + steps * (27 + 23 * n64),
+                             340 + 267 * n128 + steps * (29 + 37 * n128),
+                             114 + 744 * n256 + steps * (50 + 59 * n256)};
     int best = 0;
     for (int i = 1; i < 6; ++i)
         if (cost[i] < cost[best]) best = i;

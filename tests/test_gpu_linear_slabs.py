@@ -273,7 +273,7 @@ def test_short_k_of_one_and_two_rows(mv, n, k):
 # fp32 factors in three bf16 parts: what those cannot hold (infinities, NaN, values that round to an infinite bf16, sums in the
 # range of the smallest numbers) has the value of fp32 arithmetic, and only it: neighbours keep their bits.  Every form has a shape
 # (test_fp32_forms_of_the_shapes_here): streamed, six tiles, a k that ends inside a step
-_BEYOND = [(3, 1024, 1024), (16, 50, 516), (20, 1000, 1022), (33, 9472, 256), (200, 4000, 128), (567, 1024, 640), (333, 9472, 68),
+_BEYOND = [(3, 1024, 1024), (1100, 4112, 1000), (16, 50, 516), (20, 1000, 1022), (33, 9472, 256), (200, 4000, 128), (567, 1024, 640), (333, 9472, 68),
            (2048, 4096, 64), (4, 1024, 2048), (8, 528, 516), (1000, 5000, 516), (700, 5001, 514), (567, 9472, 1024), (2050, 9472, 1028)]
 
 
@@ -316,7 +316,7 @@ def test_fp32_values_beyond_the_parts(mv, m, n, k):
 # fp32 factors far apart in size, whose sum is an ordinary number: of a small factor the parts lose bits, and a sum of zeros may be
 # parts that are all lost.  The shapes go to each form: streamed with 4, 8, 16 rows, whole and in slices, the six tiles (the last
 # four by scalar loads)
-_FAR_APART = [(3, 1024, 1024), (3, 1024, 5120), (8, 528, 516), (16, 50, 516), (33, 9472, 256), (333, 9472, 68), (1000, 5000, 516),
+_FAR_APART = [(3, 1024, 1024), (1100, 4112, 1002), (33, 5000, 516), (3, 1024, 5120), (8, 528, 516), (16, 50, 516), (33, 9472, 256), (333, 9472, 68), (1000, 5000, 516),
               (567, 9472, 1024), (2050, 9472, 1028), (20, 1000, 1022), (200, 16390, 514), (700, 5001, 514), (2050, 9001, 1022)]
 
 
