@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256, RING == 3 || MT == 4 ? 2 : 1) void gemm_prefil
     for (int i = 0; i < NT; ++i)
         wp[i] = a.w + ((int64_t)min(nt0 + i, a.nt - 1) * a.kt + kt0) * 64 + lane;
 
-    // ---- x: global -> LDS directly, BUFS stages deep, in fragment order ---------------------
+    // ---- x: global -> LDS directly, BUFS stages deep, by whole lines ------------------------
     // The LDS image of a stage is an m-tile after the other, 16 rows of 128 bytes (64 k) each; the 16-byte chunk c of row r sits
     // at position c ^ ((r >> 1) & 7) of its row, which keeps the fragment reads (lane (r, q) reads chunk 4 kk + q of row r) free
     // of bank conflicts, and a request of global_load_lds is eight whole rows of it (no staging registers, no LDS store

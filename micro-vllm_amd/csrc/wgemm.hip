@@ -1065,8 +1065,9 @@ static int launch_mfma_act(const GemmArgs& a, int grid, hipStream_t s) {
 //   groups of seven strips (32 rows, 28672 x 1024 13.3 us, 13.9 by pairs, 28672 x 2048 21.9, 22.7, 28672 x 4096 47.5, 49.5);
 //   one 8-row block, whose operand repeats its rows, in groups narrower than four;
 //   up to 16 rows of k past 2048 in groups;
-//   groups of four strips of 128 KB up to 48 rows: their requests by pairs meet on memory channels (24 rows 16384 x 4096 25.0, 28.8 by pairs,
-//   128256 x 4096 175, 190; 48 rows 32000 x 4096 52.9, 55.7; of 96 or 160 KB pairs are ahead: 32000 x 5120 55, 51).
+//   groups of four strips, 128 KB of each, up to 48 rows: their requests by pairs meet on memory channels (24 rows 16384 x 4096 25.0, 28.8 by
+//   pairs, 128256 x 4096 175, 190, 8192 x 8192 in two slices 24.6, 28.9; 48 rows 32000 x 4096 52.9, 55.7; of 64, 96 or 160 KB pairs are
+//   ahead: 8192 x 4096 in two slices 20.2, 14.1, 32000 x 5120 55, 51).
 template <int HB>
 static int launch_mfma(const GemmArgs& a, int sg, int grid, hipStream_t s) {
     auto strips = [&](auto count) {
@@ -1075,7 +1076,7 @@ static int launch_mfma(const GemmArgs& a, int sg, int grid, hipStream_t s) {
         constexpr bool kLong = HB <= 2 && SG > 1, kMeet = SG == 4 && HB > 2 && HB <= 6;
         if constexpr (kNever || kLong || kMeet) {
             constexpr int rows = (HB + 1) / 2 * 2;
-            if (kNever || (kLong && a.k > 2048) || (kMeet && a.kt == 128))
+            if (kNever || (kLong && a.k > 2048) || (kMeet && a.ktps == 128))
                 return a.act.kind ? launch_mfma_act<rows, SG, true, false>(a, grid, s) : launch_mfma_act<rows, SG, false, false>(a, grid, s);
         }
         if constexpr (!kNever)

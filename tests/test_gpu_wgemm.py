@@ -285,5 +285,6 @@ def test_wgemm_by_pairs_of_k_tiles(mv, m, n, k, sg):
 
 @pytest.mark.parametrize("m", [16, 17, 24, 25, 40, 41, 48, 49])
 def test_wgemm_groups_of_strips_of_128_KB(mv, m):
-    """k = 4096 in groups of four strips: a k-tile a request up to 48 rows, pairs past them."""
+    """k = 4096, and 8192 in two slices, in groups of four strips: a k-tile a request up to 48 rows, pairs past them."""
     test_wgemm_by_pairs_of_k_tiles(mv, m, 336, 4096, 4)
+    test_wgemm_by_pairs_of_k_tiles(mv, m, 8192, 8192, 4)
