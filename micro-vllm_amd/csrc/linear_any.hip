@@ -659,15 +659,15 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void linear_any_f32_kern
 // 1024 x 5120 12.6 -> 12.3 | 15.3 (8 rows 13.7 -> 13.4 | 16.1), 512 x 8192 17.4 -> 17.3 | 21.9.  16 rows split x behind LDS as well:
 // 16384 x 4096 49.6 -> 50.1 | 56, 1024 x 5120 16.4 -> 17.7 | 20.7.  Rows of bf16 values are what a checkpoint in that type gives.
 // Four steps' operands are read out of LDS before the first is used (1024 x 5120 13.8 -> 12.3 | 16.8 -> 15.3); one at a time leaves registers for a third
-// workgroup on a unit, which is ahead where a wave has two pieces or fewer (3 rows 32000 x 1024 22.8 against 23.5, 65536 x 256
-// 18.6 against 23.2; 32000 x 2048 42.0 against 40.8).
+// workgroup on a unit, which is ahead where a wave has three pieces or fewer (3 rows 32000 x 1024 22.8 against 23.5, 65536 x 256
+// 18.6 against 23.2, a slice of 1280 of 1024 x 5120 7.45 against 7.98; 32000 x 2048 42.0 against 40.8).
 // From nine rows on the tiles are ahead where the output is wide and k is short (16 rows, 65536 x 256: 18.9 us against 25, 32000 x 448
 // 16.3 against 22.5; 32000 x 512 28.6 against 18.9, 16384 x 4096 74 against 49), from 17 on everywhere; at k of up to 256 and
 // 16384 outputs from five (8 rows 65536 x 256 19 against 25, 32000 x 256 10.4 against 13.7, 16384 x 256 7.8 against 8.3, 9472 x 256 7.2 against
 // 6.8; 32000 x 448 15.8 each).
 constexpr int kStreamRowsLess = 4, kStreamRows = 8, kStreamRowsMore = 16, kStreamNarrow = 8192, kStreamWide = 16384;
 constexpr int kStreamShortK = 256, kStreamLongK = 512;
-constexpr int kStreamSlice = 8, kStreamOneStep = 1024;   // (a slice's k up to which steps go one by one)
+constexpr int kStreamSlice = 8, kStreamOneStep = 1536;   // (a slice's k up to which steps go one by one)
 constexpr int kStreamK = 128, kStreamPad = kStreamK + 4;   // k of a piece, floats of a row in LDS
 constexpr int kStreamParts = kStreamK * 2 + 16;            // bytes of a row's parts in LDS
 // A wave's rows of x lie in LDS split (a lane of the instruction whose column is a row past MR reads a row again, so split behind

@@ -367,10 +367,10 @@ def test_fp32_rows_do_not_depend_on_the_others(mv, many, n, k):
 
 # fp32 weights that are bf16 values but in single steps of 32 k: which rows take six products and which three changes from step to
 # step, from one block of sixteen rows to the next, and with how many steps a form looks at together.  A row alone (streamed, a step
-# or four at a time, both sides of k = 1024), 5, 8, 9 and 16 rows (streamed, and tiles where k is short and n wide) and many (tiles of every
+# or four at a time), 5, 8, 9 and 16 rows (streamed, and tiles where k is short and n wide) and many (tiles of every
 # size that goes with k) are the same bits
 @pytest.mark.parametrize("n,k,many", [(48, 1024, 40), (1040, 1028, 300), (1040, 1030, 300), (8208, 256, 70), (8208, 260, 600), (16400, 256, 70), (9472, 544, 600),
-                                      (4112, 1000, 1100)])
+                                      (4112, 1000, 1100), (528, 2052, 300)])
 def test_low_bits_in_some_steps_only(mv, n, k, many):
     from micro_vllm_amd.kernel.ragged_ops import AnyLinear
 
