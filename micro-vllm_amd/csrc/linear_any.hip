@@ -230,8 +230,8 @@ __device__ __forceinline__ bool lf_outside(float v, float xmax, float wmax) {
 }
 
 // Four values.  A part is subtracted by v_dot2_f32_bf16, (-1, 0) or (0, -1) times the packed pair, where that is faster than to
-// unpack it (streamed 16 rows 16384 x 4096 52.5 -> 50 us, 32 x 32 tiles 33 rows 1024 x 5120 28.8 -> 26.5; the wider tiles 0 to 3 % slower): every
-// result is exact either way.
+// unpack it (streamed 16 rows 16384 x 4096 52.5 -> 50 us, 32 x 32 tiles 33 rows 1024 x 5120 28.8 -> 26.5; the wider tiles 0 to 3 % slower, x a
+// step at a time in slices of 1024 x 5120 7.8 -> 8.2): every result is exact either way.
 template <bool DOT>
 __device__ __forceinline__ void lf_split4(const f32x4_t& v, uint2& hi, uint2& mid, uint2& lo) {
     uint32_t minus_lo = 0x0000bf80u, minus_hi = 0xbf800000u;
@@ -721,7 +721,7 @@ __global__ __launch_bounds__(256, STEPS == 1 ? 3 : 2) void linear_stream_f32_ker
             if (kSplitFirst) {   // four values: a half of what lane (row, k / 4 % 4) of the instruction takes of their step
                 x_max[i] = lf_largest(v, x_max[i]);
                 uint2 hi, mid, lo;
-                lf_split4<true>(v, hi, mid, lo);
+                lf_split4<(STEPS > 1)>(v, hi, mid, lo);
                 unsigned char* to = xb + (2 * i + half) * kStreamParts + (kl >> 5) * 64 + ((kl >> 2) & 3) * 16 + ((kl >> 4) & 1) * 8;
                 *reinterpret_cast<uint2*>(to) = hi;
                 *reinterpret_cast<uint2*>(to + MR * kStreamParts) = mid;
